@@ -34,6 +34,10 @@ struct Linear {
     int lda = 0;
     const int* a_rows = nullptr;
     int a_div = 1;
+    // tiled kernel (more than kGemvMaxRows rows): the same rows rounded to bf16 by their producer (lda, a_zoff in elements alike), read
+    // in A's place unless the product is a 32-bit one; and the result rounded to bf16 for the product that reads it next (C may then be null)
+    const bf16_t* A16 = nullptr;
+    bf16_t* C16 = nullptr;
     const bf16_t* B = nullptr;
     int ldb = 0;
     float* C = nullptr;

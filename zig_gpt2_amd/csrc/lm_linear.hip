@@ -1,13 +1,14 @@
 // lm_linear.hip — the linear maps of the layered-model tier: C = act(A B^T) with fp32 activation rows A and bf16 weights B.
 //
-// Two kernels behind one launcher:
+// Behind one launcher:
 //   * lm_gemv_kernel   up to 8 rows (decode steps): a wave owns two weight rows, its lanes split K in 16-byte pieces, the
 //                      activation rows come straight from the cache hierarchy, sums are fp32 FMAs in both precision modes.
-//   * lm_gemm_kernel   prompt portions: 64 x 64 or 128 x 128 tiles on the matrix cores, four waves in a 2 x 2 arrangement of
-//                      32 x 32 MFMA tiles.  bf16 mode rounds the activations to bf16 on their way into the LDS and multiplies with
-//                      v_mfma_f32_32x32x16_bf16 (fp32 accumulation); 32-bit mode widens the weights and multiplies with
-//                      v_mfma_f32_32x32x2_f32.  Any M, N, K: tiles are zero-filled at the edges.
-// Both understand the same addressing: a row gather for A, one matrix per grid.z batch (heads), a matrix chosen per batch by
+//   * lm_wide_kernel   prompt portions that fill the chip: 128 x 128 or 64 x 64 tiles staged through the LDS.
+//   * lm_deep_kernel   short portions: 32-wide tiles with K split over the waves of a workgroup.
+//                      Both multiply with v_mfma_f32_32x32x16_bf16: bf16 mode rounds the activations on their way there, 32-bit mode
+//                      multiplies their exact three-term bf16 split (the weights are bf16), fp32 accumulation.
+//   * lm_gemm_kernel   any alignment, any K: 64 x 64 tiles, one LDS buffer, the fp32 instruction in 32-bit mode.
+// All understand the same addressing: a row gather for A, one matrix per grid.z batch (heads), a matrix chosen per batch by
 // an index array (the expert of an assignment), and row groups sorted by expert with their offsets in device memory.
 #include <stdlib.h>
 
@@ -45,6 +46,8 @@ struct LinArgs {
     int glu_gate_col;
     const float* a_poly;
     float poly_eps;
+    const bf16_t* A16;  // the same rows as bf16 (tiled kernels), or null
+    bf16_t* C16;        // the result rounded to bf16, beside or instead of C (tiled kernels), or null
     int a_vec, b_vec;  // 16-byte loads allowed (alignment of base, leading dimension and batch offsets)
 };
 
@@ -357,6 +360,378 @@ __global__ __launch_bounds__(256) void lm_gemv_ks_kernel(const LinArgs p) {
 }
 
 // ------------------------------------------------------------------------------------------------ matrix cores
+// Both kernels below multiply bf16 tiles with v_mfma_f32_32x32x16_bf16 and accumulate in fp32.  NP = 1: the activations are rounded
+// to bf16 on their way to the matrix cores.  NP = 3 (32-bit mode): an activation is the exact sum of three bf16 terms and the
+// weights are bf16 as they are, so three products give the fp32 product exactly, at 5 times the rate of the fp32 instruction.
+// Both take 16-byte pieces: aligned operands, K a multiple of 8.
+
+// f(step<0>()) ... f(step<N - 1>()): indices known to the compiler, for rings kept in registers
+template <int I>
+using step = std::integral_constant<int, I>;
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void unroll(F&& f) {
+    if constexpr (I < N) {
+        f(step<I>());
+        unroll<N, I + 1>(f);
+    }
+}
+
+// eight consecutive fp32 values -> NP planes of eight bf16 (packed pairs)
+template <int NP>
+struct Planes8 {
+    u32x4 v[NP];
+};
+// the upper bf16 half of a value (truncated), and what is left of it (nothing of an infinity or NaN)
+__device__ __forceinline__ float term_left(float x) {
+    const uint32_t b = __float_as_uint(x);
+    const float r = x - __uint_as_float(b & 0xFFFF0000u);
+    return (b & 0x7F800000u) == 0x7F800000u ? 0.0f : r;
+}
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
+template <int NP>
+__device__ __forceinline__ Planes8<NP> to_planes(const f32x4& a, const f32x4& b) {
+    Planes8<NP> o;
+    if constexpr (NP == 1) {
+        o.v[0] = u32x4{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w), cvt_pk_bf16(b.x, b.y), cvt_pk_bf16(b.z, b.w)};
+    } else {
+        float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int t = 0; t < NP; ++t) {  // 24 mantissa bits = 8 + 8 + 8: what the third term leaves is zero
+            o.v[t] = u32x4{upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7])};
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (t + 1 < NP) x[i] = t == 0 ? term_left(x[i]) : x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+        }
+    }
+    return o;
+}
+
+// Eight consecutive activations in flight: fp32 as they are, or already rounded to bf16 by the kernel that wrote them.
+template <typename AT>
+struct Act8;
+template <>
+struct Act8<float> {
+    f32x4 a, b;
+    __device__ __forceinline__ void load(const float* row, int k) {
+        a = *reinterpret_cast<const f32x4*>(row + k);
+        b = *reinterpret_cast<const f32x4*>(row + k + 4);
+    }
+    __device__ __forceinline__ void clear() { a = b = f32x4{0.0f, 0.0f, 0.0f, 0.0f}; }
+    template <int NP>
+    __device__ __forceinline__ Planes8<NP> planes() const { return to_planes<NP>(a, b); }
+};
+__device__ __forceinline__ u32x4 load_b8(const bf16_t* row, int k) { return *reinterpret_cast<const u32x4*>(row + k); }
+template <>
+struct Act8<bf16_t> {
+    u32x4 v;
+    __device__ __forceinline__ void load(const bf16_t* row, int k) { v = load_b8(row, k); }
+    __device__ __forceinline__ void clear() { v = u32x4{0u, 0u, 0u, 0u}; }
+    template <int NP>
+    __device__ __forceinline__ Planes8<NP> planes() const {
+        static_assert(NP == 1, "rounded activations have one term");
+        return Planes8<1>{{v}};
+    }
+};
+
+// The tile of a workgroup: rows [m0, m_end) of A / C, columns from n0, the matrix.  Consecutive workgroups go to the eight XCDs in
+// turn, so the tile list is dealt in eight contiguous runs: the tiles of one run share their A rows in that XCD's L2.
+struct TileAt {
+    const bf16_t* B;
+    int m0, m_end, n0;
+};
+__device__ __forceinline__ bool find_tile(const LinArgs& p, int BM, int BN, TileAt& t) {
+    const int n_tiles = (p.N + BN - 1) / BN, total = gridDim.x, id = blockIdx.x;
+    const int q = total >> 3, r = total & 7, x = id & 7;
+    const int at = x * q + min(x, r) + (id >> 3);
+    int mt = at / n_tiles;
+    t.n0 = (at - mt * n_tiles) * BN;
+    t.B = p.B + (long long)blockIdx.z * p.b_zoff;
+    t.m0 = mt * BM;
+    t.m_end = p.M;
+    if (p.grp_off) {  // the row group this tile belongs to: 64 groups' tile counts summed across the lanes at a time
+        const int lane = threadIdx.x & 63;
+        for (int e0 = 0;; e0 += 64) {
+            if (e0 >= p.n_groups) return false;
+            const int e = min(e0 + lane, p.n_groups - 1);
+            const int lo = p.grp_off[e], hi = p.grp_off[e + 1];
+            const int own = e0 + lane < p.n_groups ? (hi - lo + BM - 1) / BM : 0;
+            int upto = own;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(upto, d, 64);
+                if (lane >= d) upto += o;
+            }
+            const unsigned long long past = __ballot(mt < upto);
+            if (past) {
+                const int l = __builtin_ctzll(past);
+                t.B = p.B + (long long)(e0 + l) * p.b_zoff;
+                t.m0 = __shfl(lo, l, 64) + (mt - __shfl(upto - own, l, 64)) * BM;
+                t.m_end = __shfl(hi, l, 64);
+                break;
+            }
+            mt -= __shfl(upto, 63, 64);
+        }
+    }
+    return t.m0 < t.m_end;
+}
+template <typename AT>
+__device__ __forceinline__ const AT* a_row(const LinArgs& p, int m) {
+    const AT* A;
+    if constexpr (std::is_same<AT, float>::value) A = p.A;
+    else A = p.A16;
+    return A + (long long)blockIdx.z * p.a_zoff + (long long)((p.a_rows ? p.a_rows[m] : m) / p.a_div) * p.lda;
+}
+// output (m, n), finished
+__device__ __forceinline__ void put(const LinArgs& p, int m, int n, float v) {
+    const long long at = (long long)blockIdx.z * p.c_zoff + (long long)m * p.ldc + n;
+    v = finish(v, n, p);
+    if (p.C) p.C[at] = v;
+    if (p.C16) p.C16[at] = (bf16_t)cvt_pk_bf16(v, v);
+}
+
+// What bounds it: the bytes a compute unit takes in (31 to 37 B per clock beside matrix products) and, per K step, one LDS round trip.
+// 8184 x 3072 x 1024 takes 106 us (490 TFLOP/s; before, with one LDS buffer and 64 x 64 tiles, 176), 8184 x 1024 x 4096 107 us
+// (640 TFLOP/s; 274), 333 x 768 x 3072 17.5 us (95): there the reads of a step's fragments, which the compiler had paired with a
+// wait for each product, and loads under a condition, which it waited for at every step, were three quarters of the time.
+// Enough rows to fill the chip: 64 TM x 64 TN tiles, four waves in a 2 x 2 arrangement of TM x TN MFMA tiles each.  Operands pass
+// through two LDS buffers (rows of BK elements, their 16-byte chunks swizzled by the row so that the fragment reads of eight
+// consecutive rows hit different banks); the registers hold the K step behind the one in the LDS, so a load has a whole step of
+// MFMAs to arrive, and there is one barrier per step.
+template <typename AT, int NP, int TM, int TN, int AHEAD>
+__global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LinArgs p) {
+    constexpr int BM = 64 * TM, BN = 64 * TN, BK = NP == 1 ? 64 : 32, CH = BK / 8;
+    constexpr int AC = BM * CH / 256, BC = BN * CH / 256;
+    __shared__ __attribute__((aligned(16))) bf16_t As[2][NP][BM * BK];
+    __shared__ __attribute__((aligned(16))) bf16_t Bs[2][BN * BK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wy = wave >> 1, wx = wave & 1;
+    TileAt t;
+    if (!find_tile(p, BM, BN, t)) return;
+    auto swz = [](int row) { return CH == 8 ? row & 7 : (row >> 1) & 3; };  // (row & 31 decides)
+
+    const AT* a_src[AC];
+    const bf16_t* b_src[BC];
+    int a_lds[AC], b_lds[BC];
+    const int kc = (tid % CH) * 8;  // this thread's chunk of every row it fetches
+#pragma unroll
+    for (int j = 0; j < AC; ++j) {
+        const int row = (tid + 256 * j) / CH;
+        a_src[j] = a_row<AT>(p, min(t.m0 + row, t.m_end - 1));  // (rows beyond the edge: some valid row, never stored)
+        a_lds[j] = row * BK + (((tid % CH) ^ swz(row)) * 8);
+    }
+#pragma unroll
+    for (int j = 0; j < BC; ++j) {
+        const int row = (tid + 256 * j) / CH;
+        b_src[j] = t.B + (long long)min(t.n0 + row, p.N - 1) * p.ldb;
+        b_lds[j] = row * BK + (((tid % CH) ^ swz(row)) * 8);
+    }
+    Act8<AT> a_ring[AHEAD][AC];
+    u32x4 b_ring[AHEAD][BC];
+    auto fetch = [&](auto slot, int k0) {
+        const int k = min(k0 + kc, p.K - 8);  // (columns beyond K: valid ones, zeroed when stashed)
+#pragma unroll
+        for (int j = 0; j < AC; ++j) a_ring[slot][j].load(a_src[j], k);
+#pragma unroll
+        for (int j = 0; j < BC; ++j) b_ring[slot][j] = load_b8(b_src[j], k);
+    };
+    const int n_steps = (p.K + BK - 1) / BK;
+    auto stash = [&](auto slot, int buf, int s) {
+        auto& a_reg = a_ring[slot];
+        auto& b_reg = b_ring[slot];
+        if (s == n_steps - 1 && s * BK + kc >= p.K) {  // chunks beyond K
+#pragma unroll
+            for (int j = 0; j < AC; ++j) a_reg[j].clear();
+#pragma unroll
+            for (int j = 0; j < BC; ++j) b_reg[j] = u32x4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int j = 0; j < AC; ++j) {
+            const Planes8<NP> pl = a_reg[j].template planes<NP>();
+#pragma unroll
+            for (int q = 0; q < NP; ++q) *reinterpret_cast<u32x4*>(&As[buf][q][a_lds[j]]) = pl.v[q];
+        }
+#pragma unroll
+        for (int j = 0; j < BC; ++j) *reinterpret_cast<u32x4*>(&Bs[buf][b_lds[j]]) = b_reg[j];
+    };
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+
+    // The fragments of a step: all requested before the first product, so that the LDS latency is paid once per step.
+    const int fr = lane & 31, kh = lane >> 5;
+    int a_at[TM], b_at[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a_at[i] = ((wy * TM + i) * 32 + fr) * BK;
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b_at[j] = ((wx * TN + j) * 32 + fr) * BK;
+    const int fswz = swz(fr);  // (32 rows apart the swizzle repeats)
+    u32x4 af[CH / 2][NP][TM], bf[CH / 2][TN];
+    auto read = [&](int cur) {
+#pragma unroll
+        for (int kk = 0; kk < CH / 2; ++kk) {
+            const int c = ((2 * kk + kh) ^ fswz) * 8;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bf[kk][j] = *reinterpret_cast<const u32x4*>(&Bs[cur][b_at[j] + c]);
+#pragma unroll
+            for (int q = NP - 1; q >= 0; --q)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) af[kk][q][i] = *reinterpret_cast<const u32x4*>(&As[cur][q][a_at[i] + c]);
+        }
+    };
+    auto multiply = [&]() {
+#pragma unroll
+        for (int kk = 0; kk < CH / 2; ++kk)
+#pragma unroll
+            for (int q = NP - 1; q >= 0; --q)  // the smallest terms first
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, af[kk][q][i]), __builtin_bit_cast(bf16x8, bf[kk][j]),
+                                                                            acc[i][j], 0, 0, 0);
+    };
+    // Step s is fetched AHEAD steps before it is stashed, and stashed while the step in front of it is multiplied.  Fetches and stashes
+    // are unconditional (beyond the last step they repeat valid addresses and nobody reads what they leave): a fetch under a
+    // condition would make the compiler wait for every load at every stash.
+    unroll<AHEAD>([&](auto i) { fetch(i, i * BK); });
+    stash(step<0>(), 0, 0);
+    fetch(step<0>(), AHEAD * BK);
+    __syncthreads();
+    int cur = 0, s = 0;
+    auto body = [&](auto i) {
+        constexpr int nx = (decltype(i)::value + 1) % AHEAD;
+        read(cur);
+        stash(step<nx>(), cur ^ 1, s + 1);
+        fetch(step<nx>(), (s + 1 + AHEAD) * BK);
+        multiply();
+        // order: the fragment reads, then between the products what the next steps need
+        constexpr int products = CH / 2 * NP * TM * TN;
+        __builtin_amdgcn_sched_group_barrier(0x100, CH / 2 * (NP * TM + TN), 0);
+#pragma unroll
+        for (int x = 0; x < products; ++x) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);
+            __builtin_amdgcn_sched_group_barrier(0x200, (AC * NP + BC + products - 1) / products, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, (AC * 2 + BC + products - 1) / products, 0);
+        }
+        cur ^= 1;
+        ++s;
+        __syncthreads();
+    };
+    for (int g = n_steps / AHEAD; g > 0; --g) unroll<AHEAD>(body);
+    if constexpr (AHEAD > 1)
+        unroll<AHEAD - 1>([&](auto i) {
+            if (s < n_steps) body(i);
+        });
+
+    // accumulator element e of a 32 x 32 tile: row 8 (e / 4) + 4 (lane / 32) + e % 4, column lane % 32
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = t.n0 + (wx * TN + j) * 32 + (lane & 31);
+            if (n >= p.N) continue;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = t.m0 + (wy * TM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                if (m < t.m_end) put(p, m, n, acc[i][j][e]);
+            }
+        }
+}
+
+// Too few tiles to fill the chip (portions of some hundred rows): 32 TM x 32 TN tiles, the four waves of a workgroup split K and meet
+// in the LDS.  Nothing is staged: a lane loads its own fragments (16 consecutive k of a row, both halves of a wave the whole
+// 128-byte line), no wave waits for another before the end, and a tile's time is a quarter of its K.  Bound by latency: 37 x 2304 x
+// 768 takes 6.5 us (15.9 before); in 32-bit mode 333 x 768 x 768 9.5 us (31.6 with the fp32 instruction).
+template <typename AT, int NP, int TM, int TN, int AHEAD>
+__global__ __launch_bounds__(256, 2) void lm_deep_kernel(const LinArgs p) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, BK = 32;
+    __shared__ float part[4][TM * TN * 16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, kh = lane >> 5;
+    TileAt t;
+    if (!find_tile(p, BM, BN, t)) return;
+    const AT* a_src[TM];
+    const bf16_t* b_src[TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a_src[i] = a_row<AT>(p, min(t.m0 + 32 * i + r, t.m_end - 1));
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b_src[j] = t.B + (long long)min(t.n0 + 32 * j + r, p.N - 1) * p.ldb;
+    const int kq = ((p.K + 4 * BK - 1) / (4 * BK)) * BK;
+    const int k_lo = wave * kq, k_hi = min(p.K, k_lo + kq);
+
+    Act8<AT> a_reg[AHEAD][TM][2];
+    u32x4 b_reg[AHEAD][TN][2];
+    auto fetch = [&](auto s, int k0) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int kw = k0 + 16 * kh + 8 * h, k = min(kw, p.K - 8);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a_reg[s][i][h].load(a_src[i], k);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b_reg[s][j][h] = load_b8(b_src[j], k);
+        }
+    };
+    f32x16 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.0f;
+    auto multiply = [&](auto s, int k0) {
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bool in = k0 + 16 * kh + 8 * h < p.K;  // (beyond K the clamped load brought columns that were there before)
+            bf16x8 bf[TN];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) bf[j] = __builtin_bit_cast(bf16x8, in ? b_reg[s][j][h] : u32x4{0u, 0u, 0u, 0u});
+            Planes8<NP> pl[TM];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {
+                Act8<AT> a = a_reg[s][i][h];
+                if (!in) a.clear();
+                pl[i] = a.template planes<NP>();
+            }
+#pragma unroll
+            for (int q = NP - 1; q >= 0; --q)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, pl[i].v[q]), bf[j], acc[i][j], 0, 0, 0);
+        }
+    };
+    unroll<AHEAD>([&](auto i) {
+        if (k_lo + i * BK < k_hi) fetch(i, k_lo + i * BK);
+    });
+    for (int k0 = k_lo; k0 < k_hi; k0 += AHEAD * BK)
+        unroll<AHEAD>([&](auto i) {
+            const int k = k0 + i * BK;
+            if (k < k_hi) {
+                multiply(i, k);
+                if (k + AHEAD * BK < k_hi) fetch(i, k + AHEAD * BK);
+            }
+        });
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) part[wave][(i * TN + j) * 16 + e][lane] = acc[i][j][e];
+    __syncthreads();
+    constexpr int SHARE = TM * TN * 4;  // accumulator elements this wave sums and stores
+#pragma unroll
+    for (int x = 0; x < SHARE; ++x) {
+        const int el = wave * SHARE + x, e = el & 15, ij = el >> 4, i = ij / TN, j = ij % TN;
+        const float v = (part[0][el][lane] + part[1][el][lane]) + (part[2][el][lane] + part[3][el][lane]);
+        const int n = t.n0 + 32 * j + r, m = t.m0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+        if (n < p.N && m < t.m_end) put(p, m, n, v);
+    }
+}
+
 template <bool F32>
 struct Tile {
     static constexpr int BK = F32 ? 16 : 32;
@@ -364,11 +739,12 @@ struct Tile {
     typedef typename std::conditional<F32, float, bf16_t>::type elem;
 };
 
-template <bool F32, int WT>  // WT x WT MFMA tiles of 32 x 32 per wave; workgroup tile = 64 WT squared
+// Operands that 16-byte loads cannot take (odd leading dimensions, K no multiple of 8): 64 x 64 tiles, one buffer, a value at a time.
+template <bool F32>
 __global__ __launch_bounds__(256) void lm_gemm_kernel(const LinArgs p) {
     typedef Tile<F32> T;
     typedef typename T::elem elem;
-    constexpr int BM = 64 * WT, BN = 64 * WT, BK = T::BK, LK = T::LDS_K;
+    constexpr int WT = 1, BM = 64 * WT, BN = 64 * WT, BK = T::BK, LK = T::LDS_K;
     __shared__ __attribute__((aligned(16))) elem As[BM * LK];
     __shared__ __attribute__((aligned(16))) elem Bs[BN * LK];
 
@@ -568,6 +944,7 @@ LinArgs make_args(const Linear& L) {
     p.a_div = L.a_div; p.act = L.act; p.n_groups = L.grp_off ? L.n_groups : 0; p.a_glu = L.a_glu;
     p.act_a = L.act_a; p.act_b = L.act_b; p.bias = L.bias; p.z_limit = L.z_limit; p.glu_kind = L.glu_kind; p.glu_limit = L.glu_limit; p.glu_scale = L.glu_scale;
     p.glu_gate_col = L.glu_gate_col;
+    p.A16 = L.A16; p.C16 = L.C16;
     p.a_poly = L.a_poly;
     p.poly_eps = L.poly_eps;
     p.a_vec = ((reinterpret_cast<uintptr_t>(L.A) & 15) == 0 && L.lda % 4 == 0 && L.a_zoff % 4 == 0) ? 1 : 0;
@@ -576,9 +953,44 @@ LinArgs make_args(const Linear& L) {
 }
 }  // namespace
 
+namespace {
+template <typename AT, int NP>
+int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
+    auto tiles = [&](int bm, int bn) { return (long long)((L.N + bn - 1) / bn) * ((L.M + bm - 1) / bm + (L.grp_off ? L.n_groups : 0)); };
+    int force = 0;  // 128, 64 or 32: that form at any size (tests run small ragged shapes through all of them)
+    if (const char* e = getenv("ZGPT2_LM_GEMM_TILE")) force = atoi(e);
+    auto grid = [&](int bm, int bn) { return dim3((unsigned)tiles(bm, bn), 1, L.nz); };
+    ZG_REQUIRE(tiles(32, 32) < (1LL << 31) && L.nz <= 65535, ZG_ERR_UNSUPPORTED, "linear: %d rows in %d batches exceed the grid", L.M, L.nz);
+    // Which form (us per launch, both sides measured on an MI355X):
+    //   * 320 tiles of 128 x 128 and more fill the chip: 8184 x 1024 x 1024 35.6 against 44.4 with 64 x 64 tiles, 1791 x 3072 x 768 (336
+    //     tiles) 28.0 against 29.3; below, the smaller tiles do: 1791 x 768 x 1536 (84 tiles) 18.1 against 28.2.
+    //   * up to 256 tiles of 32 x 32 a compute unit has one of them at most: 37 x 2304 x 768 6.5 against 7.5 with 64 x 64 tiles; with
+    //     more, their rows are fetched too often: 333 x 2304 x 768 (792) 19.3 against 8.3.
+    //   * three terms are bound by their products rather than by the staging: 333 x 768 x 768 9.5 in 32 x 64 tiles with K split
+    //     against 14.4 staged, 333 x 2304 x 768 (396 tiles) 15.2 against 15.7; from there on staged 64 x 128 tiles:
+    //     333 x 3072 x 768 18.3 against 22.2, 1023 x 2304 x 768 26.5 against 32.
+    const bool deep = force ? force == 32 : tiles(32, 32) <= 256;
+    const char* which;
+#define ZG_TILES(kernel, TM, TN, AHEAD, bm, bn) (kernel<AT, NP, TM, TN, AHEAD><<<grid(bm, bn), 256, 0, s>>>(p), which = #kernel "<" #TM ", " #TN ">")
+    if (deep) ZG_TILES(lm_deep_kernel, 1, 1, 3, 32, 32);
+    else if constexpr (NP == 1) {
+        if (force ? force == 128 : tiles(128, 128) >= 320) ZG_TILES(lm_wide_kernel, 2, 2, 1, 128, 128);
+        else ZG_TILES(lm_wide_kernel, 1, 1, 2, 64, 64);
+    } else {
+        if (force ? force == 128 : tiles(32, 64) > 512) ZG_TILES(lm_wide_kernel, 1, 2, 2, 64, 128);
+        else ZG_TILES(lm_deep_kernel, 1, 2, 3, 32, 64);
+    }
+#undef ZG_TILES
+    note_kernel("%s x %d", which, NP);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+}  // namespace
+
 int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     if (L.M <= 0 || L.N <= 0 || L.nz <= 0) return ZG_OK;
-    ZG_REQUIRE(L.K > 0 && L.A && L.B && L.C, ZG_ERR_ARG, "linear: empty operand");
+    const bool tiled = L.grp_off || L.M > kGemvMaxRows;
+    ZG_REQUIRE(L.K > 0 && L.B && (tiled ? (L.A || (L.A16 && !f32)) && (L.C || L.C16) : L.A && L.C && !L.C16), ZG_ERR_ARG, "linear: empty operand");
     ZG_REQUIRE(L.a_div >= 1, ZG_ERR_ARG, "linear: a_div %d", L.a_div);
     ZG_REQUIRE(!L.a_poly || (L.M <= kPolyMaxRows && L.a_glu == 0 && !L.grp_off), ZG_ERR_ARG, "linear: the polynomial activation on load is for %d rows at most",
                kPolyMaxRows);
@@ -609,22 +1021,21 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     ZG_REQUIRE(L.a_glu == 0, ZG_ERR_ARG, "linear: the gated activation on load is for steps of few rows");
     ZG_REQUIRE(!(L.z_group && L.grp_off), ZG_ERR_ARG, "linear: a matrix per batch and row groups exclude each other");
     ZG_REQUIRE(L.z_limit == 0x7fffffff, ZG_ERR_ARG, "linear: skipped batches are for steps of few rows");
-    // 64 x 64 tiles.  The 128 x 128 form of the same kernel measured slower at every size tried (a prompt pass of 8 x 1023
-    // tokens at width 1600: 143 against 127 ms; width 768: 14.6 against 12.9 ms) and is kept behind ZGPT2_LM_GEMM_TILE=128 only
-    // (tests run ragged shapes through it).
-    bool big = false;
-    if (const char* e = getenv("ZGPT2_LM_GEMM_TILE")) big = atoi(e) == 128;
-    const int b = big ? 128 : 64;
-    const dim3 grid((L.N + b - 1) / b, (L.M + b - 1) / b + (L.grp_off ? L.n_groups : 0), L.nz);
-    ZG_REQUIRE(grid.y <= 65535 && grid.z <= 65535, ZG_ERR_UNSUPPORTED, "linear: %d rows in %d batches exceed the grid", L.M, L.nz);
-    if (f32) {
-        if (big) lm_gemm_kernel<true, 2><<<grid, 256, 0, s>>>(p);
-        else lm_gemm_kernel<true, 1><<<grid, 256, 0, s>>>(p);
-    } else {
-        if (big) lm_gemm_kernel<false, 2><<<grid, 256, 0, s>>>(p);
-        else lm_gemm_kernel<false, 1><<<grid, 256, 0, s>>>(p);
+    const bool rounded = L.A16 && !f32;
+    const bool a_vec = rounded ? (reinterpret_cast<uintptr_t>(L.A16) & 15) == 0 && L.lda % 8 == 0 && L.a_zoff % 8 == 0 : p.a_vec != 0;
+    // (32-bit products of a few columns exist in toy models only.  There the last bits of a sum that cancels almost entirely can decide a
+    // row, and they stay what the fp32 instruction makes them: 5.5 us against 3.4 at K = 64.)
+    const bool toy = f32 && L.K < 128 && L.nz == 1;
+    if (a_vec && p.b_vec && L.K % 8 == 0 && !L.z_group && !toy) {
+        if (f32) return launch_tiles<float, 3>(L, p, s);
+        return rounded ? launch_tiles<bf16_t, 1>(L, p, s) : launch_tiles<float, 1>(L, p, s);
     }
-    note_kernel("lm_gemm_kernel<%s, %d>", f32 ? "true" : "false", big ? 2 : 1);
+    ZG_REQUIRE(L.A && L.C && !L.C16, ZG_ERR_ARG, "linear: rounded rows need 16-byte pieces");
+    const dim3 grid((L.N + 63) / 64, (L.M + 63) / 64 + (L.grp_off ? L.n_groups : 0), L.nz);
+    ZG_REQUIRE(grid.y <= 65535 && grid.z <= 65535, ZG_ERR_UNSUPPORTED, "linear: %d rows in %d batches exceed the grid", L.M, L.nz);
+    if (f32) lm_gemm_kernel<true><<<grid, 256, 0, s>>>(p);
+    else lm_gemm_kernel<false><<<grid, 256, 0, s>>>(p);
+    note_kernel("lm_gemm_kernel<%s>", f32 ? "true" : "false");
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
