@@ -46,3 +46,27 @@ def test_values_that_are_not_finite(dtype, bad):
     m.close()
     assert np.isnan(got[25:]).any(axis=1).all()
     tl.assert_close(got[:25], ref[:25], dtype, (bad, dtype))
+
+
+@pytest.mark.parametrize("kv_rank,rot_dim", [(40, 6), (64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])
+def test_latent_tiles(kv_rank, rot_dim):
+    """Latent attention of portions with every tile size (rows of no whole number of pieces among them): three sequences whose portions
+    end around block and tile edges, behind histories of other lengths; five heads (the last group of four is one)."""
+    cfg = tl.config([tl.latent_layer(heads=5, dim=16, vdim=16, rot_dim=rot_dim, rot_dims=rot_dim, kv_rank=kv_rank, q_rank=40, mlp=tl.dense_mlp(ff=96))],
+                    vocab=203, width=64)
+    w = tl.weights(cfg, seed=kv_rank)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(80 + b, n, cfg["vocab"]) for b, n in enumerate((150, 97, 66))]
+    refs = [oracle.forward(t)[0] for t in toks]
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="bfloat16", max_tokens=512, max_seqs=3)
+    m.load_weights(w)
+    seqs = [m.open() for _ in toks]
+    cuts = [(33, 64, 150), (1, 96, 97), (31, 33, 66)]
+    lo = [0, 0, 0]
+    for step in range(3):
+        hi = [c[step] for c in cuts]
+        got = m.step([(s, t[a:b], list(range(b - a))) for s, t, a, b in zip(seqs, toks, lo, hi)])
+        want = np.concatenate([r[a:b] for r, a, b in zip(refs, lo, hi)])
+        tl.assert_close(got, want, "bfloat16", (kv_rank, step))
+        lo = hi
+    m.close()

@@ -241,6 +241,8 @@ struct zg_lm {
     size_t trace_floats = 0;
     float last_step_ms = 0.0f, last_decode_ms = 0.0f;
     bool use_graph = true;
+    bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
+    size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
     int step_keys = 0;  // positions the longest sequence of the running portion has reached (what its rows can see at most)
     // by rows of the step (one per entry) and, where whole-context attention splits a row's keys into shares, by the length bucket
     // of the longest sequence (512, 1024, ... tokens): a share then holds a few dozen keys at any length
@@ -327,7 +329,7 @@ void layout(zg_lm* g, Bump& b) {
     else vec("final.norm", g->final_norm, W, g->side ? INIT_PLAIN : INIT_OFFSET);
     if (g->cfg.flags & ZG_LM_SINUSOID_POSITIONS) g->pos_freq = b.take<float>((W + 1) / 2);
     size_t max_t = 1, max_win = 0, max_win_few = 0, max_vf = 0;
-    size_t max_proj = 1, max_qr = 1, max_q = 1, max_qa = 1, max_ctx = 1, max_o = 1, max_ff = 1, max_assign = 1, max_gu = 1, max_hb = 1, max_e = 1, max_att_part = 0, max_scan = 0;
+    size_t max_proj = 1, max_qr = 1, max_q = 1, max_qa = 1, max_ctx = 1, max_o = 1, max_ff = 1, max_assign = 1, max_gu = 1, max_hb = 1, max_e = 1, max_att_part = 0, max_scan = 0, max_tile = 0;
     for (size_t i = 0; i < g->layers.size(); ++i) {
         LayerW& L = g->layers[i];
         const zg_lm_layer& d = L.d;
@@ -584,6 +586,7 @@ void layout(zg_lm* g, Bump& b) {
             max_qa = std::max(max_qa, H * (KR + R));
             max_ctx = std::max(max_ctx, H * KR);
             max_att_part = std::max(max_att_part, H * (KR + 2));
+            if (!g->f32) max_tile = std::max(max_tile, latent_tile_elems((int)KR, (int)R));
             max_o = std::max(max_o, HV);
         }
         if (d.ff != ZG_LM_FF_NONE && tn) {
@@ -731,6 +734,8 @@ void layout(zg_lm* g, Bump& b) {
     g->scan_ws = b.take<float>(std::max<size_t>(1, g->scan_ws_floats));
     g->attn_ws_floats = (size_t)kGemvMaxRows * kAttnSplits * max_att_part;
     g->attn_ws = b.take<float>(std::max<size_t>(1, g->attn_ws_floats));
+    g->key_tile_elems = ((size_t)g->n_pages * g->P / 32 + NS) * max_tile;  // every cached token, a partly filled tile per sequence
+    g->key_tiles = b.take<bf16_t>(std::max<size_t>(1, g->key_tile_elems));
     // scores and partial sums of the split windowed attention: up to 2 GiB for a whole portion, else for steps of few rows only
     // (longer steps of such a model then take the general kernel)
     if (max_win > ((size_t)1 << 29)) max_win = 0;
@@ -1249,7 +1254,8 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             bool tiled = false;
             if (!f32 && !few)
                 ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
-                                                     g->max_pages, g->P, ps.cache, s, &tiled, gate, LD, L.sink));
+                                                     g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
+                                                     L.sink));
             if (!tiled)
                 ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,
                                                g->attn_ws, g->attn_ws_floats, s, gate, LD, L.sink));
@@ -1529,9 +1535,11 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
     std::vector<std::pair<int, size_t>> wants;  // (row of the portion, output row)
     int r = 0;
     g->step_keys = 0;
+    g->step_key_tiles = 0;
     for (int e = 0; e < n_ent; ++e) {
         const Piece& pc = pieces[e];
         g->step_keys = std::max(g->step_keys, pc.pos0 + pc.n);
+        g->step_key_tiles += (pc.pos0 + pc.n + 31) / 32;
         ent_start[e] = r;
         ent_len[e] = pc.n;
         ent_slot[e] = pc.slot;

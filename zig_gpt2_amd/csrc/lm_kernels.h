@@ -245,11 +245,15 @@ int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, i
                             const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);
 
 // The same for prompt portions on the matrix cores (bf16 operands, fp32 scores / softmax / accumulation): 32 queries of one entry
-// and four heads per workgroup.  *taken = false when the latent is larger than the kernel's tiles hold (nothing launched).
+// and four heads per workgroup, over the entries' cached rows laid out as bf16 tiles of 32 keys by a launch in front of it.
+// ws: room for the tiles, n_tiles = sum over the entries of ceil((position of its last row + 1) / 32), of latent_tile_elems elements each;
+// max_keys: the largest of those position counts.  *taken = false when the latent is larger than the kernel's tiles hold or ws is too
+// small (nothing launched).
+size_t latent_tile_elems(int KR, int R);
 int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
                                   const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
-                                  const float* cache, hipStream_t s, bool* taken, const float* gate = nullptr, int ldg = 0,
-                                  const float* sink = nullptr);
+                                  const float* cache, bf16_t* ws, size_t ws_elems, size_t n_tiles, int max_keys, hipStream_t s, bool* taken,
+                                  const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);
 
 // ------------------------------------------------------------------------------------------------ input convolution of decode rows, residual sum
 // Steps of one row per entry: [x += x0] or [x += norm(y) * (1 + wb), y = yl or the mean of the two normed branches yl, yr with

@@ -943,60 +943,166 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, 
     }
 }
 
-// Prompt portions in bf16 mode: the same attention on the matrix cores.  A workgroup takes 32 consecutive queries of one entry
-// and four heads (one per wave) — the heads share the cached rows, so a tile of 32 keys is staged in the LDS once for all four:
-// as bf16 rows [key][dim] for the scores and, its latent part, transposed [dim][key] for the weighted sum.  Both products are
-// computed transposed (S^T = K Q^T, O^T = C^T P^T): a lane's column is a query, so the running maximum and sum are per-lane
-// values and the probabilities a lane computed are exactly the eight per k-step it has to feed back (in a key order that the
-// transposed latent tile is read in as well: keys {0-3, 8-11} from the lower half-wave, {4-7, 12-15} from the upper one).
-// Scores, softmax and both accumulations are fp32; q, cache rows and probabilities enter the products as bf16.
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
+typedef __attribute__((ext_vector_type(4))) short s16x4;
 
-template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
-__global__ __launch_bounds__(256) void latent_attention_mfma_kernel(const float* qa, float* ctx, int H, int KR, int R, float scale,
-                                                                    const int* ent_start, const int* ent_len, const int* ent_slot, int n_entries,
-                                                                    const int* row_pos, const int* page_table, int max_pages, int page_tokens,
-                                                                    const float* cache, const float* gate, int ldg, const float* sink) {
-    constexpr int DTp = NKS * 16, KS_LD = DTp + 8, VT_LD = 40;
-    __shared__ __attribute__((aligned(16))) bf16_t Ks[32 * KS_LD];
-    __shared__ __attribute__((aligned(16))) bf16_t Vt[NT * 32 * VT_LD];
-    int id = blockIdx.x, e = 0, qb = 0;
-    for (; e < n_entries; ++e) {
-        const int nb = (ent_len[e] + 31) / 32;
-        if (id < nb) {
-            qb = id;
-            break;
+// Tiles of 32 cached rows as the matrix cores read them: bf16, rows of 16 NKS dimensions (zeros behind the last one) padded so that
+// four consecutive rows start 16 or 48 banks apart, 16-byte chunks swizzled by the row's second bit pair — then a fragment read of
+// 16 rows, and a transposed read of four, touch every bank once.
+template <int NKS>
+struct KeyTile {
+    static constexpr int DT = NKS * 16, LD = DT + ((DT / 2) % 64 == 0 ? 32 : 0);  // elements per row
+    static constexpr int BYTES = 32 * LD * 2, PIECES = BYTES / 1024;
+    static_assert(BYTES % 1024 == 0 && LD % 32 == 0, "a tile is whole 1 KB pieces");
+};
+constexpr int kLog2eBits = 0x3fb8aa3b;  // log2(e)
+
+// Entries of a step, one per lane (64 at a time): the rows of entry e cut into blocks of 32 queries, its cached rows (this step's
+// included) into tiles of 32 keys.  Finds the entry of query block `id` and the key tiles of the entries in front of it.
+struct EntryAt {
+    int e, block, first_tile;
+};
+__device__ __forceinline__ bool find_entry(int id, const int* ent_start, const int* ent_len, int n_entries, const int* row_pos, EntryAt& at) {
+    const int lane = threadIdx.x & 63;
+    int tiles_before = 0;
+    for (int e0 = 0; e0 < n_entries; e0 += 64) {
+        const int e = min(e0 + lane, n_entries - 1);
+        const int len = e0 + lane < n_entries ? ent_len[e] : 0;
+        const int blocks = (len + 31) / 32, tiles = len > 0 ? (row_pos[ent_start[e] + len - 1] + 32) / 32 : 0;
+        int b = blocks, t = tiles;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int ob = __shfl_up(b, d, 64), ot = __shfl_up(t, d, 64);
+            if (lane >= d) {
+                b += ob;
+                t += ot;
+            }
         }
-        id -= nb;
+        const unsigned long long past = __ballot(id < b);
+        if (past) {
+            const int l = __builtin_ctzll(past);
+            at.e = e0 + l;
+            at.block = id - __builtin_amdgcn_readlane(b - blocks, l);
+            at.first_tile = tiles_before + __builtin_amdgcn_readlane(t - tiles, l);
+            return true;
+        }
+        id -= __builtin_amdgcn_readlane(b, 63);
+        tiles_before += __builtin_amdgcn_readlane(t, 63);
     }
-    if (e >= n_entries) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, hf = lane >> 5;
+    return false;
+}
+
+// The cached rows of every entry of the step as key tiles, back to back in entry order.  Each tile is read by every query block
+// behind it and by all heads: converting it once (8 x 1023 rows of 288 values: 9 us) took the conversion, the page table and the
+// 4-byte loads out of loops that ran 16 times over every tile.
+template <int NKS>
+__global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, int DT, const int* ent_start, const int* ent_len, const int* ent_slot,
+                                                           int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
+                                                           bf16_t* tiles) {
+    typedef KeyTile<NKS> T;
+    const int e = blockIdx.y, lane = threadIdx.x & 63;
+    const int len = ent_len[e];
+    if (len <= 0) return;
+    const int n_keys = row_pos[ent_start[e] + len - 1] + 1;
+    if ((int)blockIdx.x * 32 >= n_keys) return;
+    int first = 0;  // tiles of the entries in front
+    for (int e0 = 0; e0 < e; e0 += 64) {
+        const int o = e0 + lane, ol = o < e ? ent_len[o] : 0;
+        int t = ol > 0 ? (row_pos[ent_start[o] + ol - 1] + 32) / 32 : 0;
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) t += __shfl_xor(t, d, 64);
+        first += t;
+    }
+    bf16_t* out = tiles + (size_t)(first + blockIdx.x) * (T::BYTES / 2);
+    const int* pt = page_table + (size_t)ent_slot[e] * max_pages;
+    const bool vec = DT % 4 == 0 && (reinterpret_cast<uintptr_t>(cache) & 15) == 0;
+    for (int idx = threadIdx.x; idx < 32 * (T::LD / 8); idx += 256) {
+        const int key = idx / (T::LD / 8), c = idx % (T::LD / 8), kpos = blockIdx.x * 32 + key;
+        float v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = 0.0f;
+        if (kpos < n_keys) {
+            const float* row = cache + ((size_t)pt[kpos / page_tokens] * page_tokens + kpos % page_tokens) * DT;
+            if (vec && c * 8 + 8 <= DT) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(row + c * 8), b = *reinterpret_cast<const f32x4*>(row + c * 8 + 4);
+                v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (c * 8 + u < DT) v[u] = row[c * 8 + u];
+            }
+        }
+        *reinterpret_cast<u32x4*>(out + key * T::LD + (c ^ ((key >> 2) & 3)) * 8) =
+            u32x4{cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]), cvt_pk_bf16(v[4], v[5]), cvt_pk_bf16(v[6], v[7])};
+    }
+}
+
+// Prompt portions in bf16 mode: the same attention on the matrix cores.  A workgroup takes 32 consecutive queries of one entry and
+// four heads (one per wave), which share the tiles of 32 keys that arrive by DMA in two LDS buffers, one barrier per tile.  Both
+// products are computed transposed (S^T = K Q^T, O^T = C^T P^T): a lane's column is a query, so the running maximum and sum are
+// per-lane values and the probabilities a lane computed are exactly the eight per k-step it has to feed back (keys {0-3, 8-11} from
+// the lower half-wave, {4-7, 12-15} from the upper one); the latent part is read back transposed from the same rows the scores used
+// (ds_read_b64_tr_b16).  Scores, softmax and both accumulations are fp32; q, cache rows and probabilities enter the products as bf16.
+// Bound by the matrix cores and the LDS together: a fragment of keys (1 KB) serves one product (32 cycles), so the four SIMDs of a
+// compute unit ask the LDS for its whole 128 B per clock; two workgroups per compute unit hide the softmax of one under the
+// products of the other (hence 256 registers a lane: 72 of queries, 128 of sums).  The blocks with the most keys are dealt first.
+// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 132 us and 9 for the tiles (73 GFLOP: 520 TFLOP/s); 827 us when every workgroup
+// converted and transposed its own tiles behind three barriers.
+template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
+__global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, float* ctx, int H, int KR, int R, float scale,
+                                                                       const int* ent_start, const int* ent_len, int n_entries, const int* row_pos,
+                                                                       const bf16_t* tiles, const float* gate, int ldg, const float* sink) {
+    typedef KeyTile<NKS> T;
+    static_assert(NT * 32 <= T::DT, "the latent part lies inside the rows");
+    __shared__ __attribute__((aligned(1024))) char Ks[2][T::BYTES];
+    EntryAt at;
+    if (!find_entry(gridDim.x - 1 - blockIdx.x, ent_start, ent_len, n_entries, row_pos, at)) return;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y * 4 + wave;
     const bool head_ok = h < H;
-    const int m_first = ent_start[e] + qb * 32, nq = min(32, ent_len[e] - qb * 32);
+    const int m_first = ent_start[at.e] + at.block * 32, nq = min(32, ent_len[at.e] - at.block * 32);
     const int pos_first = row_pos[m_first], qpos = pos_first + r, DT = KR + R;
-    const bool q_ok = r < nq;
-    const int n_keys = pos_first + nq;
-    const int* pt = page_table + (size_t)ent_slot[e] * max_pages;
+    const int n_tiles = (pos_first + nq + 31) / 32;
+    const char* src = reinterpret_cast<const char*>(tiles) + (size_t)at.first_tile * T::BYTES + lane * 16;
 
+    auto request = [&](int kt, int buf) {
+        const char* g = src + (size_t)kt * T::BYTES;
+#pragma unroll
+        for (int pc = 0; pc < (T::PIECES + 3) / 4; ++pc) {
+            const int i = wave + 4 * pc;
+            if (i < T::PIECES)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(g + i * 1024),
+                                                 (__attribute__((address_space(3))) void*)(Ks[buf] + i * 1024), 16, 0, 0);
+        }
+    };
+    request(0, 0);
     bf16x8 qf[NKS];
     {
-        const float* qrow = qa + ((size_t)(m_first + (q_ok ? r : 0)) * H + (head_ok ? h : 0)) * DT;
+        const float* qrow = qa + ((size_t)(m_first + (r < nq ? r : 0)) * H + (head_ok ? h : 0)) * DT;  // (beyond the block: some valid row, never stored)
+        auto round8 = [](const f32x4& a, const f32x4& b) {
+            return __builtin_bit_cast(bf16x8, u32x4{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w), cvt_pk_bf16(b.x, b.y), cvt_pk_bf16(b.z, b.w)});
+        };
+        const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (DT % 4 == 0 && (reinterpret_cast<uintptr_t>(qa) & 15) == 0) {
+            f32x4 q4[2 * NKS];
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            float v[8];
+            for (int i = 0; i < 2 * NKS; ++i) q4[i] = *reinterpret_cast<const f32x4*>(qrow + min((i >> 1) * 16 + 8 * hf + 4 * (i & 1), DT - 4));
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int d = ks * 16 + 8 * hf + u;
-                v[u] = (head_ok && q_ok && d < DT) ? qrow[d] : 0.0f;
+            for (int ks = 0; ks < NKS; ++ks) {
+                const int d = ks * 16 + 8 * hf;
+                qf[ks] = round8(d + 4 <= DT ? q4[2 * ks] : zero, d + 8 <= DT ? q4[2 * ks + 1] : zero);
             }
-            u32x4 pk;
-            pk.x = cvt_pk_bf16(v[0], v[1]);
-            pk.y = cvt_pk_bf16(v[2], v[3]);
-            pk.z = cvt_pk_bf16(v[4], v[5]);
-            pk.w = cvt_pk_bf16(v[6], v[7]);
-            qf[ks] = __builtin_bit_cast(bf16x8, pk);
+        } else {
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                f32x4 ab[2] = {zero, zero};
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (ks * 16 + 8 * hf + u < DT) ab[u >> 2][u & 3] = qrow[ks * 16 + 8 * hf + u];
+                qf[ks] = round8(ab[0], ab[1]);
+            }
         }
     }
     f32x16 o[NT];
@@ -1004,120 +1110,114 @@ __global__ __launch_bounds__(256) void latent_attention_mfma_kernel(const float*
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int i = 0; i < 16; ++i) o[t][i] = 0.0f;
-    float mx = -INFINITY, lsum = 0.0f;
-    const bool vec = (DT % 4 == 0) && ((reinterpret_cast<uintptr_t>(cache) & 15) == 0);
+    float mx = -INFINITY, lsum = 0.0f;  // maximum in units of log2
+    const float to_log2 = scale * __uint_as_float(kLog2eBits);
 
-    // a tile's rows travel global -> registers -> LDS; the registers of tile kt + 1 are filled while tile kt is multiplied
-    constexpr int ITEMS = 32 * (DTp / 4) / 256;  // float4 pieces per thread and tile (NKS is even)
-    f32x4 stage[ITEMS];
-    auto fetch = [&](int kt) {
+    // byte offsets inside a tile: this lane's key row for the scores (even and odd k-steps), its rows for the transposed reads
+    const int swz = (r >> 2) & 3;
+    const int k_even = r * T::LD * 2 + ((0 + hf) ^ swz) * 16, k_odd = r * T::LD * 2 + ((2 + hf) ^ swz) * 16;
+    const int i16 = lane & 15, G = (lane >> 4) & 1, vc = 2 * G + ((i16 & 3) >> 1);
+    const int v_lo = (4 * hf + (i16 >> 2)) * T::LD * 2 + ((vc ^ hf) * 16) + (i16 & 1) * 8;
+    const int v_hi = (8 + 4 * hf + (i16 >> 2)) * T::LD * 2 + ((vc ^ (hf + 2)) * 16) + (i16 & 1) * 8;
+    typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
+
+    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces have landed
+    __syncthreads();
+    for (int kt = 0; kt < n_tiles; ++kt) {
+        const char* K = Ks[kt & 1];
+        if (kt + 1 < n_tiles) request(kt + 1, (kt + 1) & 1);
+        if (head_ok) {
+            // fragments are requested AHEAD products before they are used (left alone, the compiler pairs each request with its product and
+            // waits out the LDS latency 34 times per tile)
+            constexpr int AHEAD = 5;
+            auto key_part = [&](int ks) { return *reinterpret_cast<const u32x4*>(K + ((ks & 1) ? k_odd : k_even) + (ks >> 1) * 64); };
+            u32x4 kf[AHEAD];
 #pragma unroll
-        for (int it = 0; it < ITEMS; ++it) {
-            const int idx = tid + 256 * it;
-            const int key = idx / (DTp / 4), d4 = (idx % (DTp / 4)) * 4, kpos = kt * 32 + key;
-            f32x4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-            if (kpos < n_keys) {
-                const float* row = cache + ((size_t)pt[kpos / page_tokens] * page_tokens + kpos % page_tokens) * DT;
-                if (vec && d4 + 4 <= DT) {
-                    x = *reinterpret_cast<const f32x4*>(row + d4);
-                } else {
-                    x.x = d4 + 0 < DT ? row[d4 + 0] : 0.0f;
-                    x.y = d4 + 1 < DT ? row[d4 + 1] : 0.0f;
-                    x.z = d4 + 2 < DT ? row[d4 + 2] : 0.0f;
-                    x.w = d4 + 3 < DT ? row[d4 + 3] : 0.0f;
-                }
+            for (int i = 0; i < AHEAD; ++i) kf[i] = key_part(i);
+            __builtin_amdgcn_sched_barrier(0);
+            f32x16 sacc;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) {
+                sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, kf[ks % AHEAD]), qf[ks], sacc, 0, 0, 0);
+                if (ks + AHEAD < NKS) kf[ks % AHEAD] = key_part(ks + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
             }
-            stage[it] = x;
-        }
-    };
-    fetch(0);
-    for (int kt = 0; kt * 32 < n_keys; ++kt) {
-        __syncthreads();  // the previous tile has been consumed
+            float tmax = -INFINITY;
+            if (kt * 32 + 31 > pos_first) {  // some query does not see the whole tile
 #pragma unroll
-        for (int it = 0; it < ITEMS; ++it) {
-            const int idx = tid + 256 * it;
-            const int key = idx / (DTp / 4), d4 = (idx % (DTp / 4)) * 4;
-            u32x2 pk;
-            pk.x = cvt_pk_bf16(stage[it].x, stage[it].y);
-            pk.y = cvt_pk_bf16(stage[it].z, stage[it].w);
-            *reinterpret_cast<u32x2*>(&Ks[key * KS_LD + d4]) = pk;
+                for (int i = 0; i < 16; ++i)
+                    if (kt * 32 + 8 * (i >> 2) + 4 * hf + (i & 3) > qpos) sacc[i] = -INFINITY;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                sacc[i] *= to_log2;
+                tmax = fmaxf(tmax, sacc[i]);
+            }
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+            // The reference point of the exponentials moves only when some query's maximum grew by more than 2^11 (the weights stay far
+            // inside fp32 and bf16 range): the accumulators are rescaled on few tiles instead of on every one.
+            if (__any(tmax > mx + 11.0f)) {  // also the first tile (mx = -inf)
+                const float mn = tmax > mx + 11.0f ? tmax : mx;
+                const float alpha = mx == mn ? 1.0f : __builtin_amdgcn_exp2f(mx - mn);  // mx = -inf, mn finite: 0
+                lsum *= alpha;
+#pragma unroll
+                for (int t = 0; t < NT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) o[t][i] *= alpha;
+                mx = mn;
+            }
+            const float mref = fmaxf(mx, -1e30f);  // (no key seen so far: 2^(-inf) = 0, not NaN)
+            uint32_t pk[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float p0 = __builtin_amdgcn_exp2f(sacc[2 * i] - mref), p1 = __builtin_amdgcn_exp2f(sacc[2 * i + 1] - mref);
+                lsum += p0 + p1;
+                pk[i] = cvt_pk_bf16(p0, p1);
+            }
+            const bf16x8 pf[2] = {__builtin_bit_cast(bf16x8, u32x4{pk[0], pk[1], pk[2], pk[3]}), __builtin_bit_cast(bf16x8, u32x4{pk[4], pk[5], pk[6], pk[7]})};
+            auto value_part = [&](int x) {  // 16 keys x 32 dimensions, transposed
+                const int off = (x / NT) * 16 * T::LD * 2 + (x % NT) * 64;
+                const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(K + v_lo + off));
+                const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(K + v_hi + off));
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            bf16x8 vf[AHEAD];
+#pragma unroll
+            for (int i = 0; i < (AHEAD < 2 * NT ? AHEAD : 2 * NT); ++i) vf[i] = value_part(i);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int x = 0; x < 2 * NT; ++x) {
+                o[x % NT] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[x % AHEAD], pf[x / NT], o[x % NT], 0, 0, 0);
+                if (x + AHEAD < 2 * NT) vf[x % AHEAD] = value_part(x + AHEAD);
+                __builtin_amdgcn_sched_barrier(0);
+            }
         }
+        __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the next tile's pieces
         __syncthreads();
-        if ((kt + 1) * 32 < n_keys) fetch(kt + 1);
-        // the latent part once more, transposed: consecutive lanes take consecutive keys, so the 2-byte stores of a wave fall into
-        // consecutive words (written from the rows above rather than beside them: a lane of the loop above holds four dimensions
-        // of ONE key, and its four stores would all hit the same two banks)
-        for (int idx = tid; idx < 32 * (NT * 8); idx += 256) {
-            const int key = idx & 31, d4 = (idx >> 5) * 4;
-            const u32x2 pk = *reinterpret_cast<const u32x2*>(&Ks[key * KS_LD + d4]);
-            Vt[(d4 + 0) * VT_LD + key] = (bf16_t)(pk.x & 0xFFFFu);
-            Vt[(d4 + 1) * VT_LD + key] = (bf16_t)(pk.x >> 16);
-            Vt[(d4 + 2) * VT_LD + key] = (bf16_t)(pk.y & 0xFFFFu);
-            Vt[(d4 + 3) * VT_LD + key] = (bf16_t)(pk.y >> 16);
-        }
-        __syncthreads();
-        if (!head_ok) continue;
-        f32x16 sacc;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) sacc[i] = 0.0f;
-#pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) {
-            const bf16x8 a = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&Ks[r * KS_LD + ks * 16 + 8 * hf]));
-            sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[ks], sacc, 0, 0, 0);
-        }
-        float sv[16], tmax = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int key = kt * 32 + 8 * (i >> 2) + 4 * hf + (i & 3);
-            sv[i] = (q_ok && key <= qpos) ? sacc[i] * scale : -INFINITY;
-            tmax = fmaxf(tmax, sv[i]);
-        }
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-        // The reference point of the exponentials moves only when some query's maximum grew by more than 8 (the weights then
-        // reach e^8 at most, far inside fp32 and bf16 range): the accumulators are rescaled on few tiles instead of on every one.
-        const bool grow = tmax > mx + 8.0f;  // also the first tile of a query (mx = -inf)
-        float psum = 0.0f, pv[16];
-        if (__any(grow)) {
-            const float mn = grow ? tmax : mx;
-            const float alpha = (mn == -INFINITY || mx == mn) ? 1.0f : __expf(mx - mn);  // mx = -inf, mn finite: 0
-            lsum *= alpha;
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int i = 0; i < 16; ++i) o[t][i] *= alpha;
-            mx = mn;
-        }
-        const bool none = mx == -INFINITY;  // a query row beyond the entry: nothing to weigh
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            pv[i] = none ? 0.0f : __expf(sv[i] - mx);
-            psum += pv[i];
-        }
-        lsum += psum;
-        u32x4 p0, p1;
-        p0.x = cvt_pk_bf16(pv[0], pv[1]); p0.y = cvt_pk_bf16(pv[2], pv[3]); p0.z = cvt_pk_bf16(pv[4], pv[5]); p0.w = cvt_pk_bf16(pv[6], pv[7]);
-        p1.x = cvt_pk_bf16(pv[8], pv[9]); p1.y = cvt_pk_bf16(pv[10], pv[11]); p1.z = cvt_pk_bf16(pv[12], pv[13]); p1.w = cvt_pk_bf16(pv[14], pv[15]);
-        const bf16x8 pf0 = __builtin_bit_cast(bf16x8, p0), pf1 = __builtin_bit_cast(bf16x8, p1);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const bf16_t* vrow = &Vt[(t * 32 + r) * VT_LD + 4 * hf];
-            const u32x2 a0 = *reinterpret_cast<const u32x2*>(vrow), a1 = *reinterpret_cast<const u32x2*>(vrow + 8);
-            const u32x2 b0 = *reinterpret_cast<const u32x2*>(vrow + 16), b1 = *reinterpret_cast<const u32x2*>(vrow + 24);
-            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, (u32x4){a0.x, a0.y, a1.x, a1.y}), pf0, o[t], 0, 0, 0);
-            o[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, (u32x4){b0.x, b0.y, b1.x, b1.y}), pf1, o[t], 0, 0, 0);
-        }
     }
     if (!head_ok) return;
     const float L = lsum + __shfl_xor(lsum, 32, 64);
-    if (!q_ok) return;
+    if (r >= nq) return;
     float* out = ctx + ((size_t)(m_first + r) * H + h) * KR;
-    const float gf = head_gate_f(gate, ldg, (size_t)(m_first + r), h) * (sink ? sink_norm_f(mx, L, sink, h) : 1.0f);
+    const float gf = head_gate_f(gate, ldg, (size_t)(m_first + r), h) * (sink ? sink_norm_f(mx * 0.69314718055994531f, L, sink, h) : 1.0f);
+    const bool vec = KR % 4 == 0 && (reinterpret_cast<uintptr_t>(ctx) & 15) == 0;
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int d = t * 32 + 8 * (i >> 2) + 4 * hf + (i & 3);
-            if (d < KR) out[d] = sink ? o[t][i] * gf : o[t][i] / L * gf;
+        for (int i = 0; i < 16; i += 4) {
+            const int d = t * 32 + 8 * (i >> 2) + 4 * hf;
+            f32x4 v;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = sink ? o[t][i + u] * gf : o[t][i + u] / L * gf;
+            if (vec) {
+                if (d < KR) *reinterpret_cast<f32x4*>(out + d) = v;
+            } else {
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    if (d + u < KR) out[d + u] = v[u];
+            }
         }
 }
 
@@ -1435,21 +1535,36 @@ int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, 
     return ZG_OK;
 }
 
+size_t latent_tile_elems(int KR, int R) {  // elements of a key tile in the launch's workspace, 0: the latent is larger than its tiles hold
+    const int DT = KR + R;
+    if (DT <= 96 && KR <= 64) return KeyTile<6>::BYTES / 2;
+    if (DT <= 160 && KR <= 128) return KeyTile<10>::BYTES / 2;
+    if (DT <= 288 && KR <= 256) return KeyTile<18>::BYTES / 2;
+    if (DT <= 384 && KR <= 320) return KeyTile<24>::BYTES / 2;
+    return 0;
+}
+
 int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
                                   const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
-                                  const float* cache, hipStream_t s, bool* taken, const float* gate, int ldg, const float* sink) {
+                                  const float* cache, bf16_t* ws, size_t ws_elems, size_t n_tiles, int max_keys, hipStream_t s, bool* taken,
+                                  const float* gate, int ldg, const float* sink) {
     *taken = false;
     if (M <= 0 || n_entries <= 0) return ZG_OK;
-    const int DT = KR + R;
-    const dim3 grid((M + 31) / 32 + n_entries, (H + 3) / 4);
-#define ZG_ATT_T(NKS_, NT_)                                                                                                                      \
-    latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, ctx, H, KR, R, scale, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, \
-                                                                 max_pages, page_tokens, cache, gate, ldg, sink)
-    if (DT <= 96 && KR <= 64) ZG_ATT_T(6, 2);
-    else if (DT <= 160 && KR <= 128) ZG_ATT_T(10, 4);
-    else if (DT <= 288 && KR <= 256) ZG_ATT_T(18, 8);
-    else if (DT <= 384 && KR <= 320) ZG_ATT_T(24, 10);
-    else return ZG_OK;  // larger latents: the caller's general kernel
+    const size_t tile = latent_tile_elems(KR, R);
+    if (tile == 0 || !ws || n_tiles * tile > ws_elems || n_entries > 65535) return ZG_OK;  // the caller's general kernel
+    const dim3 cgrid((max_keys + 31) / 32, n_entries), grid((M + 31) / 32 + n_entries, (H + 3) / 4);
+#define ZG_ATT_T(NKS_, NT_)                                                                                                                          \
+    do {                                                                                                                                             \
+        latent_tiles_kernel<NKS_><<<cgrid, 256, 0, s>>>(cache, KR + R, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, max_pages,      \
+                                                        page_tokens, ws);                                                                            \
+        ZG_HIP(hipGetLastError());                                                                                                                   \
+        latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, ctx, H, KR, R, scale, ent_start, ent_len, n_entries, row_pos, ws, gate, ldg, \
+                                                                     sink);                                                                          \
+    } while (0)
+    if (tile == KeyTile<6>::BYTES / 2) ZG_ATT_T(6, 2);
+    else if (tile == KeyTile<10>::BYTES / 2) ZG_ATT_T(10, 4);
+    else if (tile == KeyTile<18>::BYTES / 2) ZG_ATT_T(18, 8);
+    else ZG_ATT_T(24, 10);
 #undef ZG_ATT_T
     ZG_HIP(hipGetLastError());
     *taken = true;
