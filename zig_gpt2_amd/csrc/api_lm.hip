@@ -243,6 +243,7 @@ struct zg_lm {
     bool use_graph = true;
     bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
     size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
+    int step_longest = 0;  // rows of the longest entry of the running portion
     int step_keys = 0;  // positions the longest sequence of the running portion has reached (what its rows can see at most)
     // by rows of the step (one per entry) and, where whole-context attention splits a row's keys into shares, by the length bucket
     // of the longest sequence (512, 1024, ... tokens): a share then holds a few dozen keys at any length
@@ -1111,7 +1112,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             }
             // right: the recurrence on silu(q | k | v), the heads normed together and gated
             ZG_TRY(launch_hgrn2_scan(g->proj + orq, NP, g->o + HV, OC, g->seq_state + ps.rec_off, g->seq_floats, d_estart, d_elen, d_eslot, n_ent, M, HR,
-                                     DR, VR, nullptr, nullptr, g->scan_ws, g->scan_ws_floats, s, L.decay));
+                                     DR, VR, nullptr, nullptr, g->scan_ws, g->scan_ws_floats, g->step_longest, s, L.decay));
             ZG_TRY(launch_norm_gate(g->o + HV, OC, 1, HRV, M, L.rnorm, eps, g->proj + org, NP, s, d.right_scale));
             lin = Linear();  // both output projections at once: [c_l left | c_r right] against [left.o | right.o]
             lin.A = g->o; lin.lda = OC; lin.B = L.ocat; lin.ldb = OC; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = OC;
@@ -1189,7 +1190,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             GlaGate gate;
             gate.z = g->tb; gate.ldz = HD; gate.z_bias = L.a2b; gate.inv_tau = 1.0f / d.tau; gate.q_scale = 1.0f / sqrtf((float)D);
             ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->seq_state + ps.rec_off, g->seq_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
-                                     nullptr, nullptr, g->scan_ws, g->scan_ws_floats, s, nullptr, &gate));
+                                     nullptr, nullptr, g->scan_ws, g->scan_ws_floats, g->step_longest, s, nullptr, &gate));
             ZG_TRY(launch_norm_gate(g->o, HV, H, Vd, M, L.hnorm, eps, g->proj + og, NP, s, 1.0f, true));
             lin = Linear();
             lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
@@ -1221,7 +1222,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             lin.A = hin; lin.lda = W; lin.B = L.qfv; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
-                                     L.fb, L.lower, g->scan_ws, g->scan_ws_floats, s));
+                                     L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
             ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s));
             lin = Linear();
             lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
@@ -1536,9 +1537,11 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
     int r = 0;
     g->step_keys = 0;
     g->step_key_tiles = 0;
+    g->step_longest = 0;
     for (int e = 0; e < n_ent; ++e) {
         const Piece& pc = pieces[e];
         g->step_keys = std::max(g->step_keys, pc.pos0 + pc.n);
+        g->step_longest = std::max(g->step_longest, pc.n);
         g->step_key_tiles += (pc.pos0 + pc.n + 31) / 32;
         ent_start[e] = r;
         ent_len[e] = pc.n;

@@ -141,7 +141,7 @@ int launch_tanh_sum_norm(float* x, const SumParts& y, const float* nb, float mul
 // them:  q <- silu(q);   f <- low + (1 - low) * sigmoid(f + bias)
 // Per entry e (rows ent_start[e] .. + ent_len[e]) and head: S <- diag(f_t) S + (1 - f_t) v_t^T, o_t = S^T q_t, token by token,
 // S = state[ent_slot[e]] ([H][D][V] fp32) read at the start and written back at the end.  out rows [H V], row stride ldo.
-// M: rows of the step.  ws (may be null): workspace for the chunk-parallel form of long steps, (M / 64 + n_entries) * (H D V + H D) floats.
+// M: rows of the step, longest: of its longest entry.  ws (may be null): workspace for the chunk-parallel form of long steps, (M / 64 + n_entries) * (H D V + H D) floats.
 // decay != null: linear attention with one fixed decay per head on the same machinery — proj rows [q (H D) | k (H D) | v (H V)], all
 // three through silu on their way in:  S <- decay[h] S + k_t v_t^T, o_t = S^T q_t   (bias / low unused).
 // gla != null: gated linear attention with a decay per key channel on the same machinery — proj rows [q (H D) | k (H D) | v (H V)]
@@ -155,7 +155,13 @@ struct GlaGate {
 };
 int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start,
                       const int* ent_len, const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low,
-                      float* ws, size_t ws_floats, hipStream_t s, const float* decay = nullptr, const GlaGate* gla = nullptr);
+                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay = nullptr, const GlaGate* gla = nullptr);
+
+// The same for prompt portions in chunks of 64 tokens as fp32 matrix products (lm_scan.hip): HGRN2, or gla != null.  ws as above.
+// *taken = false when the heads are larger than its tiles (D > 128) or ws is too small (nothing launched).
+int launch_gated_chunks(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start, const int* ent_len,
+                        const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low, float* ws, size_t ws_floats,
+                        const GlaGate* gla, hipStream_t s, bool* taken);
 
 // The carry of a chunked recurrence: wsB [chunk][H][D][V] holds every chunk's end state from zero and receives its true start state,
 // wsA [chunk][H][a_rows] the chunk's decay (a_rows D: per row of the state, 1: per head); the slot's state moves on.

@@ -1431,7 +1431,7 @@ int launch_state_carry(float* state, size_t slot_stride, const int* ent_len, con
 
 int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start,
                       const int* ent_len, const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low,
-                      float* ws, size_t ws_floats, hipStream_t s, const float* decay, const GlaGate* gla) {
+                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay, const GlaGate* gla) {
     if (n_entries <= 0) return ZG_OK;
     ZG_REQUIRE(!gla || (gla->z && gla->z_bias && !decay), ZG_ERR_ARG, "gated linear attention: its gate needs z and a bias, and no fixed decay");
     const GlaGate gg = gla ? *gla : GlaGate();
@@ -1456,6 +1456,15 @@ int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* sta
             ZG_HIP(hipGetLastError());
             return ZG_OK;
         }
+    }
+    // Entries of more than 32 tokens: chunks as matrix products (us per layer of 6 heads of 128 x 128, everything else of the layer
+    // included: one entry of 33 tokens 61.6 against 61.0 token by token, of 129 65.7 against 141, of 1023 79 against 155 in scanned
+    // chunks; eight entries of 33 tokens 73 against 97).  The test hook sends them through the scan.
+    if (!decay && M > kGemvMaxRows && longest > 32 && getenv("ZGPT2_LM_SCAN_NO_CHUNKS") == nullptr) {
+        bool taken = false;
+        ZG_TRY(launch_gated_chunks(proj, ld, out, ldo, state, slot_stride, ent_start, ent_len, ent_slot, n_entries, M, H, D, V, bias, low, ws, ws_floats, gla, s,
+                                   &taken));
+        if (taken) return ZG_OK;
     }
     int G = 1;
     while (G * kScanRows < D) G <<= 1;
