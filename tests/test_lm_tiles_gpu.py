@@ -70,3 +70,35 @@ def test_latent_tiles(kv_rank, rot_dim):
         tl.assert_close(got, want, "bfloat16", (kv_rank, step))
         lo = hi
     m.close()
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("rows", [3, 4, 5, 8])
+def test_rows_of_decode_steps(rows, dtype):
+    """Decode steps of 3 to 8 sequences: widths that are no multiple of the products' pieces of 64 and 16, rows short and long enough for
+    each form, experts chosen by none and by many; a sequence whose numbers are not finite leaves its neighbours alone."""
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=152, experts=9, top=3)),
+                     tl.latent_layer(heads=2, dim=16, vdim=16, rot_dim=8, kv_rank=136, q_rank=40, mlp=tl.dense_mlp(ff=1096)),
+                     tl.hgrn2_layer(heads=1, dim=16, vdim=24, mlp=tl.moe_mlp(ff=520, experts=3, top=2))], vocab=203, width=136)
+    w = tl.weights(cfg, seed=rows)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(40 + b, 7, cfg["vocab"]) for b in range(rows)]
+    for t in toks:
+        t[t == 9] = 10
+    refs = [oracle.forward(t)[0] for t in toks]
+    w["embed"] = w["embed"].copy()
+    w["embed"][9, 5] = np.inf
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=512, max_seqs=8)
+    m.load_weights(w)
+    for bad in (None, 1):
+        seqs = [m.open() for _ in toks]
+        for i in range(7):
+            got = m.step([(s, [9 if b == bad and i == 3 else t[i]], [0]) for b, (s, t) in enumerate(zip(seqs, toks))])
+            for b in range(rows):
+                if b == bad and i >= 3:
+                    assert np.isnan(got[b]).any()
+                else:  # (fp32 arithmetic in both modes: nothing is rounded in a step of few rows)
+                    tl.assert_close(got[b:b + 1], refs[b][i:i + 1], "float32" if dtype == "float32" else dtype, (rows, b, i, bad))
+        for s in seqs:
+            m.close_seq(s)
+    m.close()

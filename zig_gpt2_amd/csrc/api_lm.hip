@@ -1297,7 +1297,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 if (!glu) up.act = ACT_GELU_ERF;
                 dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;
                 if (few) {  // one batch per assignment, its expert's matrices looked up on the device
-                    up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick;
+                    up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick; up.n_groups = dn.n_groups = E;
                     up.c_zoff = UF; dn.c_zoff = W;
                 } else {  // assignments sorted by expert, grouped products
                     ZG_TRY(launch_group(g->pick, NA, E, g->grp_off, g->sorted, g->inv, s));
@@ -1372,7 +1372,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 if (d.ff_act == ZG_LM_ACT_GELU) up.act = ACT_GELU_ERF;
                 dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;
                 if (few) {  // one batch per assignment, its expert's matrices looked up on the device
-                    up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick;
+                    up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick; up.n_groups = dn.n_groups = E;
                     up.z_limit = dn.z_limit = E;
                     up.c_zoff = UF; dn.c_zoff = W;
                 } else {  // assignments sorted by expert, grouped products
@@ -1496,7 +1496,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             if (!glu) up.act = ACT_GELU_ERF;
             dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;
             if (few) {  // one batch per assignment, its expert's matrices looked up on the device
-                up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick;
+                up.M = dn.M = 1; up.nz = dn.nz = NA; up.z_group = dn.z_group = g->pick; up.n_groups = dn.n_groups = E;
                 up.c_zoff = UF; dn.c_zoff = W;
             } else {  // assignments sorted by expert, grouped products
                 ZG_TRY(launch_group(g->pick, NA, E, g->grp_off, g->sorted, g->inv, s));

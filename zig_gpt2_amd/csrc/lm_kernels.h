@@ -55,7 +55,7 @@ struct Linear {
     float poly_eps = 0.0f;
     int nz = 1;
     long long a_zoff = 0, b_zoff = 0, c_zoff = 0;
-    const int* z_group = nullptr;
+    const int* z_group = nullptr;  // (n_groups: how many matrices it names, 0 where that is not known)
     int z_limit = 0x7fffffff;  // batches whose z_group is not below it are skipped, their rows of C left alone (row-vector kernels)
     const int* grp_off = nullptr;
     int n_groups = 0;

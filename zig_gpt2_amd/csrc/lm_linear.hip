@@ -16,67 +16,13 @@
 
 #include <type_traits>
 
-#include "lm_kernels.h"
+#include "lm_linear_args.h"
 
 namespace zg {
 namespace lm {
 
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
-typedef __attribute__((ext_vector_type(16))) float f32x16;
-
-struct LinArgs {
-    const float* A;
-    const bf16_t* B;
-    float* C;
-    const int* a_rows;
-    const int* z_group;
-    const int* grp_off;
-    long long a_zoff, b_zoff, c_zoff;
-    int lda, ldb, ldc;
-    int M, N, K;
-    int a_div, act, n_groups, a_glu;
-    float act_a, act_b;
-    const float* bias;
-    int z_limit;
-    int glu_kind;
-    float glu_limit;
-    const float* glu_scale;
-    int glu_gate_col;
-    const float* a_poly;
-    float poly_eps;
-    const bf16_t* A16;  // the same rows as bf16 (tiled kernels), or null
-    bf16_t* C16;        // the result rounded to bf16, beside or instead of C (tiled kernels), or null
-    int a_vec, b_vec;  // 16-byte loads allowed (alignment of base, leading dimension and batch offsets)
-};
-
-// output n on its way out: the bias, then the activation
-__device__ __forceinline__ float finish(float v, int n, const LinArgs& p) {
-    const int act = p.act;
-    if (p.bias) v += p.bias[n];
-    if (act == ACT_SCALE_SOFTCAP) {
-        v *= p.act_a;
-        if (p.act_b > 0.0f) v = p.act_b * tanhf(v / p.act_b);
-    } else if (act == ACT_RELU2) {
-        v = fmaxf(v, 0.0f);
-        v = v * v;
-    } else if (act == ACT_GELU_ERF) {
-        v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
-    }
-    return v;
-}
-
-// the gated activation of a [gate | up] row, applied where a product reads it (sc: the row's factor, clipped form only)
-__device__ __forceinline__ float glu_on_load(float g, float u, const LinArgs& p, float sc) {
-    if (p.glu_kind == GLU_CLIPPED) {
-        g = fminf(g * sc, p.glu_limit);
-        u = fminf(fmaxf(u * sc, -p.glu_limit), p.glu_limit);
-        return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
-    }
-    if (p.glu_kind == GLU_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
-    return g / (1.0f + expf(-g)) * u;
-}
 
 // eight consecutive weights of row `w` from column k, zero beyond K
 __device__ __forceinline__ void load_w8(const bf16_t* w, int k, int K, bool vec, float out[8]) {
@@ -374,36 +320,6 @@ __device__ __forceinline__ void unroll(F&& f) {
         f(step<I>());
         unroll<N, I + 1>(f);
     }
-}
-
-// eight consecutive fp32 values -> NP planes of eight bf16 (packed pairs)
-template <int NP>
-struct Planes8 {
-    u32x4 v[NP];
-};
-// the upper bf16 half of a value (truncated), and what is left of it (nothing of an infinity or NaN)
-__device__ __forceinline__ float term_left(float x) {
-    const uint32_t b = __float_as_uint(x);
-    const float r = x - __uint_as_float(b & 0xFFFF0000u);
-    return (b & 0x7F800000u) == 0x7F800000u ? 0.0f : r;
-}
-__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
-template <int NP>
-__device__ __forceinline__ Planes8<NP> to_planes(const f32x4& a, const f32x4& b) {
-    Planes8<NP> o;
-    if constexpr (NP == 1) {
-        o.v[0] = u32x4{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w), cvt_pk_bf16(b.x, b.y), cvt_pk_bf16(b.z, b.w)};
-    } else {
-        float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-        for (int t = 0; t < NP; ++t) {  // 24 mantissa bits = 8 + 8 + 8: what the third term leaves is zero
-            o.v[t] = u32x4{upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7])};
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (t + 1 < NP) x[i] = t == 0 ? term_left(x[i]) : x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
-        }
-    }
-    return o;
 }
 
 // Eight consecutive activations in flight: fp32 as they are, or already rounded to bf16 by the kernel that wrote them.
@@ -916,11 +832,13 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LinArgs p) {
 }  // namespace
 
 namespace {
-LinArgs make_args(const Linear& L);
 bool takes_k_split(const Linear& L) { return L.K >= 1536 && L.M <= 2 && L.nz <= 4; }
 }  // namespace
 
 int launch_linear_pair(const Linear& A, const Linear& B, bool f32, hipStream_t s) {
+    bool taken = false;
+    if (getenv("ZGPT2_LM_NO_ROWS") == nullptr) ZG_TRY(launch_rows(A, &B, s, &taken));
+    if (taken) return ZG_OK;
     const bool one_launch = A.M == 1 && B.M == 1 && A.nz >= 1 && B.nz >= 1 && A.N > 0 && B.N > 0 && !A.grp_off && !B.grp_off && !takes_k_split(A) &&
                             !takes_k_split(B) && A.K > 0 && B.K > 0 && A.A && A.B && A.C && B.A && B.B && B.C && A.a_div >= 1 && B.a_div >= 1 &&
                             A.nz + B.nz <= 65535;
@@ -935,23 +853,6 @@ int launch_linear_pair(const Linear& A, const Linear& B, bool f32, hipStream_t s
     return ZG_OK;
 }
 
-namespace {
-LinArgs make_args(const Linear& L) {
-    LinArgs p;
-    p.A = L.A; p.B = L.B; p.C = L.C; p.a_rows = L.a_rows; p.z_group = L.z_group; p.grp_off = L.grp_off;
-    p.a_zoff = L.a_zoff; p.b_zoff = L.b_zoff; p.c_zoff = L.c_zoff;
-    p.lda = L.lda; p.ldb = L.ldb; p.ldc = L.ldc; p.M = L.M; p.N = L.N; p.K = L.K;
-    p.a_div = L.a_div; p.act = L.act; p.n_groups = L.grp_off ? L.n_groups : 0; p.a_glu = L.a_glu;
-    p.act_a = L.act_a; p.act_b = L.act_b; p.bias = L.bias; p.z_limit = L.z_limit; p.glu_kind = L.glu_kind; p.glu_limit = L.glu_limit; p.glu_scale = L.glu_scale;
-    p.glu_gate_col = L.glu_gate_col;
-    p.A16 = L.A16; p.C16 = L.C16;
-    p.a_poly = L.a_poly;
-    p.poly_eps = L.poly_eps;
-    p.a_vec = ((reinterpret_cast<uintptr_t>(L.A) & 15) == 0 && L.lda % 4 == 0 && L.a_zoff % 4 == 0) ? 1 : 0;
-    p.b_vec = ((reinterpret_cast<uintptr_t>(L.B) & 15) == 0 && L.ldb % 8 == 0 && L.b_zoff % 8 == 0) ? 1 : 0;
-    return p;
-}
-}  // namespace
 
 namespace {
 template <typename AT, int NP>
@@ -996,6 +897,9 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
                kPolyMaxRows);
     const LinArgs p = make_args(L);
     if (!L.grp_off && L.M <= kGemvMaxRows) {
+        bool taken = false;
+        if (getenv("ZGPT2_LM_NO_ROWS") == nullptr) ZG_TRY(launch_rows(L, nullptr, s, &taken));
+        if (taken) return ZG_OK;
         if (takes_k_split(L)) {  // long rows, one or two of them, few batches: K split over the waves, two weight rows per workgroup
             const dim3 gks((L.N + 1) / 2, 1, L.nz);  // (from four rows on the activations are re-read by too many workgroups: measured slower)
             if (L.a_poly) {

@@ -1,0 +1,120 @@
+// lm_linear_args.h — what the kernels behind launch_linear share (lm_linear.hip, lm_rows.hip): the launch's arguments, what happens to
+// an activation on its way in and to an output on its way out, and the exact split of fp32 values into bf16 terms.
+#pragma once
+#include <type_traits>
+
+#include "lm_kernels.h"
+
+namespace zg {
+namespace lm {
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+struct LinArgs {
+    const float* A;
+    const bf16_t* B;
+    float* C;
+    const int* a_rows;
+    const int* z_group;
+    const int* grp_off;
+    long long a_zoff, b_zoff, c_zoff;
+    int lda, ldb, ldc;
+    int M, N, K;
+    int a_div, act, n_groups, a_glu;
+    float act_a, act_b;
+    const float* bias;
+    int z_limit;
+    int glu_kind;
+    float glu_limit;
+    const float* glu_scale;
+    int glu_gate_col;
+    const float* a_poly;
+    float poly_eps;
+    const bf16_t* A16;  // the same rows as bf16 (tiled kernels), or null
+    bf16_t* C16;        // the result rounded to bf16, beside or instead of C (tiled kernels), or null
+    int a_vec, b_vec;  // 16-byte loads allowed (alignment of base, leading dimension and batch offsets)
+};
+
+// output n on its way out: the bias, then the activation
+__device__ __forceinline__ float finish(float v, int n, const LinArgs& p) {
+    const int act = p.act;
+    if (p.bias) v += p.bias[n];
+    if (act == ACT_SCALE_SOFTCAP) {
+        v *= p.act_a;
+        if (p.act_b > 0.0f) v = p.act_b * tanhf(v / p.act_b);
+    } else if (act == ACT_RELU2) {
+        v = fmaxf(v, 0.0f);
+        v = v * v;
+    } else if (act == ACT_GELU_ERF) {
+        v = 0.5f * v * (1.0f + erff(v * 0.70710678118654752f));
+    }
+    return v;
+}
+
+// the gated activation of a [gate | up] row, applied where a product reads it (sc: the row's factor, clipped form only)
+__device__ __forceinline__ float glu_on_load(float g, float u, const LinArgs& p, float sc) {
+    if (p.glu_kind == GLU_CLIPPED) {
+        g = fminf(g * sc, p.glu_limit);
+        u = fminf(fmaxf(u * sc, -p.glu_limit), p.glu_limit);
+        return g / (1.0f + expf(-1.702f * g)) * (u + 1.0f);
+    }
+    if (p.glu_kind == GLU_GELU) return 0.5f * g * (1.0f + tanhf(0.7978845608028654f * (g + 0.044715f * g * g * g))) * u;
+    return g / (1.0f + expf(-g)) * u;
+}
+
+// eight consecutive fp32 values -> NP planes of eight bf16 (packed pairs)
+template <int NP>
+struct Planes8 {
+    u32x4 v[NP];
+};
+// the upper bf16 half of a value (truncated), and what is left of it (nothing of an infinity or NaN)
+__device__ __forceinline__ float term_left(float x) {
+    const uint32_t b = __float_as_uint(x);
+    const float r = x - __uint_as_float(b & 0xFFFF0000u);
+    return (b & 0x7F800000u) == 0x7F800000u ? 0.0f : r;
+}
+__device__ __forceinline__ uint32_t upper_halves(float lo, float hi) { return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u); }
+template <int NP>
+__device__ __forceinline__ Planes8<NP> to_planes(const f32x4& a, const f32x4& b) {
+    Planes8<NP> o;
+    if constexpr (NP == 1) {
+        o.v[0] = u32x4{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w), cvt_pk_bf16(b.x, b.y), cvt_pk_bf16(b.z, b.w)};
+    } else {
+        float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+        for (int t = 0; t < NP; ++t) {  // 24 mantissa bits = 8 + 8 + 8: what the third term leaves is zero
+            o.v[t] = u32x4{upper_halves(x[0], x[1]), upper_halves(x[2], x[3]), upper_halves(x[4], x[5]), upper_halves(x[6], x[7])};
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (t + 1 < NP) x[i] = t == 0 ? term_left(x[i]) : x[i] - __uint_as_float(__float_as_uint(x[i]) & 0xFFFF0000u);
+        }
+    }
+    return o;
+}
+
+inline LinArgs make_args(const Linear& L) {
+    LinArgs p;
+    p.A = L.A; p.B = L.B; p.C = L.C; p.a_rows = L.a_rows; p.z_group = L.z_group; p.grp_off = L.grp_off;
+    p.a_zoff = L.a_zoff; p.b_zoff = L.b_zoff; p.c_zoff = L.c_zoff;
+    p.lda = L.lda; p.ldb = L.ldb; p.ldc = L.ldc; p.M = L.M; p.N = L.N; p.K = L.K;
+    p.a_div = L.a_div; p.act = L.act; p.n_groups = L.grp_off ? L.n_groups : 0; p.a_glu = L.a_glu;
+    p.act_a = L.act_a; p.act_b = L.act_b; p.bias = L.bias; p.z_limit = L.z_limit; p.glu_kind = L.glu_kind; p.glu_limit = L.glu_limit; p.glu_scale = L.glu_scale;
+    p.glu_gate_col = L.glu_gate_col;
+    p.A16 = L.A16; p.C16 = L.C16;
+    p.a_poly = L.a_poly;
+    p.poly_eps = L.poly_eps;
+    p.a_vec = ((reinterpret_cast<uintptr_t>(L.A) & 15) == 0 && L.lda % 4 == 0 && L.a_zoff % 4 == 0) ? 1 : 0;
+    p.b_vec = ((reinterpret_cast<uintptr_t>(L.B) & 15) == 0 && L.ldb % 8 == 0 && L.b_zoff % 8 == 0) ? 1 : 0;
+    return p;
+}
+
+}  // namespace
+
+// lm_rows.hip: steps of 3 to 8 rows on the matrix cores.  *taken = false: not a form it has (nothing launched).
+int launch_rows(const Linear& a, const Linear* b, hipStream_t s, bool* taken);
+
+}  // namespace lm
+}  // namespace zg

@@ -1,0 +1,189 @@
+// lm_rows.hip — the linear maps of decode steps of 3 to 8 rows on the matrix cores, and the chosen experts' products of such steps.
+//
+// A workgroup owns 16 weight rows; its four waves take K in turns of 64 columns and meet in the LDS.  The weights are the MFMA's rows,
+// straight from memory (a lane loads 32 bytes of its row, four lanes a 128-byte line).  The activations stay fp32: a value is the exact
+// sum of three bf16 terms, the eight rows' leading and middle terms are the sixteen columns of one product, their last terms half of
+// a second one.  Everything a wave needs is requested at entry for K up to 1024, four turns ahead beyond.
+//
+// The general kernel (lm_gemv_kernel) reads all rows for every two weight rows: 8 x 24 KB of activations through each wave for 3 KB of
+// weights at K = 768.  Here they are read once per 16 weight rows.
+//
+// Chosen experts: a workgroup takes an EXPERT's 16 weight rows and the (up to eight) assignments that chose it, found in the step's
+// list on the device; experts nobody chose cost an empty workgroup, and one chosen by several rows is read once.
+#include "lm_linear_args.h"
+
+#include <algorithm>
+
+namespace zg {
+namespace lm {
+
+namespace {
+
+typedef __attribute__((ext_vector_type(4))) float acc4;
+
+constexpr int kTurn = 64;  // columns of K a wave takes at a time
+
+__device__ __forceinline__ int nth_bit(unsigned long long m, int n) {  // position of the n-th set bit (n < 8)
+#pragma unroll
+    for (int i = 0; i < 7; ++i)
+        if (i < n) m &= m - 1;
+    return __builtin_ctzll(m);
+}
+
+template <int TURNS, bool GLU>  // TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight
+__device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (*part)[16][17]) {
+    const int n0 = blockIdx.x * 16;
+    if (n0 >= p.N) return;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4, m = col & 7;
+    unsigned long long left = 0;  // assignments of this expert that are still to do
+    if (p.z_group) {
+        left = __ballot(lane < p.M && p.z_group[min(lane, p.M - 1)] == z);
+        if (left == 0) return;
+    }
+    const bf16_t* w = p.B + (long long)z * p.b_zoff + (long long)min(n0 + col, p.N - 1) * p.ldb;
+    do {
+        const int n_rows = p.z_group ? min(8, __popcll(left)) : p.M;
+        // (columns without a row compute on the last one's and are not stored)
+        const int rid = p.z_group ? nth_bit(left, min(m, n_rows - 1)) : min(m, n_rows - 1);
+        const float* a = p.A + (long long)(p.z_group ? rid : z) * p.a_zoff + (long long)((p.a_rows ? p.a_rows[rid] : rid) / p.a_div) * p.lda;
+        const float asc = GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
+        const float agate = GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-a[p.glu_gate_col])) : 1.0f;
+        const int n_turns = (p.K + kTurn - 1) / kTurn;
+        constexpr int RING = TURNS > 0 ? TURNS : 4;
+        u32x4 wr[RING][2];
+        f32x4 ar[RING][4], ur[GLU ? RING : 1][4];
+        auto fetch = [&](int slot, int turn) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const int k = min(turn * kTurn + 16 * kg + 8 * j, p.K - 8);
+                wr[slot][j] = *reinterpret_cast<const u32x4*>(w + k);
+                ar[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + k);
+                ar[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + k + 4);
+                if constexpr (GLU) {
+                    ur[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + p.a_glu + k);
+                    ur[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + p.a_glu + k + 4);
+                }
+            }
+        };
+        acc4 acc1 = {0.0f, 0.0f, 0.0f, 0.0f}, acc2 = acc1;
+        auto multiply = [&](int slot, int turn) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                f32x4 x = ar[slot][2 * j], y = ar[slot][2 * j + 1];
+                u32x4 wv = wr[slot][j];
+                if constexpr (GLU) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        x[u] = glu_on_load(x[u], ur[slot][2 * j][u], p, asc) * agate;
+                        y[u] = glu_on_load(y[u], ur[slot][2 * j + 1][u], p, asc) * agate;
+                    }
+                }
+                if (turn * kTurn + kTurn > p.K && turn * kTurn + 16 * kg + 8 * j >= p.K) {  // columns beyond K: the clamped load brought earlier ones
+                    x = y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    wv = u32x4{0u, 0u, 0u, 0u};
+                }
+                const Planes8<3> pl = to_planes<3>(x, y);
+                const u32x4 zero = {0u, 0u, 0u, 0u};
+                const bf16x8 wf = __builtin_bit_cast(bf16x8, wv);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, col < 8 ? pl.v[2] : zero), acc2, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, col < 8 ? pl.v[0] : pl.v[1]), acc1, 0, 0, 0);
+            }
+        };
+        if constexpr (TURNS > 0) {
+#pragma unroll
+            for (int i = 0; i < TURNS; ++i) fetch(i, wave + 4 * i);
+#pragma unroll
+            for (int i = 0; i < TURNS; ++i) multiply(i, wave + 4 * i);  // (a turn behind the last one multiplies zeros)
+        } else {
+#pragma unroll
+            for (int i = 0; i < RING; ++i) fetch(i, wave + 4 * i);
+            for (int t = wave; t < n_turns; t += 4 * RING) {
+#pragma unroll
+                for (int i = 0; i < RING; ++i) {
+                    multiply(i, t + 4 * i);
+                    fetch(i, t + 4 * (i + RING));
+                }
+            }
+        }
+        // element e: weight row 4 kg + e, column col
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = acc1[e] + acc2[e];
+        __syncthreads();
+        const int row = threadIdx.x & 15, om = threadIdx.x >> 4;
+        if (om < n_rows && n0 + row < p.N) {
+            const float hi = (part[0][row][om] + part[1][row][om]) + (part[2][row][om] + part[3][row][om]);
+            const float mid = (part[0][row][om + 8] + part[1][row][om + 8]) + (part[2][row][om + 8] + part[3][row][om + 8]);
+            float* C = p.C + (p.z_group ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
+            C[n0 + row] = finish(hi + mid, n0 + row, p);
+        }
+        if (!p.z_group) return;
+        for (int i = 0; i < 8 && left; ++i) left &= left - 1;
+        if (left) __syncthreads();
+    } while (left);
+}
+
+// batches [0, za) are product a's, the rest product b's
+template <int TURNS, bool GLU>
+__global__ __launch_bounds__(256) void lm_rows_kernel(const LinArgs a, const LinArgs b, int za) {
+    __shared__ float part[4][16][17];
+    if ((int)blockIdx.z < za) rows_body<TURNS, GLU>(a, blockIdx.z, part);
+    else rows_body<TURNS, GLU>(b, blockIdx.z - za, part);
+}
+
+// a product in the form the kernel takes: plain rows, or a list of one-row batches with the matrix chosen by a list (M: its length);
+// false: neither
+bool rows_form(const Linear& L, LinArgs& p, int& nz) {
+    if (L.grp_off || L.a_poly || L.C16 || L.K < 8 || L.N <= 0 || !L.A || !L.B || !L.C || L.a_div < 1) return false;
+    p = make_args(L);
+    nz = L.nz;
+    if (L.z_group) {
+        if (L.M != 1 || L.nz > 64 || L.n_groups <= 0 || L.n_groups > 65535) return false;
+        p.M = L.nz;
+        nz = L.n_groups;  // (entries of the list that name no matrix are left alone, as z_limit asks)
+        if (L.z_limit < L.n_groups) return false;
+    } else if (L.M == 1 && L.nz > 1 && L.b_zoff == 0 && !L.a_rows) {  // one-row batches of one matrix
+        if (L.a_zoff > 0x7fffffff || L.c_zoff > 0x7fffffff || L.a_div != 1) return false;
+        p.M = L.nz;
+        p.lda = (int)L.a_zoff;
+        p.ldc = (int)L.c_zoff;
+        nz = 1;
+    }
+    // Where it pays (us per launch, this against the general kernel): 3 rows 2304 x 768 4.3 : 5.6, 8 rows 4.9 : 9.5, 8 rows of the
+    // vocabulary 31 : 75.  Beyond K = 1024 a compute unit's intake binds it and the general kernel's finer tiles spread over more of them: 3
+    // rows 768 x 3072 9.4 : 8.5, 4 rows 9.9 : 9.2, 8 rows 11.9 : 14.8.  Lists: 16 assignments over 8 experts of 1536 x 768 7.1 : 9.9, 8 of
+    // them 6.6 : 6.8, 6 of them 6.4 : 5.3.
+    const bool pays = L.z_group ? p.M >= 8 : p.M >= (L.K <= 1024 ? 3 : 6);
+    return pays && (L.z_group || p.M <= 8) && p.a_vec && p.b_vec && L.K % 8 == 0 && L.a_glu % 4 == 0 && nz <= 65535;
+}
+
+}  // namespace
+
+int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
+    *taken = false;
+    LinArgs a, b;
+    int za = 0, zb = 0;
+    if (!rows_form(A, a, za)) return ZG_OK;
+    b = a;
+    if (B && (!rows_form(*B, b, zb) || za + zb > 65535 || (a.a_glu > 0) != (b.a_glu > 0))) return ZG_OK;
+    const int turns = (std::max(a.K, b.K) + kTurn - 1) / kTurn;
+    const dim3 grid((std::max(a.N, b.N) + 15) / 16, 1, za + zb);
+    const int per_wave = (turns + 3) / 4;
+#define ZG_ROWS(T)                                                                   \
+    do {                                                                             \
+        if (a.a_glu > 0) lm_rows_kernel<T, true><<<grid, 256, 0, s>>>(a, b, za);     \
+        else lm_rows_kernel<T, false><<<grid, 256, 0, s>>>(a, b, za);                \
+    } while (0)
+    if (per_wave == 1) ZG_ROWS(1);
+    else if (per_wave == 2) ZG_ROWS(2);
+    else if (per_wave == 3) ZG_ROWS(3);
+    else if (per_wave == 4) ZG_ROWS(4);
+    else ZG_ROWS(0);
+#undef ZG_ROWS
+    note_kernel("lm_rows_kernel<%d>", per_wave <= 4 ? per_wave : 0);
+    ZG_HIP(hipGetLastError());
+    *taken = true;
+    return ZG_OK;
+}
+
+}  // namespace lm
+}  // namespace zg
