@@ -48,6 +48,38 @@ def test_values_that_are_not_finite(dtype, bad):
     tl.assert_close(got[:25], ref[:25], dtype, (bad, dtype))
 
 
+@pytest.mark.parametrize("rows", [9, 64, 255, 257, 300])
+def test_rounded_rows(monkeypatch, rows):
+    """Portions in bf16 mode, whose rows reach the products rounded: the persistent kernel (forced at any number of tiles; widths that end
+    inside its tiles), the tile forms, and widths that are no whole 16-byte pieces, where the rows stay fp32."""
+    for width, ff, rank, bad in ((128, 328, 128, 0), (192, 320, 136, 1), (132, 100, 44, 0)):
+        layers = [tl.hgrn2_layer(heads=2, dim=24, vdim=64, mlp=tl.dense_mlp(ff=ff)),
+                  tl.latent_layer(heads=3, dim=16, vdim=16, rot_dim=8, kv_rank=rank, q_rank=rank, mlp=tl.dense_mlp(ff=ff)),
+                  tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=ff, experts=5, top=2))]
+        if bad:  # (attention multiplies the masked values of a tile by zero)
+            del layers[1]
+        cfg = tl.config(layers, vocab=203, width=width)
+        w = tl.weights(cfg, seed=rows)
+        toks = tl.tokens(30 + rows, rows, cfg["vocab"])
+        toks[toks == 7] = 8
+        ref = lm_oracle.Model(cfg, w).forward(toks)[0]
+        cut = rows
+        if bad:  # rows in front of a token that is not finite are what they are without it
+            cut = rows - rows // 3
+            toks[cut] = 7
+            w["embed"] = w["embed"].copy()
+            w["embed"][7, 3] = np.inf
+        for form in ("256", "128", "32", ""):
+            monkeypatch.setenv("ZGPT2_LM_GEMM_TILE", form) if form else monkeypatch.delenv("ZGPT2_LM_GEMM_TILE", raising=False)
+            m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="bfloat16", max_tokens=512, max_seqs=2)
+            m.load_weights(w)
+            s = m.open()
+            got = m.step([(s, toks, list(range(rows)))])
+            m.close()
+            tl.assert_close(got[:cut], ref[:cut], "bfloat16", (rows, width, form))
+            assert not np.isfinite(got[cut:]).any()
+
+
 @pytest.mark.parametrize("kv_rank,rot_dim", [(40, 6), (64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])
 def test_latent_tiles(kv_rank, rot_dim):
     """Latent attention of portions with every tile size (rows of no whole number of pieces among them): three sequences whose portions

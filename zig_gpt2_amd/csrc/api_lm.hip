@@ -241,6 +241,8 @@ struct zg_lm {
     size_t trace_floats = 0;
     float last_step_ms = 0.0f, last_decode_ms = 0.0f;
     bool use_graph = true;
+    // rows of prompt portions rounded to bf16 by the kernels that write them, for the matrix product that reads them (bf16 mode)
+    bf16_t *h16 = nullptr, *hc16 = nullptr, *o16 = nullptr, *u16 = nullptr;
     bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
     size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
     int step_longest = 0;  // rows of the longest entry of the running portion
@@ -726,6 +728,12 @@ void layout(zg_lm* g, Bump& b) {
     g->gu_buf = b.take<float>(MS * max_gu);
     g->hb = b.take<float>(MS * max_hb);
     g->ye = b.take<float>(MS * max_assign * W);
+    if (!g->f32) {
+        g->h16 = b.take<bf16_t>(MS * W);
+        if (g->side) g->hc16 = b.take<bf16_t>(MS * W);
+        g->o16 = b.take<bf16_t>(MS * max_o);
+        g->u16 = b.take<bf16_t>(MS * std::max(max_ff, max_hb));
+    }
     g->wt = b.take<float>(MS * max_assign);
     g->pick = b.take<int>(MS * max_assign);
     g->sorted = b.take<int>(MS * max_assign);
@@ -913,6 +921,11 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     ZG_TRY(launch_embed(g->embed, d_ids, g->x, readd ? g->x0 : nullptr, g->embed_scale, M, W, g->V, g->flag, d_pos, g->pos_freq, s));
     const bool side = g->side;
     const bool tnorm = g->tanh_norms;
+    // Prompt portions in bf16 mode: what only matrix products read travels rounded to bf16, from the kernel that writes it, where its rows
+    // are whole 16-byte pieces (the products would round it to the same values; half the bytes, and operands that go to the LDS as they are)
+    const bool r16 = !f32 && !few;
+    const bool h_r16 = r16 && W % 8 == 0 && !canon && !tnorm;
+    auto whole = [](int n) { return n % 8 == 0; };
     // side-by-side sublayers: the sums a layer leaves for the next layer's norm kernel to add
     OpenSums pend;
     auto copy_trace = [&](int p) -> int {
@@ -936,24 +949,29 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         return replayed ? (g->bucket_keys > 0 ? g->bucket_keys : all_keys) : std::min(all_keys, (g->step_keys + 63) / 64 * 64);
     };
     // the dense feed-forward of a layer: in -> out (first_done: its first product has been launched)
-    auto dense_up = [&](const LayerW& L, const float* in) {
+    auto dense_up = [&](const LayerW& L, const float* in, const bf16_t* in16) {
         Linear up;
-        up.A = in; up.lda = W; up.B = L.up; up.ldb = W; up.C = g->u; up.ldc = L.n_up; up.M = M; up.N = L.n_up; up.K = W;
+        up.A = in; up.A16 = in16; up.lda = W; up.B = L.up; up.ldb = W; up.C = g->u; up.ldc = L.n_up; up.M = M; up.N = L.n_up; up.K = W;
         up.act = L.d.dense_act == ZG_LM_DENSE_RELU2 ? ACT_RELU2 : ACT_NONE;
         return up;
     };
-    auto dense_ff = [&](const LayerW& L, const float* in, float* out, bool first_done = false) -> int {
+    auto dense_ff = [&](const LayerW& L, const float* in, const bf16_t* in16, float* out, bool first_done = false) -> int {
         const int F = L.d.ff_width;
         const bool poly = L.d.dense_act == ZG_LM_DENSE_POLYNORM, gated = L.d.dense_act == ZG_LM_DENSE_GLU_GELU;
         Linear dn;
-        if (!first_done) ZG_TRY(launch_linear(dense_up(L, in), f32, s));
+        bf16_t* const u16 = r16 && whole(F) ? g->u16 : nullptr;
+        if (!first_done) {
+            Linear up = dense_up(L, in, in16);
+            if (u16 && !poly && !gated && whole(W)) up.C16 = u16, up.C = nullptr;
+            ZG_TRY(launch_linear(up, f32, s));
+        }
         if (gated) {  // rows gate | up
             dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
             if (M <= 2) {  // the activation where the second product reads its rows (more rows: every workgroup would redo it)
                 dn.A = g->u; dn.lda = L.n_up; dn.a_glu = F; dn.glu_kind = GLU_GELU;
             } else {
-                ZG_TRY(launch_glu(g->u, g->hb, M, F, s, GLU_GELU));
-                dn.A = g->hb; dn.lda = F;
+                ZG_TRY(launch_glu(g->u, g->hb, M, F, s, GLU_GELU, 0, -1, u16));
+                dn.A = u16 ? nullptr : g->hb; dn.A16 = u16; dn.lda = F;
             }
             return launch_linear(dn, f32, s);
         }
@@ -961,9 +979,10 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             dn.a_poly = L.poly;
             dn.poly_eps = eps;
         } else if (poly) {
-            ZG_TRY(launch_polynorm(g->u, F, F, M, L.poly, eps, s));
+            ZG_TRY(launch_polynorm(g->u, F, F, M, L.poly, eps, s, u16));
         }
-        dn.A = g->u; dn.lda = F; dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
+        const bool u_r16 = u16 && (poly || whole(W));
+        dn.A = u_r16 ? nullptr : g->u; dn.A16 = u_r16 ? u16 : nullptr; dn.lda = F; dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
         return launch_linear(dn, f32, s);
     };
     // one-row steps of side-by-side sublayers: the dense feed-forward's first product rides in the launch of the mixer's first
@@ -971,7 +990,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     auto first_product = [&](const LayerW& L, const Linear& lin) -> int {
         if (!(side && M == 1 && L.d.ff == ZG_LM_FF_DENSE)) return launch_linear(lin, f32, s);
         up_done = &L;
-        return launch_linear_pair(lin, dense_up(L, g->hc), f32, s);
+        return launch_linear_pair(lin, dense_up(L, g->hc, nullptr), f32, s);
     };
     bool h_ready = false;  // g->h already holds this pass's shifted norm (written by the previous pass's fused tail)
     if (tnorm) {  // the norm behind the embedding (in place) and the first pass's norm; every later one rides behind a sublayer's sum
@@ -985,7 +1004,8 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         const int H = d.heads, D = d.dim, Vd = d.vdim;
         bool hc_ready = false;  // one launch has done everything up to the mixer's input (decode steps)
         if (side) {  // what the layer before left open, and both norms of this layer from one statistic
-            ZG_TRY(launch_norm_two(g->x, pend, L.norm1, d.ff != ZG_LM_FF_NONE ? L.norm2 : nullptr, eps, g->h, g->hc, M, W, s));
+            ZG_TRY(launch_norm_two(g->x, pend, L.norm1, d.ff != ZG_LM_FF_NONE ? L.norm2 : nullptr, eps, h_r16 ? nullptr : g->h,
+                                   h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->hc, M, W, s, h_r16 ? g->h16 : nullptr, h_r16 ? g->hc16 : nullptr));
             pend = OpenSums();
             h_ready = true;
         }
@@ -994,10 +1014,11 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                                            L.canon1, g->seq_state + ps.canon1_off, g->seq_floats, d_slot, g->hc, s, &hc_ready));
         if (ps.readd && !hc_ready) ZG_TRY(launch_add_rows(g->x, g->x0, M, W, s));
         if (!h_ready && !hc_ready)
-            ZG_TRY(launch_norm_shift(g->x, L.norm1, canon ? nullptr : L.shift, eps, g->h, M, W, d_prev, d_slot, g->shift_state + (size_t)p * W,
-                                     (size_t)g->n_passes * W, canon || g->no_shift ? nullptr : d_last, g->last_h + (size_t)p * NS * W, s));
+            ZG_TRY(launch_norm_shift(g->x, L.norm1, canon ? nullptr : L.shift, eps, h_r16 ? nullptr : g->h, M, W, d_prev, d_slot, g->shift_state + (size_t)p * W,
+                                     (size_t)g->n_passes * W, canon || g->no_shift ? nullptr : d_last, g->last_h + (size_t)p * NS * W, s, h_r16 ? g->h16 : nullptr));
         h_ready = false;
-        const float* hin = g->h;  // what the sublayer reads
+        const float* hin = h_r16 ? nullptr : g->h;  // what the sublayer reads
+        const bf16_t* hin16 = h_r16 ? g->h16 : nullptr;
         if (canon) {
             if (!hc_ready) ZG_TRY(input_conv(L.canon1, ps.canon1_off));
             hin = g->hc;
@@ -1007,7 +1028,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             if (p + 1 >= g->n_passes || canon || g->passes[p + 1].readd) return ZG_OK;
             const LayerW& N = g->layers[g->passes[p + 1].layer];
             if (g->no_shift && y) {  // nothing of the token before: the same fusion at any number of rows
-                ZG_TRY(launch_norm_add_norm(g->x, y, wb, N.norm1, eps, g->h, M, W, s));
+                ZG_TRY(launch_norm_add_norm(g->x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
                 h_ready = true;
                 return ZG_OK;
             }
@@ -1023,7 +1044,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             KeyMask mask;
             mask.window = d.window;
             mask.chunk = d.chunk;
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
             lin.bias = L.qkv_bias;
             ZG_TRY(first_product(L, lin));
             ValuePrep vals;
@@ -1061,7 +1082,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             ZG_TRY(launch_linear(lin, f32, s));
         } else if (d.mixer == ZG_LM_MIX_SSD) {
             const int G = d.kv_heads, HV = H * Vd, CC = HV + 2 * G * D, LD = L.ld_cat;
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             ConvArgs cv;
             cv.in = g->proj + HV; cv.ld_in = LD; cv.out = g->ta; cv.ld_out = CC; cv.C = CC; cv.taps = d.conv; cv.w = L.convw; cv.bias = L.convb;
@@ -1076,16 +1097,17 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 sa.xbc = g->ta; sa.ld_xbc = CC;
             }
             ZG_TRY(launch_ssd_scan(sa, single ? &cv : nullptr, M, d_estart, d_elen, d_eslot, n_ent, g->scan_ws, g->scan_ws_floats, s));
-            ZG_TRY(launch_part_norm(g->o, HV, HV, std::max(1, d.norm_groups), M, L.part_norm, eps, single ? &cv : nullptr, d_slot, s));
+            bf16_t* const o16 = r16 && whole(HV) ? g->o16 : nullptr;
+            ZG_TRY(launch_part_norm(g->o, HV, HV, std::max(1, d.norm_groups), M, L.part_norm, eps, single ? &cv : nullptr, d_slot, s, o16));
             lin = Linear();
-            lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
+            lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             ZG_TRY(launch_linear(lin, f32, s));
         } else if (d.mixer == ZG_LM_MIX_WINDOW_LINEAR) {
             const int G = d.kv_heads, HD = H * D, GD = G * D, GV = G * Vd, CC = HD + GD + GV, HV = H * Vd;
             const int HR = d.lin_heads, DR = d.lin_dim, VR = d.lin_vdim, HRD = HR * DR, HRV = HR * VR, NP = L.n_cat, OC = HV + HRV;
             const int og = CC, orq = CC + HV, org = orq + 2 * HRD + HRV;  // columns of the left gate, the right q | k | v, the right gate
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             // left: biases and convolutions of q | k | v at once, the whole-projection norms, keys and values into the cache
             ConvArgs cv;
@@ -1122,7 +1144,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int oy = H * D + G * D + G * Vd, ox = oy + C;  // columns of the two branches of the recurrent unit
             const Rotary rot{L.rot_freq, d.rot_dims, 1.0f};
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             // left: attention inside the window
             ZG_TRY(launch_window_prep(g->proj, NP, M, H, G, D, Vd, rot, L.vfreq, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache, s));
@@ -1159,7 +1181,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         } else if (d.mixer == ZG_LM_MIX_CHANNEL_DELTA) {
             const int G = d.kv_heads, HV = H * Vd, CC = 2 * G * D + HV, RA = d.decay_rank, RG = d.gate_rank, NP = L.n_cat;
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             ConvArgs cv;
             cv.in = g->proj; cv.ld_in = NP; cv.out = g->ta; cv.ld_out = CC; cv.C = CC; cv.taps = d.conv; cv.w = L.convw; cv.flags = CONV_SILU;
@@ -1182,7 +1204,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int HD = H * D, HV = H * Vd, RA = d.decay_rank, NP = L.n_cat;
             const int og = 2 * HD + HV, oa = og + HV;  // columns of the output gate and of the decay's first step
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             lin = Linear();  // the decay's second step
             lin.A = g->proj + oa; lin.lda = NP; lin.B = L.a2; lin.ldb = RA; lin.C = g->tb; lin.ldc = HD; lin.M = M; lin.N = HD; lin.K = RA;
@@ -1201,7 +1223,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             shape.cap = d.softcap;
             shape.slope = d.dist_bias ? L.slopes : nullptr;
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             ZG_TRY(launch_head_norm_prep(g->proj, NP, M, H, G, D, eps, d.qtemp_coef, d.qtemp_every, d_pos, d_slot, g->page_table, g->max_pages, g->P,
                                          ps.cache, s));
@@ -1219,53 +1241,61 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         } else if (d.mixer == ZG_LM_MIX_HGRN2) {
             const int HD = H * D, HV = H * Vd, NP = 2 * HD + HV;
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.qfv; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.qfv; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(launch_linear(lin, f32, s));
             ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
                                      L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
-            ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s));
+            bf16_t* const o16 = r16 && whole(HV) ? g->o16 : nullptr;
+            ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s, o16));
             lin = Linear();
-            lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
+            lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             ZG_TRY(launch_linear(lin, f32, s));
         } else {
             const int R = d.rot_dim, KR = d.kv_rank, QR = d.q_rank, HV = H * Vd, LD = L.ld_cat;
             const bool direct = QR == 0;  // queries projected directly (they sit in the fused projection's rows)
             const Rotary rot{L.rot_freq, d.rot_dims, L.rot_amp, d.rot_halves};
             lin = Linear();
-            lin.A = hin; lin.lda = W; lin.B = L.dqkv; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
+            lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.dqkv; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
             ZG_TRY(first_product(L, lin));
             const float* gate = d.head_gate ? g->proj + L.n_cat - H : nullptr;
+            // (portions on the tiled attention: its queries and results rounded, in the place of the fp32 rows)
+            const bool tiles = r16 && g->key_tiles && latent_tile_elems(KR, R) > 0 && g->step_key_tiles * latent_tile_elems(KR, R) <= g->key_tile_elems && n_ent <= 65535;
+            bf16_t* const cq16 = r16 && whole(QR) ? reinterpret_cast<bf16_t*>(g->cq) : nullptr;
+            bf16_t* const qa16 = tiles && whole(KR) && whole(R) && whole(D) && (direct ? whole(LD) : true) && whole(D + R) ? reinterpret_cast<bf16_t*>(g->qa) : nullptr;
+            bf16_t* const ctx16 = tiles && whole(KR) ? reinterpret_cast<bf16_t*>(g->ctx) : nullptr;
+            bf16_t* const o16 = ctx16 && whole(HV) ? g->o16 : nullptr;
             const float* q = direct ? g->proj : g->q;
             const int ldq = direct ? LD : H * (D + R);
             if (direct) {
                 ZG_TRY(launch_latent_direct_prep(g->proj, LD, M, H, D, R, KR, H * (D + R), L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages,
-                                                 g->P, g->qa, d.kv_from > 0 ? nullptr : ps.cache, s));
+                                                 g->P, g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, qa16));
             } else {
                 ZG_TRY(launch_latent_prep(g->proj, LD, M, QR, KR, R, L.dq_norm, L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages, g->P,
-                                          g->cq, ps.cache, s));
+                                          g->cq, ps.cache, s, cq16));
                 lin = Linear();
-                lin.A = g->cq; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
+                lin.A = cq16 ? nullptr : g->cq; lin.A16 = cq16; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
                 ZG_TRY(launch_linear(lin, f32, s));
             }
             lin = Linear();  // the unrotated query part carried into the latent space, head by head
             lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
-            lin.C = g->qa; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
+            lin.C = qa16 ? nullptr : g->qa; lin.C16 = qa16; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
             ZG_TRY(launch_linear(lin, f32, s));
-            if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s));
+            if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
             bool tiled = false;
             if (!f32 && !few)
                 ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
                                                      g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
-                                                     L.sink));
+                                                     L.sink, qa16, ctx16));
+            ZG_REQUIRE(tiled || !tiles, ZG_ERR_UNSUPPORTED, "latent attention: the tiles do not fit their workspace");
             if (!tiled)
                 ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,
                                                g->attn_ws, g->attn_ws_floats, s, gate, LD, L.sink));
             lin = Linear();  // values of the weighted latent, head by head
-            lin.A = g->ctx; lin.lda = H * KR; lin.a_zoff = KR; lin.B = L.uv; lin.ldb = KR; lin.b_zoff = (long long)Vd * KR;
-            lin.C = g->o; lin.ldc = HV; lin.c_zoff = Vd; lin.M = M; lin.N = Vd; lin.K = KR; lin.nz = H;
+            lin.A = ctx16 ? nullptr : g->ctx; lin.A16 = ctx16; lin.lda = H * KR; lin.a_zoff = KR; lin.B = L.uv; lin.ldb = KR; lin.b_zoff = (long long)Vd * KR;
+            lin.C = o16 ? nullptr : g->o; lin.C16 = o16; lin.ldc = HV; lin.c_zoff = Vd; lin.M = M; lin.N = Vd; lin.K = KR; lin.nz = H;
             ZG_TRY(launch_linear(lin, f32, s));
             lin = Linear();
-            lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
+            lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             ZG_TRY(launch_linear(lin, f32, s));
         }
         if (tnorm) {  // norms without statistics: every sum behind a sublayer carries the next sublayer's norm
@@ -1283,7 +1313,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int F = d.ff_width;
             part = SumParts();
             if (d.ff == ZG_LM_FF_DENSE) {
-                ZG_TRY(dense_ff(L, g->h, g->y));
+                ZG_TRY(dense_ff(L, g->h, nullptr, g->y));
                 part.a = g->y;
             } else if (d.ff == ZG_LM_FF_MOE) {
                 const int E = d.experts, top = d.top, NA = M * top;
@@ -1328,7 +1358,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 } else if (few) {  // the gated activation is applied where the second product reads its rows
                     dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
                 } else {
-                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s));
+                    bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
+                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
+                    if (hb16) dn.A = nullptr, dn.A16 = hb16;
                 }
                 ZG_TRY(launch_linear(dn, f32, s));
                 if (d.shared_width > 0) {  // the expert every token uses
@@ -1356,8 +1388,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         if (side) {  // the feed-forward beside the mixer, on the second norm of the same x
             const int F = d.ff_width;
             const float* fin = g->hc;
+            const bf16_t* fin16 = h_r16 ? g->hc16 : nullptr;
             if (d.ff == ZG_LM_FF_DENSE) {
-                ZG_TRY(dense_ff(L, fin, g->y2, up_done == &L));
+                ZG_TRY(dense_ff(L, h_r16 ? nullptr : fin, fin16, g->y2, up_done == &L));
                 up_done = nullptr;
             } else if (d.ff == ZG_LM_FF_MOE) {
                 const int E = d.experts, top = d.top, NA = M * top;
@@ -1367,7 +1400,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 ZG_TRY(launch_route(fin, M, W, L.router, L.correction, E + d.identity, top, g->pick, g->wt, d.router, s, d.route_groups, d.route_keep,
                                     d.route_scale != 0.0f ? d.route_scale : 1.0f));
                 Linear up, dn;
-                up.A = fin; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
+                up.A = fin; up.A16 = fin16; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
                 up.N = UF; up.K = W;
                 if (d.ff_act == ZG_LM_ACT_GELU) up.act = ACT_GELU_ERF;
                 dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;
@@ -1396,7 +1429,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 } else if (silu && few) {  // the activation is applied where the second product reads its rows
                     dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
                 } else if (silu) {
-                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s));
+                    bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
+                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
+                    if (hb16) dn.A = nullptr, dn.A16 = hb16;
                 } else if (few) {  // the activation is applied where the second product reads its rows
                     dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F; dn.glu_kind = GLU_CLIPPED; dn.glu_limit = d.ff_limit;
                     dn.glu_scale = on_input ? g->wt : nullptr;
@@ -1414,7 +1449,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 }
                 if (S > 0 && silu && !paired) {
                     lin = Linear();
-                    lin.A = fin; lin.lda = W; lin.B = L.sgu; lin.ldb = W; lin.C = g->tb; lin.ldc = SL; lin.M = M; lin.N = 2 * S + (sg_col >= 0 ? 1 : 0); lin.K = W;
+                    lin.A = fin; lin.A16 = fin16; lin.lda = W; lin.B = L.sgu; lin.ldb = W; lin.C = g->tb; lin.ldc = SL; lin.M = M; lin.N = 2 * S + (sg_col >= 0 ? 1 : 0); lin.K = W;
                     ZG_TRY(launch_linear(lin, f32, s));
                     ZG_TRY(launch_glu(g->tb, g->tc, M, S, s, GLU_SILU, SL, sg_col));
                     lin = Linear();
@@ -1423,7 +1458,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                     ys = g->td;
                 } else if (S > 0 && !silu) {  // the shared expert; its gate logit is the last column of its first product
                     lin = Linear();
-                    lin.A = fin; lin.lda = W; lin.B = L.sgu; lin.ldb = W; lin.C = g->tb; lin.ldc = 2 * S + 1; lin.M = M; lin.N = 2 * S + 1; lin.K = W;
+                    lin.A = fin; lin.A16 = fin16; lin.lda = W; lin.B = L.sgu; lin.ldb = W; lin.C = g->tb; lin.ldc = 2 * S + 1; lin.M = M; lin.N = 2 * S + 1; lin.K = W;
                     ZG_TRY(launch_linear(lin, f32, s));
                     lin = Linear();
                     lin.B = L.sdown; lin.ldb = S; lin.C = g->td; lin.ldc = W; lin.M = M; lin.N = W; lin.K = S;
@@ -1469,19 +1504,21 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             ZG_TRY(launch_norm_conv_single(g->x, nullptr, g->y, nullptr, nullptr, nullptr, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
                                            g->seq_state + ps.canon2_off, g->seq_floats, d_slot, g->hc, s, &mid_done));
         if (mid_done) {
-        } else if (d.ff != ZG_LM_FF_NONE) ZG_TRY(launch_norm_add_norm(g->x, g->y, L.norm1b, L.norm2, eps, g->h, M, W, s));
+        } else if (d.ff != ZG_LM_FF_NONE)  // (a router reads the fp32 rows)
+            ZG_TRY(launch_norm_add_norm(g->x, g->y, L.norm1b, L.norm2, eps, h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
         else {
             ZG_TRY(tail(g->y, nullptr, nullptr, 0, L.norm1b));
             if (!h_ready) ZG_TRY(launch_norm_add(g->x, g->y, L.norm1b, eps, M, W, s));
         }
         const int F = d.ff_width;
         hin = g->h;
+        hin16 = h_r16 ? g->h16 : nullptr;
         if (canon && d.ff != ZG_LM_FF_NONE) {
             if (!mid_done) ZG_TRY(input_conv(L.canon2, ps.canon2_off));
             hin = g->hc;
         }
         if (d.ff == ZG_LM_FF_DENSE) {
-            ZG_TRY(dense_ff(L, hin, g->y));
+            ZG_TRY(dense_ff(L, hin16 ? nullptr : hin, hin16, g->y));
             ZG_TRY(tail(g->y, nullptr, nullptr, 0, L.norm2b));
             if (!h_ready) ZG_TRY(launch_norm_add(g->x, g->y, L.norm2b, eps, M, W, s));
         } else if (d.ff == ZG_LM_FF_MOE) {
@@ -1491,7 +1528,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             ZG_TRY(launch_route(hin, M, W, L.router, L.correction, E, top, g->pick, g->wt, d.router, s, d.route_groups, d.route_keep,
                                 d.route_scale != 0.0f ? d.route_scale : 1.0f));
             Linear up, dn;
-            up.A = hin; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
+            up.A = hin; up.A16 = hin16; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
             up.N = UF; up.K = W;
             if (!glu) up.act = ACT_GELU_ERF;
             dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;
@@ -1508,7 +1545,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             } else if (few) {  // the gated activation is applied where the second product reads its rows
                 dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
             } else {
-                ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s));
+                bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
+                ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
+                if (hb16) dn.A = nullptr, dn.A16 = hb16;
             }
             ZG_TRY(launch_linear(dn, f32, s));
             if (few) ZG_TRY(tail(nullptr, g->ye, g->wt, top, L.norm2b));

@@ -521,9 +521,6 @@ int launch_p8_bn(const bf16_t* A, const bf16_t* B, const float* bias, void* C, i
 
 }  // namespace
 
-static unsigned long long g_gemm_launches = 0;
-unsigned long long gemm_mfma_launch_count() { return g_gemm_launches; }
-void gemm_note_launch() { ++g_gemm_launches; }
 int gemm_debug_stamps(unsigned long long* out, size_t n_words) { return gemm_s4_stamps(out, n_words); }
 
 int launch_gemm_planes(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl,
@@ -563,7 +560,7 @@ int launch_gemm_planes(const bf16_t* A, const bf16_t* B, const float* bias, void
     // M = 16384: 76 us against 88.7 us on the eight-wave kernel's 256-wide tiles at equal cost)
     int bn = cost(192) * 8 <= cost(256) * 9 ? 192 : 256;
     if (bn_env == 192 || bn_env == 256) bn = bn_env;
-    ++g_gemm_launches;
+    gemm_note_launch();
     // Two generations of the kernel: the four-wave software-pipelined one (gemm_s4.hip) wherever 192-wide tiles are the
     // choice (its 256-wide instantiation does not fit the register file without spills yet), the eight-wave one below
     // for 256-wide tiles.  ZGPT2_GEMM_KERNEL=p8 / s4 forces one (s4 then always with 192-wide tiles).  (The third generation —

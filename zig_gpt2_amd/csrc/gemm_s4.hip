@@ -1013,6 +1013,10 @@ int launch_s4_nt(const bf16_t* A, const bf16_t* B, const float* bias, void* C, i
 
 }  // namespace
 
+static unsigned long long g_gemm_launches = 0;  // of either generation of the kernel (test hook)
+unsigned long long gemm_mfma_launch_count() { return g_gemm_launches; }
+void gemm_note_launch() { ++g_gemm_launches; }
+
 // what the 14 packed argument dwords of gemm_s4_kernel can express (the dispatcher sends anything else that is not ragged
 // to the eight-wave kernel, whose arguments are not packed; api_ops.hip keeps ragged Linears beyond it on the GEMV path)
 bool gemm_s4_args_ok(const GemmPlanes& pl, int ldc) {

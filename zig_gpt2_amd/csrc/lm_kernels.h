@@ -81,16 +81,18 @@ int launch_embed(const bf16_t* table, const int* ids, float* x, float* x_copy, f
 // Rows listed in last_rows (the last token of every entry) also store their UNSHIFTED h into last_out[entry] — committed to
 // the slots' state by launch_commit_rows once the step has run, so that no row of this launch reads a state another row wrote.
 // mu == null: no shift (out = h).
+// Here and in the norms below, h16 / out16 (may be null): the same rows rounded to bf16 for the matrix products of a prompt portion; the
+// fp32 rows may then be null.
 int launch_norm_shift(const float* x, const float* w, const float* mu, float eps, float* out, int M, int W, const int* row_prev,
                       const int* row_slot, const float* shift_state, size_t slot_stride, const int* row_entry_if_last, float* last_out,
-                      hipStream_t s);
+                      hipStream_t s, bf16_t* out16 = nullptr);
 // dst[slots[e]] = src[e] for every entry e; rows of `width` floats (dst rows slot_stride apart, src rows src_stride apart)
 int launch_commit_rows(float* dst, size_t slot_stride, const float* src, size_t src_stride, const int* slots, int n_entries, int width,
                        int n_sets, size_t dst_set_stride, size_t src_set_stride, hipStream_t s);
 // x[m] += y[m] / rms(y[m]) * (1 + w)            (the norm behind a sublayer, then the residual sum)
 int launch_norm_add(float* x, const float* y, const float* w, float eps, int M, int W, hipStream_t s);
 // x[m] += y[m] / rms(y[m]) * (1 + wb);  h[m] = x[m] / rms(x[m]) * (1 + wn)   (the two above in one launch)
-int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s);
+int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s, bf16_t* h16 = nullptr);
 // Steps of one row per entry: the sum behind a pass's last sublayer (y, or the weighted sum of the chosen experts' rows yexp) and
 // the next pass's norm + shift in one launch.  *taken = false for rows too wide for its registers (nothing launched).
 int launch_sum_norm_shift(float* x, const float* y, const float* yexp, const float* weight, int top, const float* wb, const float* wn, const float* mu,
@@ -115,11 +117,13 @@ struct OpenSums {
     const float* ident = nullptr;
     __host__ __device__ bool any() const { return a || b || bias || exp; }
 };
-int launch_norm_two(float* x, const OpenSums& add, const float* wa, const float* wb, float eps, float* ha, float* hb, int M, int W, hipStream_t s);
+int launch_norm_two(float* x, const OpenSums& add, const float* wa, const float* wb, float eps, float* ha, float* hb, int M, int W, hipStream_t s,
+                    bf16_t* ha16 = nullptr, bf16_t* hb16 = nullptr);
 // x[m] += the same sums
 int launch_add_two(float* x, const OpenSums& add, int M, int W, hipStream_t s);
 // In place over `rows` rows of `width` floats with row stride ld: v / rms(v) * w  (a plain weight; per-head norms)
-int launch_norm_plain(float* v, int ld, int rows_per_m, int width, int M, const float* w, float eps, hipStream_t s);
+// (out16: the results there, rounded to bf16, instead)
+int launch_norm_plain(float* v, int ld, int rows_per_m, int width, int M, const float* w, float eps, hipStream_t s, bf16_t* out16 = nullptr);
 
 // Norms without statistics: n(v) = tanh(alpha v) * w + b.  A norm's tensors lie together, nw = [w (W) | b (W) | alpha (1)].
 // out[j] = n(x[rows ? rows[j] : j]);  pre != null (rows == null): x[j] <- pre(x[j]) first, in place (a norm behind the embedding).
@@ -215,9 +219,11 @@ int launch_ssd_scan(const SsdArgs& a, const ConvArgs* conv, int M, const int* en
                     float* ws, size_t ws_floats, hipStream_t s);
 // In place: v[m] cut into `parts` equal parts, each divided by its own root mean square, times w (one weight per channel).
 // conv != null (steps of one row per entry): conv's tail is moved on by the row's inputs in the same launch.
-int launch_part_norm(float* v, int ld, int width, int parts, int M, const float* w, float eps, const ConvArgs* conv, const int* row_slot, hipStream_t s);
+// (out16: the results there, rounded to bf16, instead; the same of the activation below)
+int launch_part_norm(float* v, int ld, int width, int parts, int M, const float* w, float eps, const ConvArgs* conv, const int* row_slot, hipStream_t s,
+                     bf16_t* out16 = nullptr);
 // In place over M rows of F floats: a N(z) + b N(z^2) + c N(z^3) + e with N over the row; act holds a, b, c, e.
-int launch_polynorm(float* z, int ld, int F, int M, const float* act, float eps, hipStream_t s);
+int launch_polynorm(float* z, int ld, int F, int M, const float* act, float eps, hipStream_t s, bf16_t* out16 = nullptr);
 
 // ------------------------------------------------------------------------------------------------ latent attention
 // Rotary table of one layer: freq[i] for the rot_dims / 2 pairs (YaRN blend applied on the host) and the amplitude factor.
@@ -231,15 +237,16 @@ struct Rotary {
 };
 int launch_latent_prep(const float* proj, int ld, int M, int q_rank, int KR, int R, const float* wq, const float* wkv, float eps, Rotary rot,
                        const int* row_pos, const int* row_slot, const int* page_table, int max_pages, int page_tokens, float* cq,
-                       float* cache, hipStream_t s);
+                       float* cache, hipStream_t s, bf16_t* cq16 = nullptr);
 // Queries projected directly: proj rows [q (H (D + R)) | dkv latent (KR) | rotated key part (R) at column kv_col].  qa[m][h][KR ..] =
 // rotary(q[m][h][D ..]) and, with cache != null, the token's cache row as above — one launch.  cache == null: the layer reads another
 // layer's latents (no dkv columns).
 int launch_latent_direct_prep(const float* proj, int ld, int M, int H, int D, int R, int KR, int kv_col, const float* wkv, float eps, Rotary rot,
                               const int* row_pos, const int* row_slot, const int* page_table, int max_pages, int page_tokens, float* qa, float* cache,
-                              hipStream_t s);
+                              hipStream_t s, bf16_t* qa16 = nullptr);
 // qa[m][h][KR ..] = rotary(q[m][h][D ..]) — the rotated query part moved behind the absorbed part (which a batched Linear wrote).
-int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, int D, int R, int KR, Rotary rot, const int* row_pos, hipStream_t s);
+int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, int D, int R, int KR, Rotary rot, const int* row_pos, hipStream_t s,
+                    bf16_t* qa16 = nullptr);
 // ctx[m][h][:KR] = sum_j softmax_j( scale * qa[m][h] . cacherow(j) ) latent(j) over the keys j <= row_pos[m] of the row's sequence.
 // ws: fp32 workspace for the partials of split key ranges (steps of at most kGemvMaxRows rows: M * H * kAttnSplits * (KR + 2)
 // floats; without it whole key rows per workgroup).
@@ -259,7 +266,8 @@ size_t latent_tile_elems(int KR, int R);
 int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
                                   const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
                                   const float* cache, bf16_t* ws, size_t ws_elems, size_t n_tiles, int max_keys, hipStream_t s, bool* taken,
-                                  const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);
+                                  const float* gate = nullptr, int ldg = 0, const float* sink = nullptr, const bf16_t* qa16 = nullptr,
+                                  bf16_t* ctx16 = nullptr);
 
 // ------------------------------------------------------------------------------------------------ input convolution of decode rows, residual sum
 // Steps of one row per entry: [x += x0] or [x += norm(y) * (1 + wb), y = yl or the mean of the two normed branches yl, yr with
@@ -407,7 +415,7 @@ int launch_route(const float* g, int M, int W, const bf16_t* router, const float
 int launch_group(const int* pick, int n_assign, int E, int* grp_off, int* sorted, int* inv, hipStream_t s);
 // h[p][j] = act(gu[p][j]) * gu[p][F + j] * t, act by kind (GLU_SILU, GLU_GELU), gu rows ld floats apart (0: 2 F)
 //   t = gate_col >= 0 ? sigmoid(gu[p][gate_col]) : 1        (a gate logit that the same product left in the row)
-int launch_glu(const float* gu, float* h, int rows, int F, hipStream_t s, int kind = GLU_SILU, int ld = 0, int gate_col = -1);
+int launch_glu(const float* gu, float* h, int rows, int F, hipStream_t s, int kind = GLU_SILU, int ld = 0, int gate_col = -1, bf16_t* h16 = nullptr);
 // h[p][j] = act(s gu[p][j], s gu[p][F + j]) * t,  act(g, u) = g' sigmoid(1.702 g') (u' + 1), g' = min(g, limit), u' = clamp(u, -limit, limit)
 //   s = row_scale ? row_scale[row_of ? row_of[p] : p] : 1   (the router's score of the assignment that sits at sorted place p)
 //   t = gate_col >= 0 ? sigmoid(gu[p][gate_col]) : 1        (a gate logit that the same product left in the row)

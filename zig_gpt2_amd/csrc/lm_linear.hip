@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "lm_linear_args.h"
+#include "zg_kernels.h"
 
 namespace zg {
 namespace lm {
@@ -832,6 +833,24 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LinArgs p) {
 }  // namespace
 
 namespace {
+// Plain products of rounded rows with enough tiles of 256 x 192 go to the persistent kernel of the large-batch Linears (gemm_s4.hip), whose
+// hand-scheduled four waves keep the matrix cores twice as busy: 8184 x 3072 x 1024 59 against 89 us, 47 with a rounded result; 8184 x 672 x
+// 1024 (128 tiles) 26.6 against 29; 1791 x 3072 x 768 (112) 23.2 against 24.5; 1023 x 3072 x 768 (64 tiles) 21.7 against 15.4.
+bool takes_persistent(const Linear& L) {
+    const char* form = getenv("ZGPT2_LM_GEMM_TILE");  // test hook: 256 = here at any number of tiles, another = never
+    const int least = form ? (atoi(form) == 256 ? 1 : 0x7fffffff) : 112;
+    GemmPlanes pl{};
+    pl.lda = L.lda;
+    pl.ldb = L.ldb;
+    pl.kpp = L.K / 64;
+    pl.npairs = 1;
+    const bool one_result = (L.C != nullptr) != (L.C16 != nullptr);
+    return !L.grp_off && !L.z_group && L.nz == 1 && !L.a_rows && L.a_div == 1 && L.act == ACT_NONE && one_result && L.K >= 128 && L.K % 64 == 0 && L.lda % 8 == 0 &&
+           L.ldb % 8 == 0 && L.lda >= L.K && L.ldc >= L.N && (L.C || (L.N % 8 == 0 && L.ldc % 8 == 0)) && gemm_s4_args_ok(pl, L.ldc) &&
+           ((reinterpret_cast<uintptr_t>(L.A16) | reinterpret_cast<uintptr_t>(L.B) | reinterpret_cast<uintptr_t>(L.C) | reinterpret_cast<uintptr_t>(L.C16)) & 15) == 0 &&
+           (size_t)L.M * L.ldc * 4 < ((size_t)1 << 32) && (size_t)L.N * L.ldb < (1u << 30) && (size_t)L.M * L.lda < (1u << 30) &&
+           (long long)((L.M + 255) / 256) * ((L.N + 191) / 192) >= least;
+}
 bool takes_k_split(const Linear& L) { return L.K >= 1536 && L.M <= 2 && L.nz <= 4; }
 }  // namespace
 
@@ -859,7 +878,7 @@ template <typename AT, int NP>
 int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
     auto tiles = [&](int bm, int bn) { return (long long)((L.N + bn - 1) / bn) * ((L.M + bm - 1) / bm + (L.grp_off ? L.n_groups : 0)); };
     int force = 0;  // 128, 64 or 32: that form at any size (tests run small ragged shapes through all of them)
-    if (const char* e = getenv("ZGPT2_LM_GEMM_TILE")) force = atoi(e);
+    if (const char* e = getenv("ZGPT2_LM_GEMM_TILE")) force = atoi(e) == 256 ? 0 : atoi(e);
     auto grid = [&](int bm, int bn) { return dim3((unsigned)tiles(bm, bn), 1, L.nz); };
     ZG_REQUIRE(tiles(32, 32) < (1LL << 31) && L.nz <= 65535, ZG_ERR_UNSUPPORTED, "linear: %d rows in %d batches exceed the grid", L.M, L.nz);
     // Which form (us per launch, both sides measured on an MI355X):
@@ -875,7 +894,8 @@ int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
 #define ZG_TILES(kernel, TM, TN, AHEAD, bm, bn) (kernel<AT, NP, TM, TN, AHEAD><<<grid(bm, bn), 256, 0, s>>>(p), which = #kernel "<" #TM ", " #TN ">")
     if (deep) ZG_TILES(lm_deep_kernel, 1, 1, 3, 32, 32);
     else if constexpr (NP == 1) {
-        if (force ? force == 128 : tiles(128, 128) >= 320) ZG_TILES(lm_wide_kernel, 2, 2, 1, 128, 128);
+        // (two steps ahead where rounded activations leave the registers for it: 8184 x 3072 x 1024 88.7 against 92.6)
+        if (force ? force == 128 : tiles(128, 128) >= 320) ZG_TILES(lm_wide_kernel, 2, 2, (std::is_same<AT, float>::value ? 1 : 2), 128, 128);
         else ZG_TILES(lm_wide_kernel, 1, 1, 2, 64, 64);
     } else {
         if (force ? force == 128 : tiles(32, 64) > 512) ZG_TILES(lm_wide_kernel, 1, 2, 2, 64, 128);
@@ -926,6 +946,15 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     ZG_REQUIRE(!(L.z_group && L.grp_off), ZG_ERR_ARG, "linear: a matrix per batch and row groups exclude each other");
     ZG_REQUIRE(L.z_limit == 0x7fffffff, ZG_ERR_ARG, "linear: skipped batches are for steps of few rows");
     const bool rounded = L.A16 && !f32;
+    if (rounded && takes_persistent(L)) {
+        GemmPlanes pl{};
+        pl.lda = L.lda;
+        pl.ldb = L.ldb;
+        pl.kpp = L.K / 64;
+        pl.npairs = 1;
+        note_kernel("gemm_s4_kernel");
+        return launch_gemm_s4(L.A16, L.B, L.bias, L.C ? static_cast<void*>(L.C) : L.C16, L.M, L.N, pl, L.ldc, false, L.C == nullptr, 192, s);
+    }
     const bool a_vec = rounded ? (reinterpret_cast<uintptr_t>(L.A16) & 15) == 0 && L.lda % 8 == 0 && L.a_zoff % 8 == 0 : p.a_vec != 0;
     // (32-bit products of a few columns exist in toy models only.  There the last bits of a sum that cancels almost entirely can decide a
     // row, and they stay what the fp32 instruction makes them: 5.5 us against 3.4 at K = 64.)

@@ -58,9 +58,15 @@ __global__ __launch_bounds__(256) void embed_kernel(const bf16_t* table, const i
 // in one go at the top of the kernel, so a one-row step (decoding) pays one memory round trip instead of one per pass.
 constexpr int kRowRegs = 16;
 
+// an output value, as it is and / or rounded to bf16 for the matrix product that reads it next
+__device__ __forceinline__ void put_row(float* out, bf16_t* out16, size_t at, float v) {
+    if (out) out[at] = v;
+    if (out16) out16[at] = (bf16_t)cvt_pk_bf16(v, v);
+}
+
 __global__ __launch_bounds__(256) void norm_shift_kernel(const float* x, const float* w, const float* mu, float eps, float* out, int W,
                                                          const int* row_prev, const int* row_slot, const float* shift_state,
-                                                         size_t slot_stride, const int* row_entry_if_last, float* last_out) {
+                                                         size_t slot_stride, const int* row_entry_if_last, float* last_out, bf16_t* out16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
     const float* xr = x + (size_t)m * W;
@@ -99,7 +105,7 @@ __global__ __launch_bounds__(256) void norm_shift_kernel(const float* x, const f
                 const float g = 1.0f + wv[j];
                 const float h = xv[j] * r * g;
                 const float before = xp ? pv[j] * rp * g : pv[j];
-                out[(size_t)m * W + i] = mu ? h + (before - h) * mv[j] : h;
+                put_row(out, out16, (size_t)m * W + i, mu ? h + (before - h) * mv[j] : h);
                 if (entry >= 0) last_out[(size_t)entry * W + i] = h;
             }
         }
@@ -109,7 +115,7 @@ __global__ __launch_bounds__(256) void norm_shift_kernel(const float* x, const f
     if (mu == nullptr) {
         for (int i = threadIdx.x; i < W; i += blockDim.x) {
             const float h = xr[i] * r * (1.0f + w[i]);
-            out[(size_t)m * W + i] = h;
+            put_row(out, out16, (size_t)m * W + i, h);
             if (entry >= 0) last_out[(size_t)entry * W + i] = h;
         }
         return;
@@ -120,7 +126,7 @@ __global__ __launch_bounds__(256) void norm_shift_kernel(const float* x, const f
         const float g = 1.0f + w[i];
         const float h = xr[i] * r * g;
         const float before = xp ? xp[i] * rp * g : hp[i];
-        out[(size_t)m * W + i] = h + (before - h) * mu[i];
+        put_row(out, out16, (size_t)m * W + i, h + (before - h) * mu[i]);
         if (entry >= 0) last_out[(size_t)entry * W + i] = h;
     }
 }
@@ -143,7 +149,8 @@ __global__ __launch_bounds__(256) void norm_add_kernel(float* x, const float* y,
 
 // x += norm(y) * (1 + wb), then h = norm(x) * (1 + wn): the norm behind the mixer, the residual sum and the norm in front of the
 // feed-forward in one pass over the row
-__global__ __launch_bounds__(256) void norm_add_norm_kernel(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int W) {
+__global__ __launch_bounds__(256) void norm_add_norm_kernel(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int W,
+                                                            bf16_t* h16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
     const float* yr = y + (size_t)m * W;
@@ -177,7 +184,7 @@ __global__ __launch_bounds__(256) void norm_add_norm_kernel(float* x, const floa
             const int i = threadIdx.x + 256 * j;
             if (i < W) {
                 xr[i] = xv[j];
-                h[(size_t)m * W + i] = xv[j] * r2 * (1.0f + nv[j]);
+                put_row(h, h16, (size_t)m * W + i, xv[j] * r2 * (1.0f + nv[j]));
             }
         }
         return;
@@ -188,7 +195,7 @@ __global__ __launch_bounds__(256) void norm_add_norm_kernel(float* x, const floa
     for (int i = threadIdx.x; i < W; i += blockDim.x) ss = fmaf(xr[i], xr[i], ss);
     ss = block_allsum(ss, s_red);
     const float r2 = 1.0f / sqrtf(ss / (float)W + eps);
-    for (int i = threadIdx.x; i < W; i += blockDim.x) h[(size_t)m * W + i] = xr[i] * r2 * (1.0f + wn[i]);
+    for (int i = threadIdx.x; i < W; i += blockDim.x) put_row(h, h16, (size_t)m * W + i, xr[i] * r2 * (1.0f + wn[i]));
 }
 
 // Steps of one row per entry (decoding): the sum behind a pass's last sublayer and the NEXT pass's norm + token shift in one
@@ -286,7 +293,7 @@ __device__ __forceinline__ float open_sums_at(const OpenSums& add, size_t m, int
 }
 
 __global__ __launch_bounds__(256) void norm_two_kernel(float* x, const OpenSums add, const float* wa, const float* wb, float eps, float* ha, float* hb,
-                                                       int W) {
+                                                       int W, bf16_t* ha16, bf16_t* hb16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
     float* xr = x + (size_t)m * W;
@@ -308,8 +315,8 @@ __global__ __launch_bounds__(256) void norm_two_kernel(float* x, const OpenSums 
             const int i = threadIdx.x + 256 * j;
             if (i < W) {
                 if (adds) xr[i] = v[j];
-                ha[(size_t)m * W + i] = v[j] * r * wa[i];
-                if (hb) hb[(size_t)m * W + i] = v[j] * r * wb[i];
+                put_row(ha, ha16, (size_t)m * W + i, v[j] * r * wa[i]);
+                if (wb) put_row(hb, hb16, (size_t)m * W + i, v[j] * r * wb[i]);
             }
         }
         return;
@@ -324,8 +331,8 @@ __global__ __launch_bounds__(256) void norm_two_kernel(float* x, const OpenSums 
     const float r = 1.0f / sqrtf(ss / (float)W + eps);
     for (int i = threadIdx.x; i < W; i += blockDim.x) {
         const float v = xr[i];
-        ha[(size_t)m * W + i] = v * r * wa[i];
-        if (hb) hb[(size_t)m * W + i] = v * r * wb[i];
+        put_row(ha, ha16, (size_t)m * W + i, v * r * wa[i]);
+        if (wb) put_row(hb, hb16, (size_t)m * W + i, v * r * wb[i]);
     }
 }
 
@@ -336,15 +343,16 @@ __global__ __launch_bounds__(256) void add_two_kernel(float* x, const OpenSums a
 }
 
 // one wave per (row, head) vector
-__global__ __launch_bounds__(256) void norm_plain_kernel(float* v, int ld, int rows_per_m, int width, int n_vec, const float* w, float eps) {
+__global__ __launch_bounds__(256) void norm_plain_kernel(float* v, int ld, int rows_per_m, int width, int n_vec, const float* w, float eps, bf16_t* out16) {
     const int vec = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (vec >= n_vec) return;
-    float* p = v + (size_t)(vec / rows_per_m) * ld + (size_t)(vec % rows_per_m) * width;
+    const size_t at = (size_t)(vec / rows_per_m) * ld + (size_t)(vec % rows_per_m) * width;
+    float* p = v + at;
     float ss = 0.0f;
     for (int i = lane; i < width; i += 64) ss = fmaf(p[i], p[i], ss);
     ss = wave_allsum(ss);
     const float r = 1.0f / sqrtf(ss / (float)width + eps);
-    for (int i = lane; i < width; i += 64) p[i] = p[i] * r * w[i];
+    for (int i = lane; i < width; i += 64) put_row(out16 ? nullptr : v, out16, at + i, p[i] * r * w[i]);
 }
 
 // ------------------------------------------------------------------------------------------------ norms without statistics
@@ -760,24 +768,24 @@ __device__ __forceinline__ size_t cache_row(const int* page_table, int max_pages
 }
 
 // pair i of `src` (channels (2i, 2i + 1), or (i, i + dims / 2)) at position pos, rotated by pos * freq[i]; angle and product in fp32
-__device__ __forceinline__ void rotate_pair(const float* src, float* dst, int i, int pos, const Rotary& rot) {
+__device__ __forceinline__ void rotate_pair(const float* src, float* dst, int i, int pos, const Rotary& rot, bf16_t* dst16 = nullptr) {
     const float a = (float)pos * rot.freq[i];
     const float c = cosf(a) * rot.amp, s = sinf(a) * rot.amp;
     const int a0 = rot.halves ? i : 2 * i, a1 = rot.halves ? i + rot.dims / 2 : 2 * i + 1;
     const float u = src[a0], v = src[a1];
-    dst[a0] = u * c - v * s;
-    dst[a1] = v * c + u * s;
+    put_row(dst, dst16, a0, u * c - v * s);
+    put_row(dst, dst16, a1, v * c + u * s);
 }
 
 __global__ __launch_bounds__(256) void latent_prep_kernel(const float* proj, int ld, int q_rank, int KR, int R, const float* wq, const float* wkv,
                                                           float eps, Rotary rot, const int* row_pos, const int* row_slot, const int* page_table,
-                                                          int max_pages, int page_tokens, float* cq, float* cache) {
+                                                          int max_pages, int page_tokens, float* cq, float* cache, bf16_t* cq16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
     const float* row = proj + (size_t)m * ld;
     const float rq = row_inv_rms(row, q_rank, eps, s_red);
     const float rc = row_inv_rms(row + q_rank, KR, eps, s_red);
-    for (int i = threadIdx.x; i < q_rank; i += blockDim.x) cq[(size_t)m * q_rank + i] = row[i] * rq * wq[i];
+    for (int i = threadIdx.x; i < q_rank; i += blockDim.x) put_row(cq16 ? nullptr : cq, cq16, (size_t)m * q_rank + i, row[i] * rq * wq[i]);
     const int pos = row_pos[m];
     float* crow = cache + cache_row(page_table, max_pages, page_tokens, row_slot[m], pos) * (size_t)(KR + R);
     for (int i = threadIdx.x; i < KR; i += blockDim.x) crow[i] = row[q_rank + i] * rc * wkv[i];
@@ -787,16 +795,17 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* proj, int
 }
 
 __global__ __launch_bounds__(256) void q_rotary_kernel(const float* q, int ldq, float* qa, int ldqa, int H, int D, int R, int KR, Rotary rot,
-                                                       const int* row_pos) {
+                                                       const int* row_pos, bf16_t* qa16) {
     const int m = blockIdx.x, pos = row_pos[m], half = rot.dims / 2;
     for (int idx = threadIdx.x; idx < H * half; idx += blockDim.x) {
         const int h = idx / half, i = idx % half;
-        rotate_pair(q + (size_t)m * ldq + (size_t)h * (D + R) + D, qa + (size_t)m * ldqa + (size_t)h * (KR + R) + KR, i, pos, rot);
+        const size_t at = (size_t)m * ldqa + (size_t)h * (KR + R) + KR;
+        rotate_pair(q + (size_t)m * ldq + (size_t)h * (D + R) + D, qa16 ? nullptr : qa + at, i, pos, rot, qa16 ? qa16 + at : nullptr);
     }
     const int rest = R - rot.dims;
     for (int idx = threadIdx.x; idx < H * rest; idx += blockDim.x) {
         const int h = idx / rest, i = rot.dims + idx % rest;
-        qa[(size_t)m * ldqa + (size_t)h * (KR + R) + KR + i] = q[(size_t)m * ldq + (size_t)h * (D + R) + D + i];
+        put_row(qa16 ? nullptr : qa, qa16, (size_t)m * ldqa + (size_t)h * (KR + R) + KR + i, q[(size_t)m * ldq + (size_t)h * (D + R) + D + i]);
     }
 }
 
@@ -804,7 +813,7 @@ __global__ __launch_bounds__(256) void q_rotary_kernel(const float* q, int ldq, 
 // own) norms the latent, rotates the shared key part and files both in the token's cache row.
 __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* proj, int ld, int H, int D, int R, int KR, int kv_col, const float* wkv,
                                                                  float eps, Rotary rot, const int* row_pos, const int* row_slot, const int* page_table,
-                                                                 int max_pages, int page_tokens, float* qa, float* cache) {
+                                                                 int max_pages, int page_tokens, float* qa, float* cache, bf16_t* qa16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x, pos = row_pos[m], half = rot.dims / 2;
     const float* row = proj + (size_t)m * ld;
@@ -813,9 +822,11 @@ __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* pr
         for (int idx = threadIdx.x; idx < H * per; idx += blockDim.x) {
             const int h = idx / per, i = idx % per;
             const float* src = row + (size_t)h * (D + R) + D;
-            float* dst = qa + ((size_t)m * H + h) * (KR + R) + KR;
-            if (i < half) rotate_pair(src, dst, i, pos, rot);
-            else dst[rot.dims + i - half] = src[rot.dims + i - half];
+            const size_t at = ((size_t)m * H + h) * (KR + R) + KR;
+            float* dst = qa16 ? nullptr : qa + at;
+            bf16_t* dst16 = qa16 ? qa16 + at : nullptr;
+            if (i < half) rotate_pair(src, dst, i, pos, rot, dst16);
+            else put_row(dst, dst16, rot.dims + i - half, src[rot.dims + i - half]);
         }
         return;
     }
@@ -1050,7 +1061,7 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
 // 8 x 1023 tokens, 16 heads on latents of 256 + 32: 132 us and 9 for the tiles (73 GFLOP: 520 TFLOP/s); 827 us when every workgroup
 // converted and transposed its own tiles behind three barriers.
 template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
-__global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, float* ctx, int H, int KR, int R, float scale,
+__global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, const bf16_t* qa16, float* ctx, bf16_t* ctx16, int H, int KR, int R, float scale,
                                                                        const int* ent_start, const int* ent_len, int n_entries, const int* row_pos,
                                                                        const bf16_t* tiles, const float* gate, int ldg, const float* sink) {
     typedef KeyTile<NKS> T;
@@ -1080,12 +1091,20 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     request(0, 0);
     bf16x8 qf[NKS];
     {
-        const float* qrow = qa + ((size_t)(m_first + (r < nq ? r : 0)) * H + (head_ok ? h : 0)) * DT;  // (beyond the block: some valid row, never stored)
+        const size_t q_at = ((size_t)(m_first + (r < nq ? r : 0)) * H + (head_ok ? h : 0)) * DT;  // (beyond the block: some valid row, never stored)
+        const float* qrow = qa + q_at;
         auto round8 = [](const f32x4& a, const f32x4& b) {
             return __builtin_bit_cast(bf16x8, u32x4{cvt_pk_bf16(a.x, a.y), cvt_pk_bf16(a.z, a.w), cvt_pk_bf16(b.x, b.y), cvt_pk_bf16(b.z, b.w)});
         };
         const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        if (DT % 4 == 0 && (reinterpret_cast<uintptr_t>(qa) & 15) == 0) {
+        if (qa16) {  // rounded by their producers (DT is a multiple of 8)
+            const u32x4 none = {0u, 0u, 0u, 0u};
+            u32x4 q8[NKS];
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) q8[ks] = *reinterpret_cast<const u32x4*>(qa16 + q_at + min(ks * 16 + 8 * hf, DT - 8));
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, ks * 16 + 8 * hf < DT ? q8[ks] : none);
+        } else if (DT % 4 == 0 && (reinterpret_cast<uintptr_t>(qa) & 15) == 0) {
             f32x4 q4[2 * NKS];
 #pragma unroll
             for (int i = 0; i < 2 * NKS; ++i) q4[i] = *reinterpret_cast<const f32x4*>(qrow + min((i >> 1) * 16 + 8 * hf + 4 * (i & 1), DT - 4));
@@ -1200,7 +1219,8 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     if (!head_ok) return;
     const float L = lsum + __shfl_xor(lsum, 32, 64);
     if (r >= nq) return;
-    float* out = ctx + ((size_t)(m_first + r) * H + h) * KR;
+    const size_t out_at = ((size_t)(m_first + r) * H + h) * KR;
+    float* out = ctx + out_at;
     const float gf = head_gate_f(gate, ldg, (size_t)(m_first + r), h) * (sink ? sink_norm_f(mx * 0.69314718055994531f, L, sink, h) : 1.0f);
     const bool vec = KR % 4 == 0 && (reinterpret_cast<uintptr_t>(ctx) & 15) == 0;
 #pragma unroll
@@ -1211,7 +1231,9 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
             f32x4 v;
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = sink ? o[t][i + u] * gf : o[t][i + u] / L * gf;
-            if (vec) {
+            if (ctx16) {  // (KR is a multiple of 8)
+                if (d < KR) *reinterpret_cast<u32x2*>(ctx16 + out_at + d) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
+            } else if (vec) {
                 if (d < KR) *reinterpret_cast<f32x4*>(out + d) = v;
             } else {
 #pragma unroll
@@ -1324,9 +1346,9 @@ int launch_embed(const bf16_t* table, const int* ids, float* x, float* x_copy, f
 
 int launch_norm_shift(const float* x, const float* w, const float* mu, float eps, float* out, int M, int W, const int* row_prev,
                       const int* row_slot, const float* shift_state, size_t slot_stride, const int* row_entry_if_last, float* last_out,
-                      hipStream_t s) {
+                      hipStream_t s, bf16_t* out16) {
     if (M <= 0) return ZG_OK;
-    norm_shift_kernel<<<M, 256, 0, s>>>(x, w, mu, eps, out, W, row_prev, row_slot, shift_state, slot_stride, row_entry_if_last, last_out);
+    norm_shift_kernel<<<M, 256, 0, s>>>(x, w, mu, eps, out, W, row_prev, row_slot, shift_state, slot_stride, row_entry_if_last, last_out, out16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1346,9 +1368,9 @@ int launch_norm_add(float* x, const float* y, const float* w, float eps, int M, 
     return ZG_OK;
 }
 
-int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s) {
+int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s, bf16_t* h16) {
     if (M <= 0) return ZG_OK;
-    norm_add_norm_kernel<<<M, 256, 0, s>>>(x, y, wb, wn, eps, h, W);
+    norm_add_norm_kernel<<<M, 256, 0, s>>>(x, y, wb, wn, eps, h, W, h16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1372,9 +1394,10 @@ int launch_norm_gather(const float* x, const int* rows, const float* w, float ep
     return ZG_OK;
 }
 
-int launch_norm_two(float* x, const OpenSums& add, const float* wa, const float* wb, float eps, float* ha, float* hb, int M, int W, hipStream_t s) {
+int launch_norm_two(float* x, const OpenSums& add, const float* wa, const float* wb, float eps, float* ha, float* hb, int M, int W, hipStream_t s, bf16_t* ha16,
+                    bf16_t* hb16) {
     if (M <= 0) return ZG_OK;
-    norm_two_kernel<<<M, 256, 0, s>>>(x, add, wa, wb, eps, ha, wb ? hb : nullptr, W);
+    norm_two_kernel<<<M, 256, 0, s>>>(x, add, wa, wb, eps, ha, hb, W, ha16, hb16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1410,10 +1433,10 @@ int launch_tanh_sum_norm(float* x, const SumParts& y, const float* nb, float mul
     return ZG_OK;
 }
 
-int launch_norm_plain(float* v, int ld, int rows_per_m, int width, int M, const float* w, float eps, hipStream_t s) {
+int launch_norm_plain(float* v, int ld, int rows_per_m, int width, int M, const float* w, float eps, hipStream_t s, bf16_t* out16) {
     const int n_vec = M * rows_per_m;
     if (n_vec <= 0) return ZG_OK;
-    norm_plain_kernel<<<(n_vec + 3) / 4, 256, 0, s>>>(v, ld, rows_per_m, width, n_vec, w, eps);
+    norm_plain_kernel<<<(n_vec + 3) / 4, 256, 0, s>>>(v, ld, rows_per_m, width, n_vec, w, eps, out16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1516,30 +1539,30 @@ int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* sta
 
 int launch_latent_prep(const float* proj, int ld, int M, int q_rank, int KR, int R, const float* wq, const float* wkv, float eps, Rotary rot,
                        const int* row_pos, const int* row_slot, const int* page_table, int max_pages, int page_tokens, float* cq,
-                       float* cache, hipStream_t s) {
+                       float* cache, hipStream_t s, bf16_t* cq16) {
     if (M <= 0) return ZG_OK;
     ZG_REQUIRE(rot.dims % 2 == 0 && rot.dims <= R, ZG_ERR_ARG, "rotary: %d rotated dimensions of a part of %d", rot.dims, R);
     latent_prep_kernel<<<M, 256, 0, s>>>(proj, ld, q_rank, KR, R, wq, wkv, eps, rot, row_pos, row_slot, page_table, max_pages, page_tokens, cq,
-                                         cache);
+                                         cache, cq16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
 int launch_latent_direct_prep(const float* proj, int ld, int M, int H, int D, int R, int KR, int kv_col, const float* wkv, float eps, Rotary rot,
                               const int* row_pos, const int* row_slot, const int* page_table, int max_pages, int page_tokens, float* qa, float* cache,
-                              hipStream_t s) {
+                              hipStream_t s, bf16_t* qa16) {
     if (M <= 0) return ZG_OK;
     ZG_REQUIRE(rot.dims % 2 == 0 && rot.dims <= R, ZG_ERR_ARG, "rotary: %d rotated dimensions of a part of %d", rot.dims, R);
     latent_direct_prep_kernel<<<dim3(M, cache ? 2 : 1), 256, 0, s>>>(proj, ld, H, D, R, KR, kv_col, wkv, eps, rot, row_pos, row_slot, page_table, max_pages,
-                                                                     page_tokens, qa, cache);
+                                                                     page_tokens, qa, cache, qa16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
 int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, int D, int R, int KR, Rotary rot, const int* row_pos,
-                    hipStream_t s) {
+                    hipStream_t s, bf16_t* qa16) {
     if (M <= 0 || R <= 0) return ZG_OK;
-    q_rotary_kernel<<<M, 256, 0, s>>>(q, ldq, qa, ldqa, H, D, R, KR, rot, row_pos);
+    q_rotary_kernel<<<M, 256, 0, s>>>(q, ldq, qa, ldqa, H, D, R, KR, rot, row_pos, qa16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1556,7 +1579,7 @@ size_t latent_tile_elems(int KR, int R) {  // elements of a key tile in the laun
 int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
                                   const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
                                   const float* cache, bf16_t* ws, size_t ws_elems, size_t n_tiles, int max_keys, hipStream_t s, bool* taken,
-                                  const float* gate, int ldg, const float* sink) {
+                                  const float* gate, int ldg, const float* sink, const bf16_t* qa16, bf16_t* ctx16) {
     *taken = false;
     if (M <= 0 || n_entries <= 0) return ZG_OK;
     const size_t tile = latent_tile_elems(KR, R);
@@ -1567,7 +1590,7 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
         latent_tiles_kernel<NKS_><<<cgrid, 256, 0, s>>>(cache, KR + R, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, max_pages,      \
                                                         page_tokens, ws);                                                                            \
         ZG_HIP(hipGetLastError());                                                                                                                   \
-        latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, ctx, H, KR, R, scale, ent_start, ent_len, n_entries, row_pos, ws, gate, ldg, \
+        latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, qa16, ctx, ctx16, H, KR, R, scale, ent_start, ent_len, n_entries, row_pos, ws, gate, ldg, \
                                                                      sink);                                                                          \
     } while (0)
     if (tile == KeyTile<6>::BYTES / 2) ZG_ATT_T(6, 2);

@@ -298,7 +298,7 @@ __global__ __launch_bounds__(1024) void group_kernel(const int* pick, int n_assi
     }
 }
 
-__global__ __launch_bounds__(256) void glu_kernel(const float* gu, int ld, float* h, size_t n, int F, int kind, int gate_col) {
+__global__ __launch_bounds__(256) void glu_kernel(const float* gu, int ld, float* h, size_t n, int F, int kind, int gate_col, bf16_t* h16) {
     const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (idx >= n) return;
     const size_t r = idx / F;
@@ -307,7 +307,8 @@ __global__ __launch_bounds__(256) void glu_kernel(const float* gu, int ld, float
     const float a = row[j], b = row[F + j];
     float v = kind == GLU_GELU ? 0.5f * a * (1.0f + tanhf(0.7978845608028654f * (a + 0.044715f * a * a * a))) * b : a / (1.0f + expf(-a)) * b;
     if (gate_col >= 0) v *= 1.0f / (1.0f + expf(-row[gate_col]));
-    h[idx] = v;
+    if (h16) h16[idx] = (bf16_t)cvt_pk_bf16(v, v);
+    else h[idx] = v;
 }
 
 // the clipped gated activation: the gate capped from above, the linear part clipped on both sides and lifted by one
@@ -396,11 +397,11 @@ int launch_group(const int* pick, int n_assign, int E, int* grp_off, int* sorted
     return ZG_OK;
 }
 
-int launch_glu(const float* gu, float* h, int rows, int F, hipStream_t s, int kind, int ld, int gate_col) {
+int launch_glu(const float* gu, float* h, int rows, int F, hipStream_t s, int kind, int ld, int gate_col, bf16_t* h16) {
     const size_t n = (size_t)rows * F;
     if (n == 0) return ZG_OK;
     ZG_REQUIRE(kind == GLU_SILU || kind == GLU_GELU, ZG_ERR_ARG, "gated activation: kind %d", kind);
-    glu_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gu, ld > 0 ? ld : 2 * F, h, n, F, kind, gate_col);
+    glu_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(gu, ld > 0 ? ld : 2 * F, h, n, F, kind, gate_col, h16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

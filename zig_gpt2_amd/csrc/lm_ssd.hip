@@ -356,7 +356,15 @@ __global__ __launch_bounds__(256, 2) void ssd_chunk_out_kernel(const SsdArgs a, 
 // ------------------------------------------------------------------------------------------------ norm in parts, polynomial activation
 constexpr int kPartRegs = 16;  // parts of up to 256 * kPartRegs channels stay in registers
 
-__global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int width, int parts, const float* w, float eps, const ConvArgs cv, const int* row_slot) {
+// a result in place, or rounded to bf16 in the twin of its array
+__device__ __forceinline__ void put_row(float* out, bf16_t* out16, size_t at, float v) {
+    if (out16) out16[at] = (bf16_t)cvt_pk_bf16(v, v);
+    else out[at] = v;
+}
+
+
+__global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int width, int parts, const float* w, float eps, const ConvArgs cv, const int* row_slot,
+                                                        bf16_t* out16) {
     __shared__ float s_red[8];
     const int m = blockIdx.x, part = blockIdx.y, n = width / parts;
     if (part >= parts) {  // the row is its entry's only one: the workgroups behind the parts move the convolution's tail on, 256 channels each
@@ -371,7 +379,8 @@ __global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int wi
         }
         return;
     }
-    float* p = v + (size_t)m * ld + (size_t)part * n;
+    const size_t at = (size_t)m * ld + (size_t)part * n;
+    float* p = v + at;
     const float* wp = w + (size_t)part * n;
     if (n <= 256 * kPartRegs) {
         float x[kPartRegs], wr[kPartRegs], ss = 0.0f;
@@ -387,7 +396,7 @@ __global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int wi
 #pragma unroll
         for (int j = 0; j < kPartRegs; ++j) {
             const int i = threadIdx.x + 256 * j;
-            if (i < n) p[i] = x[j] * rn * wr[j];
+            if (i < n) put_row(v, out16, at + i, x[j] * rn * wr[j]);
         }
         return;
     }
@@ -395,12 +404,13 @@ __global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int wi
     for (int i = threadIdx.x; i < n; i += 256) ss = fmaf(p[i], p[i], ss);
     ss = block_allsum(ss, s_red);
     const float rn = 1.0f / sqrtf(ss / (float)n + eps);
-    for (int i = threadIdx.x; i < n; i += 256) p[i] = p[i] * rn * wp[i];
+    for (int i = threadIdx.x; i < n; i += 256) put_row(v, out16, at + i, p[i] * rn * wp[i]);
 }
 
-__global__ __launch_bounds__(256) void polynorm_kernel(float* z, int ld, int F, const float* act, float eps) {
+__global__ __launch_bounds__(256) void polynorm_kernel(float* z, int ld, int F, const float* act, float eps, bf16_t* out16) {
     __shared__ float s_red[3][4];
-    float* p = z + (size_t)blockIdx.x * ld;
+    const size_t at = (size_t)blockIdx.x * ld;
+    float* p = z + at;
     const float ca = act[0], cb = act[1], cc = act[2], ce = act[3];
     float x[kPartRegs], s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
     const bool held = F <= 256 * kPartRegs;
@@ -441,10 +451,10 @@ __global__ __launch_bounds__(256) void polynorm_kernel(float* z, int ld, int F, 
 #pragma unroll
         for (int j = 0; j < kPartRegs; ++j) {
             const int i = threadIdx.x + 256 * j;
-            if (i < F) p[i] = fmaf(fmaf(fmaf(f3, x[j], f2), x[j], f1), x[j], ce);
+            if (i < F) put_row(z, out16, at + i, fmaf(fmaf(fmaf(f3, x[j], f2), x[j], f1), x[j], ce));
         }
     } else {
-        for (int i = threadIdx.x; i < F; i += 256) p[i] = fmaf(fmaf(fmaf(f3, p[i], f2), p[i], f1), p[i], ce);
+        for (int i = threadIdx.x; i < F; i += 256) put_row(z, out16, at + i, fmaf(fmaf(fmaf(f3, p[i], f2), p[i], f1), p[i], ce));
     }
 }
 
@@ -495,19 +505,20 @@ int launch_ssd_scan(const SsdArgs& a, const ConvArgs* conv, int M, const int* en
     return ZG_OK;
 }
 
-int launch_part_norm(float* v, int ld, int width, int parts, int M, const float* w, float eps, const ConvArgs* conv, const int* row_slot, hipStream_t s) {
+int launch_part_norm(float* v, int ld, int width, int parts, int M, const float* w, float eps, const ConvArgs* conv, const int* row_slot, hipStream_t s,
+                     bf16_t* out16) {
     if (M <= 0 || width <= 0) return ZG_OK;
     ZG_REQUIRE(parts >= 1 && parts <= 65535 && width % parts == 0, ZG_ERR_ARG, "norm in parts: %d channels in %d parts", width, parts);
     ZG_REQUIRE(!conv || (conv->taps >= 1 && conv->taps <= kSsdTaps), ZG_ERR_ARG, "norm in parts: a convolution of more than %d taps", kSsdTaps);
     const int tail_blocks = conv && conv->taps > 1 ? (conv->C + 255) / 256 : 0;
-    part_norm_kernel<<<dim3(M, parts + tail_blocks), 256, 0, s>>>(v, ld, width, parts, w, eps, conv ? *conv : ConvArgs(), row_slot);
+    part_norm_kernel<<<dim3(M, parts + tail_blocks), 256, 0, s>>>(v, ld, width, parts, w, eps, conv ? *conv : ConvArgs(), row_slot, out16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
-int launch_polynorm(float* z, int ld, int F, int M, const float* act, float eps, hipStream_t s) {
+int launch_polynorm(float* z, int ld, int F, int M, const float* act, float eps, hipStream_t s, bf16_t* out16) {
     if (M <= 0 || F <= 0) return ZG_OK;
-    polynorm_kernel<<<M, 256, 0, s>>>(z, ld, F, act, eps);
+    polynorm_kernel<<<M, 256, 0, s>>>(z, ld, F, act, eps, out16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
