@@ -104,6 +104,41 @@ def test_latent_tiles(kv_rank, rot_dim):
     m.close()
 
 
+@pytest.mark.parametrize("bad", [None, np.inf, np.nan])
+@pytest.mark.parametrize("kv_rank,rot_dim", [(64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])
+def test_latent_tiles_32_bit(kv_rank, rot_dim, bad):
+    """The same in 32-bit mode; a token that is not finite leaves the rows in front of it alone, also those of its own tile of keys."""
+    cfg = tl.config([tl.latent_layer(heads=5, dim=16, vdim=16, rot_dim=rot_dim, rot_dims=rot_dim, kv_rank=kv_rank, q_rank=40, mlp=tl.dense_mlp(ff=96))],
+                    vocab=203, width=64)
+    w = tl.weights(cfg, seed=kv_rank)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(80 + b, n, cfg["vocab"]) for b, n in enumerate((150, 97, 66))]
+    for t in toks:
+        t[t == 7] = 8
+    refs = [oracle.forward(t)[0] for t in toks]
+    ends = [150, 97, 66]  # rows of each sequence that stay as they are
+    if bad is not None:
+        for b, at in enumerate((141, 35, 64)):
+            toks[b][at] = 7
+            ends[b] = at
+        w["embed"] = w["embed"].copy()
+        w["embed"][7, 3] = bad
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=512, max_seqs=3)
+    m.load_weights(w)
+    seqs = [m.open() for _ in toks]
+    lo = [0, 0, 0]
+    for hi in ((33, 1, 31), (64, 96, 33), (150, 97, 66)):
+        got = m.step([(s, t[a:b], list(range(b - a))) for s, t, a, b in zip(seqs, toks, lo, hi)])
+        parts = np.split(got, np.cumsum([b - a for a, b in zip(lo, hi)])[:-1])
+        for part, ref, a, b, end in zip(parts, refs, lo, hi, ends):
+            n = min(b, end) - a
+            if n > 0:
+                tl.assert_close(part[:n], ref[a:a + n], "float32", (kv_rank, bad, a, b))
+            assert not np.isfinite(part[max(n, 0):]).all(axis=1).any()
+        lo = hi
+    m.close()
+
+
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("rows", [3, 4, 5, 8])
 def test_rows_of_decode_steps(rows, dtype):

@@ -1286,6 +1286,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
                                                      g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
                                                      L.sink, qa16, ctx16));
+            if (f32 && !few)
+                ZG_TRY(launch_latent_attention_f32(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
+                                                   g->max_pages, g->P, ps.cache, s, &tiled, gate, LD, L.sink));
             ZG_REQUIRE(tiled || !tiles, ZG_ERR_UNSUPPORTED, "latent attention: the tiles do not fit their workspace");
             if (!tiled)
                 ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,

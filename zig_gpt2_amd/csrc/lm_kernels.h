@@ -253,6 +253,9 @@ int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, 
 // gate != null: head h's result is multiplied by sigmoid(gate[m ldg + h]).
 // sink != null: exp(sink[h]) is added to head h's denominator, once.
 constexpr int kAttnSplits = 16;
+int launch_latent_attention_f32(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
+                                const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
+                                const float* cache, hipStream_t s, bool* taken, const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);
 int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* row_pos, const int* row_slot,
                             const int* page_table, int max_pages, int page_tokens, const float* cache, float* ws, size_t ws_floats, hipStream_t s,
                             const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);

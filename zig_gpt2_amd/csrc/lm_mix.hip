@@ -970,17 +970,21 @@ struct KeyTile {
 constexpr int kLog2eBits = 0x3fb8aa3b;  // log2(e)
 
 // Entries of a step, one per lane (64 at a time): the rows of entry e cut into blocks of 32 queries, its cached rows (this step's
-// included) into tiles of 32 keys.  Finds the entry of query block `id` and the key tiles of the entries in front of it.
+// included) into tiles of 32 keys.  Finds the entry of query block `id` (of BQ queries) and the key tiles of the entries in front of it.
+// Everything the caller needs of the entry comes out of the same two loads, in front of the scan.
 struct EntryAt {
-    int e, block, first_tile;
+    int block, first_tile;
+    int start, len, pos, slot;  // of the entry: first row, rows, position of the first row, cache slot
 };
-__device__ __forceinline__ bool find_entry(int id, const int* ent_start, const int* ent_len, int n_entries, const int* row_pos, EntryAt& at) {
+template <int BQ = 32>
+__device__ __forceinline__ bool find_entry(int id, const int* ent_start, const int* ent_len, const int* ent_slot, int n_entries, const int* row_pos, EntryAt& at) {
     const int lane = threadIdx.x & 63;
     int tiles_before = 0;
     for (int e0 = 0; e0 < n_entries; e0 += 64) {
         const int e = min(e0 + lane, n_entries - 1);
-        const int len = e0 + lane < n_entries ? ent_len[e] : 0;
-        const int blocks = (len + 31) / 32, tiles = len > 0 ? (row_pos[ent_start[e] + len - 1] + 32) / 32 : 0;
+        const int len = e0 + lane < n_entries ? ent_len[e] : 0, start = ent_start[e], slot = ent_slot[e];
+        const int pos = len > 0 ? row_pos[start] : 0;
+        const int blocks = (len + BQ - 1) / BQ, tiles = len > 0 ? (pos + len + 31) / 32 : 0;
         int b = blocks, t = tiles;
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
@@ -993,7 +997,10 @@ __device__ __forceinline__ bool find_entry(int id, const int* ent_start, const i
         const unsigned long long past = __ballot(id < b);
         if (past) {
             const int l = __builtin_ctzll(past);
-            at.e = e0 + l;
+            at.start = __builtin_amdgcn_readlane(start, l);
+            at.len = __builtin_amdgcn_readlane(len, l);
+            at.pos = __builtin_amdgcn_readlane(pos, l);
+            at.slot = __builtin_amdgcn_readlane(slot, l);
             at.block = id - __builtin_amdgcn_readlane(b - blocks, l);
             at.first_tile = tiles_before + __builtin_amdgcn_readlane(t - tiles, l);
             return true;
@@ -1062,19 +1069,19 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
 // converted and transposed its own tiles behind three barriers.
 template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
 __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, const bf16_t* qa16, float* ctx, bf16_t* ctx16, int H, int KR, int R, float scale,
-                                                                       const int* ent_start, const int* ent_len, int n_entries, const int* row_pos,
+                                                                       const int* ent_start, const int* ent_len, const int* ent_slot, int n_entries, const int* row_pos,
                                                                        const bf16_t* tiles, const float* gate, int ldg, const float* sink) {
     typedef KeyTile<NKS> T;
     static_assert(NT * 32 <= T::DT, "the latent part lies inside the rows");
     __shared__ __attribute__((aligned(1024))) char Ks[2][T::BYTES];
     EntryAt at;
-    if (!find_entry(gridDim.x - 1 - blockIdx.x, ent_start, ent_len, n_entries, row_pos, at)) return;
+    if (!find_entry(gridDim.x - 1 - blockIdx.x, ent_start, ent_len, ent_slot, n_entries, row_pos, at)) return;
     const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int h = blockIdx.y * 4 + wave;
     const bool head_ok = h < H;
-    const int m_first = ent_start[at.e] + at.block * 32, nq = min(32, ent_len[at.e] - at.block * 32);
-    const int pos_first = row_pos[m_first], qpos = pos_first + r, DT = KR + R;
+    const int m_first = at.start + at.block * 32, nq = min(32, at.len - at.block * 32);
+    const int pos_first = at.pos + at.block * 32, qpos = pos_first + r, DT = KR + R;
     const int n_tiles = (pos_first + nq + 31) / 32;
     const char* src = reinterpret_cast<const char*>(tiles) + (size_t)at.first_tile * T::BYTES + lane * 16;
 
@@ -1241,6 +1248,170 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
                     if (d + u < KR) out[d + u] = v[u];
             }
         }
+}
+
+// Prompt portions in 32-bit mode: the same attention on the matrix cores' fp32 products.  A workgroup takes 16 consecutive queries of one
+// entry and one head; its four waves take every fourth tile of 16 keys and are merged at the end.  Transposed as above (S^T = K Q^T,
+// O^T = C^T P^T): a lane's column is a query, and its four probabilities are the four it has to feed back.  Which of the 16 dimensions of
+// a piece a lane group multiplies is free as long as both operands agree, so that every load is 16 bytes: four consecutive dimensions of
+// a key for the scores; for the latent part four consecutive dimensions of one of the lane group's own keys, a row of four result tiles.
+// Keys go from the cache to registers (18 loads of 16 bytes a tile and 16 for the latent part, 34 KB against 4.3 k cycles of products: what
+// a compute unit can take in beside them); the latent part of a tile is requested piece by piece under its scores, the next tile's keys
+// under this tile's sums.  A masked key must not reach the sums as 0 x infinity: the tiles on the diagonal look whether a value is not
+// finite, and then add key by key.
+// 333 tokens, 12 heads on latents of 256 + 32: 31 us against 118.8 with a wave per key row and its dimensions over the lanes.
+template <int NKS, int NV, bool EXACT>  // 16 NKS >= KR + R (score dimensions), 64 NV >= KR (latent dimensions); EXACT: equal
+__global__ __launch_bounds__(256, EXACT && NKS <= 18 ? 2 : 1) void latent_attention_f32_kernel(const float* qa, float* ctx, int H, int KR, int R, float scale,
+    const int* ent_start, const int* ent_len, const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages,
+    int page_tokens, const float* cache, const float* gate, int ldg, const float* sink) {
+    static_assert(4 * NV <= NKS, "the latent part is requested under the scores");
+    constexpr int LDO = NV * 64 + 4;
+    __shared__ __attribute__((aligned(16))) float s_o[2][16][LDO];
+    __shared__ f32x4 s_q[NKS][64];
+    __shared__ float s_m[4][16], s_l[4][16];
+    EntryAt at;
+    if (!find_entry<16>(gridDim.x - 1 - blockIdx.x, ent_start, ent_len, ent_slot, n_entries, row_pos, at)) return;
+    const int tid = threadIdx.x, lane = tid & 63, q = lane & 15, g = lane >> 4, h = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m_first = at.start + at.block * 16, nq = min(16, at.len - at.block * 16), DT = KR + R;
+    const int pos_first = at.pos + at.block * 16, qpos = pos_first + q, n_keys = pos_first + nq, n_tiles = (n_keys + 15) / 16;
+    const int* pt = page_table + (size_t)at.slot * max_pages;
+    // piece c of a row of scores, of the latent part: where they end inside the last pieces, some valid piece (zeroed, never stored)
+    auto k_at = [&](int c) { return EXACT ? c * 16 + g * 4 : min(c * 16 + g * 4, DT - 4); };
+    auto v_at = [&](int d) { return EXACT ? d : min(d, KR - 4); };
+    auto row_of = [&](int tile) {  // cache row of key 16 tile + q
+        const int key = min(tile * 16 + q, n_keys - 1);
+        return pt[key / page_tokens] * page_tokens + key % page_tokens;
+    };
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 kf[NKS], vf[4 * NV], acc[4 * NV];
+    const float* qrow = qa + ((size_t)(m_first + min(q, nq - 1)) * H + h) * DT;
+    int row = row_of(min(wave, n_tiles - 1));
+    {
+        const float* kp = cache + (size_t)row * DT;
+#pragma unroll
+        for (int c = 0; c < NKS; ++c) kf[c] = *reinterpret_cast<const f32x4*>(kp + k_at(c));
+    }
+    for (int c = wave; c < NKS; c += 4) {
+        const f32x4 v = *reinterpret_cast<const f32x4*>(qrow + k_at(c));
+        s_q[c][lane] = EXACT || c * 16 + g * 4 < DT ? v : zero;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4 * NV; ++i) acc[i] = zero;
+    float mx = -INFINITY, l = 0.0f;
+    for (int kt = wave; kt < n_tiles; kt += 4) {
+        const float* vp[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) vp[i] = cache + (size_t)__shfl(row, g * 4 + i, 64) * DT;
+        const int next_row = row_of(min(kt + 4, n_tiles - 1));
+        f32x4 s0 = zero, s1 = zero, qn = s_q[0][lane];
+#pragma unroll
+        for (int c = 0; c < NKS; ++c) {
+            if (c < 4 * NV) vf[c] = *reinterpret_cast<const f32x4*>(vp[c / NV] + v_at((c % NV) * 64 + q * 4));
+            const f32x4 k = EXACT || c * 16 + g * 4 < DT ? kf[c] : zero, qc = qn;
+            qn = s_q[c + 1 < NKS ? c + 1 : 0][lane];
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k.x, qc.x, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k.y, qc.y, s1, 0, 0, 0);
+            s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(k.z, qc.z, s0, 0, 0, 0);
+            s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(k.w, qc.w, s1, 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const int key0 = kt * 16 + g * 4;
+        float p[4], top = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            p[i] = key0 + i <= qpos ? (s0[i] + s1[i]) * scale : -INFINITY;
+            top = fmaxf(top, p[i]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 16, 64));
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        const float mn = fmaxf(mx, top), base = mn == -INFINITY ? 0.0f : mn;  // (no key of the tile, and none before, is this query's)
+        const float alpha = expf(mx - base);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) p[i] = expf(p[i] - base);
+        l = l * alpha + ((p[0] + p[1]) + (p[2] + p[3]));
+        mx = mn;
+#pragma unroll
+        for (int i = 0; i < 4 * NV; ++i) acc[i] *= alpha;
+        bool by_key = false;
+        if (kt * 16 + 15 > pos_first) {  // (uniform) some query of the block does not see the whole tile
+            float z = 0.0f;
+#pragma unroll
+            for (int j = 0; j < 4 * NV; ++j) z += (vf[j].x * 0.0f + vf[j].y * 0.0f) + (vf[j].z * 0.0f + vf[j].w * 0.0f);
+            by_key = __any(!(z == 0.0f));
+        }
+        const float* kp = cache + (size_t)next_row * DT;
+        if (__builtin_expect(by_key, 0)) {
+#pragma unroll 1
+            for (int j = 0; j < 4; ++j) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float pj = __shfl(p[i], j * 16 + q, 64);
+                    const float* v = cache + (size_t)__shfl(row, j * 4 + i, 64) * DT;
+                    const bool seen = kt * 16 + j * 4 + i <= qpos;
+#pragma unroll
+                    for (int b = 0; b < 4 * NV; ++b) {  // the four dimensions of result row 4 g + b % 4
+                        const f32x4 x = *reinterpret_cast<const f32x4*>(v + v_at((b >> 2) * 64 + g * 16 + (b & 3) * 4));
+#pragma unroll
+                        for (int t = 0; t < 4; ++t)
+                            acc[(b >> 2) * 4 + t][b & 3] = seen ? fmaf(pj, x[t], acc[(b >> 2) * 4 + t][b & 3]) : acc[(b >> 2) * 4 + t][b & 3];
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                }
+            }
+#pragma unroll
+            for (int b = 0; b < 4 * NV; ++b) vf[b] = zero;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[i] = 0.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < NKS; ++j) {
+            kf[j] = *reinterpret_cast<const f32x4*>(kp + k_at(j));
+            if (j < 4 * NV) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    acc[(j % NV) * 4 + t] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[j][t], p[j / NV], acc[(j % NV) * 4 + t], 0, 0, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        row = next_row;
+    }
+    l += __shfl_xor(l, 16, 64);
+    l += __shfl_xor(l, 32, 64);
+    if (g == 0) {
+        s_m[wave][q] = mx;
+        s_l[wave][q] = l;
+    }
+    __syncthreads();
+    const float top = fmaxf(fmaxf(s_m[0][q], s_m[1][q]), fmaxf(s_m[2][q], s_m[3][q]));
+    const float w = top == -INFINITY ? 0.0f : expf(mx - top);  // (a wave without keys: 0)
+#pragma unroll
+    for (int i = 0; i < 4 * NV; ++i) acc[i] *= w;
+    for (int half = 1; half >= 0; --half) {  // waves 2 and 3 leave their sums, waves 0 and 1 add theirs
+        if (wave >> 1 == half) {
+#pragma unroll
+            for (int b = 0; b < 4 * NV; ++b) {
+                f32x4* o = reinterpret_cast<f32x4*>(&s_o[wave & 1][q][(b >> 2) * 64 + g * 16 + (b & 3) * 4]);
+                f32x4 v;
+#pragma unroll
+                for (int t = 0; t < 4; ++t) v[t] = acc[(b >> 2) * 4 + t][b & 3];
+                *o = half ? v : *o + v;
+            }
+        }
+        __syncthreads();
+    }
+    for (int i = tid; i < 16 * (KR >> 2); i += 256) {
+        const int qi = i / (KR >> 2), d = (i - qi * (KR >> 2)) * 4;
+        if (qi >= nq) break;
+        float mq = fmaxf(fmaxf(s_m[0][qi], s_m[1][qi]), fmaxf(s_m[2][qi], s_m[3][qi])), L = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) L += (mq == -INFINITY ? 0.0f : expf(s_m[k][qi] - mq)) * s_l[k][qi];
+        const size_t m = m_first + qi;
+        const float gf = head_gate_f(gate, ldg, m, h) * (sink ? sink_norm_f(mq, L, sink, h) : 1.0f / L);
+        const f32x4 v = *reinterpret_cast<const f32x4*>(&s_o[0][qi][d]) + *reinterpret_cast<const f32x4*>(&s_o[1][qi][d]);
+        *reinterpret_cast<f32x4*>(ctx + (m * H + h) * KR + d) = v * gf;
+    }
 }
 
 // ctx[m][h] from the partials of latent_attention_kernel, in a fixed order (the result does not depend on timing); only the
@@ -1590,7 +1761,7 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
         latent_tiles_kernel<NKS_><<<cgrid, 256, 0, s>>>(cache, KR + R, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, max_pages,      \
                                                         page_tokens, ws);                                                                            \
         ZG_HIP(hipGetLastError());                                                                                                                   \
-        latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, qa16, ctx, ctx16, H, KR, R, scale, ent_start, ent_len, n_entries, row_pos, ws, gate, ldg, \
+        latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, qa16, ctx, ctx16, H, KR, R, scale, ent_start, ent_len, ent_slot, n_entries, row_pos, ws, gate, ldg, \
                                                                      sink);                                                                          \
     } while (0)
     if (tile == KeyTile<6>::BYTES / 2) ZG_ATT_T(6, 2);
@@ -1598,6 +1769,33 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
     else if (tile == KeyTile<18>::BYTES / 2) ZG_ATT_T(18, 8);
     else ZG_ATT_T(24, 10);
 #undef ZG_ATT_T
+    ZG_HIP(hipGetLastError());
+    *taken = true;
+    return ZG_OK;
+}
+
+// Prompt portions in 32-bit mode.  (The general kernel stays for latents beyond the tiles and rows that are no whole 16-byte pieces.)
+int launch_latent_attention_f32(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* ent_start, const int* ent_len,
+                                const int* ent_slot, int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
+                                const float* cache, hipStream_t s, bool* taken, const float* gate, int ldg, const float* sink) {
+    *taken = false;
+    const size_t tile = latent_tile_elems(KR, R);
+    if (M <= 0 || n_entries <= 0 || tile == 0 || KR % 4 != 0 || R % 4 != 0 || H > 65535 ||
+        ((reinterpret_cast<uintptr_t>(qa) | reinterpret_cast<uintptr_t>(ctx) | reinterpret_cast<uintptr_t>(cache)) & 15) != 0)
+        return ZG_OK;
+    const dim3 grid((M + 15) / 16 + n_entries, H);
+#define ZG_ATT_FX(NKS_, NV_, EXACT_)                                                                                                           \
+    latent_attention_f32_kernel<NKS_, NV_, EXACT_><<<grid, 256, 0, s>>>(qa, ctx, H, KR, R, scale, ent_start, ent_len, ent_slot, n_entries, row_pos, \
+                                                                        page_table, max_pages, page_tokens, cache, gate, ldg, sink)
+#define ZG_ATT_F(NKS_, NV_)                                                             \
+    if (KR + R == 16 * NKS_ && KR == 64 * NV_) ZG_ATT_FX(NKS_, NV_, true);              \
+    else ZG_ATT_FX(NKS_, NV_, false)
+    if (tile == KeyTile<6>::BYTES / 2) { ZG_ATT_F(6, 1); }
+    else if (tile == KeyTile<10>::BYTES / 2) { ZG_ATT_F(10, 2); }
+    else if (tile == KeyTile<18>::BYTES / 2) { ZG_ATT_F(18, 4); }
+    else { ZG_ATT_F(24, 5); }
+#undef ZG_ATT_F
+#undef ZG_ATT_FX
     ZG_HIP(hipGetLastError());
     *taken = true;
     return ZG_OK;
