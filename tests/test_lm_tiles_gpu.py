@@ -169,3 +169,22 @@ def test_rows_of_decode_steps(rows, dtype):
         for s in seqs:
             m.close_seq(s)
     m.close()
+
+
+@pytest.mark.parametrize("ff", [20, 100, 136])
+@pytest.mark.parametrize("rows", [3, 5, 8])
+def test_gated_rows_of_decode_steps(rows, ff):
+    """The experts' gated activation in the first product's epilogue: widths that end inside a workgroup's eight gates, and that the second
+    product cannot take in 16-byte pieces."""
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=ff, experts=9, top=3))], vocab=203, width=136)
+    w = tl.weights(cfg, seed=rows + ff)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(60 + b, 4, cfg["vocab"]) for b in range(rows)]
+    refs = [oracle.forward(t)[0] for t in toks]
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=512, max_seqs=8)
+    m.load_weights(w)
+    seqs = [m.open() for _ in toks]
+    for i in range(4):
+        got = m.step([(s, [t[i]], [0]) for s, t in zip(seqs, toks)])
+        tl.assert_close(got, np.stack([r[i] for r in refs]), "float32", (rows, ff, i))
+    m.close()

@@ -960,17 +960,19 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         const bool poly = L.d.dense_act == ZG_LM_DENSE_POLYNORM, gated = L.d.dense_act == ZG_LM_DENSE_GLU_GELU;
         Linear dn;
         bf16_t* const u16 = r16 && whole(F) ? g->u16 : nullptr;
+        bool activated = false;
         if (!first_done) {
             Linear up = dense_up(L, in, in16);
+            if (gated && few && M > 2) ZG_TRY(launch_linear_gated(up, F, GLU_GELU, g->hb, s, &activated));
             if (u16 && !poly && !gated && whole(W)) up.C16 = u16, up.C = nullptr;
-            ZG_TRY(launch_linear(up, f32, s));
+            if (!activated) ZG_TRY(launch_linear(up, f32, s));
         }
         if (gated) {  // rows gate | up
             dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
             if (M <= 2) {  // the activation where the second product reads its rows (more rows: every workgroup would redo it)
                 dn.A = g->u; dn.lda = L.n_up; dn.a_glu = F; dn.glu_kind = GLU_GELU;
             } else {
-                ZG_TRY(launch_glu(g->u, g->hb, M, F, s, GLU_GELU, 0, -1, u16));
+                if (!activated) ZG_TRY(launch_glu(g->u, g->hb, M, F, s, GLU_GELU, 0, -1, u16));
                 dn.A = u16 ? nullptr : g->hb; dn.A16 = u16; dn.lda = F;
             }
             return launch_linear(dn, f32, s);
@@ -984,6 +986,24 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         const bool u_r16 = u16 && (poly || whole(W));
         dn.A = u_r16 ? nullptr : g->u; dn.A16 = u_r16 ? u16 : nullptr; dn.lda = F; dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
         return launch_linear(dn, f32, s);
+    };
+    // the chosen experts' first product, and what their second one reads (glu: rows gate | up, gated by silu)
+    auto expert_first = [&](const Linear& up, Linear& dn, int F, int NA, bool glu) -> int {
+        bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
+        bool gated = false;
+        if (glu && few) ZG_TRY(launch_linear_gated(up, F, GLU_SILU, g->hb, s, &gated));
+        if (!gated) ZG_TRY(launch_linear(up, f32, s));
+        if (!glu) {  // the first product's epilogue has applied its activation
+            dn.A = g->gu_buf; dn.lda = F;
+            return ZG_OK;
+        }
+        if (!gated && few) {  // the activation is applied where the second product reads its rows
+            dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
+            return ZG_OK;
+        }
+        if (!gated) ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
+        dn.A = hb16 ? nullptr : g->hb; dn.A16 = hb16; dn.lda = F;
+        return ZG_OK;
     };
     // one-row steps of side-by-side sublayers: the dense feed-forward's first product rides in the launch of the mixer's first
     const LayerW* up_done = nullptr;
@@ -1355,16 +1375,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                     ZG_TRY(copy_trace(p));
                     continue;
                 }
-                ZG_TRY(launch_linear(up, f32, s));
-                if (!glu) {  // the first product's epilogue has applied the activation
-                    dn.A = g->gu_buf; dn.lda = F;
-                } else if (few) {  // the gated activation is applied where the second product reads its rows
-                    dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
-                } else {
-                    bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
-                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
-                    if (hb16) dn.A = nullptr, dn.A16 = hb16;
-                }
+                ZG_TRY(expert_first(up, dn, F, NA, glu));
                 ZG_TRY(launch_linear(dn, f32, s));
                 if (d.shared_width > 0) {  // the expert every token uses
                     const int S = d.shared_width;
@@ -1424,17 +1435,15 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                     sup.M = 1; sup.nz = M; sup.N = 2 * S + (sg_col >= 0 ? 1 : 0); sup.K = W;
                     ZG_TRY(launch_linear_pair(up, sup, f32, s));
                 } else {
-                    ZG_TRY(launch_linear(up, f32, s));
+                    if (silu) ZG_TRY(expert_first(up, dn, F, NA, true));
+                    else ZG_TRY(launch_linear(up, f32, s));
                 }
                 // (the product is linear: the score that multiplies an expert's input is applied to the product, in front of the clip)
                 if (d.ff_act == ZG_LM_ACT_GELU) {
                     dn.A = g->gu_buf; dn.lda = F;
-                } else if (silu && few) {  // the activation is applied where the second product reads its rows
+                } else if (silu && paired) {  // the activation is applied where the second product reads its rows
                     dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
                 } else if (silu) {
-                    bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
-                    ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
-                    if (hb16) dn.A = nullptr, dn.A16 = hb16;
                 } else if (few) {  // the activation is applied where the second product reads its rows
                     dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F; dn.glu_kind = GLU_CLIPPED; dn.glu_limit = d.ff_limit;
                     dn.glu_scale = on_input ? g->wt : nullptr;
@@ -1542,16 +1551,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 ZG_TRY(launch_group(g->pick, NA, E, g->grp_off, g->sorted, g->inv, s));
                 up.M = dn.M = NA; up.a_rows = g->sorted; up.grp_off = dn.grp_off = g->grp_off; up.n_groups = dn.n_groups = E;
             }
-            ZG_TRY(launch_linear(up, f32, s));
-            if (!glu) {  // the first product's epilogue has applied the activation
-                dn.A = g->gu_buf; dn.lda = F;
-            } else if (few) {  // the gated activation is applied where the second product reads its rows
-                dn.A = g->gu_buf; dn.lda = 2 * F; dn.a_glu = F;
-            } else {
-                bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
-                ZG_TRY(launch_glu(g->gu_buf, g->hb, NA, F, s, GLU_SILU, 0, -1, hb16));
-                if (hb16) dn.A = nullptr, dn.A16 = hb16;
-            }
+            ZG_TRY(expert_first(up, dn, F, NA, glu));
             ZG_TRY(launch_linear(dn, f32, s));
             if (few) ZG_TRY(tail(nullptr, g->ye, g->wt, top, L.norm2b));
             if (!h_ready) ZG_TRY(launch_moe_combine(g->x, g->ye, few ? nullptr : g->inv, g->wt, top, L.norm2b, eps, M, W, s));

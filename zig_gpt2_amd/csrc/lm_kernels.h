@@ -59,7 +59,11 @@ struct Linear {
     int z_limit = 0x7fffffff;  // batches whose z_group is not below it are skipped, their rows of C left alone (row-vector kernels)
     const int* grp_off = nullptr;
     int n_groups = 0;
+    int glu_out = 0;  // set by launch_linear_gated: B rows are [gate (glu_out) | up (glu_out)], N both, and the activated rows leave (glu_kind)
 };
+// Steps of few rows: the first product of a gated feed-forward with the activation in its epilogue, h [rows][F] = act(gate) * up for B rows
+// [gate (F) | up (F)]; L as for launch_linear, its C, ldc, c_zoff and N ignored.  *taken = false: not a form that has it, nothing launched.
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t s, bool* taken);
 // Picks the row-vector kernel (few rows: decode) or the tiled matrix-core kernel (prompt portions).
 int launch_linear(const Linear& L, bool f32, hipStream_t s);
 constexpr int kGemvMaxRows = 8;

@@ -908,6 +908,16 @@ int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
 }
 }  // namespace
 
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t s, bool* taken) {
+    *taken = false;
+    if (F <= 0 || L.act != ACT_NONE || L.bias || kind == GLU_CLIPPED || L.M <= 0 || L.M > kGemvMaxRows || L.grp_off || L.a_glu ||
+        getenv("ZGPT2_LM_NO_ROWS") != nullptr)
+        return ZG_OK;
+    Linear g = L;
+    g.N = 2 * F; g.glu_out = F; g.glu_kind = kind; g.C = h; g.C16 = nullptr; g.ldc = F; g.c_zoff = F;
+    return launch_rows(g, nullptr, s, taken);
+}
+
 int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     if (L.M <= 0 || L.N <= 0 || L.nz <= 0) return ZG_OK;
     const bool tiled = L.grp_off || L.M > kGemvMaxRows;

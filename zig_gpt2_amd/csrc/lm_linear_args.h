@@ -35,6 +35,7 @@ struct LinArgs {
     float poly_eps;
     const bf16_t* A16;  // the same rows as bf16 (tiled kernels), or null
     bf16_t* C16;        // the result rounded to bf16, beside or instead of C (tiled kernels), or null
+    int glu_out;        // > 0: gated product (Linear::glu_out)
     int a_vec, b_vec;  // 16-byte loads allowed (alignment of base, leading dimension and batch offsets)
 };
 
@@ -103,7 +104,7 @@ inline LinArgs make_args(const Linear& L) {
     p.a_div = L.a_div; p.act = L.act; p.n_groups = L.grp_off ? L.n_groups : 0; p.a_glu = L.a_glu;
     p.act_a = L.act_a; p.act_b = L.act_b; p.bias = L.bias; p.z_limit = L.z_limit; p.glu_kind = L.glu_kind; p.glu_limit = L.glu_limit; p.glu_scale = L.glu_scale;
     p.glu_gate_col = L.glu_gate_col;
-    p.A16 = L.A16; p.C16 = L.C16;
+    p.A16 = L.A16; p.C16 = L.C16; p.glu_out = L.glu_out;
     p.a_poly = L.a_poly;
     p.poly_eps = L.poly_eps;
     p.a_vec = ((reinterpret_cast<uintptr_t>(L.A) & 15) == 0 && L.lda % 4 == 0 && L.a_zoff % 4 == 0) ? 1 : 0;
