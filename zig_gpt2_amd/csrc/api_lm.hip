@@ -915,10 +915,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     const int* d_off = g->meta + meta_row_off(g);
     const bool f32 = g->f32;
     const float eps = g->cfg.norm_eps;
+    // The residual stream.  In steps of one row it changes its place wherever a product does the sum and the norms in front of it itself:
+    // every workgroup of the product reads it, one writes the new one.  It ends where it began.
+    float *x = g->x, *x_other = g->hc;
     const bool few = M <= kGemvMaxRows;
     const bool canon = g->canon >= 1;
     const bool readd = (g->cfg.flags & ZG_LM_LOOP_READD) && g->cfg.loop_times > 1;
-    ZG_TRY(launch_embed(g->embed, d_ids, g->x, readd ? g->x0 : nullptr, g->embed_scale, M, W, g->V, g->flag, d_pos, g->pos_freq, s));
+    ZG_TRY(launch_embed(g->embed, d_ids, x, readd ? g->x0 : nullptr, g->embed_scale, M, W, g->V, g->flag, d_pos, g->pos_freq, s));
     const bool side = g->side;
     const bool tnorm = g->tanh_norms;
     // Prompt portions in bf16 mode: what only matrix products read travels rounded to bf16, from the kernel that writes it, where its rows
@@ -930,7 +933,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     OpenSums pend;
     auto copy_trace = [&](int p) -> int {
         if (g->trace && !capturing && (size_t)(p + 1) * M * W <= g->trace_floats) {
-            ZG_HIP(hipMemcpyAsync(g->trace + (size_t)p * M * W, g->x, (size_t)M * W * sizeof(float), hipMemcpyDeviceToHost, s));
+            ZG_HIP(hipMemcpyAsync(g->trace + (size_t)p * M * W, x, (size_t)M * W * sizeof(float), hipMemcpyDeviceToHost, s));
             ZG_HIP(hipStreamSynchronize(s));
         }
         return ZG_OK;
@@ -947,6 +950,38 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     auto whole_context_keys = [&](bool replayed) {
         const int all_keys = g->max_pages * g->P;
         return replayed ? (g->bucket_keys > 0 ? g->bucket_keys : all_keys) : std::min(all_keys, (g->step_keys + 63) / 64 * 64);
+    };
+    // a sum and two norms in front of the sublayer that is about to run, not yet launched (one row; its first product may do them)
+    const bool defer = M == 1 && g->no_shift && !side && !tnorm && !canon && !(g->trace && !capturing);
+    NormIn open;
+    auto close_norm = [&]() -> int {
+        if (!open.x) return ZG_OK;
+        ZG_TRY(launch_norm_add_norm(x, open.y, open.wb, open.wn, eps, g->h, M, W, s));
+        open = NormIn();
+        return ZG_OK;
+    };
+    // the first product of a sublayer, whose rows are the normed ones
+    auto hidden_product = [&](const Linear& lin) -> int {
+        if (open.x) {
+            bool taken = false;
+            ZG_TRY(launch_linear_normed(lin, open, s, &taken));
+            if (taken) {
+                open = NormIn();
+                std::swap(x, x_other);
+                return ZG_OK;
+            }
+            ZG_TRY(close_norm());
+        }
+        return launch_linear(lin, f32, s);
+    };
+    auto defer_norm = [&](const float* y, const float* wb, const float* wn) {
+        open.x = x; open.y = y; open.wb = wb; open.wn = wn; open.x_out = x_other; open.eps = eps;
+    };
+    auto add_normed = [&](int p, const float* w) -> int {  // x += norm(y) (1 + w); the last sum goes where the stream began
+        float* const out = p + 1 == g->n_passes ? g->x : x;
+        ZG_TRY(launch_norm_add(x, out, g->y, w, eps, M, W, s));
+        x = out;
+        return ZG_OK;
     };
     // the dense feed-forward of a layer: in -> out (first_done: its first product has been launched)
     auto dense_up = [&](const LayerW& L, const float* in, const bf16_t* in16) {
@@ -965,7 +1000,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             Linear up = dense_up(L, in, in16);
             if (gated && few && M > 2) ZG_TRY(launch_linear_gated(up, F, GLU_GELU, g->hb, s, &activated));
             if (u16 && !poly && !gated && whole(W)) up.C16 = u16, up.C = nullptr;
-            if (!activated) ZG_TRY(launch_linear(up, f32, s));
+            if (!activated) ZG_TRY(hidden_product(up));
         }
         if (gated) {  // rows gate | up
             dn.B = L.down; dn.ldb = F; dn.C = out; dn.ldc = W; dn.M = M; dn.N = W; dn.K = F;
@@ -1008,13 +1043,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     // one-row steps of side-by-side sublayers: the dense feed-forward's first product rides in the launch of the mixer's first
     const LayerW* up_done = nullptr;
     auto first_product = [&](const LayerW& L, const Linear& lin) -> int {
-        if (!(side && M == 1 && L.d.ff == ZG_LM_FF_DENSE)) return launch_linear(lin, f32, s);
+        if (!(side && M == 1 && L.d.ff == ZG_LM_FF_DENSE)) return hidden_product(lin);
         up_done = &L;
         return launch_linear_pair(lin, dense_up(L, g->hc, nullptr), f32, s);
     };
     bool h_ready = false;  // g->h already holds this pass's shifted norm (written by the previous pass's fused tail)
     if (tnorm) {  // the norm behind the embedding (in place) and the first pass's norm; every later one rides behind a sublayer's sum
-        ZG_TRY(launch_tanh_norm(g->x, g->embed_norm, g->layers[g->passes[0].layer].norm1, nullptr, g->h, M, W, s));
+        ZG_TRY(launch_tanh_norm(x, g->embed_norm, g->layers[g->passes[0].layer].norm1, nullptr, g->h, M, W, s));
         h_ready = true;
     }
     for (int p = 0; p < g->n_passes; ++p) {
@@ -1024,17 +1059,17 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         const int H = d.heads, D = d.dim, Vd = d.vdim;
         bool hc_ready = false;  // one launch has done everything up to the mixer's input (decode steps)
         if (side) {  // what the layer before left open, and both norms of this layer from one statistic
-            ZG_TRY(launch_norm_two(g->x, pend, L.norm1, d.ff != ZG_LM_FF_NONE ? L.norm2 : nullptr, eps, h_r16 ? nullptr : g->h,
+            ZG_TRY(launch_norm_two(x, pend, L.norm1, d.ff != ZG_LM_FF_NONE ? L.norm2 : nullptr, eps, h_r16 ? nullptr : g->h,
                                    h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->hc, M, W, s, h_r16 ? g->h16 : nullptr, h_r16 ? g->hc16 : nullptr));
             pend = OpenSums();
             h_ready = true;
         }
         if (canon && single && !h_ready)
-            ZG_TRY(launch_norm_conv_single(g->x, ps.readd ? g->x0 : nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, L.norm1, eps, M, W, g->canon,
+            ZG_TRY(launch_norm_conv_single(x, ps.readd ? g->x0 : nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, L.norm1, eps, M, W, g->canon,
                                            L.canon1, g->seq_state + ps.canon1_off, g->seq_floats, d_slot, g->hc, s, &hc_ready));
-        if (ps.readd && !hc_ready) ZG_TRY(launch_add_rows(g->x, g->x0, M, W, s));
+        if (ps.readd && !hc_ready) ZG_TRY(launch_add_rows(x, g->x0, M, W, s));
         if (!h_ready && !hc_ready)
-            ZG_TRY(launch_norm_shift(g->x, L.norm1, canon ? nullptr : L.shift, eps, h_r16 ? nullptr : g->h, M, W, d_prev, d_slot, g->shift_state + (size_t)p * W,
+            ZG_TRY(launch_norm_shift(x, L.norm1, canon ? nullptr : L.shift, eps, h_r16 ? nullptr : g->h, M, W, d_prev, d_slot, g->shift_state + (size_t)p * W,
                                      (size_t)g->n_passes * W, canon || g->no_shift ? nullptr : d_last, g->last_h + (size_t)p * NS * W, s, h_r16 ? g->h16 : nullptr));
         h_ready = false;
         const float* hin = h_r16 ? nullptr : g->h;  // what the sublayer reads
@@ -1048,12 +1083,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             if (p + 1 >= g->n_passes || canon || g->passes[p + 1].readd) return ZG_OK;
             const LayerW& N = g->layers[g->passes[p + 1].layer];
             if (g->no_shift && y) {  // nothing of the token before: the same fusion at any number of rows
-                ZG_TRY(launch_norm_add_norm(g->x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
+                if (defer) defer_norm(y, wb, N.norm1);
+                else ZG_TRY(launch_norm_add_norm(x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
                 h_ready = true;
                 return ZG_OK;
             }
             if (!single || g->no_shift) return ZG_OK;
-            return launch_sum_norm_shift(g->x, y, yexp, weight, top, wb, N.norm1, N.shift, eps, g->h, M, W, d_slot, g->shift_state + (size_t)(p + 1) * W,
+            return launch_sum_norm_shift(x, y, yexp, weight, top, wb, N.norm1, N.shift, eps, g->h, M, W, d_slot, g->shift_state + (size_t)(p + 1) * W,
                                          (size_t)g->n_passes * W, d_last, g->last_h + (size_t)(p + 1) * NS * W, s, &h_ready);
         };
         Linear lin;
@@ -1103,7 +1139,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         } else if (d.mixer == ZG_LM_MIX_SSD) {
             const int G = d.kv_heads, HV = H * Vd, CC = HV + 2 * G * D, LD = L.ld_cat;
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = LD; lin.M = M; lin.N = L.n_cat; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             ConvArgs cv;
             cv.in = g->proj + HV; cv.ld_in = LD; cv.out = g->ta; cv.ld_out = CC; cv.C = CC; cv.taps = d.conv; cv.w = L.convw; cv.bias = L.convb;
             cv.flags = CONV_SILU; cv.tail = g->seq_state + ps.conv_off; cv.slot_stride = g->seq_floats;
@@ -1128,7 +1164,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int og = CC, orq = CC + HV, org = orq + 2 * HRD + HRV;  // columns of the left gate, the right q | k | v, the right gate
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             // left: biases and convolutions of q | k | v at once, the whole-projection norms, keys and values into the cache
             ConvArgs cv;
             cv.in = g->proj; cv.ld_in = NP; cv.out = g->ta; cv.ld_out = CC; cv.C = CC; cv.taps = std::max(1, d.conv); cv.w = L.convw;
@@ -1165,7 +1201,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const Rotary rot{L.rot_freq, d.rot_dims, 1.0f};
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             // left: attention inside the window
             ZG_TRY(launch_window_prep(g->proj, NP, M, H, G, D, Vd, rot, L.vfreq, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache, s));
             bool split = false;
@@ -1195,14 +1231,14 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             lin.A = g->td; lin.lda = C; lin.B = L.ro; lin.ldb = C; lin.C = g->y2; lin.ldc = W; lin.M = M; lin.N = W; lin.K = C;
             ZG_TRY(launch_linear(lin, f32, s));
             if (canon && single && d.ff != ZG_LM_FF_NONE)  // the branches' mean, the residual sum, the next norm and its convolution at once
-                ZG_TRY(launch_norm_conv_single(g->x, nullptr, g->y, g->y2, L.left_out, L.right_out, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
+                ZG_TRY(launch_norm_conv_single(x, nullptr, g->y, g->y2, L.left_out, L.right_out, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
                                                g->seq_state + ps.canon2_off, g->seq_floats, d_slot, g->hc, s, &mid_done));
             if (!mid_done) ZG_TRY(launch_pair_norm_mean(g->y, g->y2, L.left_out, L.right_out, eps, g->y, M, W, s));
         } else if (d.mixer == ZG_LM_MIX_CHANNEL_DELTA) {
             const int G = d.kv_heads, HV = H * Vd, CC = 2 * G * D + HV, RA = d.decay_rank, RG = d.gate_rank, NP = L.n_cat;
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             ConvArgs cv;
             cv.in = g->proj; cv.ld_in = NP; cv.out = g->ta; cv.ld_out = CC; cv.C = CC; cv.taps = d.conv; cv.w = L.convw; cv.flags = CONV_SILU;
             cv.tail = g->seq_state + ps.conv_off; cv.slot_stride = g->seq_floats;
@@ -1225,7 +1261,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int og = 2 * HD + HV, oa = og + HV;  // columns of the output gate and of the decay's first step
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             lin = Linear();  // the decay's second step
             lin.A = g->proj + oa; lin.lda = NP; lin.B = L.a2; lin.ldb = RA; lin.C = g->tb; lin.ldc = HD; lin.M = M; lin.N = HD; lin.K = RA;
             ZG_TRY(launch_linear(lin, f32, s));
@@ -1244,7 +1280,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             shape.slope = d.dist_bias ? L.slopes : nullptr;
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.wcat; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             ZG_TRY(launch_head_norm_prep(g->proj, NP, M, H, G, D, eps, d.qtemp_coef, d.qtemp_every, d_pos, d_slot, g->page_table, g->max_pages, g->P,
                                          ps.cache, s));
             const int key_cap = whole_context_keys(single || capturing);
@@ -1262,7 +1298,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const int HD = H * D, HV = H * Vd, NP = 2 * HD + HV;
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.qfv; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(hidden_product(lin));
             ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
                                      L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
             bf16_t* const o16 = r16 && whole(HV) ? g->o16 : nullptr;
@@ -1329,9 +1365,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             RoutePre pre;
             const bool pre_routed = few && d.ff == ZG_LM_FF_MOE && W <= kRouteFuseWidth;
             if (pre_routed) {
-                pre.x = g->x; pre.y = part; pre.nb = L.norm1b; pre.mult = g->res_mult; pre.nn = L.norm2; pre.h = g->h;
+                pre.x = x; pre.y = part; pre.nb = L.norm1b; pre.mult = g->res_mult; pre.nn = L.norm2; pre.h = g->h;
             } else {
-                ZG_TRY(launch_tanh_sum_norm(g->x, part, L.norm1b, g->res_mult, d.ff != ZG_LM_FF_NONE ? L.norm2 : next_norm, g->h, M, W, s));
+                ZG_TRY(launch_tanh_sum_norm(x, part, L.norm1b, g->res_mult, d.ff != ZG_LM_FF_NONE ? L.norm2 : next_norm, g->h, M, W, s));
             }
             const int F = d.ff_width;
             part = SumParts();
@@ -1370,7 +1406,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                     sdn.c_zoff = W; sdn.M = 1; sdn.nz = M; sdn.N = W; sdn.K = S;
                     ZG_TRY(launch_linear_pair(dn, sdn, f32, s));
                     part.b = g->td;
-                    ZG_TRY(launch_tanh_sum_norm(g->x, part, L.norm2b, g->res_mult, next_norm, g->h, M, W, s));
+                    ZG_TRY(launch_tanh_sum_norm(x, part, L.norm2b, g->res_mult, next_norm, g->h, M, W, s));
                     h_ready = next_norm != nullptr;
                     ZG_TRY(copy_trace(p));
                     continue;
@@ -1394,7 +1430,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                     part.b = g->td;
                 }
             }
-            if (d.ff != ZG_LM_FF_NONE) ZG_TRY(launch_tanh_sum_norm(g->x, part, L.norm2b, g->res_mult, next_norm, g->h, M, W, s));
+            if (d.ff != ZG_LM_FF_NONE) ZG_TRY(launch_tanh_sum_norm(x, part, L.norm2b, g->res_mult, next_norm, g->h, M, W, s));
             h_ready = next_norm != nullptr;
             ZG_TRY(copy_trace(p));
             continue;
@@ -1505,7 +1541,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 pend.sb = L.ls2;
             }
             if (p + 1 == g->n_passes || (g->trace && !capturing)) {  // nobody behind to add them (or the stream is to be shown): add now
-                ZG_TRY(launch_add_two(g->x, pend, M, W, s));
+                ZG_TRY(launch_add_two(x, pend, M, W, s));
                 pend = OpenSums();
             }
             ZG_TRY(copy_trace(p));
@@ -1513,14 +1549,15 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             continue;
         }
         if (canon && single && d.ff != ZG_LM_FF_NONE && !mid_done)
-            ZG_TRY(launch_norm_conv_single(g->x, nullptr, g->y, nullptr, nullptr, nullptr, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
+            ZG_TRY(launch_norm_conv_single(x, nullptr, g->y, nullptr, nullptr, nullptr, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
                                            g->seq_state + ps.canon2_off, g->seq_floats, d_slot, g->hc, s, &mid_done));
         if (mid_done) {
-        } else if (d.ff != ZG_LM_FF_NONE)  // (a router reads the fp32 rows)
-            ZG_TRY(launch_norm_add_norm(g->x, g->y, L.norm1b, L.norm2, eps, h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
+        } else if (defer && d.ff == ZG_LM_FF_DENSE) defer_norm(g->y, L.norm1b, L.norm2);
+        else if (d.ff != ZG_LM_FF_NONE)  // (a router reads the fp32 rows)
+            ZG_TRY(launch_norm_add_norm(x, g->y, L.norm1b, L.norm2, eps, h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
         else {
             ZG_TRY(tail(g->y, nullptr, nullptr, 0, L.norm1b));
-            if (!h_ready) ZG_TRY(launch_norm_add(g->x, g->y, L.norm1b, eps, M, W, s));
+            if (!h_ready) ZG_TRY(add_normed(p, L.norm1b));
         }
         const int F = d.ff_width;
         hin = g->h;
@@ -1532,7 +1569,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         if (d.ff == ZG_LM_FF_DENSE) {
             ZG_TRY(dense_ff(L, hin16 ? nullptr : hin, hin16, g->y));
             ZG_TRY(tail(g->y, nullptr, nullptr, 0, L.norm2b));
-            if (!h_ready) ZG_TRY(launch_norm_add(g->x, g->y, L.norm2b, eps, M, W, s));
+            if (!h_ready) ZG_TRY(add_normed(p, L.norm2b));
         } else if (d.ff == ZG_LM_FF_MOE) {
             const int E = d.experts, top = d.top, NA = M * top;
             const bool glu = d.ff_act == ZG_LM_ACT_GLU_SILU;
@@ -1554,10 +1591,11 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             ZG_TRY(expert_first(up, dn, F, NA, glu));
             ZG_TRY(launch_linear(dn, f32, s));
             if (few) ZG_TRY(tail(nullptr, g->ye, g->wt, top, L.norm2b));
-            if (!h_ready) ZG_TRY(launch_moe_combine(g->x, g->ye, few ? nullptr : g->inv, g->wt, top, L.norm2b, eps, M, W, s));
+            if (!h_ready) ZG_TRY(launch_moe_combine(x, g->ye, few ? nullptr : g->inv, g->wt, top, L.norm2b, eps, M, W, s));
         }
         ZG_TRY(copy_trace(p));
     }
+    if (x != g->x) ZG_TRY(launch_copy_row(x, g->x, W, s));
     // the rows the last tokens of the entries left for the token shift of their successors
     if (!canon && !side && !tnorm && !g->no_shift) ZG_TRY(launch_commit_rows(g->shift_state, (size_t)g->n_passes * W, g->last_h, W, d_eslot, n_ent, W, g->n_passes, W, (size_t)NS * W, s));
 

@@ -1,0 +1,269 @@
+// lm_gemv.hip — the linear maps of decode steps of one or two rows, operands in whole 16-byte pieces.
+//
+// A step of one sequence is a chain of some hundred launches that each read a few MB: its time is the chain's latency, and a launch's
+// latency is the number of memory round trips it makes.  Here everything a wave reads (its share of two weight rows and of the
+// activations) is requested at entry, unconditionally and at clamped addresses, before anything is used: one round trip.  (In the
+// general kernel, lm_gemv_kernel, every piece is loaded under its own bounds check and waited for inside it.)
+//
+// One row, us a launch inside a replayed step, this against the general kernel: 768 columns 4.3 : 5.6, 3072 columns through the polynomial
+// 4.7 : 7.4.  With the sum and the two norms in front of a product inside it 4.45, where their own launch took 5.25 more.
+//
+// Short rows: a wave has two whole weight rows.  Long rows (K of 1536 and more): a workgroup has two, its four waves a quarter of K each.
+#include "lm_linear_args.h"
+
+#include <algorithm>
+
+namespace zg {
+namespace lm {
+
+namespace {
+
+enum { GEMV_PLAIN, GEMV_GLU, GEMV_POLY, GEMV_NORM };
+
+// sums of N values over the lanes of a wave, each in every lane
+template <int N>
+__device__ __forceinline__ void wave_sums(float (&v)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[i] = wave_allsum(v[i]);
+}
+
+template <int MR, int U, int KIND, bool SPLIT>
+__device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const NormIn& pre) {
+    constexpr int NS = KIND == GEMV_POLY ? 11 : 2;  // sums of a row: the two products; or q1 q2 q3 and four products for each weight row
+    __shared__ float s_part[SPLIT ? 4 : 1][MR][NS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n0 = SPLIT ? blockIdx.x * 2 : blockIdx.x * 8 + wave * 2;
+    if (n0 >= p.N) return;
+    if (p.z_group && p.z_group[z] >= p.z_limit) return;
+    const bf16_t* B = p.B + (long long)(p.z_group ? p.z_group[z] : z) * p.b_zoff;
+    const bf16_t* w[2] = {B + (long long)n0 * p.ldb, B + (long long)min(n0 + 1, p.N - 1) * p.ldb};
+    const int kq = SPLIT ? (((p.K + 3) / 4) + 7) & ~7 : p.K;  // a wave's share of K, whole pieces of 8
+    const int k_lo = SPLIT ? wave * kq : 0, k_hi = SPLIT ? min(p.K, k_lo + kq) : p.K;
+    int at[U];
+    bool in[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int k = k_lo + lane * 8 + 512 * u;
+        in[u] = k < k_hi;
+        at[u] = min(k, p.K - 8);
+    }
+    u32x4 wr[2][U];
+    f32x4 a[MR][U][2], g[KIND == GEMV_GLU ? MR : 1][U][2];
+    float asc[MR], agate[MR];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) wr[c][u] = *reinterpret_cast<const u32x4*>(w[c] + at[u]);
+    if constexpr (KIND == GEMV_NORM) {
+        // the row is norm(x + norm(y) (1 + wb)) (1 + wn): every wave works it out for itself, the first one keeps the sum
+        f32x4 y[U][2], vb[U][2], vn[U][2];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                a[0][u][i] = *reinterpret_cast<const f32x4*>(pre.x + at[u] + 4 * i);
+                y[u][i] = *reinterpret_cast<const f32x4*>(pre.y + at[u] + 4 * i);
+                vb[u][i] = *reinterpret_cast<const f32x4*>(pre.wb + at[u] + 4 * i);
+                vn[u][i] = *reinterpret_cast<const f32x4*>(pre.wn + at[u] + 4 * i);
+            }
+        float ss = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (in[u]) ss = fmaf(y[u][i][e], y[u][i][e], ss);
+        const float r = 1.0f / sqrtf(wave_allsum(ss) / (float)p.K + pre.eps);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    a[0][u][i][e] += y[u][i][e] * r * (1.0f + vb[u][i][e]);
+                    if (in[u]) s2 = fmaf(a[0][u][i][e], a[0][u][i][e], s2);
+                }
+                if (n0 == 0 && in[u]) *reinterpret_cast<f32x4*>(pre.x_out + at[u] + 4 * i) = a[0][u][i];
+            }
+        const float r2 = 1.0f / sqrtf(wave_allsum(s2) / (float)p.K + pre.eps);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a[0][u][i][e] = a[0][u][i][e] * r2 * (1.0f + vn[u][i][e]);
+    } else {
+        const float* A = p.A + (long long)z * p.a_zoff;
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const int rid = p.z_group ? z * p.M + m : m;
+            const float* row = A + (long long)((p.a_rows ? p.a_rows[rid] : rid) / p.a_div) * p.lda;
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[m][u][i] = *reinterpret_cast<const f32x4*>(row + at[u] + 4 * i);
+                    if constexpr (KIND == GEMV_GLU) g[m][u][i] = *reinterpret_cast<const f32x4*>(row + p.a_glu + at[u] + 4 * i);
+                }
+            asc[m] = KIND == GEMV_GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
+            agate[m] = KIND == GEMV_GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-row[p.glu_gate_col])) : 1.0f;
+        }
+    }
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const u32x4 none = {0u, 0u, 0u, 0u};
+    float sum[MR][NS];
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int i = 0; i < NS; ++i) sum[m][i] = 0.0f;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        float wf[2][8];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const u32x4 v = in[u] ? wr[c][u] : none;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wf[c][2 * i] = bf16_lo(v[i]);
+                wf[c][2 * i + 1] = bf16_hi(v[i]);
+            }
+        }
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                f32x4 x = a[m][u][i];
+                if constexpr (KIND == GEMV_GLU) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = glu_on_load(x[e], g[m][u][i][e], p, asc[m]) * agate[m];
+                }
+                if (!in[u]) x = zero;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float w0 = wf[0][4 * i + e], w1 = wf[1][4 * i + e];
+                    if constexpr (KIND == GEMV_POLY) {
+                        float* s = sum[m];
+                        const float v = x[e], q = v * v, c = q * v;
+                        s[0] += q;
+                        s[1] = fmaf(q, q, s[1]);
+                        s[2] = fmaf(c, c, s[2]);
+                        s[3] = fmaf(v, w0, s[3]); s[7] = fmaf(v, w1, s[7]);
+                        s[4] = fmaf(q, w0, s[4]); s[8] = fmaf(q, w1, s[8]);
+                        s[5] = fmaf(c, w0, s[5]); s[9] = fmaf(c, w1, s[9]);
+                        s[6] += w0; s[10] += w1;
+                    } else {
+                        sum[m][0] = fmaf(x[e], w0, sum[m][0]);
+                        sum[m][1] = fmaf(x[e], w1, sum[m][1]);
+                    }
+                }
+            }
+    }
+#pragma unroll
+    for (int m = 0; m < MR; ++m) wave_sums(sum[m]);
+    float* C = p.C + (long long)z * p.c_zoff;
+    if constexpr (!SPLIT) {
+        static_assert(KIND != GEMV_POLY, "the polynomial's rows are long");
+        if (lane < 2 && n0 + lane < p.N) {
+#pragma unroll
+            for (int m = 0; m < MR; ++m) C[(long long)m * p.ldc + n0 + lane] = finish(lane ? sum[m][1] : sum[m][0], n0 + lane, p);
+        }
+    } else {
+        if (lane == 0) {
+#pragma unroll
+            for (int m = 0; m < MR; ++m)
+#pragma unroll
+                for (int i = 0; i < NS; ++i) s_part[wave][m][i] = sum[m][i];
+        }
+        __syncthreads();
+        const int m = threadIdx.x >> 1, c = threadIdx.x & 1;
+        if (m < MR && n0 + c < p.N) {
+            auto sum4 = [&](int i) { return (s_part[0][m][i] + s_part[1][m][i]) + (s_part[2][m][i] + s_part[3][m][i]); };
+            float v;
+            if constexpr (KIND == GEMV_POLY) {
+                const float K = (float)p.K, eps = p.poly_eps, *d = p.a_poly;
+                v = (d[0] / sqrtf(sum4(0) / K + eps) * sum4(3 + 4 * c) + d[1] / sqrtf(sum4(1) / K + eps) * sum4(4 + 4 * c)) +
+                    (d[2] / sqrtf(sum4(2) / K + eps) * sum4(5 + 4 * c) + d[3] * sum4(6 + 4 * c));
+            } else v = sum4(c);
+            C[(long long)m * p.ldc + n0 + c] = finish(v, n0 + c, p);
+        }
+    }
+}
+
+template <int MR, int U, int KIND, bool SPLIT>
+__global__ __launch_bounds__(256) void lm_gemv_at_once_kernel(const LinArgs p, const NormIn pre) {
+    gemv_body<MR, U, KIND, SPLIT>(p, blockIdx.z, pre);
+}
+// batches [0, za) are product a's, the rest product b's
+template <int U, int KIND>
+__global__ __launch_bounds__(256) void lm_gemv_at_once_pair_kernel(const LinArgs a, const LinArgs b, int za) {
+    if ((int)blockIdx.z < za) gemv_body<1, U, KIND, false>(a, blockIdx.z, NormIn());
+    else gemv_body<1, U, KIND, false>(b, blockIdx.z - za, NormIn());
+}
+
+constexpr int kLongRow = 1536;  // from here on K is split over the waves
+
+int kind_of(const Linear& L) { return L.a_poly ? GEMV_POLY : L.a_glu > 0 ? GEMV_GLU : GEMV_PLAIN; }
+bool pieces_ok(const Linear& L, const LinArgs& p) {
+    return L.M >= 1 && L.M <= 2 && !L.grp_off && !L.C16 && !L.glu_out && L.N > 0 && L.nz >= 1 && L.nz <= 65535 && L.K >= 8 && L.K % 8 == 0 && L.A && L.B && L.C &&
+           p.a_vec && p.b_vec && L.a_glu % 4 == 0 && L.a_div >= 1;
+}
+
+}  // namespace
+
+int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hipStream_t s, bool* taken) {
+    *taken = false;
+    const LinArgs a = make_args(A), b = B ? make_args(*B) : a;
+    if (!pieces_ok(A, a) || (B && (!pieces_ok(*B, b) || B->M != A.M || kind_of(*B) != kind_of(A) || A.nz + B->nz > 65535))) return ZG_OK;
+    const int kind = norm ? (int)GEMV_NORM : kind_of(A);
+    const int k_min = B ? std::min(A.K, B->K) : A.K, k_max = B ? std::max(A.K, B->K) : A.K;
+    // (batches of long rows fill the chip without the split)
+    const bool split = k_min >= kLongRow && A.nz + (B ? B->nz : 0) <= 4;
+    if (kind == GEMV_POLY && !split) return ZG_OK;
+    if (norm && (split || B || A.M != 1 || A.nz != 1)) return ZG_OK;
+    if (B && (split || A.M != 1)) return ZG_OK;
+    const int share = split ? (((k_max + 3) / 4) + 7) & ~7 : k_max, pieces = (share + 511) / 512;
+    if (pieces > (norm ? 2 : 3)) return ZG_OK;
+    const int rows = split ? 2 : 8;
+    const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, 1, A.nz + (B ? B->nz : 0));
+    const NormIn none{}, &pre = norm ? *norm : none;
+#define ZG_GV(MR, U, KIND, SPLIT) (lm_gemv_at_once_kernel<MR, U, KIND, SPLIT><<<grid, 256, 0, s>>>(a, pre))
+#define ZG_GV_P(KIND)                                                                              \
+    do {                                                                                           \
+        if (pieces == 1) lm_gemv_at_once_pair_kernel<1, KIND><<<grid, 256, 0, s>>>(a, b, A.nz);      \
+        else if (pieces == 2) lm_gemv_at_once_pair_kernel<2, KIND><<<grid, 256, 0, s>>>(a, b, A.nz); \
+        else lm_gemv_at_once_pair_kernel<3, KIND><<<grid, 256, 0, s>>>(a, b, A.nz);                  \
+    } while (0)
+#define ZG_GV_U(MR, KIND, SPLIT)                      \
+    do {                                              \
+        if (pieces == 1) ZG_GV(MR, 1, KIND, SPLIT);   \
+        else if (pieces == 2) ZG_GV(MR, 2, KIND, SPLIT); \
+        else ZG_GV(MR, 3, KIND, SPLIT);               \
+    } while (0)
+#define ZG_GV_M(KIND, SPLIT)                    \
+    do {                                        \
+        if (A.M == 1) ZG_GV_U(1, KIND, SPLIT);  \
+        else ZG_GV_U(2, KIND, SPLIT);           \
+    } while (0)
+    if (B && kind == GEMV_GLU) ZG_GV_P(GEMV_GLU);
+    else if (B) ZG_GV_P(GEMV_PLAIN);
+    else if (norm) {
+        if (pieces == 1) ZG_GV(1, 1, GEMV_NORM, false);
+        else ZG_GV(1, 2, GEMV_NORM, false);
+    } else if (kind == GEMV_POLY) ZG_GV_M(GEMV_POLY, true);
+    else if (kind == GEMV_GLU && split) ZG_GV_M(GEMV_GLU, true);
+    else if (kind == GEMV_GLU) ZG_GV_M(GEMV_GLU, false);
+    else if (split) ZG_GV_M(GEMV_PLAIN, true);
+    else ZG_GV_M(GEMV_PLAIN, false);
+#undef ZG_GV
+#undef ZG_GV_P
+#undef ZG_GV_U
+#undef ZG_GV_M
+    note_kernel("lm_gemv_at_once_kernel<%d>", A.M);
+    ZG_HIP(hipGetLastError());
+    *taken = true;
+    return ZG_OK;
+}
+
+}  // namespace lm
+}  // namespace zg

@@ -64,6 +64,15 @@ struct Linear {
 // Steps of few rows: the first product of a gated feed-forward with the activation in its epilogue, h [rows][F] = act(gate) * up for B rows
 // [gate (F) | up (F)]; L as for launch_linear, its C, ldc, c_zoff and N ignored.  *taken = false: not a form that has it, nothing launched.
 int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t s, bool* taken);
+// What launch_norm_add_norm does, inside the product that reads the row: x_out = x + norm(y) (1 + wb), and the product's row is
+// norm(x_out) (1 + wn).  x_out must not be x (every workgroup reads x, one writes x_out).
+struct NormIn {
+    const float *x = nullptr, *y = nullptr, *wb = nullptr, *wn = nullptr;
+    float* x_out = nullptr;
+    float eps = 0.0f;
+};
+// One row (L.A only names where the row would be); *taken = false: not a form that has it, nothing launched.
+int launch_linear_normed(const Linear& L, const NormIn& norm, hipStream_t s, bool* taken);
 // Picks the row-vector kernel (few rows: decode) or the tiled matrix-core kernel (prompt portions).
 int launch_linear(const Linear& L, bool f32, hipStream_t s);
 constexpr int kGemvMaxRows = 8;
@@ -93,8 +102,9 @@ int launch_norm_shift(const float* x, const float* w, const float* mu, float eps
 // dst[slots[e]] = src[e] for every entry e; rows of `width` floats (dst rows slot_stride apart, src rows src_stride apart)
 int launch_commit_rows(float* dst, size_t slot_stride, const float* src, size_t src_stride, const int* slots, int n_entries, int width,
                        int n_sets, size_t dst_set_stride, size_t src_set_stride, hipStream_t s);
-// x[m] += y[m] / rms(y[m]) * (1 + w)            (the norm behind a sublayer, then the residual sum)
-int launch_norm_add(float* x, const float* y, const float* w, float eps, int M, int W, hipStream_t s);
+int launch_copy_row(const float* x, float* out, int W, hipStream_t s);
+// out[m] = x[m] + y[m] / rms(y[m]) * (1 + w)     (the norm behind a sublayer, then the residual sum; out may be x)
+int launch_norm_add(const float* x, float* out, const float* y, const float* w, float eps, int M, int W, hipStream_t s);
 // x[m] += y[m] / rms(y[m]) * (1 + wb);  h[m] = x[m] / rms(x[m]) * (1 + wn)   (the two above in one launch)
 int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s, bf16_t* h16 = nullptr);
 // Steps of one row per entry: the sum behind a pass's last sublayer (y, or the weighted sum of the chosen experts' rows yexp) and

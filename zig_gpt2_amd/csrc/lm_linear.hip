@@ -858,6 +858,8 @@ int launch_linear_pair(const Linear& A, const Linear& B, bool f32, hipStream_t s
     bool taken = false;
     if (getenv("ZGPT2_LM_NO_ROWS") == nullptr) ZG_TRY(launch_rows(A, &B, s, &taken));
     if (taken) return ZG_OK;
+    ZG_TRY(launch_gemv_at_once(A, &B, nullptr, s, &taken));
+    if (taken) return ZG_OK;
     const bool one_launch = A.M == 1 && B.M == 1 && A.nz >= 1 && B.nz >= 1 && A.N > 0 && B.N > 0 && !A.grp_off && !B.grp_off && !takes_k_split(A) &&
                             !takes_k_split(B) && A.K > 0 && B.K > 0 && A.A && A.B && A.C && B.A && B.B && B.C && A.a_div >= 1 && B.a_div >= 1 &&
                             A.nz + B.nz <= 65535;
@@ -918,6 +920,14 @@ int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t 
     return launch_rows(g, nullptr, s, taken);
 }
 
+int launch_linear_normed(const Linear& L, const NormIn& n, hipStream_t s, bool* taken) {
+    *taken = false;
+    const uintptr_t all = reinterpret_cast<uintptr_t>(n.x) | reinterpret_cast<uintptr_t>(n.y) | reinterpret_cast<uintptr_t>(n.wb) | reinterpret_cast<uintptr_t>(n.wn) |
+                          reinterpret_cast<uintptr_t>(n.x_out);
+    if (L.M != 1 || (all & 15) != 0 || n.x == n.x_out || L.a_glu || L.a_poly || L.a_rows || L.z_group) return ZG_OK;
+    return launch_gemv_at_once(L, nullptr, &n, s, taken);
+}
+
 int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     if (L.M <= 0 || L.N <= 0 || L.nz <= 0) return ZG_OK;
     const bool tiled = L.grp_off || L.M > kGemvMaxRows;
@@ -929,6 +939,8 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     if (!L.grp_off && L.M <= kGemvMaxRows) {
         bool taken = false;
         if (getenv("ZGPT2_LM_NO_ROWS") == nullptr) ZG_TRY(launch_rows(L, nullptr, s, &taken));
+        if (taken) return ZG_OK;
+        ZG_TRY(launch_gemv_at_once(L, nullptr, nullptr, s, &taken));
         if (taken) return ZG_OK;
         if (takes_k_split(L)) {  // long rows, one or two of them, few batches: K split over the waves, two weight rows per workgroup
             const dim3 gks((L.N + 1) / 2, 1, L.nz);  // (from four rows on the activations are re-read by too many workgroups: measured slower)

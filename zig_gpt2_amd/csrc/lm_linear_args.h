@@ -116,6 +116,8 @@ inline LinArgs make_args(const Linear& L) {
 
 // lm_rows.hip: steps of 3 to 8 rows on the matrix cores.  *taken = false: not a form it has (nothing launched).
 int launch_rows(const Linear& a, const Linear* b, hipStream_t s, bool* taken);
+// lm_gemv.hip: steps of one or two rows whose operands are whole 16-byte pieces.  *taken as above.
+int launch_gemv_at_once(const Linear& a, const Linear* b, const NormIn* norm, hipStream_t s, bool* taken);
 
 }  // namespace lm
 }  // namespace zg

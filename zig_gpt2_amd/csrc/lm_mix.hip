@@ -139,12 +139,16 @@ __global__ __launch_bounds__(256) void commit_rows_kernel(float* dst, size_t slo
     for (int i = threadIdx.x; i < width; i += blockDim.x) d[i] = s[i];
 }
 
-__global__ __launch_bounds__(256) void norm_add_kernel(float* x, const float* y, const float* w, float eps, int W) {
+__global__ __launch_bounds__(256) void norm_add_kernel(const float* x, float* out, const float* y, const float* w, float eps, int W) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
     const float* yr = y + (size_t)m * W;
     const float r = row_inv_rms(yr, W, eps, s_red);
-    for (int i = threadIdx.x; i < W; i += blockDim.x) x[(size_t)m * W + i] += yr[i] * r * (1.0f + w[i]);
+    for (int i = threadIdx.x; i < W; i += blockDim.x) out[(size_t)m * W + i] = x[(size_t)m * W + i] + yr[i] * r * (1.0f + w[i]);
+}
+
+__global__ __launch_bounds__(256) void copy_row_kernel(const float* x, float* out, int W) {
+    for (int i = threadIdx.x; i < W; i += 256) out[i] = x[i];
 }
 
 // x += norm(y) * (1 + wb), then h = norm(x) * (1 + wn): the norm behind the mixer, the residual sum and the norm in front of the
@@ -1532,9 +1536,15 @@ int launch_commit_rows(float* dst, size_t slot_stride, const float* src, size_t 
     return ZG_OK;
 }
 
-int launch_norm_add(float* x, const float* y, const float* w, float eps, int M, int W, hipStream_t s) {
+int launch_norm_add(const float* x, float* out, const float* y, const float* w, float eps, int M, int W, hipStream_t s) {
     if (M <= 0) return ZG_OK;
-    norm_add_kernel<<<M, 256, 0, s>>>(x, y, w, eps, W);
+    norm_add_kernel<<<M, 256, 0, s>>>(x, out, y, w, eps, W);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_copy_row(const float* x, float* out, int W, hipStream_t s) {
+    copy_row_kernel<<<1, 256, 0, s>>>(x, out, W);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
