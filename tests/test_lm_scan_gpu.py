@@ -28,6 +28,21 @@ def steps(m, toks, cuts):
     return [np.concatenate(r) for r in rows]
 
 
+def assert_rows_close(got, model, w, toks, what):
+    """Every row within TOL, or within eight times what perturbing the embedding and the query map by one part in 2^24 does to it: where
+    a head's q . k nearly cancels, the norm behind the head magnifies the rounding of its inputs (sequence 1, row 187 of the smallest
+    heads at once forgotten: 3.6e-5 for a perturbation of 6e-8; the median row 5e-8)."""
+    ref = model(w).forward(toks)[0]
+    scale, moved = np.abs(ref).max(), np.zeros(len(ref))
+    for seed in range(3):
+        rng, near = np.random.default_rng(seed), dict(w)
+        for name in ("embed", "l0.mix.q"):
+            near[name] = np.asarray(w[name], np.float64) * (1 + 2.0**-24 * rng.standard_normal(w[name].shape))
+        moved = np.maximum(moved, np.abs(model(near).forward(toks)[0] - ref).max(axis=1) / scale)
+    err = np.abs(np.asarray(got, np.float64) - ref).max(axis=1) / scale
+    assert (err < np.maximum(tl.TOL["float32"], 8 * moved)).all(), (what, err.max(), err.argmax())
+
+
 CUTS = [(33, 1, 65), (97, 64, 66), (161, 192, 129), (200, 193, 200)]
 
 
@@ -38,12 +53,11 @@ def test_hgrn2_chunks(heads, dim, vdim, forget):
     w = tl.weights(cfg, seed=dim + vdim, lower={"slow": (0.97, 1.0), "mixed": (0.0, 1.0), "sudden": (0.0, 1e-4)}[forget])
     if forget == "sudden":  # gates down to 1e-6: their products underflow within a block
         w["l0.mix.f.b"] = w["l0.mix.f.b"] - 10.0
-    oracle = lm_oracle.Model(cfg, w)
     toks = [tl.tokens(90 + b, 200, cfg["vocab"]) for b in range(3)]
     m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=1024, max_seqs=3)
     m.load_weights(w)
     for got, t in zip(steps(m, toks, CUTS), toks):
-        tl.assert_close(got, oracle.forward(t[: len(got)])[0], "float32", (dim, vdim, forget))
+        assert_rows_close(got, lambda v: lm_oracle.Model(cfg, v), w, t[: len(got)], (dim, vdim, forget))
     m.close()
 
 

@@ -915,8 +915,8 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     const int* d_off = g->meta + meta_row_off(g);
     const bool f32 = g->f32;
     const float eps = g->cfg.norm_eps;
-    // The residual stream.  In steps of one row it changes its place wherever a product does the sum and the norms in front of it itself:
-    // every workgroup of the product reads it, one writes the new one.  It ends where it began.
+    // The residual stream.  It changes its place where the sum behind a sublayer is written while others still read the stream: in steps of
+    // one row inside the next product, in portions with a token shift across the waves of the next norm.  It ends where it began.
     float *x = g->x, *x_other = g->hc;
     const bool few = M <= kGemvMaxRows;
     const bool canon = g->canon >= 1;
@@ -1082,13 +1082,31 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         auto tail = [&](const float* y, const float* yexp, const float* weight, int top, const float* wb) -> int {
             if (p + 1 >= g->n_passes || canon || g->passes[p + 1].readd) return ZG_OK;
             const LayerW& N = g->layers[g->passes[p + 1].layer];
-            if (g->no_shift && y) {  // nothing of the token before: the same fusion at any number of rows
-                if (defer) defer_norm(y, wb, N.norm1);
-                else ZG_TRY(launch_norm_add_norm(x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
+            if (g->no_shift && y && defer) {
+                defer_norm(y, wb, N.norm1);
                 h_ready = true;
                 return ZG_OK;
             }
-            if (!single || g->no_shift) return ZG_OK;
+            NormRows r;
+            r.x = x; r.y = y; r.yexp = yexp; r.weight = weight; r.top = top; r.inv = few ? nullptr : g->inv; r.wb = wb; r.wn = N.norm1; r.eps = eps;
+            r.out = h_r16 ? nullptr : g->h; r.out16 = h_r16 ? g->h16 : nullptr; r.M = M; r.W = W;
+            if (!g->no_shift) {
+                r.mu = N.shift; r.row_prev = single ? nullptr : d_prev; r.row_slot = d_slot; r.shift_state = g->shift_state + (size_t)(p + 1) * W;
+                r.slot_stride = (size_t)g->n_passes * W; r.row_entry_if_last = d_last; r.last_out = g->last_h + (size_t)(p + 1) * NS * W;
+            }
+            r.x_out = r.row_prev ? x_other : x;
+            ZG_TRY(launch_norm_rows(r, s, &h_ready));
+            if (h_ready) {
+                if (r.x_out != x) std::swap(x, x_other);
+                return ZG_OK;
+            }
+            if (yexp && !few) return ZG_OK;  // (rows the general kernels take)
+            if (g->no_shift && y) {  // nothing of the token before: the same fusion at any number of rows
+                ZG_TRY(launch_norm_add_norm(x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
+                h_ready = true;
+                return ZG_OK;
+            }
+            if (!single || g->no_shift || h_r16) return ZG_OK;
             return launch_sum_norm_shift(x, y, yexp, weight, top, wb, N.norm1, N.shift, eps, g->h, M, W, d_slot, g->shift_state + (size_t)(p + 1) * W,
                                          (size_t)g->n_passes * W, d_last, g->last_h + (size_t)(p + 1) * NS * W, s, &h_ready);
         };
@@ -1590,12 +1608,14 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             }
             ZG_TRY(expert_first(up, dn, F, NA, glu));
             ZG_TRY(launch_linear(dn, f32, s));
-            if (few) ZG_TRY(tail(nullptr, g->ye, g->wt, top, L.norm2b));
-            if (!h_ready) ZG_TRY(launch_moe_combine(x, g->ye, few ? nullptr : g->inv, g->wt, top, L.norm2b, eps, M, W, s));
+            ZG_TRY(tail(nullptr, g->ye, g->wt, top, L.norm2b));
+            float* const out = p + 1 == g->n_passes ? g->x : x;
+            if (!h_ready) ZG_TRY(launch_moe_combine(x, out, g->ye, few ? nullptr : g->inv, g->wt, top, L.norm2b, eps, M, W, s));
+            if (!h_ready) x = out;
         }
         ZG_TRY(copy_trace(p));
     }
-    if (x != g->x) ZG_TRY(launch_copy_row(x, g->x, W, s));
+    if (x != g->x) ZG_TRY(launch_copy_floats(x, g->x, (size_t)M * W, s));
     // the rows the last tokens of the entries left for the token shift of their successors
     if (!canon && !side && !tnorm && !g->no_shift) ZG_TRY(launch_commit_rows(g->shift_state, (size_t)g->n_passes * W, g->last_h, W, d_eslot, n_ent, W, g->n_passes, W, (size_t)NS * W, s));
 

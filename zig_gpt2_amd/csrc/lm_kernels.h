@@ -102,7 +102,33 @@ int launch_norm_shift(const float* x, const float* w, const float* mu, float eps
 // dst[slots[e]] = src[e] for every entry e; rows of `width` floats (dst rows slot_stride apart, src rows src_stride apart)
 int launch_commit_rows(float* dst, size_t slot_stride, const float* src, size_t src_stride, const int* slots, int n_entries, int width,
                        int n_sets, size_t dst_set_stride, size_t src_set_stride, hipStream_t s);
-int launch_copy_row(const float* x, float* out, int W, hipStream_t s);
+int launch_copy_floats(const float* x, float* out, size_t n, hipStream_t s);
+// Rows of the residual stream between two sublayers, in one launch (lm_norm.hip); what is null is left out:
+//   y' = y[m], or sum_k weight[m top + k] yexp[inv ? inv[m top + k] : m top + k];   x_out[m] = x[m] + y' / rms(y') (1 + wb)
+//   h = x_out[m] / rms (1 + wn);   out[m] (and out16, rounded) = h, or with mu: h + (h of row_prev[m], or its slot's row if < 0, - h) mu
+//   last_out[row_entry_if_last[m]] = h where that is >= 0
+// row_prev[m] is m - 1 or negative (null: all negative).  x_out may be x unless rows are shifted by their predecessors.  *taken = false: rows too
+// wide or in no whole 16-byte pieces, nothing launched.
+struct NormRows {
+    const float* x = nullptr;
+    float* x_out = nullptr;
+    const float *y = nullptr, *yexp = nullptr;
+    const int* inv = nullptr;
+    const float* weight = nullptr;
+    int top = 0;
+    const float *wb = nullptr, *wn = nullptr, *mu = nullptr;
+    float eps = 0.0f;
+    float* out = nullptr;
+    bf16_t* out16 = nullptr;
+    int M = 0, W = 0;
+    const int *row_prev = nullptr, *row_slot = nullptr;
+    const float* shift_state = nullptr;
+    size_t slot_stride = 0;
+    const int* row_entry_if_last = nullptr;
+    float* last_out = nullptr;
+    int run = 1;  // (set by the launch) consecutive rows of a wave
+};
+int launch_norm_rows(const NormRows& p, hipStream_t s, bool* taken);
 // out[m] = x[m] + y[m] / rms(y[m]) * (1 + w)     (the norm behind a sublayer, then the residual sum; out may be x)
 int launch_norm_add(const float* x, float* out, const float* y, const float* w, float eps, int M, int W, hipStream_t s);
 // x[m] += y[m] / rms(y[m]) * (1 + wb);  h[m] = x[m] / rms(x[m]) * (1 + wn)   (the two above in one launch)
@@ -443,8 +469,8 @@ int launch_glu_clipped(const float* gu, int ld, float* h, int rows, int F, float
 // pick != null: assignments whose pick is not below n_exp take ident[m] instead of a row of yexp
 int launch_expert_sum(float* y, const float* yexp, const int* inv, const float* weight, int top, const float* ys, int M, int W, hipStream_t s,
                       const int* pick = nullptr, int n_exp = 0, const float* ident = nullptr);
-// y = sum_k weight[m][k] * yexp[inv ? inv[m top + k] : m top + k];   x[m] += y / rms(y) * (1 + w)
-int launch_moe_combine(float* x, const float* yexp, const int* inv, const float* weight, int top, const float* w, float eps, int M, int W,
+// y = sum_k weight[m][k] * yexp[inv ? inv[m top + k] : m top + k];   out[m] = x[m] + y / rms(y) * (1 + w)   (out may be x)
+int launch_moe_combine(const float* x, float* out, const float* yexp, const int* inv, const float* weight, int top, const float* w, float eps, int M, int W,
                        hipStream_t s);
 
 // ------------------------------------------------------------------------------------------------ sampling support

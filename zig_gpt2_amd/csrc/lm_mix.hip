@@ -147,8 +147,9 @@ __global__ __launch_bounds__(256) void norm_add_kernel(const float* x, float* ou
     for (int i = threadIdx.x; i < W; i += blockDim.x) out[(size_t)m * W + i] = x[(size_t)m * W + i] + yr[i] * r * (1.0f + w[i]);
 }
 
-__global__ __launch_bounds__(256) void copy_row_kernel(const float* x, float* out, int W) {
-    for (int i = threadIdx.x; i < W; i += 256) out[i] = x[i];
+__global__ __launch_bounds__(256) void copy_floats_kernel(const float* x, float* out, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = x[i];
 }
 
 // x += norm(y) * (1 + wb), then h = norm(x) * (1 + wn): the norm behind the mixer, the residual sum and the norm in front of the
@@ -1523,6 +1524,12 @@ int launch_norm_shift(const float* x, const float* w, const float* mu, float eps
                       const int* row_slot, const float* shift_state, size_t slot_stride, const int* row_entry_if_last, float* last_out,
                       hipStream_t s, bf16_t* out16) {
     if (M <= 0) return ZG_OK;
+    NormRows r;
+    r.x = x; r.wn = w; r.mu = mu; r.eps = eps; r.out = out; r.out16 = out16; r.M = M; r.W = W; r.row_prev = row_prev; r.row_slot = row_slot;
+    r.shift_state = shift_state; r.slot_stride = slot_stride; r.row_entry_if_last = row_entry_if_last; r.last_out = last_out;
+    bool taken = false;
+    if (mu || !row_entry_if_last) ZG_TRY(launch_norm_rows(r, s, &taken));  // (without a shift it keeps no last rows)
+    if (taken) return ZG_OK;
     norm_shift_kernel<<<M, 256, 0, s>>>(x, w, mu, eps, out, W, row_prev, row_slot, shift_state, slot_stride, row_entry_if_last, last_out, out16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -1538,19 +1545,30 @@ int launch_commit_rows(float* dst, size_t slot_stride, const float* src, size_t 
 
 int launch_norm_add(const float* x, float* out, const float* y, const float* w, float eps, int M, int W, hipStream_t s) {
     if (M <= 0) return ZG_OK;
+    NormRows r;
+    r.x = x; r.x_out = out; r.y = y; r.wb = w; r.eps = eps; r.M = M; r.W = W;
+    bool taken = false;
+    ZG_TRY(launch_norm_rows(r, s, &taken));
+    if (taken) return ZG_OK;
     norm_add_kernel<<<M, 256, 0, s>>>(x, out, y, w, eps, W);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
-int launch_copy_row(const float* x, float* out, int W, hipStream_t s) {
-    copy_row_kernel<<<1, 256, 0, s>>>(x, out, W);
+int launch_copy_floats(const float* x, float* out, size_t n, hipStream_t s) {
+    if (n == 0) return ZG_OK;
+    copy_floats_kernel<<<(unsigned)((n + 255) / 256), 256, 0, s>>>(x, out, n);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
 int launch_norm_add_norm(float* x, const float* y, const float* wb, const float* wn, float eps, float* h, int M, int W, hipStream_t s, bf16_t* h16) {
     if (M <= 0) return ZG_OK;
+    NormRows r;
+    r.x = x; r.x_out = x; r.y = y; r.wb = wb; r.wn = wn; r.eps = eps; r.out = h; r.out16 = h16; r.M = M; r.W = W;
+    bool taken = false;
+    ZG_TRY(launch_norm_rows(r, s, &taken));
+    if (taken) return ZG_OK;
     norm_add_norm_kernel<<<M, 256, 0, s>>>(x, y, wb, wn, eps, h, W, h16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;

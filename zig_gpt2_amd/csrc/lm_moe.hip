@@ -347,7 +347,7 @@ __global__ __launch_bounds__(256) void expert_sum_kernel(float* y, const float* 
     y[idx] = a;
 }
 
-__global__ __launch_bounds__(256) void moe_combine_kernel(float* x, const float* yexp, const int* inv, const float* weight, int top, const float* w,
+__global__ __launch_bounds__(256) void moe_combine_kernel(const float* x, float* out, const float* yexp, const int* inv, const float* weight, int top, const float* w,
                                                           float eps, int W) {
     __shared__ float s_red[8];
     const int m = blockIdx.x;
@@ -366,7 +366,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(float* x, const float*
     }
     ss = block_allsum(ss, s_red);
     const float r = 1.0f / sqrtf(ss / (float)W + eps);
-    for (int i = threadIdx.x; i < W; i += blockDim.x) x[(size_t)m * W + i] += mix(i) * r * (1.0f + w[i]);
+    for (int i = threadIdx.x; i < W; i += blockDim.x) out[(size_t)m * W + i] = x[(size_t)m * W + i] + mix(i) * r * (1.0f + w[i]);
 }
 
 }  // namespace
@@ -425,10 +425,15 @@ int launch_expert_sum(float* y, const float* yexp, const int* inv, const float* 
     return ZG_OK;
 }
 
-int launch_moe_combine(float* x, const float* yexp, const int* inv, const float* weight, int top, const float* w, float eps, int M, int W,
+int launch_moe_combine(const float* x, float* out, const float* yexp, const int* inv, const float* weight, int top, const float* w, float eps, int M, int W,
                        hipStream_t s) {
     if (M <= 0) return ZG_OK;
-    moe_combine_kernel<<<M, 256, 0, s>>>(x, yexp, inv, weight, top, w, eps, W);
+    NormRows r;
+    r.x = x; r.x_out = out; r.yexp = yexp; r.inv = inv; r.weight = weight; r.top = top; r.wb = w; r.eps = eps; r.M = M; r.W = W;
+    bool taken = false;
+    ZG_TRY(launch_norm_rows(r, s, &taken));
+    if (taken) return ZG_OK;
+    moe_combine_kernel<<<M, 256, 0, s>>>(x, out, yexp, inv, weight, top, w, eps, W);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

@@ -1,0 +1,182 @@
+// lm_norm.hip — what happens to a row of the residual stream between two sublayers: the sublayer's output (a row, or the chosen experts'
+// rows with their weights) normed and added, the sum normed for the next sublayer and, in designs with a token shift, mixed with the
+// normed row of the token before.  Rows of up to 1024 values in whole 16-byte pieces; lm_mix.hip and lm_moe.hip have the general kernels.
+//
+// Bound by memory: a wave holds a row in its registers (16-byte pieces, all requested in one go), so the two statistics between the
+// loads and the stores are sums over one wave and nothing waits for other waves.  A wave takes a run of consecutive rows: the shift's
+// row before is the one it has just normed, except for the first of the run, which it works out again.  (Then x must not be updated in
+// place, since the run in front of it may have been written already.)
+// us per launch, in front with a workgroup per row and two barriers a statistic: 8184 rows of 1024, sum and two norms 27 (of 117 MB) : 55,
+// experts' rows added, normed and shifted 32 : 44 + 37 in two launches; 8 rows of 768 3.6 : 6.5 and 5.2 : 7.2.
+#include "lm_kernels.h"
+
+#include <algorithm>
+#include <cstdlib>
+
+namespace zg {
+namespace lm {
+
+namespace {
+
+enum { FROM_NOTHING, FROM_ROW, FROM_EXPERTS };
+enum { TO_NOTHING, TO_NORM, TO_SHIFT };
+
+template <int NV, int FROM, int TO>
+__global__ __launch_bounds__(256) void norm_rows_kernel(const NormRows p) {
+    const int lane = threadIdx.x & 63;
+    const int first = __builtin_amdgcn_readfirstlane((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * p.run);
+    if (first >= p.M) return;
+    const int W = p.W;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    int at[NV];
+    bool in[NV];
+#pragma unroll
+    for (int j = 0; j < NV; ++j) {
+        in[j] = lane * 4 + 256 * j < W;
+        at[j] = min(lane * 4 + 256 * j, W - 4);
+    }
+    auto load = [&](const float* row, f32x4 (&v)[NV]) {
+#pragma unroll
+        for (int j = 0; j < NV; ++j) v[j] = *reinterpret_cast<const f32x4*>(row + at[j]);
+    };
+    auto inv_rms = [&](const f32x4 (&v)[NV]) {
+        float ss = 0.0f;
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            const f32x4 a = in[j] ? v[j] : zero;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) ss = fmaf(a[e], a[e], ss);
+        }
+        return 1.0f / sqrtf(wave_allsum(ss) / (float)W + p.eps);
+    };
+    f32x4 wb[NV], wn[NV], mu[NV];
+    if constexpr (FROM != FROM_NOTHING) load(p.wb, wb);
+    if constexpr (TO != TO_NOTHING) load(p.wn, wn);
+    if constexpr (TO == TO_SHIFT) load(p.mu, mu);
+    // row m of the stream with the sublayer's output added
+    auto sum = [&](int m, f32x4 (&x)[NV]) {
+        load(p.x + (size_t)m * W, x);
+        if constexpr (FROM == FROM_NOTHING) return;
+        f32x4 y[NV];
+        if constexpr (FROM == FROM_ROW) load(p.y + (size_t)m * W, y);
+        else {
+#pragma unroll
+            for (int j = 0; j < NV; ++j) y[j] = zero;
+            for (int k = 0; k < p.top; k += 2) {
+                const size_t a = (size_t)m * p.top + k, b = a + (k + 1 < p.top ? 1 : 0);
+                const float fa = p.weight[a], fb = p.weight[b];
+                f32x4 u[NV], v[NV];
+                load(p.yexp + (size_t)(p.inv ? p.inv[a] : (int)a) * W, u);
+                load(p.yexp + (size_t)(p.inv ? p.inv[b] : (int)b) * W, v);
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) y[j][e] = fmaf(fa, u[j][e], y[j][e]);
+                if (k + 1 < p.top) {
+#pragma unroll
+                    for (int j = 0; j < NV; ++j)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) y[j][e] = fmaf(fb, v[j][e], y[j][e]);
+                }
+            }
+        }
+        const float r = inv_rms(y);
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[j][e] += y[j][e] * r * (1.0f + wb[j][e]);
+    };
+    auto norm = [&](const f32x4 (&x)[NV], f32x4 (&h)[NV]) {
+        const float r = inv_rms(x);
+#pragma unroll
+        for (int j = 0; j < NV; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) h[j][e] = x[j][e] * r * (1.0f + wn[j][e]);
+    };
+    f32x4 x[NV], h[NV], before[NV];
+    if constexpr (TO == TO_SHIFT) {
+        const int prev = p.row_prev ? p.row_prev[first] : -1;
+        if (prev >= 0) {
+            sum(prev, x);
+            norm(x, before);
+        }
+    }
+    for (int m = first; m < min(first + p.run, p.M); ++m) {
+        if constexpr (TO == TO_SHIFT) {
+            if (!p.row_prev || p.row_prev[m] < 0) load(p.shift_state + (size_t)p.row_slot[m] * p.slot_stride, before);
+        }
+        sum(m, x);
+        if constexpr (FROM != FROM_NOTHING) {
+#pragma unroll
+            for (int j = 0; j < NV; ++j)
+                if (in[j]) *reinterpret_cast<f32x4*>(p.x_out + (size_t)m * W + at[j]) = x[j];
+        }
+        if constexpr (TO == TO_NOTHING) continue;
+        norm(x, h);
+        if constexpr (TO == TO_SHIFT) {
+            const int entry = p.row_entry_if_last ? p.row_entry_if_last[m] : -1;
+            if (entry >= 0) {
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+                    if (in[j]) *reinterpret_cast<f32x4*>(p.last_out + (size_t)entry * W + at[j]) = h[j];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NV; ++j) {
+            f32x4 o = h[j];
+            if constexpr (TO == TO_SHIFT) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o[e] = h[j][e] + (before[j][e] - h[j][e]) * mu[j][e];
+                before[j] = h[j];
+            }
+            if (in[j]) {
+                if (p.out) *reinterpret_cast<f32x4*>(p.out + (size_t)m * W + at[j]) = o;
+                if (p.out16) *reinterpret_cast<u32x2*>(p.out16 + (size_t)m * W + at[j]) = u32x2{cvt_pk_bf16(o[0], o[1]), cvt_pk_bf16(o[2], o[3])};
+            }
+        }
+    }
+}
+
+}  // namespace
+
+int launch_norm_rows(const NormRows& in, hipStream_t s, bool* taken) {
+    *taken = false;
+    NormRows p = in;
+    if (p.M <= 0 || p.W < 4 || p.W > 1024 || p.W % 4 != 0) return ZG_OK;
+    const uintptr_t all = reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.x_out) | reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.yexp) |
+                          reinterpret_cast<uintptr_t>(p.wb) | reinterpret_cast<uintptr_t>(p.wn) | reinterpret_cast<uintptr_t>(p.mu) | reinterpret_cast<uintptr_t>(p.out) |
+                          reinterpret_cast<uintptr_t>(p.out16) | reinterpret_cast<uintptr_t>(p.shift_state) | reinterpret_cast<uintptr_t>(p.last_out);
+    if ((all & 15) != 0 || p.slot_stride % 4 != 0) return ZG_OK;
+    const int from = p.yexp ? FROM_EXPERTS : p.y ? FROM_ROW : FROM_NOTHING, to = p.mu ? TO_SHIFT : p.wn ? TO_NORM : TO_NOTHING;
+    if (from == FROM_NOTHING && to == TO_NOTHING) return ZG_OK;
+    if (from != FROM_NOTHING && to == TO_SHIFT && p.row_prev && p.x == p.x_out) return ZG_OK;  // (a run would read what another has written)
+    // Runs as long as 2048 waves are left (a run of eight works out one row in nine twice); few rows a wave each in workgroups of their own.
+    p.run = std::max(1, std::min(8, p.M / 2048));
+    if (const char* e = getenv("ZGPT2_LM_NORM_RUN")) p.run = std::max(1, atoi(e));  // (test hook: runs in short portions)
+    const int waves = (p.M + p.run - 1) / p.run, per_group = p.M <= 64 ? 1 : 4;
+    const dim3 grid((waves + per_group - 1) / per_group), block(64 * per_group);
+#define ZG_NR(NV, FROM, TO) (norm_rows_kernel<NV, FROM, TO><<<grid, block, 0, s>>>(p))
+#define ZG_NR_V(FROM, TO)                       \
+    do {                                        \
+        if (p.W <= 256) ZG_NR(1, FROM, TO);     \
+        else if (p.W <= 512) ZG_NR(2, FROM, TO); \
+        else if (p.W <= 768) ZG_NR(3, FROM, TO); \
+        else ZG_NR(4, FROM, TO);                \
+    } while (0)
+    if (from == FROM_NOTHING && to == TO_NORM) ZG_NR_V(FROM_NOTHING, TO_NORM);
+    else if (from == FROM_NOTHING) ZG_NR_V(FROM_NOTHING, TO_SHIFT);
+    else if (from == FROM_ROW && to == TO_NOTHING) ZG_NR_V(FROM_ROW, TO_NOTHING);
+    else if (from == FROM_ROW && to == TO_NORM) ZG_NR_V(FROM_ROW, TO_NORM);
+    else if (from == FROM_ROW) ZG_NR_V(FROM_ROW, TO_SHIFT);
+    else if (to == TO_NOTHING) ZG_NR_V(FROM_EXPERTS, TO_NOTHING);
+    else if (to == TO_NORM) ZG_NR_V(FROM_EXPERTS, TO_NORM);
+    else ZG_NR_V(FROM_EXPERTS, TO_SHIFT);
+#undef ZG_NR
+#undef ZG_NR_V
+    ZG_HIP(hipGetLastError());
+    *taken = true;
+    return ZG_OK;
+}
+
+}  // namespace lm
+}  // namespace zg
