@@ -786,15 +786,46 @@ __global__ __launch_bounds__(256) void latent_prep_kernel(const float* proj, int
                                                           float eps, Rotary rot, const int* row_pos, const int* row_slot, const int* page_table,
                                                           int max_pages, int page_tokens, float* cq, float* cache, bf16_t* cq16) {
     __shared__ float s_red[8];
-    const int m = blockIdx.x;
+    const int m = blockIdx.x, pos = row_pos[m];
     const float* row = proj + (size_t)m * ld;
-    const float rq = row_inv_rms(row, q_rank, eps, s_red);
-    const float rc = row_inv_rms(row + q_rank, KR, eps, s_red);
-    for (int i = threadIdx.x; i < q_rank; i += blockDim.x) put_row(cq16 ? nullptr : cq, cq16, (size_t)m * q_rank + i, row[i] * rq * wq[i]);
-    const int pos = row_pos[m];
     float* crow = cache + cache_row(page_table, max_pages, page_tokens, row_slot[m], pos) * (size_t)(KR + R);
-    for (int i = threadIdx.x; i < KR; i += blockDim.x) crow[i] = row[q_rank + i] * rc * wkv[i];
     const float* kr = row + q_rank + KR;
+    if (q_rank + KR <= 1024) {  // both parts in registers, requested in one go with their weights
+        const int n = q_rank + KR;
+        float v[4], w[4], sq = 0.0f, sc = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = min((int)threadIdx.x + 256 * j, n - 1);
+            v[j] = row[i];
+            w[j] = i < q_rank ? wq[i] : wkv[i - q_rank];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            if (i < q_rank) sq = fmaf(v[j], v[j], sq);
+            else if (i < n) sc = fmaf(v[j], v[j], sc);
+        }
+        sq = wave_allsum(sq);
+        sc = wave_allsum(sc);
+        if ((threadIdx.x & 63) == 0) {
+            s_red[threadIdx.x >> 6] = sq;
+            s_red[4 + (threadIdx.x >> 6)] = sc;
+        }
+        __syncthreads();
+        const float rq = 1.0f / sqrtf(((s_red[0] + s_red[1]) + (s_red[2] + s_red[3])) / (float)q_rank + eps);
+        const float rc = 1.0f / sqrtf(((s_red[4] + s_red[5]) + (s_red[6] + s_red[7])) / (float)KR + eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = threadIdx.x + 256 * j;
+            if (i < q_rank) put_row(cq16 ? nullptr : cq, cq16, (size_t)m * q_rank + i, v[j] * rq * w[j]);
+            else if (i < n) crow[i - q_rank] = v[j] * rc * w[j];
+        }
+    } else {
+        const float rq = row_inv_rms(row, q_rank, eps, s_red);
+        const float rc = row_inv_rms(row + q_rank, KR, eps, s_red);
+        for (int i = threadIdx.x; i < q_rank; i += blockDim.x) put_row(cq16 ? nullptr : cq, cq16, (size_t)m * q_rank + i, row[i] * rq * wq[i]);
+        for (int i = threadIdx.x; i < KR; i += blockDim.x) crow[i] = row[q_rank + i] * rc * wkv[i];
+    }
     for (int i = threadIdx.x; i < rot.dims / 2; i += blockDim.x) rotate_pair(kr, crow + KR, i, pos, rot);
     for (int i = rot.dims + threadIdx.x; i < R; i += blockDim.x) crow[KR + i] = kr[i];
 }
@@ -846,9 +877,11 @@ __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* pr
 
 // One workgroup per (row, head).  The lanes of a wave split the KR + R dimensions of a cache row (ND per lane); a wave walks
 // its share of the keys four at a time with a running (maximum, sum, weighted latent) and the four waves are merged at the end.
-// With n_split > 1 (decode steps: few rows, long key ranges) grid.z workgroups share a row's keys in ranges of at least 64
+// With n_split > 1 (decode steps: few rows, long key ranges) grid.z workgroups share a row's keys in ranges of whole groups of 16
 // and leave (maximum, sum, weighted latent) partials in ws for latent_merge_kernel.
 // gate (may be null): head h's result is multiplied by sigmoid(gate[m ldg + h]) where it is written.
+// 8 rows, 12 heads on latents of 256 + 32, some 300 keys: 4.6 us and 3.2 for the merge (13.4 and 4.6 with loads under their own bounds
+// checks and ranges of 64 keys and more: four dependent round trips instead of one).
 // 1 / (L + exp(sink - mx)) times what brings weights of reference point mx to that denominator's (L: sum of exp(score - mx); mx -inf:
 // no keys).  sink null: 1 / L.
 __device__ __forceinline__ float sink_norm_f(float mx, float L, const float* sink, int h) {
@@ -872,7 +905,7 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, 
     int k_lo = 0, k_hi = n_keys;
     if (n_split > 1) {
         int chunk = (n_keys + n_split - 1) / n_split;
-        chunk = max(64, (chunk + 15) & ~15);
+        chunk = (chunk + 15) & ~15;
         k_lo = min(n_keys, (int)blockIdx.z * chunk);
         k_hi = min(n_keys, k_lo + chunk);
     }
@@ -881,7 +914,8 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, 
 #pragma unroll
     for (int i = 0; i < ND; ++i) {
         const int d = lane + 64 * i;
-        q[i] = d < DT ? qrow[d] : 0.0f;
+        const float v = qrow[min(d, DT - 1)];
+        q[i] = d < DT ? v : 0.0f;
         acc[i] = 0.0f;
     }
     float mx = -INFINITY, l = 0.0f;
@@ -892,11 +926,17 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, 
         for (int u = 0; u < 4; ++u) {
             const int key = kb + u < k_hi ? kb + u : kb;
             const float* row = cache + ((size_t)pt[key / page_tokens] * page_tokens + key % page_tokens) * DT;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) {
+                r[u][i] = row[min(lane + 64 * i, DT - 1)];  // (unconditional: every load in flight before the first is used)
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
             float part = 0.0f;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
-                const int d = lane + 64 * i;
-                r[u][i] = d < DT ? row[d] : 0.0f;
+                if (lane + 64 * i >= DT) r[u][i] = 0.0f;
                 part = fmaf(q[i], r[u][i], part);
             }
             s[u] = part;
@@ -1427,7 +1467,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* ws, floa
     __shared__ float s_L, s_M;
     const int m = blockIdx.x, h = blockIdx.y, n_keys = row_pos[m] + 1;
     int chunk = (n_keys + n_split - 1) / n_split;
-    chunk = max(64, (chunk + 15) & ~15);
+    chunk = (chunk + 15) & ~15;
     const int used = min(n_split, (n_keys + chunk - 1) / chunk);
     const float* part = ws + ((size_t)m * H + h) * n_split * (KR + 2);
     if (threadIdx.x < 64) {
@@ -1447,7 +1487,14 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* ws, floa
     const float L = s_L, gf = head_gate_f(gate, ldg, m, h) * (sink ? sink_norm_f(s_M, L, sink, h) : 1.0f);
     for (int d = threadIdx.x; d < KR; d += blockDim.x) {
         float a = 0.0f;
-        for (int sidx = 0; sidx < used; ++sidx) a = fmaf(s_w[sidx], part[(size_t)sidx * (KR + 2) + 2 + d], a);
+        for (int s0 = 0; s0 < used; s0 += 16) {  // sixteen partials in flight (those beyond the last repeat it with weight 0)
+            float v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = part[(size_t)min(s0 + u, used - 1) * (KR + 2) + 2 + d];
+#pragma unroll
+            for (int u = 0; u < 16; ++u)
+                if (s0 + u < used) a = fmaf(s_w[s0 + u], v[u], a);
+        }
         out[d] = sink ? a * gf : a / L * gf;
     }
 }
@@ -1847,6 +1894,7 @@ int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, i
     else if (nd <= 2) ZG_ATT(2);
     else if (nd <= 3) ZG_ATT(3);
     else if (nd <= 4) ZG_ATT(4);
+    else if (nd <= 5) ZG_ATT(5);
     else if (nd <= 6) ZG_ATT(6);
     else if (nd <= 9) ZG_ATT(9);
     else if (nd <= 12) ZG_ATT(12);
