@@ -1,0 +1,61 @@
+"""Generation that enqueues its steps ahead against the same steps taken one by one (use_graph=False takes them so): tokens of greedy and
+sampled runs longer than the ring of steps in flight, pages that run over and go back to the pool behind windows, key-length buckets,
+and a cache that is full half way."""
+import numpy as np
+import pytest
+
+import duvulix_testlib as dl
+import lm_testlib as tl
+from zig_gpt2_amd import lm
+
+pytestmark = pytest.mark.gpu
+
+DESIGNS = {
+    "latent": (tl, tl.config([tl.hgrn2_layer(mlp=tl.moe_mlp()), tl.latent_layer(mlp=tl.dense_mlp())], vocab=97, width=48)),
+    "chunks": (dl, dl.config([dl.attn_layer(mlp=dl.dense()), dl.attn_layer(size=5, mlp=None)], width=48)),
+    "mixed": (dl, dl.config([dl.mamba_layer(mlp=dl.dense()), dl.latent_layer(mlp=dl.dense()), dl.attn_layer(mlp=None)], width=48)),
+    "whole": (dl, dl.config([dl.attn_layer(size=None, mlp=dl.dense())], width=48)),
+}
+
+
+@pytest.mark.parametrize("n_seqs", [1, 3, 8])
+@pytest.mark.parametrize("design", sorted(DESIGNS))
+def test_tokens_of_steps_ahead(design, n_seqs):
+    lib, cfg = DESIGNS[design]
+    w = lib.weights(cfg, seed=7)
+    prompts = [lib.tokens(b, 3 + 5 * b, cfg["vocab"]) for b in range(n_seqs)]
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=1024, max_seqs=8, page_tokens=8, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append([m.generate(prompts, n, temp=t, seed=s) for n, t, s in ((1, 0.0, 0), (2, 0.0, 0), (9, 0.0, 0), (40, 0.0, 0), (40, 1.5, 5))])
+        runs[-1].append(m.generate(prompts, 40))  # the slots and pages are all back
+        m.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
+def test_key_buckets():
+    lib, cfg = DESIGNS["whole"]
+    w = lib.weights(cfg, seed=2)
+    prompts = [lib.tokens(1, 500, cfg["vocab"])]
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=2048, max_seqs=2, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append(m.generate(prompts, 30))
+        m.close()
+    assert np.array_equal(*runs)
+
+
+def test_a_cache_that_is_full_half_way():
+    lib, cfg = DESIGNS["latent"]
+    w = lib.weights(cfg, seed=3)
+    prompts = [lib.tokens(b, 6, cfg["vocab"]) for b in range(2)]
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=48, max_seqs=4, page_tokens=8)
+    m.load_weights(w)
+    want = m.generate(prompts, 17)
+    with pytest.raises(Exception, match="pages needed|tokens in the cache"):
+        m.generate(prompts, 60)
+    assert np.array_equal(m.generate(prompts, 17), want)
+    m.close()

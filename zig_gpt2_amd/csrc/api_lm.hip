@@ -237,6 +237,11 @@ struct zg_lm {
     float* h_logits = nullptr;  // pinned [logit_rows][V]
     int* h_small = nullptr;     // pinned: sampled tokens [logit_rows], fault flag
     float* h_u = nullptr;       // pinned uniforms [logit_rows]
+    // generation enqueues steps ahead of the tokens it has seen: of the last kAhead steps the tokens, the uniforms and an event (pinned)
+    static constexpr int kAhead = 8;
+    int* h_ahead = nullptr;        // [kAhead][kGemvMaxRows]
+    float* h_ahead_u = nullptr;    // [kAhead][kGemvMaxRows]
+    hipEvent_t ahead_done[kAhead] = {};
     float* trace = nullptr;
     size_t trace_floats = 0;
     float last_step_ms = 0.0f, last_decode_ms = 0.0f;
@@ -1622,18 +1627,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     return ZG_OK;
 }
 
-// ------------------------------------------------------------------------------------------------ one portion of rows
-int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, const Sampler* sampler) {
+// The rows of a portion and their pages: metadata to the pinned twin and to the device.  wants: (row of the portion, output row)
+int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair<int, size_t>>& wants) {
     hipStream_t s = g->stream;
-    const int W = g->W, MS = g->MS, NS = g->NS;
-    int M = 0;
-    for (const Piece& pc : pieces) M += pc.n;
-    if (M == 0) return ZG_OK;
-    const int n_ent = (int)pieces.size();
+    const int MS = g->MS, NS = g->NS, n_ent = (int)pieces.size();
     int *ids = g->h_meta, *pos = ids + MS, *slot = pos + MS, *prev = slot + MS, *lastent = prev + MS, *want_rows = lastent + MS;
     int *ent_start = want_rows + MS, *ent_len = ent_start + NS, *ent_slot = ent_len + NS;
     int* row_off = g->h_meta + meta_row_off(g);
-    std::vector<std::pair<int, size_t>> wants;  // (row of the portion, output row)
     int r = 0;
     g->step_keys = 0;
     g->step_key_tiles = 0;
@@ -1659,13 +1659,11 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
         ZG_HIP(hipMemcpyAsync(g->page_table + (size_t)pc.slot * g->max_pages, sl.ring.data(), sl.ring.size() * sizeof(int), hipMemcpyHostToDevice, s));
     }
     ZG_HIP(hipMemcpyAsync(g->meta, g->h_meta, meta_ints(g) * sizeof(int), hipMemcpyHostToDevice, s));
-    const int* d_want = g->meta + 5 * (size_t)MS;
-    const bool f32 = g->f32;
-    const float eps = g->cfg.norm_eps;
+    return ZG_OK;
+}
 
-    ZG_HIP(hipEventRecord(g->ev0, s));
-    bool single = M <= kGemvMaxRows && !g->trace && g->use_graph;
-    for (const Piece& pc : pieces) single = single && pc.n == 1;
+// key-length bucket of the captured decode step the running one replays
+int key_bucket(zg_lm* g) {
     int bucket = 0;
     g->bucket_keys = 0;
     if (g->whole_context) {  // the smallest bucket that holds the longest sequence of the step
@@ -1673,21 +1671,71 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
         while (bucket + 1 < zg_lm::kKeyBuckets && (512LL << bucket) < g->step_keys) ++bucket;
         g->bucket_keys = (int)std::min<long long>(all_keys, 512LL << bucket);
     }
-    if (single) {  // a decode step: replay the captured sequence of this batch size
-        if (!g->decode_graph[M][bucket]) {
-            hipGraph_t graph = nullptr;
-            ZG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-            const int st = enqueue_layers(g, M, n_ent, true, true);
-            const hipError_t ce = hipStreamEndCapture(s, &graph);
-            if (st != ZG_OK) {
-                if (graph) (void)hipGraphDestroy(graph);
-                return st;
-            }
-            ZG_HIP(ce);
-            ZG_HIP(hipGraphInstantiate(&g->decode_graph[M][bucket], graph, nullptr, nullptr, 0));
-            ZG_HIP(hipGraphDestroy(graph));
+    return bucket;
+}
+
+// a decode step: replay the captured sequence of this batch size
+int replay_step(zg_lm* g, int M, int bucket) {
+    hipStream_t s = g->stream;
+    if (!g->decode_graph[M][bucket]) {
+        hipGraph_t graph = nullptr;
+        ZG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+        const int st = enqueue_layers(g, M, M, true, true);
+        const hipError_t ce = hipStreamEndCapture(s, &graph);
+        if (st != ZG_OK) {
+            if (graph) (void)hipGraphDestroy(graph);
+            return st;
         }
-        ZG_HIP(hipGraphLaunch(g->decode_graph[M][bucket], s));
+        ZG_HIP(ce);
+        ZG_HIP(hipGraphInstantiate(&g->decode_graph[M][bucket], graph, nullptr, nullptr, 0));
+        ZG_HIP(hipGraphDestroy(graph));
+    }
+    ZG_HIP(hipGraphLaunch(g->decode_graph[M][bucket], s));
+    return ZG_OK;
+}
+
+// logits of the nw rows the metadata asks for
+int enqueue_logits(zg_lm* g, int nw) {
+    const int* d_want = g->meta + 5 * (size_t)g->MS;
+    const int W = g->W;
+    if (g->tanh_norms) ZG_TRY(launch_tanh_norm(g->x, nullptr, g->final_norm, d_want, g->hn, nw, W, g->stream));
+    else ZG_TRY(launch_norm_gather(g->x, d_want, g->final_norm, g->cfg.norm_eps, g->hn, nw, W, g->side, g->stream));
+    Linear lin;
+    lin.A = g->hn; lin.lda = W; lin.B = g->head; lin.ldb = W; lin.C = g->logits; lin.ldc = g->V; lin.M = nw; lin.N = g->V; lin.K = W;
+    if ((g->cfg.logit_scale != 0.0f && g->cfg.logit_scale != 1.0f) || g->cfg.logit_softcap > 0.0f) {
+        lin.act = ACT_SCALE_SOFTCAP;
+        lin.act_a = g->cfg.logit_scale != 0.0f ? g->cfg.logit_scale : 1.0f;
+        lin.act_b = g->cfg.logit_softcap;
+    }
+    return launch_linear(lin, g->f32, g->stream);
+}
+
+// the uniform of (seed, length of the sequence with the token to be drawn, output row)
+float draw_uniform(uint64_t seed, int pos, size_t out_row) {
+    uint64_t z = seed * 0x9E3779B97F4A7C15ULL + (uint64_t)(pos + 2) * 0xD1B54A32D192ED03ULL + out_row + 1;
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
+    z ^= z >> 31;
+    return (float)(uint32_t)(z >> 40) * 5.9604644775390625e-08f;
+}
+
+// ------------------------------------------------------------------------------------------------ one portion of rows
+int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, const Sampler* sampler) {
+    hipStream_t s = g->stream;
+    const int MS = g->MS;
+    int M = 0;
+    for (const Piece& pc : pieces) M += pc.n;
+    if (M == 0) return ZG_OK;
+    const int n_ent = (int)pieces.size();
+    int *pos = g->h_meta + MS, *want_rows = g->h_meta + 5 * (size_t)MS;
+    std::vector<std::pair<int, size_t>> wants;  // (row of the portion, output row)
+    ZG_TRY(stage_rows(g, pieces, wants));
+    ZG_HIP(hipEventRecord(g->ev0, s));
+    bool single = M <= kGemvMaxRows && !g->trace && g->use_graph;
+    for (const Piece& pc : pieces) single = single && pc.n == 1;
+    const int bucket = key_bucket(g);
+    if (single) {
+        ZG_TRY(replay_step(g, M, bucket));
     } else {
         bool one_row = M <= kGemvMaxRows;
         for (const Piece& pc : pieces) one_row = one_row && pc.n == 1;
@@ -1703,27 +1751,11 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
             // so the twin is free again when the next batch fills it)
             for (int j = 0; j < nw; ++j) want_rows[j] = wants[w0 + j].first;
             ZG_HIP(hipMemcpyAsync(g->meta + 5 * (size_t)MS, want_rows, nw * sizeof(int), hipMemcpyHostToDevice, s));
-            if (g->tanh_norms) ZG_TRY(launch_tanh_norm(g->x, nullptr, g->final_norm, d_want, g->hn, nw, W, s));
-            else ZG_TRY(launch_norm_gather(g->x, d_want, g->final_norm, eps, g->hn, nw, W, g->side, s));
-            Linear lin;
-            lin.A = g->hn; lin.lda = W; lin.B = g->head; lin.ldb = W; lin.C = g->logits; lin.ldc = g->V; lin.M = nw; lin.N = g->V; lin.K = W;
-            if ((g->cfg.logit_scale != 0.0f && g->cfg.logit_scale != 1.0f) || g->cfg.logit_softcap > 0.0f) {
-                lin.act = ACT_SCALE_SOFTCAP;
-                lin.act_a = g->cfg.logit_scale != 0.0f ? g->cfg.logit_scale : 1.0f;
-                lin.act_b = g->cfg.logit_softcap;
-            }
-            ZG_TRY(launch_linear(lin, f32, s));
+            ZG_TRY(enqueue_logits(g, nw));
             if (sampler) {
                 ZG_TRY(launch_row_argmax(g->logits, nw, g->V, g->row_max, g->tok_out, g->amax_val, g->amax_idx, s));
                 if (sampler->temp > 0.0f) {
-                    for (int j = 0; j < nw; ++j) {  // the uniform of (seed, length of the sequence with the token to be drawn, output row)
-                        const int row = wants[w0 + j].first;
-                        uint64_t z = sampler->seed * 0x9E3779B97F4A7C15ULL + (uint64_t)(pos[row] + 2) * 0xD1B54A32D192ED03ULL + wants[w0 + j].second + 1;
-                        z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ULL;
-                        z = (z ^ (z >> 27)) * 0x94D049BB133111EBULL;
-                        z ^= z >> 31;
-                        g->h_u[j] = (float)(uint32_t)(z >> 40) * 5.9604644775390625e-08f;
-                    }
+                    for (int j = 0; j < nw; ++j) g->h_u[j] = draw_uniform(sampler->seed, pos[wants[w0 + j].first], wants[w0 + j].second);
                     ZG_HIP(hipMemcpyAsync(g->samp_u, g->h_u, nw * sizeof(float), hipMemcpyHostToDevice, s));
                     ZG_TRY(launch_sample(g->logits, nw, g->V, sampler->temp, g->samp_u, g->row_max, 1, 1, g->samp_ws, g->tok_out, false, s));
                 }
@@ -1749,6 +1781,42 @@ int run_portion(zg_lm* g, const std::vector<Piece>& pieces, float* logits_out, c
     return ZG_OK;
 }
 
+// Pages of a sequence that grows by n tokens: what it needs (an error where the cache cannot hold it), whether the pool has them, taken;
+// and given back, once every token of theirs lies behind the longest window.
+int count_pages(const zg_lm* g, int seq, size_t n, size_t& need) {
+    const Slot& sl = g->slots[seq];
+    const size_t pages = (sl.len + n + g->P - 1) / g->P;
+    ZG_REQUIRE(pages - sl.first_live <= (size_t)g->max_pages, ZG_ERR_SHAPE, "lm_step: sequence %d would hold %zu tokens in the cache (at most %zu)", seq,
+               sl.len + n - sl.first_live * g->P, (size_t)g->max_pages * g->P);
+    need += pages > sl.pages.size() ? pages - sl.pages.size() : 0;
+    return ZG_OK;
+}
+int pages_left(const zg_lm* g, size_t need) {
+    ZG_REQUIRE(need <= g->free_pages.size(), ZG_ERR_SHAPE, "lm_step: %zu cache pages needed, %zu free (max_tokens %zu)", need, g->free_pages.size(),
+               g->cfg.max_tokens);
+    return ZG_OK;
+}
+bool take_pages(zg_lm* g, Slot& sl, size_t n) {
+    const size_t pages = (sl.len + n + g->P - 1) / g->P;
+    const bool any = sl.pages.size() < pages;
+    while (sl.pages.size() < pages) {
+        sl.ring[sl.pages.size() % g->max_pages] = g->free_pages.back();
+        sl.pages.push_back(g->free_pages.back());
+        g->free_pages.pop_back();
+    }
+    return any;
+}
+void return_pages(zg_lm* g, Slot& sl) {
+    if (g->keep_tokens <= 0 || sl.len + 1 <= (size_t)g->keep_tokens) return;
+    const size_t dead = (sl.len + 1 - g->keep_tokens) / g->P;  // the next token sees positions >= len + 1 - keep
+    for (size_t pg = g->keep_pages; pg < dead && pg < sl.pages.size(); ++pg)
+        if (sl.pages[pg] >= 0) {
+            g->free_pages.push_back(sl.pages[pg]);
+            sl.pages[pg] = -1;
+        }
+    if (g->keep_pages == 0) sl.first_live = std::max(sl.first_live, std::min(dead, sl.pages.size()));
+}
+
 int step_impl(zg_lm* g, const zg_lm_entry* entries, size_t n_entries, float* logits_out, size_t logits_len, const Sampler* sampler) {
     ZG_REQUIRE(g && (entries || n_entries == 0), ZG_ERR_ARG, "lm_step: bad argument");
     ZG_HIP(hipSetDevice(g->device));
@@ -1765,25 +1833,12 @@ int step_impl(zg_lm* g, const zg_lm_entry* entries, size_t n_entries, float* log
             ZG_REQUIRE(e.want[j] >= 0 && (size_t)e.want[j] < e.n_tokens, ZG_ERR_ARG, "lm_step: entry %zu asks for place %d of %zu tokens", i, e.want[j],
                        e.n_tokens);
         n_want += e.n_want;
-        const Slot& sl = g->slots[e.seq];
-        const size_t pages = (sl.len + e.n_tokens + g->P - 1) / g->P;
-        ZG_REQUIRE(pages - sl.first_live <= (size_t)g->max_pages, ZG_ERR_SHAPE, "lm_step: sequence %d would hold %zu tokens in the cache (at most %zu)",
-                   e.seq, sl.len + e.n_tokens - sl.first_live * g->P, (size_t)g->max_pages * g->P);
-        need_pages += pages > sl.pages.size() ? pages - sl.pages.size() : 0;
+        ZG_TRY(count_pages(g, e.seq, e.n_tokens, need_pages));
     }
-    ZG_REQUIRE(need_pages <= g->free_pages.size(), ZG_ERR_SHAPE, "lm_step: %zu cache pages needed, %zu free (max_tokens %zu)", need_pages,
-               g->free_pages.size(), g->cfg.max_tokens);
+    ZG_TRY(pages_left(g, need_pages));
     ZG_REQUIRE(sampler || n_want == 0 || (logits_out && logits_len >= n_want * (size_t)g->V), ZG_ERR_SHAPE, "lm_step: logits_out needs %zu elements",
                n_want * (size_t)g->V);
-    for (size_t i = 0; i < n_entries; ++i) {
-        Slot& sl = g->slots[entries[i].seq];
-        const size_t pages = (sl.len + entries[i].n_tokens + g->P - 1) / g->P;
-        while (sl.pages.size() < pages) {
-            sl.ring[sl.pages.size() % g->max_pages] = g->free_pages.back();
-            sl.pages.push_back(g->free_pages.back());
-            g->free_pages.pop_back();
-        }
-    }
+    for (size_t i = 0; i < n_entries; ++i) take_pages(g, g->slots[entries[i].seq], entries[i].n_tokens);
     g->last_step_ms = 0.0f;
     // cut the entries into portions of at most max_step_tokens rows
     std::vector<Piece> pieces;
@@ -1815,18 +1870,82 @@ int step_impl(zg_lm* g, const zg_lm_entry* entries, size_t n_entries, float* log
         out_base += e.n_want;
     }
     if (!pieces.empty()) ZG_TRY(run_portion(g, pieces, logits_out, sampler));
-    if (g->keep_tokens > 0)  // pages whose every token lies behind the longest window return to the pool
-        for (size_t i = 0; i < n_entries; ++i) {
-            Slot& sl = g->slots[entries[i].seq];
-            if (sl.len + 1 <= (size_t)g->keep_tokens) continue;
-            const size_t dead = (sl.len + 1 - g->keep_tokens) / g->P;  // the next token sees positions >= len + 1 - keep
-            for (size_t pg = g->keep_pages; pg < dead && pg < sl.pages.size(); ++pg)
-                if (sl.pages[pg] >= 0) {
-                    g->free_pages.push_back(sl.pages[pg]);
-                    sl.pages[pg] = -1;
-                }
-            if (g->keep_pages == 0) sl.first_live = std::max(sl.first_live, std::min(dead, sl.pages.size()));
+    for (size_t i = 0; i < n_entries; ++i) return_pages(g, g->slots[entries[i].seq]);
+    return ZG_OK;
+}
+
+// The steps of a generation behind its prompts: every sequence one token at a time.  What a step needs from the one before it, the tokens
+// and positions, is handed on by the device (advance_rows), so steps are enqueued ahead of the tokens the host has seen (at most kAhead)
+// and no step waits for a round trip to the host.  Bookkeeping and errors are those of the steps taken one by one: tokens of the steps
+// in front of a failing one are delivered.  first: the tokens the prompts' step drew.
+int decode_ahead(zg_lm* g, const std::vector<int>& seqs, const int32_t* first, size_t n_new, float temp, uint64_t seed, int32_t* out_tokens) {
+    hipStream_t s = g->stream;
+    const int M = (int)seqs.size(), MS = g->MS;
+    ZG_HIP(hipSetDevice(g->device));
+    size_t enqueued = 1, seen = 1;  // tokens of every sequence
+    auto collect = [&]() -> int {
+        const int at = (int)(seen % zg_lm::kAhead);
+        ZG_HIP(hipEventSynchronize(g->ahead_done[at]));
+        for (int b = 0; b < M; ++b) out_tokens[b * n_new + seen] = g->h_ahead[at * kGemvMaxRows + b];
+        ++seen;
+        return ZG_OK;
+    };
+    auto enqueue = [&]() -> int {
+        size_t need = 0;
+        for (int b = 0; b < M; ++b) ZG_TRY(count_pages(g, seqs[b], 1, need));
+        ZG_TRY(pages_left(g, need));
+        std::vector<Piece> pieces;
+        g->step_keys = 0;
+        for (int b = 0; b < M; ++b) {
+            Slot& sl = g->slots[seqs[b]];
+            const bool grew = take_pages(g, sl, 1);
+            if (enqueued == 1) {
+                Piece pc;
+                pc.slot = seqs[b]; pc.tok = first + b; pc.n = 1; pc.pos0 = (int)sl.len;
+                pieces.push_back(pc);
+            } else if (grew) {
+                ZG_HIP(hipMemcpyAsync(g->page_table + (size_t)seqs[b] * g->max_pages, sl.ring.data(), sl.ring.size() * sizeof(int), hipMemcpyHostToDevice, s));
+            }
+            g->step_keys = std::max(g->step_keys, (int)sl.len + 1);
         }
+        if (enqueued == 1) {
+            std::vector<std::pair<int, size_t>> wants;
+            for (int b = 0; b < M; ++b) g->h_meta[5 * (size_t)MS + b] = b;
+            ZG_TRY(stage_rows(g, pieces, wants));
+            ZG_HIP(hipEventRecord(g->ev0, s));
+        }
+        const int at = (int)(enqueued % zg_lm::kAhead);
+        ZG_TRY(replay_step(g, M, key_bucket(g)));
+        ZG_TRY(enqueue_logits(g, M));
+        ZG_TRY(launch_row_argmax(g->logits, M, g->V, g->row_max, g->tok_out, g->amax_val, g->amax_idx, s));
+        if (temp > 0.0f) {
+            float* u = g->h_ahead_u + at * kGemvMaxRows;
+            for (int b = 0; b < M; ++b) u[b] = draw_uniform(seed, (int)g->slots[seqs[b]].len, b);
+            ZG_HIP(hipMemcpyAsync(g->samp_u, u, M * sizeof(float), hipMemcpyHostToDevice, s));
+            ZG_TRY(launch_sample(g->logits, M, g->V, temp, g->samp_u, g->row_max, 1, 1, g->samp_ws, g->tok_out, false, s));
+        }
+        ZG_TRY(launch_advance_rows(g->tok_out, M, g->meta, g->meta + MS, g->h_ahead + at * kGemvMaxRows, s));
+        ZG_HIP(hipEventRecord(g->ahead_done[at], s));
+        for (int b = 0; b < M; ++b) {
+            ++g->slots[seqs[b]].len;
+            return_pages(g, g->slots[seqs[b]]);
+        }
+        ++enqueued;
+        return ZG_OK;
+    };
+    int status = ZG_OK;
+    while (enqueued < n_new && status == ZG_OK) {
+        if (enqueued - seen == (size_t)zg_lm::kAhead) status = collect();  // (its place in the rings is needed again)
+        if (status == ZG_OK) status = enqueue();
+    }
+    if (enqueued > 1) (void)hipEventRecord(g->ev1, s);
+    const hipError_t drained = hipStreamSynchronize(s);
+    while (drained == hipSuccess && seen < enqueued) ZG_TRY(collect());
+    if (status != ZG_OK) return status;
+    ZG_HIP(drained);
+    float ms = 0.0f;
+    if (enqueued > 1) ZG_HIP(hipEventElapsedTime(&ms, g->ev0, g->ev1));
+    g->last_step_ms = g->last_decode_ms = enqueued > 1 ? ms / (float)(enqueued - 1) : 0.0f;
     return ZG_OK;
 }
 
@@ -2034,6 +2153,9 @@ int zg_lm_create(zg_lm** out, const zg_lm_config* config, int device) {
     ZG_LM_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->h_logits), (size_t)g->logit_rows * g->V * sizeof(float), hipHostMallocDefault));
     ZG_LM_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->h_small), (g->logit_rows + 16) * sizeof(int), hipHostMallocDefault));
     ZG_LM_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->h_u), g->logit_rows * sizeof(float), hipHostMallocDefault));
+    ZG_LM_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->h_ahead), zg_lm::kAhead * kGemvMaxRows * sizeof(int), hipHostMallocDefault));
+    ZG_LM_TRY_HIP(hipHostMalloc(reinterpret_cast<void**>(&g->h_ahead_u), zg_lm::kAhead * kGemvMaxRows * sizeof(float), hipHostMallocDefault));
+    for (hipEvent_t& e : g->ahead_done) ZG_LM_TRY_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     memset(g->h_meta, 0, meta_ints(g) * sizeof(int));
     // state and flags start at zero; rotary tables
     const size_t state_floats = (size_t)g->NS * g->n_passes * g->W;
@@ -2095,6 +2217,10 @@ int zg_lm_destroy(zg_lm* g) {
     if (g->h_logits) (void)hipHostFree(g->h_logits);
     if (g->h_small) (void)hipHostFree(g->h_small);
     if (g->h_u) (void)hipHostFree(g->h_u);
+    if (g->h_ahead) (void)hipHostFree(g->h_ahead);
+    if (g->h_ahead_u) (void)hipHostFree(g->h_ahead_u);
+    for (hipEvent_t e : g->ahead_done)
+        if (e) (void)hipEventDestroy(e);
     if (g->arena) (void)hipFree(g->arena);
     delete g;
     return ZG_OK;
@@ -2268,6 +2394,12 @@ int zg_lm_generate(zg_lm* g, const int32_t* prompts, size_t prompt_stride, const
         }
         status = step_impl(g, ent.data(), n_prompts, nullptr, 0, &sm);
         if (status != ZG_OK) break;
+        if (i == 0 && n_new > 1 && n_prompts <= (size_t)kGemvMaxRows && !g->trace && g->use_graph) {
+            for (size_t b = 0; b < n_prompts; ++b) out_tokens[b * n_new] = cur[b];
+            status = decode_ahead(g, seqs, cur.data(), n_new, temp, seed, out_tokens);
+            for (int sq : seqs) zg_lm_seq_close(g, sq);
+            return status;
+        }
         if (i > 0) {
             decode_ms += g->last_step_ms;
             ++decode_steps;

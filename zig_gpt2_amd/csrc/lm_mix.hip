@@ -1499,6 +1499,16 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* ws, floa
     }
 }
 
+// the next step's rows: the tokens this one drew, one position further; also to host memory
+__global__ __launch_bounds__(64) void advance_rows_kernel(const int* tok, int M, int* ids, int* pos, int* seen) {
+    const int r = blockIdx.x * 64 + threadIdx.x;
+    if (r >= M) return;
+    const int t = tok[r];
+    ids[r] = t;
+    pos[r] += 1;
+    seen[r] = t;
+}
+
 // Stage 1: block (row, part) finds the maximum and its first index in its slice of the row; stage 2 (parts == 1 in the grid,
 // n_parts > 0 as argument): one block per row combines the parts.  The first maximum wins; a row of NaNs gives index 0.
 __global__ __launch_bounds__(256) void row_argmax_kernel(const float* logits, int n, float* max_out, int* idx_out, float* part_val, int* part_idx,
@@ -1905,6 +1915,13 @@ int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, i
         latent_merge_kernel<<<dim3(M, H), 256, 0, s>>>(ws, ctx, H, KR, n_split, row_pos, gate, ldg, sink);
         ZG_HIP(hipGetLastError());
     }
+    return ZG_OK;
+}
+
+int launch_advance_rows(const int* tok, int M, int* ids, int* pos, int* seen, hipStream_t s) {
+    if (M <= 0) return ZG_OK;
+    advance_rows_kernel<<<(M + 63) / 64, 64, 0, s>>>(tok, M, ids, pos, seen);
+    ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
