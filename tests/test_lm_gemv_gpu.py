@@ -47,3 +47,30 @@ def test_activations_on_load(ff, dtype):
     refs = [oracle.forward(t)[0] for t in toks]
     for n in (1, 2):
         check(cfg, w, refs, toks, n, dtype)
+
+
+@pytest.mark.parametrize("dim,vdim", [(1, 4), (16, 24), (100, 36), (128, 64), (129, 68), (160, 128), (256, 132), (24, 256), (40, 6), (40, 260)])
+def test_one_token_of_the_recurrence(dim, vdim):
+    """A token of every entry: states of fewer and more rows than the threads hold at a time, value widths around a row of lanes and beyond
+    the kernel's."""
+    cfg = tl.config([tl.hgrn2_layer(heads=3, dim=dim, vdim=vdim, mlp=tl.dense_mlp(ff=24))], vocab=97, width=48)
+    w = tl.weights(cfg, seed=dim + vdim)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(70 + b, 9, cfg["vocab"]) for b in range(2)]
+    refs = [oracle.forward(t)[0] for t in toks]
+    for n in (1, 2):
+        check(cfg, w, refs, toks, n, "float32")
+
+
+@pytest.mark.parametrize("width", [8, 136, 520, 1024, 1032, 44])
+@pytest.mark.parametrize("experts,top", [(3, 2), (8, 2), (21, 5)])
+def test_router_with_the_norms_in_front(width, experts, top):
+    """Steps of few rows: the sum and norms inside the router's launch; fewer experts than waves, more, widths it leaves to two launches."""
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=16, vdim=24, mlp=tl.moe_mlp(ff=24, experts=experts, top=top)),
+                     tl.hgrn2_layer(heads=2, dim=16, vdim=24, mlp=tl.moe_mlp(ff=24, experts=experts, top=top))], vocab=97, width=width)
+    w = tl.weights(cfg, seed=width + experts)
+    oracle = lm_oracle.Model(cfg, w)
+    toks = [tl.tokens(90 + b, 5, cfg["vocab"]) for b in range(2)]
+    refs = [oracle.forward(t)[0] for t in toks]
+    for n in (1, 2):
+        check(cfg, w, refs, toks, n, "float32")

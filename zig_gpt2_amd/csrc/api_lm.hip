@@ -1322,10 +1322,15 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             lin = Linear();
             lin.A = hin; lin.A16 = hin16; lin.lda = W; lin.B = L.qfv; lin.ldb = W; lin.C = g->proj; lin.ldc = NP; lin.M = M; lin.N = NP; lin.K = W;
             ZG_TRY(hidden_product(lin));
-            ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
-                                     L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
+            bool stepped = false;
             bf16_t* const o16 = r16 && whole(HV) ? g->o16 : nullptr;
-            ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s, o16));
+            if (single) ZG_TRY(launch_gated_step(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_eslot, n_ent, H, D, Vd, L.fb,
+                                                 L.lower, L.hnorm, eps, s, &stepped));
+            if (!stepped) {
+                ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
+                                         L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
+                ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s, o16));
+            }
             lin = Linear();
             lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             ZG_TRY(launch_linear(lin, f32, s));
@@ -1574,8 +1579,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         if (canon && single && d.ff != ZG_LM_FF_NONE && !mid_done)
             ZG_TRY(launch_norm_conv_single(x, nullptr, g->y, nullptr, nullptr, nullptr, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
                                            g->seq_state + ps.canon2_off, g->seq_floats, d_slot, g->hc, s, &mid_done));
+        RoutePre pre;
         if (mid_done) {
         } else if (defer && d.ff == ZG_LM_FF_DENSE) defer_norm(g->y, L.norm1b, L.norm2);
+        else if (few && !canon && d.ff == ZG_LM_FF_MOE && route_norm_fits(L.router, W)) {  // steps of few rows: the router's workgroups do it
+            pre.rms = true;
+            pre.x = x; pre.y.a = g->y; pre.nb = L.norm1b; pre.nn = L.norm2; pre.h = g->h; pre.eps = eps;
+        }
         else if (d.ff != ZG_LM_FF_NONE)  // (a router reads the fp32 rows)
             ZG_TRY(launch_norm_add_norm(x, g->y, L.norm1b, L.norm2, eps, h_r16 && d.ff == ZG_LM_FF_DENSE ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
         else {
@@ -1598,7 +1608,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             const bool glu = d.ff_act == ZG_LM_ACT_GLU_SILU;
             const int UF = glu ? 2 * F : F;
             ZG_TRY(launch_route(hin, M, W, L.router, L.correction, E, top, g->pick, g->wt, d.router, s, d.route_groups, d.route_keep,
-                                d.route_scale != 0.0f ? d.route_scale : 1.0f));
+                                d.route_scale != 0.0f ? d.route_scale : 1.0f, pre.x ? &pre : nullptr));
             Linear up, dn;
             up.A = hin; up.A16 = hin16; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
             up.N = UF; up.K = W;

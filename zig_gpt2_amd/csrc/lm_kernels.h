@@ -207,6 +207,11 @@ int launch_gated_chunks(const float* proj, int ld, float* out, int ldo, float* s
                         const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low, float* ws, size_t ws_floats,
                         const GlaGate* gla, hipStream_t s, bool* taken);
 
+// One token of every entry (HGRN2, decode steps) and the norm of each head's result, out = o / rms(o) * w, in one launch.  *taken = false:
+// heads wider than its tiles or values in no whole 16-byte pieces, nothing launched.
+int launch_gated_step(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start, const int* ent_slot,
+                      int n_entries, int H, int D, int V, const float* bias, const float* low, const float* w, float eps, hipStream_t s, bool* taken);
+
 // The carry of a chunked recurrence: wsB [chunk][H][D][V] holds every chunk's end state from zero and receives its true start state,
 // wsA [chunk][H][a_rows] the chunk's decay (a_rows D: per row of the state, 1: per head); the slot's state moves on.
 int launch_state_carry(float* state, size_t slot_stride, const int* ent_len, const int* ent_slot, int n_entries, int H, int D, int V, float* wsB,
@@ -449,7 +454,10 @@ struct RoutePre {
     float mult = 1.0f;
     const float* nn = nullptr;
     float* h = nullptr;
+    bool rms = false;  // norms by the root mean square (y.a alone): x += y.a / rms * (1 + nb), h = x / rms * (1 + nn)
+    float eps = 0.0f;
 };
+bool route_norm_fits(const bf16_t* router, int W);  // rows the norm by the root mean square can be done for
 constexpr int kRouteFuseWidth = 8192;
 int launch_route(const float* g, int M, int W, const bf16_t* router, const float* correction, int E, int top, int* pick, float* weight,
                  int rule, hipStream_t s, int groups = 1, int keep = 1, float out_scale = 1.0f, const RoutePre* pre = nullptr);

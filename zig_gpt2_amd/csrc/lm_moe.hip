@@ -36,7 +36,10 @@ __device__ __forceinline__ float block_allsum(float v, float* s_red) {
 // the sigmoid and a block ranked by its best r alone.
 // pre.x != null: the workgroup first finishes its own row — x += mult * nb(sum of the sublayer's parts), h = nn(x), both written
 // out, h also kept in the LDS — and routes on that (steps of few rows: the sum and norm in front of the router need no launch
-// of their own).
+// of their own).  PRE_RMS: the same for norms by the root mean square, rows of up to 1024 values; each wave's first router row is on its
+// way while the row is normed (8 rows of 768, 8 experts: 6.6 us; 5.4 and 3.9 for the norm's launch in front).
+enum { PRE_NONE, PRE_TANH, PRE_RMS };
+template <int PRE>
 __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int W, const bf16_t* router, const float* correction, int E, int top,
                                                     int* pick, float* weight, int rule, int groups, int keep, float out_scale, const RoutePre pre) {
     const bool top_logits = rule == 1 || rule == 2;  // rules that choose by the logits themselves
@@ -46,7 +49,55 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
     __shared__ float s_gs[kMaxExperts];
     const int m = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const float* row = g + (size_t)m * W;
-    if (pre.x) {
+    u32x4 w_first[2];  // (PRE_RMS) the wave's first router row
+    if constexpr (PRE == PRE_RMS) {
+        __shared__ float s_sum[2][16];
+        const int T = blockDim.x, waves = T >> 6;
+        float y[4], x[4], b[4], n[4], ss = 0.0f, s2 = 0.0f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {  // (at least 256 threads)
+            const int i = min((int)threadIdx.x + T * j, W - 1);
+            y[j] = pre.y.a[(size_t)m * W + i];
+            x[j] = pre.x[(size_t)m * W + i];
+            b[j] = pre.nb[i];
+            n[j] = pre.nn[i];
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) w_first[u] = *reinterpret_cast<const u32x4*>(router + (size_t)min(wave, E - 1) * W + min(lane * 8 + 512 * u, W - 8));
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if ((int)threadIdx.x + T * j < W) ss = fmaf(y[j], y[j], ss);
+        ss = wave_allsum(ss);
+        if (lane == 0) s_sum[0][wave] = ss;
+        __syncthreads();
+        ss = 0.0f;
+        for (int k = 0; k < waves; ++k) ss += s_sum[0][k];
+        const float r = 1.0f / sqrtf(ss / (float)W + pre.eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            x[j] += y[j] * r * (1.0f + b[j]);
+            if ((int)threadIdx.x + T * j < W) s2 = fmaf(x[j], x[j], s2);
+        }
+        s2 = wave_allsum(s2);
+        if (lane == 0) s_sum[1][wave] = s2;
+        __syncthreads();
+        s2 = 0.0f;
+        for (int k = 0; k < waves; ++k) s2 += s_sum[1][k];
+        const float r2 = 1.0f / sqrtf(s2 / (float)W + pre.eps);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int i = threadIdx.x + T * j;
+            if (i < W) {
+                const float hv = x[j] * r2 * (1.0f + n[j]);
+                pre.x[(size_t)m * W + i] = x[j];
+                pre.h[(size_t)m * W + i] = hv;
+                s_row[i] = hv;
+            }
+        }
+        __syncthreads();
+        row = s_row;
+    }
+    if constexpr (PRE == PRE_TANH) {
         const float ab = pre.nb[2 * W], an = pre.nn[2 * W];
         for (int i = threadIdx.x; i < W; i += blockDim.x) {
             const size_t idx = (size_t)m * W + i;
@@ -65,11 +116,22 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
         __syncthreads();
         row = s_row;
     }
-    const bool vec = (W % 8 == 0) && (pre.x || (reinterpret_cast<uintptr_t>(g) & 15) == 0) && ((reinterpret_cast<uintptr_t>(router) & 15) == 0);
+    const bool vec = (W % 8 == 0) && (PRE != PRE_NONE || (reinterpret_cast<uintptr_t>(g) & 15) == 0) && ((reinterpret_cast<uintptr_t>(router) & 15) == 0);
     for (int e = wave; e < E; e += (int)(blockDim.x >> 6)) {
         const bf16_t* wr = router + (size_t)e * W;
         float a = 0.0f;
-        if (vec) {
+        if constexpr (PRE == PRE_RMS) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const int k = lane * 8 + 512 * u, at = min(k, W - 8);
+                const u32x4 v = e == wave ? w_first[u] : *reinterpret_cast<const u32x4*>(wr + at);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    a = fmaf(k < W ? row[at + 2 * i] : 0.0f, bf16_lo(v[i]), a);
+                    a = fmaf(k < W ? row[at + 2 * i + 1] : 0.0f, bf16_hi(v[i]), a);
+                }
+            }
+        } else if (vec) {
             for (int k0 = lane * 8; k0 < W; k0 += 2048) {
                 f32x4 x0[4], x1[4];
                 u32x4 wv[4];
@@ -371,6 +433,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const float* x, float*
 
 }  // namespace
 
+bool route_norm_fits(const bf16_t* router, int W) { return W >= 8 && W <= 1024 && W % 8 == 0 && (reinterpret_cast<uintptr_t>(router) & 15) == 0; }
+
 int launch_route(const float* g, int M, int W, const bf16_t* router, const float* correction, int E, int top, int* pick, float* weight,
                  int rule, hipStream_t s, int groups, int keep, float out_scale, const RoutePre* pre) {
     if (M <= 0) return ZG_OK;
@@ -380,12 +444,17 @@ int launch_route(const float* g, int M, int W, const bf16_t* router, const float
     if (keep < 1) keep = groups;  // (a descriptor that names no groups)
     ZG_REQUIRE(E % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (E / groups), ZG_ERR_ARG,
                "router: %d experts in %d groups, %d groups kept, %d chosen", E, groups, keep, top);
-    ZG_REQUIRE(!pre || (pre->x && pre->nb && pre->nn && pre->h == g && W <= kRouteFuseWidth), ZG_ERR_ARG,
+    ZG_REQUIRE(!pre || (pre->x && pre->nb && pre->nn && pre->h == g && W <= kRouteFuseWidth && (!pre->rms || route_norm_fits(router, W))), ZG_ERR_ARG,
                "router: the sum in front of it needs x, both norms, its output as the router's input, and a width of at most %d", kRouteFuseWidth);
     // steps of few rows: a wave per expert where there are not too many, so that every router row is requested at once
     const int waves = M > kGemvMaxRows ? 4 : std::max(4, std::min(16, E));
-    route_kernel<<<M, 64 * waves, pre ? (size_t)W * sizeof(float) : 0, s>>>(g, M, W, router, correction, E, top, pick, weight, rule, groups, keep, out_scale,
-                                                                     pre ? *pre : RoutePre());
+    const size_t lds = pre ? (size_t)W * sizeof(float) : 0;
+    const RoutePre p = pre ? *pre : RoutePre();
+#define ZG_ROUTE(PRE) route_kernel<PRE><<<M, 64 * waves, lds, s>>>(g, M, W, router, correction, E, top, pick, weight, rule, groups, keep, out_scale, p)
+    if (!pre) ZG_ROUTE(PRE_NONE);
+    else if (pre->rms) ZG_ROUTE(PRE_RMS);
+    else ZG_ROUTE(PRE_TANH);
+#undef ZG_ROUTE
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

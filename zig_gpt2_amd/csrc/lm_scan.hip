@@ -342,7 +342,90 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
     }
 }
 
+// One token of every entry (decode steps), HGRN2, and the norm behind the head: a workgroup per (entry, head), four value channels a lane
+// (CW lanes a row of the state), the key channels dealt over the rest of the 512 threads.  A step reads and writes each state once, so
+// everything is requested at entry: the rows of the state before the gates that scale them.  8 entries, 6 heads of 128 x 128: 6.0 us,
+// 8.0 for the token-by-token scan's kernel and 4.0 for the norm's launch behind it.
+constexpr int kStepRows = 8;  // rows of the state in flight per thread
+template <int CW>
+__global__ __launch_bounds__(512) void gated_step_kernel(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride,
+                                                         const int* ent_start, const int* ent_slot, int H, int D, int V, const float* bias, const float* low,
+                                                         const float* w, float eps) {
+    constexpr int GROUPS = 512 / CW;
+    __shared__ float s_q[256], s_f[256], s_red[8];
+    __shared__ __attribute__((aligned(16))) float s_o[GROUPS][CW * 4 + 4];
+    const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, c = tid % CW, r = tid / CW;
+    const size_t m = ent_start[e];
+    float* S = state + (size_t)ent_slot[e] * slot_stride + (size_t)h * D * V;
+    const float* row = proj + m * ld;
+    const int HD = H * D, col = min(c * 4, V - 4);
+    const bool ok = c * 4 < V;
+    f32x4 s[kStepRows];
+#pragma unroll
+    for (int u = 0; u < kStepRows; ++u) s[u] = *reinterpret_cast<const f32x4*>(S + (size_t)min(r + GROUPS * u, D - 1) * V + col);
+    f32x4 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = row[2 * HD + h * V + col + i];
+    if (tid < D) {
+        const float z = row[h * D + tid], l = low[h * D + tid];
+        s_q[tid] = z / (1.0f + expf(-z));
+        s_f[tid] = l + (1.0f - l) / (1.0f + expf(-(row[HD + h * D + tid] + bias[h * D + tid])));
+    }
+    __syncthreads();
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (int i0 = 0; i0 < D; i0 += GROUPS * kStepRows) {
+        if (i0 > 0) {
+#pragma unroll
+            for (int u = 0; u < kStepRows; ++u) s[u] = *reinterpret_cast<const f32x4*>(S + (size_t)min(i0 + r + GROUPS * u, D - 1) * V + col);
+        }
+#pragma unroll
+        for (int u = 0; u < kStepRows; ++u) {
+            const int i = i0 + r + GROUPS * u;
+            if (i < D && ok) {
+                const float f = s_f[i], q = s_q[i];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    s[u][k] = fmaf(f, s[u][k], (1.0f - f) * v[k]);
+                    o[k] = fmaf(s[u][k], q, o[k]);
+                }
+                *reinterpret_cast<f32x4*>(S + (size_t)i * V + col) = s[u];
+            }
+        }
+    }
+    *reinterpret_cast<f32x4*>(&s_o[r][c * 4]) = o;
+    __syncthreads();
+    float a = 0.0f;
+    if (tid < V) {
+#pragma unroll
+        for (int k = 0; k < GROUPS; ++k) a += s_o[k][tid];
+    }
+    const float ss = wave_allsum(a * a);
+    if ((tid & 63) == 0) s_red[tid >> 6] = ss;
+    __syncthreads();
+    if (tid < V) {
+        const float rms = ((s_red[0] + s_red[1]) + (s_red[2] + s_red[3])) + ((s_red[4] + s_red[5]) + (s_red[6] + s_red[7]));
+        out[m * ldo + h * V + tid] = a * (1.0f / sqrtf(rms / (float)V + eps)) * w[tid];
+    }
+}
+
 }  // namespace
+
+int launch_gated_step(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start, const int* ent_slot,
+                      int n_entries, int H, int D, int V, const float* bias, const float* low, const float* w, float eps, hipStream_t s, bool* taken) {
+    *taken = false;
+    if (n_entries <= 0 || D > 256 || V < 4 || V > 256 || V % 4 != 0 || slot_stride % 4 != 0 || (reinterpret_cast<uintptr_t>(state) & 15) != 0 || H > 65535)
+        return ZG_OK;
+    const dim3 grid(n_entries, H);
+#define ZG_GSTEP(CW) gated_step_kernel<CW><<<grid, 512, 0, s>>>(proj, ld, out, ldo, state, slot_stride, ent_start, ent_slot, H, D, V, bias, low, w, eps)
+    if (V <= 32) ZG_GSTEP(8);
+    else if (V <= 64) ZG_GSTEP(16);
+    else if (V <= 128) ZG_GSTEP(32);
+    else ZG_GSTEP(64);
+#undef ZG_GSTEP
+    ZG_HIP(hipGetLastError());
+    *taken = true;
+    return ZG_OK;
+}
 
 int launch_gated_chunks(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start, const int* ent_len,
                         const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low, float* ws, size_t ws_floats,
