@@ -267,12 +267,35 @@ static int linear_mfma(Call& call, size_t in_f, size_t out_f, const float* w, co
     return launch_gemm_planes(xp, wp, bias, y, (int)m, (int)out_f, pl, (int)out_f, false, false, call.stream());
 }
 
+// rows one launch of the GEMV kernels takes (they hold them in the LDS)
+static size_t gemv_rows(size_t in_f) {
+    size_t mb = 8;
+    while (mb > 1 && (mb * in_f + 8 * mb + 64) * sizeof(float) > 160 * 1024) mb >>= 1;
+    return mb;
+}
+
+// Linears of more rows than one launch of the GEMV kernels takes, up to where the large tiles fill the chip: both operands split in the
+// kernel's own staging (linear_tiles.hip).
+static bool linear_tiles_ok(size_t in_f, size_t out_f, size_t m, size_t arena_left) {
+    if (in_f > 8192 ? !linear_mfma_ok(in_f, out_f, m, arena_left) : m <= gemv_rows(in_f)) return false;
+    if (in_f < 128 || in_f % 64 != 0 || m >= (1u << 30) / in_f || out_f >= (1u << 30) / in_f) return false;
+    if (!linear_tiles_pay(m, out_f)) return false;
+    const int slices = linear_tiles_slices(m, out_f, in_f);
+    return slices == 1 || (size_t)slices * m * out_f * sizeof(float) + 1024 <= arena_left;
+}
+
+static int linear_tiles(Call& call, size_t in_f, size_t out_f, const float* w, const float* bias, const float* x, size_t m, float* y) {
+    const int slices = linear_tiles_slices(m, out_f, in_f);
+    float* slabs = nullptr;
+    if (slices > 1) ZG_TRY(call.scratch((size_t)slices * m * out_f, &slabs));
+    return launch_linear_tiles(x, w, bias, y, (int)m, (int)out_f, (int)in_f, slabs, call.stream());
+}
+
 static int linear_device(size_t in_f, size_t out_f, const float* w, const float* bias, const float* x,
                          size_t m, float* y, hipStream_t s) {
     if (m == 0 || out_f == 0) return ZG_OK;
     ZG_REQUIRE(in_f > 0 && in_f <= 8192, ZG_ERR_UNSUPPORTED, "Linear: in_features %zu outside 1..8192", in_f);
-    size_t mb = 8;
-    while (mb > 1 && (mb * in_f + 8 * mb + 64) * sizeof(float) > 160 * 1024) mb >>= 1;
+    const size_t mb = gemv_rows(in_f);
     for (size_t m0 = 0; m0 < m; m0 += mb) {
         GemvArgs a{};
         a.W = w;
@@ -536,7 +559,9 @@ int zg_linear_forward(size_t in_features, size_t out_features, const float* weig
     ZG_TRY(call.in(inputs, inputs_len, &x));  // (read by every workgroup: device memory)
     if (in_features <= 8192) ZG_TRY(call.out_once(outputs, batch * out_features, &y));  // every element stored once
     else ZG_TRY(call.out(outputs, batch * out_features, &y));                          // K chunks accumulate into y
-    if (linear_mfma_ok(in_features, out_features, batch, call.arena_left()))
+    if (linear_tiles_ok(in_features, out_features, batch, call.arena_left()))
+        ZG_TRY(linear_tiles(call, in_features, out_features, w, b, x, batch, y));
+    else if (linear_mfma_ok(in_features, out_features, batch, call.arena_left()))
         ZG_TRY(linear_mfma(call, in_features, out_features, w, b, x, batch, y));
     else
         ZG_TRY(linear_device_wide(call, in_features, out_features, w, b, x, batch, y));

@@ -1,0 +1,189 @@
+// linear_tiles.hip — fp32 Linears of 16 rows to some thousand (y = x W^T + bias, src/ops.zig:21-46) in one pass over both operands.
+//
+// Both operands are split exactly into three bf16 terms on their way into the LDS (x = hi + mid + lo) and the six products above 2^-24 of
+// the leading one are summed, as the persistent kernel for many rows does (gemm_s4.hip); here no planes are written to memory first, and
+// the tiles are small enough to use the whole chip: 64 x 64, and K in slices over grid.z while there are too few of them (each slice leaves
+// a slab, linear_slabs_kernel adds them).  The leading products have sums of their own, so that the small ones are not rounded at their size.
+#include "zg_kernels.h"
+
+#include <algorithm>
+
+namespace zg {
+
+namespace {
+
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+constexpr int kBk = 32, kChunks = kBk / 8;  // columns of K a step stages, 16-byte pieces of a row of them
+constexpr int kAheadSteps = 3;
+
+// rows of 32 bf16 (64 bytes): pieces swizzled by the row, so that a fragment read of eight rows touches every bank once
+__device__ __forceinline__ int lds_at(int row, int piece) { return row * kBk + ((piece ^ ((row >> 1) & 3)) * 8); }
+
+struct Terms {
+    u32x4 v[3];  // hi, mid, lo of eight values
+};
+__device__ __forceinline__ Terms split8(const f32x4& a, const f32x4& b) {
+    Terms t;
+    const float x[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t h, m, l;
+        split3_pk(x[2 * i], x[2 * i + 1], h, m, l);
+        t.v[0][i] = h;
+        t.v[1][i] = m;
+        t.v[2][i] = l;
+    }
+    return t;
+}
+
+// What bounds it: the LDS, which takes 24 KB of terms and gives 48 KB of fragments a step, beside 384 cycles of products.
+__global__ __launch_bounds__(256, 2) void linear_tiles_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
+                                                              float* __restrict__ Y, int M, int N, int K, int steps) {
+    __shared__ __attribute__((aligned(16))) bf16_t As[2][3][64 * kBk];
+    __shared__ __attribute__((aligned(16))) bf16_t Bs[2][3][64 * kBk];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wy = wave >> 1, wx = wave & 1;
+    // consecutive workgroups go to the eight XCDs in turn: each gets a contiguous run of the tiles, row tiles of one column tile together
+    const int tiles_m = (M + 63) / 64, total = gridDim.x, q = total >> 3, r8 = total & 7, xcd = blockIdx.x & 7;
+    const int at = xcd * q + min(xcd, r8) + (int)(blockIdx.x >> 3);
+    const int m0 = (at % tiles_m) * 64, n0 = (at / tiles_m) * 64;
+    const int k_first = blockIdx.z * steps * kBk;
+    steps = min(steps, (K - k_first) / kBk);
+
+    const int row = tid / kChunks, piece = tid % kChunks, to = lds_at(row, piece);
+    const float* x = X + (size_t)min(m0 + row, M - 1) * K + k_first + piece * 8;  // (rows beyond the edge: some valid row, never stored)
+    const float* w = W + (size_t)min(n0 + row, N - 1) * K + k_first + piece * 8;
+    f32x4 xr[kAheadSteps][2], wr[kAheadSteps][2];
+    auto fetch = [&](int slot, int s) {
+        const int k = min(s, steps - 1) * kBk;  // (beyond the last step: fetched again, not used)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            xr[slot][i] = *reinterpret_cast<const f32x4*>(x + k + 4 * i);
+            wr[slot][i] = *reinterpret_cast<const f32x4*>(w + k + 4 * i);
+        }
+    };
+    auto stash = [&](int slot, int buf) {
+        const Terms a = split8(xr[slot][0], xr[slot][1]), b = split8(wr[slot][0], wr[slot][1]);
+#pragma unroll
+        for (int t = 0; t < 3; ++t) {
+            *reinterpret_cast<u32x4*>(&As[buf][t][to]) = a.v[t];
+            *reinterpret_cast<u32x4*>(&Bs[buf][t][to]) = b.v[t];
+        }
+    };
+    f32x16 lead, small;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) lead[e] = small[e] = 0.0f;
+    const int fr = lane & 31, kh = lane >> 5;
+    bf16x8 af[2][3], bf[2][3];
+    auto read = [&](int buf) {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                af[kk][t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&As[buf][t][lds_at(wy * 32 + fr, 2 * kk + kh)]));
+                bf[kk][t] = __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(&Bs[buf][t][lds_at(wx * 32 + fr, 2 * kk + kh)]));
+            }
+    };
+    auto multiply = [&]() {
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][2], bf[kk][0], small, 0, 0, 0);
+            lead = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][0], bf[kk][0], lead, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][1], bf[kk][1], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][0], bf[kk][2], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][1], bf[kk][0], small, 0, 0, 0);
+            small = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[kk][0], bf[kk][1], small, 0, 0, 0);
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < kAheadSteps; ++i) fetch(i, i);
+    stash(0, 0);
+    fetch(0, kAheadSteps);
+    __syncthreads();
+    int buf = 0;
+    for (int s0 = 0; s0 < steps; s0 += kAheadSteps) {
+#pragma unroll
+        for (int i = 0; i < kAheadSteps; ++i) {
+            if (s0 + i < steps) {  // (uniform)
+                const int nx = (i + 1) % kAheadSteps;
+                read(buf);
+                stash(nx, buf ^ 1);
+                fetch(nx, s0 + i + 1 + kAheadSteps);
+                multiply();
+                buf ^= 1;
+                __syncthreads();
+            }
+        }
+    }
+    // element e of the wave's 32 x 32: row 8 (e / 4) + 4 (lane / 32) + e % 4, column lane % 32
+    float* y = Y + (gridDim.z > 1 ? (size_t)blockIdx.z * M * N : 0);
+    const int n = n0 + wx * 32 + fr;
+    if (n >= N) return;
+    const float b = bias != nullptr && gridDim.z == 1 ? bias[n] : 0.0f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        const int m = m0 + wy * 32 + 8 * (e >> 2) + 4 * kh + (e & 3);
+        if (m < M) y[(size_t)m * N + n] = lead[e] + (small[e] + b);
+    }
+}
+
+__global__ __launch_bounds__(256) void linear_slabs_kernel(const float* __restrict__ slabs, int n_slabs, const float* __restrict__ bias, float* __restrict__ Y,
+                                                           size_t n, int N) {
+    const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
+    if (i >= n) return;
+    float v[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int here = (int)min((size_t)4, n - i);
+    if (here == 4 && n % 4 == 0) {
+        for (int s = 0; s < n_slabs; ++s) {
+            const f32x4 t = *reinterpret_cast<const f32x4*>(slabs + s * n + i);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] += t[e];
+        }
+    } else {
+        for (int s = 0; s < n_slabs; ++s)
+            for (int e = 0; e < here; ++e) v[e] += slabs[s * n + i + e];
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (e < here) Y[i + e] = v[e] + (bias ? bias[(i + e) % N] : 0.0f);
+}
+
+}  // namespace
+
+bool linear_tiles_pay(size_t M, size_t N) {
+    // Against the persistent kernel behind two splitting passes, whose time goes by rounds of 256 tiles of 256 x 192 whether they are full or
+    // not (us of a call, this : that): 768 -> 3072 16 rows 21 : 83, 512 rows 42 : 90, 1500 rows (1152 tiles) 76 : 91, 2048 (1536) 90 : 95, 4096
+    // (3072) 165 : 122; 3072 -> 768 16 rows 24 : 255, 4096 (768) 161 : 271; 1600 -> 1600 2048 (800) 112 : 151, 4096 (1600) 184 : 168;
+    // 1600 -> 4800 1023 (1200) 135 : 159, 1500 (1800) 203 : 170; 6400 -> 1600 16 rows 33 : 504, 4096 (1600) 675 : 593.
+    const size_t tiles = ((M + 63) / 64) * ((N + 63) / 64), rounds = (((M + 255) / 256) * ((N + 191) / 192) + 255) / 256;
+    return tiles <= 1400 * rounds;
+}
+
+int linear_tiles_slices(size_t M, size_t N, size_t K) {
+    // two workgroups a compute unit, slices of at least four steps
+    const size_t tiles = ((M + 63) / 64) * ((N + 63) / 64), steps = K / kBk;
+    size_t s = std::min<size_t>({(512 + tiles - 1) / tiles, steps / 4, 16});
+    s = std::max<size_t>(1, s);
+    const size_t per = (steps + s - 1) / s;
+    return (int)((steps + per - 1) / per);  // (none is empty)
+}
+
+int launch_linear_tiles(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, float* slabs, hipStream_t s) {
+    ZG_REQUIRE(M > 0 && N > 0 && K > 0 && K % kBk == 0, ZG_ERR_UNSUPPORTED, "linear tiles: M=%d N=%d K=%d", M, N, K);
+    const long long tiles = (long long)((M + 63) / 64) * ((N + 63) / 64);
+    ZG_REQUIRE(tiles < (1LL << 31) - 8, ZG_ERR_UNSUPPORTED, "linear tiles: %d x %d outputs exceed the grid", M, N);
+    const int slices = linear_tiles_slices(M, N, K), steps = (K / kBk + slices - 1) / slices;
+    ZG_REQUIRE(slices == 1 || slabs != nullptr, ZG_ERR_ARG, "linear tiles: %d slices and no room for their slabs", slices);
+    linear_tiles_kernel<<<dim3((unsigned)tiles, 1, slices), 256, 0, s>>>(X, W, bias, slices > 1 ? slabs : Y, M, N, K, steps);
+    ZG_HIP(hipGetLastError());
+    if (slices > 1) {
+        const size_t n = (size_t)M * N;
+        linear_slabs_kernel<<<(unsigned)((n + 1023) / 1024), 256, 0, s>>>(slabs, slices, bias, Y, n, N);
+        ZG_HIP(hipGetLastError());
+    }
+    gemm_note_launch();
+    return ZG_OK;
+}
+
+}  // namespace zg
