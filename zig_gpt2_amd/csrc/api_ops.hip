@@ -559,7 +559,9 @@ int zg_linear_forward(size_t in_features, size_t out_features, const float* weig
     ZG_TRY(call.in(inputs, inputs_len, &x));  // (read by every workgroup: device memory)
     if (in_features <= 8192) ZG_TRY(call.out_once(outputs, batch * out_features, &y));  // every element stored once
     else ZG_TRY(call.out(outputs, batch * out_features, &y));                          // K chunks accumulate into y
-    if (linear_tiles_ok(in_features, out_features, batch, call.arena_left()))
+    if (linear_few_ok(batch, out_features, in_features) && out_features < (1u << 30))
+        ZG_TRY(launch_linear_few(x, w, b, y, (int)batch, (int)out_features, (int)in_features, call.stream()));
+    else if (linear_tiles_ok(in_features, out_features, batch, call.arena_left()))
         ZG_TRY(linear_tiles(call, in_features, out_features, w, b, x, batch, y));
     else if (linear_mfma_ok(in_features, out_features, batch, call.arena_left()))
         ZG_TRY(linear_mfma(call, in_features, out_features, w, b, x, batch, y));

@@ -149,6 +149,73 @@ __global__ __launch_bounds__(256) void linear_slabs_kernel(const float* __restri
         if (e < here) Y[i + e] = v[e] + (bias ? bias[(i + e) % N] : 0.0f);
 }
 
+constexpr int kLongRow = 1536;
+
+// Up to eight rows: a wave multiplies R weight rows with all of them, two pieces of 512 columns in flight; long rows (SPLIT) are cut over the
+// four waves of a workgroup.  Everything is loaded at clamped addresses without a condition, and the workgroups are small enough for
+// every compute unit to have one.  A call, us, this against the general kernel: 8 rows 768 -> 3072 15.4 : 20.0, 6400 -> 1600 26 : 32, 1 row
+// 768 -> 50257 32 : 39, 1600 -> 4800 16.8 : 18.2.
+template <int MR, int R, bool SPLIT>
+__global__ __launch_bounds__(256) void linear_few_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
+                                                         float* __restrict__ Y, int M, int N, int K) {
+    __shared__ float s_part[SPLIT ? 4 : 1][MR * R];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n0 = SPLIT ? blockIdx.x * R : (blockIdx.x * 4 + wave) * R;
+    if (n0 >= N) return;
+    const int kq = SPLIT ? (((K + 3) / 4) + 7) & ~7 : K, k_lo = SPLIT ? wave * kq : 0, k_hi = SPLIT ? min(K, k_lo + kq) : K;
+    f32x4 xr[2][MR][2], wr[2][R][2];
+    auto fetch = [&](int slot, int k0) {
+        const int k = min(k0 + lane * 8, K - 8);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) wr[slot][r][i] = *reinterpret_cast<const f32x4*>(W + (size_t)min(n0 + r, N - 1) * K + k + 4 * i);
+#pragma unroll
+            for (int m = 0; m < MR; ++m) xr[slot][m][i] = *reinterpret_cast<const f32x4*>(X + (size_t)min(m, M - 1) * K + k + 4 * i);
+        }
+    };
+    float sum[MR][R];
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int r = 0; r < R; ++r) sum[m][r] = 0.0f;
+    auto add = [&](int slot, int k0) {
+        if (k0 + lane * 8 >= k_hi) return;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int m = 0; m < MR; ++m)
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) sum[m][r] = fmaf(xr[slot][m][i][e], wr[slot][r][i][e], sum[m][r]);
+    };
+    fetch(0, k_lo);
+    fetch(1, k_lo + 512);
+    for (int k0 = k_lo; k0 < k_hi; k0 += 1024) {
+        add(0, k0);
+        fetch(0, k0 + 1024);
+        add(1, k0 + 512);
+        fetch(1, k0 + 1536);
+    }
+    float mine = 0.0f;  // lane m R + r: the sum of row m, weight row n0 + r
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float v = wave_allsum(sum[m][r]);
+            mine = lane == m * R + r ? v : mine;
+        }
+    if constexpr (SPLIT) {
+        if (lane < MR * R) s_part[wave][lane] = mine;
+        __syncthreads();
+        if (wave != 0 || lane >= MR * R) return;
+        mine = (s_part[0][lane] + s_part[1][lane]) + (s_part[2][lane] + s_part[3][lane]);
+    }
+    const int m = lane / R, n = n0 + lane % R;
+    if (lane < MR * R && m < M && n < N) Y[(size_t)m * N + n] = mine + (bias ? bias[n] : 0.0f);
+}
+
 }  // namespace
 
 bool linear_tiles_pay(size_t M, size_t N) {
@@ -183,6 +250,30 @@ int launch_linear_tiles(const float* X, const float* W, const float* bias, float
         ZG_HIP(hipGetLastError());
     }
     gemm_note_launch();
+    return ZG_OK;
+}
+
+bool linear_few_ok(size_t M, size_t N, size_t K) {
+    // Beyond four rows every workgroup's share of the activations outweighs its weights: with more than some three workgroups a compute unit
+    // the general kernel, which reads them less often, is faster (8 rows 1600 -> 4800, 1200 of them, 32.9 : 27.9; 6400 -> 1600, 400, 26 : 32).
+    const size_t groups = K >= kLongRow ? (N + 3) / 4 : (N + 7) / 8;
+    return M >= 1 && M <= 8 && K >= 64 && K <= 8192 && K % 8 == 0 && groups < (1u << 30) && (M <= 4 || groups <= 768);
+}
+
+int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s) {
+    ZG_REQUIRE(M >= 1 && M <= 8 && N > 0 && K >= 8 && K % 8 == 0, ZG_ERR_UNSUPPORTED, "linear: M=%d N=%d K=%d", M, N, K);
+    const bool split = K >= kLongRow;
+#define ZG_FEW(MR)                                                                                             \
+    do {                                                                                                       \
+        if (split) linear_few_kernel<MR, 4, true><<<(N + 3) / 4, 256, 0, s>>>(X, W, bias, Y, M, N, K);         \
+        else linear_few_kernel<MR, 2, false><<<(N + 7) / 8, 256, 0, s>>>(X, W, bias, Y, M, N, K);              \
+    } while (0)
+    if (M == 1) ZG_FEW(1);
+    else if (M == 2) ZG_FEW(2);
+    else if (M <= 4) ZG_FEW(4);
+    else ZG_FEW(8);
+#undef ZG_FEW
+    ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
