@@ -202,6 +202,7 @@ __device__ __forceinline__ void read_b_all(bf16x8 (&fb)[4][NT], const unsigned (
 //               too few tiles (N = n_embed) slice K over the tile list; prefill.hip's reduce kernels sum the slabs in fixed
 //               order and finish (bias, residual, LayerNorm + plane split)
 //   S4_QKV      bias, fp32 rows of qkv[M][3E] AND the cache append of src/ops.zig:152-157 for the K / V columns
+//   S4_RELU2    bias, then max(., 0)^2, rows as S4_PLAIN            (the layered tier's dense feed-forward)
 //   S4_SPLIT3   bias + GELU, then the exact three-term bf16 split as planes C[M][3N] = [hi | mid | lo]  (src/main.zig:79-80 feeding
 //               the next Linear's A operand)
 
@@ -793,6 +794,13 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 f32x2v x[8];
 #pragma unroll
                 for (int k = 0; k < 8; ++k) x[k] = f32x2v{av[2 * k], av[2 * k + 1]};  // (the bias is in: the tile started there)
+                if constexpr (KIND == S4_RELU2) {
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) {
+                        const f32x2v p = {fmaxf(x[k].x, 0.0f), fmaxf(x[k].y, 0.0f)};
+                        x[k] = p * p;
+                    }
+                }
                 if constexpr (GELU) {
                     const float k1 = -2.0f * 1.4426950408889634f * 0.7978845608f, k2 = k1 * 0.044715f;
                     f32x2v t[8];
@@ -1044,6 +1052,12 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
                    bool gelu, bool out_bf16, int bn, hipStream_t s) {
     (void)bn;  // 192-wide tiles only: 256 x 256 needs all 256 accumulator registers plus 128 of B fragments
     return launch_s4_nt<3>(A, B, bias, C, M, N, pl, ldc, gelu, out_bf16, s);
+}
+
+int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s) {
+    const PrefillQkv none{};
+    return out_bf16 ? launch_s4_kind<3, S4_RELU2, false, true>(A, B, bias, C, M, N, pl, ldc, 1, none, s)
+                    : launch_s4_kind<3, S4_RELU2, false, false>(A, B, bias, C, M, N, pl, ldc, 1, none, s);
 }
 
 // The whole-prompt Linears on the same kernel (prefill.hip decides when): A = the activation planes [M][nplanes K] (hi | mid | lo),

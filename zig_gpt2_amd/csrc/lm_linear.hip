@@ -834,8 +834,9 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LinArgs p) {
 
 namespace {
 // Plain products of rounded rows with enough tiles of 256 x 192 go to the persistent kernel of the large-batch Linears (gemm_s4.hip), whose
-// hand-scheduled four waves keep the matrix cores twice as busy: 8184 x 3072 x 1024 59 against 89 us, 47 with a rounded result; 8184 x 672 x
-// 1024 (128 tiles) 26.6 against 29; 1791 x 3072 x 768 (112) 23.2 against 24.5; 1023 x 3072 x 768 (64 tiles) 21.7 against 15.4.
+// hand-scheduled four waves keep the matrix cores twice as busy: 8184 x 3072 x 1024 59 against 89 us, 47 with a rounded result; 8184 x
+// 4096 x 1024 with max(., 0)^2 and a rounded result 71 against 117; 8184 x 672 x 1024 (128 tiles) 26.6 against 29; 1791 x 3072 x 768 (112)
+// 23.2 against 24.5; 1023 x 3072 x 768 (64 tiles) 21.7 against 15.4.
 bool takes_persistent(const Linear& L) {
     const char* form = getenv("ZGPT2_LM_GEMM_TILE");  // test hook: 256 = here at any number of tiles, another = never
     const int least = form ? (atoi(form) == 256 ? 1 : 0x7fffffff) : 112;
@@ -845,7 +846,7 @@ bool takes_persistent(const Linear& L) {
     pl.kpp = L.K / 64;
     pl.npairs = 1;
     const bool one_result = (L.C != nullptr) != (L.C16 != nullptr);
-    return !L.grp_off && !L.z_group && L.nz == 1 && !L.a_rows && L.a_div == 1 && L.act == ACT_NONE && one_result && L.K >= 128 && L.K % 64 == 0 && L.lda % 8 == 0 &&
+    return !L.grp_off && !L.z_group && L.nz == 1 && !L.a_rows && L.a_div == 1 && (L.act == ACT_NONE || L.act == ACT_RELU2) && one_result && L.K >= 128 && L.K % 64 == 0 && L.lda % 8 == 0 &&
            L.ldb % 8 == 0 && L.lda >= L.K && L.ldc >= L.N && (L.C || (L.N % 8 == 0 && L.ldc % 8 == 0)) && gemm_s4_args_ok(pl, L.ldc) &&
            ((reinterpret_cast<uintptr_t>(L.A16) | reinterpret_cast<uintptr_t>(L.B) | reinterpret_cast<uintptr_t>(L.C) | reinterpret_cast<uintptr_t>(L.C16)) & 15) == 0 &&
            (size_t)L.M * L.ldc * 4 < ((size_t)1 << 32) && (size_t)L.N * L.ldb < (1u << 30) && (size_t)L.M * L.lda < (1u << 30) &&
@@ -975,6 +976,7 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
         pl.kpp = L.K / 64;
         pl.npairs = 1;
         note_kernel("gemm_s4_kernel");
+        if (L.act == ACT_RELU2) return launch_gemm_s4_relu2(L.A16, L.B, L.bias, L.C ? static_cast<void*>(L.C) : L.C16, L.M, L.N, pl, L.ldc, L.C == nullptr, s);
         return launch_gemm_s4(L.A16, L.B, L.bias, L.C ? static_cast<void*>(L.C) : L.C16, L.M, L.N, pl, L.ldc, false, L.C == nullptr, 192, s);
     }
     const bool a_vec = rounded ? (reinterpret_cast<uintptr_t>(L.A16) & 15) == 0 && L.lda % 8 == 0 && L.a_zoff % 8 == 0 : p.a_vec != 0;

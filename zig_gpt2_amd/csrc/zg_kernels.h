@@ -197,7 +197,8 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
                    bool gelu, bool out_bf16, int bn, hipStream_t s);  // gemm_s4.hip
 bool gemm_s4_args_ok(const GemmPlanes& pl, int ldc);            // the bounds of gemm_s4_kernel's packed arguments
 // ... and its epilogue kinds for the whole-prompt Linears (gemm_s4.hip; PrefillQkv below)
-enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT3 = 3 };
+enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT3 = 3, S4_RELU2 = 4 };
+int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s);
 struct PrefillQkv;
 int launch_gemm_s4_prefill(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int nplanes, int kind, int n_slices,
                            const PrefillQkv* qkv, hipStream_t s);
