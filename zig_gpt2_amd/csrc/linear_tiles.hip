@@ -151,10 +151,10 @@ __global__ __launch_bounds__(256) void linear_slabs_kernel(const float* __restri
 
 constexpr int kLongRow = 1536;
 
-// Up to eight rows: a wave multiplies R weight rows with all of them, two pieces of 512 columns in flight; long rows (SPLIT) are cut over the
+// Two to eight rows: a wave multiplies R weight rows with all of them, two pieces of 512 columns in flight; long rows (SPLIT) are cut over the
 // four waves of a workgroup.  Everything is loaded at clamped addresses without a condition, and the workgroups are small enough for
-// every compute unit to have one.  A call, us, this against the general kernel: 8 rows 768 -> 3072 15.4 : 20.0, 6400 -> 1600 26 : 32, 1 row
-// 768 -> 50257 32 : 39, 1600 -> 4800 16.8 : 18.2.
+// every compute unit to have one.  A call, us, this against the general kernel: 8 rows 768 -> 3072 15.4 : 20.0, 6400 -> 1600 26 : 32, 2 rows
+// 768 -> 50257 32 : 47, 1600 -> 4800 17.0 : 22.8.
 template <int MR, int R, bool SPLIT>
 __global__ __launch_bounds__(256) void linear_few_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
                                                          float* __restrict__ Y, int M, int N, int K) {
@@ -257,7 +257,8 @@ bool linear_few_ok(size_t M, size_t N, size_t K) {
     // Beyond four rows every workgroup's share of the activations outweighs its weights: with more than some three workgroups a compute unit
     // the general kernel, which reads them less often, is faster (8 rows 1600 -> 4800, 1200 of them, 32.9 : 27.9; 6400 -> 1600, 400, 26 : 32).
     const size_t groups = K >= kLongRow ? (N + 3) / 4 : (N + 7) / 8;
-    return M >= 1 && M <= 8 && K >= 64 && K <= 8192 && K % 8 == 0 && groups < (1u << 30) && (M <= 4 || groups <= 768);
+    // One row stays on the general kernels: a generation through op-tier calls with host buffers measured 782 tokens/s with it here, 819 there.
+    return M >= 2 && M <= 8 && K >= 64 && K <= 8192 && K % 8 == 0 && groups < (1u << 30) && (M <= 4 || groups <= 768);
 }
 
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s) {
@@ -268,8 +269,7 @@ int launch_linear_few(const float* X, const float* W, const float* bias, float* 
         if (split) linear_few_kernel<MR, 4, true><<<(N + 3) / 4, 256, 0, s>>>(X, W, bias, Y, M, N, K);         \
         else linear_few_kernel<MR, 2, false><<<(N + 7) / 8, 256, 0, s>>>(X, W, bias, Y, M, N, K);              \
     } while (0)
-    if (M == 1) ZG_FEW(1);
-    else if (M == 2) ZG_FEW(2);
+    if (M <= 2) ZG_FEW(2);
     else if (M <= 4) ZG_FEW(4);
     else ZG_FEW(8);
 #undef ZG_FEW

@@ -209,7 +209,7 @@ unsigned long long gemm_mfma_launch_count();  // launches of the persistent MFMA
 void gemm_note_launch();
 // fp32 Linears of few rows and of a medium number of rows (linear_tiles.hip): X [M][K], W [N][K], K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N
 // floats where that is more than one.
-bool linear_few_ok(size_t M, size_t N, size_t K);  // up to eight rows
+bool linear_few_ok(size_t M, size_t N, size_t K);  // two to eight rows
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 bool linear_tiles_pay(size_t M, size_t N);
 int linear_tiles_slices(size_t M, size_t N, size_t K);
