@@ -40,6 +40,18 @@ def test_both_sides_of_the_rule(zg, m, k, n):
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 
+@pytest.mark.parametrize("m", [0, 1, 2, 8, 9, 16, 70])
+@pytest.mark.parametrize("k", [100, 128, 768, 8200, 16384])
+def test_no_outputs(zg, m, k):
+    """No output columns, or no rows: nothing to do, whichever kernel's rule would have been asked."""
+    x = synth.fill_normal(1, m * k, 0, 1.0).reshape(m, k)
+    ops.Linear(k, 0, np.zeros((1, k), np.float32), None).forward(x, np.zeros((m, 0), np.float32))
+    ops.Linear(k, 0, np.zeros((1, k), np.float32), np.zeros(1, np.float32)).forward(x, np.zeros(0, np.float32))
+    y = np.full((1, 3), 7.0, np.float32)
+    ops.Linear(k, 3, synth.fill_normal(2, 3 * k, 0, 1.0).reshape(3, k), None).forward(x[:0], y)
+    assert (y == 7.0).all()
+
+
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 @pytest.mark.parametrize("m,k", [(70, 768), (8, 520), (3, 2056)])
 def test_values_that_are_not_finite(zg, bad, m, k):

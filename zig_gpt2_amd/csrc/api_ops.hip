@@ -550,6 +550,7 @@ int zg_linear_forward(size_t in_features, size_t out_features, const float* weig
                "Linear: inputs.len %zu is not a multiple of in_features %zu", inputs_len, in_features);
     ZG_REQUIRE(outputs_len >= batch * out_features, ZG_ERR_SHAPE,
                "Linear: outputs.len %zu < batch %zu * out_features %zu", outputs_len, batch, out_features);
+    if (batch * out_features == 0) return ZG_OK;  // nothing to store (the rules below divide by what there is)
     Call call;
     CallGuard guard(call);
     const float *w, *b, *x;
