@@ -52,6 +52,16 @@ def test_no_outputs(zg, m, k):
     assert (y == 7.0).all()
 
 
+def assert_same_class(want, y, what):
+    """Infinities and NaN where the oracle has them, of its sign; the rest close to it (row by row: their sizes differ)."""
+    assert np.array_equal(np.isnan(y), np.isnan(want)), what
+    inf = np.isinf(want)
+    assert np.array_equal(np.isinf(y), inf) and np.array_equal(y[inf], want[inf]), what
+    for w, v in zip(want, y):
+        ok = np.isfinite(w)
+        assert_ref_close(w[ok], v[ok], what, scale_floor=2e-6)
+
+
 @pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
 @pytest.mark.parametrize("m,k", [(70, 768), (8, 520), (3, 2056)])
 def test_values_that_are_not_finite(zg, bad, m, k):
@@ -59,7 +69,45 @@ def test_values_that_are_not_finite(zg, bad, m, k):
     x = synth.fill_normal(1, m * k, 0, 1.0).reshape(m, k).copy()
     clean = run(m, k, n, x=x)[3]
     x[at, k - 1] = bad  # (what a lane beyond the row's end loads again)
-    y = run(m, k, n, x=x)[3]
-    assert not np.isfinite(y[at]).any()
+    run_w, run_b, _, y = run(m, k, n, x=x)
+    with np.errstate(all="ignore"):
+        assert_same_class(oracle.linear_forward(k, n, run_w, run_b, x)[at:at + 1], y[at:at + 1], f"{bad}")
     keep = np.arange(m) != at
     assert np.array_equal(y[keep], clean[keep])
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan, 3.4e38, -3.4e38])
+@pytest.mark.parametrize("m,k,n", [(9, 128, 96), (12, 768, 130), (15, 3072, 65), (70, 768, 96), (9, 128, 33000), (130, 192, 8300)])
+def test_what_an_fp32_sum_keeps(zg, bad, m, k, n):
+    """An infinity times a number is an infinity, times zero NaN; a number beyond the largest bf16 is a number: in a row of inputs, and in
+    a row of weights (one slice of K and several).  Some of what they meet has one bf16 term only, whose other terms are zero."""
+    x = synth.fill_normal(1, m * k, 0, 1.0).reshape(m, k).copy()
+    w = synth.fill_normal(2, n * k, 0, 0.05).reshape(n, k).copy()
+    b = synth.fill_normal(3, n, 0, 0.05)
+    row, at = m - 2, k - 3
+    w[: n // 2, at] = np.resize(np.array([1.0, -2.0, 0.5, 0.0, 1e-30, -1e-30, 2.0 ** -130], np.float32), n // 2)
+    xs, ws = x.copy(), w.copy()
+    xs[row, at] = bad
+    with np.errstate(all="ignore"):
+        want = oracle.linear_forward(k, n, w, b, xs)
+        y = np.full((m, n), 7.0, np.float32)
+        ops.Linear(k, n, w, b).forward(xs, y)
+        assert_same_class(want, y, f"input {bad}")
+        col = n - 1
+        x[: m // 2, at] = np.resize(np.array([1.0, -2.0, 0.0, 1e-30], np.float32), m // 2)
+        ws[col, at] = bad
+        want = oracle.linear_forward(k, n, ws, b, x)
+        ops.Linear(k, n, ws, b).forward(x, y)
+        assert_same_class(want[:, :col], y[:, :col], f"beside weight {bad}")
+        assert_same_class(want[:, col:], y[:, col:], f"weight {bad}")
+
+
+@pytest.mark.parametrize("m,k,n", [(9, 128, 96), (12, 768, 130), (70, 3072, 96)])
+@pytest.mark.parametrize("size", [1e-37, 2e-38, 1e-30])
+def test_small_numbers(zg, size, m, k, n):
+    """Inputs whose second and third terms are below the smallest normal number (their products are normal numbers again)."""
+    x = (synth.fill_normal(1, m * k, 0, 1.0) * np.float32(size)).reshape(m, k)
+    w = (synth.fill_normal(2, n * k, 0, 1.0) * np.float32(1e30)).reshape(n, k)
+    y = np.full((m, n), 7.0, np.float32)
+    ops.Linear(k, n, w, None).forward(x, y)
+    assert_ref_close(oracle.linear_forward(k, n, w, None, x), y, f"Linear {m}x{k}x{n} at {size}", scale_floor=2e-6)
