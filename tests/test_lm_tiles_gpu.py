@@ -56,8 +56,6 @@ def test_rounded_rows(monkeypatch, rows):
         layers = [tl.hgrn2_layer(heads=2, dim=24, vdim=64, mlp=tl.dense_mlp(ff=ff)),
                   tl.latent_layer(heads=3, dim=16, vdim=16, rot_dim=8, kv_rank=rank, q_rank=rank, mlp=tl.dense_mlp(ff=ff)),
                   tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=ff, experts=5, top=2))]
-        if bad:  # (attention multiplies the masked values of a tile by zero)
-            del layers[1]
         cfg = tl.config(layers, vocab=203, width=width)
         w = tl.weights(cfg, seed=rows)
         toks = tl.tokens(30 + rows, rows, cfg["vocab"])
@@ -104,10 +102,7 @@ def test_latent_tiles(kv_rank, rot_dim):
     m.close()
 
 
-@pytest.mark.parametrize("bad", [None, np.inf, np.nan])
-@pytest.mark.parametrize("kv_rank,rot_dim", [(64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])
-def test_latent_tiles_32_bit(kv_rank, rot_dim, bad):
-    """The same in 32-bit mode; a token that is not finite leaves the rows in front of it alone, also those of its own tile of keys."""
+def portions_with_a_bad_token(kv_rank, rot_dim, bad, dtype):
     cfg = tl.config([tl.latent_layer(heads=5, dim=16, vdim=16, rot_dim=rot_dim, rot_dims=rot_dim, kv_rank=kv_rank, q_rank=40, mlp=tl.dense_mlp(ff=96))],
                     vocab=203, width=64)
     w = tl.weights(cfg, seed=kv_rank)
@@ -123,7 +118,7 @@ def test_latent_tiles_32_bit(kv_rank, rot_dim, bad):
             ends[b] = at
         w["embed"] = w["embed"].copy()
         w["embed"][7, 3] = bad
-    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=512, max_seqs=3)
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=512, max_seqs=3)
     m.load_weights(w)
     seqs = [m.open() for _ in toks]
     lo = [0, 0, 0]
@@ -133,10 +128,25 @@ def test_latent_tiles_32_bit(kv_rank, rot_dim, bad):
         for part, ref, a, b, end in zip(parts, refs, lo, hi, ends):
             n = min(b, end) - a
             if n > 0:
-                tl.assert_close(part[:n], ref[a:a + n], "float32", (kv_rank, bad, a, b))
+                tl.assert_close(part[:n], ref[a:a + n], dtype, (kv_rank, bad, a, b))
             assert not np.isfinite(part[max(n, 0):]).all(axis=1).any()
         lo = hi
     m.close()
+
+
+@pytest.mark.parametrize("bad", [None, np.inf, np.nan])
+@pytest.mark.parametrize("kv_rank,rot_dim", [(64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])
+def test_latent_tiles_32_bit(kv_rank, rot_dim, bad):
+    """The same in 32-bit mode; a token that is not finite leaves the rows in front of it alone, also those of its own tile of keys."""
+    portions_with_a_bad_token(kv_rank, rot_dim, bad, "float32")
+
+
+@pytest.mark.parametrize("bad", [np.inf, -np.inf, np.nan])
+@pytest.mark.parametrize("kv_rank,rot_dim", [(64, 0), (64, 32), (100, 20), (128, 0), (256, 0), (256, 32), (300, 12), (320, 0), (320, 64)])
+def test_latent_tiles_and_a_bad_token(kv_rank, rot_dim, bad):
+    """... and in bf16 mode: rows of its own block of queries, and of earlier blocks whose last tile holds it (a portion that begins inside
+    a tile of keys); latents that fill the tile's value columns, with a rotated part behind them and without."""
+    portions_with_a_bad_token(kv_rank, rot_dim, bad, "bfloat16")
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])

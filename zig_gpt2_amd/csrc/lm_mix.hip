@@ -1059,16 +1059,22 @@ __device__ __forceinline__ bool find_entry(int id, const int* ent_start, const i
 // The cached rows of every entry of the step as key tiles, back to back in entry order.  Each tile is read by every query block
 // behind it and by all heads: converting it once (8 x 1023 rows of 288 values: 9 us) took the conversion, the page table and the
 // 4-byte loads out of loops that ran 16 times over every tile.
+// A tile is multiplied for queries in front of some of its keys too, with weight zero, and zero times a value that is not finite is not
+// zero: such values of the latent part are left out, and the row's last column, which only the scores read, says so (NaN): the queries that see
+// the key come out NaN, the others do not meet it.
 template <int NKS>
-__global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, int DT, const int* ent_start, const int* ent_len, const int* ent_slot,
+__global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, int DT, int KR, const int* ent_start, const int* ent_len, const int* ent_slot,
                                                            int n_entries, const int* row_pos, const int* page_table, int max_pages, int page_tokens,
                                                            bf16_t* tiles) {
     typedef KeyTile<NKS> T;
+    __shared__ unsigned s_bad;  // rows with a latent value that is not finite (as bf16)
     const int e = blockIdx.y, lane = threadIdx.x & 63;
     const int len = ent_len[e];
     if (len <= 0) return;
     const int n_keys = row_pos[ent_start[e] + len - 1] + 1;
     if ((int)blockIdx.x * 32 >= n_keys) return;
+    if (threadIdx.x == 0) s_bad = 0;
+    __syncthreads();
     int first = 0;  // tiles of the entries in front
     for (int e0 = 0; e0 < e; e0 += 64) {
         const int o = e0 + lane, ol = o < e ? ent_len[o] : 0;
@@ -1095,9 +1101,22 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
                 for (int u = 0; u < 8; ++u)
                     if (c * 8 + u < DT) v[u] = row[c * 8 + u];
             }
+            bool bad = false;
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (c * 8 + u < KR && !(fabsf(v[u]) < 3.3961775e38f)) {  // (from here on it rounds to an infinity)
+                    v[u] = 0.0f;
+                    bad = true;
+                }
+            if (bad) atomicOr(&s_bad, 1u << key);
         }
         *reinterpret_cast<u32x4*>(out + key * T::LD + (c ^ ((key >> 2) & 3)) * 8) =
             u32x4{cvt_pk_bf16(v[0], v[1]), cvt_pk_bf16(v[2], v[3]), cvt_pk_bf16(v[4], v[5]), cvt_pk_bf16(v[6], v[7])};
+    }
+    __syncthreads();
+    if (threadIdx.x < 32 && (s_bad >> threadIdx.x & 1u) != 0) {
+        constexpr int c = T::DT / 8 - 1;  // (behind the 32 NT value columns of every kernel that reads these tiles)
+        out[threadIdx.x * T::LD + (c ^ ((threadIdx.x >> 2) & 3)) * 8 + 7] = 0x7FC0;
     }
 }
 
@@ -1117,7 +1136,7 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
                                                                        const int* ent_start, const int* ent_len, const int* ent_slot, int n_entries, const int* row_pos,
                                                                        const bf16_t* tiles, const float* gate, int ldg, const float* sink) {
     typedef KeyTile<NKS> T;
-    static_assert(NT * 32 <= T::DT, "the latent part lies inside the rows");
+    static_assert(NT * 32 < T::DT, "the latent part lies inside the rows, in front of their last column");
     __shared__ __attribute__((aligned(1024))) char Ks[2][T::BYTES];
     EntryAt at;
     if (!find_entry(gridDim.x - 1 - blockIdx.x, ent_start, ent_len, ent_slot, n_entries, row_pos, at)) return;
@@ -1843,7 +1862,7 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
     const dim3 cgrid((max_keys + 31) / 32, n_entries), grid((M + 31) / 32 + n_entries, (H + 3) / 4);
 #define ZG_ATT_T(NKS_, NT_)                                                                                                                          \
     do {                                                                                                                                             \
-        latent_tiles_kernel<NKS_><<<cgrid, 256, 0, s>>>(cache, KR + R, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, max_pages,      \
+        latent_tiles_kernel<NKS_><<<cgrid, 256, 0, s>>>(cache, KR + R, KR, ent_start, ent_len, ent_slot, n_entries, row_pos, page_table, max_pages,      \
                                                         page_tokens, ws);                                                                            \
         ZG_HIP(hipGetLastError());                                                                                                                   \
         latent_attention_mfma_kernel<NKS_, NT_><<<grid, 256, 0, s>>>(qa, qa16, ctx, ctx16, H, KR, R, scale, ent_start, ent_len, ent_slot, n_entries, row_pos, ws, gate, ldg, \
