@@ -35,6 +35,23 @@ def test_tokens_of_steps_ahead(design, n_seqs):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("page_tokens", [1, 3])
+@pytest.mark.parametrize("design", sorted(DESIGNS))
+def test_a_page_every_step(design, page_tokens):
+    """Every sequence grows by a page with nearly every step in flight, and tables of windowed designs wrap round."""
+    lib, cfg = DESIGNS[design]
+    w = lib.weights(cfg, seed=11)
+    prompts = [lib.tokens(b, 2 + 3 * b, cfg["vocab"]) for b in range(8)]
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=768, max_seqs=8, page_tokens=page_tokens, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append([m.generate(prompts, 60), m.generate(prompts[::-1], 33, temp=1.0, seed=3)])
+        m.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
 def test_key_buckets():
     lib, cfg = DESIGNS["whole"]
     w = lib.weights(cfg, seed=2)

@@ -1637,8 +1637,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     return ZG_OK;
 }
 
-// The rows of a portion and their pages: metadata to the pinned twin and to the device.  wants: (row of the portion, output row)
-int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair<int, size_t>>& wants) {
+// The rows of a portion and (tables) their pages: metadata to the pinned twin and to the device.  wants: (row of the portion, output row).
+// The tables leave from pageable memory: only where the stream is drained before the host changes them again.
+int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair<int, size_t>>& wants, bool tables = true) {
     hipStream_t s = g->stream;
     const int MS = g->MS, NS = g->NS, n_ent = (int)pieces.size();
     int *ids = g->h_meta, *pos = ids + MS, *slot = pos + MS, *prev = slot + MS, *lastent = prev + MS, *want_rows = lastent + MS;
@@ -1666,7 +1667,7 @@ int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair
         }
         for (auto& w : pc.wants) wants.push_back({ent_start[e] + w.first, w.second});
         const Slot& sl = g->slots[pc.slot];
-        ZG_HIP(hipMemcpyAsync(g->page_table + (size_t)pc.slot * g->max_pages, sl.ring.data(), sl.ring.size() * sizeof(int), hipMemcpyHostToDevice, s));
+        if (tables) ZG_HIP(hipMemcpyAsync(g->page_table + (size_t)pc.slot * g->max_pages, sl.ring.data(), sl.ring.size() * sizeof(int), hipMemcpyHostToDevice, s));
     }
     ZG_HIP(hipMemcpyAsync(g->meta, g->h_meta, meta_ints(g) * sizeof(int), hipMemcpyHostToDevice, s));
     return ZG_OK;
@@ -1886,7 +1887,7 @@ int step_impl(zg_lm* g, const zg_lm_entry* entries, size_t n_entries, float* log
 
 // The steps of a generation behind its prompts: every sequence one token at a time.  What a step needs from the one before it, the tokens
 // and positions, is handed on by the device (advance_rows), so steps are enqueued ahead of the tokens the host has seen (at most kAhead)
-// and no step waits for a round trip to the host.  Bookkeeping and errors are those of the steps taken one by one: tokens of the steps
+// and no step waits for a round trip to the host.  New pages travel as launch arguments: the host goes on changing its tables.  Bookkeeping and errors are those of the steps taken one by one: tokens of the steps
 // in front of a failing one are delivered.  first: the tokens the prompts' step drew.
 int decode_ahead(zg_lm* g, const std::vector<int>& seqs, const int32_t* first, size_t n_new, float temp, uint64_t seed, int32_t* out_tokens) {
     hipStream_t s = g->stream;
@@ -1905,25 +1906,28 @@ int decode_ahead(zg_lm* g, const std::vector<int>& seqs, const int32_t* first, s
         for (int b = 0; b < M; ++b) ZG_TRY(count_pages(g, seqs[b], 1, need));
         ZG_TRY(pages_left(g, need));
         std::vector<Piece> pieces;
+        NewPages grown;
         g->step_keys = 0;
         for (int b = 0; b < M; ++b) {
             Slot& sl = g->slots[seqs[b]];
-            const bool grew = take_pages(g, sl, 1);
+            if (take_pages(g, sl, 1)) {  // one token takes one page at most
+                grown.at[grown.n] = (int)((size_t)seqs[b] * g->max_pages + (sl.pages.size() - 1) % g->max_pages);
+                grown.page[grown.n++] = sl.pages.back();
+            }
             if (enqueued == 1) {
                 Piece pc;
                 pc.slot = seqs[b]; pc.tok = first + b; pc.n = 1; pc.pos0 = (int)sl.len;
                 pieces.push_back(pc);
-            } else if (grew) {
-                ZG_HIP(hipMemcpyAsync(g->page_table + (size_t)seqs[b] * g->max_pages, sl.ring.data(), sl.ring.size() * sizeof(int), hipMemcpyHostToDevice, s));
             }
             g->step_keys = std::max(g->step_keys, (int)sl.len + 1);
         }
         if (enqueued == 1) {
             std::vector<std::pair<int, size_t>> wants;
             for (int b = 0; b < M; ++b) g->h_meta[5 * (size_t)MS + b] = b;
-            ZG_TRY(stage_rows(g, pieces, wants));
+            ZG_TRY(stage_rows(g, pieces, wants, false));  // (the prompts' step has left the tables)
             ZG_HIP(hipEventRecord(g->ev0, s));
         }
+        ZG_TRY(launch_new_pages(g->page_table, grown, s));
         const int at = (int)(enqueued % zg_lm::kAhead);
         ZG_TRY(replay_step(g, M, key_bucket(g)));
         ZG_TRY(enqueue_logits(g, M));

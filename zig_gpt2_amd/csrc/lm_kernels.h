@@ -484,6 +484,11 @@ int launch_moe_combine(const float* x, float* out, const float* yexp, const int*
 // ------------------------------------------------------------------------------------------------ sampling support
 // rows of the next step of a generation: ids[r] = seen[r] = tok[r], pos[r] += 1  (seen: pinned host memory)
 int launch_advance_rows(const int* tok, int M, int* ids, int* pos, int* seen, hipStream_t s);
+// entries of the page table that such a step adds, one a row at most: table[at[i]] = page[i]
+struct NewPages {
+    int at[kGemvMaxRows] = {}, page[kGemvMaxRows] = {}, n = 0;
+};
+int launch_new_pages(int* table, const NewPages& pages, hipStream_t s);
 // Per row: the maximum of its logits and the index of the first element that reaches it.  part_val / part_idx: workspace of
 // rows * kArgmaxParts elements each (the row is scanned in slices by that many workgroups, a second launch combines them).
 constexpr int kArgmaxParts = 64;

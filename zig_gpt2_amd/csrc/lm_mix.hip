@@ -1528,6 +1528,12 @@ __global__ __launch_bounds__(64) void advance_rows_kernel(const int* tok, int M,
     seen[r] = t;
 }
 
+__global__ __launch_bounds__(64) void new_pages_kernel(int* table, const NewPages pages) {
+#pragma unroll
+    for (int i = 0; i < kGemvMaxRows; ++i)
+        if ((int)threadIdx.x == i && i < pages.n) table[pages.at[i]] = pages.page[i];
+}
+
 // Stage 1: block (row, part) finds the maximum and its first index in its slice of the row; stage 2 (parts == 1 in the grid,
 // n_parts > 0 as argument): one block per row combines the parts.  The first maximum wins; a row of NaNs gives index 0.
 __global__ __launch_bounds__(256) void row_argmax_kernel(const float* logits, int n, float* max_out, int* idx_out, float* part_val, int* part_idx,
@@ -1940,6 +1946,14 @@ int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, i
 int launch_advance_rows(const int* tok, int M, int* ids, int* pos, int* seen, hipStream_t s) {
     if (M <= 0) return ZG_OK;
     advance_rows_kernel<<<(M + 63) / 64, 64, 0, s>>>(tok, M, ids, pos, seen);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_new_pages(int* table, const NewPages& pages, hipStream_t s) {
+    if (pages.n <= 0) return ZG_OK;
+    ZG_REQUIRE(pages.n <= kGemvMaxRows, ZG_ERR_ARG, "new pages: %d at a time", pages.n);
+    new_pages_kernel<<<1, 64, 0, s>>>(table, pages);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
