@@ -23,6 +23,7 @@
 
 #include "prefill_epi.h"
 #include "zg_kernels.h"
+#include "zg_once.h"
 
 namespace zg {
 
@@ -977,12 +978,14 @@ template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false>
 int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, int n_sl,
                   const PrefillQkv& qa, hipStream_t s) {
     using P = S4<NT>;
-    static bool raised = false;
-    if (!raised) {
+    static OncePerDevice raised;  // (handles of the layered tier may be on different devices)
+    int device = 0;
+    ZG_HIP(hipGetDevice(&device));
+    ZG_TRY(raised.run(device, []() -> int {
         ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK>),
                                    hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS));
-        raised = true;
-    }
+        return ZG_OK;
+    }));
     const int tiles_m = (M + 255) / 256, tiles_n = (N + P::BN - 1) / P::BN, n_tiles = tiles_m * tiles_n * n_sl;
     int gw = 8;  // tile-order band width (sweep 1 .. 16: profiles/NOTEBOOK.md)
     if (gw > tiles_n) gw = tiles_n;
