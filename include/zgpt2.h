@@ -516,7 +516,9 @@ typedef struct {
     float residual_mult;    /* ZG_LM_TANH_NORMS: x += residual_mult * norm(sublayer output) (0: 1) */
 } zg_lm_config;
 typedef struct zg_lm zg_lm;
-/* One arena for weights, state and scratch; the handle owns a stream on `device`.  Needs no zg_init. */
+/* One arena for weights, state and scratch (bf16 mode: with rounded copies of a portion's rows and, for latent attention, of every token
+ * the cache holds; a device without room for these gets a handle without them, whose portions are slower); the handle owns a stream on
+ * `device`.  Needs no zg_init. */
 int zg_lm_create(zg_lm** out, const zg_lm_config* config, int device);
 int zg_lm_destroy(zg_lm* g);
 /* Weights by checkpoint name: `embed`, `head`, `final.norm`, and per layer i `l<i>.norm1|norm1b|norm2|norm2b|shift|canon1|canon2`

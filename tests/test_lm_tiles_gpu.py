@@ -2,6 +2,7 @@
 (rows around a tile's edge, K with a remainder behind the last K step, groups of experts that are empty or one row long)."""
 import numpy as np
 import pytest
+import torch
 
 import lm_oracle
 import lm_testlib as tl
@@ -76,6 +77,31 @@ def test_rounded_rows(monkeypatch, rows):
             m.close()
             tl.assert_close(got[:cut], ref[:cut], "bfloat16", (rows, width, form))
             assert not np.isfinite(got[cut:]).any()
+
+
+def test_without_room_for_rounded_rows(monkeypatch):
+    """A device without room for the rounded rows and key tiles: the handle is made without them, portions and steps are the same."""
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=24, vdim=64, mlp=tl.dense_mlp(ff=328)),
+                     tl.latent_layer(heads=3, dim=16, vdim=16, rot_dim=8, kv_rank=128, q_rank=40, mlp=tl.dense_mlp(ff=96)),
+                     tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=152, experts=2, top=2))], vocab=203, width=136)
+    w = tl.weights(cfg, seed=1)
+    toks = [tl.tokens(90 + b, n, cfg["vocab"]) for b, n in enumerate((150, 97, 66))]
+    refs = [lm_oracle.Model(cfg, w).forward(t)[0] for t in toks]
+    used = []
+    for lean in (True, False):
+        monkeypatch.setenv("ZGPT2_LM_LEAN", "1") if lean else monkeypatch.delenv("ZGPT2_LM_LEAN")
+        free = torch.cuda.mem_get_info()[0]
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="bfloat16", max_tokens=1 << 18, max_seqs=3, max_step_tokens=512)
+        used.append(free - torch.cuda.mem_get_info()[0])
+        m.load_weights(w)
+        seqs = [m.open() for _ in toks]
+        lo = [0, 0, 0]
+        for hi in ((33, 1, 31), (149, 96, 65), (150, 97, 66)):
+            got = m.step([(s, t[a:b], list(range(b - a))) for s, t, a, b in zip(seqs, toks, lo, hi)])
+            tl.assert_close(got, np.concatenate([r[a:b] for r, a, b in zip(refs, lo, hi)]), "bfloat16", (lean, hi))
+            lo = hi
+        m.close()
+    assert used[1] - used[0] >= (1 << 18) * 160 * 2  # a tile row of 160 columns a token
 
 
 @pytest.mark.parametrize("kv_rank,rot_dim", [(40, 6), (64, 32), (100, 20), (256, 32), (300, 12), (320, 64)])

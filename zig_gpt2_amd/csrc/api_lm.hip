@@ -246,7 +246,9 @@ struct zg_lm {
     size_t trace_floats = 0;
     float last_step_ms = 0.0f, last_decode_ms = 0.0f;
     bool use_graph = true;
-    // rows of prompt portions rounded to bf16 by the kernels that write them, for the matrix product that reads them (bf16 mode)
+    // bf16 mode, where the device has room for them: rows of prompt portions rounded to bf16 by the kernels that write them, for the matrix
+    // product that reads them, and tiles of cached keys.  lean: it has not, and portions take the kernels that need neither.
+    bool lean = false;
     bf16_t *h16 = nullptr, *hc16 = nullptr, *o16 = nullptr, *u16 = nullptr;
     bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
     size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
@@ -733,7 +735,7 @@ void layout(zg_lm* g, Bump& b) {
     g->gu_buf = b.take<float>(MS * max_gu);
     g->hb = b.take<float>(MS * max_hb);
     g->ye = b.take<float>(MS * max_assign * W);
-    if (!g->f32) {
+    if (!g->f32 && !g->lean) {
         g->h16 = b.take<bf16_t>(MS * W);
         if (g->side) g->hc16 = b.take<bf16_t>(MS * W);
         g->o16 = b.take<bf16_t>(MS * max_o);
@@ -748,8 +750,8 @@ void layout(zg_lm* g, Bump& b) {
     g->scan_ws = b.take<float>(std::max<size_t>(1, g->scan_ws_floats));
     g->attn_ws_floats = (size_t)kGemvMaxRows * kAttnSplits * max_att_part;
     g->attn_ws = b.take<float>(std::max<size_t>(1, g->attn_ws_floats));
-    g->key_tile_elems = ((size_t)g->n_pages * g->P / 32 + NS) * max_tile;  // every cached token, a partly filled tile per sequence
-    g->key_tiles = b.take<bf16_t>(std::max<size_t>(1, g->key_tile_elems));
+    g->key_tile_elems = g->lean ? 0 : ((size_t)g->n_pages * g->P / 32 + NS) * max_tile;  // every cached token, a partly filled tile per sequence
+    g->key_tiles = g->key_tile_elems > 0 ? b.take<bf16_t>(g->key_tile_elems) : nullptr;
     // scores and partial sums of the split windowed attention: up to 2 GiB for a whole portion, else for steps of few rows only
     // (longer steps of such a model then take the general kernel)
     if (max_win > ((size_t)1 << 29)) max_win = 0;
@@ -931,7 +933,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     const bool tnorm = g->tanh_norms;
     // Prompt portions in bf16 mode: what only matrix products read travels rounded to bf16, from the kernel that writes it, where its rows
     // are whole 16-byte pieces (the products would round it to the same values; half the bytes, and operands that go to the LDS as they are)
-    const bool r16 = !f32 && !few;
+    const bool r16 = !f32 && !few && !g->lean;
     const bool h_r16 = r16 && W % 8 == 0 && !canon && !tnorm;
     auto whole = [](int n) { return n % 8 == 0; };
     // side-by-side sublayers: the sums a layer leaves for the next layer's norm kernel to add
@@ -2140,17 +2142,24 @@ int zg_lm_create(zg_lm** out, const zg_lm_config* config, int device) {
     // kept first tokens hold their pages for good: the pages between them and the window go back to the pool, but the page table
     // cannot wrap round (a sequence is then bounded by the table: max_tokens)
     g->keep_pages = g->keep_tokens > 0 ? (g->keep_first + g->P - 1) / g->P : 0;
-    Bump measure{nullptr};
-    layout(g, measure);
-    g->arena_bytes = measure.off + 256;
     auto fail = [&](int code) {
         zg_lm_destroy(g);
         return code;
     };
-    if (hipMalloc(reinterpret_cast<void**>(&g->arena), g->arena_bytes) != hipSuccess) {
+    // (the rounded rows and key tiles of portions, 192 to 832 bytes a token of the cache, are left out rather than the handle refused)
+    g->lean = !g->f32 && getenv("ZGPT2_LM_LEAN") != nullptr;  // (test hook)
+    for (;;) {
+        Bump measure{nullptr};
+        layout(g, measure);
+        g->arena_bytes = measure.off + 256;
+        if (hipMalloc(reinterpret_cast<void**>(&g->arena), g->arena_bytes) == hipSuccess) break;
         (void)hipGetLastError();
-        set_error("lm_create: %zu bytes of device memory not available", g->arena_bytes);
         g->arena = nullptr;
+        if (!g->f32 && !g->lean) {
+            g->lean = true;
+            continue;
+        }
+        set_error("lm_create: %zu bytes of device memory not available", g->arena_bytes);
         return fail(ZG_ERR_HIP);
     }
     Bump place{g->arena};
