@@ -1,12 +1,14 @@
 """fp32 Linears of few rows and of a medium number of rows (linear_tiles.hip): rows and columns around the edges of its tiles, one slice of K and several,
 the fewest and the most steps a slice has, sizes on both sides of the rule that leaves a Linear to the other kernels, values that are
 not finite."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import oracle
 from golden_io import assert_ref_close
-from zig_gpt2_amd import ops, synth
+from zig_gpt2_amd import _lib, ops, synth
 
 pytestmark = pytest.mark.gpu
 
@@ -34,9 +36,16 @@ def test_few_rows(zg, m, k, n):
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 
-@pytest.mark.parametrize("m,k,n", [(5, 6400, 70), (8, 8192, 40), (1500, 128, 3072), (2000, 128, 3072), (4100, 128, 1600), (20, 16448, 24), (40, 100, 37), (12, 64, 9)])
-def test_both_sides_of_the_rule(zg, m, k, n):
+@pytest.mark.parametrize("m,k,n,kernel", [(5, 6400, 70, "linear_few"), (8, 8192, 40, "linear_few"), (8, 128, 6144, "linear_few"), (8, 128, 6152, "gemv"),
+                                          (4, 128, 6152, "linear_few"), (1500, 128, 3072, "linear_tiles"), (1856, 128, 3072, "linear_tiles"),
+                                          (1857, 128, 3072, "gemm_s4"), (2000, 128, 3072, "gemm_s4"), (4100, 128, 1600, "gemm_s4"), (20, 16448, 24, "linear_tiles"),
+                                          (40, 100, 37, "gemv"), (12, 64, 9, "gemv"), (1, 768, 768, "gemv")])
+def test_both_sides_of_the_rule(zg, m, k, n, kernel):
+    run(1, 768, 768)  # (a general kernel; the ragged ones among them leave the note as it is)
     w, b, x, y = run(m, k, n)
+    name = C.create_string_buffer(160)
+    _lib.check(zg.zg_debug_last_kernel(name, 160))
+    assert name.value.decode().startswith(kernel)
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 

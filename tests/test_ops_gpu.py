@@ -5,6 +5,7 @@ vectors (tests/golden/ops.npz, produced by the reference's generate_test_data.py
 tolerance (src/tests.zig:4-20).  The second block compares against the CPU oracle on seeded inputs
 over shapes / edge cases the reference's tests do not reach.
 """
+import ctypes as C
 import os
 
 import numpy as np
@@ -111,32 +112,52 @@ def test_linear_sweep(zg, m, k, n):
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 
+def last_kernel(zg):
+    name = C.create_string_buffer(160)
+    _lib.check(zg.zg_debug_last_kernel(name, 160))
+    return name.value.decode()
+
+
 @pytest.mark.parametrize("m,k,n", [(1024, 768, 3072), (16, 128, 8), (300, 3072, 768), (1023, 768, 2304), (64, 1600, 6400),
                                    (16, 768, 50257), (40, 128, 37), (257, 192, 131), (33, 256, 1031)])  # widths that are not multiples of 4
 def test_linear_large_batch_runs_on_the_matrix_cores(zg, m, k, n):
-    """Linear.forward with batch >= 16 (ops.zig:22: batch = inputs.len / in_features) takes the MFMA GEMM — fp32
-    operands split exactly into bf16 planes — and still meets the reference tolerance against the fp32 oracle."""
+    """Linear.forward with batch >= 16 (ops.zig:22: batch = inputs.len / in_features) takes matrix-core tiles — fp32
+    operands split exactly into bf16 terms — and still meets the reference tolerance against the fp32 oracle."""
     w = synth.fill_normal(100 + n, n * k, 0, 0.05).reshape(n, k)
     b = synth.fill_normal(200 + n, n, 0, 0.05)
     x = synth.fill_normal(300 + m, m * k, 0, 1.0).reshape(m, k)
     y = z(m, n)
     before = zg.zg_debug_gemm_launches()
     ops.Linear(k, n, w, b).forward(x, y)
-    assert zg.zg_debug_gemm_launches() == before + 1, "batch >= 16 Linear did not take the MFMA path"
+    assert last_kernel(zg) == "linear_tiles_kernel" and zg.zg_debug_gemm_launches() == before
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n} (MFMA)", scale_floor=2e-6)
-    # batch < 16 stays on the GEMV kernels
+    # batch <= 8 stays on the row-vector kernels
     before = zg.zg_debug_gemm_launches()
     y8 = z(8, n)
     ops.Linear(k, n, w, b).forward(x[:8], y8)
-    assert zg.zg_debug_gemm_launches() == before
+    assert last_kernel(zg) == "linear_few_kernel" or last_kernel(zg).startswith("gemv_")
     assert_ref_close(y[:8], y8, "GEMV path vs MFMA path", scale_floor=2e-6)
 
 
+@pytest.mark.parametrize("m,k,n", [(4096, 128, 1600), (4096, 128, 1601), (6000, 192, 1031), (30000, 128, 131), (256, 128, 50257)])
+def test_linear_of_many_rows_runs_on_the_persistent_gemm(zg, m, k, n):
+    """Beyond what the small tiles are chosen for both operands are written as planes and the four-wave GEMM multiplies them, widths that
+    are not multiples of 4 among them."""
+    w = synth.fill_normal(100 + n, n * k, 0, 0.05).reshape(n, k)
+    b = synth.fill_normal(200 + n, n, 0, 0.05)
+    x = synth.fill_normal(300 + m, m * k, 0, 1.0).reshape(m, k)
+    y = z(m, n)
+    before = zg.zg_debug_gemm_launches()
+    ops.Linear(k, n, w, b).forward(x, y)
+    assert zg.zg_debug_gemm_launches() == before + 1 and last_kernel(zg) == "gemm_s4_kernel"
+    assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n} (planes)", scale_floor=2e-6)
+
+
 def test_linear_wider_than_the_four_wave_gemm_arguments(zg):
-    """in_features = 16384 at batch 16: rows of three planes (49152 elements) and 256 K-steps per plane are beyond what
-    gemm_s4_kernel's packed arguments express — the Linear must fall through to the eight-wave GEMM instead of failing
-    (the reference Linear has no size limit, src/ops.zig:21-46).  A ragged width, which only the four-wave kernel stores,
-    goes to the GEMV kernels — in K chunks of 8192 (round 5; it answered ZG_ERR_UNSUPPORTED before)."""
+    """in_features = 16384: rows of three planes (49152 elements) and 256 K-steps per plane are beyond what gemm_s4_kernel's
+    packed arguments express — a Linear of many rows must fall through to the eight-wave GEMM instead of failing (the
+    reference Linear has no size limit, src/ops.zig:21-46); batch 16 takes the small tiles.  A ragged width, which only the
+    four-wave kernel stores, goes to the GEMV kernels — in K chunks of 8192."""
     m, k, n = 16, 16384, 128
     w = synth.fill_normal(100 + n, n * k, 0, 0.02).reshape(n, k)
     b = synth.fill_normal(200 + n, n, 0, 0.05)
@@ -144,13 +165,31 @@ def test_linear_wider_than_the_four_wave_gemm_arguments(zg):
     y = z(m, n)
     before = zg.zg_debug_gemm_launches()
     ops.Linear(k, n, w, b).forward(x, y)
-    assert zg.zg_debug_gemm_launches() == before + 1
+    assert last_kernel(zg) == "linear_tiles_kernel"
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
     w130 = np.ascontiguousarray(np.resize(w, (130, k)))
     y130 = z(m, 130)
     ops.Linear(k, 130, w130, None).forward(x, y130)
-    assert zg.zg_debug_gemm_launches() == before + 1, "the ragged width must not take the MFMA path"
+    assert last_kernel(zg).startswith("gemv_"), "the ragged width must not take the MFMA path"
     assert_ref_close(oracle.linear_forward(k, 130, w130, None, x), y130, f"Linear {m}x{k}x130 (K chunks)", scale_floor=2e-6)
+    assert zg.zg_debug_gemm_launches() == before
+
+    import torch
+
+    m = n = 2400  # (1444 small tiles; both operands' planes take 450 MiB of the staging arena)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    x, w, b = (torch.randn(*s, generator=g, device="cuda") for s in ((m, k), (n, k), (n,)))
+    w *= 0.02
+    y = torch.empty(m, n, device="cuda")
+    torch.cuda.synchronize()
+    ops.Linear(k, n, w, b).forward(x, y)
+    assert zg.zg_debug_gemm_launches() == before + 1 and last_kernel(zg) == "gemm_p8_kernel"
+    want = torch.addmm(b.double(), x.double(), w.double().T)
+    # an output (2.6 in size, 13 at most) is a chain of 6 x 16384 / 16 = 6144 fp32 additions, each off by 0.29 x 2^-24 of the sum so far:
+    # sqrt(6144) x 0.29 x 2^-24 = 1.4e-6 of the largest sum, 1e-6 of the outputs as a whole (sums grow to their size: times 0.7); the worst
+    # of 5.8 million outputs lies 5.2 times as far off, 5.2 x 1.4e-6 x 13 = 9e-5
+    err = y - want
+    assert float(err.abs().max()) < 1e-4 and float(err.norm() / want.norm()) < 2e-6
 
 
 @pytest.mark.parametrize("m,k,n,bias", [(1, 8200, 37, True), (3, 12328, 70, True), (9, 20000, 16, False), (2, 16384, 2100, True),

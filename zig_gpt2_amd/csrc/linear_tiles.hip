@@ -282,7 +282,7 @@ int launch_linear_tiles(const float* X, const float* W, const float* bias, float
         linear_slabs_kernel<<<(unsigned)((n + 1023) / 1024), 256, 0, s>>>(slabs, slices, bias, Y, n, N, X, W, K);
         ZG_HIP(hipGetLastError());
     }
-    gemm_note_launch();
+    note_kernel("linear_tiles_kernel");
     return ZG_OK;
 }
 
@@ -306,6 +306,7 @@ int launch_linear_few(const float* X, const float* W, const float* bias, float* 
     else if (M <= 4) ZG_FEW(4);
     else ZG_FEW(8);
 #undef ZG_FEW
+    note_kernel("linear_few_kernel");
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
