@@ -224,3 +224,44 @@ def test_gated_rows_of_decode_steps(rows, ff):
         got = m.step([(s, [t[i]], [0]) for s, t in zip(seqs, toks)])
         tl.assert_close(got, np.stack([r[i] for r in refs]), "float32", (rows, ff, i))
     m.close()
+
+
+@pytest.mark.parametrize("form", ["128", "32", ""])
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+def test_weights_that_are_not_finite(monkeypatch, dtype, form):
+    """An infinite weight times a number is an infinity, also where lower terms of the number's split are zero: rows of the head that hold
+    one, in steps of one to eight rows and portions of a few and many."""
+    monkeypatch.setenv("ZGPT2_LM_GEMM_TILE", form) if form else monkeypatch.delenv("ZGPT2_LM_GEMM_TILE", raising=False)
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=24, vdim=64, mlp=tl.dense_mlp(ff=40))], vocab=203, width=136)
+    w = tl.weights(cfg, seed=4)
+    toks = tl.tokens(8, 300, cfg["vocab"])
+    clean = lm_oracle.Model(cfg, w).forward(toks)[0]
+    w["head"] = w["head"].copy()
+    for v in range(0, 200, 4):
+        w["head"][v, (7 * v) % 136] = np.inf if v % 8 else -np.inf
+    w["head"][201, 3] = np.nan
+    with np.errstate(all="ignore"):
+        ref = lm_oracle.Model(cfg, w).forward(toks)[0]
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=1024, max_seqs=8, max_step_tokens=512)
+    m.load_weights(w)
+
+    def check(got, want, plain, rounded):
+        assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(np.isinf(got), np.isinf(want))
+        inf = np.isinf(want)
+        # (a value that rounding moves across zero changes an infinity's sign: one in some hundred in bf16 mode)
+        assert np.mean(got[inf] == want[inf]) >= (0.97 if rounded else 1.0)
+        ok = np.isfinite(want).all(axis=0)
+        tl.assert_close(got[:, ok], plain[:, ok], dtype)
+
+    for rows in (9, 40, 300):
+        s = m.open()
+        check(m.step([(s, toks[:rows], list(range(rows)))]), ref[:rows], clean[:rows], dtype == "bfloat16")
+        m.close_seq(s)
+    for rows in range(1, 9):
+        seqs = [m.open() for _ in range(rows)]
+        for i in range(4):
+            got = m.step([(s, [toks[i]], [0]) for s in seqs])
+            check(got, np.repeat(ref[i:i + 1], rows, 0), np.repeat(clean[i:i + 1], rows, 0), False)
+        for s in seqs:
+            m.close_seq(s)
+    m.close()

@@ -406,6 +406,29 @@ __device__ __forceinline__ void put(const LinArgs& p, int m, int n, float v) {
     if (p.C16) p.C16[at] = (bf16_t)cvt_pk_bf16(v, v);
 }
 
+// Three terms: a weight that is infinite meets terms that are zero, and the sum is NaN where an fp32 sum is an infinity.  The outputs
+// (bit b of `which`: at(b)) that came out NaN again, as plain fp32 sums (one that has become NaN ends at once).
+template <typename F>
+__device__ __forceinline__ void again(const LinArgs& p, const TileAt& t, unsigned which, F&& at) {
+#pragma unroll 1
+    for (; which != 0; which &= which - 1) {
+        int m, n;
+        at(__builtin_ctz(which), m, n);
+        const float* a = a_row<float>(p, m);
+        const bf16_t* b = t.B + (long long)n * p.ldb;
+        float s = 0.0f;
+#pragma unroll 1
+        for (int k = 0; k < p.K && s == s; k += 8) {
+            Act8<float> x;
+            x.load(a, k);
+            const u32x4 w = load_b8(b, k);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s = fmaf(i < 2 ? x.a[2 * i + 1] : x.b[2 * i - 3], bf16_hi(w[i]), fmaf(i < 2 ? x.a[2 * i] : x.b[2 * i - 4], bf16_lo(w[i]), s));
+        }
+        put(p, m, n, s);
+    }
+}
+
 // What bounds it: the bytes a compute unit takes in (31 to 37 B per clock beside matrix products) and, per K step, one LDS round trip.
 // 8184 x 3072 x 1024 takes 106 us (490 TFLOP/s; before, with one LDS buffer and 64 x 64 tiles, 176), 8184 x 1024 x 4096 107 us
 // (640 TFLOP/s; 274), 333 x 768 x 3072 17.5 us (95): there the reads of a step's fragments, which the compiler had paired with a
@@ -545,18 +568,44 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LinArgs p) {
         });
 
     // accumulator element e of a 32 x 32 tile: row 8 (e / 4) + 4 (lane / 32) + e % 4, column lane % 32
+    auto row_of = [&](int i, int e) { return t.m0 + (wy * TM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3); };
+    auto column_of = [&](int j) { return t.n0 + (wx * TN + j) * 32 + (lane & 31); };
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const int n = t.n0 + (wx * TN + j) * 32 + (lane & 31);
+            const int n = column_of(j);
             if (n >= p.N) continue;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const int m = t.m0 + (wy * TM + i) * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
+                const int m = row_of(i, e);
                 if (m < t.m_end) put(p, m, n, acc[i][j][e]);
             }
         }
+    if constexpr (NP > 1) {
+        static_assert(TM * TN <= 2, "an output, a bit");
+        f32x16 all = acc[0][0];  // (NaN if one of them is)
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = i == 0 ? 1 : 0; j < TN; ++j) all += acc[i][j];
+        const float sum = (((all[0] + all[1]) + (all[2] + all[3])) + ((all[4] + all[5]) + (all[6] + all[7]))) +
+                          (((all[8] + all[9]) + (all[10] + all[11])) + ((all[12] + all[13]) + (all[14] + all[15])));
+        if (__builtin_expect(sum != sum, 0)) {
+            unsigned which = 0;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e)
+                        if (acc[i][j][e] != acc[i][j][e] && row_of(i, e) < t.m_end && column_of(j) < p.N) which |= 1u << ((i * TN + j) * 16 + e);
+            again(p, t, which, [&](int b, int& m, int& n) {
+                m = row_of((b >> 4) / TN, b & 15);
+                n = column_of((b >> 4) % TN);
+            });
+        }
+    }
 }
 
 // Too few tiles to fill the chip (portions of some hundred rows): 32 TM x 32 TN tiles, the four waves of a workgroup split K and meet
@@ -640,12 +689,34 @@ __global__ __launch_bounds__(256, 2) void lm_deep_kernel(const LinArgs p) {
             for (int e = 0; e < 16; ++e) part[wave][(i * TN + j) * 16 + e][lane] = acc[i][j][e];
     __syncthreads();
     constexpr int SHARE = TM * TN * 4;  // accumulator elements this wave sums and stores
+    auto place = [&](int x, int& m, int& n) {
+        const int el = wave * SHARE + x, e = el & 15, ij = el >> 4, i = ij / TN, j = ij % TN;
+        n = t.n0 + 32 * j + r;
+        m = t.m0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+    };
+    float all = 0.0f;  // (NaN if one of them is)
+    auto sum = [&](int x) {
+        const int el = wave * SHARE + x;
+        return (part[0][el][lane] + part[1][el][lane]) + (part[2][el][lane] + part[3][el][lane]);
+    };
 #pragma unroll
     for (int x = 0; x < SHARE; ++x) {
-        const int el = wave * SHARE + x, e = el & 15, ij = el >> 4, i = ij / TN, j = ij % TN;
-        const float v = (part[0][el][lane] + part[1][el][lane]) + (part[2][el][lane] + part[3][el][lane]);
-        const int n = t.n0 + 32 * j + r, m = t.m0 + 32 * i + 8 * (e >> 2) + 4 * kh + (e & 3);
+        const float v = sum(x);
+        int m, n;
+        place(x, m, n);
         if (n < p.N && m < t.m_end) put(p, m, n, v);
+        if (NP > 1) all += v;
+    }
+    if (NP > 1 && __builtin_expect(all != all, 0)) {
+        unsigned which = 0;
+#pragma unroll 1
+        for (int x = 0; x < SHARE; ++x) {
+            const float v = sum(x);
+            int m, n;
+            place(x, m, n);
+            if (v != v && n < p.N && m < t.m_end) which |= 1u << x;
+        }
+        again(p, t, which, place);
     }
 }
 

@@ -114,16 +114,17 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
                 }
             }
         }
-        // element e: weight row 4 kg + e, column col
+        // element e: weight row 4 kg + e, column col (leading and last terms, or middle ones).  An infinite sum of the leading terms is the
+        // result: the other terms of what met the infinity may be zero, and zero times infinity is not
 #pragma unroll
-        for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = acc1[e] + acc2[e];
+        for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = col < 8 && fabsf(acc1[e]) <= 3.4028235e38f ? acc1[e] + acc2[e] : acc1[e];
         __syncthreads();
         const int row = threadIdx.x & 15, om = threadIdx.x >> 4;
         if (om < n_rows && row < half && n0 + row < n_out) {
             auto sum = [&](int r) {
                 const float hi = (part[0][r][om] + part[1][r][om]) + (part[2][r][om] + part[3][r][om]);
                 const float mid = (part[0][r][om + 8] + part[1][r][om + 8]) + (part[2][r][om + 8] + part[3][r][om + 8]);
-                return hi + mid;
+                return fabsf(hi) <= 3.4028235e38f ? hi + mid : hi;
             };
             const float v = sum(row);
             float* C = p.C + (p.z_group ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
