@@ -164,9 +164,12 @@ bool rows_form(const Linear& L, LinArgs& p, int& nz) {
     }
     // Where it pays (us per launch, this against the general kernel): 3 rows 2304 x 768 4.3 : 5.6, 8 rows 4.9 : 9.5, 8 rows of the
     // vocabulary 31 : 75.  Beyond K = 1024 a compute unit's intake binds it and the general kernel's finer tiles spread over more of them: 3
-    // rows 768 x 3072 9.4 : 8.5, 4 rows 9.9 : 9.2, 8 rows 11.9 : 14.8.  Lists: 16 assignments over 8 experts of 1536 x 768 7.1 : 9.9, 8 of
-    // them 6.6 : 6.8, 6 of them 6.4 : 5.3.
-    const bool pays = L.z_group ? p.M >= 8 : p.M >= (L.K <= 1024 ? 3 : 6);
+    // rows 768 x 3072 9.4 : 8.5, 4 rows 9.9 : 9.2, 8 rows 11.9 : 14.8.
+    // Lists: an expert nobody chose costs a grid plane of empty workgroups, one chosen twice saves a reading, so the line rises with the number
+    // of experts.  Steps of four such layers, us, this against the general kernel, experts of 768 x 768: 8 of them, 8 assignments 172 : 168, 16
+    // 189 : 197, 32 206 : 239; 32 of them, 16 214 : 209, 24 231 : 235; 64, 16 227 : 217, 24 247 : 248, 32 257 : 265; 256, 8 (one row) 323 : 270,
+    // 32 352 : 337, 48 376 : 383.
+    const bool pays = L.z_group ? p.M >= 14 + L.n_groups / 8 : p.M >= (L.K <= 1024 ? 3 : 6);
     if (L.glu_out && L.a_glu) return false;
     return pays && (L.z_group || p.M <= 8) && p.a_vec && p.b_vec && L.K % 8 == 0 && L.a_glu % 4 == 0 && nz <= 65535;
 }
