@@ -94,7 +94,7 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
                 const Planes8<3> pl = to_planes<3>(x, y);
                 const u32x4 zero = {0u, 0u, 0u, 0u};
                 const bf16x8 wf = __builtin_bit_cast(bf16x8, wv);
-                acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, col < 8 ? pl.v[2] : zero), acc2, 0, 0, 0);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, col < 8 ? zero : pl.v[2]), acc2, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, col < 8 ? pl.v[0] : pl.v[1]), acc1, 0, 0, 0);
             }
         };
@@ -114,10 +114,10 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
                 }
             }
         }
-        // element e: weight row 4 kg + e, column col (leading and last terms, or middle ones).  An infinite sum of the leading terms is the
+        // element e: weight row 4 kg + e, column col (leading terms, or middle and last ones).  An infinite sum of the leading terms is the
         // result: the other terms of what met the infinity may be zero, and zero times infinity is not
 #pragma unroll
-        for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = col < 8 && fabsf(acc1[e]) <= 3.4028235e38f ? acc1[e] + acc2[e] : acc1[e];
+        for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = col < 8 ? acc1[e] : acc1[e] + acc2[e];
         __syncthreads();
         const int row = threadIdx.x & 15, om = threadIdx.x >> 4;
         if (om < n_rows && row < half && n0 + row < n_out) {
