@@ -142,13 +142,13 @@ int zg_softmax(float* inputs, size_t inputs_len);
  * any M; N a multiple of 8 for bf16 C, any N for fp32 C (an N that is not a multiple of 4 is stored by the four-wave kernel
  * only, whose packed arguments end at K = 16320: beyond that ZG_ERR_UNSUPPORTED — zg_linear_forward, which has no such limit,
  * takes such a Linear through its GEMV kernels); K a multiple of 64 and at least 128.  Asynchronous on
- * the library stream.  zg_linear_forward itself takes this path for batch >= 16 (fp32 operands split
- * exactly into bf16 planes, so the result stays fp32-sgemm grade).
+ * the library stream.  zg_linear_forward itself takes this path for some thousand rows and more (fp32 operands split
+ * exactly into bf16 planes, so the result stays fp32-sgemm grade); from nine rows on it splits inside smaller tiles.
  * zg_f32_to_bf16 converts a device or host fp32 array into a device bf16 array (round to nearest even). */
 int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_null, void* C, size_t M,
                     size_t N, size_t K, int gelu, int out_bf16);
-/* Diagnostic: number of matrix-core GEMM launches so far in this process (tests assert which path a
- * Linear took; no reference counterpart). */
+/* Diagnostic: number of launches of the persistent matrix-core GEMMs (four and eight waves) by the op and GPT-2 tiers so far in this
+ * process (tests assert which path a Linear took; no reference counterpart). */
 unsigned long long zg_debug_gemm_launches(void);
 /* Diagnostic: shader-clock stamps {count, start, end} of workgroup 0 / wave 0 of the last GEMM launched with
  * ZGPT2_GEMM_DBG bit 256 (tools/microbench/gemm_bench.cpp: cycles vs wall time = the clock the chip ran at). */

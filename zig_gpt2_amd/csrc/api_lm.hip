@@ -2146,7 +2146,7 @@ int zg_lm_create(zg_lm** out, const zg_lm_config* config, int device) {
         zg_lm_destroy(g);
         return code;
     };
-    // (the rounded rows and key tiles of portions, 192 to 832 bytes a token of the cache, are left out rather than the handle refused)
+    // (the rounded rows and key tiles of portions are left out rather than the handle refused)
     g->lean = !g->f32 && getenv("ZGPT2_LM_LEAN") != nullptr;  // (test hook)
     for (;;) {
         Bump measure{nullptr};

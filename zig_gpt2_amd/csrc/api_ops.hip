@@ -236,7 +236,8 @@ struct CallGuard {
     }
 };
 
-// Linear.forward for batch >= 16 on the matrix cores (ops.zig:21-46 with M = inputs.len / in_features, :22).
+// Linear.forward on the persistent matrix-core GEMMs, for the sizes that fill the chip with their tiles (16 rows at least; the rule in front
+// is linear_tiles_ok's; ops.zig:21-46 with M = inputs.len / in_features, :22).
 // The op tier is fp32 in, fp32 out, arbitrary fp32 weights: both operands are split EXACTLY into three bf16
 // planes (x = hi + mid + lo, 3 x 8 mantissa bits) and the GEMM sums the six plane products whose weight is
 // above 2^-24 of the leading one — every bf16 x bf16 product is exact in fp32 and accumulation is fp32, i.e. the

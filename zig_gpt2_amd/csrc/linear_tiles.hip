@@ -1,4 +1,5 @@
-// linear_tiles.hip — fp32 Linears of 16 rows to some thousand (y = x W^T + bias, src/ops.zig:21-46) in one pass over both operands.
+// linear_tiles.hip — fp32 Linears of nine rows to some thousand (y = x W^T + bias, src/ops.zig:21-46) in one pass over both operands, and of
+// two to eight rows (linear_few_kernel, below).
 //
 // Both operands are split exactly into three bf16 terms on their way into the LDS (x = hi + mid + lo) and the six products above 2^-24 of
 // the leading one are summed, as the persistent kernel for many rows does (gemm_s4.hip); here no planes are written to memory first, and

@@ -1,8 +1,11 @@
 // lm_linear.hip — the linear maps of the layered-model tier: C = act(A B^T) with fp32 activation rows A and bf16 weights B.
 //
 // Behind one launcher:
-//   * lm_gemv_kernel   up to 8 rows (decode steps): a wave owns two weight rows, its lanes split K in 16-byte pieces, the
+//   * steps of up to 8 rows: lm_gemv_at_once_kernel (lm_gemv.hip; one or two rows in whole 16-byte pieces), lm_rows_kernel (lm_rows.hip;
+//                      three rows and more, lists of experts), and for what these leave
+//   * lm_gemv_kernel   (long rows: lm_gemv_ks_kernel) a wave owns two weight rows, its lanes split K in 16-byte pieces, the
 //                      activation rows come straight from the cache hierarchy, sums are fp32 FMAs in both precision modes.
+//   * gemm_s4_kernel   (gemm_s4.hip) plain products of prompt portions whose rows are rounded already, from 112 tiles of 256 x 192 on.
 //   * lm_wide_kernel   prompt portions that fill the chip: 128 x 128 or 64 x 64 tiles staged through the LDS.
 //   * lm_deep_kernel   short portions: 32-wide tiles with K split over the waves of a workgroup.
 //                      Both multiply with v_mfma_f32_32x32x16_bf16: bf16 mode rounds the activations on their way there, 32-bit mode

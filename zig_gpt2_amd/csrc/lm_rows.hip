@@ -2,8 +2,8 @@
 //
 // A workgroup owns 16 weight rows; its four waves take K in turns of 64 columns and meet in the LDS.  The weights are the MFMA's rows,
 // straight from memory (a lane loads 32 bytes of its row, four lanes a 128-byte line).  The activations stay fp32: a value is the exact
-// sum of three bf16 terms, the eight rows' leading and middle terms are the sixteen columns of one product, their last terms half of
-// a second one.  Everything a wave needs is requested at entry for K up to 1024, four turns ahead beyond.
+// sum of three bf16 terms, the eight rows' leading and middle terms are the sixteen columns of one product, their last terms, under the
+// middle ones, half of a second one.  Everything a wave needs is requested at entry for K up to 1024, four turns ahead beyond.
 //
 // The general kernel (lm_gemv_kernel) reads all rows for every two weight rows: 8 x 24 KB of activations through each wave for 3 KB of
 // weights at K = 768.  Here they are read once per 16 weight rows.

@@ -362,7 +362,6 @@ __device__ __forceinline__ void put_row(float* out, bf16_t* out16, size_t at, fl
     else out[at] = v;
 }
 
-
 __global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int width, int parts, const float* w, float eps, const ConvArgs cv, const int* row_slot,
                                                         bf16_t* out16) {
     __shared__ float s_red[8];
