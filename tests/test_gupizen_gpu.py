@@ -205,6 +205,17 @@ def test_general_window_kernel(monkeypatch):
         m.close()
 
 
+@pytest.mark.parametrize("dim", [130, 192, 194, 256])
+def test_heads_wider_than_the_tiled_scores(dim):
+    """Heads of more than 128 channels: scores a row at a time in steps of any number of rows, two to four pieces of 64 channels a key."""
+    cfg = gl.config([gl.parallel_layer(heads=6, kv_heads=3, dim=dim, vdim=10, window=21, rot_dims=4, scale=dim ** -0.5)])
+    w = gl.weights(cfg, seed=dim)
+    toks = gl.tokens(26, 60, cfg["vocab"])
+    m = make(cfg, w)
+    tl.assert_close(run_cut(m, toks, [9, 10, 40]), go.Model(cfg, w).forward(toks)[0], "float32")
+    m.close()
+
+
 @pytest.mark.parametrize("hook", ["ZGPT2_LM_WINDOW_NO_TILES", "ZGPT2_LM_WINDOW_TILES"])
 def test_both_score_kernels_on_all_steps(monkeypatch, hook):
     """Prompt portions take their scores from matrix-core tiles of 32 rows x 32 keys, steps of few rows from the wave-per-key

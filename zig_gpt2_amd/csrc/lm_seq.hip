@@ -1437,7 +1437,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
         if (atoi(e) != 0) return ZG_OK;
     int n_split = 1;
     const size_t need = window_split_workspace(M, H, V, key_capacity, &n_split);
-    const int rpl = (D + 63) / 64;
+    const int rpl = D <= 64 ? 1 : D <= 128 ? 2 : 4;  // 64 channels each: the kernel's instantiations, which lay out the LDS by them
     const size_t lds_a = ((size_t)H * 64 * rpl + (size_t)H * kScoreTile + 2 * (size_t)H) * sizeof(float);
     const size_t lds_b = (2 * (size_t)H * kMixTile + (size_t)H * H + 2 * (size_t)H) * sizeof(float);
     if (!ws || need > ws_floats || H > kWinMaxHeads || H % G != 0 || H * V > 256 * kWinAcc || D > 256 || (vfreq && V % 2 != 0) || lds_a > 60 * 1024 ||
@@ -1471,8 +1471,8 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
 #define ZG_WS(R)                                                                                                                              \
     window_scores_kernel<R><<<dim3(n_split, M, G), 256, lds_a, s>>>(q, ldq, H, G, D, V, scale, mask, row_pos, row_slot, page_table, max_pages, page_tokens, cache, \
                                                      sc, key_capacity, st, shape)
-    if (rpl <= 1) ZG_WS(1);
-    else if (rpl <= 2) ZG_WS(2);
+    if (rpl == 1) ZG_WS(1);
+    else if (rpl == 2) ZG_WS(2);
     else ZG_WS(4);
 #undef ZG_WS
         ZG_HIP(hipGetLastError());
