@@ -216,6 +216,20 @@ def test_heads_wider_than_the_tiled_scores(dim):
     m.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(18, 6, 4, 34), (20, 5, 8, 8), (6, 3, 132, 10), (2, 1, 256, 6)])
+def test_rows_around_the_planes_of_key_heads(heads, kv_heads, dim, vdim):
+    """Steps of few rows have a plane of workgroups per key head in the kernels that take a row at a time, longer ones none: portions around the
+    line, with more heads than the tiled value product takes and heads wider than the tiled scores take."""
+    cfg = gl.config([gl.parallel_layer(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, window=21, rot_dims=4)])
+    w = gl.weights(cfg, seed=heads)
+    toks = gl.tokens(26, 90, cfg["vocab"])
+    ref = go.Model(cfg, w).forward(toks)[0]
+    m = make(cfg, w)
+    for cuts in ([9, 25, 42, 43], [16, 33, 40], [1, 2]):
+        tl.assert_close(run_cut(m, toks, cuts), ref, "float32", cuts)
+    m.close()
+
+
 @pytest.mark.parametrize("hook", ["ZGPT2_LM_WINDOW_NO_TILES", "ZGPT2_LM_WINDOW_TILES"])
 def test_both_score_kernels_on_all_steps(monkeypatch, hook):
     """Prompt portions take their scores from matrix-core tiles of 32 rows x 32 keys, steps of few rows from the wave-per-key

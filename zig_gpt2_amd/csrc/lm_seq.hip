@@ -481,8 +481,11 @@ __device__ __forceinline__ KeySpan window_range(int pos, const KeyMask& mask, in
 constexpr int kScoreTile = 128;  // keys whose scores a workgroup holds in the LDS at a time
 constexpr int kScoreKeys = 8;    // keys a wave has in flight
 
-// A workgroup takes one key head (blockIdx.z) and the heads that read it, here and in the mix: one row, three key heads, 16 shares 6.6 us
-// each, 13 and 8.7 when a workgroup went through the key heads one after the other.
+// In steps of few rows a workgroup takes one key head (blockIdx.z) and the heads that read it, here and in the mix: one row, three key heads,
+// 16 shares 6.6 us each, 13 and 8.7 when a workgroup goes through the key heads one after the other.  With more rows it does that: a plane of
+// the mix weighs every head where a matrix mixes them, and rows fill the chip by themselves (20 heads on 5 key heads, mixed, a stack
+// of four layers, us, planes : none: 9 rows 742 : 774, 16 rows 796 : 812, 24 rows 759 : 731, 120 rows 1047 : 855, 1600 rows 5381 : 2636).
+constexpr int kPlaneRows = 16;
 template <int RPL>
 __global__ __launch_bounds__(256) void window_scores_kernel(const float* q, int ldq, int H, int G, int D, int V, float scale, KeyMask mask, const int* row_pos, const int* row_slot, const int* page_table, int max_pages,
                                                             int page_tokens, const float* cache, float* sc, int NK, float* st,
@@ -498,7 +501,7 @@ __global__ __launch_bounds__(256) void window_scores_kernel(const float* q, int 
     int k0, k1;
     const KeySpan span = window_range(pos, mask, n_split, split, k0, k1);
     const int* pages = page_table + (size_t)row_slot[m] * max_pages;
-    const int rep = H / G, g = blockIdx.z, h0 = g * rep, h1 = h0 + rep;  // a key head and the heads that read it
+    const int per = G / gridDim.z, rep = H / G, g0 = blockIdx.z * per, h0 = g0 * rep, h1 = h0 + per * rep;  // key heads and the heads that read them
     const size_t cstride = (size_t)G * (D + V);
     for (int i = h0 * 64 * RPL + threadIdx.x; i < h1 * 64 * RPL; i += blockDim.x) {
         const int h = i / (64 * RPL), d = i % (64 * RPL);
@@ -519,7 +522,7 @@ __global__ __launch_bounds__(256) void window_scores_kernel(const float* q, int 
         __syncthreads();
         // a wave takes kScoreKeys keys at a time: all their loads are requested before the first product
         for (int kk = wave * kScoreKeys; kk < nt; kk += 4 * kScoreKeys) {
-            {
+            for (int g = g0; g < g0 + per; ++g) {
                 float kd[kScoreKeys][RPL];
 #pragma unroll
                 for (int u = 0; u < kScoreKeys; ++u) {
@@ -703,8 +706,8 @@ __global__ __launch_bounds__(256) void window_mix_kernel(int H, int G, int D, in
     int k0, k1;
     const KeySpan span = window_range(pos, mask, n_split, split, k0, k1);
     const int* pages = page_table + (size_t)row_slot[m] * max_pages;
-    // a key head and the heads that read it; their weights need every head's where a matrix mixes them
-    const int rep = H / G, g0 = blockIdx.z, h0 = g0 * rep, h1 = h0 + rep, w0 = talk ? 0 : h0, w1 = talk ? H : h1;
+    // key heads and the heads that read them; their weights need every head's where a matrix mixes them
+    const int per = G / gridDim.z, rep = H / G, h0 = blockIdx.z * per * rep, h1 = h0 + per * rep, w0 = talk ? 0 : h0, w1 = talk ? H : h1;
     const size_t cstride = (size_t)G * (D + V);
     for (int i = tid; i < H * H; i += blockDim.x) s_talk[i] = talk ? talk[i] : ((i / H) == (i % H) ? 1.0f : 0.0f);
     for (int h = w0 + (tid >> 6); h < w1; h += 4) {  // a wave per head, its lanes over the shares (at most kWinSplits = 64): one round trip
@@ -1446,7 +1449,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
     float* sc = ws;
     float* st = sc + (size_t)M * H * key_capacity;
     float* po = st + (size_t)M * n_split * H * 2;
-    const dim3 grid(n_split, M);
+    const int planes = M <= kPlaneRows ? G : 1;  // of key heads, in the kernels that take a row at a time
     bool tiles = false;
     if (const char* e = getenv("ZGPT2_LM_WINDOW_TILES")) tiles = atoi(e) != 0;  // test hook: the tiled scores also for steps of few rows
     const bool tiled = (M > kGemvMaxRows || tiles) && D <= 128 && ent_start && getenv("ZGPT2_LM_WINDOW_NO_TILES") == nullptr;
@@ -1469,7 +1472,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
         ZG_HIP(hipGetLastError());
     } else {
 #define ZG_WS(R)                                                                                                                              \
-    window_scores_kernel<R><<<dim3(n_split, M, G), 256, lds_a, s>>>(q, ldq, H, G, D, V, scale, mask, row_pos, row_slot, page_table, max_pages, page_tokens, cache, \
+    window_scores_kernel<R><<<dim3(n_split, M, planes), 256, lds_a, s>>>(q, ldq, H, G, D, V, scale, mask, row_pos, row_slot, page_table, max_pages, page_tokens, cache, \
                                                      sc, key_capacity, st, shape)
     if (rpl == 1) ZG_WS(1);
     else if (rpl == 2) ZG_WS(2);
@@ -1486,7 +1489,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
         window_mix_mfma_kernel<<<pg, 256, lds_c, s>>>(H, G, D, V, mask, sink, talk, ent_start, ent_len, n_entries, row_pos, row_slot, page_table,
                                                       max_pages, page_tokens, cache, sc, key_capacity, st, n_split, po);
     } else {
-        window_mix_kernel<<<dim3(n_split, M, G), 256, lds_b, s>>>(H, G, D, V, mask, sink, talk, row_pos, row_slot, page_table, max_pages, page_tokens, cache, sc,
+        window_mix_kernel<<<dim3(n_split, M, planes), 256, lds_b, s>>>(H, G, D, V, mask, sink, talk, row_pos, row_slot, page_table, max_pages, page_tokens, cache, sc,
                                                    key_capacity, st, po);
     }
     ZG_HIP(hipGetLastError());
