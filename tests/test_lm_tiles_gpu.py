@@ -53,7 +53,7 @@ def test_values_that_are_not_finite(dtype, bad):
 def test_rounded_rows(monkeypatch, rows):
     """Portions in bf16 mode, whose rows reach the products rounded: the persistent kernel (forced at any number of tiles; widths that end
     inside its tiles), the tile forms, and widths that are no whole 16-byte pieces, where the rows stay fp32."""
-    for width, ff, rank, bad in ((128, 328, 128, 0), (192, 320, 136, 1), (132, 100, 44, 0)):
+    for width, ff, rank, bad in ((128, 328, 128, 0), (192, 320, 136, 1), (132, 100, 44, 0), (128, 100, 40, 0), (192, 102, 64, 0)):
         layers = [tl.hgrn2_layer(heads=2, dim=24, vdim=64, mlp=tl.dense_mlp(ff=ff)),
                   tl.latent_layer(heads=3, dim=16, vdim=16, rot_dim=8, kv_rank=rank, q_rank=rank, mlp=tl.dense_mlp(ff=ff)),
                   tl.hgrn2_layer(heads=2, dim=24, vdim=68, mlp=tl.moe_mlp(ff=ff, experts=5, top=2))]
