@@ -485,11 +485,11 @@ constexpr int kScoreKeys = 8;    // keys a wave has in flight
 // 16 shares 6.6 us each, 13 and 8.7 when a workgroup goes through the key heads one after the other.  With more rows it does that: a plane of
 // the mix weighs every head where a matrix mixes them, and rows fill the chip by themselves (20 heads on 5 key heads, mixed, a stack
 // of four layers, us, planes : none: 9 rows 742 : 774, 16 rows 796 : 812, 24 rows 759 : 731, 120 rows 1047 : 855, 1600 rows 5381 : 2636).
-constexpr int kPlaneRows = 16;
+constexpr int kPlaneRows = 16;  // (per: key heads of a plane)
 template <int RPL>
 __global__ __launch_bounds__(256) void window_scores_kernel(const float* q, int ldq, int H, int G, int D, int V, float scale, KeyMask mask, const int* row_pos, const int* row_slot, const int* page_table, int max_pages,
                                                             int page_tokens, const float* cache, float* sc, int NK, float* st,
-                                                            const ScoreShape shape) {
+                                                            const ScoreShape shape, int per) {
     extern __shared__ __attribute__((aligned(16))) float s_sc[];
     float* s_q = s_sc;                     // [H][64 RPL] (zero beyond D)
     float* s_t = s_q + H * 64 * RPL;       // [H][kScoreTile] scores of the tile
@@ -501,7 +501,7 @@ __global__ __launch_bounds__(256) void window_scores_kernel(const float* q, int 
     int k0, k1;
     const KeySpan span = window_range(pos, mask, n_split, split, k0, k1);
     const int* pages = page_table + (size_t)row_slot[m] * max_pages;
-    const int per = G / gridDim.z, rep = H / G, g0 = blockIdx.z * per, h0 = g0 * rep, h1 = h0 + per * rep;  // key heads and the heads that read them
+    const int rep = H / G, g0 = blockIdx.z * per, h0 = g0 * rep, h1 = h0 + per * rep;  // key heads and the heads that read them
     const size_t cstride = (size_t)G * (D + V);
     for (int i = h0 * 64 * RPL + threadIdx.x; i < h1 * 64 * RPL; i += blockDim.x) {
         const int h = i / (64 * RPL), d = i % (64 * RPL);
@@ -693,7 +693,7 @@ __global__ __launch_bounds__(256) void window_stats_kernel(const float* sc, int 
 __global__ __launch_bounds__(256) void window_mix_kernel(int H, int G, int D, int V, KeyMask mask, const float* sink, const float* talk,
                                                          const int* row_pos, const int* row_slot, const int* page_table, int max_pages,
                                                          int page_tokens, const float* cache, const float* sc, int NK, const float* st,
-                                                         float* po) {
+                                                         float* po, int per) {
     extern __shared__ __attribute__((aligned(16))) float s_mx[];
     float* s_p = s_mx;                  // [H][kMixTile]
     float* s_w = s_p + H * kMixTile;    // [H][kMixTile]
@@ -707,7 +707,7 @@ __global__ __launch_bounds__(256) void window_mix_kernel(int H, int G, int D, in
     const KeySpan span = window_range(pos, mask, n_split, split, k0, k1);
     const int* pages = page_table + (size_t)row_slot[m] * max_pages;
     // key heads and the heads that read them; their weights need every head's where a matrix mixes them
-    const int per = G / gridDim.z, rep = H / G, h0 = blockIdx.z * per * rep, h1 = h0 + per * rep, w0 = talk ? 0 : h0, w1 = talk ? H : h1;
+    const int rep = H / G, h0 = blockIdx.z * per * rep, h1 = h0 + per * rep, w0 = talk ? 0 : h0, w1 = talk ? H : h1;
     const size_t cstride = (size_t)G * (D + V);
     for (int i = tid; i < H * H; i += blockDim.x) s_talk[i] = talk ? talk[i] : ((i / H) == (i % H) ? 1.0f : 0.0f);
     for (int h = w0 + (tid >> 6); h < w1; h += 4) {  // a wave per head, its lanes over the shares (at most kWinSplits = 64): one round trip
@@ -1473,7 +1473,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
     } else {
 #define ZG_WS(R)                                                                                                                              \
     window_scores_kernel<R><<<dim3(n_split, M, planes), 256, lds_a, s>>>(q, ldq, H, G, D, V, scale, mask, row_pos, row_slot, page_table, max_pages, page_tokens, cache, \
-                                                     sc, key_capacity, st, shape)
+                                                     sc, key_capacity, st, shape, G / planes)
     if (rpl == 1) ZG_WS(1);
     else if (rpl == 2) ZG_WS(2);
     else ZG_WS(4);
@@ -1490,7 +1490,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
                                                       max_pages, page_tokens, cache, sc, key_capacity, st, n_split, po);
     } else {
         window_mix_kernel<<<dim3(n_split, M, planes), 256, lds_b, s>>>(H, G, D, V, mask, sink, talk, row_pos, row_slot, page_table, max_pages, page_tokens, cache, sc,
-                                                   key_capacity, st, po);
+                                                   key_capacity, st, po, G / planes);
     }
     ZG_HIP(hipGetLastError());
     window_merge_kernel<<<M, 256, 0, s>>>(po, n_split, out, ldo, H, V, vfreq, row_pos, out_gate, ld_gate, out_factor);
