@@ -27,25 +27,36 @@ __device__ __forceinline__ void wave_sums(float (&v)[N]) {
     for (int i = 0; i < N; ++i) v[i] = wave_allsum(v[i]);
 }
 
-template <int MR, int U, int KIND, bool SPLIT>
-__device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const NormIn& pre) {
+// What the loads at entry need.  These travel as the leading arguments (14 dwords at most), which a wave finds in its registers; anything else
+// of a launch's arguments is a round trip to memory of its own, cold in a step that has a new block of them for every launch.  Behind one
+// such round trip a step of one sequence took 448 us, of eight 823; without it, here and in lm_rows.hip, 408 and 737, and with the norms, the
+// router and the recurrence's step done alike 705.
+struct GemvAt {
+    const float* A;
+    const bf16_t* B;
+    int K, N, ldb, lda, a_zoff, b_zoff, a_glu;
+};
+
+// INDIRECT: rows through an array, or a matrix chosen by a list
+template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT>
+__device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, const int z, const NormIn& pre) {
     constexpr int NS = KIND == GEMV_POLY ? 11 : 2;  // sums of a row: the two products; or q1 q2 q3 and four products for each weight row
     __shared__ float s_part[SPLIT ? 4 : 1][MR][NS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n0 = SPLIT ? blockIdx.x * 2 : blockIdx.x * 8 + wave * 2;
-    if (n0 >= p.N) return;
-    if (p.z_group && p.z_group[z] >= p.z_limit) return;
-    const bf16_t* B = p.B + (long long)(p.z_group ? p.z_group[z] : z) * p.b_zoff;
-    const bf16_t* w[2] = {B + (long long)n0 * p.ldb, B + (long long)min(n0 + 1, p.N - 1) * p.ldb};
-    const int kq = SPLIT ? (((p.K + 3) / 4) + 7) & ~7 : p.K;  // a wave's share of K, whole pieces of 8
-    const int k_lo = SPLIT ? wave * kq : 0, k_hi = SPLIT ? min(p.K, k_lo + kq) : p.K;
+    if (n0 >= t.N) return;
+    if (INDIRECT && p.z_group && p.z_group[z] >= p.z_limit) return;
+    const bf16_t* B = t.B + (long long)(INDIRECT && p.z_group ? p.z_group[z] : z) * t.b_zoff;
+    const bf16_t* w[2] = {B + (long long)n0 * t.ldb, B + (long long)min(n0 + 1, t.N - 1) * t.ldb};
+    const int kq = SPLIT ? (((t.K + 3) / 4) + 7) & ~7 : t.K;  // a wave's share of K, whole pieces of 8
+    const int k_lo = SPLIT ? wave * kq : 0, k_hi = SPLIT ? min(t.K, k_lo + kq) : t.K;
     int at[U];
     bool in[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
         const int k = k_lo + lane * 8 + 512 * u;
         in[u] = k < k_hi;
-        at[u] = min(k, p.K - 8);
+        at[u] = min(k, t.K - 8);
     }
     u32x4 wr[2][U];
     f32x4 a[MR][U][2], g[KIND == GEMV_GLU ? MR : 1][U][2];
@@ -74,7 +85,7 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (in[u]) ss = fmaf(y[u][i][e], y[u][i][e], ss);
-        const float r = 1.0f / sqrtf(wave_allsum(ss) / (float)p.K + pre.eps);
+        const float r = 1.0f / sqrtf(wave_allsum(ss) / (float)t.K + pre.eps);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -86,7 +97,7 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
                 }
                 if (n0 == 0 && in[u]) *reinterpret_cast<f32x4*>(pre.x_out + at[u] + 4 * i) = a[0][u][i];
             }
-        const float r2 = 1.0f / sqrtf(wave_allsum(s2) / (float)p.K + pre.eps);
+        const float r2 = 1.0f / sqrtf(wave_allsum(s2) / (float)t.K + pre.eps);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -94,22 +105,25 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
 #pragma unroll
                 for (int e = 0; e < 4; ++e) a[0][u][i][e] = a[0][u][i][e] * r2 * (1.0f + vn[u][i][e]);
     } else {
-        const float* A = p.A + (long long)z * p.a_zoff;
+        const float* A = t.A + (long long)z * t.a_zoff;
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-            const int rid = p.z_group ? z * p.M + m : m;
-            const float* row = A + (long long)((p.a_rows ? p.a_rows[rid] : rid) / p.a_div) * p.lda;
+            const int rid = INDIRECT && p.z_group ? z * p.M + m : m;
+            const float* row = A + (long long)(INDIRECT ? (p.a_rows ? p.a_rows[rid] : rid) / p.a_div : rid) * t.lda;
 #pragma unroll
             for (int u = 0; u < U; ++u)
 #pragma unroll
                 for (int i = 0; i < 2; ++i) {
                     a[m][u][i] = *reinterpret_cast<const f32x4*>(row + at[u] + 4 * i);
-                    if constexpr (KIND == GEMV_GLU) g[m][u][i] = *reinterpret_cast<const f32x4*>(row + p.a_glu + at[u] + 4 * i);
+                    if constexpr (KIND == GEMV_GLU) g[m][u][i] = *reinterpret_cast<const f32x4*>(row + t.a_glu + at[u] + 4 * i);
                 }
             asc[m] = KIND == GEMV_GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
             agate[m] = KIND == GEMV_GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-row[p.glu_gate_col])) : 1.0f;
         }
     }
+    ZG_PIN(p.C);
+    ZG_PIN(p.bias);
+    ZG_PIN(p.act);
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     const u32x4 none = {0u, 0u, 0u, 0u};
     float sum[MR][NS];
@@ -164,7 +178,7 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
     float* C = p.C + (long long)z * p.c_zoff;
     if constexpr (!SPLIT) {
         static_assert(KIND != GEMV_POLY, "the polynomial's rows are long");
-        if (lane < 2 && n0 + lane < p.N) {
+        if (lane < 2 && n0 + lane < t.N) {
 #pragma unroll
             for (int m = 0; m < MR; ++m) C[(long long)m * p.ldc + n0 + lane] = finish(lane ? sum[m][1] : sum[m][0], n0 + lane, p);
         }
@@ -177,11 +191,11 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
         }
         __syncthreads();
         const int m = threadIdx.x >> 1, c = threadIdx.x & 1;
-        if (m < MR && n0 + c < p.N) {
+        if (m < MR && n0 + c < t.N) {
             auto sum4 = [&](int i) { return (s_part[0][m][i] + s_part[1][m][i]) + (s_part[2][m][i] + s_part[3][m][i]); };
             float v;
             if constexpr (KIND == GEMV_POLY) {
-                const float K = (float)p.K, eps = p.poly_eps, *d = p.a_poly;
+                const float K = (float)t.K, eps = p.poly_eps, *d = p.a_poly;
                 v = (d[0] / sqrtf(sum4(0) / K + eps) * sum4(3 + 4 * c) + d[1] / sqrtf(sum4(1) / K + eps) * sum4(4 + 4 * c)) +
                     (d[2] / sqrtf(sum4(2) / K + eps) * sum4(5 + 4 * c) + d[3] * sum4(6 + 4 * c));
             } else v = sum4(c);
@@ -190,15 +204,24 @@ __device__ __forceinline__ void gemv_body(const LinArgs& p, const int z, const N
     }
 }
 
-template <int MR, int U, int KIND, bool SPLIT>
-__global__ __launch_bounds__(256) void lm_gemv_at_once_kernel(const LinArgs p, const NormIn pre) {
-    gemv_body<MR, U, KIND, SPLIT>(p, blockIdx.z, pre);
+template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT>
+__global__ __launch_bounds__(256) void lm_gemv_at_once_kernel(const float* A, const bf16_t* B, int K, int N, int ldb, int lda, int a_zoff, int b_zoff, int a_glu,
+                                                              const LinArgs p) {
+    gemv_body<MR, U, KIND, SPLIT, INDIRECT>(GemvAt{A, B, K, N, ldb, lda, a_zoff, b_zoff, a_glu}, p, blockIdx.z, NormIn());
+}
+template <int U>
+__global__ __launch_bounds__(256) void lm_gemv_normed_kernel(const float* x, const float* y, const float* wb, const float* wn, const bf16_t* B, int K, int N, int ldb,
+                                                             float eps, float* x_out, const LinArgs p) {
+    gemv_body<1, U, GEMV_NORM, false, false>(GemvAt{nullptr, B, K, N, ldb, 0, 0, 0, 0}, p, 0, NormIn{x, y, wb, wn, x_out, eps});
 }
 // batches [0, za) are product a's, the rest product b's
 template <int U, int KIND>
 __global__ __launch_bounds__(256) void lm_gemv_at_once_pair_kernel(const LinArgs a, const LinArgs b, int za) {
-    if ((int)blockIdx.z < za) gemv_body<1, U, KIND, false>(a, blockIdx.z, NormIn());
-    else gemv_body<1, U, KIND, false>(b, blockIdx.z - za, NormIn());
+    auto one = [](const LinArgs& p, int z) {
+        gemv_body<1, U, KIND, false, true>(GemvAt{p.A, p.B, p.K, p.N, p.ldb, p.lda, (int)p.a_zoff, (int)p.b_zoff, p.a_glu}, p, z, NormIn());
+    };
+    if ((int)blockIdx.z < za) one(a, blockIdx.z);
+    else one(b, blockIdx.z - za);
 }
 
 constexpr int kLongRow = 1536;  // from here on K is split over the waves
@@ -206,7 +229,7 @@ constexpr int kLongRow = 1536;  // from here on K is split over the waves
 int kind_of(const Linear& L) { return L.a_poly ? GEMV_POLY : L.a_glu > 0 ? GEMV_GLU : GEMV_PLAIN; }
 bool pieces_ok(const Linear& L, const LinArgs& p) {
     return L.M >= 1 && L.M <= 2 && !L.grp_off && !L.C16 && !L.glu_out && L.N > 0 && L.nz >= 1 && L.nz <= 65535 && L.K >= 8 && L.K % 8 == 0 && L.A && L.B && L.C &&
-           p.a_vec && p.b_vec && L.a_glu % 4 == 0 && L.a_div >= 1;
+           p.a_vec && p.b_vec && L.a_glu % 4 == 0 && L.a_div >= 1 && L.a_zoff <= 0x7fffffff && L.b_zoff <= 0x7fffffff;
 }
 
 }  // namespace
@@ -226,8 +249,14 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     if (pieces > (norm ? 2 : 3)) return ZG_OK;
     const int rows = split ? 2 : 8;
     const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, 1, A.nz + (B ? B->nz : 0));
-    const NormIn none{}, &pre = norm ? *norm : none;
-#define ZG_GV(MR, U, KIND, SPLIT) (lm_gemv_at_once_kernel<MR, U, KIND, SPLIT><<<grid, 256, 0, s>>>(a, pre))
+    const bool indirect = A.z_group || A.a_rows || A.a_div != 1;
+#define ZG_GV(MR, U, KIND, SPLIT)                                                                                                                   \
+    do {                                                                                                                                            \
+        if (indirect) ZG_GV_I(MR, U, KIND, SPLIT, true);                                                                                            \
+        else ZG_GV_I(MR, U, KIND, SPLIT, false);                                                                                                    \
+    } while (0)
+#define ZG_GV_I(MR, U, KIND, SPLIT, IND)                                                                                                            \
+    lm_gemv_at_once_kernel<MR, U, KIND, SPLIT, IND><<<grid, 256, 0, s>>>(a.A, a.B, a.K, a.N, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_glu, a)
 #define ZG_GV_P(KIND)                                                                              \
     do {                                                                                           \
         if (pieces == 1) lm_gemv_at_once_pair_kernel<1, KIND><<<grid, 256, 0, s>>>(a, b, A.nz);      \
@@ -248,14 +277,15 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     if (B && kind == GEMV_GLU) ZG_GV_P(GEMV_GLU);
     else if (B) ZG_GV_P(GEMV_PLAIN);
     else if (norm) {
-        if (pieces == 1) ZG_GV(1, 1, GEMV_NORM, false);
-        else ZG_GV(1, 2, GEMV_NORM, false);
+        if (pieces == 1) lm_gemv_normed_kernel<1><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
+        else lm_gemv_normed_kernel<2><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
     } else if (kind == GEMV_POLY) ZG_GV_M(GEMV_POLY, true);
     else if (kind == GEMV_GLU && split) ZG_GV_M(GEMV_GLU, true);
     else if (kind == GEMV_GLU) ZG_GV_M(GEMV_GLU, false);
     else if (split) ZG_GV_M(GEMV_PLAIN, true);
     else ZG_GV_M(GEMV_PLAIN, false);
 #undef ZG_GV
+#undef ZG_GV_I
 #undef ZG_GV_P
 #undef ZG_GV_U
 #undef ZG_GV_M

@@ -39,9 +39,11 @@ __device__ __forceinline__ float block_allsum(float v, float* s_red) {
 // of their own).  PRE_RMS: the same for norms by the root mean square, rows of up to 1024 values; each wave's first router row is on its
 // way while the row is normed (8 rows of 768, 8 experts: 6.6 us; 5.4 and 3.9 for the norm's launch in front).
 enum { PRE_NONE, PRE_TANH, PRE_RMS };
+// (In front what the loads of the norms need: the leading arguments are in registers when a wave starts.)
 template <int PRE>
-__global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int W, const bf16_t* router, const float* correction, int E, int top,
-                                                    int* pick, float* weight, int rule, int groups, int keep, float out_scale, const RoutePre pre) {
+__global__ __launch_bounds__(1024) void route_kernel(const float* ya, const float* xa, const float* nb, const float* nn, const bf16_t* router, int W, int E, float eps,
+                                                    int T, const float* g, const float* correction, int top, int* pick, float* weight, int rule, int groups, int keep,
+                                                    float out_scale, const RoutePre pre) {
     const bool top_logits = rule == 1 || rule == 2;  // rules that choose by the logits themselves
     const bool sigmoid_w = rule == 2;   // ... and weigh a chosen expert by sigmoid(z), nothing renormalised
     extern __shared__ __attribute__((aligned(16))) float s_row[];  // [W] with pre
@@ -52,15 +54,15 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
     u32x4 w_first[2];  // (PRE_RMS) the wave's first router row
     if constexpr (PRE == PRE_RMS) {
         __shared__ float s_sum[2][16];
-        const int T = blockDim.x, waves = T >> 6;
+        const int waves = T >> 6;
         float y[4], x[4], b[4], n[4], ss = 0.0f, s2 = 0.0f;
 #pragma unroll
         for (int j = 0; j < 4; ++j) {  // (at least 256 threads)
             const int i = min((int)threadIdx.x + T * j, W - 1);
-            y[j] = pre.y.a[(size_t)m * W + i];
-            x[j] = pre.x[(size_t)m * W + i];
-            b[j] = pre.nb[i];
-            n[j] = pre.nn[i];
+            y[j] = ya[(size_t)m * W + i];
+            x[j] = xa[(size_t)m * W + i];
+            b[j] = nb[i];
+            n[j] = nn[i];
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) w_first[u] = *reinterpret_cast<const u32x4*>(router + (size_t)min(wave, E - 1) * W + min(lane * 8 + 512 * u, W - 8));
@@ -72,7 +74,7 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
         __syncthreads();
         ss = 0.0f;
         for (int k = 0; k < waves; ++k) ss += s_sum[0][k];
-        const float r = 1.0f / sqrtf(ss / (float)W + pre.eps);
+        const float r = 1.0f / sqrtf(ss / (float)W + eps);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             x[j] += y[j] * r * (1.0f + b[j]);
@@ -83,7 +85,7 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
         __syncthreads();
         s2 = 0.0f;
         for (int k = 0; k < waves; ++k) s2 += s_sum[1][k];
-        const float r2 = 1.0f / sqrtf(s2 / (float)W + pre.eps);
+        const float r2 = 1.0f / sqrtf(s2 / (float)W + eps);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int i = threadIdx.x + T * j;
@@ -117,7 +119,7 @@ __global__ __launch_bounds__(1024) void route_kernel(const float* g, int M, int 
         row = s_row;
     }
     const bool vec = (W % 8 == 0) && (PRE != PRE_NONE || (reinterpret_cast<uintptr_t>(g) & 15) == 0) && ((reinterpret_cast<uintptr_t>(router) & 15) == 0);
-    for (int e = wave; e < E; e += (int)(blockDim.x >> 6)) {
+    for (int e = wave; e < E; e += T >> 6) {
         const bf16_t* wr = router + (size_t)e * W;
         float a = 0.0f;
         if constexpr (PRE == PRE_RMS) {
@@ -450,7 +452,9 @@ int launch_route(const float* g, int M, int W, const bf16_t* router, const float
     const int waves = M > kGemvMaxRows ? 4 : std::max(4, std::min(16, E));
     const size_t lds = pre ? (size_t)W * sizeof(float) : 0;
     const RoutePre p = pre ? *pre : RoutePre();
-#define ZG_ROUTE(PRE) route_kernel<PRE><<<M, 64 * waves, lds, s>>>(g, M, W, router, correction, E, top, pick, weight, rule, groups, keep, out_scale, p)
+#define ZG_ROUTE(PRE)                                                                                                                                       \
+    route_kernel<PRE><<<M, 64 * waves, lds, s>>>(p.y.a, p.x, p.nb, p.nn, router, W, E, p.eps, 64 * waves, g, correction, top, pick, weight, rule, groups, keep, \
+                                                 out_scale, p)
     if (!pre) ZG_ROUTE(PRE_NONE);
     else if (pre->rms) ZG_ROUTE(PRE_RMS);
     else ZG_ROUTE(PRE_TANH);

@@ -21,12 +21,14 @@ namespace {
 enum { FROM_NOTHING, FROM_ROW, FROM_EXPERTS };
 enum { TO_NOTHING, TO_NORM, TO_SHIFT };
 
+// (In front of p what the first loads need: the leading arguments are in registers when a wave starts, the others a cold round trip away.
+// from: p.y or p.yexp; shape: rows | waves of a workgroup << 28.)
 template <int NV, int FROM, int TO>
-__global__ __launch_bounds__(256) void norm_rows_kernel(const NormRows p) {
-    const int lane = threadIdx.x & 63;
-    const int first = __builtin_amdgcn_readfirstlane((blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6)) * p.run);
-    if (first >= p.M) return;
-    const int W = p.W;
+__global__ __launch_bounds__(256) void norm_rows_kernel(const float* x_in, const float* from, const float* p_wb, const float* p_wn, const float* p_mu, int W, unsigned shape,
+                                                        int run, int top, const NormRows p) {
+    const int lane = threadIdx.x & 63, M = shape & 0x0fffffff;
+    const int first = __builtin_amdgcn_readfirstlane((blockIdx.x * (shape >> 28) + (threadIdx.x >> 6)) * run);
+    if (first >= M) return;
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     int at[NV];
     bool in[NV];
@@ -50,29 +52,29 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const NormRows p) {
         return 1.0f / sqrtf(wave_allsum(ss) / (float)W + p.eps);
     };
     f32x4 wb[NV], wn[NV], mu[NV];
-    if constexpr (FROM != FROM_NOTHING) load(p.wb, wb);
-    if constexpr (TO != TO_NOTHING) load(p.wn, wn);
-    if constexpr (TO == TO_SHIFT) load(p.mu, mu);
+    if constexpr (FROM != FROM_NOTHING) load(p_wb, wb);
+    if constexpr (TO != TO_NOTHING) load(p_wn, wn);
+    if constexpr (TO == TO_SHIFT) load(p_mu, mu);
     // row m of the stream with the sublayer's output added
     auto sum = [&](int m, f32x4 (&x)[NV]) {
-        load(p.x + (size_t)m * W, x);
+        load(x_in + (size_t)m * W, x);
         if constexpr (FROM == FROM_NOTHING) return;
         f32x4 y[NV];
-        if constexpr (FROM == FROM_ROW) load(p.y + (size_t)m * W, y);
+        if constexpr (FROM == FROM_ROW) load(from + (size_t)m * W, y);
         else {
 #pragma unroll
             for (int j = 0; j < NV; ++j) y[j] = zero;
-            for (int k = 0; k < p.top; k += 2) {
-                const size_t a = (size_t)m * p.top + k, b = a + (k + 1 < p.top ? 1 : 0);
+            for (int k = 0; k < top; k += 2) {
+                const size_t a = (size_t)m * top + k, b = a + (k + 1 < top ? 1 : 0);
                 const float fa = p.weight[a], fb = p.weight[b];
                 f32x4 u[NV], v[NV];
-                load(p.yexp + (size_t)(p.inv ? p.inv[a] : (int)a) * W, u);
-                load(p.yexp + (size_t)(p.inv ? p.inv[b] : (int)b) * W, v);
+                load(from + (size_t)(p.inv ? p.inv[a] : (int)a) * W, u);
+                load(from + (size_t)(p.inv ? p.inv[b] : (int)b) * W, v);
 #pragma unroll
                 for (int j = 0; j < NV; ++j)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) y[j][e] = fmaf(fa, u[j][e], y[j][e]);
-                if (k + 1 < p.top) {
+                if (k + 1 < top) {
 #pragma unroll
                     for (int j = 0; j < NV; ++j)
 #pragma unroll
@@ -101,7 +103,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const NormRows p) {
             norm(x, before);
         }
     }
-    for (int m = first; m < min(first + p.run, p.M); ++m) {
+    for (int m = first; m < min(first + run, M); ++m) {
         if constexpr (TO == TO_SHIFT) {
             if (!p.row_prev || p.row_prev[m] < 0) load(p.shift_state + (size_t)p.row_slot[m] * p.slot_stride, before);
         }
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const NormRows p) {
 int launch_norm_rows(const NormRows& in, hipStream_t s, bool* taken) {
     *taken = false;
     NormRows p = in;
-    if (p.M <= 0 || p.W < 4 || p.W > 1024 || p.W % 4 != 0) return ZG_OK;
+    if (p.M <= 0 || p.M >= (1 << 28) || p.W < 4 || p.W > 1024 || p.W % 4 != 0) return ZG_OK;
     const uintptr_t all = reinterpret_cast<uintptr_t>(p.x) | reinterpret_cast<uintptr_t>(p.x_out) | reinterpret_cast<uintptr_t>(p.y) | reinterpret_cast<uintptr_t>(p.yexp) |
                           reinterpret_cast<uintptr_t>(p.wb) | reinterpret_cast<uintptr_t>(p.wn) | reinterpret_cast<uintptr_t>(p.mu) | reinterpret_cast<uintptr_t>(p.out) |
                           reinterpret_cast<uintptr_t>(p.out16) | reinterpret_cast<uintptr_t>(p.shift_state) | reinterpret_cast<uintptr_t>(p.last_out);
@@ -155,7 +157,7 @@ int launch_norm_rows(const NormRows& in, hipStream_t s, bool* taken) {
     if (const char* e = getenv("ZGPT2_LM_NORM_RUN")) p.run = std::max(1, atoi(e));  // (test hook: runs in short portions)
     const int waves = (p.M + p.run - 1) / p.run, per_group = p.M <= 64 ? 1 : 4;
     const dim3 grid((waves + per_group - 1) / per_group), block(64 * per_group);
-#define ZG_NR(NV, FROM, TO) (norm_rows_kernel<NV, FROM, TO><<<grid, block, 0, s>>>(p))
+#define ZG_NR(NV, FROM, TO) (norm_rows_kernel<NV, FROM, TO><<<grid, block, 0, s>>>(p.x, p.yexp ? p.yexp : p.y, p.wb, p.wn, p.mu, p.W, (unsigned)p.M | (unsigned)per_group << 28, p.run, p.top, p))
 #define ZG_NR_V(FROM, TO)                       \
     do {                                        \
         if (p.W <= 256) ZG_NR(1, FROM, TO);     \

@@ -35,36 +35,46 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int n) {  // positi
 }
 
 enum { ROWS_PLAIN, ROWS_GLU_ON_LOAD, ROWS_GLU_OUT };
-template <int TURNS, int KIND>  // TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight
-__device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (*part)[16][17]) {
-    constexpr bool GLU = KIND == ROWS_GLU_ON_LOAD, OUT = KIND == ROWS_GLU_OUT;
+// What the loads at entry need (leading arguments, see lm_gemv.hip).
+struct RowsAt {
+    const float* A;
+    const bf16_t* B;
+    const int* z_group;
+    int K, N, M, ldb, lda, a_zoff, b_zoff, a_div;
+};
+enum { FORM_PLAIN, FORM_LIST, FORM_ANY };  // rows and matrices in a row; a matrix per list entry; either, and rows through an array
+// TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight
+template <int TURNS, int KIND, int FORM>
+__device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, const int z, float (*part)[16][17]) {
+    constexpr bool GLU = KIND == ROWS_GLU_ON_LOAD, OUT = KIND == ROWS_GLU_OUT, ARRAY = FORM == FORM_ANY;
+    const bool list = FORM == FORM_LIST || (FORM == FORM_ANY && t.z_group != nullptr);
     // (gated products: eight gates and the eight values they gate)
     constexpr int half = OUT ? 8 : 16;
-    const int n0 = blockIdx.x * half, n_out = OUT ? p.glu_out : p.N;
+    const int n0 = blockIdx.x * half, n_out = OUT ? t.N / 2 : t.N;
     if (n0 >= n_out) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4, m = col & 7;
     unsigned long long left = 0;  // assignments of this expert that are still to do
-    if (p.z_group) {
-        left = __ballot(lane < p.M && p.z_group[min(lane, p.M - 1)] == z);
+    if (list) {
+        left = __ballot(lane < t.M && t.z_group[min(lane, t.M - 1)] == z);
         if (left == 0) return;
     }
-    const int w_row = OUT ? (col & 8 ? p.glu_out : 0) + min(n0 + (col & 7), p.glu_out - 1) : min(n0 + col, p.N - 1);
-    const bf16_t* w = p.B + (long long)z * p.b_zoff + (long long)w_row * p.ldb;
+    const int w_row = OUT ? (col & 8 ? n_out : 0) + min(n0 + (col & 7), n_out - 1) : min(n0 + col, t.N - 1);
+    const bf16_t* w = t.B + (long long)z * t.b_zoff + (long long)w_row * t.ldb;
     do {
-        const int n_rows = p.z_group ? min(8, __popcll(left)) : p.M;
+        const int n_rows = list ? min(8, __popcll(left)) : t.M;
         // (columns without a row compute on the last one's and are not stored)
-        const int rid = p.z_group ? nth_bit(left, min(m, n_rows - 1)) : min(m, n_rows - 1);
-        const float* a = p.A + (long long)(p.z_group ? rid : z) * p.a_zoff + (long long)((p.a_rows ? p.a_rows[rid] : rid) / p.a_div) * p.lda;
+        const int rid = list ? nth_bit(left, min(m, n_rows - 1)) : min(m, n_rows - 1);
+        const float* a = t.A + (long long)(list ? rid : z) * t.a_zoff + (long long)(FORM == FORM_PLAIN ? rid : (ARRAY && p.a_rows ? p.a_rows[rid] : rid) / t.a_div) * t.lda;
         const float asc = GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
         const float agate = GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-a[p.glu_gate_col])) : 1.0f;
-        const int n_turns = (p.K + kTurn - 1) / kTurn;
+        const int n_turns = (t.K + kTurn - 1) / kTurn;
         constexpr int RING = TURNS > 0 ? TURNS : 4;
         u32x4 wr[RING][2];
         f32x4 ar[RING][4], ur[GLU ? RING : 1][4];
         auto fetch = [&](int slot, int turn) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
-                const int k = min(turn * kTurn + 16 * kg + 8 * j, p.K - 8);
+                const int k = min(turn * kTurn + 16 * kg + 8 * j, t.K - 8);
                 wr[slot][j] = *reinterpret_cast<const u32x4*>(w + k);
                 ar[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + k);
                 ar[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + k + 4);
@@ -87,7 +97,7 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
                         y[u] = glu_on_load(y[u], ur[slot][2 * j + 1][u], p, asc) * agate;
                     }
                 }
-                if (turn * kTurn + kTurn > p.K && turn * kTurn + 16 * kg + 8 * j >= p.K) {  // columns beyond K: the clamped load brought earlier ones
+                if (turn * kTurn + kTurn > t.K && turn * kTurn + 16 * kg + 8 * j >= t.K) {  // columns beyond K: the clamped load brought earlier ones
                     x = y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     wv = u32x4{0u, 0u, 0u, 0u};
                 }
@@ -106,11 +116,11 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
         } else {
 #pragma unroll
             for (int i = 0; i < RING; ++i) fetch(i, wave + 4 * i);
-            for (int t = wave; t < n_turns; t += 4 * RING) {
+            for (int turn = wave; turn < n_turns; turn += 4 * RING) {
 #pragma unroll
                 for (int i = 0; i < RING; ++i) {
-                    multiply(i, t + 4 * i);
-                    fetch(i, t + 4 * (i + RING));
+                    multiply(i, turn + 4 * i);
+                    fetch(i, turn + 4 * (i + RING));
                 }
             }
         }
@@ -127,10 +137,10 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
                 return fabsf(hi) <= 3.4028235e38f ? hi + mid : hi;
             };
             const float v = sum(row);
-            float* C = p.C + (p.z_group ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
+            float* C = p.C + (list ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
             C[n0 + row] = OUT ? glu_on_load(v, sum(row + 8), p, 1.0f) : finish(v, n0 + row, p);
         }
-        if (!p.z_group) return;
+        if (!list) return;
         for (int i = 0; i < 8 && left; ++i) left &= left - 1;
         if (left) __syncthreads();
     } while (left);
@@ -140,8 +150,23 @@ __device__ __forceinline__ void rows_body(const LinArgs& p, const int z, float (
 template <int TURNS, int KIND>
 __global__ __launch_bounds__(256) void lm_rows_kernel(const LinArgs a, const LinArgs b, int za) {
     __shared__ float part[4][16][17];
-    if ((int)blockIdx.z < za) rows_body<TURNS, KIND>(a, blockIdx.z, part);
-    else rows_body<TURNS, KIND>(b, blockIdx.z - za, part);
+    auto one = [&](const LinArgs& p, int z) {
+        rows_body<TURNS, KIND, FORM_ANY>(RowsAt{p.A, p.B, p.z_group, p.K, p.N, p.M, p.ldb, p.lda, (int)p.a_zoff, (int)p.b_zoff, p.a_div}, p, z, part);
+    };
+    if ((int)blockIdx.z < za) one(a, blockIdx.z);
+    else one(b, blockIdx.z - za);
+}
+// one product, rows in their order
+template <int TURNS, int KIND>
+__global__ __launch_bounds__(256) void lm_rows_one_kernel(const float* A, const bf16_t* B, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff, const LinArgs p) {
+    __shared__ float part[4][16][17];
+    rows_body<TURNS, KIND, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, a_zoff, b_zoff, 1}, p, blockIdx.z, part);
+}
+template <int TURNS, int KIND>
+__global__ __launch_bounds__(256) void lm_rows_list_kernel(const float* A, const bf16_t* B, const int* z_group, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff,
+                                                           int a_div, const LinArgs p) {
+    __shared__ float part[4][16][17];
+    rows_body<TURNS, KIND, FORM_LIST>(RowsAt{A, B, z_group, K, N, M, ldb, lda, a_zoff, b_zoff, a_div}, p, blockIdx.z, part);
 }
 
 // a product in the form the kernel takes: plain rows, or a list of one-row batches with the matrix chosen by a list (M: its length);
@@ -150,6 +175,7 @@ bool rows_form(const Linear& L, LinArgs& p, int& nz) {
     if (L.grp_off || L.a_poly || L.C16 || L.K < 8 || L.N <= 0 || !L.A || !L.B || !L.C || L.a_div < 1) return false;
     p = make_args(L);
     nz = L.nz;
+    if (L.a_zoff > 0x7fffffff || L.b_zoff > 0x7fffffff) return false;
     if (L.z_group) {
         if (L.M != 1 || L.nz > 64 || L.n_groups <= 0 || L.n_groups > 65535) return false;
         p.M = L.nz;
@@ -187,9 +213,17 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     auto tiles = [](const LinArgs& p) { return p.glu_out ? (p.glu_out + 7) / 8 : (p.N + 15) / 16; };
     const dim3 grid(std::max(tiles(a), tiles(b)), 1, za + zb);
     const int per_wave = (turns + 3) / 4;
-#define ZG_ROWS(T)                                                                   \
+    const bool one = !B && !a.a_rows && a.a_glu == 0 && (a.z_group || a.a_div == 1);
+#define ZG_ROWS_ONE(T, KIND)                                                                                                                            \
+    do {                                                                                                                                                \
+        if (a.z_group) lm_rows_list_kernel<T, KIND><<<grid, 256, 0, s>>>(a.A, a.B, a.z_group, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_div, a); \
+        else lm_rows_one_kernel<T, KIND><<<grid, 256, 0, s>>>(a.A, a.B, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a);                  \
+    } while (0)
+#define ZG_ROWS(T)                                                                                \
     do {                                                                                          \
-        if (a.a_glu > 0) lm_rows_kernel<T, ROWS_GLU_ON_LOAD><<<grid, 256, 0, s>>>(a, b, za);      \
+        if (one && a.glu_out > 0) ZG_ROWS_ONE(T, ROWS_GLU_OUT);                                   \
+        else if (one) ZG_ROWS_ONE(T, ROWS_PLAIN);                                                 \
+        else if (a.a_glu > 0) lm_rows_kernel<T, ROWS_GLU_ON_LOAD><<<grid, 256, 0, s>>>(a, b, za);      \
         else if (a.glu_out > 0) lm_rows_kernel<T, ROWS_GLU_OUT><<<grid, 256, 0, s>>>(a, b, za);   \
         else lm_rows_kernel<T, ROWS_PLAIN><<<grid, 256, 0, s>>>(a, b, za);                        \
     } while (0)
@@ -199,6 +233,7 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     else if (per_wave == 4) ZG_ROWS(4);
     else ZG_ROWS(0);
 #undef ZG_ROWS
+#undef ZG_ROWS_ONE
     note_kernel("lm_rows_kernel<%d>", per_wave <= 4 ? per_wave : 0);
     ZG_HIP(hipGetLastError());
     *taken = true;

@@ -348,9 +348,8 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
 // 8.0 for the token-by-token scan's kernel and 4.0 for the norm's launch behind it.
 constexpr int kStepRows = 8;  // rows of the state in flight per thread
 template <int CW>
-__global__ __launch_bounds__(512) void gated_step_kernel(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride,
-                                                         const int* ent_start, const int* ent_slot, int H, int D, int V, const float* bias, const float* low,
-                                                         const float* w, float eps) {
+__global__ __launch_bounds__(512) void gated_step_kernel(const float* proj, float* state, size_t slot_stride, const int* ent_start, const int* ent_slot, int ld, int H,
+                                                         int D, int V, const float* bias, const float* low, float* out, int ldo, const float* w, float eps) {
     constexpr int GROUPS = 512 / CW;
     __shared__ float s_q[256], s_f[256], s_red[8];
     __shared__ __attribute__((aligned(16))) float s_o[GROUPS][CW * 4 + 4];
@@ -366,10 +365,11 @@ __global__ __launch_bounds__(512) void gated_step_kernel(const float* proj, int 
     f32x4 v;
 #pragma unroll
     for (int i = 0; i < 4; ++i) v[i] = row[2 * HD + h * V + col + i];
+    const int gi = h * D + min(tid, D - 1);
+    const float gq = row[gi], gf = row[HD + gi], gl = low[gi], gb = bias[gi], gw = w[min(tid, V - 1)];
     if (tid < D) {
-        const float z = row[h * D + tid], l = low[h * D + tid];
-        s_q[tid] = z / (1.0f + expf(-z));
-        s_f[tid] = l + (1.0f - l) / (1.0f + expf(-(row[HD + h * D + tid] + bias[h * D + tid])));
+        s_q[tid] = gq / (1.0f + expf(-gq));
+        s_f[tid] = gl + (1.0f - gl) / (1.0f + expf(-(gf + gb)));
     }
     __syncthreads();
     f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -404,7 +404,7 @@ __global__ __launch_bounds__(512) void gated_step_kernel(const float* proj, int 
     __syncthreads();
     if (tid < V) {
         const float rms = ((s_red[0] + s_red[1]) + (s_red[2] + s_red[3])) + ((s_red[4] + s_red[5]) + (s_red[6] + s_red[7]));
-        out[m * ldo + h * V + tid] = a * (1.0f / sqrtf(rms / (float)V + eps)) * w[tid];
+        out[m * ldo + h * V + tid] = a * (1.0f / sqrtf(rms / (float)V + eps)) * gw;
     }
 }
 
@@ -416,7 +416,7 @@ int launch_gated_step(const float* proj, int ld, float* out, int ldo, float* sta
     if (n_entries <= 0 || D > 256 || V < 4 || V > 256 || V % 4 != 0 || slot_stride % 4 != 0 || (reinterpret_cast<uintptr_t>(state) & 15) != 0 || H > 65535)
         return ZG_OK;
     const dim3 grid(n_entries, H);
-#define ZG_GSTEP(CW) gated_step_kernel<CW><<<grid, 512, 0, s>>>(proj, ld, out, ldo, state, slot_stride, ent_start, ent_slot, H, D, V, bias, low, w, eps)
+#define ZG_GSTEP(CW) gated_step_kernel<CW><<<grid, 512, 0, s>>>(proj, state, slot_stride, ent_start, ent_slot, ld, H, D, V, bias, low, out, ldo, w, eps)
     if (V <= 32) ZG_GSTEP(8);
     else if (V <= 64) ZG_GSTEP(16);
     else if (V <= 128) ZG_GSTEP(32);
