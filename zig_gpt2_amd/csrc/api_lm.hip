@@ -1352,37 +1352,60 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             bf16_t* const o16 = ctx16 && whole(HV) ? g->o16 : nullptr;
             const float* q = direct ? g->proj : g->q;
             const int ldq = direct ? LD : H * (D + R);
-            if (direct) {
-                ZG_TRY(launch_latent_direct_prep(g->proj, LD, M, H, D, R, KR, H * (D + R), L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages,
-                                                 g->P, g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, qa16));
-            } else {
-                ZG_TRY(launch_latent_prep(g->proj, LD, M, QR, KR, R, L.dq_norm, L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages, g->P,
-                                          g->cq, ps.cache, s, cq16));
-                lin = Linear();
-                lin.A = cq16 ? nullptr : g->cq; lin.A16 = cq16; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
+            // decode steps: from the projected queries to the values in two launches, with the queries' own norm inside the product in front
+            bool stepped = false;
+            LatentStep st;
+            st.q = q; st.ldq = ldq; st.ukT = L.ukT; st.uv = L.uv; st.M = M; st.H = H; st.D = D; st.R = R; st.KR = KR; st.Vd = Vd; st.scale = d.scale; st.eps = eps; st.rot = rot;
+            st.row_pos = d_pos; st.row_slot = d_slot; st.page_table = g->page_table; st.max_pages = g->max_pages; st.page_tokens = g->P; st.cache = ps.cache;
+            st.ws = g->attn_ws; st.ws_floats = g->attn_ws_floats; st.gate = gate; st.ldg = LD; st.sink = L.sink; st.out = g->o; st.ldo = HV;
+            if (d.kv_from <= 0) {
+                st.lat = g->proj + (direct ? H * (D + R) : QR);
+                st.ld_lat = LD;
+                st.wkv = L.dkv_norm;
+            }
+            if (few && (single || !st.lat) && latent_step_fits(H, D, R, KR, Vd, ldq, LD)) {
+                bool queries = direct;
+                if (!direct) {
+                    lin = Linear();
+                    lin.A = g->proj; lin.lda = LD; lin.a_norm = L.dq_norm; lin.norm_eps = eps; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M;
+                    lin.N = H * (D + R); lin.K = QR;
+                    ZG_TRY(launch_linear_row_norm(lin, s, &queries));
+                }
+                if (queries) ZG_TRY(launch_latent_step(st, s, &stepped));
+            }
+            if (!stepped) {
+                if (direct) {
+                    ZG_TRY(launch_latent_direct_prep(g->proj, LD, M, H, D, R, KR, H * (D + R), L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages,
+                                                     g->P, g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, qa16));
+                } else {
+                    ZG_TRY(launch_latent_prep(g->proj, LD, M, QR, KR, R, L.dq_norm, L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages, g->P,
+                                              g->cq, ps.cache, s, cq16));
+                    lin = Linear();
+                    lin.A = cq16 ? nullptr : g->cq; lin.A16 = cq16; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
+                    ZG_TRY(launch_linear(lin, f32, s));
+                }
+                lin = Linear();  // the unrotated query part carried into the latent space, head by head
+                lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
+                lin.C = qa16 ? nullptr : g->qa; lin.C16 = qa16; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
+                ZG_TRY(launch_linear(lin, f32, s));
+                if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
+                bool tiled = false;
+                if (!f32 && !few)
+                    ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
+                                                         g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
+                                                         L.sink, qa16, ctx16));
+                if (f32 && !few)
+                    ZG_TRY(launch_latent_attention_f32(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
+                                                       g->max_pages, g->P, ps.cache, s, &tiled, gate, LD, L.sink));
+                ZG_REQUIRE(tiled || !tiles, ZG_ERR_UNSUPPORTED, "latent attention: the tiles do not fit their workspace");
+                if (!tiled)
+                    ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,
+                                                   g->attn_ws, g->attn_ws_floats, s, gate, LD, L.sink));
+                lin = Linear();  // values of the weighted latent, head by head
+                lin.A = ctx16 ? nullptr : g->ctx; lin.A16 = ctx16; lin.lda = H * KR; lin.a_zoff = KR; lin.B = L.uv; lin.ldb = KR; lin.b_zoff = (long long)Vd * KR;
+                lin.C = o16 ? nullptr : g->o; lin.C16 = o16; lin.ldc = HV; lin.c_zoff = Vd; lin.M = M; lin.N = Vd; lin.K = KR; lin.nz = H;
                 ZG_TRY(launch_linear(lin, f32, s));
             }
-            lin = Linear();  // the unrotated query part carried into the latent space, head by head
-            lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
-            lin.C = qa16 ? nullptr : g->qa; lin.C16 = qa16; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
-            ZG_TRY(launch_linear(lin, f32, s));
-            if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
-            bool tiled = false;
-            if (!f32 && !few)
-                ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
-                                                     g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
-                                                     L.sink, qa16, ctx16));
-            if (f32 && !few)
-                ZG_TRY(launch_latent_attention_f32(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
-                                                   g->max_pages, g->P, ps.cache, s, &tiled, gate, LD, L.sink));
-            ZG_REQUIRE(tiled || !tiles, ZG_ERR_UNSUPPORTED, "latent attention: the tiles do not fit their workspace");
-            if (!tiled)
-                ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,
-                                               g->attn_ws, g->attn_ws_floats, s, gate, LD, L.sink));
-            lin = Linear();  // values of the weighted latent, head by head
-            lin.A = ctx16 ? nullptr : g->ctx; lin.A16 = ctx16; lin.lda = H * KR; lin.a_zoff = KR; lin.B = L.uv; lin.ldb = KR; lin.b_zoff = (long long)Vd * KR;
-            lin.C = o16 ? nullptr : g->o; lin.C16 = o16; lin.ldc = HV; lin.c_zoff = Vd; lin.M = M; lin.N = Vd; lin.K = KR; lin.nz = H;
-            ZG_TRY(launch_linear(lin, f32, s));
             lin = Linear();
             lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             ZG_TRY(launch_linear(lin, f32, s));

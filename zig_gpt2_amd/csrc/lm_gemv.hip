@@ -18,7 +18,7 @@ namespace lm {
 
 namespace {
 
-enum { GEMV_PLAIN, GEMV_GLU, GEMV_POLY, GEMV_NORM };
+enum { GEMV_PLAIN, GEMV_GLU, GEMV_POLY, GEMV_NORM, GEMV_RMS };
 
 // sums of N values over the lanes of a wave, each in every lane
 template <int N>
@@ -35,12 +35,14 @@ struct GemvAt {
     const float* A;
     const bf16_t* B;
     int K, N, ldb, lda, a_zoff, b_zoff, a_glu;
+    const float* a_norm = nullptr;  // GEMV_RMS: the rows' norm weights
+    float eps = 0.0f;
 };
 
 // INDIRECT: rows through an array, or a matrix chosen by a list
 template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT>
 __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, const int z, const NormIn& pre) {
-    constexpr int NS = KIND == GEMV_POLY ? 11 : 2;  // sums of a row: the two products; or q1 q2 q3 and four products for each weight row
+    constexpr int NS = KIND == GEMV_POLY ? 11 : KIND == GEMV_RMS ? 3 : 2;  // sums of a row: the two products, with the norm of squares; or q1 q2 q3 and four products for each weight row
     __shared__ float s_part[SPLIT ? 4 : 1][MR][NS];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n0 = SPLIT ? blockIdx.x * 2 : blockIdx.x * 8 + wave * 2;
@@ -59,7 +61,7 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
         at[u] = min(k, t.K - 8);
     }
     u32x4 wr[2][U];
-    f32x4 a[MR][U][2], g[KIND == GEMV_GLU ? MR : 1][U][2];
+    f32x4 a[MR][U][2], g[KIND == GEMV_GLU ? MR : 1][U][2], nw[U][2];
     float asc[MR], agate[MR];
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -106,6 +108,12 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
                 for (int e = 0; e < 4; ++e) a[0][u][i][e] = a[0][u][i][e] * r2 * (1.0f + vn[u][i][e]);
     } else {
         const float* A = t.A + (long long)z * t.a_zoff;
+        if constexpr (KIND == GEMV_RMS) {
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) nw[u][i] = *reinterpret_cast<const f32x4*>(t.a_norm + at[u] + 4 * i);
+        }
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
             const int rid = INDIRECT && p.z_group ? z * p.M + m : m;
@@ -153,6 +161,13 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
                     for (int e = 0; e < 4; ++e) x[e] = glu_on_load(x[e], g[m][u][i][e], p, asc[m]) * agate[m];
                 }
                 if (!in[u]) x = zero;
+                if constexpr (KIND == GEMV_RMS) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        sum[m][2] = fmaf(x[e], x[e], sum[m][2]);
+                        x[e] *= nw[u][i][e];
+                    }
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const float w0 = wf[0][4 * i + e], w1 = wf[1][4 * i + e];
@@ -180,7 +195,11 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
         static_assert(KIND != GEMV_POLY, "the polynomial's rows are long");
         if (lane < 2 && n0 + lane < t.N) {
 #pragma unroll
-            for (int m = 0; m < MR; ++m) C[(long long)m * p.ldc + n0 + lane] = finish(lane ? sum[m][1] : sum[m][0], n0 + lane, p);
+            for (int m = 0; m < MR; ++m) {
+                float v = lane ? sum[m][1] : sum[m][0];
+                if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum[m][2] / (float)t.K + t.eps);
+                C[(long long)m * p.ldc + n0 + lane] = finish(v, n0 + lane, p);
+            }
         }
     } else {
         if (lane == 0) {
@@ -199,6 +218,7 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
                 v = (d[0] / sqrtf(sum4(0) / K + eps) * sum4(3 + 4 * c) + d[1] / sqrtf(sum4(1) / K + eps) * sum4(4 + 4 * c)) +
                     (d[2] / sqrtf(sum4(2) / K + eps) * sum4(5 + 4 * c) + d[3] * sum4(6 + 4 * c));
             } else v = sum4(c);
+            if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum4(2) / (float)t.K + t.eps);
             C[(long long)m * p.ldc + n0 + c] = finish(v, n0 + c, p);
         }
     }
@@ -213,6 +233,10 @@ template <int U>
 __global__ __launch_bounds__(256) void lm_gemv_normed_kernel(const float* x, const float* y, const float* wb, const float* wn, const bf16_t* B, int K, int N, int ldb,
                                                              float eps, float* x_out, const LinArgs p) {
     gemv_body<1, U, GEMV_NORM, false, false>(GemvAt{nullptr, B, K, N, ldb, 0, 0, 0, 0}, p, 0, NormIn{x, y, wb, wn, x_out, eps});
+}
+template <int MR, int U, bool SPLIT>
+__global__ __launch_bounds__(256) void lm_gemv_row_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int ldb, int lda, float eps, const LinArgs p) {
+    gemv_body<MR, U, GEMV_RMS, SPLIT, false>(GemvAt{A, B, K, N, ldb, lda, 0, 0, 0, a_norm, eps}, p, 0, NormIn());
 }
 // batches [0, za) are product a's, the rest product b's
 template <int U, int KIND>
@@ -238,7 +262,8 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     *taken = false;
     const LinArgs a = make_args(A), b = B ? make_args(*B) : a;
     if (!pieces_ok(A, a) || (B && (!pieces_ok(*B, b) || B->M != A.M || kind_of(*B) != kind_of(A) || A.nz + B->nz > 65535))) return ZG_OK;
-    const int kind = norm ? (int)GEMV_NORM : kind_of(A);
+    const int kind = norm ? (int)GEMV_NORM : A.a_norm ? (int)GEMV_RMS : kind_of(A);
+    if (kind == GEMV_RMS && (B || kind_of(A) != GEMV_PLAIN || A.nz != 1 || A.a_rows || A.z_group || A.a_div != 1 || (reinterpret_cast<uintptr_t>(A.a_norm) & 15) != 0)) return ZG_OK;
     const int k_min = B ? std::min(A.K, B->K) : A.K, k_max = B ? std::max(A.K, B->K) : A.K;
     // (batches of long rows fill the chip without the split)
     const bool split = k_min >= kLongRow && A.nz + (B ? B->nz : 0) <= 4;
@@ -279,6 +304,22 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     else if (norm) {
         if (pieces == 1) lm_gemv_normed_kernel<1><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
         else lm_gemv_normed_kernel<2><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
+    } else if (kind == GEMV_RMS) {
+#define ZG_GV_R(MR, U)                                                                                                                                      \
+    do {                                                                                                                                                    \
+        if (split) lm_gemv_row_norm_kernel<MR, U, true><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a);                    \
+        else lm_gemv_row_norm_kernel<MR, U, false><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a);                         \
+    } while (0)
+#define ZG_GV_RU(MR)                     \
+    do {                                 \
+        if (pieces == 1) ZG_GV_R(MR, 1); \
+        else if (pieces == 2) ZG_GV_R(MR, 2); \
+        else ZG_GV_R(MR, 3);             \
+    } while (0)
+        if (A.M == 1) ZG_GV_RU(1);
+        else ZG_GV_RU(2);
+#undef ZG_GV_R
+#undef ZG_GV_RU
     } else if (kind == GEMV_POLY) ZG_GV_M(GEMV_POLY, true);
     else if (kind == GEMV_GLU && split) ZG_GV_M(GEMV_GLU, true);
     else if (kind == GEMV_GLU) ZG_GV_M(GEMV_GLU, false);

@@ -53,6 +53,8 @@ struct Linear {
     int glu_gate_col = -1;             // >= 0: the activated row is multiplied by sigmoid(A row[glu_gate_col]) (a gate logit behind gate | up)
     const float* a_poly = nullptr;     // != null (at most kPolyMaxRows rows): A rows enter as a N(z) + b N(z^2) + c N(z^3) + e, N over the row's K values
     float poly_eps = 0.0f;
+    const float* a_norm = nullptr;     // != null (launch_linear_row_norm alone): A rows enter as x / sqrt(mean(x^2) + norm_eps) * a_norm
+    float norm_eps = 0.0f;
     int nz = 1;
     long long a_zoff = 0, b_zoff = 0, c_zoff = 0;
     const int* z_group = nullptr;  // (n_groups: how many matrices it names, 0 where that is not known)
@@ -73,6 +75,8 @@ struct NormIn {
 };
 // One row (L.A only names where the row would be); *taken = false: not a form that has it, nothing launched.
 int launch_linear_normed(const Linear& L, const NormIn& norm, hipStream_t s, bool* taken);
+// Up to kGemvMaxRows rows, each normed on its way in (L.a_norm); *taken as above.
+int launch_linear_row_norm(const Linear& L, hipStream_t s, bool* taken);
 // Picks the row-vector kernel (few rows: decode) or the tiled matrix-core kernel (prompt portions).
 int launch_linear(const Linear& L, bool f32, hipStream_t s);
 constexpr int kGemvMaxRows = 8;
@@ -304,6 +308,29 @@ int launch_latent_attention_f32(const float* qa, float* ctx, int M, int H, int K
 int launch_latent_attention(const float* qa, float* ctx, int M, int H, int KR, int R, float scale, const int* row_pos, const int* row_slot,
                             const int* page_table, int max_pages, int page_tokens, const float* cache, float* ws, size_t ws_floats, hipStream_t s,
                             const float* gate = nullptr, int ldg = 0, const float* sink = nullptr);
+
+// Decode steps, every row the only one of its sequence (or of a layer that reads another's latents), in two launches: q rows of heads
+// [D | R], unrotated; lat rows [KR | R], neither normed nor rotated, filed at the row's position (null: the layer reads another layer's
+// latents); out[m][h Vd + n] = uv[h][n] . (head h's weighted latent, times its gate).  *taken = false: not a form that has them, nothing launched.
+struct LatentStep {
+    const float* q = nullptr;
+    const bf16_t *ukT = nullptr, *uv = nullptr;  // [H][KR][D], [H][Vd][KR]
+    const float *lat = nullptr, *wkv = nullptr;
+    int ldq = 0, ld_lat = 0, M = 0, H = 0, D = 0, R = 0, KR = 0, Vd = 0;
+    float scale = 1.0f, eps = 0.0f;
+    Rotary rot{nullptr, 0, 1.0f, 0};
+    const int *row_pos = nullptr, *row_slot = nullptr, *page_table = nullptr;
+    int max_pages = 0, page_tokens = 0;
+    float* cache = nullptr;
+    float* ws = nullptr;
+    size_t ws_floats = 0;
+    const float *gate = nullptr, *sink = nullptr;
+    int ldg = 0;
+    float* out = nullptr;
+    int ldo = 0;
+};
+bool latent_step_fits(int H, int D, int R, int KR, int Vd, int ldq, int ld_lat);
+int launch_latent_step(const LatentStep& a, hipStream_t s, bool* taken);
 
 // The same for prompt portions on the matrix cores (bf16 operands, fp32 scores / softmax / accumulation): 32 queries of one entry
 // and four heads per workgroup, over the entries' cached rows laid out as bf16 tiles of 32 keys by a launch in front of it.

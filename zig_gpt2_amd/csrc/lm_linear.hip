@@ -1003,11 +1003,19 @@ int launch_linear_normed(const Linear& L, const NormIn& n, hipStream_t s, bool* 
     return launch_gemv_at_once(L, nullptr, &n, s, taken);
 }
 
+int launch_linear_row_norm(const Linear& L, hipStream_t s, bool* taken) {
+    *taken = false;
+    if (!L.a_norm || L.M <= 0 || L.M > kGemvMaxRows || L.grp_off || L.a_poly) return ZG_OK;
+    if (getenv("ZGPT2_LM_NO_ROWS") == nullptr) ZG_TRY(launch_rows(L, nullptr, s, taken));
+    return *taken ? ZG_OK : launch_gemv_at_once(L, nullptr, nullptr, s, taken);
+}
+
 int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     if (L.M <= 0 || L.N <= 0 || L.nz <= 0) return ZG_OK;
     const bool tiled = L.grp_off || L.M > kGemvMaxRows;
     ZG_REQUIRE(L.K > 0 && L.B && (tiled ? (L.A || (L.A16 && !f32)) && (L.C || L.C16) : L.A && L.C && !L.C16), ZG_ERR_ARG, "linear: empty operand");
     ZG_REQUIRE(L.a_div >= 1, ZG_ERR_ARG, "linear: a_div %d", L.a_div);
+    ZG_REQUIRE(!L.a_norm, ZG_ERR_ARG, "linear: a norm on load is launch_linear_row_norm's");
     ZG_REQUIRE(!L.a_poly || (L.M <= kPolyMaxRows && L.a_glu == 0 && !L.grp_off), ZG_ERR_ARG, "linear: the polynomial activation on load is for %d rows at most",
                kPolyMaxRows);
     const LinArgs p = make_args(L);

@@ -33,6 +33,8 @@ struct LinArgs {
     int glu_gate_col;
     const float* a_poly;
     float poly_eps;
+    const float* a_norm;
+    float norm_eps;
     const bf16_t* A16;  // the same rows as bf16 (tiled kernels), or null
     bf16_t* C16;        // the result rounded to bf16, beside or instead of C (tiled kernels), or null
     int glu_out;        // > 0: gated product (Linear::glu_out)
@@ -107,6 +109,8 @@ inline LinArgs make_args(const Linear& L) {
     p.A16 = L.A16; p.C16 = L.C16; p.glu_out = L.glu_out;
     p.a_poly = L.a_poly;
     p.poly_eps = L.poly_eps;
+    p.a_norm = L.a_norm;
+    p.norm_eps = L.norm_eps;
     p.a_vec = ((reinterpret_cast<uintptr_t>(L.A) & 15) == 0 && L.lda % 4 == 0 && L.a_zoff % 4 == 0) ? 1 : 0;
     p.b_vec = ((reinterpret_cast<uintptr_t>(L.B) & 15) == 0 && L.ldb % 8 == 0 && L.b_zoff % 8 == 0) ? 1 : 0;
     return p;

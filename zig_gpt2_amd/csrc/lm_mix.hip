@@ -6,7 +6,7 @@
 
 #include <algorithm>
 
-#include "lm_kernels.h"
+#include "lm_latent_parts.h"
 
 namespace zg {
 namespace lm {
@@ -34,7 +34,6 @@ __device__ __forceinline__ float row_inv_rms(const float* v, int n, float eps, f
 }
 
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
-__device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 
 __global__ __launch_bounds__(256) void embed_kernel(const bf16_t* table, const int* ids, float* x, float* x_copy, float scale, int W, int vocab,
                                                     int* flag, const int* row_pos, const float* pos_freq) {
@@ -57,12 +56,6 @@ __global__ __launch_bounds__(256) void embed_kernel(const bf16_t* table, const i
 // Rows of up to 256 * kRowRegs floats are held in registers between the statistics and the result: every operand is requested
 // in one go at the top of the kernel, so a one-row step (decoding) pays one memory round trip instead of one per pass.
 constexpr int kRowRegs = 16;
-
-// an output value, as it is and / or rounded to bf16 for the matrix product that reads it next
-__device__ __forceinline__ void put_row(float* out, bf16_t* out16, size_t at, float v) {
-    if (out) out[at] = v;
-    if (out16) out16[at] = (bf16_t)cvt_pk_bf16(v, v);
-}
 
 __global__ __launch_bounds__(256) void norm_shift_kernel(const float* x, const float* w, const float* mu, float eps, float* out, int W,
                                                          const int* row_prev, const int* row_slot, const float* shift_state,
@@ -768,20 +761,6 @@ __global__ __launch_bounds__(256) void linear_chunk_out_kernel(const float* __re
 }
 
 // ------------------------------------------------------------------------------------------------ latent attention
-__device__ __forceinline__ size_t cache_row(const int* page_table, int max_pages, int page_tokens, int slot, int pos) {
-    return (size_t)page_table[(size_t)slot * max_pages + pos / page_tokens] * page_tokens + pos % page_tokens;
-}
-
-// pair i of `src` (channels (2i, 2i + 1), or (i, i + dims / 2)) at position pos, rotated by pos * freq[i]; angle and product in fp32
-__device__ __forceinline__ void rotate_pair(const float* src, float* dst, int i, int pos, const Rotary& rot, bf16_t* dst16 = nullptr) {
-    const float a = (float)pos * rot.freq[i];
-    const float c = cosf(a) * rot.amp, s = sinf(a) * rot.amp;
-    const int a0 = rot.halves ? i : 2 * i, a1 = rot.halves ? i + rot.dims / 2 : 2 * i + 1;
-    const float u = src[a0], v = src[a1];
-    put_row(dst, dst16, a0, u * c - v * s);
-    put_row(dst, dst16, a1, v * c + u * s);
-}
-
 __global__ __launch_bounds__(256) void latent_prep_kernel(const float* proj, int ld, int q_rank, int KR, int R, const float* wq, const float* wkv,
                                                           float eps, Rotary rot, const int* row_pos, const int* row_slot, const int* page_table,
                                                           int max_pages, int page_tokens, float* cq, float* cache, bf16_t* cq16) {
@@ -882,17 +861,6 @@ __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* pr
 // gate (may be null): head h's result is multiplied by sigmoid(gate[m ldg + h]) where it is written.
 // 8 rows, 12 heads on latents of 256 + 32, some 300 keys: 4.6 us and 3.2 for the merge (13.4 and 4.6 with loads under their own bounds
 // checks and ranges of 64 keys and more: four dependent round trips instead of one).
-// 1 / (L + exp(sink - mx)) times what brings weights of reference point mx to that denominator's (L: sum of exp(score - mx); mx -inf:
-// no keys).  sink null: 1 / L.
-__device__ __forceinline__ float sink_norm_f(float mx, float L, const float* sink, int h) {
-    if (!sink) return 1.0f / L;
-    const float s = sink[h];
-    if (s <= mx) return 1.0f / (L + expf(s - mx));
-    const float e = expf(mx - s);
-    return e / (L * e + 1.0f);
-}
-__device__ __forceinline__ float head_gate_f(const float* gate, int ldg, size_t m, int h) { return gate ? sigmoid_f(gate[m * ldg + h]) : 1.0f; }
-
 template <int ND>
 __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, float* ctx, int H, int KR, int R, float scale, const int* row_pos,
                                                                const int* row_slot, const int* page_table, int max_pages, int page_tokens,
@@ -904,8 +872,7 @@ __global__ __launch_bounds__(256) void latent_attention_kernel(const float* qa, 
     const int DT = KR + R, n_keys = row_pos[m] + 1, slot = row_slot[m];
     int k_lo = 0, k_hi = n_keys;
     if (n_split > 1) {
-        int chunk = (n_keys + n_split - 1) / n_split;
-        chunk = (chunk + 15) & ~15;
+        const int chunk = split_chunk(n_keys, n_split);
         k_lo = min(n_keys, (int)blockIdx.z * chunk);
         k_hi = min(n_keys, k_lo + chunk);
     }
@@ -1485,8 +1452,7 @@ __global__ __launch_bounds__(256) void latent_merge_kernel(const float* ws, floa
     __shared__ float s_w[64];
     __shared__ float s_L, s_M;
     const int m = blockIdx.x, h = blockIdx.y, n_keys = row_pos[m] + 1;
-    int chunk = (n_keys + n_split - 1) / n_split;
-    chunk = (chunk + 15) & ~15;
+    const int chunk = split_chunk(n_keys, n_split);
     const int used = min(n_split, (n_keys + chunk - 1) / chunk);
     const float* part = ws + ((size_t)m * H + h) * n_split * (KR + 2);
     if (threadIdx.x < 64) {

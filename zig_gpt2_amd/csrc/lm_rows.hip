@@ -34,19 +34,21 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int n) {  // positi
     return __builtin_ctzll(m);
 }
 
-enum { ROWS_PLAIN, ROWS_GLU_ON_LOAD, ROWS_GLU_OUT };
+enum { ROWS_PLAIN, ROWS_GLU_ON_LOAD, ROWS_GLU_OUT, ROWS_RMS };
 // What the loads at entry need (leading arguments, see lm_gemv.hip).
 struct RowsAt {
     const float* A;
     const bf16_t* B;
     const int* z_group;
     int K, N, M, ldb, lda, a_zoff, b_zoff, a_div;
+    const float* a_norm = nullptr;  // ROWS_RMS: the rows' norm weights
+    float eps = 0.0f;
 };
 enum { FORM_PLAIN, FORM_LIST, FORM_ANY };  // rows and matrices in a row; a matrix per list entry; either, and rows through an array
 // TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight
 template <int TURNS, int KIND, int FORM>
 __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, const int z, float (*part)[16][17]) {
-    constexpr bool GLU = KIND == ROWS_GLU_ON_LOAD, OUT = KIND == ROWS_GLU_OUT, ARRAY = FORM == FORM_ANY;
+    constexpr bool GLU = KIND == ROWS_GLU_ON_LOAD, OUT = KIND == ROWS_GLU_OUT, RMS = KIND == ROWS_RMS, ARRAY = FORM == FORM_ANY;
     const bool list = FORM == FORM_LIST || (FORM == FORM_ANY && t.z_group != nullptr);
     // (gated products: eight gates and the eight values they gate)
     constexpr int half = OUT ? 8 : 16;
@@ -70,7 +72,8 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         const int n_turns = (t.K + kTurn - 1) / kTurn;
         constexpr int RING = TURNS > 0 ? TURNS : 4;
         u32x4 wr[RING][2];
-        f32x4 ar[RING][4], ur[GLU ? RING : 1][4];
+        f32x4 ar[RING][4], ur[GLU || RMS ? RING : 1][4];
+        float ss = 0.0f;  // (RMS) squares of the lane's share of its row
         auto fetch = [&](int slot, int turn) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
@@ -78,9 +81,10 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
                 wr[slot][j] = *reinterpret_cast<const u32x4*>(w + k);
                 ar[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + k);
                 ar[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + k + 4);
-                if constexpr (GLU) {
-                    ur[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + p.a_glu + k);
-                    ur[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + p.a_glu + k + 4);
+                if constexpr (GLU || RMS) {  // the values a gate multiplies, or the norm's weights
+                    const float* u = RMS ? t.a_norm : a + p.a_glu;
+                    ur[slot][2 * j] = *reinterpret_cast<const f32x4*>(u + k);
+                    ur[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(u + k + 4);
                 }
             }
         };
@@ -100,6 +104,14 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
                 if (turn * kTurn + kTurn > t.K && turn * kTurn + 16 * kg + 8 * j >= t.K) {  // columns beyond K: the clamped load brought earlier ones
                     x = y = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     wv = u32x4{0u, 0u, 0u, 0u};
+                }
+                if constexpr (RMS) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        ss = fmaf(x[u], x[u], fmaf(y[u], y[u], ss));
+                        x[u] *= ur[slot][2 * j][u];
+                        y[u] *= ur[slot][2 * j + 1][u];
+                    }
                 }
                 const Planes8<3> pl = to_planes<3>(x, y);
                 const u32x4 zero = {0u, 0u, 0u, 0u};
@@ -128,6 +140,10 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         // result: the other terms of what met the infinity may be zero, and zero times infinity is not
 #pragma unroll
         for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = col < 8 ? acc1[e] : acc1[e] + acc2[e];
+        __shared__ float s_ss[RMS ? 16 : 1][8];
+        if constexpr (RMS) {
+            if (col < 8) s_ss[4 * wave + kg][m] = ss;
+        }
         __syncthreads();
         const int row = threadIdx.x & 15, om = threadIdx.x >> 4;
         if (om < n_rows && row < half && n0 + row < n_out) {
@@ -136,7 +152,13 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
                 const float mid = (part[0][r][om + 8] + part[1][r][om + 8]) + (part[2][r][om + 8] + part[3][r][om + 8]);
                 return fabsf(hi) <= 3.4028235e38f ? hi + mid : hi;
             };
-            const float v = sum(row);
+            float v = sum(row);
+            if constexpr (RMS) {
+                float q = 0.0f;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) q += s_ss[i][om];
+                v *= 1.0f / sqrtf(q / (float)t.K + t.eps);
+            }
             float* C = p.C + (list ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
             C[n0 + row] = OUT ? glu_on_load(v, sum(row + 8), p, 1.0f) : finish(v, n0 + row, p);
         }
@@ -161,6 +183,11 @@ template <int TURNS, int KIND>
 __global__ __launch_bounds__(256) void lm_rows_one_kernel(const float* A, const bf16_t* B, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff, const LinArgs p) {
     __shared__ float part[4][16][17];
     rows_body<TURNS, KIND, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, a_zoff, b_zoff, 1}, p, blockIdx.z, part);
+}
+template <int TURNS>
+__global__ __launch_bounds__(256) void lm_rows_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int M, int ldb, int lda, float eps, const LinArgs p) {
+    __shared__ float part[4][16][17];
+    rows_body<TURNS, ROWS_RMS, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, 0, 0, 1, a_norm, eps}, p, blockIdx.z, part);
 }
 template <int TURNS, int KIND>
 __global__ __launch_bounds__(256) void lm_rows_list_kernel(const float* A, const bf16_t* B, const int* z_group, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff,
@@ -197,6 +224,7 @@ bool rows_form(const Linear& L, LinArgs& p, int& nz) {
     // 32 352 : 337, 48 376 : 383.
     const bool pays = L.z_group ? p.M >= 14 + L.n_groups / 8 : p.M >= (L.K <= 1024 ? 3 : 6);
     if (L.glu_out && L.a_glu) return false;
+    if (L.a_norm && (L.z_group || L.a_rows || L.a_glu || L.glu_out || nz != 1 || p.a_div != 1 || (reinterpret_cast<uintptr_t>(L.a_norm) & 15) != 0)) return false;
     return pays && (L.z_group || p.M <= 8) && p.a_vec && p.b_vec && L.K % 8 == 0 && L.a_glu % 4 == 0 && nz <= 65535;
 }
 
@@ -208,7 +236,7 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     int za = 0, zb = 0;
     if (!rows_form(A, a, za)) return ZG_OK;
     b = a;
-    if (B && (!rows_form(*B, b, zb) || za + zb > 65535 || (a.a_glu > 0) != (b.a_glu > 0) || a.glu_out || b.glu_out)) return ZG_OK;
+    if (B && (a.a_norm || B->a_norm || !rows_form(*B, b, zb) || za + zb > 65535 || (a.a_glu > 0) != (b.a_glu > 0) || a.glu_out || b.glu_out)) return ZG_OK;
     const int turns = (std::max(a.K, b.K) + kTurn - 1) / kTurn;
     auto tiles = [](const LinArgs& p) { return p.glu_out ? (p.glu_out + 7) / 8 : (p.N + 15) / 16; };
     const dim3 grid(std::max(tiles(a), tiles(b)), 1, za + zb);
@@ -221,7 +249,8 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     } while (0)
 #define ZG_ROWS(T)                                                                                \
     do {                                                                                          \
-        if (one && a.glu_out > 0) ZG_ROWS_ONE(T, ROWS_GLU_OUT);                                   \
+        if (a.a_norm) lm_rows_norm_kernel<T><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.M, a.ldb, a.lda, a.norm_eps, a); \
+        else if (one && a.glu_out > 0) ZG_ROWS_ONE(T, ROWS_GLU_OUT);                                   \
         else if (one) ZG_ROWS_ONE(T, ROWS_PLAIN);                                                 \
         else if (a.a_glu > 0) lm_rows_kernel<T, ROWS_GLU_ON_LOAD><<<grid, 256, 0, s>>>(a, b, za);      \
         else if (a.glu_out > 0) lm_rows_kernel<T, ROWS_GLU_OUT><<<grid, 256, 0, s>>>(a, b, za);   \
