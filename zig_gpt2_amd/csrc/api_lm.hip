@@ -1142,7 +1142,16 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                                              g->page_table, g->max_pages, g->P, ps.cache, key_cap, g->win_ws, g->win_ws_floats, d_estart, d_elen, n_ent,
                                              s, &done);
             };
-            if (d.sigmoid_weights && single) ZG_TRY(gated(&rot));  // decode steps: the rows' preparation inside the attention's launch
+            // decode steps: the rows' preparation inside the attention's launch
+            if (d.sigmoid_weights && single) ZG_TRY(gated(&rot));
+            else if (single && !vals.norm && !vals.first_out && !vals.mix_first) {
+                WindowStep ws;
+                ws.q = g->proj; ws.ldq = LD; ws.out = g->o; ws.ldo = HV; ws.M = M; ws.H = H; ws.G = G; ws.D = D; ws.V = Vd; ws.scale = d.scale; ws.mask = mask;
+                ws.row_pos = d_pos; ws.row_slot = d_slot; ws.page_table = g->page_table; ws.max_pages = g->max_pages; ws.page_tokens = g->P; ws.cache = ps.cache;
+                ws.ws = g->win_ws; ws.ws_floats = g->win_ws_floats; ws.prep = &rot;
+                window_split_workspace(M, H, Vd, key_cap, &ws.n_split);
+                ZG_TRY(launch_window_step(ws, s, &done));
+            }
             if (!done) {
                 ZG_TRY(launch_window_prep(g->proj, LD, M, H, G, D, Vd, rot, nullptr, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache, s, vals));
                 if (d.sigmoid_weights) ZG_TRY(gated(nullptr));

@@ -415,6 +415,27 @@ int launch_whole_norm_prep(float* qkv, int ld, int M, int HD, int GD, int GV, co
 // of at most 128 channels) take their scores from 32 x 32 tiles on the matrix cores in true fp32 (rows of an entry are consecutive
 // rows with consecutive positions: ent_start / ent_len).
 constexpr int kWinSplits = 64;
+// Steps of up to kGemvMaxRows rows, no mixing matrix, values as they are: the attention in two launches (the keys' shares; where they meet).
+// prep: rows [q (H D) | k (G D) | v (G V)] at q as the projection left them, every row the only one of its sequence: the queries and the
+// token's key are rotated inside, the token's cache row is written (what launch_window_prep does); null: that has been done.
+struct WindowStep {
+    const float* q = nullptr;
+    float* out = nullptr;
+    int ldq = 0, ldo = 0, M = 0, H = 0, G = 0, D = 0, V = 0, max_pages = 0, page_tokens = 0, n_split = 1;
+    float scale = 1.0f;
+    KeyMask mask;
+    const float* sink = nullptr;
+    const int *row_pos = nullptr, *row_slot = nullptr, *page_table = nullptr;
+    float *cache = nullptr, *ws = nullptr;
+    size_t ws_floats = 0;
+    const Rotary* prep = nullptr;
+    const float* out_gate = nullptr;
+    int ld_gate = 0;
+    float out_factor = 1.0f;
+    ScoreShape shape;
+};
+int launch_window_step(const WindowStep& a, hipStream_t s, bool* taken);
+
 size_t window_split_workspace(int rows, int H, int V, int key_capacity, int* n_split_out);
 int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, int M, int H, int G, int D, int V, float scale, KeyMask mask,
                                   const float* sink, const float* talk, const float* vfreq, const int* row_pos, const int* row_slot,

@@ -66,6 +66,12 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
         lv[j] = lr[i];
         lw[j] = own ? a.wkv[i] : 0.0f;
     }
+    // thread rt of its half of the workgroup: rotated pair rt, or a channel behind the rotated ones
+    const int half = a.rot.dims / 2, rt = tid & 127;
+    const int r0 = rt < half ? (a.rot.halves ? rt : 2 * rt) : a.rot.dims + rt - half, r1 = a.rot.halves ? rt + half : 2 * rt + 1;
+    const float* rsrc = tid < 128 || !own ? qh + D : lr + KR;
+    const bool any = R > 0;  // (without a rotated part: some valid channel)
+    const float rx = (any ? rsrc : qh)[any ? min(r0, R - 1) : 0], ry = (any ? rsrc : qh)[any ? min(r1, R - 1) : 0], rf = half > 0 ? a.rot.freq[min(rt, half - 1)] : 0.0f;
     float r[4][ND];
     auto fetch = [&](int kb, float (&to)[4][ND]) {
 #pragma unroll
@@ -101,13 +107,15 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
         ss = wave_allsum(ss);
         if (lane == 0) s_red[wave] = ss;
     }
-    const int half = a.rot.dims / 2, rest = R - a.rot.dims;
-    if (tid < half) rotate_pair(qh + D, s_q + KR, tid, pos, a.rot);
-    else if (tid - half < rest) s_q[KR + a.rot.dims + tid - half] = qh[D + a.rot.dims + tid - half];
-    if (has_new && tid >= 128) {
-        const int t = tid - 128;
-        if (t < half) rotate_pair(lr + KR, s_new + KR, t, pos, a.rot);
-        else if (t - half < rest) s_new[KR + a.rot.dims + t - half] = lr[KR + a.rot.dims + t - half];
+    {   // the rotated parts: the query's by the first two waves, the new key's by the others
+        float* to = tid < 128 ? s_q + KR : s_new + KR;
+        if (tid < 128 || has_new) {
+            if (rt < half) {
+                const float ang = (float)pos * rf, cs = cosf(ang) * a.rot.amp, sn = sinf(ang) * a.rot.amp;
+                to[r0] = rx * cs - ry * sn;
+                to[r1] = ry * cs + rx * sn;
+            } else if (rt < R - half) to[r0] = rx;  // (rotated in pairs, the others alone)
+        }
     }
     __syncthreads();
     if (has_new) {
@@ -130,9 +138,8 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
         acc[i] = 0.0f;
     }
     float mx = -INFINITY, l = 0.0f;
-    for (int kb = kb0; kb < k_hi; kb += 16) {
-        float next[4][ND], s[4];
-        fetch(kb + 16, next);  // (behind the last keys: the last one again, not used)
+    auto take = [&](int kb) {
+        float s[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const bool is_new = has_new && min(kb + u, k_hi - 1) == pos;
@@ -164,11 +171,18 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
             acc[i] = v;
         }
         mx = mn;
+    };
+    int kb = kb0;
+    for (; kb + 16 < k_hi; kb += 16) {
+        float next[4][ND];
+        fetch(kb + 16, next);
+        take(kb);
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int i = 0; i < ND; ++i) r[u][i] = next[u][i];
     }
+    if (kb < k_hi) take(kb);
     if (lane == 0) {
         s_m[wave] = mx;
         s_l[wave] = l;

@@ -12,14 +12,13 @@
 
 #include <algorithm>
 
-#include "lm_kernels.h"
+#include "lm_window_parts.h"
 
 namespace zg {
 namespace lm {
 
 namespace {
 
-__device__ __forceinline__ float sigmoid_f(float z) { return 1.0f / (1.0f + expf(-z)); }
 __device__ __forceinline__ float silu_f(float z) { return z / (1.0f + expf(-z)); }
 __device__ __forceinline__ float softplus_f(float z) { return z > 20.0f ? z : log1pf(expf(z)); }
 __device__ __forceinline__ float gelu_tanh_f(float z) { return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z))); }
@@ -319,30 +318,6 @@ __global__ __launch_bounds__(256) void window_prep_kernel(float* proj, int ld, i
 // normalised weights, their mix over the heads, and the weighted sum of the values of the head's own key/value head.  The
 // result is turned back by the query's position and stored.  Tiles start at the first key of the window: the order of every
 // sum depends on the position alone.
-// The keys a row sees, numbered from 0: first the kept tokens that lie in front of its window (the first `keep` positions of the
-// sequence stay visible), then the window's keys up to the row's own position.  Every kernel below walks this numbering, so the
-// order of a row's sums depends on its position alone.
-struct KeySpan {
-    int j_lo, n_first, n_keys;
-};
-__device__ __forceinline__ KeySpan key_span(int pos, const KeyMask& mask) {
-    KeySpan k;
-    k.j_lo = mask.chunk > 0 ? pos - pos % mask.chunk : mask.window > 0 ? max(0, pos - mask.window + 1) : 0;
-    k.n_first = min(mask.keep, k.j_lo);
-    k.n_keys = k.n_first + pos - k.j_lo + 1;
-    return k;
-}
-__device__ __forceinline__ int key_pos(const KeySpan& k, int n) { return n < k.n_first ? n : k.j_lo + (n - k.n_first); }
-
-// a scaled score on its way to the softmax: capped, then less the head's slope per position of distance (fp32); with a gate the
-// result is the key's weight itself
-__device__ __forceinline__ float shape_score(float sc, const ScoreShape& sh, int h, int dist) {
-    if (sh.cap > 0.0f) sc = sh.cap * tanhf(sc / sh.cap);
-    if (sh.slope) sc -= sh.slope[h] * (float)dist;
-    if (sh.gate) sc = sigmoid_f(sc + sh.gate[h]);
-    return sc;
-}
-
 constexpr int kWinTile = 64;
 constexpr int kWinMaxHeads = 64;
 constexpr int kWinAcc = 16;  // outputs per thread: H * V <= 256 * kWinAcc
@@ -1446,6 +1421,14 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
     if (!ws || need > ws_floats || H > kWinMaxHeads || H % G != 0 || H * V > 256 * kWinAcc || D > 256 || (vfreq && V % 2 != 0) || lds_a > 60 * 1024 ||
         lds_b > 60 * 1024 || M > 65535)
         return ZG_OK;  // the general kernel takes it
+    if (!talk && !vfreq) {  // steps of few rows: scores, weights and values of a share in one launch
+        WindowStep w;
+        w.q = q; w.ldq = ldq; w.out = out; w.ldo = ldo; w.M = M; w.H = H; w.G = G; w.D = D; w.V = V; w.scale = scale; w.mask = mask; w.sink = sink; w.row_pos = row_pos;
+        w.row_slot = row_slot; w.page_table = page_table; w.max_pages = max_pages; w.page_tokens = page_tokens; w.cache = const_cast<float*>(cache); w.n_split = n_split;
+        w.ws = ws; w.ws_floats = ws_floats; w.out_gate = out_gate; w.ld_gate = ld_gate; w.out_factor = out_factor; w.shape = shape;
+        ZG_TRY(launch_window_step(w, s, taken));
+        if (*taken) return ZG_OK;
+    }
     float* sc = ws;
     float* st = sc + (size_t)M * H * key_capacity;
     float* po = st + (size_t)M * n_split * H * 2;
