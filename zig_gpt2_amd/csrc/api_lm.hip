@@ -1188,10 +1188,20 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             }
             ZG_TRY(launch_ssd_scan(sa, single ? &cv : nullptr, M, d_estart, d_elen, d_eslot, n_ent, g->scan_ws, g->scan_ws_floats, s));
             bf16_t* const o16 = r16 && whole(HV) ? g->o16 : nullptr;
-            ZG_TRY(launch_part_norm(g->o, HV, HV, std::max(1, d.norm_groups), M, L.part_norm, eps, single ? &cv : nullptr, d_slot, s, o16));
             lin = Linear();
-            lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
-            ZG_TRY(launch_linear(lin, f32, s));
+            lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
+            bool normed = false;
+            if (few && d.norm_groups <= 1) {  // the norm of the whole row where the product reads it
+                Linear ln = lin;
+                ln.A = g->o; ln.a_norm = L.part_norm; ln.norm_eps = eps;
+                if (single && cv.taps > 1) ln.tail = &cv, ln.tail_slot = d_slot;
+                ZG_TRY(launch_linear_row_norm(ln, s, &normed));
+            }
+            if (!normed) {
+                ZG_TRY(launch_part_norm(g->o, HV, HV, std::max(1, d.norm_groups), M, L.part_norm, eps, single ? &cv : nullptr, d_slot, s, o16));
+                lin.A = o16 ? nullptr : g->o; lin.A16 = o16;
+                ZG_TRY(launch_linear(lin, f32, s));
+            }
         } else if (d.mixer == ZG_LM_MIX_WINDOW_LINEAR) {
             const int G = d.kv_heads, HD = H * D, GD = G * D, GV = G * Vd, CC = HD + GD + GV, HV = H * Vd;
             const int HR = d.lin_heads, DR = d.lin_dim, VR = d.lin_vdim, HRD = HR * DR, HRV = HR * VR, NP = L.n_cat, OC = HV + HRV;

@@ -235,7 +235,9 @@ __global__ __launch_bounds__(256) void lm_gemv_normed_kernel(const float* x, con
     gemv_body<1, U, GEMV_NORM, false, false>(GemvAt{nullptr, B, K, N, ldb, 0, 0, 0, 0}, p, 0, NormIn{x, y, wb, wn, x_out, eps});
 }
 template <int MR, int U, bool SPLIT>
-__global__ __launch_bounds__(256) void lm_gemv_row_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int ldb, int lda, float eps, const LinArgs p) {
+__global__ __launch_bounds__(256) void lm_gemv_row_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int ldb, int lda, float eps, const LinArgs p,
+                                                               const TailArgs tail) {
+    if (blockIdx.y > 0) return move_tails(tail);
     gemv_body<MR, U, GEMV_RMS, SPLIT, false>(GemvAt{A, B, K, N, ldb, lda, 0, 0, 0, a_norm, eps}, p, 0, NormIn());
 }
 // batches [0, za) are product a's, the rest product b's
@@ -273,7 +275,7 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     const int share = split ? (((k_max + 3) / 4) + 7) & ~7 : k_max, pieces = (share + 511) / 512;
     if (pieces > (norm ? 2 : 3)) return ZG_OK;
     const int rows = split ? 2 : 8;
-    const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, 1, A.nz + (B ? B->nz : 0));
+    const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, A.a_norm && A.tail ? 2 : 1, A.nz + (B ? B->nz : 0));
     const bool indirect = A.z_group || A.a_rows || A.a_div != 1;
 #define ZG_GV(MR, U, KIND, SPLIT)                                                                                                                   \
     do {                                                                                                                                            \
@@ -307,8 +309,8 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     } else if (kind == GEMV_RMS) {
 #define ZG_GV_R(MR, U)                                                                                                                                      \
     do {                                                                                                                                                    \
-        if (split) lm_gemv_row_norm_kernel<MR, U, true><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a);                    \
-        else lm_gemv_row_norm_kernel<MR, U, false><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a);                         \
+        if (split) lm_gemv_row_norm_kernel<MR, U, true><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a, tail_args(A));                    \
+        else lm_gemv_row_norm_kernel<MR, U, false><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a, tail_args(A));                         \
     } while (0)
 #define ZG_GV_RU(MR)                     \
     do {                                 \

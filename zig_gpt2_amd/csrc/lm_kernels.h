@@ -29,6 +29,7 @@ enum {
 //   z_group != null: batch z reads the matrix B + z_group[z] * b_zoff instead (the expert an assignment was routed to)
 //   grp_off != null (n_groups > 0): rows [grp_off[e], grp_off[e + 1]) of A / C use the matrix B + e * b_zoff (rows sorted by
 //   expert); M is then the total row count, an upper bound for the tile list
+struct ConvArgs;
 struct Linear {
     const float* A = nullptr;
     int lda = 0;
@@ -55,6 +56,8 @@ struct Linear {
     float poly_eps = 0.0f;
     const float* a_norm = nullptr;     // != null (launch_linear_row_norm alone): A rows enter as x / sqrt(mean(x^2) + norm_eps) * a_norm
     float norm_eps = 0.0f;
+    const ConvArgs* tail = nullptr;    // (with a_norm) a convolution whose tails nobody reads any more, row m's slot in tail_slot[m]
+    const int* tail_slot = nullptr;
     int nz = 1;
     long long a_zoff = 0, b_zoff = 0, c_zoff = 0;
     const int* z_group = nullptr;  // (n_groups: how many matrices it names, 0 where that is not known)
@@ -75,7 +78,7 @@ struct NormIn {
 };
 // One row (L.A only names where the row would be); *taken = false: not a form that has it, nothing launched.
 int launch_linear_normed(const Linear& L, const NormIn& norm, hipStream_t s, bool* taken);
-// Up to kGemvMaxRows rows, each normed on its way in (L.a_norm); *taken as above.
+// Up to kGemvMaxRows rows, each normed on its way in (L.a_norm); *taken as above.  L.tail: the launch also moves the tails of the rows' slots on.
 int launch_linear_row_norm(const Linear& L, hipStream_t s, bool* taken);
 // Picks the row-vector kernel (few rows: decode) or the tiled matrix-core kernel (prompt portions).
 int launch_linear(const Linear& L, bool f32, hipStream_t s);
@@ -239,6 +242,16 @@ struct ConvArgs {
     float* tail = nullptr;
     size_t slot_stride = 0;
 };
+// Channel c of the tail of row m's slot moved on by that row, the only one of its entry: every value takes its successor's place.
+__device__ __forceinline__ void move_tail(const ConvArgs& cv, int slot, int m, int c) {
+    float* tl = cv.tail + (size_t)slot * cv.slot_stride + c;
+    float val = cv.in[(size_t)m * cv.ld_in + c];
+    for (int i = cv.taps - 2; i >= 0; --i) {
+        const float old = tl[(size_t)i * cv.C];
+        tl[(size_t)i * cv.C] = val;
+        val = old;
+    }
+}
 // one_row_each: every entry brings exactly one row (decode steps): the convolution's own threads move the tails on, no second launch.
 int launch_causal_conv(const ConvArgs& a, int M, int n_entries, bool one_row_each, const int* row_off, const int* row_slot, const int* ent_start,
                        const int* ent_len, const int* ent_slot, hipStream_t s);

@@ -118,6 +118,27 @@ inline LinArgs make_args(const Linear& L) {
 
 }  // namespace
 
+namespace {
+// What rides in a launch of row-normed products (Linear::tail), in the second row of the grid.
+struct TailArgs {
+    ConvArgs cv;
+    const int* slot = nullptr;
+    int M = 0;
+};
+inline TailArgs tail_args(const Linear& L) {
+    TailArgs t;
+    if (L.tail) t.cv = *L.tail, t.slot = L.tail_slot, t.M = L.M;
+    return t;
+}
+__device__ __forceinline__ void move_tails(const TailArgs& t) {
+    const int per = (t.cv.C + 255) / 256;
+    for (int b = blockIdx.x; b < t.M * per; b += gridDim.x) {
+        const int m = b / per, c = (b - m * per) * 256 + threadIdx.x;
+        if (c < t.cv.C) move_tail(t.cv, t.slot[m], m, c);
+    }
+}
+}  // namespace
+
 // lm_rows.hip: steps of 3 to 8 rows on the matrix cores.  *taken = false: not a form it has (nothing launched).
 int launch_rows(const Linear& a, const Linear* b, hipStream_t s, bool* taken);
 // lm_gemv.hip: steps of one or two rows whose operands are whole 16-byte pieces.  *taken as above.

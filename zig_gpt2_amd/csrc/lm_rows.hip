@@ -185,7 +185,9 @@ __global__ __launch_bounds__(256) void lm_rows_one_kernel(const float* A, const 
     rows_body<TURNS, KIND, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, a_zoff, b_zoff, 1}, p, blockIdx.z, part);
 }
 template <int TURNS>
-__global__ __launch_bounds__(256) void lm_rows_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int M, int ldb, int lda, float eps, const LinArgs p) {
+__global__ __launch_bounds__(256) void lm_rows_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int M, int ldb, int lda, float eps, const LinArgs p,
+                                                           const TailArgs tail) {
+    if (blockIdx.y > 0) return move_tails(tail);
     __shared__ float part[4][16][17];
     rows_body<TURNS, ROWS_RMS, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, 0, 0, 1, a_norm, eps}, p, blockIdx.z, part);
 }
@@ -239,7 +241,7 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     if (B && (a.a_norm || B->a_norm || !rows_form(*B, b, zb) || za + zb > 65535 || (a.a_glu > 0) != (b.a_glu > 0) || a.glu_out || b.glu_out)) return ZG_OK;
     const int turns = (std::max(a.K, b.K) + kTurn - 1) / kTurn;
     auto tiles = [](const LinArgs& p) { return p.glu_out ? (p.glu_out + 7) / 8 : (p.N + 15) / 16; };
-    const dim3 grid(std::max(tiles(a), tiles(b)), 1, za + zb);
+    const dim3 grid(std::max(tiles(a), tiles(b)), A.a_norm && A.tail ? 2 : 1, za + zb);
     const int per_wave = (turns + 3) / 4;
     const bool one = !B && !a.a_rows && a.a_glu == 0 && (a.z_group || a.a_div == 1);
 #define ZG_ROWS_ONE(T, KIND)                                                                                                                            \
@@ -249,7 +251,7 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     } while (0)
 #define ZG_ROWS(T)                                                                                \
     do {                                                                                          \
-        if (a.a_norm) lm_rows_norm_kernel<T><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.M, a.ldb, a.lda, a.norm_eps, a); \
+        if (a.a_norm) lm_rows_norm_kernel<T><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.M, a.ldb, a.lda, a.norm_eps, a, tail_args(A)); \
         else if (one && a.glu_out > 0) ZG_ROWS_ONE(T, ROWS_GLU_OUT);                                   \
         else if (one) ZG_ROWS_ONE(T, ROWS_PLAIN);                                                 \
         else if (a.a_glu > 0) lm_rows_kernel<T, ROWS_GLU_ON_LOAD><<<grid, 256, 0, s>>>(a, b, za);      \

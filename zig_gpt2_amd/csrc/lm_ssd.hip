@@ -130,6 +130,83 @@ __global__ __launch_bounds__(256) void ssd_scan_kernel(const SsdArgs a, const Co
     }
 }
 
+// One token of every entry (decode steps), convolution of up to four taps inside: a workgroup per (entry, head, 32 columns), a thread four
+// columns of every 32nd row of the state.  A step reads and writes each state once and is a few microseconds of latency: the state's rows,
+// the channels, their tails and weights are all requested at entry.  (In the kernel above every channel's loads wait under a condition.)
+// 24 heads of 128 x 64, three such layers of twelve: a step of one sequence 340 -> 325 us with the norm in the output product and the tails
+// moved on in its launch.  N <= 32 NR, V a multiple of 4.
+template <int NR>
+__global__ __launch_bounds__(256) void ssd_step_kernel(const int* ent_start, const int* ent_slot, const SsdArgs a, const ConvArgs cv) {
+    constexpr int NP = 32 * NR, NJ = (2 * NP + kSsdCols + 255) / 256;
+    __shared__ float s_B[NP], s_C[NP], s_x[kSsdCols];
+    __shared__ __attribute__((aligned(16))) float s_part[4][kSsdCols];
+    const int e = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, c0 = blockIdx.z * kSsdCols, c = (tid & 7) * 4, r0 = tid >> 3;
+    const int slot = ent_slot[e];
+    const size_t m = ent_start[e];
+    const int HV = a.H * a.V, grp = h / (a.H / a.G), oB = HV + grp * a.N, oC = HV + (a.G + grp) * a.N, ox = h * a.V + c0, K = cv.taps - 1;
+    float* Sg = a.state + (size_t)slot * a.slot_stride + (size_t)h * a.N * a.V + min(c0 + c, a.V - 4);
+    const bool ok = c0 + c < a.V;
+    f32x4 S[NR];
+#pragma unroll
+    for (int j = 0; j < NR; ++j) S[j] = *reinterpret_cast<const f32x4*>(Sg + (size_t)min(r0 + 32 * j, a.N - 1) * a.V);
+    const float* tl = cv.tail + (size_t)slot * cv.slot_stride;
+    float v[NJ], wt[NJ][kSsdFastTaps], tv[NJ][kSsdFastTaps], cb[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {  // channel of item o of [B | C | x]; items behind the last one repeat a channel
+        const int o = tid + 256 * j;
+        const int ch = o < NP ? oB + min(o, a.N - 1) : o < 2 * NP ? oC + min(o - NP, a.N - 1) : ox + min(o - 2 * NP, a.V - 1 - c0);
+        v[j] = a.xbc[m * a.ld_xbc + ch];
+        cb[j] = cv.bias ? cv.bias[ch] : 0.0f;
+#pragma unroll
+        for (int t = 0; t < kSsdFastTaps; ++t) {
+            wt[j][t] = cv.w[(size_t)ch * cv.taps + min(t, K)];
+            tv[j][t] = K > 0 ? tl[(size_t)min(t, K - 1) * cv.C + ch] : 0.0f;
+        }
+    }
+    const int oc = min((int)(threadIdx.x & 31), a.V - 1 - c0);  // the column a thread finishes
+    const float zv = a.z[m * a.ld_proj + (size_t)h * a.V + c0 + oc], dtr = a.dt[m * a.ld_proj + h];
+    const float bias = a.dt_bias[h], al = a.a_log[h], skip = a.skip[h];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+        const int o = tid + 256 * j;
+        float acc = cb[j];
+#pragma unroll
+        for (int t = 0; t < kSsdFastTaps; ++t) acc = t <= K ? fmaf(wt[j][t], t < K ? tv[j][t] : v[j], acc) : acc;
+        acc = silu_f(acc);
+        if (o < NP) s_B[o] = acc;
+        else if (o < 2 * NP) s_C[o - NP] = acc;
+        else if (o < 2 * NP + kSsdCols) s_x[o - 2 * NP] = acc;
+    }
+    const float dt = softplus_f(dtr + bias), dec = expf(-expf(al) * dt);
+    __syncthreads();
+    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int j = 0; j < NR; ++j) {
+        const int i = r0 + 32 * j;
+        if (i < a.N) {
+            const float b = s_B[i], cc = s_C[i];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                S[j][k] = fmaf(dec, S[j][k], b * (s_x[c + k] * dt));
+                o[k] = fmaf(S[j][k], cc, o[k]);
+            }
+            if (ok) *reinterpret_cast<f32x4*>(Sg + (size_t)i * a.V) = S[j];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {  // rows of a wave: lanes 8 apart
+        o[k] += __shfl_xor(o[k], 8, 64);
+        o[k] += __shfl_xor(o[k], 16, 64);
+        o[k] += __shfl_xor(o[k], 32, 64);
+    }
+    if ((tid & 63) < 8) *reinterpret_cast<f32x4*>(&s_part[tid >> 6][c]) = o;
+    __syncthreads();
+    if (tid < kSsdCols && c0 + tid < a.V) {
+        const float y = (s_part[0][tid] + s_part[1][tid]) + (s_part[2][tid] + s_part[3][tid]) + skip * s_x[tid];
+        a.out[m * a.ldo + (size_t)h * a.V + c0 + tid] = y * silu_f(zv);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ chunks on the matrix cores
 // With one decay per head and token the recurrence of a chunk of n <= 32 tokens is three matrix products (true fp32,
 // v_mfma_f32_32x32x2_f32); l_t = -exp(a_log) dt_t, L(j, i) = exp(l_(j+1) + ... + l_i):
@@ -367,15 +444,8 @@ __global__ __launch_bounds__(256) void part_norm_kernel(float* v, int ld, int wi
     __shared__ float s_red[8];
     const int m = blockIdx.x, part = blockIdx.y, n = width / parts;
     if (part >= parts) {  // the row is its entry's only one: the workgroups behind the parts move the convolution's tail on, 256 channels each
-        const int K = cv.taps - 1, c = (part - parts) * 256 + threadIdx.x;
-        if (c >= cv.C) return;
-        float* tl = cv.tail + (size_t)row_slot[m] * cv.slot_stride + c;
-        float val = cv.in[(size_t)m * cv.ld_in + c];  // every entry takes its successor's place, the newest one the current input
-        for (int i = K - 1; i >= 0; --i) {
-            const float old = tl[(size_t)i * cv.C];
-            tl[(size_t)i * cv.C] = val;
-            val = old;
-        }
+        const int c = (part - parts) * 256 + threadIdx.x;
+        if (c < cv.C) move_tail(cv, row_slot[m], m, c);
         return;
     }
     const size_t at = (size_t)m * ld + (size_t)part * n;
@@ -487,6 +557,17 @@ int launch_ssd_scan(const SsdArgs& a, const ConvArgs* conv, int M, const int* en
         return ZG_OK;
     }
     const ConvArgs cv = conv ? *conv : ConvArgs();
+    if (conv && cv.taps <= kSsdFastTaps && a.V % 4 == 0 && a.slot_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(a.state) & 15) == 0) {
+        const dim3 grid(n_entries, a.H, (a.V + kSsdCols - 1) / kSsdCols);
+#define ZG_SSD_STEP(NR) ssd_step_kernel<NR><<<grid, 256, 0, s>>>(ent_start, ent_slot, a, cv)
+        if (a.N <= 32) ZG_SSD_STEP(1);
+        else if (a.N <= 64) ZG_SSD_STEP(2);
+        else if (a.N <= 128) ZG_SSD_STEP(4);
+        else ZG_SSD_STEP(8);
+#undef ZG_SSD_STEP
+        ZG_HIP(hipGetLastError());
+        return ZG_OK;
+    }
     const int rr = (a.N + kSsdGroups - 1) / kSsdGroups;
     const dim3 grid(n_entries, a.H, (a.V + kSsdCols - 1) / kSsdCols);
 #define ZG_SSD(R_)                                                                                       \
