@@ -258,6 +258,7 @@ struct zg_lm {
     // of the longest sequence (512, 1024, ... tokens): a share then holds a few dozen keys at any length
     static constexpr int kKeyBuckets = 24;
     hipGraphExec_t decode_graph[kGemvMaxRows + 1][kKeyBuckets] = {};
+    hipGraphExec_t chain_graph[kGemvMaxRows + 1][kKeyBuckets] = {};  // the same as a link of a generation, from its token's rows to the next token's
     bool whole_context = false;  // some pass attends over the whole sequence through the split kernels
     int bucket_keys = 0;         // key capacity of the running decode step's bucket
 };
@@ -911,10 +912,18 @@ int check_layer(const zg_lm_layer& d, size_t i, unsigned flags) {
     return ZG_OK;
 }
 
+// rows the kernels between sublayers take in one piece (lm_norm.hip)
+bool rows_fit(const zg_lm* g) { return g->W % 4 == 0 && g->W <= 1024; }
+// generations that hand a step's token to the next step's layers in one launch
+bool steps_chain(const zg_lm* g) {
+    return rows_fit(g) && g->canon < 1 && !g->side && !g->tanh_norms && !((g->cfg.flags & ZG_LM_LOOP_READD) && g->cfg.loop_times > 1) && !g->pos_freq;
+}
+
 // The kernels of one portion, from the embedding to the commit of the token-shift rows: launches only, every per-step value
 // (tokens, positions, slots, page tables) is read from device memory — so for a given number of rows and entries the sequence
 // is the same every step and can be replayed from a captured graph (decode steps: one row per entry).
-int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
+// chained: a step of a generation whose embedding and first norm the step before has left in x and h; ends with the last norm's rows in hn.
+int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool chained = false) {
     hipStream_t s = g->stream;
     const int W = g->W, MS = g->MS, NS = g->NS;
     const int *d_ids = g->meta, *d_pos = d_ids + MS, *d_slot = d_pos + MS, *d_prev = d_slot + MS, *d_last = d_prev + MS, *d_want = d_last + MS;
@@ -928,7 +937,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     const bool few = M <= kGemvMaxRows;
     const bool canon = g->canon >= 1;
     const bool readd = (g->cfg.flags & ZG_LM_LOOP_READD) && g->cfg.loop_times > 1;
-    ZG_TRY(launch_embed(g->embed, d_ids, x, readd ? g->x0 : nullptr, g->embed_scale, M, W, g->V, g->flag, d_pos, g->pos_freq, s));
+    if (!chained) ZG_TRY(launch_embed(g->embed, d_ids, x, readd ? g->x0 : nullptr, g->embed_scale, M, W, g->V, g->flag, d_pos, g->pos_freq, s));
     const bool side = g->side;
     const bool tnorm = g->tanh_norms;
     // Prompt portions in bf16 mode: what only matrix products read travels rounded to bf16, from the kernel that writes it, where its rows
@@ -1054,7 +1063,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         up_done = &L;
         return launch_linear_pair(lin, dense_up(L, g->hc, nullptr), f32, s);
     };
-    bool h_ready = false;  // g->h already holds this pass's shifted norm (written by the previous pass's fused tail)
+    // the token shift of steps of one row per entry: a row's normed form goes straight into its slot (each slot has one reader)
+    const bool shift_in_place = single && !canon && !side && !tnorm && !g->no_shift && rows_fit(g);
+    bool h_ready = chained;  // g->h already holds this pass's shifted norm (written by the previous pass's fused tail)
     if (tnorm) {  // the norm behind the embedding (in place) and the first pass's norm; every later one rides behind a sublayer's sum
         ZG_TRY(launch_tanh_norm(x, g->embed_norm, g->layers[g->passes[0].layer].norm1, nullptr, g->h, M, W, s));
         h_ready = true;
@@ -1075,6 +1086,13 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             ZG_TRY(launch_norm_conv_single(x, ps.readd ? g->x0 : nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, L.norm1, eps, M, W, g->canon,
                                            L.canon1, g->seq_state + ps.canon1_off, g->seq_floats, d_slot, g->hc, s, &hc_ready));
         if (ps.readd && !hc_ready) ZG_TRY(launch_add_rows(x, g->x0, M, W, s));
+        if (!h_ready && !hc_ready && shift_in_place) {
+            NormRows r;
+            r.x = x; r.wn = L.norm1; r.mu = L.shift; r.eps = eps; r.out = g->h; r.M = M; r.W = W; r.row_slot = d_slot; r.shift_state = g->shift_state + (size_t)p * W;
+            r.slot_stride = (size_t)g->n_passes * W; r.shift_out = g->shift_state + (size_t)p * W;
+            ZG_TRY(launch_norm_rows(r, s, &h_ready));
+            ZG_REQUIRE(h_ready, ZG_ERR_UNSUPPORTED, "norms between sublayers: rows of %d", W);
+        }
         if (!h_ready && !hc_ready)
             ZG_TRY(launch_norm_shift(x, L.norm1, canon ? nullptr : L.shift, eps, h_r16 ? nullptr : g->h, M, W, d_prev, d_slot, g->shift_state + (size_t)p * W,
                                      (size_t)g->n_passes * W, canon || g->no_shift ? nullptr : d_last, g->last_h + (size_t)p * NS * W, s, h_r16 ? g->h16 : nullptr));
@@ -1087,6 +1105,14 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
         }
         // the pass's last sum fused with the next pass's norm (with a token shift: in steps of one row per entry)
         auto tail = [&](const float* y, const float* yexp, const float* weight, int top, const float* wb) -> int {
+            if (chained && p + 1 == g->n_passes) {  // the last sum, and the norm in front of the head
+                NormRows r;
+                r.x = x; r.y = y; r.yexp = yexp; r.weight = weight; r.top = top; r.wb = wb; r.wn = g->final_norm; r.eps = eps; r.out = g->hn; r.M = M; r.W = W; r.x_out = g->x;
+                ZG_TRY(launch_norm_rows(r, s, &h_ready));
+                ZG_REQUIRE(h_ready, ZG_ERR_UNSUPPORTED, "norms between sublayers: rows of %d", W);
+                x = g->x;
+                return ZG_OK;
+            }
             if (p + 1 >= g->n_passes || canon || g->passes[p + 1].readd) return ZG_OK;
             const LayerW& N = g->layers[g->passes[p + 1].layer];
             if (g->no_shift && y && defer) {
@@ -1100,6 +1126,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
             if (!g->no_shift) {
                 r.mu = N.shift; r.row_prev = single ? nullptr : d_prev; r.row_slot = d_slot; r.shift_state = g->shift_state + (size_t)(p + 1) * W;
                 r.slot_stride = (size_t)g->n_passes * W; r.row_entry_if_last = d_last; r.last_out = g->last_h + (size_t)(p + 1) * NS * W;
+                if (shift_in_place) r.row_entry_if_last = nullptr, r.last_out = nullptr, r.shift_out = g->shift_state + (size_t)(p + 1) * W;
             }
             r.x_out = r.row_prev ? x_other : x;
             ZG_TRY(launch_norm_rows(r, s, &h_ready));
@@ -1107,6 +1134,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
                 if (r.x_out != x) std::swap(x, x_other);
                 return ZG_OK;
             }
+            ZG_REQUIRE(!shift_in_place, ZG_ERR_UNSUPPORTED, "norms between sublayers: rows of %d", W);
             if (yexp && !few) return ZG_OK;  // (rows the general kernels take)
             if (g->no_shift && y) {  // nothing of the token before: the same fusion at any number of rows
                 ZG_TRY(launch_norm_add_norm(x, y, wb, N.norm1, eps, h_r16 ? nullptr : g->h, M, W, s, h_r16 ? g->h16 : nullptr));
@@ -1676,7 +1704,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single) {
     }
     if (x != g->x) ZG_TRY(launch_copy_floats(x, g->x, (size_t)M * W, s));
     // the rows the last tokens of the entries left for the token shift of their successors
-    if (!canon && !side && !tnorm && !g->no_shift) ZG_TRY(launch_commit_rows(g->shift_state, (size_t)g->n_passes * W, g->last_h, W, d_eslot, n_ent, W, g->n_passes, W, (size_t)NS * W, s));
+    if (!canon && !side && !tnorm && !g->no_shift && !shift_in_place) ZG_TRY(launch_commit_rows(g->shift_state, (size_t)g->n_passes * W, g->last_h, W, d_eslot, n_ent, W, g->n_passes, W, (size_t)NS * W, s));
 
     return ZG_OK;
 }
@@ -1729,23 +1757,52 @@ int key_bucket(zg_lm* g) {
     return bucket;
 }
 
+// the product with the head of nw normed rows
+int enqueue_head(zg_lm* g, int nw) {
+    Linear lin;
+    lin.A = g->hn; lin.lda = g->W; lin.B = g->head; lin.ldb = g->W; lin.C = g->logits; lin.ldc = g->V; lin.M = nw; lin.N = g->V; lin.K = g->W;
+    if ((g->cfg.logit_scale != 0.0f && g->cfg.logit_scale != 1.0f) || g->cfg.logit_softcap > 0.0f) {
+        lin.act = ACT_SCALE_SOFTCAP;
+        lin.act_a = g->cfg.logit_scale != 0.0f ? g->cfg.logit_scale : 1.0f;
+        lin.act_b = g->cfg.logit_softcap;
+    }
+    return launch_linear(lin, g->f32, g->stream);
+}
+
+// a link of a generation: the layers behind rows that are embedded and normed already, the logits, the next token and its rows
+int enqueue_chained(zg_lm* g, int M) {
+    ZG_TRY(enqueue_layers(g, M, M, true, true, true));
+    ZG_TRY(enqueue_head(g, M));
+    const LayerW& first = g->layers[g->passes[0].layer];
+    NextToken t;
+    ZG_TRY(launch_argmax_parts(g->logits, M, g->V, g->amax_val, g->amax_idx, &t.n_parts, g->stream));
+    const size_t MS = g->MS;
+    t.part_val = g->amax_val; t.part_idx = g->amax_idx; t.table = g->embed; t.W = g->W; t.scale = g->embed_scale; t.eps = g->cfg.norm_eps; t.wn = first.norm1;
+    t.mu = g->no_shift ? nullptr : first.shift; t.ids = g->meta; t.pos = g->meta + MS; t.row_slot = g->meta + 2 * MS; t.count = g->meta + meta_row_off(g); t.seen = g->h_ahead;
+    t.ahead = zg_lm::kAhead; t.seen_stride = kGemvMaxRows; t.x = g->x; t.h = g->h; t.last_h = g->last_h; t.shift_state = g->shift_state;
+    t.slot_stride = (size_t)g->n_passes * g->W;
+    return launch_next_token(t, M, g->stream);
+}
+
 // a decode step: replay the captured sequence of this batch size
-int replay_step(zg_lm* g, int M, int bucket) {
+int replay_step(zg_lm* g, int M, int bucket, bool chained = false) {
     hipStream_t s = g->stream;
-    if (!g->decode_graph[M][bucket]) {
+    hipGraphExec_t& exec = chained ? g->chain_graph[M][bucket] : g->decode_graph[M][bucket];
+    if (!exec) {
         hipGraph_t graph = nullptr;
         ZG_HIP(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        const int st = enqueue_layers(g, M, M, true, true);
+        const int st = chained ? enqueue_chained(g, M) : enqueue_layers(g, M, M, true, true);
         const hipError_t ce = hipStreamEndCapture(s, &graph);
         if (st != ZG_OK) {
             if (graph) (void)hipGraphDestroy(graph);
             return st;
         }
         ZG_HIP(ce);
-        ZG_HIP(hipGraphInstantiate(&g->decode_graph[M][bucket], graph, nullptr, nullptr, 0));
-        ZG_HIP(hipGraphDestroy(graph));
+        const hipError_t ie = hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(graph);
+        ZG_HIP(ie);
     }
-    ZG_HIP(hipGraphLaunch(g->decode_graph[M][bucket], s));
+    ZG_HIP(hipGraphLaunch(exec, s));
     return ZG_OK;
 }
 
@@ -1755,14 +1812,7 @@ int enqueue_logits(zg_lm* g, int nw) {
     const int W = g->W;
     if (g->tanh_norms) ZG_TRY(launch_tanh_norm(g->x, nullptr, g->final_norm, d_want, g->hn, nw, W, g->stream));
     else ZG_TRY(launch_norm_gather(g->x, d_want, g->final_norm, g->cfg.norm_eps, g->hn, nw, W, g->side, g->stream));
-    Linear lin;
-    lin.A = g->hn; lin.lda = W; lin.B = g->head; lin.ldb = W; lin.C = g->logits; lin.ldc = g->V; lin.M = nw; lin.N = g->V; lin.K = W;
-    if ((g->cfg.logit_scale != 0.0f && g->cfg.logit_scale != 1.0f) || g->cfg.logit_softcap > 0.0f) {
-        lin.act = ACT_SCALE_SOFTCAP;
-        lin.act_a = g->cfg.logit_scale != 0.0f ? g->cfg.logit_scale : 1.0f;
-        lin.act_b = g->cfg.logit_softcap;
-    }
-    return launch_linear(lin, g->f32, g->stream);
+    return enqueue_head(g, nw);
 }
 
 // the uniform of (seed, length of the sequence with the token to be drawn, output row)
@@ -1929,6 +1979,16 @@ int step_impl(zg_lm* g, const zg_lm_entry* entries, size_t n_entries, float* log
     return ZG_OK;
 }
 
+// the first link's rows: what enqueue_chained leaves for the others
+int enqueue_first_rows(zg_lm* g, int M) {
+    const LayerW& first = g->layers[g->passes[0].layer];
+    const size_t MS = g->MS;
+    const int *d_pos = g->meta + MS, *d_slot = d_pos + MS, *d_prev = d_slot + MS, *d_last = d_prev + MS;
+    ZG_TRY(launch_embed(g->embed, g->meta, g->x, nullptr, g->embed_scale, M, g->W, g->V, g->flag, d_pos, g->pos_freq, g->stream));
+    return launch_norm_shift(g->x, first.norm1, first.shift, g->cfg.norm_eps, g->h, M, g->W, d_prev, d_slot, g->shift_state, (size_t)g->n_passes * g->W,
+                             g->no_shift ? nullptr : d_last, g->last_h, g->stream);
+}
+
 // The steps of a generation behind its prompts: every sequence one token at a time.  What a step needs from the one before it, the tokens
 // and positions, is handed on by the device (advance_rows), so steps are enqueued ahead of the tokens the host has seen (at most kAhead)
 // and no step waits for a round trip to the host.  New pages travel as launch arguments: the host goes on changing its tables.  Bookkeeping and errors are those of the steps taken one by one: tokens of the steps
@@ -1938,6 +1998,7 @@ int decode_ahead(zg_lm* g, const std::vector<int>& seqs, const int32_t* first, s
     const int M = (int)seqs.size(), MS = g->MS;
     ZG_HIP(hipSetDevice(g->device));
     size_t enqueued = 1, seen = 1;  // tokens of every sequence
+    const bool chained = temp <= 0.0f && steps_chain(g);  // the largest logit decides: a step ends with the next one's first rows
     auto collect = [&]() -> int {
         const int at = (int)(seen % zg_lm::kAhead);
         ZG_HIP(hipEventSynchronize(g->ahead_done[at]));
@@ -1973,16 +2034,21 @@ int decode_ahead(zg_lm* g, const std::vector<int>& seqs, const int32_t* first, s
         }
         ZG_TRY(launch_new_pages(g->page_table, grown, s));
         const int at = (int)(enqueued % zg_lm::kAhead);
-        ZG_TRY(replay_step(g, M, key_bucket(g)));
-        ZG_TRY(enqueue_logits(g, M));
-        ZG_TRY(launch_row_argmax(g->logits, M, g->V, g->row_max, g->tok_out, g->amax_val, g->amax_idx, s));
-        if (temp > 0.0f) {
-            float* u = g->h_ahead_u + at * kGemvMaxRows;
-            for (int b = 0; b < M; ++b) u[b] = draw_uniform(seed, (int)g->slots[seqs[b]].len, b);
-            ZG_HIP(hipMemcpyAsync(g->samp_u, u, M * sizeof(float), hipMemcpyHostToDevice, s));
-            ZG_TRY(launch_sample(g->logits, M, g->V, temp, g->samp_u, g->row_max, 1, 1, g->samp_ws, g->tok_out, false, s));
+        if (chained) {
+            if (enqueued == 1) ZG_TRY(enqueue_first_rows(g, M));
+            ZG_TRY(replay_step(g, M, key_bucket(g), true));
+        } else {
+            ZG_TRY(replay_step(g, M, key_bucket(g)));
+            ZG_TRY(enqueue_logits(g, M));
+            ZG_TRY(launch_row_argmax(g->logits, M, g->V, g->row_max, g->tok_out, g->amax_val, g->amax_idx, s));
+            if (temp > 0.0f) {
+                float* u = g->h_ahead_u + at * kGemvMaxRows;
+                for (int b = 0; b < M; ++b) u[b] = draw_uniform(seed, (int)g->slots[seqs[b]].len, b);
+                ZG_HIP(hipMemcpyAsync(g->samp_u, u, M * sizeof(float), hipMemcpyHostToDevice, s));
+                ZG_TRY(launch_sample(g->logits, M, g->V, temp, g->samp_u, g->row_max, 1, 1, g->samp_ws, g->tok_out, false, s));
+            }
+            ZG_TRY(launch_advance_rows(g->tok_out, M, g->meta, g->meta + MS, g->h_ahead + at * kGemvMaxRows, s));
         }
-        ZG_TRY(launch_advance_rows(g->tok_out, M, g->meta, g->meta + MS, g->h_ahead + at * kGemvMaxRows, s));
         ZG_HIP(hipEventRecord(g->ahead_done[at], s));
         for (int b = 0; b < M; ++b) {
             ++g->slots[seqs[b]].len;
@@ -2272,9 +2338,10 @@ int zg_lm_destroy(zg_lm* g) {
     if (!g) return ZG_OK;
     (void)hipSetDevice(g->device);
     if (g->stream) (void)hipStreamSynchronize(g->stream);
-    for (auto& by_rows : g->decode_graph)
-        for (hipGraphExec_t e : by_rows)
-            if (e) (void)hipGraphExecDestroy(e);
+    for (auto* graphs : {&g->decode_graph, &g->chain_graph})
+        for (auto& by_rows : *graphs)
+            for (hipGraphExec_t e : by_rows)
+                if (e) (void)hipGraphExecDestroy(e);
     if (g->ev0) (void)hipEventDestroy(g->ev0);
     if (g->ev1) (void)hipEventDestroy(g->ev1);
     if (g->stream) (void)hipStreamDestroy(g->stream);

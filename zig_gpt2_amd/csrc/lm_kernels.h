@@ -133,6 +133,7 @@ struct NormRows {
     size_t slot_stride = 0;
     const int* row_entry_if_last = nullptr;
     float* last_out = nullptr;
+    float* shift_out = nullptr;  // steps of one row per entry: the row's own normed form straight into its slot's state (shift_state's layout)
     int run = 1;  // (set by the launch) consecutive rows of a wave
 };
 int launch_norm_rows(const NormRows& p, hipStream_t s, bool* taken);
@@ -544,6 +545,24 @@ int launch_moe_combine(const float* x, float* out, const float* yexp, const int*
 
 // ------------------------------------------------------------------------------------------------ sampling support
 // rows of the next step of a generation: ids[r] = seen[r] = tok[r], pos[r] += 1  (seen: pinned host memory)
+// What stands between two steps of a generation that takes the largest logit (rows of up to 1024 values in whole 16-byte pieces): the token from
+// the partial maxima of launch_argmax_parts, the row's metadata moved on and the token handed to the host (the place in its ring by the
+// row's count), its embedding, and the first pass's norm with the token shift.  The shift's state takes the row of the token this step
+// consumed (last_h), whose place the new row takes; the new one is consumed by the next step, if there is one.
+struct NextToken {
+    const float* part_val = nullptr;
+    const int* part_idx = nullptr;
+    const bf16_t* table = nullptr;
+    const float *wn = nullptr, *mu = nullptr;  // mu null: no shift
+    int n_parts = 0, W = 0, ahead = 1, seen_stride = 0;
+    float scale = 1.0f, eps = 0.0f;
+    int *ids = nullptr, *pos = nullptr, *count = nullptr, *seen = nullptr;
+    float *x = nullptr, *h = nullptr, *last_h = nullptr, *shift_state = nullptr;
+    const int* row_slot = nullptr;
+    size_t slot_stride = 0;
+};
+int launch_argmax_parts(const float* logits, int rows, int n, float* part_val, int* part_idx, int* n_parts, hipStream_t s);
+int launch_next_token(const NextToken& a, int M, hipStream_t s);
 int launch_advance_rows(const int* tok, int M, int* ids, int* pos, int* seen, hipStream_t s);
 // entries of the page table that such a step adds, one a row at most: table[at[i]] = page[i]
 struct NewPages {

@@ -1502,6 +1502,74 @@ __global__ __launch_bounds__(64) void new_pages_kernel(int* table, const NewPage
 
 // Stage 1: block (row, part) finds the maximum and its first index in its slice of the row; stage 2 (parts == 1 in the grid,
 // n_parts > 0 as argument): one block per row combines the parts.  The first maximum wins; a row of NaNs gives index 0.
+// The largest of a workgroup's values and its index (the smaller one of equals), in every thread; s_v, s_i: four each.
+__device__ __forceinline__ void block_argmax(float& best, int& bi, float* s_v, int* s_i) {
+    const float wbest = wave_allmax(best);
+    int cand = (best == wbest) ? bi : 0x7fffffff;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) cand = min(cand, __shfl_xor(cand, off, 64));
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (lane == 0) {
+        s_v[wave] = wbest;
+        s_i[wave] = cand;
+    }
+    __syncthreads();
+    best = s_v[0];
+    bi = s_i[0];
+    for (int w = 1; w < 4; ++w)
+        if (s_v[w] > best || (s_v[w] == best && s_i[w] < bi)) {
+            best = s_v[w];
+            bi = s_i[w];
+        }
+}
+
+__global__ __launch_bounds__(256) void next_token_kernel(const NextToken a) {
+    __shared__ float s_v[4], s_red[4];
+    __shared__ int s_i[4];
+    const int m = blockIdx.x, tid = threadIdx.x, at = min(tid * 4, a.W - 4);
+    const bool in = tid * 4 < a.W;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    const int part = min(tid, a.n_parts - 1);
+    float best = a.part_val[(size_t)m * a.n_parts + part];
+    int bi = a.part_idx[(size_t)m * a.n_parts + part];
+    const f32x4 wn = *reinterpret_cast<const f32x4*>(a.wn + at);
+    f32x4 mu = zero, before = zero;
+    if (a.mu) {
+        mu = *reinterpret_cast<const f32x4*>(a.mu + at);
+        before = *reinterpret_cast<const f32x4*>(a.last_h + (size_t)m * a.W + at);
+    }
+    if (tid >= a.n_parts || !(best > -INFINITY)) bi = 0x7fffffff, best = -INFINITY;
+    block_argmax(best, bi, s_v, s_i);
+    if (bi == 0x7fffffff) bi = 0;  // (no logit is a number)
+    const u32x2 e = *reinterpret_cast<const u32x2*>(a.table + (size_t)bi * a.W + at);
+    if (tid == 0) {
+        const int n = a.count[m] + 1;  // the step's number, from 1
+        a.ids[m] = bi;
+        a.pos[m] += 1;
+        a.count[m] = n;
+        a.seen[(n % a.ahead) * a.seen_stride + m] = bi;
+    }
+    const f32x4 x = {bf16_lo(e.x) * a.scale, bf16_hi(e.x) * a.scale, bf16_lo(e.y) * a.scale, bf16_hi(e.y) * a.scale};
+    float ss = in ? fmaf(x.x, x.x, fmaf(x.y, x.y, fmaf(x.z, x.z, x.w * x.w))) : 0.0f;
+    ss = wave_allsum(ss);
+    if ((tid & 63) == 0) s_red[tid >> 6] = ss;
+    __syncthreads();
+    const float r = 1.0f / sqrtf(((s_red[0] + s_red[1]) + (s_red[2] + s_red[3])) / (float)a.W + a.eps);
+    if (!in) return;
+    f32x4 h, o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        h[i] = x[i] * r * (1.0f + wn[i]);
+        o[i] = a.mu ? h[i] + (before[i] - h[i]) * mu[i] : h[i];
+    }
+    *reinterpret_cast<f32x4*>(a.x + (size_t)m * a.W + at) = x;
+    *reinterpret_cast<f32x4*>(a.h + (size_t)m * a.W + at) = o;
+    if (a.mu) {
+        *reinterpret_cast<f32x4*>(a.shift_state + (size_t)a.row_slot[m] * a.slot_stride + at) = before;
+        *reinterpret_cast<f32x4*>(a.last_h + (size_t)m * a.W + at) = h;
+    }
+}
+
 __global__ __launch_bounds__(256) void row_argmax_kernel(const float* logits, int n, float* max_out, int* idx_out, float* part_val, int* part_idx,
                                                          int n_parts, int combine) {
     __shared__ float s_v[4];
@@ -1529,24 +1597,10 @@ __global__ __launch_bounds__(256) void row_argmax_kernel(const float* logits, in
             }
         }
     }
-    const float wbest = wave_allmax(best);
-    int cand = (best == wbest) ? bi : 0x7fffffff;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) cand = min(cand, __shfl_xor(cand, off, 64));
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if (lane == 0) {
-        s_v[wave] = wbest;
-        s_i[wave] = cand;
-    }
-    __syncthreads();
+    block_argmax(best, bi, s_v, s_i);
     if (threadIdx.x == 0) {
-        float v = s_v[0];
-        int ix = s_i[0];
-        for (int w = 1; w < 4; ++w)
-            if (s_v[w] > v || (s_v[w] == v && s_i[w] < ix)) {
-                v = s_v[w];
-                ix = s_i[w];
-            }
+        const float v = best;
+        int ix = bi;
         if (!combine) {
             part_val[(size_t)row * n_parts + blockIdx.y] = v;
             part_idx[(size_t)row * n_parts + blockIdx.y] = ix;
@@ -1920,6 +1974,22 @@ int launch_new_pages(int* table, const NewPages& pages, hipStream_t s) {
     if (pages.n <= 0) return ZG_OK;
     ZG_REQUIRE(pages.n <= kGemvMaxRows, ZG_ERR_ARG, "new pages: %d at a time", pages.n);
     new_pages_kernel<<<1, 64, 0, s>>>(table, pages);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_argmax_parts(const float* logits, int rows, int n, float* part_val, int* part_idx, int* n_parts, hipStream_t s) {
+    *n_parts = std::max(1, std::min(kArgmaxParts, (n + 1023) / 1024));
+    if (rows <= 0) return ZG_OK;
+    row_argmax_kernel<<<dim3(rows, *n_parts), 256, 0, s>>>(logits, n, nullptr, nullptr, part_val, part_idx, *n_parts, 0);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_next_token(const NextToken& a, int M, hipStream_t s) {
+    if (M <= 0) return ZG_OK;
+    ZG_REQUIRE(a.W >= 4 && a.W <= 1024 && a.W % 4 == 0 && a.n_parts >= 1 && a.n_parts <= 256 && a.ahead >= 1, ZG_ERR_ARG, "next token: rows of %d, %d parts", a.W, a.n_parts);
+    next_token_kernel<<<M, 256, 0, s>>>(a);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

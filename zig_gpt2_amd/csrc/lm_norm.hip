@@ -116,6 +116,11 @@ __global__ __launch_bounds__(256) void norm_rows_kernel(const float* x_in, const
         if constexpr (TO == TO_NOTHING) continue;
         norm(x, h);
         if constexpr (TO == TO_SHIFT) {
+            if (p.shift_out) {
+#pragma unroll
+                for (int j = 0; j < NV; ++j)
+                    if (in[j]) *reinterpret_cast<f32x4*>(p.shift_out + (size_t)p.row_slot[m] * p.slot_stride + at[j]) = h[j];
+            }
             const int entry = p.row_entry_if_last ? p.row_entry_if_last[m] : -1;
             if (entry >= 0) {
 #pragma unroll
