@@ -68,7 +68,7 @@ struct Linear {
 };
 // Steps of few rows: the first product of a gated feed-forward with the activation in its epilogue, h [rows][F] = act(gate) * up for B rows
 // [gate (F) | up (F)]; L as for launch_linear, its C, ldc, c_zoff and N ignored.  *taken = false: not a form that has it, nothing launched.
-int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t s, bool* taken);
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, hipStream_t s, bool* taken);
 // What launch_norm_add_norm does, inside the product that reads the row: x_out = x + norm(y) (1 + wb), and the product's row is
 // norm(x_out) (1 + wn).  x_out must not be x (every workgroup reads x, one writes x_out).
 struct NormIn {

@@ -5,7 +5,8 @@
 //                      three rows and more, lists of experts), and for what these leave
 //   * lm_gemv_kernel   (long rows: lm_gemv_ks_kernel) a wave owns two weight rows, its lanes split K in 16-byte pieces, the
 //                      activation rows come straight from the cache hierarchy, sums are fp32 FMAs in both precision modes.
-//   * gemm_s4_kernel   (gemm_s4.hip) plain products of prompt portions whose rows are rounded already, from 112 tiles of 256 x 192 on.
+//   * gemm_s4_kernel   (gemm_s4.hip) plain products of prompt portions whose rows are rounded already, where they fill the chip several times.
+//   * lm_stream_kernel (lm_stream.hip) the other products of rounded rows whose K is whole steps of 64, experts' among them.
 //   * lm_wide_kernel   prompt portions that fill the chip: 128 x 128 or 64 x 64 tiles staged through the LDS.
 //   * lm_deep_kernel   short portions: 32-wide tiles with K split over the waves of a workgroup.
 //                      Both multiply with v_mfma_f32_32x32x16_bf16: bf16 mode rounds the activations on their way there, 32-bit mode
@@ -353,47 +354,6 @@ struct Act8<bf16_t> {
     }
 };
 
-// The tile of a workgroup: rows [m0, m_end) of A / C, columns from n0, the matrix.  Consecutive workgroups go to the eight XCDs in
-// turn, so the tile list is dealt in eight contiguous runs: the tiles of one run share their A rows in that XCD's L2.
-struct TileAt {
-    const bf16_t* B;
-    int m0, m_end, n0;
-};
-__device__ __forceinline__ bool find_tile(const LinArgs& p, int BM, int BN, TileAt& t) {
-    const int n_tiles = (p.N + BN - 1) / BN, total = gridDim.x, id = blockIdx.x;
-    const int q = total >> 3, r = total & 7, x = id & 7;
-    const int at = x * q + min(x, r) + (id >> 3);
-    int mt = at / n_tiles;
-    t.n0 = (at - mt * n_tiles) * BN;
-    t.B = p.B + (long long)blockIdx.z * p.b_zoff;
-    t.m0 = mt * BM;
-    t.m_end = p.M;
-    if (p.grp_off) {  // the row group this tile belongs to: 64 groups' tile counts summed across the lanes at a time
-        const int lane = threadIdx.x & 63;
-        for (int e0 = 0;; e0 += 64) {
-            if (e0 >= p.n_groups) return false;
-            const int e = min(e0 + lane, p.n_groups - 1);
-            const int lo = p.grp_off[e], hi = p.grp_off[e + 1];
-            const int own = e0 + lane < p.n_groups ? (hi - lo + BM - 1) / BM : 0;
-            int upto = own;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const int o = __shfl_up(upto, d, 64);
-                if (lane >= d) upto += o;
-            }
-            const unsigned long long past = __ballot(mt < upto);
-            if (past) {
-                const int l = __builtin_ctzll(past);
-                t.B = p.B + (long long)(e0 + l) * p.b_zoff;
-                t.m0 = __shfl(lo, l, 64) + (mt - __shfl(upto - own, l, 64)) * BM;
-                t.m_end = __shfl(hi, l, 64);
-                break;
-            }
-            mt -= __shfl(upto, 63, 64);
-        }
-    }
-    return t.m0 < t.m_end;
-}
 template <typename AT>
 __device__ __forceinline__ const AT* a_row(const LinArgs& p, int m) {
     const AT* A;
@@ -448,7 +408,7 @@ __global__ __launch_bounds__(256, 2) void lm_wide_kernel(const LinArgs p) {
     __shared__ __attribute__((aligned(16))) bf16_t Bs[2][BN * BK];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, wy = wave >> 1, wx = wave & 1;
     TileAt t;
-    if (!find_tile(p, BM, BN, t)) return;
+    if (!find_tile(p, p.N, BM, BN, t)) return;
     auto swz = [](int row) { return CH == 8 ? row & 7 : (row >> 1) & 3; };  // (row & 31 decides)
 
     const AT* a_src[AC];
@@ -621,7 +581,7 @@ __global__ __launch_bounds__(256, 2) void lm_deep_kernel(const LinArgs p) {
     __shared__ float part[4][TM * TN * 16][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 31, kh = lane >> 5;
     TileAt t;
-    if (!find_tile(p, BM, BN, t)) return;
+    if (!find_tile(p, p.N, BM, BN, t)) return;
     const AT* a_src[TM];
     const bf16_t* b_src[TN];
 #pragma unroll
@@ -908,12 +868,15 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LinArgs p) {
 
 namespace {
 // Plain products of rounded rows with enough tiles of 256 x 192 go to the persistent kernel of the large-batch Linears (gemm_s4.hip), whose
-// hand-scheduled four waves keep the matrix cores twice as busy: 8184 x 3072 x 1024 59 against 89 us, 47 with a rounded result; 8184 x
-// 4096 x 1024 with max(., 0)^2 and a rounded result 71 against 117; 8184 x 672 x 1024 (128 tiles) 26.6 against 29; 1791 x 3072 x 768 (112)
-// 23.2 against 24.5; 1023 x 3072 x 768 (64 tiles) 21.7 against 15.4.
+// hand-scheduled four waves read the LDS less for every product: 8184 x 3072 x 1024 67 against 78 us (lm_stream.hip); 8184 x 4096 x 1024 with max(., 0)^2
+// and a rounded result 68 against 85; 8184 x 1536 x 384 20.5 against 23.6.  Its time goes by rounds of 256 tiles, each what 640 tiles of 128 x 128
+// cost there: 8184 x 1024 x 1024 (512 of those) 29.1 against 25.3, 8184 x 672 x 1024 25.7 against 21.9, 2048 x 3072 x 768 23.7 against 19.5.
+// Products that kernel cannot take (columns in no whole pieces of eight) come here from 112 tiles on: 1791 x 3072 x 768 23.2 against 24.5 on the
+// staged tiles.
 bool takes_persistent(const Linear& L) {
     const char* form = getenv("ZGPT2_LM_GEMM_TILE");  // test hook: 256 = here at any number of tiles, another = never
-    const int least = form ? (atoi(form) == 256 ? 1 : 0x7fffffff) : 112;
+    const long long tiles = (long long)((L.M + 255) / 256) * ((L.N + 191) / 192), fine = (long long)((L.M + 127) / 128) * ((L.N + 127) / 128);
+    const bool pays = form ? atoi(form) == 256 : getenv("ZGPT2_LM_STREAM") ? false : stream_fits(L) ? fine >= 640 * ((tiles + 255) / 256) : tiles >= 112;
     GemmPlanes pl{};
     pl.lda = L.lda;
     pl.ldb = L.ldb;
@@ -923,8 +886,7 @@ bool takes_persistent(const Linear& L) {
     return !L.grp_off && !L.z_group && L.nz == 1 && !L.a_rows && L.a_div == 1 && (L.act == ACT_NONE || L.act == ACT_RELU2) && one_result && L.K >= 128 && L.K % 64 == 0 && L.lda % 8 == 0 &&
            L.ldb % 8 == 0 && L.lda >= L.K && L.ldc >= L.N && (L.C || (L.N % 8 == 0 && L.ldc % 8 == 0)) && gemm_s4_args_ok(pl, L.ldc) &&
            ((reinterpret_cast<uintptr_t>(L.A16) | reinterpret_cast<uintptr_t>(L.B) | reinterpret_cast<uintptr_t>(L.C) | reinterpret_cast<uintptr_t>(L.C16)) & 15) == 0 &&
-           (size_t)L.M * L.ldc * 4 < ((size_t)1 << 32) && (size_t)L.N * L.ldb < (1u << 30) && (size_t)L.M * L.lda < (1u << 30) &&
-           (long long)((L.M + 255) / 256) * ((L.N + 191) / 192) >= least;
+           (size_t)L.M * L.ldc * 4 < ((size_t)1 << 32) && (size_t)L.N * L.ldb < (1u << 30) && (size_t)L.M * L.lda < (1u << 30) && pays;
 }
 bool takes_k_split(const Linear& L) { return L.K >= 1536 && L.M <= 2 && L.nz <= 4; }
 }  // namespace
@@ -985,13 +947,17 @@ int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
 }
 }  // namespace
 
-int launch_linear_gated(const Linear& L, int F, int kind, float* h, hipStream_t s, bool* taken) {
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, hipStream_t s, bool* taken) {
     *taken = false;
-    if (F <= 0 || L.act != ACT_NONE || L.bias || kind == GLU_CLIPPED || L.M <= 0 || L.M > kGemvMaxRows || L.grp_off || L.a_glu ||
-        getenv("ZGPT2_LM_NO_ROWS") != nullptr)
-        return ZG_OK;
+    if (F <= 0 || L.act != ACT_NONE || L.bias || kind == GLU_CLIPPED || L.M <= 0 || L.a_glu) return ZG_OK;
     Linear g = L;
     g.N = 2 * F; g.glu_out = F; g.glu_kind = kind; g.C = h; g.C16 = nullptr; g.ldc = F; g.c_zoff = F;
+    if (h16) {  // prompt portions
+        g.C = nullptr;
+        g.C16 = h16;
+        return launch_stream(g, s, taken);
+    }
+    if (L.M > kGemvMaxRows || L.grp_off || getenv("ZGPT2_LM_NO_ROWS") != nullptr) return ZG_OK;
     return launch_rows(g, nullptr, s, taken);
 }
 
@@ -1051,7 +1017,13 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     ZG_REQUIRE(!(L.z_group && L.grp_off), ZG_ERR_ARG, "linear: a matrix per batch and row groups exclude each other");
     ZG_REQUIRE(L.z_limit == 0x7fffffff, ZG_ERR_ARG, "linear: skipped batches are for steps of few rows");
     const bool rounded = L.A16 && !f32;
-    if (rounded && takes_persistent(L)) {
+    const bool persistent = rounded && takes_persistent(L);
+    if (rounded && !persistent) {
+        bool taken = false;
+        ZG_TRY(launch_stream(L, s, &taken));
+        if (taken) return ZG_OK;
+    }
+    if (persistent) {
         GemmPlanes pl{};
         pl.lda = L.lda;
         pl.ldb = L.ldb;

@@ -98,6 +98,47 @@ __device__ __forceinline__ Planes8<NP> to_planes(const f32x4& a, const f32x4& b)
     return o;
 }
 
+// The tile of a workgroup: rows [m0, m_end) of A / C, columns from n0, the matrix.  Consecutive workgroups go to the eight XCDs in
+// turn, so the tile list is dealt in eight contiguous runs: the tiles of one run share their A rows in that XCD's L2.
+struct TileAt {
+    const bf16_t* B;
+    int m0, m_end, n0;
+};
+__device__ __forceinline__ bool find_tile(const LinArgs& p, int N, int BM, int BN, TileAt& t) {
+    const int n_tiles = (N + BN - 1) / BN, total = gridDim.x, id = blockIdx.x;
+    const int q = total >> 3, r = total & 7, x = id & 7;
+    const int at = x * q + min(x, r) + (id >> 3);
+    int mt = at / n_tiles;
+    t.n0 = (at - mt * n_tiles) * BN;
+    t.B = p.B + (long long)blockIdx.z * p.b_zoff;
+    t.m0 = mt * BM;
+    t.m_end = p.M;
+    if (p.grp_off) {  // the row group this tile belongs to: 64 groups' tile counts summed across the lanes at a time
+        const int lane = threadIdx.x & 63;
+        for (int e0 = 0;; e0 += 64) {
+            if (e0 >= p.n_groups) return false;
+            const int e = min(e0 + lane, p.n_groups - 1);
+            const int lo = p.grp_off[e], hi = p.grp_off[e + 1];
+            const int own = e0 + lane < p.n_groups ? (hi - lo + BM - 1) / BM : 0;
+            int upto = own;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const int o = __shfl_up(upto, d, 64);
+                if (lane >= d) upto += o;
+            }
+            const unsigned long long past = __ballot(mt < upto);
+            if (past) {
+                const int l = __builtin_ctzll(past);
+                t.B = p.B + (long long)(e0 + l) * p.b_zoff;
+                t.m0 = __shfl(lo, l, 64) + (mt - __shfl(upto - own, l, 64)) * BM;
+                t.m_end = __shfl(hi, l, 64);
+                break;
+            }
+            mt -= __shfl(upto, 63, 64);
+        }
+    }
+    return t.m0 < t.m_end;
+}
 inline LinArgs make_args(const Linear& L) {
     LinArgs p;
     p.A = L.A; p.B = L.B; p.C = L.C; p.a_rows = L.a_rows; p.z_group = L.z_group; p.grp_off = L.grp_off;
@@ -141,6 +182,9 @@ __device__ __forceinline__ void move_tails(const TailArgs& t) {
 
 // lm_rows.hip: steps of 3 to 8 rows on the matrix cores.  *taken = false: not a form it has (nothing launched).
 int launch_rows(const Linear& a, const Linear* b, hipStream_t s, bool* taken);
+// lm_stream.hip: rounded rows of prompt portions.  *taken as above.
+bool stream_fits(const Linear& L);
+int launch_stream(const Linear& a, hipStream_t s, bool* taken);
 // lm_gemv.hip: steps of one or two rows whose operands are whole 16-byte pieces.  *taken as above.
 int launch_gemv_at_once(const Linear& a, const Linear* b, const NormIn* norm, hipStream_t s, bool* taken);
 
