@@ -34,16 +34,6 @@ typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-// four consecutive values -> 8 B into each of the kSplit planes (plane stride `plane` elements); the split
-// is exact: x = hi + mid + lo (zg_common.h split3_pk)
-__device__ __forceinline__ void store_split4(bf16_t* dst, size_t plane, f32x4 v) {
-    uint32_t a[3], b[3];
-    split3_pk(v.x, v.y, a[0], a[1], a[2]);
-    split3_pk(v.z, v.w, b[0], b[1], b[2]);
-#pragma unroll
-    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{a[p], b[p]};
-}
-
 // ------------------------------------------------------------------------------------------ embed
 __global__ __launch_bounds__(256) void embed_prefill_kernel(const int* __restrict__ tokens, int token_stride, int P,
                                                             const void* __restrict__ wte, const void* __restrict__ wpe,
@@ -111,12 +101,6 @@ constexpr int lds_bytes(int ns) { return kStages * stage_bytes(ns); }  // 128 / 
 __device__ __forceinline__ bf16x8 read_frag(const char* lds_tile, int row, int chunk) {
     const int off = row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
     return *reinterpret_cast<const bf16x8*>(lds_tile + off);
-}
-
-__device__ __forceinline__ float gelu_fast(float x) {
-    const float k1 = -2.0f * 1.4426950408889634f * 0.7978845608f, k2 = k1 * 0.044715f;
-    const float arg = x * fmaf(x * x, k2, k1);
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
 }
 
 // A: [M][3K] bf16 (hi | mid | lo), B: [N][K] bf16, bias [N].  C: fp32 [M][ldc] (PF_F32, PF_RESID) or bf16
@@ -654,7 +638,7 @@ int launch_ln_split(const float* x, int M, int E, const float* g, const float* b
 // N = n_embed Linears (residual adds) get there by slicing K over the tile list, their partial slabs summed by the reduce
 // kernels above in fixed order (which also apply bias, residual and the LayerNorm + split that follows).  Returns the slice
 // count, 0 = the 128-row kernels of this file take the launch.
-static int g_force_kernel = 0, g_force_slices = 0;  // zg_debug_prefill_route / _linear: 1 = gemm_s4, 2 = the 128-row kernels; K slices
+static int g_force_kernel = 0, g_force_slices = 0;  // zg_debug_prefill_route / _linear: 1 = gemm_s4, 2 = the 128-row kernels, 3 = prefill_ring; K slices
 void prefill_force_route(int kernel, int slices) {
     g_force_kernel = kernel;
     g_force_slices = slices;
@@ -688,6 +672,20 @@ static int s4_route(int M, int N, int K, int epi, size_t ws_floats, bool have_ws
     return best;
 }
 
+// the second half of a residual Linear whose product lies in K-slice slabs of ws: their sum, bias and residual (C [M][N]), and the LayerNorm behind it
+static int finish_resid(const float* ws, int n_sp, const float* bias, void* C, int M, int N, int ldc, const PrefillLn* ln, hipStream_t s) {
+    if (ln && N <= 2048) {
+        hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, n_sp, bias, reinterpret_cast<float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out);
+        ZG_HIP(hipGetLastError());
+        return ZG_OK;
+    }
+    const size_t n = (size_t)M * (N / 4);
+    hipLaunchKernelGGL((prefill_reduce_kernel<PF_RESID>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, n_sp, bias, C, M, N, ldc, PrefillQkv{});
+    ZG_HIP(hipGetLastError());
+    if (ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, s);
+    return ZG_OK;
+}
+
 int launch_prefill_gemm(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc, int epi,
                         float* ws, size_t ws_floats, const PrefillLn* ln, hipStream_t s, const PrefillQkv* qkv, int nsplit) {
     ZG_REQUIRE(M > 0 && N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0, ZG_ERR_UNSUPPORTED, "prefill gemm: M=%d N=%d K=%d", M, N, K);
@@ -695,21 +693,19 @@ int launch_prefill_gemm(const bf16_t* A, const bf16_t* B, const float* bias, voi
         const int n_sl = s4_route(M, N, K, epi, ws_floats, ws != nullptr);
         if (n_sl > 0 && epi == PF_RESID && ldc == N) {
             ZG_TRY(launch_gemm_s4_prefill(A, B, nullptr, ws, M, N, K, nsplit, S4_PARTIAL, n_sl, nullptr, s));
-            if (ln && N <= 2048) {
-                hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, n_sl, bias, reinterpret_cast<float*>(C), M, N, ln->g,
-                                   ln->b, ln->eps, ln->out);
-                ZG_HIP(hipGetLastError());
-                return ZG_OK;
-            }
-            const size_t n = (size_t)M * (N / 4);
-            hipLaunchKernelGGL((prefill_reduce_kernel<PF_RESID>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, n_sl, bias, C, M, N, ldc,
-                               PrefillQkv{});
-            ZG_HIP(hipGetLastError());
-            if (ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, s);
-            return ZG_OK;
+            return finish_resid(ws, n_sl, bias, C, M, N, ldc, ln, s);
         }
         if (n_sl == 1 && epi == PF_GELU_SPLIT) return launch_gemm_s4_prefill(A, B, bias, C, M, N, K, nsplit, S4_SPLIT3, 1, nullptr, s);
         if (n_sl == 1 && epi == PF_QKV && qkv && ldc == N) return launch_gemm_s4_prefill(A, B, bias, C, M, N, K, nsplit, S4_QKV, 1, qkv, s);
+    }
+    if (g_force_kernel == 0 || g_force_kernel == 3) {  // prompts of some hundred rows (prefill_ring.hip)
+        int tm = 1;
+        const bool planes = nsplit == kWeightPlanes, resid = epi == PF_RESID;
+        const int n_sp = (nsplit == kSplit || planes) && (!resid || (ldc == N && ws)) ? prefill_ring_route(M, N, K, resid, planes, ws_floats, g_force_kernel == 3, &tm) : 0;
+        if (n_sp > 0 && (size_t)N * K * 2 * 3 < ((size_t)1 << 31) && (size_t)M * kSplit * K * 2 < ((size_t)1 << 31)) {
+            ZG_TRY(launch_prefill_ring(A, B, bias, resid ? static_cast<void*>(ws) : C, M, N, K, ldc, resid ? PF_PARTIAL : epi, planes, tm, n_sp, qkv ? *qkv : PrefillQkv{}, s));
+            return resid ? finish_resid(ws, n_sp, bias, C, M, N, ldc, ln, s) : ZG_OK;
+        }
     }
     // (the operands are addressed through 32-bit buffer descriptors; a piece is switched off by adding 2 GiB to its scalar offset,
     // which must then lie past the descriptor's end without wrapping: operands < 2 GiB.  That a raw buffer access is range-checked

@@ -1,8 +1,24 @@
-// prefill_epi.h — device helpers shared by the epilogues of the whole-prompt Linears (prefill.hip, gemm_s4.hip).
+// prefill_epi.h — device helpers shared by the epilogues of the whole-prompt Linears (prefill.hip, prefill_ring.hip, gemm_s4.hip).
 #pragma once
 #include "zg_kernels.h"
 
 namespace zg {
+
+// four consecutive values -> 8 B into each of the kSplit planes (plane stride `plane` elements); the split
+// is exact: x = hi + mid + lo (zg_common.h split3_pk)
+__device__ __forceinline__ void store_split4(bf16_t* dst, size_t plane, f32x4 v) {
+    uint32_t a[3], b[3];
+    split3_pk(v.x, v.y, a[0], a[1], a[2]);
+    split3_pk(v.z, v.w, b[0], b[1], b[2]);
+#pragma unroll
+    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{a[p], b[p]};
+}
+
+__device__ __forceinline__ float gelu_fast(float x) {
+    const float k1 = -2.0f * 1.4426950408889634f * 0.7978845608f, k2 = k1 * 0.044715f;
+    const float arg = x * fmaf(x * x, k2, k1);
+    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(arg));
+}
 
 // Cache append (src/ops.zig:152-157) of four consecutive values of one K or V row into the head-major caches [b][h][ctx][64]:
 // element offset `off` = ((b H + head) ctx + t) 64 + d, in the cache's storage form (fp32, fp16 saturating, or the 24-bit pair of

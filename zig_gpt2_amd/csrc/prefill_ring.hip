@@ -1,0 +1,263 @@
+// prefill_ring.hip — the Linears of the whole-prompt pass (src/ops.zig:21-46 for M = batch x prompt rows) where the large tiles leave the chip
+// idle: prompts of some hundred rows.
+//
+// A = the activation planes [M][3 K] (hi | mid | lo), W = the bf16 weight [N][K], or the three plane matrices [3][N][K] of an fp32 weight.  All the
+// products of a K step of 64 columns are made from ONE staging of the planes (three, or the six above 2^-24 of the leading one), where
+// the 128-row kernels of prefill.hip walk an fp32 weight in three passes that each stage the activations again and meet in slabs.
+// What bounds it: a compute unit takes in some 30 bytes a clock (48 KB a step of a 64 x 64 tile of six products: 1600 clocks, beside 768 of
+// products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
+// K steps; a step costs one barrier; its fragments were read beside the products of the step before.  The leading products have sums of
+// their own, so that the small ones are not rounded at their size.
+#include <algorithm>
+#include <type_traits>
+
+#include "prefill_epi.h"
+#include "zg_kernels.h"
+#include "zg_once.h"
+
+namespace zg {
+
+namespace {
+
+typedef __attribute__((address_space(3))) char* lds_at_t;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(16))) float f32x16;
+
+constexpr int kBk = 64, kRow = 128, kCh = 8;  // columns of K of a step; bytes and 16-byte chunks of a row of them
+
+// (written here, not by the builtin: the compiler would wait for every request in flight in front of any read of the LDS.  m0: the address of
+// the wave's 1 KB piece; the wait state is what a request needs behind a write of m0)
+__device__ __forceinline__ void dma_16(unsigned lds, const u32x4& rsrc, unsigned v_off, unsigned s_off) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(v_off), "s"(rsrc), "s"(s_off) : "memory", "m0");
+}
+template <int N>
+__device__ __forceinline__ void arrive() {  // N requests may be in flight; what was read of the LDS is here; every wave has come this far
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+__device__ __forceinline__ u32x4 rsrc_of(const void* base) {
+    const uint64_t a = reinterpret_cast<uint64_t>(base);
+    return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, 0x80000000u, 0x00020000u};
+}
+
+// 2 x 2 waves of TM x 1 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
+template <int EPI, int TM, int NW, int ST>
+__global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
+                                                              const PrefillQkv qa) {
+    constexpr int BM = 64 * TM, BN = 64, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = 3 * A_PLANE + NW * B_PLANE;
+    constexpr int REQ = 3 * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
+    extern __shared__ __attribute__((aligned(1024))) char s_ring[];
+    const unsigned lds0 = (unsigned)(unsigned long)(lds_at_t)s_ring;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wy = wave >> 1, wx = wave & 1;
+    // workgroups go round the eight XCDs: each gets a run of the tiles, row tiles of a column tile next to each other (the weights are read once)
+    const int tiles_m = (M + BM - 1) / BM, n_tiles = tiles_m * (N / BN), q8 = n_tiles >> 3, r8 = n_tiles & 7, xcd = blockIdx.x & 7;
+    const int tile = xcd * q8 + min(xcd, r8) + (int)(blockIdx.x >> 3);
+    const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
+    const int in_row = lane >> 3, chunk = (lane & 7) ^ in_row;  // (every eighth row the swizzle repeats)
+    const u32x4 ra = rsrc_of(A), rb = rsrc_of(W);
+    unsigned va[PA], vb[PB];
+#pragma unroll
+    for (int i = 0; i < PA; ++i) va[i] = (unsigned)min(m0 + (wave + 4 * i) * 8 + in_row, M - 1) * (unsigned)(kSplit * K) * 2u + chunk * 16u;  // (rows beyond the edge: never stored)
+#pragma unroll
+    for (int i = 0; i < PB; ++i) vb[i] = (unsigned)(n0 + (wave + 4 * i) * 8 + in_row) * (unsigned)K * 2u + chunk * 16u;
+    const int nk = K / kBk, t0 = nk * (int)blockIdx.y / n_sp, steps = nk * ((int)blockIdx.y + 1) / n_sp - t0;
+    auto request = [&](int slot, int s) {
+        const unsigned off = (unsigned)(t0 + min(s, steps - 1)) * kRow, to = lds0 + slot * SLOT + wave * 1024;
+#pragma unroll
+        for (int p = 0; p < 3; ++p)
+#pragma unroll
+            for (int i = 0; i < PA; ++i) dma_16(to + p * A_PLANE + i * 4096, ra, va[i], off + (unsigned)p * (unsigned)K * 2u);
+#pragma unroll
+        for (int p = 0; p < NW; ++p)
+#pragma unroll
+            for (int i = 0; i < PB; ++i) dma_16(to + 3 * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
+    };
+    f32x16 lead[TM], small[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) lead[i][e] = small[i][e] = 0.0f;
+    const int fr = lane & 31, kh = lane >> 5, fswz = fr & 7;
+    u32x4 af[2][kCh / 2][3][TM], bf[2][kCh / 2][NW];  // of the step that is multiplied, and of the one behind it on its way
+    auto read = [&](auto b, int slot) {
+        const char* base = s_ring + slot * SLOT;
+#pragma unroll
+        for (int kk = 0; kk < kCh / 2; ++kk) {
+            const int c = ((2 * kk + kh) ^ fswz) * 16;
+#pragma unroll
+            for (int p = 0; p < NW; ++p) bf[b][kk][p] = *reinterpret_cast<const u32x4*>(base + 3 * A_PLANE + p * B_PLANE + (wx * 32 + fr) * kRow + c);
+#pragma unroll
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) af[b][kk][p][i] = *reinterpret_cast<const u32x4*>(base + p * A_PLANE + ((wy * TM + i) * 32 + fr) * kRow + c);
+        }
+    };
+    // (the operands change places: an accumulator's registers are then runs of four columns of a row)
+    auto multiply = [&](auto b) {
+        auto one = [&](f32x16& acc, int kk, int pa, int pw, int i) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bf[b][kk][pw]), __builtin_bit_cast(bf16x8, af[b][kk][pa][i]), acc, 0, 0, 0);
+        };
+#pragma unroll
+        for (int kk = 0; kk < kCh / 2; ++kk)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) {  // the smallest first
+                one(small[i], kk, 2, 0, i);
+                if constexpr (NW == 3) {
+                    one(lead[i], kk, 0, 0, i);
+                    one(small[i], kk, 1, 1, i);
+                    one(small[i], kk, 0, 2, i);
+                    one(small[i], kk, 1, 0, i);
+                    one(small[i], kk, 0, 1, i);
+                } else {
+                    one(lead[i], kk, 0, 0, i);
+                    one(small[i], kk, 1, 0, i);
+                }
+            }
+    };
+#pragma unroll
+    for (int s = 0; s < ST; ++s) request(s, s);
+    if (EPI == PF_QKV) {  // the epilogue's arguments, fetched under the first requests
+        ZG_PIN(qa.P); ZG_PIN(qa.E); ZG_PIN(qa.H); ZG_PIN(qa.ctx); ZG_PIN(qa.kv_mode); ZG_PIN(qa.kv_lo); ZG_PIN(qa.k_cache); ZG_PIN(qa.v_cache);
+    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), said to the compiler: with scalar loads in flight it would wait for all fragments at once
+    arrive<(ST - 1) * REQ>();
+    read(std::integral_constant<int, 0>(), 0);
+    int slot = 0, s = 0;
+    // Step s: its fragments have been read, so its slot takes step s + ST; those of s + 1 are read beside its products.
+    auto body = [&](auto b) {
+        constexpr int other = 1 - decltype(b)::value;
+        arrive<(ST - 2) * REQ>();
+        request(slot, s + ST);
+        slot = slot == ST - 1 ? 0 : slot + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        read(std::integral_constant<int, other>(), slot);
+        multiply(b);
+        constexpr int products = kCh / 2 * TM * (NW == 3 ? 6 : 3), reads = kCh / 2 * (3 * TM + NW);
+#pragma unroll
+        for (int x = 0; x < products; ++x) {
+            __builtin_amdgcn_sched_group_barrier(0x100, (reads + products - 1) / products, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        ++s;
+    };
+    for (int pairs = steps >> 1; pairs > 0; --pairs) {
+        body(std::integral_constant<int, 0>());
+        body(std::integral_constant<int, 1>());
+    }
+    if (steps & 1) body(std::integral_constant<int, 0>());
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the requests behind the last step still write the ring)
+
+    // element e of a 32 x 32 tile: column 8 (e / 4) + 4 (lane / 32) + e % 4, row lane % 32.  Every wave turns its rows in an image of its own
+    // (its accesses to the LDS are in order), so that eight lanes store 128 bytes of a row.
+    constexpr int PITCH = 32 * 4 + 16;
+    static_assert(4 * 32 * PITCH <= SLOT, "the images fit the ring");
+    char* img = s_ring + wave * 32 * PITCH;
+    const int cc = (lane & 7) * 4, n = n0 + wx * 32 + cc;
+    const f32x4 bv = EPI != PF_PARTIAL && bias ? *reinterpret_cast<const f32x4*>(bias + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            f32x4 v;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = lead[i][4 * g + e] + small[i][4 * g + e];
+            *reinterpret_cast<f32x4*>(img + fr * PITCH + (8 * g + 4 * kh) * 4) = v;
+        }
+#pragma unroll
+        for (int r8i = 0; r8i < 4; ++r8i) {
+            const int r = 8 * r8i + (lane >> 3), m = m0 + (wy * TM + i) * 32 + r;
+            f32x4 v = *reinterpret_cast<const f32x4*>(img + r * PITCH + cc * 4) + bv;
+            if (m >= M) continue;
+            if constexpr (EPI == PF_GELU_SPLIT) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = gelu_fast(v[e]);
+                store_split4(reinterpret_cast<bf16_t*>(C) + (size_t)m * kSplit * N + n, N, v);
+            } else if constexpr (EPI == PF_PARTIAL) {  // C: slabs [n_sp][M][N]
+                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)blockIdx.y * M + m) * N + n) = v;
+            } else {
+                *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + (size_t)m * ldc + n) = v;
+                if constexpr (EPI == PF_QKV) qkv_cache_store(qa, m, n, v);
+            }
+        }
+    }
+}
+
+template <int EPI, int TM, int NW, int ST>
+int launch_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, hipStream_t s) {
+    constexpr int LDS = ST * (3 * 64 * TM + NW * 64) * kRow;
+    static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
+    static OncePerDevice raised;
+    int device = 0;
+    ZG_HIP(hipGetDevice(&device));
+    ZG_TRY(raised.run(device, []() -> int {
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_ring_kernel<EPI, TM, NW, ST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        return ZG_OK;
+    }));
+    const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * (N / 64);
+    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A, W, bias, C, M, N, K, ldc, n_sp, qa);
+    note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+template <int EPI>
+int launch_ring_epi(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, bool planes, int tm, int n_sp, const PrefillQkv& qa,
+                    hipStream_t s) {
+    if (planes) return tm == 1 ? launch_ring<EPI, 1, 3, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s) : launch_ring<EPI, 2, 3, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s);
+    return tm == 1 ? launch_ring<EPI, 1, 1, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s) : launch_ring<EPI, 2, 1, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s);
+}
+
+}  // namespace
+
+// K slices of the launch (1 unless it is a residual Linear, whose slices meet in slabs) and rows of a tile (64 tm); 0: the 128-row kernels take it.
+// Both sides are priced in us by what one compute unit takes in (65 bytes a ns; 57 with the weight's planes; 42 where two slots of 56 KB are
+// the whole ring), 3 us for each round of workgroups, and slabs at 4 TB/s.  At K = 768, bf16: 300 x 3072 predicts 9 here and 14 there
+// (measured 10.5 and 16.6), 800 x 3072 41 and 15 (31.7, 20.4); K = 3072: 300 x 768 10 and 13 (14.3, 16.1), 800 x 768 28 and 18 (27.6, 24.7);
+// fp32 weights: 300 x 3072 13 and 34 (14.5, 27.5), 1000 x 768 x 3072 36 and 62 (41, 51), 1600 x 768 x 3072 66 and 68 (68.5, 62.8).
+// bf16: beyond a few hundred rows what wins by less than a microsecond is lost again in the reduce kernel behind it, which finds one slab where
+// it found several (a whole prompt of 4 x 200 rows of 768 columns: 1377 us against 1359, 8 x 255 of 384: 600 against 588).
+int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm) {
+    if (!planes && M > 700 && !force) return 0;
+    const int nk = K / kBk;
+    const double slab = (double)M * N * 8.0 / 4e6;
+    auto rounds = [](long n) { return (double)((n + 255) / 256); };
+    int best = 0;
+    double best_us = 0.0;
+    for (int t = 1; t <= 2; ++t) {
+        const long tiles = (long)((M + 64 * t - 1) / (64 * t)) * (N / 64);
+        int n_sp = resid ? (int)std::max(1l, std::min(256 / tiles, (long)nk / 3)) : 1;
+        while (resid && n_sp > 1 && (size_t)n_sp * M * N > ws_floats) --n_sp;
+        if (resid && (size_t)n_sp * M * N > ws_floats) continue;
+        const double us = rounds(tiles * n_sp) * (3.0 + ((nk + n_sp - 1) / n_sp) * (planes ? (24.0 * t + 24.0) / 57.0 : t == 1 ? 32.0 / 65.0 : 56.0 / 42.0)) + (resid ? n_sp * slab : 0.0);
+        if (best == 0 || us < best_us) {
+            best = n_sp;
+            best_us = us;
+            *tm = t;
+        }
+    }
+    if (best == 0 || force) return best;
+    const bool wide = (long)((M + 127) / 128) * ((N + 255) / 256) >= 256;
+    const int bn = wide ? 256 : 128;
+    const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
+    const int passes = planes ? 3 : 1;
+    const int n_sp = (int)std::max(1l, std::min(planes ? (256 + 3 * tiles - 1) / (3 * tiles) : 256 / tiles, (long)nk / 3));
+    const double us = rounds(tiles * n_sp * passes) * (3.0 + ((nk + n_sp - 1) / n_sp) * (48.0 + bn / 8.0) / 65.0) +
+                      (resid || n_sp * passes > 1 ? n_sp * passes * slab : 0.0) + (!resid && n_sp * passes > 1 ? 3.0 : 0.0);
+    return best_us + (planes || M <= 256 ? 0.0 : 1.0) <= us ? best : 0;
+}
+
+int launch_prefill_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, bool planes, int tm, int n_sp, const PrefillQkv& qa,
+                        hipStream_t s) {
+    ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kSplit * K * 2 < ((size_t)1 << 31) &&
+                   (size_t)N * K * 2 * (planes ? 3 : 1) < ((size_t)1 << 31),
+               ZG_ERR_UNSUPPORTED, "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
+    switch (epi) {
+        case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
+        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, planes, tm, n_sp, qa, s);
+        case PF_GELU_SPLIT: return launch_ring_epi<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
+        case PF_QKV: return launch_ring_epi<PF_QKV>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
+    }
+    ZG_REQUIRE(false, ZG_ERR_ARG, "prefill gemm: epilogue %d", epi);
+}
+
+}  // namespace zg

@@ -254,6 +254,10 @@ int launch_prefill_gemm(const bf16_t* A, const bf16_t* W, const float* bias, voi
                         int nsplit = kSplit);  // nsplit = 2: multiply the hi + mid planes only (2/3 of the matrix work);
                                                // kWeightPlanes: W is the plane-major three-term split [3][N][K] of an fp32 matrix
 constexpr int kWeightPlanes = 33;
+// prefill_ring.hip: whole-prompt Linears of some hundred rows.  The route: K slices (slabs of a residual Linear, else 1), 0 = not taken; tm: rows / 64 of a tile.
+int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
+int launch_prefill_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, bool planes, int tm, int n_sp, const PrefillQkv& qa,
+                        hipStream_t s);
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels) and the K slices
 // out[M][kSplit E] = split(causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t)
 // (attn_prefill.hip: bf16 matrix cores on exact plane splits; ws = fp32 workspace for the partials of split key ranges)
