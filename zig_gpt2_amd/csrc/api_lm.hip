@@ -1014,7 +1014,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
         bool activated = false;
         if (!first_done) {
             Linear up = dense_up(L, in, in16);
-            if (gated && few && M > 2) ZG_TRY(launch_linear_gated(up, F, GLU_GELU, g->hb, nullptr, s, &activated));
+            if (gated && few && M > 2) ZG_TRY(launch_linear_gated(up, F, GLU_GELU, g->hb, nullptr, f32, s, &activated));
             if (u16 && !poly && !gated && whole(W)) up.C16 = u16, up.C = nullptr;
             if (!activated) ZG_TRY(hidden_product(up));
         }
@@ -1042,7 +1042,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
     auto expert_first = [&](const Linear& up, Linear& dn, int F, int NA, bool glu) -> int {
         bf16_t* const hb16 = r16 && whole(F) ? g->u16 : nullptr;
         bool gated = false;
-        if (glu && (few || (hb16 && up.A16))) ZG_TRY(launch_linear_gated(up, F, GLU_SILU, g->hb, few ? nullptr : hb16, s, &gated));
+        if (glu && (few || f32 || (hb16 && up.A16))) ZG_TRY(launch_linear_gated(up, F, GLU_SILU, g->hb, few ? nullptr : hb16, f32, s, &gated));
         if (!gated) ZG_TRY(launch_linear(up, f32, s));
         if (!glu) {  // the first product's epilogue has applied its activation
             dn.A = g->gu_buf; dn.lda = F;

@@ -66,9 +66,9 @@ struct Linear {
     int n_groups = 0;
     int glu_out = 0;  // set by launch_linear_gated: B rows are [gate (glu_out) | up (glu_out)], N both, and the activated rows leave (glu_kind)
 };
-// Steps of few rows: the first product of a gated feed-forward with the activation in its epilogue, h [rows][F] = act(gate) * up for B rows
+// The first product of a gated feed-forward with the activation in its epilogue, h (steps, or h16) [rows][F] = act(gate) * up for B rows
 // [gate (F) | up (F)]; L as for launch_linear, its C, ldc, c_zoff and N ignored.  *taken = false: not a form that has it, nothing launched.
-int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, hipStream_t s, bool* taken);
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, bool f32, hipStream_t s, bool* taken);
 // What launch_norm_add_norm does, inside the product that reads the row: x_out = x + norm(y) (1 + wb), and the product's row is
 // norm(x_out) (1 + wn).  x_out must not be x (every workgroup reads x, one writes x_out).
 struct NormIn {

@@ -6,7 +6,7 @@
 //   * lm_gemv_kernel   (long rows: lm_gemv_ks_kernel) a wave owns two weight rows, its lanes split K in 16-byte pieces, the
 //                      activation rows come straight from the cache hierarchy, sums are fp32 FMAs in both precision modes.
 //   * gemm_s4_kernel   (gemm_s4.hip) plain products of prompt portions whose rows are rounded already, where they fill the chip several times.
-//   * lm_stream_kernel (lm_stream.hip) the other products of rounded rows whose K is whole steps of 64, experts' among them.
+//   * lm_stream_kernel (lm_stream.hip) the other products of rounded rows, and those of 32-bit mode, whose K is whole steps of 64, experts' among them.
 //   * lm_wide_kernel   prompt portions that fill the chip: 128 x 128 or 64 x 64 tiles staged through the LDS.
 //   * lm_deep_kernel   short portions: 32-wide tiles with K split over the waves of a workgroup.
 //                      Both multiply with v_mfma_f32_32x32x16_bf16: bf16 mode rounds the activations on their way there, 32-bit mode
@@ -876,7 +876,7 @@ namespace {
 bool takes_persistent(const Linear& L) {
     const char* form = getenv("ZGPT2_LM_GEMM_TILE");  // test hook: 256 = here at any number of tiles, another = never
     const long long tiles = (long long)((L.M + 255) / 256) * ((L.N + 191) / 192), fine = (long long)((L.M + 127) / 128) * ((L.N + 127) / 128);
-    const bool pays = form ? atoi(form) == 256 : getenv("ZGPT2_LM_STREAM") ? false : stream_fits(L) ? fine >= 640 * ((tiles + 255) / 256) : tiles >= 112;
+    const bool pays = form ? atoi(form) == 256 : getenv("ZGPT2_LM_STREAM") ? false : stream_fits(L, false) ? fine >= 640 * ((tiles + 255) / 256) : tiles >= 112;
     GemmPlanes pl{};
     pl.lda = L.lda;
     pl.ldb = L.ldb;
@@ -947,17 +947,16 @@ int launch_tiles(const Linear& L, const LinArgs& p, hipStream_t s) {
 }
 }  // namespace
 
-int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, hipStream_t s, bool* taken) {
+int launch_linear_gated(const Linear& L, int F, int kind, float* h, bf16_t* h16, bool f32, hipStream_t s, bool* taken) {
     *taken = false;
     if (F <= 0 || L.act != ACT_NONE || L.bias || kind == GLU_CLIPPED || L.M <= 0 || L.a_glu) return ZG_OK;
     Linear g = L;
     g.N = 2 * F; g.glu_out = F; g.glu_kind = kind; g.C = h; g.C16 = nullptr; g.ldc = F; g.c_zoff = F;
-    if (h16) {  // prompt portions
-        g.C = nullptr;
-        g.C16 = h16;
-        return launch_stream(g, s, taken);
+    if (L.M > kGemvMaxRows || L.grp_off) {  // prompt portions
+        if (h16) g.C = nullptr, g.C16 = h16;
+        return launch_stream(g, f32, s, taken);
     }
-    if (L.M > kGemvMaxRows || L.grp_off || getenv("ZGPT2_LM_NO_ROWS") != nullptr) return ZG_OK;
+    if (getenv("ZGPT2_LM_NO_ROWS") != nullptr) return ZG_OK;
     return launch_rows(g, nullptr, s, taken);
 }
 
@@ -1018,9 +1017,12 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     ZG_REQUIRE(L.z_limit == 0x7fffffff, ZG_ERR_ARG, "linear: skipped batches are for steps of few rows");
     const bool rounded = L.A16 && !f32;
     const bool persistent = rounded && takes_persistent(L);
-    if (rounded && !persistent) {
+    // (32-bit products of a few columns exist in toy models only.  There the last bits of a sum that cancels almost entirely can decide a
+    // row, and they stay what the fp32 instruction makes them: 5.5 us against 3.4 at K = 64.)
+    const bool toy = f32 && L.K < 128 && L.nz == 1;
+    if (!persistent && !toy) {
         bool taken = false;
-        ZG_TRY(launch_stream(L, s, &taken));
+        ZG_TRY(launch_stream(L, f32, s, &taken));
         if (taken) return ZG_OK;
     }
     if (persistent) {
@@ -1034,9 +1036,6 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
         return launch_gemm_s4(L.A16, L.B, L.bias, L.C ? static_cast<void*>(L.C) : L.C16, L.M, L.N, pl, L.ldc, false, L.C == nullptr, 192, s);
     }
     const bool a_vec = rounded ? (reinterpret_cast<uintptr_t>(L.A16) & 15) == 0 && L.lda % 8 == 0 && L.a_zoff % 8 == 0 : p.a_vec != 0;
-    // (32-bit products of a few columns exist in toy models only.  There the last bits of a sum that cancels almost entirely can decide a
-    // row, and they stay what the fp32 instruction makes them: 5.5 us against 3.4 at K = 64.)
-    const bool toy = f32 && L.K < 128 && L.nz == 1;
     if (a_vec && p.b_vec && L.K % 8 == 0 && !L.z_group && !toy) {
         if (f32) return launch_tiles<float, 3>(L, p, s);
         return rounded ? launch_tiles<bf16_t, 1>(L, p, s) : launch_tiles<float, 1>(L, p, s);

@@ -182,9 +182,9 @@ __device__ __forceinline__ void move_tails(const TailArgs& t) {
 
 // lm_rows.hip: steps of 3 to 8 rows on the matrix cores.  *taken = false: not a form it has (nothing launched).
 int launch_rows(const Linear& a, const Linear* b, hipStream_t s, bool* taken);
-// lm_stream.hip: rounded rows of prompt portions.  *taken as above.
-bool stream_fits(const Linear& L);
-int launch_stream(const Linear& a, hipStream_t s, bool* taken);
+// lm_stream.hip: prompt portions whose K is whole steps of 64.  *taken as above.
+bool stream_fits(const Linear& L, bool f32);
+int launch_stream(const Linear& a, bool f32, hipStream_t s, bool* taken);
 // lm_gemv.hip: steps of one or two rows whose operands are whole 16-byte pieces.  *taken as above.
 int launch_gemv_at_once(const Linear& a, const Linear* b, const NormIn* norm, hipStream_t s, bool* taken);
 
