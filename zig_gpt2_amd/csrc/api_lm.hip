@@ -1394,7 +1394,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             // (portions on the tiled attention: its queries and results rounded, in the place of the fp32 rows)
             const bool tiles = r16 && g->key_tiles && latent_tile_elems(KR, R) > 0 && g->step_key_tiles * latent_tile_elems(KR, R) <= g->key_tile_elems && n_ent <= 65535;
             bf16_t* const cq16 = r16 && whole(QR) ? reinterpret_cast<bf16_t*>(g->cq) : nullptr;
-            bf16_t* const qa16 = tiles && whole(KR) && whole(R) && whole(D) && (direct ? whole(LD) : true) && whole(D + R) ? reinterpret_cast<bf16_t*>(g->qa) : nullptr;
+            bf16_t* const qa16 = tiles && whole(KR) && whole(R) && whole(D) && (direct ? LD % 4 == 0 : true) && whole(D + R) ? reinterpret_cast<bf16_t*>(g->qa) : nullptr;
             bf16_t* const ctx16 = tiles && whole(KR) ? reinterpret_cast<bf16_t*>(g->ctx) : nullptr;
             bf16_t* const o16 = ctx16 && whole(HV) ? g->o16 : nullptr;
             const float* q = direct ? g->proj : g->q;
@@ -1421,9 +1421,11 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 if (queries) ZG_TRY(launch_latent_step(st, s, &stepped));
             }
             if (!stepped) {
+                bool absorbed = false;
                 if (direct) {
+                    if (qa16) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
                     ZG_TRY(launch_latent_direct_prep(g->proj, LD, M, H, D, R, KR, H * (D + R), L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages,
-                                                     g->P, g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, qa16));
+                                                     g->P, absorbed ? nullptr : g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, absorbed ? nullptr : qa16));
                 } else {
                     ZG_TRY(launch_latent_prep(g->proj, LD, M, QR, KR, R, L.dq_norm, L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages, g->P,
                                               g->cq, ps.cache, s, cq16));
@@ -1431,11 +1433,14 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                     lin.A = cq16 ? nullptr : g->cq; lin.A16 = cq16; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
                     ZG_TRY(launch_linear(lin, f32, s));
                 }
-                lin = Linear();  // the unrotated query part carried into the latent space, head by head
-                lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
-                lin.C = qa16 ? nullptr : g->qa; lin.C16 = qa16; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
-                ZG_TRY(launch_linear(lin, f32, s));
-                if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
+                if (qa16 && !direct) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
+                if (!absorbed) {
+                    lin = Linear();  // the unrotated query part carried into the latent space, head by head
+                    lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
+                    lin.C = qa16 ? nullptr : g->qa; lin.C16 = qa16; lin.ldc = H * (KR + R); lin.c_zoff = KR + R; lin.M = M; lin.N = KR; lin.K = D; lin.nz = H;
+                    ZG_TRY(launch_linear(lin, f32, s));
+                    if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
+                }
                 bool tiled = false;
                 if (!f32 && !few)
                     ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,

@@ -303,13 +303,16 @@ int launch_latent_prep(const float* proj, int ld, int M, int q_rank, int KR, int
                        float* cache, hipStream_t s, bf16_t* cq16 = nullptr);
 // Queries projected directly: proj rows [q (H (D + R)) | dkv latent (KR) | rotated key part (R) at column kv_col].  qa[m][h][KR ..] =
 // rotary(q[m][h][D ..]) and, with cache != null, the token's cache row as above — one launch.  cache == null: the layer reads another
-// layer's latents (no dkv columns).
+// layer's latents (no dkv columns).  qa, qa16 null: the cache row alone.
 int launch_latent_direct_prep(const float* proj, int ld, int M, int H, int D, int R, int KR, int kv_col, const float* wkv, float eps, Rotary rot,
                               const int* row_pos, const int* row_slot, const int* page_table, int max_pages, int page_tokens, float* qa, float* cache,
                               hipStream_t s, bf16_t* qa16 = nullptr);
 // qa[m][h][KR ..] = rotary(q[m][h][D ..]) — the rotated query part moved behind the absorbed part (which a batched Linear wrote).
 int launch_q_rotary(const float* q, int ldq, float* qa, int ldqa, int M, int H, int D, int R, int KR, Rotary rot, const int* row_pos, hipStream_t s,
                     bf16_t* qa16 = nullptr);
+// Both parts of the queries in one launch (bf16 mode, prompt portions): qa16[m][h][:KR] = q[m][h][:D] ukT[h]^T, qa16[m][h][KR ..] = rotary(q[m][h][D ..]).
+//  *taken = false: not a form it has, nothing launched.
+int launch_latent_queries(const float* q, int ldq, const bf16_t* ukT, bf16_t* qa16, int M, int H, int D, int R, int KR, const Rotary& rot, const int* row_pos, hipStream_t s, bool* taken);
 // ctx[m][h][:KR] = sum_j softmax_j( scale * qa[m][h] . cacherow(j) ) latent(j) over the keys j <= row_pos[m] of the row's sequence.
 // ws: fp32 workspace for the partials of split key ranges (steps of at most kGemvMaxRows rows: M * H * kAttnSplits * (KR + 2)
 // floats; without it whole key rows per workgroup).

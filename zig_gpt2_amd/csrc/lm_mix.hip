@@ -824,7 +824,7 @@ __global__ __launch_bounds__(256) void q_rotary_kernel(const float* q, int ldq, 
     }
 }
 
-// Queries projected directly: blockIdx.y == 0 rotates the heads' query parts into qa, blockIdx.y == 1 (layers with latents of their
+// Queries projected directly: blockIdx.y == 0 rotates the heads' query parts into qa (neither qa nor qa16: not asked for), blockIdx.y == 1 (layers with latents of their
 // own) norms the latent, rotates the shared key part and files both in the token's cache row.
 __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* proj, int ld, int H, int D, int R, int KR, int kv_col, const float* wkv,
                                                                  float eps, Rotary rot, const int* row_pos, const int* row_slot, const int* page_table,
@@ -832,7 +832,7 @@ __global__ __launch_bounds__(256) void latent_direct_prep_kernel(const float* pr
     __shared__ float s_red[8];
     const int m = blockIdx.x, pos = row_pos[m], half = rot.dims / 2;
     const float* row = proj + (size_t)m * ld;
-    if (blockIdx.y == 0) {
+    if (blockIdx.y == 0 && (qa || qa16)) {
         const int rest = R - rot.dims, per = half + rest;
         for (int idx = threadIdx.x; idx < H * per; idx += blockDim.x) {
             const int h = idx / per, i = idx % per;
@@ -1854,7 +1854,9 @@ int launch_latent_direct_prep(const float* proj, int ld, int M, int H, int D, in
                               hipStream_t s, bf16_t* qa16) {
     if (M <= 0) return ZG_OK;
     ZG_REQUIRE(rot.dims % 2 == 0 && rot.dims <= R, ZG_ERR_ARG, "rotary: %d rotated dimensions of a part of %d", rot.dims, R);
-    latent_direct_prep_kernel<<<dim3(M, cache ? 2 : 1), 256, 0, s>>>(proj, ld, H, D, R, KR, kv_col, wkv, eps, rot, row_pos, row_slot, page_table, max_pages,
+    const int parts = (qa || qa16 ? 1 : 0) + (cache ? 1 : 0);
+    if (parts == 0) return ZG_OK;
+    latent_direct_prep_kernel<<<dim3(M, parts), 256, 0, s>>>(proj, ld, H, D, R, KR, kv_col, wkv, eps, rot, row_pos, row_slot, page_table, max_pages,
                                                                      page_tokens, qa, cache, qa16);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
