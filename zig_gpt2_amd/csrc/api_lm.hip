@@ -1180,9 +1180,19 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 window_split_workspace(M, H, Vd, key_cap, &ws.n_split);
                 ZG_TRY(launch_window_step(ws, s, &done));
             }
+            bf16_t* o16 = r16 && whole(HV) ? g->o16 : nullptr;
+            bool rounded = false;
             if (!done) {
                 ZG_TRY(launch_window_prep(g->proj, LD, M, H, G, D, Vd, rot, nullptr, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache, s, vals));
-                if (d.sigmoid_weights) ZG_TRY(gated(nullptr));
+                if (o16 && !d.sigmoid_weights) {
+                    WindowStep ws;
+                    ws.q = g->proj; ws.ldq = LD; ws.ldo = HV; ws.M = M; ws.H = H; ws.G = G; ws.D = D; ws.V = Vd; ws.scale = d.scale; ws.mask = mask;
+                    ws.row_pos = d_pos; ws.row_slot = d_slot; ws.page_table = g->page_table; ws.max_pages = g->max_pages; ws.page_tokens = g->P; ws.cache = ps.cache;
+                    ZG_TRY(launch_window_rows(ws, d_estart, d_elen, n_ent, o16, s, &rounded));
+                    done = rounded;
+                }
+                if (done) {
+                } else if (d.sigmoid_weights) ZG_TRY(gated(nullptr));
                 else
                     ZG_TRY(launch_window_attention_split(g->proj, LD, g->o, HV, M, H, G, D, Vd, d.scale, mask, nullptr, nullptr, nullptr, d_pos, d_slot,
                                                          g->page_table, g->max_pages, g->P, ps.cache, key_cap, g->win_ws, g->win_ws_floats, d_estart,
@@ -1195,7 +1205,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                                                g->page_table, g->max_pages, g->P, ps.cache, s, shape));
             }
             lin = Linear();
-            lin.A = g->o; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
+            lin.A = rounded ? nullptr : g->o; lin.A16 = rounded ? o16 : nullptr; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             lin.bias = L.obias;
             ZG_TRY(launch_linear(lin, f32, s));
         } else if (d.mixer == ZG_LM_MIX_SSD) {

@@ -452,6 +452,9 @@ struct WindowStep {
     ScoreShape shape;
 };
 int launch_window_step(const WindowStep& a, hipStream_t s, bool* taken);
+// Prompt portions, no mixing matrix, values as they are, heads of whole pieces of eight channels up to 64 (values of four): the attention in one
+// launch without a workspace.  out16 != null: the rows rounded to bf16, in the place of out.  *taken = false: not a form it has, nothing launched.
+int launch_window_rows(const WindowStep& a, const int* ent_start, const int* ent_len, int n_entries, bf16_t* out16, hipStream_t s, bool* taken);
 
 size_t window_split_workspace(int rows, int H, int V, int key_capacity, int* n_split_out);
 int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, int M, int H, int G, int D, int V, float scale, KeyMask mask,

@@ -1421,12 +1421,13 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
     if (!ws || need > ws_floats || H > kWinMaxHeads || H % G != 0 || H * V > 256 * kWinAcc || D > 256 || (vfreq && V % 2 != 0) || lds_a > 60 * 1024 ||
         lds_b > 60 * 1024 || M > 65535)
         return ZG_OK;  // the general kernel takes it
-    if (!talk && !vfreq) {  // steps of few rows: scores, weights and values of a share in one launch
+    if (!talk && !vfreq) {  // steps of few rows: scores, weights and values of a share in one launch; portions: all of it
         WindowStep w;
         w.q = q; w.ldq = ldq; w.out = out; w.ldo = ldo; w.M = M; w.H = H; w.G = G; w.D = D; w.V = V; w.scale = scale; w.mask = mask; w.sink = sink; w.row_pos = row_pos;
         w.row_slot = row_slot; w.page_table = page_table; w.max_pages = max_pages; w.page_tokens = page_tokens; w.cache = const_cast<float*>(cache); w.n_split = n_split;
         w.ws = ws; w.ws_floats = ws_floats; w.out_gate = out_gate; w.ld_gate = ld_gate; w.out_factor = out_factor; w.shape = shape;
         ZG_TRY(launch_window_step(w, s, taken));
+        if (!*taken) ZG_TRY(launch_window_rows(w, ent_start, ent_len, n_entries, nullptr, s, taken));
         if (*taken) return ZG_OK;
     }
     float* sc = ws;
