@@ -1116,14 +1116,15 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     const int n_tiles = (pos_first + nq + 31) / 32;
     const char* src = reinterpret_cast<const char*>(tiles) + (size_t)at.first_tile * T::BYTES + lane * 16;
 
+    const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)&Ks[0][0];
     auto request = [&](int kt, int buf) {
         const char* g = src + (size_t)kt * T::BYTES;
 #pragma unroll
         for (int pc = 0; pc < (T::PIECES + 3) / 4; ++pc) {
             const int i = wave + 4 * pc;
+            // (written here, not by the builtin: the compiler would wait for the next tile in front of this tile's latent part)
             if (i < T::PIECES)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(g + i * 1024),
-                                                 (__attribute__((address_space(3))) void*)(Ks[buf] + i * 1024), 16, 0, 0);
+                asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds0 + buf * T::BYTES + i * 1024), "v"(g + i * 1024) : "memory", "m0");
         }
     };
     request(0, 0);
@@ -1178,7 +1179,8 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     const int v_hi = (8 + 4 * hf + (i16 >> 2)) * T::LD * 2 + ((vc ^ (hf + 2)) * 16) + (i16 & 1) * 8;
     typedef __attribute__((address_space(3))) s16x4* lds_s16x4_ptr;
 
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's pieces have landed
+    // vmcnt(0): this wave's pieces have landed; lgkmcnt(0), said to the compiler: with scalar loads in flight it would wait for all fragments at once
+    __builtin_amdgcn_s_waitcnt(0x0070);
     __syncthreads();
     for (int kt = 0; kt < n_tiles; ++kt) {
         const char* K = Ks[kt & 1];
