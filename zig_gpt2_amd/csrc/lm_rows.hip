@@ -34,6 +34,9 @@ __device__ __forceinline__ int nth_bit(unsigned long long m, int n) {  // positi
     return __builtin_ctzll(m);
 }
 
+template <int I>
+using step = std::integral_constant<int, I>;
+
 enum { ROWS_PLAIN, ROWS_GLU_ON_LOAD, ROWS_GLU_OUT, ROWS_RMS };
 // What the loads at entry need (leading arguments, see lm_gemv.hip).
 struct RowsAt {
@@ -44,24 +47,40 @@ struct RowsAt {
     const float* a_norm = nullptr;  // ROWS_RMS: the rows' norm weights
     float eps = 0.0f;
 };
-enum { FORM_PLAIN, FORM_LIST, FORM_ANY };  // rows and matrices in a row; a matrix per list entry; either, and rows through an array
-// TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight
-template <int TURNS, int KIND, int FORM>
+// rows and matrices in a row; a matrix per list entry; either, and rows through an array; a list of at least as many entries as there are matrices
+enum { FORM_PLAIN, FORM_LIST, FORM_ANY, FORM_FULL_LIST };
+// TURNS > 0: every wave's turns are at most TURNS, all in flight at once; 0: any number, four in flight.
+template <int TURNS, int KIND, int FORM, int WAVES = 4>
 __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, const int z, float (*part)[16][17]) {
+    // (nearly every matrix of a full list is somebody's: its rows are asked for in front of the list.  16 rows on 8 experts of 768 x 768: 6.5 us
+    // against 7.0.  Gated products, bound by the terms they make, gain nothing: 8.6 against 8.2)
+    constexpr bool EARLY = FORM == FORM_FULL_LIST && TURNS > 0;
     constexpr bool GLU = KIND == ROWS_GLU_ON_LOAD, OUT = KIND == ROWS_GLU_OUT, RMS = KIND == ROWS_RMS, ARRAY = FORM == FORM_ANY;
-    const bool list = FORM == FORM_LIST || (FORM == FORM_ANY && t.z_group != nullptr);
+    const bool list = FORM == FORM_LIST || FORM == FORM_FULL_LIST || (FORM == FORM_ANY && t.z_group != nullptr);
     // (gated products: eight gates and the eight values they gate)
     constexpr int half = OUT ? 8 : 16;
     const int n0 = blockIdx.x * half, n_out = OUT ? t.N / 2 : t.N;
     if (n0 >= n_out) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4, m = col & 7;
-    unsigned long long left = 0;  // assignments of this expert that are still to do
-    if (list) {
-        left = __ballot(lane < t.M && t.z_group[min(lane, t.M - 1)] == z);
-        if (left == 0) return;
-    }
     const int w_row = OUT ? (col & 8 ? n_out : 0) + min(n0 + (col & 7), n_out - 1) : min(n0 + col, t.N - 1);
     const bf16_t* w = t.B + (long long)z * t.b_zoff + (long long)w_row * t.ldb;
+    constexpr int RING = TURNS > 0 ? TURNS : 4;
+    u32x4 wr[RING][2];
+    auto fetch_w = [&](int slot, int turn) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wr[slot][j] = *reinterpret_cast<const u32x4*>(w + min(turn * kTurn + 16 * kg + 8 * j, t.K - 8));
+    };
+    unsigned long long left = 0;  // assignments of this expert that are still to do
+    if (list) {
+        const int mine = t.z_group[min(lane, t.M - 1)];
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int i = 0; i < TURNS; ++i) fetch_w(i, wave + WAVES * i);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        left = __ballot(lane < t.M && mine == z);
+        if (left == 0) return;
+    }
     do {
         const int n_rows = list ? min(8, __popcll(left)) : t.M;
         // (columns without a row compute on the last one's and are not stored)
@@ -70,15 +89,13 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         const float asc = GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
         const float agate = GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-a[p.glu_gate_col])) : 1.0f;
         const int n_turns = (t.K + kTurn - 1) / kTurn;
-        constexpr int RING = TURNS > 0 ? TURNS : 4;
-        u32x4 wr[RING][2];
         f32x4 ar[RING][4], ur[GLU || RMS ? RING : 1][4];
         float ss = 0.0f;  // (RMS) squares of the lane's share of its row
         auto fetch = [&](int slot, int turn) {
+            if constexpr (!EARLY) fetch_w(slot, turn);
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int k = min(turn * kTurn + 16 * kg + 8 * j, t.K - 8);
-                wr[slot][j] = *reinterpret_cast<const u32x4*>(w + k);
                 ar[slot][2 * j] = *reinterpret_cast<const f32x4*>(a + k);
                 ar[slot][2 * j + 1] = *reinterpret_cast<const f32x4*>(a + k + 4);
                 if constexpr (GLU || RMS) {  // the values a gate multiplies, or the norm's weights
@@ -122,17 +139,17 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         };
         if constexpr (TURNS > 0) {
 #pragma unroll
-            for (int i = 0; i < TURNS; ++i) fetch(i, wave + 4 * i);
+            for (int i = 0; i < TURNS; ++i) fetch(i, wave + WAVES * i);
 #pragma unroll
-            for (int i = 0; i < TURNS; ++i) multiply(i, wave + 4 * i);  // (a turn behind the last one multiplies zeros)
+            for (int i = 0; i < TURNS; ++i) multiply(i, wave + WAVES * i);  // (a turn behind the last one multiplies zeros)
         } else {
 #pragma unroll
-            for (int i = 0; i < RING; ++i) fetch(i, wave + 4 * i);
-            for (int turn = wave; turn < n_turns; turn += 4 * RING) {
+            for (int i = 0; i < RING; ++i) fetch(i, wave + WAVES * i);
+            for (int turn = wave; turn < n_turns; turn += WAVES * RING) {
 #pragma unroll
                 for (int i = 0; i < RING; ++i) {
-                    multiply(i, turn + 4 * i);
-                    fetch(i, turn + 4 * (i + RING));
+                    multiply(i, turn + WAVES * i);
+                    fetch(i, turn + WAVES * (i + RING));
                 }
             }
         }
@@ -140,7 +157,7 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         // result: the other terms of what met the infinity may be zero, and zero times infinity is not
 #pragma unroll
         for (int e = 0; e < 4; ++e) part[wave][4 * kg + e][col] = col < 8 ? acc1[e] : acc1[e] + acc2[e];
-        __shared__ float s_ss[RMS ? 16 : 1][8];
+        __shared__ float s_ss[RMS ? 4 * WAVES : 1][8];
         if constexpr (RMS) {
             if (col < 8) s_ss[4 * wave + kg][m] = ss;
         }
@@ -148,15 +165,19 @@ __device__ __forceinline__ void rows_body(const RowsAt& t, const LinArgs& p, con
         const int row = threadIdx.x & 15, om = threadIdx.x >> 4;
         if (om < n_rows && row < half && n0 + row < n_out) {
             auto sum = [&](int r) {
-                const float hi = (part[0][r][om] + part[1][r][om]) + (part[2][r][om] + part[3][r][om]);
-                const float mid = (part[0][r][om + 8] + part[1][r][om + 8]) + (part[2][r][om + 8] + part[3][r][om + 8]);
+                float hi = 0.0f, mid = 0.0f;
+#pragma unroll
+                for (int i = 0; i < WAVES; i += 4) {
+                    hi += (part[i][r][om] + part[i + 1][r][om]) + (part[i + 2][r][om] + part[i + 3][r][om]);
+                    mid += (part[i][r][om + 8] + part[i + 1][r][om + 8]) + (part[i + 2][r][om + 8] + part[i + 3][r][om + 8]);
+                }
                 return fabsf(hi) <= 3.4028235e38f ? hi + mid : hi;
             };
             float v = sum(row);
             if constexpr (RMS) {
                 float q = 0.0f;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) q += s_ss[i][om];
+                for (int i = 0; i < 4 * WAVES; ++i) q += s_ss[i][om];
                 v *= 1.0f / sqrtf(q / (float)t.K + t.eps);
             }
             float* C = p.C + (list ? (long long)nth_bit(left, om) * p.c_zoff : (long long)z * p.c_zoff + (long long)om * p.ldc);
@@ -179,10 +200,10 @@ __global__ __launch_bounds__(256) void lm_rows_kernel(const LinArgs a, const Lin
     else one(b, blockIdx.z - za);
 }
 // one product, rows in their order
-template <int TURNS, int KIND>
-__global__ __launch_bounds__(256) void lm_rows_one_kernel(const float* A, const bf16_t* B, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff, const LinArgs p) {
-    __shared__ float part[4][16][17];
-    rows_body<TURNS, KIND, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, a_zoff, b_zoff, 1}, p, blockIdx.z, part);
+template <int TURNS, int KIND, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void lm_rows_one_kernel(const float* A, const bf16_t* B, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff, const LinArgs p) {
+    __shared__ float part[WAVES][16][17];
+    rows_body<TURNS, KIND, FORM_PLAIN, WAVES>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, a_zoff, b_zoff, 1}, p, blockIdx.z, part);
 }
 template <int TURNS>
 __global__ __launch_bounds__(256) void lm_rows_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int M, int ldb, int lda, float eps, const LinArgs p,
@@ -191,11 +212,73 @@ __global__ __launch_bounds__(256) void lm_rows_norm_kernel(const float* A, const
     __shared__ float part[4][16][17];
     rows_body<TURNS, ROWS_RMS, FORM_PLAIN>(RowsAt{A, B, nullptr, K, N, M, ldb, lda, 0, 0, 1, a_norm, eps}, p, blockIdx.z, part);
 }
-template <int TURNS, int KIND>
+template <int TURNS, int KIND, int FORM>
 __global__ __launch_bounds__(256) void lm_rows_list_kernel(const float* A, const bf16_t* B, const int* z_group, int K, int N, int M, int ldb, int lda, int a_zoff, int b_zoff,
                                                            int a_div, const LinArgs p) {
     __shared__ float part[4][16][17];
-    rows_body<TURNS, KIND, FORM_LIST>(RowsAt{A, B, z_group, K, N, M, ldb, lda, a_zoff, b_zoff, a_div}, p, blockIdx.z, part);
+    rows_body<TURNS, KIND, FORM>(RowsAt{A, B, z_group, K, N, M, ldb, lda, a_zoff, b_zoff, a_div}, p, blockIdx.z, part);
+}
+
+// One product of very many weight rows (the vocabulary): a workgroup makes the activations' terms once and takes every gridDim.x-th 16 weight
+// rows, the next ones on their way beside the products.  Bound by the memory: 8 rows x 768 of 50257 weight rows (77 MB) 24.4 us against 30.6 for 3142
+// workgroups that each made the terms again (9 us of vector work and as much again of activations read).
+template <int TURNS>
+__global__ __launch_bounds__(256) void lm_rows_many_kernel(const float* A, const bf16_t* B, int K, int N, int M, int ldb, int lda, const LinArgs p) {
+    __shared__ float part[2][4][16][17];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, kg = lane >> 4, n_tiles = (N + 15) / 16;
+    u32x4 wr[2][TURNS][2], first[TURNS][2], second[TURNS][2];  // leading and middle terms (columns 0 .. 7 and 8 .. 15), and under the middle ones the last
+    int k_at[TURNS][2];
+    auto fetch = [&](auto buf, int tile) {
+        const bf16_t* w = B + (size_t)min(min(tile, n_tiles - 1) * 16 + col, N - 1) * ldb;
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) wr[buf][i][j] = *reinterpret_cast<const u32x4*>(w + k_at[i][j]);
+    };
+#pragma unroll
+    for (int i = 0; i < TURNS; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) k_at[i][j] = min((wave + 4 * i) * kTurn + 16 * kg + 8 * j, K - 8);
+    fetch(step<0>(), blockIdx.x);
+    const float* a = A + (size_t)min(col & 7, M - 1) * lda;
+#pragma unroll
+    for (int i = 0; i < TURNS; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bool beyond = (wave + 4 * i) * kTurn + 16 * kg + 8 * j >= K;  // (the clamped load brings earlier columns: they weigh nothing)
+            const Planes8<3> pl = to_planes<3>(*reinterpret_cast<const f32x4*>(a + k_at[i][j]), *reinterpret_cast<const f32x4*>(a + k_at[i][j] + 4));
+            const u32x4 zero = {0u, 0u, 0u, 0u};
+            first[i][j] = beyond ? zero : col < 8 ? pl.v[0] : pl.v[1];
+            second[i][j] = beyond || col < 8 ? zero : pl.v[2];
+        }
+    auto body = [&](auto buf, int tile) {
+        constexpr int b = decltype(buf)::value;
+        fetch(step<1 - b>(), tile + gridDim.x);
+        acc4 acc1 = {0.0f, 0.0f, 0.0f, 0.0f}, acc2 = acc1;
+#pragma unroll
+        for (int i = 0; i < TURNS; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const u32x4 zero = {0u, 0u, 0u, 0u};
+                const bool beyond = (wave + 4 * i) * kTurn + kTurn > K && (wave + 4 * i) * kTurn + 16 * kg + 8 * j >= K;
+                const bf16x8 wf = __builtin_bit_cast(bf16x8, beyond ? zero : wr[b][i][j]);
+                acc2 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, second[i][j]), acc2, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, __builtin_bit_cast(bf16x8, first[i][j]), acc1, 0, 0, 0);
+            }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) part[b][wave][4 * kg + e][col] = col < 8 ? acc1[e] : acc1[e] + acc2[e];
+        __syncthreads();  // (the tile after next writes this place again: everybody has passed the next tile's barrier by then)
+        const int row = threadIdx.x & 15, om = threadIdx.x >> 4, n = tile * 16 + row;
+        if (om < M && n < N) {
+            const float hi = (part[b][0][row][om] + part[b][1][row][om]) + (part[b][2][row][om] + part[b][3][row][om]);
+            const float mid = (part[b][0][row][om + 8] + part[b][1][row][om + 8]) + (part[b][2][row][om + 8] + part[b][3][row][om + 8]);
+            p.C[(long long)om * p.ldc + n] = finish(fabsf(hi) <= 3.4028235e38f ? hi + mid : hi, n, p);
+        }
+    };
+    for (int tile = blockIdx.x; tile < n_tiles; tile += 2 * gridDim.x) {
+        body(step<0>(), tile);
+        if (tile + (int)gridDim.x < n_tiles) body(step<1>(), tile + gridDim.x);  // (uniform)
+    }
 }
 
 // a product in the form the kernel takes: plain rows, or a list of one-row batches with the matrix chosen by a list (M: its length);
@@ -244,10 +327,18 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
     const dim3 grid(std::max(tiles(a), tiles(b)), A.a_norm && A.tail ? 2 : 1, za + zb);
     const int per_wave = (turns + 3) / 4;
     const bool one = !B && !a.a_rows && a.a_glu == 0 && (a.z_group || a.a_div == 1);
-#define ZG_ROWS_ONE(T, KIND)                                                                                                                            \
-    do {                                                                                                                                                \
-        if (a.z_group) lm_rows_list_kernel<T, KIND><<<grid, 256, 0, s>>>(a.A, a.B, a.z_group, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_div, a); \
-        else lm_rows_one_kernel<T, KIND><<<grid, 256, 0, s>>>(a.A, a.B, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a);                  \
+    // (rows beyond 1024 columns: sixteen waves, and every turn in flight again.  8 rows 768 x 3072 10.9 us against 12.8 with four waves and a ring)
+    const int per_16 = (turns + 15) / 16;
+    const bool wide = one && !a.z_group && !a.a_norm && a.glu_out == 0 && per_wave > 4 && per_16 <= 4;
+    const bool many = one && !a.z_group && !a.a_norm && a.glu_out == 0 && per_wave <= 4 && za == 1 && tiles(a) >= 1024;
+    const bool full = a.z_group && a.M >= za;
+#define ZG_ROWS_ARGS a.A, a.B, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a
+#define ZG_ROWS_LIST a.A, a.B, a.z_group, a.K, a.N, a.M, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_div, a
+#define ZG_ROWS_ONE(T, KIND)                                                                                      \
+    do {                                                                                                          \
+        if (full) lm_rows_list_kernel<T, KIND, T && KIND == ROWS_PLAIN ? FORM_FULL_LIST : FORM_LIST><<<grid, 256, 0, s>>>(ZG_ROWS_LIST);                \
+        else if (a.z_group) lm_rows_list_kernel<T, KIND, FORM_LIST><<<grid, 256, 0, s>>>(ZG_ROWS_LIST);           \
+        else lm_rows_one_kernel<T, KIND, 4><<<grid, 256, 0, s>>>(ZG_ROWS_ARGS);                                   \
     } while (0)
 #define ZG_ROWS(T)                                                                                \
     do {                                                                                          \
@@ -258,13 +349,25 @@ int launch_rows(const Linear& A, const Linear* B, hipStream_t s, bool* taken) {
         else if (a.glu_out > 0) lm_rows_kernel<T, ROWS_GLU_OUT><<<grid, 256, 0, s>>>(a, b, za);   \
         else lm_rows_kernel<T, ROWS_PLAIN><<<grid, 256, 0, s>>>(a, b, za);                        \
     } while (0)
-    if (per_wave == 1) ZG_ROWS(1);
+    const int share = (tiles(a) + 1023) / 1024, groups = (tiles(a) + share - 1) / share;
+#define ZG_ROWS_MANY(T) lm_rows_many_kernel<T><<<groups, 256, 0, s>>>(a.A, a.B, a.K, a.N, a.M, a.ldb, a.lda, a)
+    if (wide && per_16 == 2) lm_rows_one_kernel<2, ROWS_PLAIN, 16><<<grid, 1024, 0, s>>>(ZG_ROWS_ARGS);
+    else if (wide && per_16 == 3) lm_rows_one_kernel<3, ROWS_PLAIN, 16><<<grid, 1024, 0, s>>>(ZG_ROWS_ARGS);
+    else if (wide) lm_rows_one_kernel<4, ROWS_PLAIN, 16><<<grid, 1024, 0, s>>>(ZG_ROWS_ARGS);
+    else if (many && per_wave == 1) ZG_ROWS_MANY(1);
+    else if (many && per_wave == 2) ZG_ROWS_MANY(2);
+    else if (many && per_wave == 3) ZG_ROWS_MANY(3);
+    else if (many) ZG_ROWS_MANY(4);
+    else if (per_wave == 1) ZG_ROWS(1);
     else if (per_wave == 2) ZG_ROWS(2);
     else if (per_wave == 3) ZG_ROWS(3);
     else if (per_wave == 4) ZG_ROWS(4);
     else ZG_ROWS(0);
 #undef ZG_ROWS
 #undef ZG_ROWS_ONE
+#undef ZG_ROWS_MANY
+#undef ZG_ROWS_ARGS
+#undef ZG_ROWS_LIST
     note_kernel("lm_rows_kernel<%d>", per_wave <= 4 ? per_wave : 0);
     ZG_HIP(hipGetLastError());
     *taken = true;
