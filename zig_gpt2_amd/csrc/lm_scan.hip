@@ -13,7 +13,7 @@
 //
 // What bounds it: the fp32 matrix instruction (64 cycles per 32 x 32 x 2: 12.8 k cycles per chunk and head of 128 x 128 in the output
 // kernel, 4 k in the state kernel) and the chunk states, written, carried and read (64 KB per chunk and head).  8 x 1023 tokens, 8 heads of
-// 128 x 128: state 42 us, carry 28, output 92 = 162 us per layer; scanned token by token inside chunks it was 265 + 25 + 265.
+// 128 x 128: state 47 us, carry 29, output 77 = 153 us per layer; scanned token by token inside chunks it was 265 + 25 + 265.
 #include <math.h>
 #include <stdlib.h>
 
@@ -171,43 +171,45 @@ __global__ __launch_bounds__(512) void gated_chunk_state_kernel(const ScanArgs p
 }
 
 // phase C: the outputs of a (chunk, head) from its start state (wsB).  Eight waves; the state and the values come straight from memory as
-// matrix operands, requested in front of the work on the gates.
+// matrix operands, half of the state requested in front of the work on the gates, the rest beside the products.  A workgroup alone takes 22 us,
+// 5 of them in the matrix cores: A takes the place of gates that have been used and waits in registers until then, so that two workgroups of
+// HGRN2 share a compute unit (72 KB each, 128 registers a lane; keys of GLA need an array of their own, and one is alone).  8 x 1023 tokens, 8
+// heads of 128 x 128: 77 us against 95 for one workgroup of 89 KB; 6 heads 62 against 69, GLA 78 against 81; 333 tokens, 6 heads: 22 on both.
 template <int KIND, int DP>
-__global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) {
+__global__ __launch_bounds__(512, KIND == KIND_HGRN2 && DP == 128 ? 4 : 2) void gated_chunk_out_kernel(const ScanArgs p) {
     constexpr int LD = DP + 4, LA = kChunk + 4;
     __shared__ __attribute__((aligned(16))) float s_q[kChunk * LD];
     __shared__ __attribute__((aligned(16))) float s_f[kChunk * LD];
     __shared__ __attribute__((aligned(16))) float s_k[KIND == KIND_GLA ? kChunk * LD : 4];
-    __shared__ __attribute__((aligned(16))) float s_A[kChunk * LA];
     __shared__ __attribute__((aligned(16))) float s_F[8 * DP];  // gates of every block of 8 multiplied
     int e, c;
     if (!find_chunk(blockIdx.x, p.ent_len, p.n_entries, e, c)) return;
     const int h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, kh = lane >> 5;
     const int n = min(kChunk, p.ent_len[e] - c * kChunk), m0 = p.ent_start[e] + c * kChunk, HD = p.H * p.D;
     float* const s_key = KIND == KIND_GLA ? s_k : s_f;
+    float* const s_A = s_f;  // once gates and keys have been used
     const float* vrow = p.proj + (size_t)m0 * p.ld + 2 * HD + (size_t)h * p.V;
     const float* S0 = p.wsB + ((size_t)blockIdx.x * p.H + h) * p.D * p.V;
     const int mt = wave & 1;  // this wave's 32 tokens
     float Sf[DP / 2], vf[32];
     bool odd_v = false;
-    auto load_operands = [&](int sl) {  // this lane's column of the slice: channels 8 g + 4 kh + j of the state, tokens alike
-        // (channels beyond D and tokens behind the chunk: the last valid ones, met by zeros)
-        const int col = min(sl * 32 + r, p.V - 1);
+    // this lane's column of the slice: channels 8 g + 4 kh + j of the state, tokens alike (channels beyond D and tokens behind the chunk: the last
+    // valid ones, met by zeros)
+    const int sl = blockIdx.z * 4 + (wave >> 1), col = min(sl * 32 + r, p.V - 1);
+    constexpr int SHARE = DP / 4;  // the state in two shares: two workgroups fit a compute unit with at most 128 registers a lane
+    auto load_state = [&](int from) {
 #pragma unroll
-        for (int x = 0; x < DP / 2; ++x) Sf[x] = S0[min(8 * (x >> 2) + 4 * kh + (x & 3), p.D - 1) * p.V + col];
-#pragma unroll
-        for (int x = 0; x < 32; ++x) vf[x] = vrow[min(8 * (x >> 2) + 4 * kh + (x & 3), n - 1) * p.ld + col];
+        for (int x = from; x < from + SHARE; ++x) Sf[x] = S0[min(8 * (x >> 2) + 4 * kh + (x & 3), p.D - 1) * p.V + col];
+        __builtin_amdgcn_sched_barrier(0);
     };
     load_chunk<KIND, DP, LD, true>(p, h, m0, n, s_q, s_f, s_k);
-    for (int idx = tid; idx < kChunk * LA; idx += 512) s_A[idx] = 0.0f;
     __syncthreads();
-    const int sl = blockIdx.z * 4 + (wave >> 1);
-    load_operands(sl);
-    __builtin_amdgcn_sched_barrier(0);
+    load_state(0);
 
+    float near0 = 0.0f, near1 = 0.0f;  // A of token part of the wave's block against s0 and s0 + 4
+    const int part = lane & 15, s0 = lane >> 4;
     {  // pairs of one block of 8 (a wave's own): lane (s, part) carries k_s P(s+1, t) of its channels from t to t, for s and s + 4
         constexpr int PARTS = DP / 64;
-        const int part = lane & 15, s0 = lane >> 4;
         f32x4 a0[PARTS], a1[PARTS];
         for (int t = 0; t < 8; ++t) {
             float x0 = 0.0f, x1 = 0.0f;
@@ -228,10 +230,9 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
             }
             x0 = row16_allsum(x0);
             x1 = row16_allsum(x1);
-            if (part == 0) {
-                float* row = &s_A[(8 * wave + t) * LA + 8 * wave + s0];
-                if (t >= s0) row[0] = x0;
-                if (t >= s0 + 4) row[4] = x1;
+            if (part == t) {
+                near0 = t >= s0 ? x0 : 0.0f;
+                near1 = t >= s0 + 4 ? x1 : 0.0f;
             }
         }
     }
@@ -269,12 +270,8 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
         }
         return acc;  // element x: token 16 i + 4 kg + x against token 16 j + m16
     };
-    if (wave < 4) {  // the second half of a block of 16 against its first
-        const f32x4 a = pair_tile(wave, wave);
-        if (kg >= 2 && m16 < 8)
-#pragma unroll
-            for (int x = 0; x < 4; ++x) s_A[(16 * wave + 4 * kg + x) * LA + 16 * wave + m16] = a[x];
-    }
+    f32x4 half = {0.0f, 0.0f, 0.0f, 0.0f}, cross = half;
+    if (wave < 4) half = pair_tile(wave, wave);  // the second half of a block of 16 against its first
     __syncthreads();
     for (int idx = tid; idx < kChunk * (DP / 4); idx += 512) {  // blocks of 16: the halves meet
         const int t = idx / (DP / 4), d = (idx % (DP / 4)) * 4, b = t >> 3;
@@ -282,13 +279,20 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
         *v *= *reinterpret_cast<const f32x4*>(&s_F[(b ^ 1) * DP + d]);
     }
     __syncthreads();
-    if (wave < 6) {  // blocks of 16 against earlier ones
-        const int i = wave < 1 ? 1 : wave < 3 ? 2 : 3, j = wave < 1 ? 0 : wave < 3 ? wave - 1 : wave - 3;
-        const f32x4 a = pair_tile(i, j);
-#pragma unroll
-        for (int x = 0; x < 4; ++x) s_A[(16 * i + 4 * kg + x) * LA + 16 * j + m16] = a[x];
-    }
+    // blocks of 16 against earlier ones; the last two waves have the zeros behind the diagonal that a product of 32 tokens meets
+    const int ti = wave < 1 ? 1 : wave < 3 ? 2 : wave < 6 ? 3 : wave == 6 ? 0 : 2, tj = wave < 1 ? 0 : wave < 3 ? wave - 1 : wave < 6 ? wave - 3 : wave == 6 ? 1 : 3;
+    if (wave < 6) cross = pair_tile(ti, tj);
     __syncthreads();
+    load_state(SHARE);
+    if (part < 8) {
+        s_A[(8 * wave + part) * LA + 8 * wave + s0] = near0;
+        s_A[(8 * wave + part) * LA + 8 * wave + s0 + 4] = near1;
+    }
+    if (wave < 4 && (kg >= 2) == (m16 < 8))
+#pragma unroll
+        for (int x = 0; x < 4; ++x) s_A[(16 * wave + 4 * kg + x) * LA + 16 * wave + m16] = kg >= 2 ? half[x] : 0.0f;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) s_A[(16 * ti + 4 * kg + x) * LA + 16 * tj + m16] = cross[x];
     for (int idx = tid; idx < 48 * (DP / 4); idx += 512) {  // the queries from the chunk's start
         const int t = 16 + idx / (DP / 4), d = (idx % (DP / 4)) * 4;
         f32x4* v = reinterpret_cast<f32x4*>(&s_q[t * LD + d]);
@@ -301,12 +305,20 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
         f32x16 acc;
 #pragma unroll
         for (int x = 0; x < 16; ++x) acc[x] = 0.0f;
+        auto state_share = [&](int from) {
 #pragma unroll
-        for (int g = 0; g < DP / 8; ++g) {
-            const f32x4 q = *reinterpret_cast<const f32x4*>(&s_q[(32 * mt + r) * LD + 8 * g + 4 * kh]);
+            for (int g = from / 4; g < (from + SHARE) / 4; ++g) {
+                const f32x4 q = *reinterpret_cast<const f32x4*>(&s_q[(32 * mt + r) * LD + 8 * g + 4 * kh]);
 #pragma unroll
-            for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(q[u], Sf[4 * g + u], acc, 0, 0, 0);
-        }
+                for (int u = 0; u < 4; ++u) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(q[u], Sf[4 * g + u], acc, 0, 0, 0);
+            }
+        };
+        state_share(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int x = 0; x < 32; ++x) vf[x] = vrow[min(8 * (x >> 2) + 4 * kh + (x & 3), n - 1) * p.ld + col];
+        __builtin_amdgcn_sched_barrier(0);
+        state_share(SHARE);
         // A is zero above its diagonal, but zero times a value that is not finite is not: such values are left out here and added below,
         // token by token, to the outputs at and behind them only
         odd_v = false;
@@ -323,10 +335,9 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u], fabsf(v) <= 3.4028235e38f ? v : 0.0f, acc, 0, 0, 0);
             }
         }
-        const int col = sl * 32 + r;
         if (any_odd)
             for (int s = 0; s < n; ++s) {
-                const float v = vrow[(size_t)s * p.ld + min(col, p.V - 1)];
+                const float v = vrow[(size_t)s * p.ld + col];
                 if (!(fabsf(v) <= 3.4028235e38f))
 #pragma unroll
                     for (int x = 0; x < 16; ++x) {
@@ -337,7 +348,7 @@ __global__ __launch_bounds__(512) void gated_chunk_out_kernel(const ScanArgs p) 
 #pragma unroll
         for (int x = 0; x < 16; ++x) {
             const int t = 32 * mt + 8 * (x >> 2) + 4 * kh + (x & 3);
-            if (t < n && col < p.V) p.out[(size_t)(m0 + t) * p.ldo + h * p.V + col] = acc[x];
+            if (t < n && sl * 32 + r < p.V) p.out[(size_t)(m0 + t) * p.ldo + h * p.V + col] = acc[x];
         }
     }
 }
