@@ -579,34 +579,40 @@ __global__ __launch_bounds__(256) void hgrn2_scan_kernel(const float* proj, int 
     }
 }
 
-// phase B: one thread per state element walks the chunks of its entry
+// phase B: a thread per VEC state elements in a row walks the chunks of its entry.  Bound by the memory: every chunk's state is read and written.
+// 8 entries of 16 chunks, 8 heads of 128 x 128: 142 MB in 27.4 us with two elements a thread against 29.2 with one; 24 heads of 128 x 64, 60 chunks of
+// 8 entries 20.1 against 22.3.
+template <int VEC>
 __global__ __launch_bounds__(256) void hgrn2_carry_kernel(float* state, size_t slot_stride, const int* ent_len, const int* ent_slot, int n_entries, int H,
                                                           int D, int V, float* wsB, const float* wsA, int a_rows, int chunk) {
+    typedef __attribute__((ext_vector_type(VEC))) float vec;
     const int e = blockIdx.y;
-    const size_t n = (size_t)H * D * V, idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const size_t n = (size_t)H * D * V, idx = ((size_t)blockIdx.x * blockDim.x + threadIdx.x) * VEC;
     if (idx >= n) return;
     int first = 0;
     for (int k = 0; k < e; ++k) first += (ent_len[k] + chunk - 1) / chunk;
     const int nc = (ent_len[e] + chunk - 1) / chunk;
     const size_t ai = idx / ((size_t)V * (D / a_rows)), na = (size_t)H * a_rows;  // the decay of the element's (head, row), or of its head
-    float* slot = state + (size_t)ent_slot[e] * slot_stride;
-    float S = slot[idx];
+    vec* slot = reinterpret_cast<vec*>(state + (size_t)ent_slot[e] * slot_stride + idx);
+    vec S = *slot;
     for (int c0 = 0; c0 < nc; c0 += 8) {  // eight chunks' operands requested together: the chain itself is eight multiply-adds
-        float Bv[8], Av[8];
+        vec Bv[8];
+        float Av[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
             const int c = min(c0 + u, nc - 1);
-            Bv[u] = wsB[(size_t)(first + c) * n + idx];
+            Bv[u] = *reinterpret_cast<const vec*>(wsB + (size_t)(first + c) * n + idx);
             Av[u] = wsA[(size_t)(first + c) * na + ai];
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (c0 + u < nc) {
-                wsB[(size_t)(first + c0 + u) * n + idx] = S;  // the chunk's start state for phase C
-                S = fmaf(Av[u], S, Bv[u]);
+                *reinterpret_cast<vec*>(wsB + (size_t)(first + c0 + u) * n + idx) = S;  // the chunk's start state for phase C
+#pragma unroll
+                for (int i = 0; i < VEC; ++i) S[i] = fmaf(Av[u], S[i], Bv[u][i]);
             }
     }
-    if (nc > 0) slot[idx] = S;
+    if (nc > 0) *slot = S;
 }
 
 // ------------------------------------------------------------------------------------------------ linear attention, chunks on the matrix cores
@@ -1749,8 +1755,12 @@ int launch_state_carry(float* state, size_t slot_stride, const int* ent_len, con
     const size_t n = (size_t)H * D * V;
     if (n_entries <= 0 || n == 0) return ZG_OK;
     ZG_REQUIRE(a_rows == 1 || a_rows == D, ZG_ERR_ARG, "state carry: %d decays per head of %d rows", a_rows, D);
-    hgrn2_carry_kernel<<<dim3((unsigned)((n + 255) / 256), n_entries), 256, 0, s>>>(state, slot_stride, ent_len, ent_slot, n_entries, H, D, V, wsB, wsA, a_rows,
-                                                                                  chunk);
+    // two elements a thread where rows, slots and pointers allow
+    const bool two = V % 2 == 0 && slot_stride % 2 == 0 && ((reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(wsB)) & 7) == 0;
+    const int per = two ? 512 : 256;
+    const dim3 grid((unsigned)((n + per - 1) / per), n_entries);
+    if (two) hgrn2_carry_kernel<2><<<grid, 256, 0, s>>>(state, slot_stride, ent_len, ent_slot, n_entries, H, D, V, wsB, wsA, a_rows, chunk);
+    else hgrn2_carry_kernel<1><<<grid, 256, 0, s>>>(state, slot_stride, ent_len, ent_slot, n_entries, H, D, V, wsB, wsA, a_rows, chunk);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
