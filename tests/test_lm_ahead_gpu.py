@@ -5,6 +5,7 @@ import numpy as np
 import pytest
 
 import duvulix_testlib as dl
+import gupizen_testlib as gl
 import lm_testlib as tl
 from zig_gpt2_amd import lm
 
@@ -76,3 +77,35 @@ def test_a_cache_that_is_full_half_way():
         m.generate(prompts, 60)
     assert np.array_equal(m.generate(prompts, 17), want)
     m.close()
+
+
+def without_canon(layers, **kw):
+    """Mixers with a convolution of their own behind a token shift (no convolution of the sublayers' inputs)."""
+    cfg = gl.config(layers, **kw)
+    del cfg["canon"]
+    return cfg
+
+
+CONVOLVED = {
+    "delta": without_canon([gl.delta_layer(conv=4, mlp=gl.moe_mlp()), gl.delta_layer(conv=2, mlp=None)]),
+    "parallel": without_canon([gl.parallel_layer(conv=4, mlp=gl.moe_mlp()), gl.parallel_layer(conv=2, mlp=None)]),
+    "both": without_canon([gl.parallel_layer(conv=4, mlp=None), gl.delta_layer(conv=4, mlp=gl.moe_mlp()), gl.parallel_layer(conv=16, mlp=gl.moe_mlp())]),
+    "one tap": without_canon([gl.delta_layer(conv=1, mlp=gl.moe_mlp())]),
+}
+
+
+@pytest.mark.parametrize("n_seqs", [1, 3, 8])
+@pytest.mark.parametrize("design", sorted(CONVOLVED))
+def test_convolutions_of_the_mixers(design, n_seqs):
+    """A row's place inside its entry stays 0 through a generation: every token's convolution reads its own slot's tail."""
+    cfg = CONVOLVED[design]
+    w = gl.weights(cfg, seed=7)
+    prompts = [gl.tokens(b, 1 + 3 * b, cfg["vocab"]) for b in range(n_seqs)]
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=1024, max_seqs=8, page_tokens=8, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append([m.generate(prompts, n, temp=t, seed=s) for n, t, s in ((3, 0.0, 0), (40, 0.0, 0), (20, 1.5, 5), (40, 0.0, 0))])
+        m.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)

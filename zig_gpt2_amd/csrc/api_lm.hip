@@ -265,9 +265,11 @@ struct zg_lm {
 
 namespace {
 
-// ids | pos | slot | prev | last-entry | want rows | entry start | entry len | entry slot | place of the row inside its entry
-size_t meta_ints(const zg_lm* g) { return (size_t)7 * g->MS + (size_t)3 * g->NS; }
+// ids | pos | slot | prev | last-entry | want rows | entry start | entry len | entry slot | place of the row inside its entry | steps of the
+// running generation by row (every staging of rows leaves zeros there)
 size_t meta_row_off(const zg_lm* g) { return (size_t)6 * g->MS + (size_t)3 * g->NS; }
+size_t meta_steps(const zg_lm* g) { return (size_t)7 * g->MS + (size_t)3 * g->NS; }
+size_t meta_ints(const zg_lm* g) { return meta_steps(g) + kGemvMaxRows; }
 
 // The most keys a row of a rotary attention layer can see.
 int rotary_key_capacity(const zg_lm* g, const zg_lm_layer& d) {
@@ -1793,7 +1795,7 @@ int enqueue_chained(zg_lm* g, int M) {
     ZG_TRY(launch_argmax_parts(g->logits, M, g->V, g->amax_val, g->amax_idx, &t.n_parts, g->stream));
     const size_t MS = g->MS;
     t.part_val = g->amax_val; t.part_idx = g->amax_idx; t.table = g->embed; t.W = g->W; t.scale = g->embed_scale; t.eps = g->cfg.norm_eps; t.wn = first.norm1;
-    t.mu = g->no_shift ? nullptr : first.shift; t.ids = g->meta; t.pos = g->meta + MS; t.row_slot = g->meta + 2 * MS; t.count = g->meta + meta_row_off(g); t.seen = g->h_ahead;
+    t.mu = g->no_shift ? nullptr : first.shift; t.ids = g->meta; t.pos = g->meta + MS; t.row_slot = g->meta + 2 * MS; t.count = g->meta + meta_steps(g); t.seen = g->h_ahead;
     t.ahead = zg_lm::kAhead; t.seen_stride = kGemvMaxRows; t.x = g->x; t.h = g->h; t.last_h = g->last_h; t.shift_state = g->shift_state;
     t.slot_stride = (size_t)g->n_passes * g->W;
     return launch_next_token(t, M, g->stream);
