@@ -66,3 +66,25 @@ def test_sinks(n):
     cfg = pl.config([pl.latent_layer(heads=3, dim=64, vdim=20, rot_dim=16, kv_rank=72, mlp=pl.dense(ff=32)) for _ in range(2)], width=48)
     w = pl.weights(cfg, seed=9)
     check(cfg, w, lambda t: po.forward(w, cfg, t), n)
+
+
+@pytest.mark.parametrize("page_tokens", [1, 3, 16, 0])
+@pytest.mark.parametrize("dim,kv_rank,rot_dim", [(64, 64, 64), (64, 72, 8), (128, 512, 64)])
+def test_long_ranges(dim, kv_rank, rot_dim, page_tokens):
+    """Ranges of several turns of sixteen keys, whose pages are asked for a turn ahead: around whole turns, pages of one token to many."""
+    lat = dict(heads=2, dim=dim, vdim=8, rot_dim=rot_dim, kv_rank=kv_rank)
+    cfg = dl.config([dl.latent_layer(mlp=None, **lat)], width=32)
+    w = dl.weights(cfg, seed=kv_rank)
+    starts = [1279, 1023, 767, 800]
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=4224, max_seqs=4, page_tokens=page_tokens, max_step_tokens=1280)
+    m.load_weights(w)
+    toks = [tl.tokens(90 + b, s + 2, cfg["vocab"]) for b, s in enumerate(starts)]
+    refs = [do.forward(w, cfg, t) for t in toks]
+    seqs = [m.open() for _ in starts]
+    for s, t, k in zip(seqs, toks, starts):
+        m.step([(s, t[:k], [])])
+    for i in range(2):
+        for some in ([0], [1, 2, 3]):  # (more rows: the weights are asked for behind the row's position)
+            got = m.step([(seqs[b], [toks[b][starts[b] + i]], [0]) for b in some])
+            tl.assert_close(got, np.stack([refs[b][starts[b] + i] for b in some]), "float32", (i, some))
+    m.close()

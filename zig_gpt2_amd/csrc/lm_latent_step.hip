@@ -6,6 +6,11 @@
 // products that make values of the weighted latents (lm_mix.hip, lm_linear.hip; steps with several rows of a sequence keep them, since
 // a row's keys are then written in the same step).  64 x 256 + 32, 12 heads, six such layers of twelve: a step of one sequence 408 -> 375 us, of
 // eight, with the queries' norm inside the product in front (lm_rows.hip), 705 -> 653.
+// Long ranges are bound by a wave's own instructions and one round trip a turn of sixteen keys.  us a layer (projections and launches around it
+// included), in five launches -> here: 16 heads, 64 x 256 + 64, one row behind 1000 keys 35.8 -> 25.3, behind 16000 98 -> 74; eight rows behind 4000
+// 110 -> 86; 64 x 512 + 64, eight rows behind 4000 128 -> 112.
+#include <type_traits>
+
 #include "lm_latent_parts.h"
 
 namespace zg {
@@ -73,17 +78,33 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
     const bool any = R > 0;  // (without a rotated part: some valid channel)
     const float rx = (any ? rsrc : qh)[any ? min(r0, R - 1) : 0], ry = (any ? rsrc : qh)[any ? min(r1, R - 1) : 0], rf = half > 0 ? a.rot.freq[min(rt, half - 1)] : 0.0f;
     float r[4][ND];
-    auto fetch = [&](int kb, float (&to)[4][ND]) {
+    // (a turn's pages are asked for a turn before its keys, all four at once: behind the store of the token's row the compiler takes a look-up
+    // for a vector load of its own, and one that stands between the keys' loads waits for them: four round trips a turn)
+    int page[4];
+    unsigned place[4], col[ND];  // of the keys looked up last: their pages, their places inside them; byte offsets of this lane's channels
+#pragma unroll
+    for (int i = 0; i < ND; ++i) col[i] = 4u * (unsigned)min(lane + 64 * i, DT - 1);
+    auto look_up = [&](int kb) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const int key = min(kb + u, k_hi - 1);
-            const float* row = a.cache + ((size_t)pt[key / a.page_tokens] * a.page_tokens + key % a.page_tokens) * DT;
+            const unsigned key = (unsigned)min(kb + u, k_hi - 1), at = key / (unsigned)a.page_tokens;
+            page[u] = pt[at];
+            place[u] = key - at * (unsigned)a.page_tokens;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto fetch = [&](float (&to)[4][ND]) {
 #pragma unroll
-            for (int i = 0; i < ND; ++i) to[u][i] = row[min(lane + 64 * i, DT - 1)];
+        for (int u = 0; u < 4; ++u) {
+            const float* row = a.cache + ((size_t)(unsigned)__builtin_amdgcn_readfirstlane(page[u]) * (unsigned)a.page_tokens + place[u]) * (unsigned)DT;
+#pragma unroll
+            for (int i = 0; i < ND; ++i) to[u][i] = *reinterpret_cast<const float*>(reinterpret_cast<const char*>(row) + col[i]);
         }
     };
     const int kb0 = k_lo + wave * 4;
-    fetch(kb0, r);
+    look_up(kb0);
+    fetch(r);
+    look_up(kb0 + 16);
     // the query in the latent space
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
@@ -134,20 +155,27 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
     for (int i = 0; i < ND; ++i) {
         const int d = lane + 64 * i;
         qd[i] = d < DT ? s_q[min(d, DT - 1)] : 0.0f;
-        fresh[i] = has_new ? s_new[min(d, DT - 1)] : 0.0f;
+        fresh[i] = has_new && d < DT ? s_new[min(d, DT - 1)] : 0.0f;
         acc[i] = 0.0f;
     }
     float mx = -INFINITY, l = 0.0f;
-    auto take = [&](int kb) {
+    // LAST: the turn that may hold the token's own key, or fewer than four
+    auto take = [&](int kb, auto last) {
+        constexpr bool LAST = decltype(last)::value;
+        if (DT < 64 * ND) {  // (channels behind the last one brought it again, which need not be finite)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int i = 0; i < ND; ++i) r[u][i] = lane + 64 * i < DT ? r[u][i] : 0.0f;
+        }
         float s[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            const bool is_new = has_new && min(kb + u, k_hi - 1) == pos;
+            const bool is_new = LAST && has_new && min(kb + u, k_hi - 1) == pos;
             float part = 0.0f;
 #pragma unroll
             for (int i = 0; i < ND; ++i) {
                 if (is_new) r[u][i] = fresh[i];
-                if (lane + 64 * i >= DT) r[u][i] = 0.0f;
                 part = fmaf(qd[i], r[u][i], part);
             }
             s[u] = part;
@@ -155,7 +183,7 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             s[u] = wave_allsum(s[u]) * a.scale;
-            if (kb + u >= k_hi) s[u] = -INFINITY;
+            if (LAST && kb + u >= k_hi) s[u] = -INFINITY;
         }
         const float mn = fmaxf(fmaxf(mx, s[0]), fmaxf(fmaxf(s[1], s[2]), s[3]));
         const float alpha = expf(mx - mn);  // 0 for the first group (mx = -inf, mn finite: key kb is always valid)
@@ -175,14 +203,15 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
     int kb = kb0;
     for (; kb + 16 < k_hi; kb += 16) {
         float next[4][ND];
-        fetch(kb + 16, next);
-        take(kb);
+        fetch(next);
+        look_up(kb + 32);
+        take(kb, std::false_type());
 #pragma unroll
         for (int u = 0; u < 4; ++u)
 #pragma unroll
             for (int i = 0; i < ND; ++i) r[u][i] = next[u][i];
     }
-    if (kb < k_hi) take(kb);
+    if (kb < k_hi) take(kb, std::true_type());
     if (lane == 0) {
         s_m[wave] = mx;
         s_l[wave] = l;
