@@ -32,3 +32,10 @@ def test_one_token_of_every_entry(heads, vdim, state, groups, conv, norm_groups,
         # (fp32 sums through two layers: the layered tier's bound for 32-bit mode)
         assert np.abs(got - want).max() < 3e-5 * np.abs(want).max(), (n, i)
     m.close()
+
+
+@pytest.mark.parametrize("n", [5, 6, 8])
+@pytest.mark.parametrize("heads,vdim", [(16, 64), (86, 12), (16, 128), (32, 128), (129, 32)])
+def test_norms_of_long_rows(heads, vdim, n):
+    """Rows of up to 1024 columns are normed inside the product, longer ones in a launch in front of the product that splits them over sixteen waves."""
+    test_one_token_of_every_entry(heads, vdim, 16, 1, 4, 1, n)

@@ -1231,7 +1231,10 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             lin = Linear();
             lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
             bool normed = false;
-            if (few && d.norm_groups <= 1) {  // the norm of the whole row where the product reads it
+            // The norm of the whole row where the product reads it.  Three rows and more: up to 1024 columns, for longer ones are split over sixteen
+            // waves without the norm, and that outweighs the norm's launch (us a layer of 8 rows, normed in the product : in front of it: 1152
+            // columns 25.8 : 24.6, 1536 27.8 : 25.1, 3072 36.2 : 30.0, 8192 70.6 : 64.7; 6 rows of 1152 24.7 : 23.4).
+            if (few && d.norm_groups <= 1 && (M <= 2 || HV <= 1024)) {
                 Linear ln = lin;
                 ln.A = g->o; ln.a_norm = L.part_norm; ln.norm_eps = eps;
                 if (single && cv.taps > 1) ln.tail = &cv, ln.tail_slot = d_slot;
