@@ -88,3 +88,13 @@ def test_long_ranges(dim, kv_rank, rot_dim, page_tokens):
             got = m.step([(seqs[b], [toks[b][starts[b] + i]], [0]) for b in some])
             tl.assert_close(got, np.stack([refs[b][starts[b] + i] for b in some]), "float32", (i, some))
     m.close()
+
+
+@pytest.mark.parametrize("n", [2, 6, 7, 8])
+@pytest.mark.parametrize("heads,dim,kv_rank", [(13, 128, 512), (40, 64, 512), (64, 64, 256), (24, 128, 264)])
+def test_weights_of_many_heads(heads, dim, kv_rank, n):
+    """Around the rows x heads x weights from which the five launches take the step: both forms, one layer filing its latents for the next."""
+    lat = dict(heads=heads, dim=dim, vdim=4, rot_dim=8, kv_rank=kv_rank)
+    cfg = dl.config([dl.latent_layer(mlp=None, **lat), dl.latent_layer(kv_from=0, mlp=None, **lat)], width=32)
+    w = dl.weights(cfg, seed=heads)
+    check(cfg, w, lambda t: do.forward(w, cfg, t), n, steps=2)

@@ -1425,7 +1425,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 st.ld_lat = LD;
                 st.wkv = L.dkv_norm;
             }
-            if (few && (single || !st.lat) && latent_step_fits(H, D, R, KR, Vd, ldq, LD)) {
+            if (few && (single || !st.lat) && latent_step_fits(M, H, D, R, KR, Vd, ldq, LD)) {
                 bool queries = direct;
                 if (!direct) {
                     lin = Linear();

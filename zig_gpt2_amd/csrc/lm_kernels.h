@@ -346,7 +346,7 @@ struct LatentStep {
     float* out = nullptr;
     int ldo = 0;
 };
-bool latent_step_fits(int H, int D, int R, int KR, int Vd, int ldq, int ld_lat);
+bool latent_step_fits(int M, int H, int D, int R, int KR, int Vd, int ldq, int ld_lat);
 int launch_latent_step(const LatentStep& a, hipStream_t s, bool* taken);
 
 // The same for prompt portions on the matrix cores (bf16 operands, fp32 scores / softmax / accumulation): 32 queries of one entry

@@ -38,6 +38,9 @@ template <int KP, int LPR, bool EAGER>
 __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, const int* row_slot, const float* q, const bf16_t* ukT, const float* lat, int ldq, int ld_lat,
                                                           int KR, int R, const LatentStepRest a) {
     constexpr int ND = KP + 1, D = 8 * LPR, RPI = 64 / LPR, NP = KP * LPR / 4, NL = (KP + 3) / 4;
+    // weights a lane holds at a time (128 x 512: 146 registers, three workgroups to a compute unit, against 205 and two: 16 heads, six rows 63.5 us a
+    // layer : 71.1)
+    constexpr int BATCH = EAGER ? NP : 16;
     __shared__ float s_q[ND * 64], s_new[ND * 64], s_m[4], s_l[4], s_red[4];
     __shared__ float s_acc[4][ND * 64];
     const int m = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63, tid = threadIdx.x;
@@ -47,22 +50,25 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
     const bool own = lat != nullptr;
     const float* lr = own ? lat + (size_t)m * ld_lat : qh;
     f32x4 q8[2];
-    u32x4 wr[NP];
-    auto fetch_weights = [&]() {
+    u32x4 wr[NP < BATCH ? NP : BATCH];
+    auto fetch_weights = [&](int from) {
 #pragma unroll
-        for (int j = 0; j < NP; ++j) {
-            const int row = min((4 * j + wave) * RPI + lane / LPR, KR - 1);
+        for (int j = 0; j < NP && j < BATCH; ++j) {
+            if (from + j >= NP) break;
+            const int row = min((4 * (from + j) + wave) * RPI + lane / LPR, KR - 1);
             wr[j] = *reinterpret_cast<const u32x4*>(ukT + ((size_t)h * KR + row) * D + (lane % LPR) * 8);
         }
+    };
+    auto fetch_query = [&]() {
 #pragma unroll
         for (int i = 0; i < 2; ++i) q8[i] = *reinterpret_cast<const f32x4*>(qh + (lane % LPR) * 8 + 4 * i);
     };
-    if constexpr (EAGER) fetch_weights();
+    if constexpr (EAGER) fetch_weights(0), fetch_query();
     const int pos = row_pos[m], n_keys = pos + 1, chunk = split_chunk(n_keys, kAttnSplits);
     const int k_lo = min(n_keys, (int)blockIdx.z * chunk), k_hi = min(n_keys, k_lo + chunk);
     if (k_lo >= k_hi) return;
     const int* pt = a.page_table + (size_t)row_slot[m] * a.max_pages;
-    if constexpr (!EAGER) fetch_weights();
+    if constexpr (!EAGER) fetch_weights(0), fetch_query();
     const bool has_new = own && k_hi == n_keys;
     float lv[NL], lw[NL];
 #pragma unroll
@@ -108,9 +114,13 @@ __global__ __launch_bounds__(256) void latent_step_kernel(const int* row_pos, co
     // the query in the latent space
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
+        if (j > 0 && j % BATCH == 0) {
+            __builtin_amdgcn_sched_barrier(0);
+            fetch_weights(j);
+        }
         float s = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) s = fmaf(q8[i / 2][2 * (i & 1) + 1], bf16_hi(wr[j][i]), fmaf(q8[i / 2][2 * (i & 1)], bf16_lo(wr[j][i]), s));
+        for (int i = 0; i < 4; ++i) s = fmaf(q8[i / 2][2 * (i & 1) + 1], bf16_hi(wr[j % BATCH][i]), fmaf(q8[i / 2][2 * (i & 1)], bf16_lo(wr[j % BATCH][i]), s));
         if constexpr (LPR == 16) s = row16_allsum(s);
         else {  // eight lanes
             s += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(s), 0x141, 0xF, 0xF, true));  // 7 - lane
@@ -288,15 +298,23 @@ __global__ __launch_bounds__(256) void latent_values_kernel(const float* ws, con
 
 }  // namespace
 
-// The forms these kernels have: heads of 64 or 128 unrotated channels, latents of up to 512 + 64 in whole 16-byte pieces.
-bool latent_step_fits(int H, int D, int R, int KR, int Vd, int ldq, int ld_lat) {
-    return (D == 64 || D == 128) && KR >= 8 && KR <= 512 && KR % 8 == 0 && R >= 0 && R <= 64 && R % 4 == 0 && ldq % 4 == 0 && Vd > 0 && H > 0 && H <= 65535 && ld_lat >= 0;
+// The forms these kernels have: heads of 64 or 128 unrotated channels, latents of up to 512 + 64 in whole 16-byte pieces.  And where they pay: each of a
+// row's sixteen key ranges reads its head's KR x D weights again.  us a layer, five launches : here, the farthest apart of one to twelve thousand
+// keys (E: rows x heads x KR x D / 2^20):
+//   KR x D <= 16 K: 128 heads of 64 x 64, eight rows 124 : 105; of 128 x 64 (E 8) 158 : 140; of 64 x 256 (E 16) 136 : 130
+//   32 K: 32 heads of 128 x 256, eight rows (E 8) 67.8 : 66.3; 48 heads, six rows (E 9) 79 : 74, eight (E 12) 84.8 : 87.6; 64 heads of 64 x 512, eight (E 16) 99 : 109
+//   more: 24 heads of 128 x 320, six rows (E 5.6) 60.6 : 52.8; 16 heads of 128 x 512, six rows (E 6) 67.7 : 63.5, eight (E 8) 56.8 : 57.3; 128 heads, one row
+//   (E 8) 94.6 : 97.1, eight (E 64) 207 : 404
+bool latent_step_fits(int M, int H, int D, int R, int KR, int Vd, int ldq, int ld_lat) {
+    const bool form = (D == 64 || D == 128) && KR >= 8 && KR <= 512 && KR % 8 == 0 && R >= 0 && R <= 64 && R % 4 == 0 && ldq % 4 == 0 && Vd > 0 && H > 0 && H <= 65535 && ld_lat >= 0;
+    const long long weights = (long long)KR * D, all = weights * M * H;
+    return form && (weights <= 16 * 1024 || all <= (weights <= 32 * 1024 ? 8ll << 20 : 6ll << 20));
 }
 
 int launch_latent_step(const LatentStep& a, hipStream_t s, bool* taken) {
     *taken = false;
     const uintptr_t all = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.ukT) | reinterpret_cast<uintptr_t>(a.uv);
-    if (a.M <= 0 || a.M > kGemvMaxRows || (all & 15) != 0 || !latent_step_fits(a.H, a.D, a.R, a.KR, a.Vd, a.ldq, a.ld_lat) || !a.ws ||
+    if (a.M <= 0 || a.M > kGemvMaxRows || (all & 15) != 0 || !latent_step_fits(a.M, a.H, a.D, a.R, a.KR, a.Vd, a.ldq, a.ld_lat) || !a.ws ||
         a.ws_floats < (size_t)a.M * a.H * kAttnSplits * (a.KR + 2))
         return ZG_OK;
     ZG_REQUIRE(a.rot.dims % 2 == 0 && a.rot.dims <= a.R, ZG_ERR_ARG, "rotary: %d rotated dimensions of a part of %d", a.rot.dims, a.R);
