@@ -54,3 +54,16 @@ def test_infinite_weights(monkeypatch, form):
     ok = np.isfinite(ref).all(axis=1)
     assert ok.any() and not ok.all() and (np.isfinite(got).all(axis=1) == ok).all()
     tl.assert_close(got[ok], ref[ok], "float32", form)
+
+
+@pytest.mark.parametrize("rows", [40, 300, 505])
+def test_toy_products_stay_on_the_fp32_instruction(monkeypatch, rows):
+    """Products of fewer than 128 columns, the experts' gated ones among them: the same bits with the ring and without it, at any number of rows."""
+    cfg = tl.config([tl.hgrn2_layer(heads=2, dim=24, vdim=32, mlp=tl.moe_mlp(ff=64, experts=6, top=4)) for _ in range(2)], vocab=203, width=64)
+    w = tl.weights(cfg, seed=rows)
+    toks = tl.tokens(370 + rows, rows, cfg["vocab"])
+    monkeypatch.delenv("ZGPT2_LM_STREAM", raising=False)
+    got = run(cfg, w, toks)
+    monkeypatch.setenv("ZGPT2_LM_STREAM", "-1")
+    assert np.array_equal(got, run(cfg, w, toks))
+    tl.assert_close(got, lm_oracle.Model(cfg, w).forward(toks)[0], "float32", rows)

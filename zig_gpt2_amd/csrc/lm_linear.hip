@@ -1017,10 +1017,7 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
     ZG_REQUIRE(L.z_limit == 0x7fffffff, ZG_ERR_ARG, "linear: skipped batches are for steps of few rows");
     const bool rounded = L.A16 && !f32;
     const bool persistent = rounded && takes_persistent(L);
-    // (32-bit products of a few columns exist in toy models only.  There the last bits of a sum that cancels almost entirely can decide a
-    // row, and they stay what the fp32 instruction makes them: 5.5 us against 3.4 at K = 64.)
-    const bool toy = f32 && L.K < 128 && L.nz == 1;
-    if (!persistent && !toy) {
+    if (!persistent) {
         bool taken = false;
         ZG_TRY(launch_stream(L, f32, s, &taken));
         if (taken) return ZG_OK;
@@ -1036,7 +1033,7 @@ int launch_linear(const Linear& L, bool f32, hipStream_t s) {
         return launch_gemm_s4(L.A16, L.B, L.bias, L.C ? static_cast<void*>(L.C) : L.C16, L.M, L.N, pl, L.ldc, false, L.C == nullptr, 192, s);
     }
     const bool a_vec = rounded ? (reinterpret_cast<uintptr_t>(L.A16) & 15) == 0 && L.lda % 8 == 0 && L.a_zoff % 8 == 0 : p.a_vec != 0;
-    if (a_vec && p.b_vec && L.K % 8 == 0 && !L.z_group && !toy) {
+    if (a_vec && p.b_vec && L.K % 8 == 0 && !L.z_group && !toy_product(L, f32)) {
         if (f32) return launch_tiles<float, 3>(L, p, s);
         return rounded ? launch_tiles<bf16_t, 1>(L, p, s) : launch_tiles<float, 1>(L, p, s);
     }

@@ -296,7 +296,7 @@ int launch_form(const LinArgs& p, int nz, hipStream_t s) {
 }  // namespace
 
 bool stream_fits(const Linear& L, bool f32) {
-    if ((f32 ? !L.A : !L.A16) || L.z_group || L.a_glu || L.a_poly || L.a_norm || L.K < kBk || L.K % kBk != 0 || (L.C != nullptr) == (L.C16 != nullptr) || L.nz < 1 || L.nz > 65535 ||
+    if (toy_product(L, f32) || (f32 ? !L.A : !L.A16) || L.z_group || L.a_glu || L.a_poly || L.a_norm || L.K < kBk || L.K % kBk != 0 || (L.C != nullptr) == (L.C16 != nullptr) || L.nz < 1 || L.nz > 65535 ||
         (L.glu_out > 0 && L.glu_kind != GLU_SILU))
         return false;
     const int n_out = L.glu_out > 0 ? L.glu_out : L.N;
