@@ -64,9 +64,11 @@ def test_capped_scores(heads, kv_heads, dim, softcap, portions):
 
 
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
-def test_values_that_are_not_finite(bad):
-    """A row that is not finite reaches no block of 32 rows in front of its own."""
-    cfg = dl.config([dl.attn_layer(heads=4, kv_heads=2, dim=16, vdim=16, size=128, scale=0.25, mlp=dl.dense(ff=32))], width=48)
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("dim,vdim,size", [(16, 16, 128), (64, 64, 128), (32, 44, 40), (64, 28, 7)])
+def test_values_that_are_not_finite(dim, vdim, size, dtype, bad):
+    """A row that is not finite reaches the rows that see it and no others, those in front of it and of the next chunk in its block of 32 included."""
+    cfg = dl.config([dl.attn_layer(heads=4, kv_heads=2, dim=dim, vdim=vdim, size=size, scale=dim ** -0.5, mlp=dl.dense(ff=32))], width=48)
     w = dl.weights(cfg, seed=3)
     toks = dl.tokens(5, 90, cfg["vocab"])
     toks[toks == 7] = 8
@@ -74,9 +76,13 @@ def test_values_that_are_not_finite(bad):
     toks[75] = 7
     w["embed"] = w["embed"].copy()
     w["embed"][7, 3] = bad
-    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=512, max_seqs=2)
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=512, max_seqs=2)
     m.load_weights(w)
     got = m.step([(m.open(), toks, list(range(90)))])
     m.close()
-    assert not np.isfinite(got[75:]).any(axis=1).any()
-    assert np.abs(got[:64] - ref[:64]).max() < 3e-5 * np.abs(ref).max()
+    sees = np.array([r >= 75 and r // size == 75 // size for r in range(90)])
+    assert not np.isfinite(got[sees]).any(axis=1).any() and np.isfinite(got[~sees]).all()
+    if dtype == "float32":
+        assert np.abs(got[~sees] - ref[~sees]).max() < 3e-5 * np.abs(ref).max()
+    else:
+        tl.assert_close(got[~sees], ref[~sees], dtype)

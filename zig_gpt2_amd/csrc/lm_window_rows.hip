@@ -121,9 +121,40 @@ __global__ __launch_bounds__(512, 2) void window_rows_kernel(const RowsArgs a) {
     const int n_hi = min(n_blk - 1, blk.n_first + pos0 + r - blk.j_lo), n_lo = blk.n_first + mine.j_lo - blk.j_lo;
     const int n_keep = blk.n_first + max(0, mine.n_first - blk.j_lo);
     float mx = -INFINITY, l = 0.0f;
-    auto body = [&](int tile) {
+    auto file_keys = [&]() {  // the tile asked for last into the LDS
 #pragma unroll
         for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(s_k + (4 * i + (lane >> 4)) * 64 + ((lane & 15) ^ ((4 * i + (lane >> 4)) & 15)) * 4) = knext[i];
+    };
+    auto sees_all = [&](int tile) {  // every row sees every key of the tile
+        const int n0 = 32 * tile, j0 = blk.j_lo + n0 - blk.n_first;
+        return n0 >= blk.n_first && j0 >= lo_last && j0 + 31 <= pos0;
+    };
+    // the tile in the LDS against the queries; element i: key 8 (i / 4) + 4 half + i % 4 of the tile, query lane % 32
+    auto scores = [&](int tile, bool whole, f32x16& s) {
+        float kreg[kHalf];
+#pragma unroll
+        for (int t = 0; t < kHalf; t += 4) {
+            const f32x4 x = t < Dh ? *reinterpret_cast<const f32x4*>(s_k + r * 64 + (((kh * Dh + t) / 4) ^ (r & 15)) * 4) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            kreg[t] = x.x; kreg[t + 1] = x.y; kreg[t + 2] = x.z; kreg[t + 3] = x.w;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+        for (int t = 0; t < kHalf; ++t) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kreg[t], qreg[t], s, 0, 0, 0);
+        auto score_at = [&](int i) { return 32 * tile + 8 * (i >> 2) + 4 * kh + (i & 3); };
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = SHAPED ? shape_score(s[i] * a.scale, a.shape, h, pos0 + r - key_pos(blk, score_at(i))) : s[i] * a.scale;
+        if (!whole)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int n = score_at(i);
+                s[i] = n <= n_hi && (n >= n_lo || n < n_keep) ? s[i] : -INFINITY;
+            }
+    };
+    bool odd = false;  // some masked key may have values that are not finite
+    auto body = [&](int tile) {
+        file_keys();
         float v[CT][16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -133,31 +164,10 @@ __global__ __launch_bounds__(512, 2) void window_rows_kernel(const RowsArgs a) {
         }
         fetch();
         look_up(tile + 2 * a.ks);
-        float kreg[kHalf];
-#pragma unroll
-        for (int t = 0; t < kHalf; t += 4) {
-            const f32x4 x = t < Dh ? *reinterpret_cast<const f32x4*>(s_k + r * 64 + (((kh * Dh + t) / 4) ^ (r & 15)) * 4) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            kreg[t] = x.x; kreg[t + 1] = x.y; kreg[t + 2] = x.z; kreg[t + 3] = x.w;
-        }
-        __builtin_amdgcn_sched_barrier(0);
+        const bool whole = sees_all(tile);
         f32x16 s;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
-#pragma unroll
-        for (int t = 0; t < kHalf; ++t) s = __builtin_amdgcn_mfma_f32_32x32x2f32(kreg[t], qreg[t], s, 0, 0, 0);
-        // element i: key 8 (i / 4) + 4 half + i % 4 of the tile, query lane % 32
-        const int n0 = 32 * tile, j0 = blk.j_lo + n0 - blk.n_first;
-        const bool whole = n0 >= blk.n_first && j0 >= lo_last && j0 + 31 <= pos0;  // every row sees every key
+        scores(tile, whole, s);
         float top = -INFINITY;
-        auto score_at = [&](int i) { return n0 + 8 * (i >> 2) + 4 * kh + (i & 3); };
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = SHAPED ? shape_score(s[i] * a.scale, a.shape, h, pos0 + r - key_pos(blk, score_at(i))) : s[i] * a.scale;
-        if (!whole)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int n = score_at(i);
-                s[i] = n <= n_hi && (n >= n_lo || n < n_keep) ? s[i] : -INFINITY;
-            }
 #pragma unroll
         for (int i = 0; i < 16; ++i) top = fmaxf(top, s[i]);
         top = fmaxf(mx, both_halves_max(top));
@@ -176,6 +186,20 @@ __global__ __launch_bounds__(512, 2) void window_rows_kernel(const RowsArgs a) {
             s[i] = exp_of(s[i] - ref);
             l += s[i];
         }
+        if (!whole) {  // a masked weight is zero, but zero times a value that is not finite is not: such values wait until the other tiles are done
+            float z = 0.0f;
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) z = fmaf(v[c][i], 0.0f, z);
+            if (__builtin_expect(__any(z != z), 0)) {
+                odd = true;
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[c][i] = fabsf(v[c][i]) <= 3.4028235e38f ? v[c][i] : 0.0f;
+            }
+        }
 #pragma unroll
         for (int i = 0; i < 16; ++i)
 #pragma unroll
@@ -186,6 +210,34 @@ __global__ __launch_bounds__(512, 2) void window_rows_kernel(const RowsArgs a) {
         fetch();
         look_up(range + a.ks);
         for (int tile = range; tile < n_tiles; tile += a.ks) body(tile);
+    }
+    if (__builtin_expect(odd, 0)) {  // what waited, key by key, for the rows that see it
+        const float ref = mx == -INFINITY ? 0.0f : mx;
+#pragma unroll 1
+        for (int tile = range; tile < n_tiles; tile += a.ks) {
+            if (sees_all(tile)) continue;
+            look_up(tile);
+            fetch();
+            file_keys();
+            f32x16 s;
+            scores(tile, false, s);
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s_k[(8 * (i >> 2) + 4 * kh + (i & 3)) * 32 + r] = exp_of(s[i] - ref);  // (the keys have been used)
+#pragma unroll 1
+            for (int key = 0; key < 32; ++key) {
+                const int n = 32 * tile + key;
+                const float* vr = row_of(key) + v_at;
+                const float p = s_k[key * 32 + r];
+                const bool sees = n <= n_hi && (n >= n_lo || n < n_keep);
+#pragma unroll
+                for (int c = 0; c < CT; ++c)
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) {
+                        const float y = vr[min(c * 32 + 8 * (x >> 2) + 4 * kh + (x & 3), a.V - 1)];
+                        if (sees && !(fabsf(y) <= 3.4028235e38f)) o[c][x] = fmaf(p, y, o[c][x]);
+                    }
+            }
+        }
     }
     __syncthreads();
     l += __shfl_xor(l, 32, 64);  // (the halves hold different keys' weights)
