@@ -48,3 +48,37 @@ def test_windows_with_kept_tokens(heads, kv_heads, dim, vdim, window, keep, n):
     cfg = sl.config([sl.pair_layer(heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, window=window, keep_first=keep)])
     w = sl.weights(cfg, seed=dim + window)
     check(cfg, w, lambda t: so.forward(w, cfg, t)[0], sl.tokens, n)
+
+
+@pytest.mark.parametrize("n", [1, 3])
+@pytest.mark.parametrize("dim,vdim", [(8, 8), (68, 128)])
+def test_scores_of_minus_infinity(dim, vdim, n):
+    """Keys whose scores fall below what fp32 holds weigh nothing, a whole share of them too."""
+    cfg = dl.config([dl.attn_layer(heads=2, kv_heads=1, dim=dim, vdim=vdim, size=None, rot_dims=0, scale=1.0, mlp=None)], vocab=89, width=48)
+    w = dl.weights(cfg, seed=dim)
+    q, k = (next(x for x in w if x.endswith(leaf)) for leaf in ("mix.q", "mix.k"))
+    w["embed"] = w["embed"].copy()
+    w["embed"][:, 0] = 0.0
+    w["embed"][7, 0] = 1.0  # token 7: a key of -2^70 and more in its first channel
+    w["embed"][:, 1] = 1.0  # every token: a query of 2^70 there
+    w[q], w[k] = w[q].copy(), w[k].copy()
+    w[q][0::dim] = 0.0
+    w[q][0::dim, 1] = 2.0 ** 72
+    w[k][0] = 0.0
+    w[k][0, 0] = -(2.0 ** 72)
+    w[q][:, 0] = 0.0
+    w[k][1:, 0] = 0.0
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=1536, max_seqs=8)
+    m.load_weights(w)
+    toks = [dl.tokens(40 + b, 150 + 16 * b, cfg["vocab"]) for b in range(n)]
+    for b, t in enumerate(toks):
+        t[t == 7] = 8
+        t[16:130 + b] = 7
+    refs = [do.forward(w, cfg, t) for t in toks]
+    seqs = [m.open() for _ in toks]
+    m.step([(s, t[:-2], []) for s, t in zip(seqs, toks)])
+    for i in (-2, -1):
+        got = m.step([(s, [t[i]], [0]) for s, t in zip(seqs, toks)])
+        want = np.stack([r[i] for r in refs])
+        assert np.abs(got - want).max() < 3e-5 * np.abs(want).max(), (n, i)
+    m.close()

@@ -233,11 +233,11 @@ __global__ __launch_bounds__(256) void window_step_kernel(const int* row_pos, co
     __syncthreads();
     for (int o = tid; o < rep * V; o += 256) {
         const int h = o / V, ch = o % V;
-        const float top = fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h]));
+        const float top = fmaxf(fmaxf(s_m[0][h], s_m[1][h]), fmaxf(s_m[2][h], s_m[3][h])), ref = top == -INFINITY ? 0.0f : top;
         float v = 0.0f, lt = 0.0f;
 #pragma unroll
         for (int w = 0; w < 4; ++w) {
-            const float f = expf(s_m[w][h] - top);  // (a wave without keys: exp(-inf) = 0)
+            const float f = expf(s_m[w][h] - ref);  // (a wave without keys, or whose scores are all minus infinity: 0)
             v = fmaf(f, s_acc[w][h][ch], v);
             lt = fmaf(f, s_l[w][h], lt);
         }
