@@ -109,3 +109,40 @@ def test_convolutions_of_the_mixers(design, n_seqs):
         m.close()
     for a, b in zip(*runs):
         assert np.array_equal(a, b)
+
+
+def against_single_steps(lib, cfg, dtype, n_seqs, n=24):
+    w = lib.weights(cfg, seed=5)
+    prompts = [lib.tokens(b, 2 + 4 * b, cfg["vocab"]) for b in range(n_seqs)]
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=1024, max_seqs=8, page_tokens=8, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append([m.generate(prompts, n), m.generate(prompts[:1], n)])
+        m.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("n_seqs", [1, 3, 8])
+@pytest.mark.parametrize("loop", [{"start": 0, "stop": 3, "times": 2}, {"start": 1, "stop": 2, "times": 3}, {"start": 2, "stop": 3, "times": 2}])
+def test_looped_stacks(loop, n_seqs):
+    cfg = tl.config([tl.hgrn2_layer(mlp=tl.moe_mlp()), tl.latent_layer(mlp=None), tl.hgrn2_layer(mlp=tl.dense_mlp())], width=48, loop=loop)
+    cfg.update(logit_scale=0.5, logit_softcap=3.0)
+    against_single_steps(tl, cfg, "float32", n_seqs)
+
+
+@pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
+@pytest.mark.parametrize("width", [1020, 1024, 1028])
+def test_widths_around_what_a_wave_holds(width, dtype):
+    """Rows of more than 1024 columns are not handed on inside a step: the kernels of single steps there, links of a chain up to it."""
+    for n_seqs in (1, 3):
+        against_single_steps(tl, tl.config([tl.hgrn2_layer(mlp=tl.moe_mlp()), tl.latent_layer(mlp=tl.dense_mlp())], width=width), dtype, n_seqs)
+        against_single_steps(dl, dl.config([dl.mamba_layer(mlp=dl.dense()), dl.attn_layer(mlp=None), dl.latent_layer(mlp=dl.dense())], width=width), dtype, n_seqs)
+        against_single_steps(gl, without_canon([gl.delta_layer(mlp=gl.moe_mlp()), gl.parallel_layer(mlp=None)], width=width), dtype, n_seqs)
+
+
+@pytest.mark.parametrize("design", sorted(DESIGNS) + sorted(CONVOLVED))
+def test_bfloat16(design):
+    lib, cfg = DESIGNS[design] if design in DESIGNS else (gl, CONVOLVED[design])
+    against_single_steps(lib, cfg, "bfloat16", 8, 40)
