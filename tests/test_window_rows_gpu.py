@@ -63,6 +63,32 @@ def test_capped_scores(heads, kv_heads, dim, softcap, portions):
     check(cfg, w, lambda t: vo.forward(w, cfg, t), vl.tokens, portions)
 
 
+@pytest.mark.parametrize("n", [9, 33])
+@pytest.mark.parametrize("heads,kv_heads,dim,size", [(5, 1, 64, None), (12, 2, 16, 100), (21, 3, 8, None), (3, 3, 32, 33)])
+def test_many_sequences_of_one_row(heads, kv_heads, dim, size, n):
+    """Blocks of one row each, beside one of many rows: workgroups of every number of heads, the last of a key head's with fewer."""
+    cfg = dl.config([dl.attn_layer(heads=heads, kv_heads=kv_heads, dim=dim, vdim=12, size=size, scale=dim ** -0.5, mlp=dl.dense(ff=32))], width=48)
+    w = dl.weights(cfg, seed=heads)
+    for dtype in ("float32", "bfloat16"):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype=dtype, max_tokens=8192, max_seqs=n, max_step_tokens=256)
+        m.load_weights(w)
+        starts = [(37 * b + 5) % 150 for b in range(n)]
+        toks = [dl.tokens(40 + b, k + 45, cfg["vocab"]) for b, k in enumerate(starts)]
+        refs = [do.forward(w, cfg, t) for t in toks]
+        seqs = [m.open() for _ in toks]
+        for s, t, k in zip(seqs, toks, starts):
+            m.step([(s, t[:k], [])])
+        for more in (1, 40):  # every sequence a row; then the last one forty of them
+            got = m.step([(s, t[k:k + (more if b == n - 1 else 1)], [0]) for b, (s, t, k) in enumerate(zip(seqs, toks, starts))])
+            want = np.stack([r[k] for r, k in zip(refs, starts)])
+            if dtype == "float32":
+                assert np.abs(got - want).max() < 3e-5 * np.abs(want).max(), more
+            else:
+                tl.assert_close(got, want, dtype, more)
+            starts = [k + 1 for k in starts]
+        m.close()
+
+
 @pytest.mark.parametrize("bad", [np.inf, np.nan])
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
 @pytest.mark.parametrize("dim,vdim,size", [(16, 16, 128), (64, 64, 128), (32, 44, 40), (64, 28, 7)])

@@ -253,6 +253,7 @@ struct zg_lm {
     bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
     size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
     int step_longest = 0;  // rows of the longest entry of the running portion
+    int step_blocks = 0;   // blocks of 32 rows of its entries
     int step_keys = 0;  // positions the longest sequence of the running portion has reached (what its rows can see at most)
     // by rows of the step (one per entry) and, where whole-context attention splits a row's keys into shares, by the length bucket
     // of the longest sequence (512, 1024, ... tokens): a share then holds a few dozen keys at any length
@@ -1190,6 +1191,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                     WindowStep ws;
                     ws.q = g->proj; ws.ldq = LD; ws.ldo = HV; ws.M = M; ws.H = H; ws.G = G; ws.D = D; ws.V = Vd; ws.scale = d.scale; ws.mask = mask;
                     ws.row_pos = d_pos; ws.row_slot = d_slot; ws.page_table = g->page_table; ws.max_pages = g->max_pages; ws.page_tokens = g->P; ws.cache = ps.cache;
+                    ws.keys = key_cap; ws.blocks = g->step_blocks;
                     ZG_TRY(launch_window_rows(ws, d_estart, d_elen, n_ent, o16, s, &rounded));
                     done = rounded;
                 }
@@ -1198,7 +1200,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 else
                     ZG_TRY(launch_window_attention_split(g->proj, LD, g->o, HV, M, H, G, D, Vd, d.scale, mask, nullptr, nullptr, nullptr, d_pos, d_slot,
                                                          g->page_table, g->max_pages, g->P, ps.cache, key_cap, g->win_ws, g->win_ws_floats, d_estart,
-                                                         d_elen, n_ent, s, &done));
+                                                         d_elen, n_ent, s, &done, nullptr, 0, 1.0f, ScoreShape(), g->step_blocks));
             }
             if (!done) {
                 ScoreShape shape;
@@ -1269,7 +1271,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             ZG_TRY(launch_window_attention_split(g->ta, CC, g->o, OC, M, H, G, D, Vd, d.scale, KeyMask{d.window, d.keep_first, 0}, nullptr, nullptr, nullptr, d_pos,
                                                  d_slot, g->page_table, g->max_pages, g->P, ps.cache,
                                                  d.window > 0 ? d.window + d.keep_first : g->max_pages * g->P, g->win_ws, g->win_ws_floats, d_estart,
-                                                 d_elen, n_ent, s, &split, g->proj + og, NP, d.left_scale));  // (the gate where the shares meet)
+                                                 d_elen, n_ent, s, &split, g->proj + og, NP, d.left_scale, ScoreShape(), g->step_blocks));  // (the gate where the shares meet)
             if (!split) {
                 ZG_TRY(launch_window_attention(g->ta, CC, g->o, OC, M, H, G, D, Vd, d.scale, KeyMask{d.window, d.keep_first, 0}, nullptr, nullptr, nullptr, d_pos,
                                                d_slot, g->page_table, g->max_pages, g->P, ps.cache, s));
@@ -1374,7 +1376,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             bool split = false;
             ZG_TRY(launch_window_attention_split(g->proj, NP, g->o, HD, M, H, G, D, D, d.scale, KeyMask(), nullptr, nullptr, nullptr, d_pos, d_slot,
                                                  g->page_table, g->max_pages, g->P, ps.cache, key_cap, g->win_ws, g->win_ws_floats, d_estart, d_elen,
-                                                 n_ent, s, &split, nullptr, 0, 1.0f, shape));
+                                                 n_ent, s, &split, nullptr, 0, 1.0f, shape, g->step_blocks));
             if (!split)
                 ZG_TRY(launch_window_attention(g->proj, NP, g->o, HD, M, H, G, D, D, d.scale, KeyMask(), nullptr, nullptr, nullptr, d_pos, d_slot,
                                                g->page_table, g->max_pages, g->P, ps.cache, s, shape));
@@ -1740,12 +1742,13 @@ int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair
     int r = 0;
     g->step_keys = 0;
     g->step_key_tiles = 0;
-    g->step_longest = 0;
+    g->step_longest = g->step_blocks = 0;
     for (int e = 0; e < n_ent; ++e) {
         const Piece& pc = pieces[e];
         g->step_keys = std::max(g->step_keys, pc.pos0 + pc.n);
         g->step_longest = std::max(g->step_longest, pc.n);
         g->step_key_tiles += (pc.pos0 + pc.n + 31) / 32;
+        g->step_blocks += (pc.n + 31) / 32;
         ent_start[e] = r;
         ent_len[e] = pc.n;
         ent_slot[e] = pc.slot;

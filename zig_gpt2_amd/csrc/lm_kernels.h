@@ -450,6 +450,7 @@ struct WindowStep {
     int ld_gate = 0;
     float out_factor = 1.0f;
     ScoreShape shape;
+    int keys = 0, blocks = 0;  // (portions) the most keys a row sees; blocks of 32 rows of an entry, 0: not counted
 };
 int launch_window_step(const WindowStep& a, hipStream_t s, bool* taken);
 // Prompt portions, no mixing matrix, values as they are, heads of whole pieces of eight channels up to 64 (values of four): the attention in one
@@ -461,8 +462,8 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
                                   const float* sink, const float* talk, const float* vfreq, const int* row_pos, const int* row_slot,
                                   const int* page_table, int max_pages, int page_tokens, const float* cache, int key_capacity, float* ws,
                                   size_t ws_floats, const int* ent_start, const int* ent_len, int n_entries, hipStream_t s, bool* taken,
-                                  const float* out_gate = nullptr, int ld_gate = 0, float out_factor = 1.0f, ScoreShape shape = ScoreShape());
-// (out_gate != null: a taken step multiplies the result by sigmoid(out_gate[m][.]) * out_factor where the shares are added)
+                                  const float* out_gate = nullptr, int ld_gate = 0, float out_factor = 1.0f, ScoreShape shape = ScoreShape(), int blocks = 0);
+// (blocks: of 32 rows of an entry, 0: not counted.  out_gate != null: a taken step multiplies the result by sigmoid(out_gate[m][.]) * out_factor where the shares are added)
 
 // ------------------------------------------------------------------------------------------------ attention with sigmoid weights
 // out[m][h] = sum_j sigmoid(scale q_h . k(j) + bias[h]) value(j) over the keys the mask shows (windows and chunks; no kept tokens), q rows

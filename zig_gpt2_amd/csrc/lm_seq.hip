@@ -1407,7 +1407,7 @@ size_t window_split_workspace(int rows, int H, int V, int key_capacity, int* n_s
 int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, int M, int H, int G, int D, int V, float scale, KeyMask mask, const float* sink, const float* talk, const float* vfreq, const int* row_pos, const int* row_slot,
                                   const int* page_table, int max_pages, int page_tokens, const float* cache, int key_capacity, float* ws,
                                   size_t ws_floats, const int* ent_start, const int* ent_len, int n_entries, hipStream_t s, bool* taken,
-                                  const float* out_gate, int ld_gate, float out_factor, ScoreShape shape) {
+                                  const float* out_gate, int ld_gate, float out_factor, ScoreShape shape, int blocks) {
     *taken = false;
     if (M <= 0 || shape.gate) return ZG_OK;  // (weights that need no statistics: launch_gate_attention)
     if (mask.window <= 0) mask.keep = 0;
@@ -1426,6 +1426,7 @@ int launch_window_attention_split(const float* q, int ldq, float* out, int ldo, 
         w.q = q; w.ldq = ldq; w.out = out; w.ldo = ldo; w.M = M; w.H = H; w.G = G; w.D = D; w.V = V; w.scale = scale; w.mask = mask; w.sink = sink; w.row_pos = row_pos;
         w.row_slot = row_slot; w.page_table = page_table; w.max_pages = max_pages; w.page_tokens = page_tokens; w.cache = const_cast<float*>(cache); w.n_split = n_split;
         w.ws = ws; w.ws_floats = ws_floats; w.out_gate = out_gate; w.ld_gate = ld_gate; w.out_factor = out_factor; w.shape = shape;
+        w.keys = key_capacity; w.blocks = blocks;
         ZG_TRY(launch_window_step(w, s, taken));
         if (!*taken) ZG_TRY(launch_window_rows(w, ent_start, ent_len, n_entries, nullptr, s, taken));
         if (*taken) return ZG_OK;

@@ -299,11 +299,20 @@ int launch_window_rows(const WindowStep& w, const int* ent_start, const int* ent
     a.ent_start = ent_start; a.ent_len = ent_len; a.row_pos = w.row_pos; a.row_slot = w.row_slot; a.page_table = w.page_table;
     a.mask = w.mask; a.shape = w.shape; a.scale = w.scale; a.out_factor = w.out_factor;
     a.ldq = w.ldq; a.ldo = w.ldo; a.ld_gate = w.ld_gate; a.H = w.H; a.G = w.G; a.D = w.D; a.V = w.V; a.max_pages = w.max_pages; a.page_tokens = w.page_tokens; a.n_entries = n_entries;
-    // Heads of a workgroup and ranges of the keys: four and two once they fill half the chip, fewer heads and more ranges below.  us, one : two :
-    // four heads: 64 blocks of 32 rows (256 keys at most) 46 : 41 : 36, 58 (512 keys) 62 : 59 : 60, 16 (512 keys) 31 : 33 : 54.
-    const int blocks = (w.M + 31) / 32 + n_entries;
+    // Heads of a workgroup (its waves beyond them share the keys).  A compute unit has room for one workgroup, so the price is rounds of 256 workgroups
+    // times a wave's longest range of the keys, in tiles of 32, and two tiles for the rest; fewer heads read the keys more often and have to
+    // promise a tenth.  The grid holds counted blocks alone: with empty ones among 256 the last were a round of their own.  us a layer, one : two : four
+    // heads (or the two named): 64 blocks of 12 heads on 3 (256 keys at most) 46 : 41 : 36, 58 (512) 62 : 59 : 60, 16 (512) 31 : 33 : 54; 16 sequences of one row,
+    // 16 heads on 4 behind 4000 keys one 136, two 233; 32 sequences, 10 heads on 2 behind 4000 keys two 224, four 419; 25 heads on 5 behind 1000 two 142, four
+    // 227; 48 sequences, 24 heads on 4 behind 100 keys two 71, four 69; 200 rows of 32 heads on 8 behind 4000 keys one 156, two 269.
+    const int blocks = w.blocks > 0 ? w.blocks : (w.M + 31) / 32 + n_entries;
+    auto price = [&](int hw) {
+        const long long groups = (long long)blocks * w.G * ((rep + hw - 1) / hw);
+        return (double)((groups + 255) / 256) * (2.0 + (double)w.keys / (32 * (8 / hw)));
+    };
     a.hw = std::min(rep, 4);
-    while (a.hw > 1 && (long long)blocks * w.G * ((rep + a.hw - 1) / a.hw) < 128) a.hw = (a.hw + 1) / 2;
+    for (int hw = a.hw - 1; hw >= 1; --hw)
+        if (price(hw) < 0.9 * price(a.hw)) a.hw = hw;
     a.ks = 8 / a.hw;
     const dim3 grid(blocks, w.G * ((rep + a.hw - 1) / a.hw));
     if (grid.y > 65535) return ZG_OK;
