@@ -18,7 +18,7 @@ namespace {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-constexpr int kRows = 64, kPairs = 32, kPitch = 64 * 2 + 16;
+constexpr int kRows = 64, kPitch = 64 * 2 + 16;
 
 // D = 16 DK.  A workgroup: a head, 256 columns of its latent (a wave 64, whose weights it keeps), `blocks` times 64 rows one after the other.
 template <int DK>

@@ -551,10 +551,9 @@ int launch_moe_combine(const float* x, float* out, const float* yexp, const int*
                        hipStream_t s);
 
 // ------------------------------------------------------------------------------------------------ sampling support
-// rows of the next step of a generation: ids[r] = seen[r] = tok[r], pos[r] += 1  (seen: pinned host memory)
 // What stands between two steps of a generation that takes the largest logit (rows of up to 1024 values in whole 16-byte pieces): the token from
 // the partial maxima of launch_argmax_parts, the row's metadata moved on and the token handed to the host (the place in its ring by the
-// row's count), its embedding, and the first pass's norm with the token shift.  The shift's state takes the row of the token this step
+// row's count of the generation's steps), its embedding, and the first pass's norm with the token shift.  The shift's state takes the row of the token this step
 // consumed (last_h), whose place the new row takes; the new one is consumed by the next step, if there is one.
 struct NextToken {
     const float* part_val = nullptr;
@@ -570,6 +569,7 @@ struct NextToken {
 };
 int launch_argmax_parts(const float* logits, int rows, int n, float* part_val, int* part_idx, int* n_parts, hipStream_t s);
 int launch_next_token(const NextToken& a, int M, hipStream_t s);
+// rows of the next step of a generation: ids[r] = seen[r] = tok[r], pos[r] += 1  (seen: pinned host memory)
 int launch_advance_rows(const int* tok, int M, int* ids, int* pos, int* seen, hipStream_t s);
 // entries of the page table that such a step adds, one a row at most: table[at[i]] = page[i]
 struct NewPages {

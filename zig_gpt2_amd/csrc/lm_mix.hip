@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
 // Bound by the matrix cores and the LDS together: a fragment of keys (1 KB) serves one product (32 cycles), so the four SIMDs of a
 // compute unit ask the LDS for its whole 128 B per clock; two workgroups per compute unit hide the softmax of one under the
 // products of the other (hence 256 registers a lane: 72 of queries, 128 of sums).  The blocks with the most keys are dealt first.
-// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 132 us and 9 for the tiles (73 GFLOP: 520 TFLOP/s); 827 us when every workgroup
+// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 121 us and 9 for the tiles (73 GFLOP: 560 TFLOP/s); 827 us when every workgroup
 // converted and transposed its own tiles behind three barriers.
 template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
 __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, const bf16_t* qa16, float* ctx, bf16_t* ctx16, int H, int KR, int R, float scale,
@@ -1508,8 +1508,6 @@ __global__ __launch_bounds__(64) void new_pages_kernel(int* table, const NewPage
         if ((int)threadIdx.x == i && i < pages.n) table[pages.at[i]] = pages.page[i];
 }
 
-// Stage 1: block (row, part) finds the maximum and its first index in its slice of the row; stage 2 (parts == 1 in the grid,
-// n_parts > 0 as argument): one block per row combines the parts.  The first maximum wins; a row of NaNs gives index 0.
 // The largest of a workgroup's values and its index (the smaller one of equals), in every thread; s_v, s_i: four each.
 __device__ __forceinline__ void block_argmax(float& best, int& bi, float* s_v, int* s_i) {
     const float wbest = wave_allmax(best);
@@ -1578,6 +1576,8 @@ __global__ __launch_bounds__(256) void next_token_kernel(const NextToken a) {
     }
 }
 
+// Stage 1: block (row, part) finds the maximum and its first index in its slice of the row; stage 2 (parts == 1 in the grid,
+// n_parts > 0 as argument): one block per row combines the parts.  The first maximum wins; a row of NaNs gives index 0.
 __global__ __launch_bounds__(256) void row_argmax_kernel(const float* logits, int n, float* max_out, int* idx_out, float* part_val, int* part_idx,
                                                          int n_parts, int combine) {
     __shared__ float s_v[4];

@@ -13,7 +13,7 @@
 //
 // What bounds it: the fp32 matrix instruction (64 cycles per 32 x 32 x 2: 12.8 k cycles per chunk and head of 128 x 128 in the output
 // kernel, 4 k in the state kernel) and the chunk states, written, carried and read (64 KB per chunk and head).  8 x 1023 tokens, 8 heads of
-// 128 x 128: state 47 us, carry 29, output 77 = 153 us per layer; scanned token by token inside chunks it was 265 + 25 + 265.
+// 128 x 128: state 47 us, carry 27, output 77 = 151 us per layer; scanned token by token inside chunks it was 265 + 25 + 265.
 #include <math.h>
 #include <stdlib.h>
 

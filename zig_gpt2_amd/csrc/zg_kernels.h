@@ -258,7 +258,7 @@ constexpr int kWeightPlanes = 33;
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
 int launch_prefill_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, bool planes, int tm, int n_sp, const PrefillQkv& qa,
                         hipStream_t s);
-void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels) and the K slices
+void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
 // out[M][kSplit E] = split(causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t)
 // (attn_prefill.hip: bf16 matrix cores on exact plane splits; ws = fp32 workspace for the partials of split key ranges)
 int launch_attn_prefill(const float* qkv, bf16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache_or_null,
