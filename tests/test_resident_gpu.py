@@ -1,0 +1,141 @@
+"""Greedy decode of one sequence as a resident kernel (zig_gpt2_amd/csrc/decode_resident.hip) against the launch chain it replaces and
+the oracle: the edges of its shapes (64 positions of a workgroup, 64 steps of a launch, vocabularies that do not divide by the
+256 workgroups, XCDs with no, one and two heads), what a generation leaves behind, a withdrawn launch and a wait that runs out."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import oracle
+from golden_io import assert_greedy_ids_match
+from zig_gpt2_amd import _lib, synth
+from zig_gpt2_amd import gpt as zgpt
+
+pytestmark = pytest.mark.gpu
+
+# n_embed 384 (6 heads: two XCDs without), 512 (8), 768 (12: XCDs with one and with two)
+SHAPES = {
+    "384": synth.GPTConfig(1031, 130, 2, 6, 384),
+    "512": synth.GPTConfig(257, 129, 1, 8, 512),
+    "768": synth.GPTConfig(65, 200, 3, 12, 768),
+    "768-odd": synth.GPTConfig(12289, 66, 2, 12, 768),
+}
+
+
+def make(monkeypatch, cfg, w, resident, **kw):
+    monkeypatch.setenv("ZGPT2_RESIDENT", str(int(resident)))
+    m = zgpt.GPT(cfg, **kw)
+    m.load_weights(w)
+    return m
+
+
+def last_kernel():
+    name = C.create_string_buffer(160)
+    _lib.check(_lib.load().zg_debug_last_kernel(name, 160))
+    return name.value.decode()
+
+
+def rel(a, b):
+    return float(np.linalg.norm(np.float64(a) - np.float64(b)) / np.linalg.norm(np.float64(b)))
+
+
+@pytest.mark.parametrize("name", sorted(SHAPES))
+@pytest.mark.parametrize("f32", [False, True])
+def test_same_tokens_and_state_as_the_launch_chain(zg, monkeypatch, name, f32):
+    cfg = SHAPES[name]
+    w = synth.make_weights(cfg, seed=31, bf16=not f32)
+    res, chain = (make(monkeypatch, cfg, w, r, weights_f32=f32) for r in (True, False))
+    ctx = cfg.context_size
+    for plen, steps in ((1, 1), (1, 2), (3, ctx), (2, 64), (5, 65), (63, ctx), (64, ctx), (ctx - 1, ctx), (ctx, ctx), (9, 5)):
+        p = [synth.rand_tokens(300 + plen, plen, cfg.vocab_size)]
+        a, b = res.generate(p, steps), chain.generate(p, steps)
+        if steps > plen:
+            res.generate(p, steps)
+            assert "decode_resident_kernel" in last_kernel()
+        assert np.array_equal(a, b), (plen, steps)
+        # the residual stream, the pick and the cache it leaves: fp32 sums in another order
+        if steps > plen:
+            assert rel(res.hidden(), chain.hidden()) < 2e-6, (plen, steps)
+            assert np.array_equal(res.argmax(), chain.argmax())
+        if steps < ctx:
+            tok = a[:, -1]
+            assert rel(res.forward(steps + 1, tok), chain.forward(steps + 1, tok)) < 2e-6, (plen, steps)
+    res.close()
+    chain.close()
+
+
+def test_tokens_of_the_oracle(zg, monkeypatch):
+    cfg = SHAPES["384"]
+    w = synth.make_weights(cfg, seed=32, bf16=True)
+    m = make(monkeypatch, cfg, w, True)
+    p = synth.rand_tokens(321, 3, cfg.vocab_size)
+    ids = m.generate([p], cfg.context_size)[0]
+    assert "decode_resident_kernel" in last_kernel()
+    ref, lg = oracle.GPT(cfg, w).generate_greedy(p, cfg.context_size, want_logits=True)
+    top = np.sort(lg, axis=1)
+    assert_greedy_ids_match(ref[len(p):], ids[len(p):], top[:, -1], top[:, -2], "resident decode")
+    m.close()
+
+
+def test_nan_logits_pick_index_zero(zg, monkeypatch):
+    """As the chain: logits that are all NaN pick index 0, and the next generation on repaired weights is clean."""
+    cfg = SHAPES["768"]
+    w = synth.make_weights(cfg, seed=33, bf16=True)
+    m = make(monkeypatch, cfg, w, True)
+    p = [synth.rand_tokens(331, 2, cfg.vocab_size)]
+    want = m.generate(p, 70)
+    bad = dict(w)
+    bad["ln_f_g"] = np.full_like(w["ln_f_g"], np.nan)
+    m.load_weights(bad)
+    assert np.array_equal(m.generate(p, 70)[0][2:], np.zeros(68, np.uint64))
+    m.load_weights(w)
+    assert np.array_equal(m.generate(p, 70), want)
+    m.close()
+
+
+def test_withdrawn_launch_runs_on_the_chain(zg, monkeypatch):
+    """No patience at the start: every workgroup leaves before it has touched anything, and the launch chain makes up for it, also
+    where another call than the fetch asks first.  The handle then stays on the chain for some generations."""
+    cfg = SHAPES["768"]
+    w = synth.make_weights(cfg, seed=34, bf16=True)
+    p = [synth.rand_tokens(341, 5, cfg.vocab_size)]
+    chain = make(monkeypatch, cfg, w, False)
+    want = chain.generate(p, 150)
+    hid = chain.hidden()
+    monkeypatch.setenv("ZGPT2_RESIDENT_START", "0")
+    m = make(monkeypatch, cfg, w, True)
+    assert np.array_equal(m.generate(p, 150), want)
+    for _ in range(8):
+        assert np.array_equal(m.generate(p, 150), want)
+    m.generate_enqueue(p, 150)  # tried again, withdrawn again
+    assert rel(m.hidden(), hid) < 2e-6
+    assert np.array_equal(m.generate_fetch(150), want)
+    m.close()
+    chain.close()
+
+
+def test_wait_that_runs_out_fails_the_call(zg, monkeypatch):
+    cfg = SHAPES["512"]
+    w = synth.make_weights(cfg, seed=35, bf16=True)
+    p = [synth.rand_tokens(351, 2, cfg.vocab_size)]
+    monkeypatch.setenv("ZGPT2_TAG_SPIN_LIMIT", "0")
+    m = make(monkeypatch, cfg, w, True)
+    monkeypatch.delenv("ZGPT2_TAG_SPIN_LIMIT")
+    with pytest.raises(_lib.ZgError, match="timed out"):
+        m.generate(p, 129)
+    m.close()
+
+
+def test_what_the_chain_keeps(zg, monkeypatch):
+    """Narrow caches, several sequences, sampling, no graph: the launch chain, as before."""
+    cfg = SHAPES["512"]
+    w = synth.make_weights(cfg, seed=36, bf16=True)
+    for kw in ({"kv_f16": True}, {"kv_b24": True}, {"use_graph": False}, {"batch": 2}):
+        m = make(monkeypatch, cfg, w, True, **kw)
+        m.generate([synth.rand_tokens(361, 2, cfg.vocab_size)] * m.batch, 20)
+        assert "decode_resident_kernel" not in last_kernel(), kw
+        m.close()
+    m = make(monkeypatch, cfg, w, True)
+    m.generate_sample([synth.rand_tokens(361, 2, cfg.vocab_size)], 20, 0.8, seed=3)
+    assert "decode_resident_kernel" not in last_kernel()
+    m.close()

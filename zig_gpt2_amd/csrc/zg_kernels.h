@@ -314,6 +314,42 @@ struct SampleParams {
 int launch_sample_step(float* logits, int batch, int vocab, const SampleParams* params, const StepCtrl* ctrl, const float* part_val, int n_part,
                        int part_stride, float* seg_ws, int* token_out, hipStream_t s);
 
+// ------------------------------------------------------------------------------------ resident decode (decode_resident.hip)
+struct ResidentCtl {
+    unsigned done;  // steps of the generation that resident launches have finished
+    unsigned pad[31];
+    // zeroed in front of every launch
+    unsigned reg[8];  // workgroups registered by XCD
+    unsigned total;   // in all
+    unsigned state;   // 0 open, 1 committed: all workgroups are resident, 2 withdrawn
+    unsigned pad2[22];
+};
+struct ResidentArgs {
+    // layer 0; the others lie w_stride / kv_stride bytes apart
+    const void *c_attn_w, *c_proj_w, *c_fc_w, *mlp_proj_w;
+    const float *ln_1_g, *c_attn_c2, *c_attn_c3, *c_proj_b, *ln_2_g, *c_fc_c2, *c_fc_c3, *mlp_proj_b;
+    size_t w_stride, kv_stride;
+    char *k_cache, *v_cache;  // fp32, [head][ctx][64]
+    const void *wte, *wpe;
+    const float *ln_f_g, *ln_f_b;
+    int n_layer, n_heads, ctx, vocab;
+    int n_prompt, s0, s1;  // steps s0 .. s1 - 1 of the generation
+    const int* prompt;
+    int *out_tokens, *cur_token;
+    StepCtrl* ctrl;
+    float *x, *logits, *part_val;
+    int* part_idx;
+    int n_part;
+    unsigned long long* words;  // resident_words(n_embed), zeroed once; tags tag0 .. tag0 + (s1 - s0) (n_layer + 1) - 1 are this launch's alone
+    ResidentCtl* ctl;
+    unsigned tag0;
+    unsigned spin_limit, start_limit;
+    unsigned *fault, *withdrawn;  // pinned host words
+};
+bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx);
+size_t resident_words(size_t n_embed);
+int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s);
+
 // ------------------------------------------------------------------------------------ multi-GPU (dist.hip)
 int dist_broadcast(void* buf, size_t bytes, int root, hipStream_t s);  // in place, over the communicator of zg_dist_init
 
