@@ -33,9 +33,9 @@ def zg():
     yield lib
 
 
-# files whose subject is the launch chain of one sequence: it stays the path of narrow caches, private streams, sampling and every
-# shape the resident kernel has not been built for
-LAUNCH_CHAIN = {"test_prefetch_gpu.py"}
+# files whose subject is the launch chain: it stays the path of narrow caches, private streams, sampling and every shape the resident
+# kernels have not been built for
+LAUNCH_CHAIN = {"test_prefetch_gpu.py", "test_planes_gpu.py"}
 
 
 @pytest.fixture(autouse=True)

@@ -1,6 +1,7 @@
-"""Greedy decode of one sequence as a resident kernel (zig_gpt2_amd/csrc/decode_resident.hip) against the launch chain it replaces and
-the oracle: the edges of its shapes (64 positions of a workgroup, 64 steps of a launch, vocabularies that do not divide by the
-256 workgroups, XCDs with no, one and two heads), what a generation leaves behind, a withdrawn launch and a wait that runs out."""
+"""Greedy decode as resident kernels (zig_gpt2_amd/csrc/decode_resident.hip: one sequence, decode_resident_batch.hip: two to eight)
+against the launch chain they replace and the oracle: the edges of their shapes (64 positions of a workgroup, 64 steps of a launch,
+vocabularies that do not divide by the 256 workgroups, XCDs with no, one and two heads, sequences a tile of terms is not filled by),
+what a generation leaves behind, a withdrawn launch and a wait that runs out."""
 import ctypes as C
 
 import numpy as np
@@ -16,7 +17,7 @@ pytestmark = pytest.mark.gpu
 # n_embed 384 (6 heads: two XCDs without), 512 (8), 768 (12: XCDs with one and with two)
 SHAPES = {
     "384": synth.GPTConfig(1031, 130, 2, 6, 384),
-    "512": synth.GPTConfig(257, 129, 1, 8, 512),
+    "512": synth.GPTConfig(257, 129, 2, 8, 512),
     "768": synth.GPTConfig(65, 200, 3, 12, 768),
     "768-odd": synth.GPTConfig(12289, 66, 2, 12, 768),
 }
@@ -64,46 +65,72 @@ def test_same_tokens_and_state_as_the_launch_chain(zg, monkeypatch, name, f32):
     chain.close()
 
 
-def test_tokens_of_the_oracle(zg, monkeypatch):
+@pytest.mark.parametrize("name", sorted(SHAPES))
+@pytest.mark.parametrize("batch", [2, 3, 4, 5, 8])
+def test_lock_step_batch_same_tokens_and_state_as_the_launch_chain(zg, monkeypatch, name, batch):
+    cfg = SHAPES[name]
+    w = synth.make_weights(cfg, seed=38, bf16=True)
+    res, chain = (make(monkeypatch, cfg, w, r, batch=batch) for r in (True, False))
+    ctx = cfg.context_size
+    for plen, steps in ((1, 1), (2, 64), (6, ctx), (3, 65), (ctx, ctx)):
+        p = [synth.rand_tokens(380 + plen + 7 * b, max(1, plen - b), cfg.vocab_size) for b in range(batch)]  # ragged
+        a, b = res.generate(p, steps), chain.generate(p, steps)
+        res.generate(p, steps)
+        assert np.array_equal(a, b), (plen, steps)
+        if steps > min(len(q) for q in p):
+            assert "decode_resident_batch_kernel" in last_kernel()
+            assert rel(res.hidden(), chain.hidden()) < 2e-6, (plen, steps)
+            assert np.array_equal(res.argmax(), chain.argmax())
+        if steps < ctx:
+            assert rel(res.forward(steps + 1, a[:, -1]), chain.forward(steps + 1, a[:, -1])) < 2e-6, (plen, steps)
+    res.close()
+    chain.close()
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+def test_tokens_of_the_oracle(zg, monkeypatch, batch):
     cfg = SHAPES["384"]
     w = synth.make_weights(cfg, seed=32, bf16=True)
-    m = make(monkeypatch, cfg, w, True)
-    p = synth.rand_tokens(321, 3, cfg.vocab_size)
-    ids = m.generate([p], cfg.context_size)[0]
-    assert "decode_resident_kernel" in last_kernel()
-    ref, lg = oracle.GPT(cfg, w).generate_greedy(p, cfg.context_size, want_logits=True)
-    top = np.sort(lg, axis=1)
-    assert_greedy_ids_match(ref[len(p):], ids[len(p):], top[:, -1], top[:, -2], "resident decode")
+    m = make(monkeypatch, cfg, w, True, batch=batch)
+    prompts = [synth.rand_tokens(321 + b, 3 - b, cfg.vocab_size) for b in range(batch)]
+    ids = m.generate(prompts, cfg.context_size)
+    assert "decode_resident_" in last_kernel()
+    for p, got in zip(prompts, ids):
+        ref, lg = oracle.GPT(cfg, w).generate_greedy(p, cfg.context_size, want_logits=True)
+        top = np.sort(lg, axis=1)
+        assert_greedy_ids_match(ref[len(p):], got[len(p):], top[:, -1], top[:, -2], "resident decode")
     m.close()
 
 
-def test_nan_logits_pick_index_zero(zg, monkeypatch):
+@pytest.mark.parametrize("batch", [1, 5])
+def test_nan_logits_pick_index_zero(zg, monkeypatch, batch):
     """As the chain: logits that are all NaN pick index 0, and the next generation on repaired weights is clean."""
     cfg = SHAPES["768"]
     w = synth.make_weights(cfg, seed=33, bf16=True)
-    m = make(monkeypatch, cfg, w, True)
-    p = [synth.rand_tokens(331, 2, cfg.vocab_size)]
+    m = make(monkeypatch, cfg, w, True, batch=batch)
+    p = [synth.rand_tokens(331 + b, 2, cfg.vocab_size) for b in range(batch)]
     want = m.generate(p, 70)
     bad = dict(w)
     bad["ln_f_g"] = np.full_like(w["ln_f_g"], np.nan)
     m.load_weights(bad)
-    assert np.array_equal(m.generate(p, 70)[0][2:], np.zeros(68, np.uint64))
+    assert not m.generate(p, 70)[:, 2:].any()
     m.load_weights(w)
     assert np.array_equal(m.generate(p, 70), want)
     m.close()
 
 
-def test_withdrawn_launch_runs_on_the_chain(zg, monkeypatch):
+@pytest.mark.parametrize("batch", [1, 2])
+def test_withdrawn_launch_runs_on_the_chain(zg, monkeypatch, batch):
     """No patience at the start: every workgroup leaves before it has touched anything, and the launch chain makes up for it, also
     where another call than the fetch asks first.  The handle then stays on the chain for some generations."""
     cfg = SHAPES["768"]
     w = synth.make_weights(cfg, seed=34, bf16=True)
-    p = [synth.rand_tokens(341, 5, cfg.vocab_size)]
-    chain = make(monkeypatch, cfg, w, False)
+    p = [synth.rand_tokens(341 + b, 5, cfg.vocab_size) for b in range(batch)]
+    chain = make(monkeypatch, cfg, w, False, batch=batch)
     want = chain.generate(p, 150)
     hid = chain.hidden()
     monkeypatch.setenv("ZGPT2_RESIDENT_START", "0")
-    m = make(monkeypatch, cfg, w, True)
+    m = make(monkeypatch, cfg, w, True, batch=batch)
     assert np.array_equal(m.generate(p, 150), want)
     for _ in range(8):
         assert np.array_equal(m.generate(p, 150), want)
@@ -114,12 +141,13 @@ def test_withdrawn_launch_runs_on_the_chain(zg, monkeypatch):
     chain.close()
 
 
-def test_wait_that_runs_out_fails_the_call(zg, monkeypatch):
+@pytest.mark.parametrize("batch", [1, 4])
+def test_wait_that_runs_out_fails_the_call(zg, monkeypatch, batch):
     cfg = SHAPES["512"]
     w = synth.make_weights(cfg, seed=35, bf16=True)
-    p = [synth.rand_tokens(351, 2, cfg.vocab_size)]
+    p = [synth.rand_tokens(351, 2, cfg.vocab_size)] * batch
     monkeypatch.setenv("ZGPT2_TAG_SPIN_LIMIT", "0")
-    m = make(monkeypatch, cfg, w, True)
+    m = make(monkeypatch, cfg, w, True, batch=batch)
     monkeypatch.delenv("ZGPT2_TAG_SPIN_LIMIT")
     with pytest.raises(_lib.ZgError, match="timed out"):
         m.generate(p, 129)
@@ -127,15 +155,20 @@ def test_wait_that_runs_out_fails_the_call(zg, monkeypatch):
 
 
 def test_what_the_chain_keeps(zg, monkeypatch):
-    """Narrow caches, several sequences, sampling, no graph: the launch chain, as before."""
+    """Narrow caches, several sequences with fp32 weights, sampling, no graph, one layer: the launch chain, as before."""
     cfg = SHAPES["512"]
     w = synth.make_weights(cfg, seed=36, bf16=True)
-    for kw in ({"kv_f16": True}, {"kv_b24": True}, {"use_graph": False}, {"batch": 2}):
+    for kw in ({"kv_f16": True}, {"kv_b24": True}, {"use_graph": False}, {"batch": 2, "weights_f32": True}):
         m = make(monkeypatch, cfg, w, True, **kw)
         m.generate([synth.rand_tokens(361, 2, cfg.vocab_size)] * m.batch, 20)
-        assert "decode_resident_kernel" not in last_kernel(), kw
+        assert "decode_resident" not in last_kernel(), kw
         m.close()
+    one = synth.GPTConfig(257, 129, 1, 8, 512)
+    m = make(monkeypatch, one, synth.make_weights(one, seed=37, bf16=True), True)
+    m.generate([synth.rand_tokens(361, 2, one.vocab_size)], 20)
+    assert "decode_resident" not in last_kernel()
+    m.close()
     m = make(monkeypatch, cfg, w, True)
     m.generate_sample([synth.rand_tokens(361, 2, cfg.vocab_size)], 20, 0.8, seed=3)
-    assert "decode_resident_kernel" not in last_kernel()
+    assert "decode_resident" not in last_kernel()
     m.close()

@@ -238,7 +238,7 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
     g->sk_tiles = (int)((E + 15) / 16);
     g->sk_ws = (float*)P((size_t)g->sk_tiles * 4 * 128 * 4);
     g->sk_cnt = (int*)P((size_t)g->sk_tiles * 4 * 4);  // [tile][4]: the four-wave plane-fed kernel takes one ticket per wave
-    g->res_words_bytes = resident_words(E) * 8;
+    g->res_words_bytes = resident_words(E, B) * 8;
     g->res_words = (unsigned long long*)P(g->res_words_bytes);
     g->res_ctl = (ResidentCtl*)P(sizeof(ResidentCtl));
     g->pf_njobs = (int)(2 + 5 * L);
@@ -765,8 +765,8 @@ int pf_stop(zg_gpt* g, hipStream_t s) {
     return ZG_OK;
 }
 
-// The resident kernel takes greedy generations of one sequence on the library's stream: shapes it is built for, fp32 cache, all 256
-// compute units.  A handle with a private stream is one of several chains on the chip, and borrowed weights may be reloaded by
+// The resident kernels take greedy generations of one sequence, or of two to eight with bf16 weights, on the library's stream: shapes
+// they are built for, fp32 cache, all 256 compute units.  A handle with a private stream is one of several chains on the chip, and borrowed weights may be reloaded by
 // their owner before a withdrawn launch is made up for: both keep the launch chain.
 void setup_resident(zg_gpt* g) {
     g->res_on = g->res_gen = g->res_pending = false;
@@ -776,8 +776,8 @@ void setup_resident(zg_gpt* g) {
     g->res_withdrawn = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(g->h_ctrl) + 264);
     *g->res_withdrawn = 0;
     g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms (0: the test of a withdrawn launch)
-    if (g->batch != 1 || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
-    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size) || !env_int("ZGPT2_RESIDENT", 1)) return;
+    if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
+    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer) || !env_int("ZGPT2_RESIDENT", 1)) return;
     int cus = 0;
     g->res_on = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx().device) == hipSuccess && cus == 256;
 }
@@ -797,7 +797,7 @@ constexpr size_t kResidentSteps = 64;
 int enqueue_resident(zg_gpt* g, hipStream_t s) {
     const size_t L = g->cfg.n_layer;
     const size_t st = g->gen_pos, n = std::min(kResidentSteps, g->gen_n - st);
-    const unsigned tags = (unsigned)(n * (L + 1));
+    const unsigned tags = (unsigned)(n * (L + 2));
     if (g->res_tag > 0xffffffffu - tags) {  // tags start over: none of the old ones may be found
         ZG_HIP(hipMemsetAsync(g->res_words, 0, g->res_words_bytes, s));
         g->res_tag = 1;
@@ -814,6 +814,7 @@ int enqueue_resident(zg_gpt* g, hipStream_t s) {
     a.v_cache = reinterpret_cast<char*>(y.v_cache);
     a.wte = g->wte; a.wpe = g->wpe; a.ln_f_g = g->ln_f_g; a.ln_f_b = g->ln_f_b;
     a.n_layer = (int)L; a.n_heads = (int)g->cfg.n_heads; a.ctx = (int)g->cfg.context_size; a.vocab = (int)g->cfg.vocab_size;
+    a.batch = (int)g->batch; a.prompt_len = g->prompt_len; a.out_stride = (int)g->cfg.context_size; a.lm_c2 = g->lm_c2; a.lm_c3 = g->lm_c3;
     a.n_prompt = (int)g->gen_min_prompt; a.s0 = (int)st; a.s1 = (int)(st + n);
     a.prompt = g->prompt; a.out_tokens = g->out_tokens; a.cur_token = g->cur_token;
     a.ctrl = g->ctrl; a.x = g->x; a.logits = g->logits; a.part_val = g->part_val; a.part_idx = g->part_idx; a.n_part = g->lm_grid;
@@ -1557,6 +1558,7 @@ static int settle(zg_gpt* g) {
     ZG_TRY(check_fault(g));  // (launches behind a failed one withdraw as well)
     ++g->res_strikes;
     g->res_sit_out = 8;
+    g->res_tag = 0xffffffffu;  // (what was not written keeps an old tag: all words are cleared in front of the next launch)
     unsigned done = 0;
     ZG_HIP(hipMemcpy(&done, &g->res_ctl->done, sizeof done, hipMemcpyDeviceToHost));
     hipStream_t s = gs(g);

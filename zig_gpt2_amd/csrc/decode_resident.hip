@@ -28,75 +28,20 @@
 // Safety: every workgroup must be resident before any may wait for another.  Workgroups register; the last one commits, and
 // one that has waited too long withdraws the launch for all (a compare-and-swap decides, so all agree): then nothing has been
 // touched and the host runs the launch chain instead.  Behind the commitment every wait is bounded as well (fault word).
-#include "zg_common.h"
-#include "zg_kernels.h"
+#include "decode_resident_parts.h"
 #include "zg_once.h"
 
 namespace zg {
 
 namespace {
 
-constexpr int kXcds = 8, kRanks = 32;
+using namespace resident;
 constexpr int kFar = 32;         // words of a workgroup's partial sums: two cache lines of its own
 // Pauses, x 64 cycles, measured at 124M and the char model: before the first look at words of other XCDs (0: +4 %; 16: +1 %); before the
 // fetches of a Block, behind c_attn's words (0: +6 %) and behind the attention (4: +3 %)
 constexpr int kFarSleep = 8, kAfterA = 20, kAfterB = 12;
-constexpr float kNone = -1e30f;  // score of a position that is not there
-
-typedef unsigned long long u64;
-
-// A base that stays in scalar registers, an offset that is made again where it is used: without them the compiler keeps some
-// sixty loop-invariant 64-bit addresses of every lane in registers it then has to spill.
-typedef __attribute__((address_space(1))) char gchar;  // (said to be global memory: the compiler cannot see through the asm)
-typedef __attribute__((address_space(1))) u64 gword;
-template <typename T>
-using gptr = __attribute__((address_space(1))) T*;
-__device__ __forceinline__ gchar* base_at(const void* p, size_t off = 0) {
-    const char* q = reinterpret_cast<const char*>(p) + off;
-    asm volatile("" : "+s"(q));
-    return (gchar*)const_cast<char*>(q);
-}
-__device__ __forceinline__ unsigned fresh(unsigned v) {
-    asm volatile("" : "+v"(v));
-    return v;
-}
-
-// ------------------------------------------------------------------------------------------------ words with tags
-__device__ __forceinline__ u64 tagged(unsigned tag, float v) { return ((u64)tag << 32) | (u64)__float_as_uint(v); }
-__device__ __forceinline__ gword* word(const u64* base, unsigned i) { return (gword*)(base_at(base) + fresh(i * 8u)); }
-// word i of base.  Within the XCD: no bit of a wider scope, the word stays in this L2
-__device__ __forceinline__ void put_near(u64* base, unsigned i, u64 v) { __hip_atomic_store(word(base, i), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
-// for every XCD: written through
-__device__ __forceinline__ void put_far(u64* base, unsigned i, u64 v) { __hip_atomic_store(word(base, i), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
-
-struct Waiter {
-    unsigned limit;  // polls of one wait; 0 once one has run out
-    unsigned* fail;  // LDS
-    __device__ __forceinline__ u64 wait(const gword* p, unsigned tag) {
-        u64 v;
-        for (unsigned n = 0;; ++n) {
-            v = __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if ((unsigned)(v >> 32) == tag) break;
-            if (n >= limit) {
-                *fail = 1u;
-                limit = 0u;
-                break;
-            }
-        }
-        return v;
-    }
-    __device__ __forceinline__ float get(const u64* base, unsigned i, unsigned tag) { return __uint_as_float((unsigned)wait(word(base, i), tag)); }
-};
-
-// LDS is exchanged between waves, vector memory is not: loads in flight stay in flight (a __syncthreads() drains them)
-__device__ __forceinline__ void barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 // ------------------------------------------------------------------------------------------------ pieces of rows in registers
-typedef __attribute__((ext_vector_type(2))) float f32x2;
-typedef __attribute__((address_space(3))) char lds_char;
-__device__ __forceinline__ unsigned lds_at(const void* p) { return (unsigned)(uintptr_t)(lds_char*)(p); }
-template <typename T>
-__device__ __forceinline__ T lds_read(unsigned at) { return *(const __attribute__((address_space(3))) T*)(uintptr_t)at; }
 // N consecutive elements of a row, at a byte offset of 32 bits from a scalar base (the address costs a lane one register)
 template <typename WT, int N>
 struct Piece;
@@ -155,46 +100,6 @@ __device__ __forceinline__ void fma_piece(const Piece<WT, N>& w, const float* z,
 #pragma unroll
     for (int i = 0; i < N; ++i) acc[i & 3] = fmaf(w.at(i), z[i], acc[i & 3]);
 }
-template <int N>
-__device__ __forceinline__ void lds_floats(const float* p, float* out) {
-    if (N == 2) {
-        const float2 v = *reinterpret_cast<const float2*>(p);
-        out[0] = v.x;
-        out[1] = v.y;
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; i += 4) {
-            const f32x4 v = *reinterpret_cast<const f32x4*>(p + i);
-            out[i] = v.x; out[i + 1] = v.y; out[i + 2] = v.z; out[i + 3] = v.w;
-        }
-    }
-}
-
-// sum over eight consecutive lanes, on all of them, the same bits on all of them (commutative pairs)
-__device__ __forceinline__ float sum8(float v) {
-    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0xB1, 0xF, 0xF, true));
-    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x4E, 0xF, 0xF, true));
-    v += __uint_as_float(__builtin_amdgcn_update_dpp(0u, __float_as_uint(v), 0x141, 0xF, 0xF, true));
-    return v;
-}
-
-__device__ __forceinline__ void better(float& v, int& i, float ov, int oi) {  // the larger value, of equal ones the lower index
-    if (ov > v || (ov == v && oi < i)) {
-        v = ov;
-        i = oi;
-    }
-}
-
-__device__ __forceinline__ void argmax_wave(float& v, int& i) {  // on all lanes
-#define ZG_AM_STEP(N) better(v, i, dpp_row_ror<N>(v), __builtin_amdgcn_update_dpp(0, i, 0x120 | N, 0xF, 0xF, true));
-    ZG_AM_STEP(8) ZG_AM_STEP(4) ZG_AM_STEP(2) ZG_AM_STEP(1)
-#undef ZG_AM_STEP
-    const float rv = v;
-    const int ri = i;
-#pragma unroll
-    for (int q = 0; q < 64; q += 16) better(v, i, lane_value(rv, q), __builtin_amdgcn_readlane(ri, q));
-}
-
 // ------------------------------------------------------------------------------------------------ the words' places
 // per XCD: q | k | v of its heads, attention partials, x behind c_proj, h, x behind the MLP; then, for all: partial sums, picks
 template <int NW, int NH>
@@ -204,15 +109,6 @@ struct Places {
     static constexpr int far1 = kXcds * near_words, far2 = far1 + kXcds * kRanks * kFar, pick = far2 + kXcds * kRanks * kFar, words = pick + kXcds * 16;
 };
 
-// ------------------------------------------------------------------------------------------------ weights: memory -> LDS
-// 64 lanes x 16 bytes from the lanes' offsets into the LDS from `to` on.  In flight until vmcnt says otherwise.
-__device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t from, unsigned off, unsigned to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(to), "v"(off), "s"(from) : "memory", "m0");
-}
-template <int N>
-__device__ __forceinline__ void in_flight() {  // at most N of this wave's vector memory operations
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
 // The LDS, in bytes from the start of the dynamic part.  Blocks of weights end on whole turns of the four fetching waves (4 KiB).
 template <typename WT, int NW, int NH>
 struct Room {
@@ -266,27 +162,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
     // ---- register; all workgroups resident, or nobody starts
     if (tid == 0) {
         s_fail = 0u;
-        s_rank = __hip_atomic_fetch_add(&a.ctl->reg[xcc], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        const unsigned before = __hip_atomic_fetch_add(&a.ctl->total, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (before == (unsigned)(kXcds * kRanks) - 1u) {
-            bool ok = a.ctl->done == (unsigned)a.s0;  // the steps in front of these have run
-            for (int i = 0; i < kXcds; ++i) ok = ok && __hip_atomic_load(&a.ctl->reg[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)kRanks;
-            unsigned open = 0u;
-            __hip_atomic_compare_exchange_strong(&a.ctl->state, &open, ok ? 1u : 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        unsigned st = 0u;
-        for (unsigned n = 0;; ++n) {
-            st = __hip_atomic_load(&a.ctl->state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            if (st != 0u) break;
-            if (n >= a.start_limit) {
-                unsigned open = 0u;
-                __hip_atomic_compare_exchange_strong(&a.ctl->state, &open, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                st = open == 0u ? 2u : open;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
-        }
-        s_go = st;
+        s_go = join(a.ctl, xcc, (unsigned)a.s0, a.start_limit, &s_rank);
     }
     __syncthreads();
     if (s_go != 1u) {
@@ -853,14 +729,17 @@ int launch(const ResidentArgs& a, hipStream_t s) {
 
 }  // namespace
 
-bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx) {
-    if (n_heads * 64 != n_embed || n_heads > 16) return false;
+// (Two layers at least: the cache rows of the next step's first layer are requested during the last layer of this one, which has to be
+// another for the newest row to be known to have arrived.)
+bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer) {
+    if (n_heads * 64 != n_embed || n_heads > 16 || n_layer < 2) return false;
     const size_t nw = n_embed / 64;
     if (nw != 6 && nw != 8 && nw != 12) return false;
     return ctx <= 64 * (n_heads > 8 ? kRanks / 2 : kRanks);  // a workgroup attends to 64 positions of one head
 }
 
-size_t resident_words(size_t n_embed) {
+size_t resident_words(size_t n_embed, size_t batch) {
+    if (batch > 1) return resident_batch_words(n_embed);
     switch (n_embed / 64) {
         case 6: return Places<6, 1>::words;
         case 8: return Places<8, 1>::words;
@@ -870,9 +749,13 @@ size_t resident_words(size_t n_embed) {
 }
 
 int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s) {
-    ZG_REQUIRE(resident_shape((size_t)n_embed, (size_t)a.n_heads, (size_t)a.ctx) && a.s0 >= 0 && a.s0 < a.s1 && a.s1 <= a.ctx && a.n_prompt >= 1 &&
-                   a.n_layer >= 1 && a.vocab >= 1 && (size_t)a.vocab * n_embed * 4 < ((size_t)1 << 32),
+    ZG_REQUIRE(resident_shape((size_t)n_embed, (size_t)a.n_heads, (size_t)a.ctx, (size_t)a.n_layer) && a.s0 >= 0 && a.s0 < a.s1 && a.s1 <= a.ctx && a.n_prompt >= 1 &&
+                   a.vocab >= 1 && (size_t)a.vocab * n_embed * 4 < ((size_t)1 << 32),
                ZG_ERR_ARG, "resident decode: bad arguments");
+    if (a.batch > 1) {
+        ZG_REQUIRE(weight_type == WT_BF16, ZG_ERR_UNSUPPORTED, "resident decode: several sequences with fp32 weights");
+        return launch_decode_resident_batch(a, n_embed, s);
+    }
 #define ZG_CASE(nw, nh)                                                         \
     case nw:                                                                     \
         return weight_type == WT_BF16 ? launch<bf16_t, nw, nh>(a, s) : launch<float, nw, nh>(a, s);

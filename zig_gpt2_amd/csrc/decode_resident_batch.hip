@@ -1,0 +1,938 @@
+// Greedy decode of two to eight sequences in lock step as a resident kernel: decode_resident.hip's cut of a Block over the XCDs and its
+// hand-overs, the products on the matrix cores.  GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 41.0 ms (318 -> 222 us a step; 33 + 991
+// tokens 322 -> 245 ms), 2 sequences 244 -> 150 us a step; char model, 8 sequences 36.8 -> 17.0 ms.
+//  bf16 weights: an activation travels as the exact three-term bf16 split of its
+// fp32 value (zg_common.h split3_pk), split once by the thread that makes it, all three terms and a tag of 16 bits in ONE word; a wave
+// multiplies 16 weight rows with the terms of all sequences (v_mfma_f32_16x16x32_bf16: columns of a product are terms x sequences),
+// the waves split K and meet in the LDS.
+//
+// Per Block: x -> A c_attn -> q, k, v -> B attention -> C merge + c_proj -> (all XCDs) -> x -> D c_fc + GELU -> h -> E mlp c_proj -> (all XCDs) -> x.
+// The thread that adds up a column of x (bias, residual, eight partial sums) also multiplies it with the gain of the LayerNorm that
+// follows; mean and variance arrive as sums of 8 columns beside it and are applied to the product's outputs (LayerNorm linearised, as
+// in gemv_ksplit.hip).
+//
+// What bounds it (8 sequences, 256 tokens, 14 us a Block): x is 48 KB of words for every workgroup, twice a Block, weights 60, keys and values 64:
+// the compute unit's one queue of vector memory (27 to 64 B a cycle).  Measured and left out: a look at the sums alone before
+// the columns are asked for (+2 %, a round trip more), pauses between looks (+0.5 %), rows of keys kept in registers across Blocks (spills).
+#include "decode_resident_parts.h"
+#include "zg_once.h"
+
+#include <type_traits>
+
+namespace zg {
+
+namespace {
+
+using namespace resident;
+typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef unsigned short u16;
+constexpr int kPause = 8;                     // x 64 cycles before the first look at words of other XCDs
+constexpr int kAfterA = 20;                   // before the fetches of a Block, behind c_attn's words
+constexpr int kMostSplits = 4;                // workgroups that share the positions of a (head, sequence)
+
+// three terms and the low half of the tag
+__device__ __forceinline__ u64 terms(unsigned tag, float v) {
+    uint32_t hi, mid, lo;
+    split3_pk(v, 0.0f, hi, mid, lo);
+    return ((u64)((tag << 16) | (lo & 0xffffu)) << 32) | (u64)((mid << 16) | (hi & 0xffffu));
+}
+
+// a lane's value and the ones 16 lanes (rows 0 and 1, 2 and 3) or 32 lanes away: both, on both lanes
+__device__ __forceinline__ void rows_apart_16(unsigned v, unsigned& a, unsigned& b) {
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+}
+__device__ __forceinline__ void rows_apart_32(unsigned v, unsigned& a, unsigned& b) {
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    a = r[0];
+    b = r[1];
+}
+// over the lanes with the same lane & 7, on all of them
+__device__ __forceinline__ float sum_over_8(float v) {
+    v += dpp_row_ror<8>(v);
+    unsigned a, b;
+    rows_apart_16(__float_as_uint(v), a, b);
+    v = __uint_as_float(a) + __uint_as_float(b);
+    rows_apart_32(__float_as_uint(v), a, b);
+    return __uint_as_float(a) + __uint_as_float(b);
+}
+__device__ __forceinline__ void best_over_rows(float& v, int& i) {  // over the lanes 16 apart, on all of them
+    unsigned a, b, ia, ib;
+    rows_apart_16(__float_as_uint(v), a, b);
+    rows_apart_16((unsigned)i, ia, ib);
+    v = __uint_as_float(a);
+    i = (int)ia;
+    better(v, i, __uint_as_float(b), (int)ib);
+    rows_apart_32(__float_as_uint(v), a, b);
+    rows_apart_32((unsigned)i, ia, ib);
+    v = __uint_as_float(a);
+    i = (int)ia;
+    better(v, i, __uint_as_float(b), (int)ib);
+}
+
+template <int NW, int NH, int MB>
+struct Spots {  // words
+    static constexpr int E = 64 * NW, F = E / 2, CPR = 2 * NW;
+    static constexpr int OW = (CPR * 8 + 63) / 64;             // waves that own columns of x
+    static constexpr int sums = 2 * kRanks * OW * 8;           // (sum, sum of squares) of 8 columns by (workgroup, wave, sequence)
+    static constexpr int block = (CPR * 8 + 15) & ~15;         // partial sums of a workgroup, all sequences
+    static constexpr int qkv = 0, att = qkv + 8 * NH * 192, ml = att + 8 * NH * kMostSplits * 64, x1 = ml + 8 * NH * kMostSplits * 2, st1 = x1 + 8 * E, h = st1 + sums,
+                         x2 = h + 8 * F, st2 = x2 + 8 * E, best = st2 + sums, near_words = best + kRanks * 8 * 2;
+    static constexpr int far1 = kXcds * near_words, far2 = far1 + kXcds * kRanks * block, pick = far2 + kXcds * kRanks * block, words = pick + kXcds * 16;
+};
+
+// LDS, bytes of the dynamic part
+template <int NW, int NH, int MB>
+struct Hall {
+    static constexpr int E = 64 * NW, F = E / 2, CPR = 2 * NW;
+    static constexpr int turns(int bytes) { return (bytes + 4095) / 4096; }
+    static constexpr int nA = turns(6 * NH * E * 2), nC = turns(CPR * NH * 64 * 2), nD = turns(NW * E * 2), nE = turns(CPR * F * 2);
+    static constexpr int step = 3 * MB * 64 + 64;              // the terms of 32 columns of all sequences (64 more: consecutive steps start in other banks)
+    static constexpr int TI = (CPR + 15) / 16;                 // tiles of 16 rows of C and E
+    static constexpr int A = 0, C = A + 2 * nA * 4096, D = C + nC * 4096, Eo = D + nD * 4096, X = Eo + nE * 4096, acc = X + (E / 32) * step,
+                         far_ = acc + NW * TI * 128 * 4, bytes = far_ + kXcds * CPR * 8 * 4;
+};
+
+template <int NW, int NH, int MB>
+__global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(const ResidentArgs a) {
+    typedef Spots<NW, NH, MB> P;
+    typedef Hall<NW, NH, MB> R;
+    constexpr int E = 64 * NW, F = E / 2, CPR = 2 * NW, NT = 64 * NW;
+    constexpr int HC = NH * 64, TI = R::TI, OW = P::OW;
+    constexpr int MX = MB / 2, MF = MB / 4;                        // sequences of a thread's pair of columns of x (two groups), of h (four groups)
+    constexpr int NS = (P::sums / 2 + NT - 1) / NT, NF8 = (kXcds * CPR * 4 + NT - 1) / NT;
+    constexpr int CJ = 2 * NH * TI;                                // (K step, tile) pairs of C
+    static_assert(CJ <= NW && 2 * R::nA + R::nC + R::nD + R::nE + 20 < 64 && OW <= NW && 8 * 32 * NH <= NT, "shapes");
+    static_assert(R::bytes + 10 * 1024 <= 160 * 1024, "LDS");
+
+    extern __shared__ __attribute__((aligned(16))) char s_hall[];
+    __shared__ float s_vec[2][192];                                // c2, c3 of the rows of A (12 each) and D (20 each); biases of the columns (32 each); ln_1 g, ln_2 g (32 each)
+    __shared__ __attribute__((aligned(8))) float s_sum[NW][8][2];
+    __shared__ __attribute__((aligned(16))) float s_new[192];      // q, k, v
+    __shared__ __attribute__((aligned(16))) float s_o[16][64];
+    __shared__ float s_m[4], s_l[4];
+    __shared__ float s_bv[16][8];
+    __shared__ int s_bi[16][8];
+    __shared__ int s_tok[8];
+    __shared__ unsigned s_rank, s_go, s_fail;
+
+    // (made opaque once a Block: what follows from them is made again where it is used instead of being kept, and spilled, for all Blocks)
+    int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    auto anew = [&]() {
+        tid = (int)fresh((unsigned)tid);
+        lane = tid & 63;
+    };
+    const unsigned xcc = __builtin_amdgcn_s_getreg((3 << 11) | 20) & 7u;  // HW_REG_XCC_ID
+    if (tid == 0) {
+        s_fail = 0u;
+        s_go = join(a.ctl, xcc, (unsigned)a.s0, a.start_limit, &s_rank);
+    }
+    __syncthreads();
+    if (s_go != 1u) {
+        if (tid == 0) __hip_atomic_store(a.withdrawn, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        return;
+    }
+    const int k = __builtin_amdgcn_readfirstlane((int)xcc), r = __builtin_amdgcn_readfirstlane((int)s_rank);
+    const int H = a.n_heads, M = a.batch;
+    const int nh = k < H ? (H - k + kXcds - 1) / kXcds : 0;       // heads of this XCD: k, k + 8, ...
+    const int nx = H < kXcds ? H : kXcds;                         // XCDs with heads
+    const int pairs = nh * M;                                     // (head, sequence)
+    const int G = pairs > 0 ? min(kRanks / pairs, kMostSplits) : 1;  // workgroups of a pair
+    const int my = r / G, sp = r % G;                             // this workgroup's
+    const int ih = my < pairs ? my / M : 0, im = my < pairs ? my % M : 0;
+    const int head = (k < H ? k : 0) + kXcds * ih;
+    // positions 0 .. T - 1 in chunks of 64: a split's, this workgroup's (c0 .. c1 - 1), the splits there are
+    int cps, c0, c1, n_sp;
+    auto divide = [&](int T) {
+        const int n = (T + 63) >> 6;
+        cps = __builtin_amdgcn_readfirstlane((n + G - 1) / G);
+        n_sp = __builtin_amdgcn_readfirstlane((n + cps - 1) / cps);
+        c0 = sp * cps;
+        c1 = min(c0 + cps, n);
+        return my < pairs && c0 < n;
+    };
+    u64* const near = a.words + (size_t)k * P::near_words;
+    u64* const far1 = a.words + P::far1;
+    u64* const far2 = a.words + P::far2;
+    u64* const picks = a.words + P::pick;
+    auto row_A = [&](int j) {  // row j of this workgroup's 6 nh rows of c_attn
+        const int n = r * 6 * nh + j, i = n / 192, part = (n % 192) / 64;
+        return part * E + (k + kXcds * i) * 64 + (n & 63);
+    };
+    const unsigned hall = lds_at(s_hall);
+
+    // ---- the vocabulary's rows: 16 of them with all sequences, by any wave
+    auto head_tiles = [&](bool last) {
+        const int V = a.vocab, tiles = (V + 15) >> 4, row16 = lane & 15, g4 = lane >> 4, m = lane & 15;
+        float bv = -3.0e38f;
+        int bi = 0x7fffffff;
+        for (int j = wave; j * kXcds * kRanks + k * kRanks + r < tiles; j += NW + 4) {
+            const int tile = j * kXcds * kRanks + k * kRanks + r;
+            const gchar* const p = base_at(a.wte);
+            const unsigned off = fresh((unsigned)(min(tile * 16 + row16, V - 1) * E) * 2u + (unsigned)g4 * 16u);
+            constexpr int KS = E / 32, RING = 8;
+            u32x4 wr[RING];
+            f32x4 c2, c3;
+#pragma unroll
+            for (int t = 0; t < RING; ++t) wr[t] = *(gptr<const u32x4>)(p + off + t * 64);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const unsigned q = fresh((unsigned)min(tile * 16 + g4 * 4 + i, V - 1) * 4u);
+                c2[i] = *(gptr<const float>)(base_at(a.lm_c2) + q);
+                c3[i] = *(gptr<const float>)(base_at(a.lm_c3) + q);
+            }
+            f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, acc1 = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int t = 0; t < KS; ++t) {
+                const bf16x8 w = __builtin_bit_cast(bf16x8, wr[t % RING]);
+                if (t + RING < KS) wr[t % RING] = *(gptr<const u32x4>)(p + off + (t + RING) * 64);
+                const unsigned at = fresh(hall + R::X + (unsigned)t * R::step + (unsigned)(g4 * 16));
+                if (MB == 8) {
+                    acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, lds_read<u32x4>(at + (16u + (m & 7)) * 64u)), acc1, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, lds_read<u32x4>(at + (unsigned)m * 64u)), acc, 0, 0, 0);
+                } else {
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, __builtin_bit_cast(bf16x8, lds_read<u32x4>(at + (unsigned)min(m, 11) * 64u)), acc, 0, 0, 0);
+                }
+            }
+            float mean, rstd;
+            {
+                float sx = 0.0f, sxx = 0.0f;
+#pragma unroll
+                for (int q = 0; q < NW; ++q) {
+                    const f32x2 s2 = *reinterpret_cast<const f32x2*>(s_sum[q][m & 7]);
+                    sx += s2.x;
+                    sxx += s2.y;
+                }
+                mean = sx * (1.0f / (float)E);
+                rstd = __builtin_amdgcn_rsqf(sxx * (1.0f / (float)E) - mean * mean + 1e-5f);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float s = MB == 8 ? (acc1[i] + dpp_row_ror<8>(acc[i])) + acc[i] : (dpp_row_ror<8>(acc[i]) + dpp_row_ror<12>(acc[i])) + acc[i];
+                const float y = fmaf(rstd, fmaf(-mean, c2[i], s), c3[i]);
+                const int row = tile * 16 + g4 * 4 + i;
+                if (m < M && row < V) {
+                    if (y > bv) {
+                        bv = y;
+                        bi = row;
+                    }
+                    if (last) *(gptr<float>)(base_at(a.logits) + fresh((unsigned)(m * V + row) * 4u)) = y;
+                }
+            }
+        }
+        best_over_rows(bv, bi);
+        if (lane < 8) {
+            s_bv[wave][lane] = bv;
+            s_bi[wave][lane] = bi;
+        }
+    };
+
+    // ---- weights: memory -> LDS, in pieces of 1 KB: pieces p0, p0 + dp, ... of a Block's matrices by one wave.  Rows of 16-byte units, unit u
+    // of row j at u ^ (j & 7): the 16 rows a product reads at once lie in different banks
+    auto from = [&](const void* base, int l, size_t bytes) {
+        return __builtin_amdgcn_make_buffer_rsrc((void*)base_at(base, (size_t)l * a.w_stride), 0, (int)bytes, 0x00020000);
+    };
+    constexpr int uE = E / 8, uF = F / 8, uC = HC / 8;
+    auto unit = [](int c, int u_row) { return (c % u_row) ^ ((c / u_row) & 7); };
+    auto unit_at = [&](int p, int most) { return min((int)fresh((unsigned)(p * 64 + lane)), most); };
+    auto fetch_A = [&](int l, int copy, int p0, int dp) {
+        const auto b = from(a.c_attn_w, l, 3 * (size_t)E * E * 2);
+#pragma unroll 1
+        for (int p = p0; p < R::nA * 4; p += dp) {
+            const int c = unit_at(p, max(6 * nh * uE - 1, 0));
+            dma16(b, (unsigned)((nh > 0 ? row_A(c / uE) : 0) * E) * 2u + (unsigned)unit(c, uE) * 16u, hall + R::A + copy * R::nA * 4096 + p * 1024);
+        }
+    };
+    auto fetch_C = [&](int l, int p0, int dp) {
+        const auto b = from(a.c_proj_w, l, (size_t)E * E * 2);
+#pragma unroll 1
+        for (int p = p0; p < R::nC * 4; p += dp) {
+            const int c = unit_at(p, CPR * uC - 1), u = unit(c, uC), i_h = u / 8;
+            dma16(b, (unsigned)((r * CPR + c / uC) * E + ((k < H ? k : 0) + kXcds * (i_h < nh ? i_h : 0)) * 64) * 2u + (unsigned)(u % 8) * 16u, hall + R::C + p * 1024);
+        }
+    };
+    auto fetch_D = [&](int l, int p0, int dp) {
+        const auto b = from(a.c_fc_w, l, 4 * (size_t)E * E * 2);
+#pragma unroll 1
+        for (int p = p0; p < R::nD * 4; p += dp) {
+            const int c = unit_at(p, NW * uE - 1);
+            dma16(b, (unsigned)((k * F + r * NW + c / uE) * E) * 2u + (unsigned)unit(c, uE) * 16u, hall + R::D + p * 1024);
+        }
+    };
+    auto fetch_E = [&](int l, int p0, int dp) {
+        const auto b = from(a.mlp_proj_w, l, 4 * (size_t)E * E * 2);
+#pragma unroll 1
+        for (int p = p0; p < R::nE * 4; p += dp) {
+            const int c = unit_at(p, CPR * uF - 1);
+            dma16(b, (unsigned)((r * CPR + c / uF) * 4 * E + k * F) * 2u + (unsigned)unit(c, uF) * 16u, hall + R::Eo + p * 1024);
+        }
+    };
+    auto fetch_V = [&](int l, int to, int w4) {
+        const int q = min(w4, 2);  // 0: rows of A and D, 1: biases, 2: gains
+        const float* v = q == 0 ? (lane < 12 ? a.c_attn_c2 : lane < 24 ? a.c_attn_c3 : lane < 44 ? a.c_fc_c2 : a.c_fc_c3)
+                                : q == 1 ? (lane < 32 ? a.c_proj_b : a.mlp_proj_b) : (lane < 32 ? a.ln_1_g : a.ln_2_g);
+        const int jA = lane < 12 ? lane : lane - 12;
+        const int n = q == 0 ? (lane < 24 ? (jA < 6 * nh ? row_A(jA) : 0) : k * F + r * NW + min(lane < 44 ? lane - 24 : lane - 44, NW - 1))
+                             : r * CPR + min(lane & 31, CPR - 1);
+        const float* const p = reinterpret_cast<const float*>(reinterpret_cast<const char*>(v) + (size_t)l * a.w_stride) + n;
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(lds_at(&s_vec[to][q * 64])), "v"(p) : "memory", "m0");
+    };
+
+    if (wave >= NW) {
+        // =========================================================================================== fetch and attend
+        const int fw = wave - NW;
+        struct Rows {
+            f32x4 k[2][2], v[4];  // 16 positions: 8 x 8 dims of keys, 4 x 4 dims of values a lane
+        };
+        // (in front of loads that are not always made: the registers would be kept for the rows they held before)
+        auto forget = [&](Rows& x) {
+            asm volatile("" : "=v"(x.k[0][0]), "=v"(x.k[0][1]), "=v"(x.k[1][0]), "=v"(x.k[1][1]));
+            asm volatile("" : "=v"(x.v[0]), "=v"(x.v[1]), "=v"(x.v[2]), "=v"(x.v[3]));
+        };
+        // chunk c of 64 positions of this workgroup's (head, sequence): 16 a wave
+        auto load_KV = [&](Rows& to, int l, int T, int c) {
+            // rows this XCD's workgroups wrote: past the L1 (sc1), whose lines may be older.  Positions that are not there yet re-read
+            // the last one that is; they weigh nothing
+            const size_t slab = (size_t)l * a.kv_stride + ((size_t)im * H + head) * a.ctx * 256;
+            const int bytes = a.ctx * 256;
+            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(a.k_cache + slab, 0, bytes, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(a.v_cache + slab, 0, bytes, 0x00020000);
+            const int p0 = c * 64 + fw * 16, last = max(T - 2, 0);
+            const int l8 = (int)fresh((unsigned)lane);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int off = min(p0 + i * 8 + (l8 >> 3), last) * 256 + (l8 & 7) * 32;
+                to.k[i][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 16));
+                to.k[i][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16, 0, 16));
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                to.v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i * 4 + (l8 >> 4), last) * 256 + (l8 & 15) * 16, 0, 16));
+        };
+        int vp = 0;
+        fetch_V(0, 0, fw);
+        fetch_A(0, 0, fw, 4);
+        in_flight<0>();
+        barrier();  // B0
+        for (int s = a.s0; s < a.s1; ++s) {
+            const int T = s + 1;
+            const bool here = divide(T);
+            for (int l = 0; l < a.n_layer; ++l) {
+                const int ln = l + 1 < a.n_layer ? l + 1 : 0;
+                anew();
+                barrier();  // B1
+                if (nh > 0) {
+                    if (!here) {
+                        fetch_C(l, fw, 4);
+                        barrier();  // B1a
+                        __builtin_amdgcn_s_sleep(kAfterA);
+                    } else {
+                        // (asked for here: c_attn and its hand-over take longer than they do; across Blocks they would want 64 registers all along)
+                        Rows kv[2];
+                        load_KV(kv[0], l, T, c0);
+                        fetch_C(l, fw, 4);
+                        barrier();  // B1a
+                        forget(kv[1]);
+                        if (c0 + 1 < c1) load_KV(kv[1], l, T, c0 + 1);
+                        barrier();  // B2
+                        // ---- B
+                        float m = kNone, lsum = 0.0f;
+                        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};  // four columns, every fourth position
+                        auto attend = [&](auto n_chunks, int c) {  // one chunk or two: their dependent steps side by side
+                            constexpr int N = decltype(n_chunks)::value;
+                            const int p0 = c * 64 + fw * 16;
+                            // (query and newest row are read where they are used: both chunks in flight take 64 registers)
+                            float sc[2 * N], mn = m;
+                            {
+                                const unsigned at = fresh(lds_at(&s_new[(lane & 7) * 8]));
+                                const f32x4 q0 = lds_read<f32x4>(at), q1 = lds_read<f32x4>(at + 16), n0 = lds_read<f32x4>(at + 256), n1 = lds_read<f32x4>(at + 272);
+#pragma unroll
+                                for (int i = 0; i < 2 * N; ++i) {
+                                    const Rows& x = kv[i / 2];
+                                    const int t = p0 + i / 2 * 64 + i % 2 * 8 + (lane >> 3);
+                                    const bool nw = t == T - 1;
+                                    float acc0 = 0.0f, acc1 = 0.0f;
+#pragma unroll
+                                    for (int d = 0; d < 4; ++d) {
+                                        acc0 = fmaf(q0[d], nw ? n0[d] : x.k[i % 2][0][d], acc0);
+                                        acc1 = fmaf(q1[d], nw ? n1[d] : x.k[i % 2][1][d], acc1);
+                                    }
+                                    const float dot = sum8(acc0 + acc1) * 0.125f;  // 1 / sqrt(64): ops.zig:275
+                                    sc[i] = t < T ? dot : kNone;
+                                }
+                            }
+                            {
+                                float top = sc[0];
+#pragma unroll
+                                for (int i = 1; i < 2 * N; ++i) top = fmaxf(top, sc[i]);
+                                mn = fmaxf(mn, wave_allmax(top));
+                            }
+                            const f32x4 vn = lds_read<f32x4>(fresh(lds_at(&s_new[128 + (lane & 15) * 4])));
+                            const float e0 = __expf(m - mn);
+                            lsum *= e0;
+                            o *= e0;
+#pragma unroll
+                            for (int i = 0; i < 2 * N; ++i) {
+                                const int tb = p0 + i / 2 * 64 + i % 2 * 8, t = tb + (lane >> 3);
+                                const float p = t < T ? __expf(sc[i] - mn) : 0.0f;
+                                float pj[8];
+#pragma unroll
+                                for (int j = 0; j < 8; ++j) {
+                                    pj[j] = lane_value(p, 8 * j);
+                                    lsum += pj[j];
+                                }
+#pragma unroll
+                                for (int q = 0; q < 2; ++q) {
+                                    const int g = lane >> 4, tj = tb + q * 4 + g;
+                                    const float pq = g & 2 ? (g & 1 ? pj[q * 4 + 3] : pj[q * 4 + 2]) : (g & 1 ? pj[q * 4 + 1] : pj[q * 4]);
+#pragma unroll
+                                    for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? kv[i / 2].v[i % 2 * 2 + q][d] : 0.0f, o[d]);
+                                }
+                            }
+                            m = mn;
+                        };
+                        for (int c = c0;;) {
+                            if (c + 1 < c1) attend(std::integral_constant<int, 2>{}, c);
+                            else attend(std::integral_constant<int, 1>{}, c);
+                            c += 2;
+                            if (c >= c1) break;
+                            load_KV(kv[0], l, T, c);
+                            forget(kv[1]);
+                            if (c + 1 < c1) load_KV(kv[1], l, T, c + 1);
+                        }
+                        *reinterpret_cast<f32x4*>(&s_o[fw * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
+                        if (lane == 0) {
+                            s_m[fw] = m;
+                            s_l[fw] = lsum;
+                        }
+                        barrier();  // B3
+                    }
+                }
+                if (!(here && cps > 1)) {
+                    fetch_D(l, fw, 4);
+                    fetch_E(l, fw, 4);
+                    fetch_V(ln, vp ^ 1, fw);
+                    fetch_A(ln, vp ^ 1, fw, 4);
+                }
+                if (nh > 0) {
+                    in_flight<R::nD + R::nE + 1 + R::nA>();  // C has arrived (behind the attention's rows where there were any)
+                    barrier();  // B4
+                    barrier();  // B4a
+                }
+                barrier();  // B4b
+                in_flight<R::nE + 1 + R::nA>();  // D has
+                barrier();  // B5
+                barrier();  // B5a
+                in_flight<0>();
+                barrier();  // B6
+                barrier();  // B6a
+                barrier();  // B6b
+                vp ^= 1;
+            }
+            if (s >= a.n_prompt) {
+                barrier();  // B7
+                head_tiles(s + 1 == a.s1);
+                barrier();  // B8
+            }
+            barrier();  // B9
+            if (s_fail != 0u) return;
+            barrier();  // B10
+        }
+        return;
+    }
+
+    // ================================================================================================ rows and words
+    Waiter w{a.spin_limit, &s_fail};
+    int vp = 0;
+    const unsigned all_words = (unsigned)P::words * 8u;
+    // 16 bytes, two words, of lanes' own addresses: all of them checked by `ok`, asked for again until it holds
+    auto words_at = [&](u64* base) { return __builtin_amdgcn_make_buffer_rsrc((void*)base_at(base), 0, (int)all_words, 0x00020000); };
+    auto again = [&](unsigned& n) {  // another look?
+        asm volatile("" ::: "memory");
+        if (n >= w.limit) {
+            s_fail = 1u;
+            w.limit = 0u;
+            return false;
+        }
+        ++n;
+        return true;
+    };
+    auto load16 = [&](__amdgpu_buffer_rsrc_t b, unsigned i) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int)fresh(i * 8u), 0, 16)); };
+    // terms of columns (c, c + 1) of sequence m: their place among the K steps' operands
+    auto put_terms = [&](int c, int m, const u32x4& v) {
+        const unsigned at = fresh(hall + R::X + (unsigned)(c >> 5) * R::step + (unsigned)m * 64u + (unsigned)(c & 31) * 2u);
+        typedef __attribute__((address_space(3))) uint32_t lds_u32;
+        *(lds_u32*)(uintptr_t)(at) = (v.x & 0xffffu) | (v.z << 16);
+        *(lds_u32*)(uintptr_t)(at + MB * 64u) = (v.x >> 16) | (v.z & 0xffff0000u);
+        *(lds_u32*)(uintptr_t)(at + 2 * MB * 64u) = (v.y & 0xffffu) | (v.w << 16);
+    };
+    // x and its sums of `tag` -> the operands of a product, the waves' shares of the sums
+    auto get_x = [&](unsigned at_x, unsigned at_st, unsigned tag) {
+        const auto b = words_at(near);
+        const int xc = 2 * (tid % (E / 2)), xm = tid / (E / 2) * MX;  // this thread's columns and first sequence
+        u32x4 v[MX], st[NS];
+        for (unsigned n = 0;;) {
+            bool ok = true;
+#pragma unroll
+            for (int j = 0; j < MX; ++j) v[j] = load16(b, at_x + (unsigned)(min(xm + j, M - 1) * E + xc));
+#pragma unroll
+            for (int i = 0; i < NS; ++i) st[i] = load16(b, at_st + 2u * (unsigned)min(tid + i * NT, P::sums / 2 - 1));
+#pragma unroll
+            for (int j = 0; j < MX; ++j) ok = ok && (v[j].y >> 16) == (tag & 0xffffu) && (v[j].w >> 16) == (tag & 0xffffu);
+#pragma unroll
+            for (int i = 0; i < NS; ++i) ok = ok && st[i].y == tag && st[i].w == tag;
+            if (ok || !again(n)) break;
+        }
+#pragma unroll
+        for (int j = 0; j < MX; ++j) put_terms(xc, xm + j, v[j]);
+        float sx = __uint_as_float(st[0].x), sxx = __uint_as_float(st[0].z);
+        if (NS > 1 && tid + NT < P::sums / 2) {
+            sx += __uint_as_float(st[NS - 1].x);
+            sxx += __uint_as_float(st[NS - 1].z);
+        }
+        sx = sum_over_8(sx);  // pair tid: sequence tid & 7
+        sxx = sum_over_8(sxx);
+        if (lane < 8) {
+            s_sum[wave][lane][0] = sx;
+            s_sum[wave][lane][1] = sxx;
+        }
+    };
+    auto stats = [&](int m, float& mean, float& rstd) {
+        float sx = 0.0f, sxx = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            const f32x2 s2 = *reinterpret_cast<const f32x2*>(s_sum[q][m]);
+            sx += s2.x;
+            sxx += s2.y;
+        }
+        mean = sx * (1.0f / (float)E);
+        rstd = __builtin_amdgcn_rsqf(sxx * (1.0f / (float)E) - mean * mean + 1e-5f);
+    };
+    // N K steps from `ws` on (weights: rows of u_row units at `at_w`) times operands' steps of the same numbers, 16 rows from row0 on
+    auto product = [&](auto n_steps, unsigned at_w, int u_row, int row0, int ws, f32x4& acc) {
+        constexpr int N = decltype(n_steps)::value;
+        const int row = row0 + (lane & 15), g = lane >> 4, n = lane & 15;
+        const unsigned at_r = fresh(at_w + (unsigned)(row * u_row) * 16u), sw = (unsigned)(row & 7);
+        const unsigned at_x = fresh(hall + R::X + (unsigned)ws * R::step + (unsigned)g * 16u);
+        u32x4 wt[N], top[N], low[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            wt[i] = lds_read<u32x4>(at_r + (((unsigned)((ws + i) * 4 + g)) ^ sw) * 16u);
+            if (MB == 8) low[i] = lds_read<u32x4>(at_x + i * R::step + (16u + (n & 7)) * 64u);
+            top[i] = lds_read<u32x4>(at_x + i * R::step + (unsigned)(MB == 8 ? n : min(n, 11)) * 64u);
+        }
+        f32x4 s_low = {0.0f, 0.0f, 0.0f, 0.0f}, s_top = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+            if (MB == 8) s_low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wt[i]), __builtin_bit_cast(bf16x8, low[i]), s_low, 0, 0, 0);
+            s_top = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wt[i]), __builtin_bit_cast(bf16x8, top[i]), s_top, 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            acc[i] = MB == 8 ? (s_low[i] + dpp_row_ror<8>(s_top[i])) + s_top[i] : (dpp_row_ror<8>(s_top[i]) + dpp_row_ror<12>(s_top[i])) + s_top[i];
+    };
+    constexpr std::integral_constant<int, 1> k1{};
+    constexpr std::integral_constant<int, 2> k2{};
+    // (row, sequence) of 16 x 8 outputs: thread row * 8 + sequence finds the waves' shares at the same place
+    float* const s_acc = reinterpret_cast<float*>(s_hall + R::acc);
+    auto share = [&](int slot, const f32x4& acc) {
+        if ((lane & 15) < 8) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) s_acc[fresh((unsigned)(slot * 128 + (lane >> 4) * 32 + (lane & 7))) + i * 8] = acc[i];
+        }
+    };
+    auto total = [&](int tile, int stride, int t) {
+        const unsigned at = fresh((unsigned)(tile * 128 + t));
+        float v[NW], y = 0.0f;
+#pragma unroll
+        for (int q = 0; q < NW; ++q) v[q] = s_acc[at + q * stride * 128];
+#pragma unroll
+        for (int q = 0; q < NW; ++q) y += v[q];
+        return y;
+    };
+    float* const s_far = reinterpret_cast<float*>(s_hall + R::far_);
+    // thread -> column oc of this workgroup, sequence om, which it owns
+    auto om = [&]() { return tid & 7; };
+    auto oc = [&]() { return tid >> 3; };
+    auto owns = [&]() { return oc() < CPR && om() < M; };
+    auto ocol = [&]() { return r * CPR + min(oc(), CPR - 1); };
+    float res = 0.0f;
+    // x (in res) -> its terms times `gain`, sums of 8 columns
+    auto put_x = [&](unsigned at_x, unsigned at_st, unsigned tag, float gain) {
+        if (owns()) put_near(near, at_x + (unsigned)(om() * E + ocol()), terms(tag, res * gain));
+        if (wave < OW) {
+            const float v = owns() ? res : 0.0f;
+            const float sx = sum_over_8(v), sxx = sum_over_8(v * v);
+            if (lane < 8) {
+                const unsigned to = at_st + (unsigned)((r * OW + wave) * 16 + 2 * lane);
+                put_near(near, to, tagged(tag, sx));
+                put_near(near, to + 1u, tagged(tag, sxx));
+            }
+        }
+    };
+    // the eight partial sums of every column
+    auto gather = [&](u64* from, int n_from, unsigned tag) {
+        const auto b = words_at(from);
+        __builtin_amdgcn_s_sleep(kPause);
+        u32x4 v[NF8];
+        for (unsigned n = 0;;) {
+            bool ok = true;
+#pragma unroll
+            for (int i = 0; i < NF8; ++i) {
+                const int u = min(tid + i * NT, kXcds * CPR * 4 - 1), q = u / (CPR * 4);
+                v[i] = load16(b, (unsigned)((min(q, n_from - 1) * kRanks + r) * P::block + 2 * (u % (CPR * 4))));
+                ok = ok && v[i].y == tag && v[i].w == tag;
+            }
+            if (ok || !again(n)) break;
+        }
+#pragma unroll
+        for (int i = 0; i < NF8; ++i) {
+            const int u = tid + i * NT;
+            if (u < n_from * CPR * 4) *reinterpret_cast<f32x2*>(&s_far[u * 2]) = f32x2{__uint_as_float(v[i].x), __uint_as_float(v[i].z)};
+        }
+    };
+    auto add_up = [&](int n_from, float bias) {
+        if (oc() < CPR) {
+            const unsigned at = fresh((unsigned)tid);
+            float v[kXcds], y = 0.0f;
+#pragma unroll
+            for (int q = 0; q < kXcds; ++q) v[q] = s_far[q * CPR * 8 + at];
+#pragma unroll
+            for (int q = 0; q < kXcds; ++q) y += q < n_from ? v[q] : 0.0f;
+            res += y + bias;
+        }
+    };
+    __builtin_amdgcn_s_setprio(3);
+    if (tid < 8) s_tok[tid] = tid < M && a.s0 > a.prompt_len[min(tid, M - 1)] ? a.out_tokens[(size_t)min(tid, M - 1) * a.out_stride + max(a.s0 - 1, 0)] : 0;
+    const int np = a.prompt_len[min(om(), M - 1)];
+    const float fin_g = a.ln_f_g[ocol()];
+    barrier();  // B0
+    for (int s = a.s0; s < a.s1; ++s) {
+        const int T = s + 1;
+        const bool here = divide(T), newest = sp == n_sp - 1;  // attends; to position T - 1 too
+        const unsigned tag0 = a.tag0 + (unsigned)(s - a.s0) * (unsigned)(a.n_layer + 2);
+        int tok = 0;
+        if (owns()) {
+            tok = s < np ? a.prompt[(size_t)om() * a.out_stride + s] : s == np ? a.prompt[(size_t)om() * a.out_stride + np - 1] : s_tok[om()];
+            if (s < np && k == 0 && r == 0 && oc() == 0) a.out_tokens[(size_t)om() * a.out_stride + s] = tok;
+            auto value = [&](const void* base, size_t row) -> float {
+                return __uint_as_float((uint32_t)(reinterpret_cast<const bf16_t*>(base)[row * E + ocol()]) << 16);
+            };
+            res = value(a.wte, (size_t)tok) + value(a.wpe, (size_t)s);
+        }
+        put_x(P::x2, P::st2, tag0, s_vec[vp][128 + min(oc(), 31)]);
+        for (int l = 0; l < a.n_layer; ++l) {
+            const unsigned tag = tag0 + 1u + (unsigned)l;
+            anew();
+            if (nh > 0) {
+                get_x(P::x2, P::st2, tag - 1u);
+                barrier();  // B1
+                // ---- A
+                float mean = 0.0f, rstd = 0.0f;
+                if (wave * 8 < 6 * nh) stats(om(), mean, rstd);
+                {
+                    f32x4 acc;
+                    product(k2, hall + R::A + vp * R::nA * 4096, E / 8, 0, 2 * wave, acc);
+                    share(wave, acc);
+                }
+                barrier();  // B1a
+                float yA = 0.0f;
+                const int jA = tid >> 3, nA = r * 6 * nh + jA;
+                const bool hasA = jA < 6 * nh && om() < M;
+                if (jA < 6 * nh) {
+                    yA = fmaf(rstd, fmaf(-mean, s_vec[vp][jA], total(0, 1, tid)), s_vec[vp][12 + jA]);
+                    if (hasA) put_near(near, P::qkv + (unsigned)(om() * NH * 192 + nA), tagged(tag, yA));
+                }
+                if (here) {
+                    if (tid < 192 && (tid < 64 || newest)) s_new[tid] = w.get(near, P::qkv + (unsigned)(im * NH * 192 + ih * 192 + tid), tag);
+                    barrier();  // B2
+                    // While four waves attend to more than 64 positions: the rest of this Block's weights and the next one's first.  What a
+                    // thread polls for next returns behind them, but takes as long; and with it they are known to have arrived, long before
+                    // anyone multiplies with them.  (124M, 8 sequences, 256 tokens 41.8 -> 41.0 ms, 1024 255 -> 247; up to 64 positions the attending
+                    // waves fetch behind their attention: char model, 8 sequences 17.3 against 17.7 ms)
+                    if (cps > 1) {
+                        const int ln = l + 1 < a.n_layer ? l + 1 : 0;
+                        fetch_D(l, wave, NW);
+                        fetch_E(l, wave, NW);
+                        if (wave < 3) fetch_V(ln, vp ^ 1, wave);
+                        fetch_A(ln, vp ^ 1, wave, NW);
+                    }
+                    barrier();  // B3
+                    if (wave == 0) {
+                        float m = kNone, o = 0.0f, lsum = 0.0f;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) m = fmaxf(m, s_m[i]);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const float e = __expf(s_m[i] - m);
+                            o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
+                            lsum = fmaf(e, s_l[i], lsum);
+                        }
+                        const unsigned to = (unsigned)((im * NH + ih) * kMostSplits + sp);
+                        if (lane < 2) put_near(near, P::ml + to * 2u + lane, tagged(tag, lane ? lsum : m));
+                        put_near(near, P::att + to * 64u + lane, tagged(tag, o));
+                    }
+                }
+                if (hasA) {  // the cache, while the partials are on their way
+                    const int row = row_A(jA), part = row / E, c = row % E;
+                    gchar *const kb = base_at(a.k_cache, (size_t)l * a.kv_stride), *const vb = base_at(a.v_cache, (size_t)l * a.kv_stride);
+                    if (part > 0) *(gptr<float>)((part == 1 ? kb : vb) + (((size_t)(om() * H + (c >> 6)) * a.ctx + (T - 1)) * 64 + (c & 63)) * 4) = yA;
+                }
+                // ---- C: two columns of a sequence a thread, merged over the splits
+                {
+                    const int c2 = tid % (HC / 2), m = tid / (HC / 2), i_h = c2 >> 5;
+                    if (m < MB) {
+                        u32x4 z4 = {0u, 0u, 0u, 0u};
+                        if (m < M && i_h < nh) {
+                            const auto b = words_at(near);
+                            u32x4 o4[kMostSplits], m4[kMostSplits];
+                            for (unsigned n = 0;;) {
+                                bool ok = true;
+#pragma unroll
+                                for (int q = 0; q < kMostSplits; ++q) {
+                                    const unsigned at = (unsigned)((m * NH + i_h) * kMostSplits + min(q, n_sp - 1));
+                                    if (q < n_sp) {
+                                        o4[q] = load16(b, P::att + at * 64u + 2u * (unsigned)(c2 & 31));
+                                        m4[q] = load16(b, P::ml + at * 2u);
+                                    }
+                                }
+#pragma unroll
+                                for (int q = 0; q < kMostSplits; ++q)
+                                    if (q < n_sp) ok = ok && o4[q].y == tag && o4[q].w == tag && m4[q].y == tag && m4[q].w == tag;
+                                if (ok || !again(n)) break;
+                            }
+                            float mx = kNone, lsum = 0.0f, z0 = 0.0f, z1 = 0.0f;
+#pragma unroll
+                            for (int q = 0; q < kMostSplits; ++q)
+                                if (q < n_sp) mx = fmaxf(mx, __uint_as_float(m4[q].x));
+#pragma unroll
+                            for (int q = 0; q < kMostSplits; ++q)
+                                if (q < n_sp) {
+                                    const float e = __expf(__uint_as_float(m4[q].x) - mx);
+                                    lsum = fmaf(e, __uint_as_float(m4[q].z), lsum);
+                                    z0 = fmaf(e, __uint_as_float(o4[q].x), z0);
+                                    z1 = fmaf(e, __uint_as_float(o4[q].z), z1);
+                                }
+                            const float inv = 1.0f / lsum;
+                            const u64 t0 = terms(0u, z0 * inv), t1 = terms(0u, z1 * inv);
+                            z4 = u32x4{(uint32_t)t0, (uint32_t)(t0 >> 32), (uint32_t)t1, (uint32_t)(t1 >> 32)};
+                        }
+                        put_terms(2 * c2, m, z4);
+                    }
+                }
+                barrier();  // B4
+                if (wave < CJ) {
+                    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+                    const int ws = wave % (2 * NH), ti = wave / (2 * NH);
+                    if (ws < 2 * nh) product(k1, hall + R::C, HC / 8, ti * 16, ws, acc);
+                    share(wave, acc);
+                }
+                barrier();  // B4a
+                if (tid < CPR * 8) {
+                    const int ti = tid >> 7;
+                    float y = 0.0f;
+                    const unsigned at = fresh((unsigned)(ti * 2 * NH * 128 + (tid & 127)));
+                    float v[2 * NH];
+#pragma unroll
+                    for (int q = 0; q < 2 * NH; ++q) v[q] = s_acc[at + q * 128];
+#pragma unroll
+                    for (int q = 0; q < 2 * NH; ++q) y += q < 2 * nh ? v[q] : 0.0f;
+                    if (om() < M) put_far(far1, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, y));
+                    else put_far(far1, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, 0.0f));
+                }
+            } else {
+                barrier();  // B1
+            }
+            gather(far1, nx, tag);
+            barrier();  // B4b
+            add_up(nx, s_vec[vp][64 + min(oc(), 31)]);
+            put_x(P::x1, P::st1, tag, s_vec[vp][160 + min(oc(), 31)]);
+            get_x(P::x1, P::st1, tag);
+            barrier();  // B5
+            // ---- D
+            float mean = 0.0f, rstd = 0.0f;
+            if (wave * 8 < NW) stats(om(), mean, rstd);
+            {
+                f32x4 acc;
+                product(k2, hall + R::D, E / 8, 0, 2 * wave, acc);
+                share(wave, acc);
+            }
+            barrier();  // B5a
+            if (oc() < NW) {
+                const float y = gelu_ref(fmaf(rstd, fmaf(-mean, s_vec[vp][24 + oc()], total(0, 1, tid)), s_vec[vp][44 + oc()]));
+                if (om() < M) put_near(near, P::h + (unsigned)(om() * F + r * NW + oc()), terms(tag, y));
+            }
+            // ---- E
+            {
+                const int c = 2 * (tid % (F / 2)), m0 = tid / (F / 2) * MF;
+                const auto b = words_at(near);
+                u32x4 v[MF];
+                for (unsigned n = 0;;) {
+                    bool ok = true;
+#pragma unroll
+                    for (int j = 0; j < MF; ++j) {
+                        v[j] = load16(b, P::h + (unsigned)(min(m0 + j, M - 1) * F + c));
+                        ok = ok && (v[j].y >> 16) == (tag & 0xffffu) && (v[j].w >> 16) == (tag & 0xffffu);
+                    }
+                    if (ok || !again(n)) break;
+                }
+#pragma unroll
+                for (int j = 0; j < MF; ++j) put_terms(c, m0 + j, v[j]);
+            }
+            barrier();  // B6
+            {
+#pragma unroll
+                for (int ti = 0; ti < TI; ++ti) {
+                    f32x4 acc;
+                    product(k1, hall + R::Eo, F / 8, ti * 16, wave, acc);
+                    share(wave * TI + ti, acc);
+                }
+            }
+            barrier();  // B6a
+            if (tid < CPR * 8) put_far(far2, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, total(tid >> 7, TI, tid & 127)));
+            gather(far2, kXcds, tag);
+            barrier();  // B6b
+            add_up(kXcds, s_vec[vp][96 + min(oc(), 31)]);
+            vp ^= 1;
+            put_x(P::x2, P::st2, tag, l + 1 < a.n_layer ? s_vec[vp][128 + min(oc(), 31)] : fin_g);
+        }
+        const bool last = s + 1 == a.s1;
+        if (s >= a.n_prompt) {  // ---- ln_f + lm_head + argmax (main.zig:189-194, :337)
+            get_x(P::x2, P::st2, tag0 + (unsigned)a.n_layer);
+            barrier();  // B7
+            head_tiles(last);
+            barrier();  // B8
+            const unsigned tag = tag0 + (unsigned)a.n_layer + 1u;
+            if (wave == 0 && lane < 8) {  // the workgroup's
+                float v = -3.0e38f;
+                int i = 0x7fffffff;
+                for (int q = 0; q < NW + 4; ++q) better(v, i, s_bv[q][lane], s_bi[q][lane]);
+                put_near(near, P::best + (unsigned)(r * 16 + 2 * lane), tagged(tag, v));
+                put_near(near, P::best + (unsigned)(r * 16 + 2 * lane + 1), tagged(tag, __int_as_float(i)));
+            }
+            auto reduce8 = [&](float& v, int& i) {  // over lanes with the same lane & 7
+                better(v, i, dpp_row_ror<8>(v), __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true));
+                best_over_rows(v, i);
+            };
+            auto pair_at = [&](u64* base, unsigned at, float& v, int& i) {
+                const auto b = words_at(base);
+                u32x4 p;
+                for (unsigned n = 0;;) {
+                    p = load16(b, at);
+                    if ((p.y == tag && p.w == tag) || !again(n)) break;
+                }
+                v = __uint_as_float(p.x);
+                i = (int)p.z;
+            };
+            if (r == 0 && wave == 0) {  // the XCD's: lane -> (workgroup lane >> 3 + 8 q, sequence lane & 7)
+                float v = -3.0e38f;
+                int i = 0x7fffffff;
+                const auto b = words_at(near);
+                u32x4 p[4];
+                for (unsigned n = 0;;) {
+                    bool ok = true;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        p[q] = load16(b, P::best + (unsigned)(((lane >> 3) + 8 * q) * 16 + 2 * (lane & 7)));
+                        ok = ok && p[q].y == tag && p[q].w == tag;
+                    }
+                    if (ok || !again(n)) break;
+                }
+#pragma unroll
+                for (int q = 0; q < 4; ++q) better(v, i, __uint_as_float(p[q].x), (int)p[q].z);
+                reduce8(v, i);
+                if (lane < 8) {
+                    put_far(picks, (unsigned)(k * 16 + 2 * lane), tagged(tag, v));
+                    put_far(picks, (unsigned)(k * 16 + 2 * lane + 1), tagged(tag, __int_as_float(i)));
+                }
+            }
+            if (wave == 0) {
+                float v;
+                int i;
+                __builtin_amdgcn_s_sleep(kPause);
+                pair_at(picks, (unsigned)((lane >> 3) * 16 + 2 * (lane & 7)), v, i);
+                reduce8(v, i);
+                // logits that are all NaN: index 0, never one behind the table (embed_step_kernel)
+                if (lane < 8) {
+                    s_tok[lane] = (unsigned)i < (unsigned)a.vocab ? i : 0;
+                    if (lane < M && k == 0 && r == 0) {
+                        if (s >= np) a.out_tokens[(size_t)lane * a.out_stride + s] = s_tok[lane];
+                        if (last) {  // for the launches that may follow: one partial holds the pick
+                            a.part_val[(size_t)lane * a.n_part] = v;
+                            a.part_idx[(size_t)lane * a.n_part] = i;
+                        }
+                    }
+                }
+            }
+        }
+        barrier();  // B9
+        if (s_fail != 0u) {  // a wait ran out: results are worthless and everyone leaves
+            if (tid == 0) __hip_atomic_store(a.fault, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            return;
+        }
+        barrier();  // B10
+        if (last) {
+            if (owns() && k == 0) a.x[(size_t)om() * E + ocol()] = res;
+            if (k == 0 && r == 0) {
+                if (s >= a.n_prompt)
+                    for (int q = tid; q < M * a.n_part; q += NT)
+                        if (q % a.n_part != 0) {
+                            a.part_val[q] = -3.0e38f;
+                            a.part_idx[q] = 0x7fffffff;
+                        }
+                if (owns() && oc() == 0) a.cur_token[om()] = tok;
+                if (tid == 0) {
+                    a.ctrl->seq_len = T;
+                    a.ctrl->step = T;
+                    a.ctl->done = (unsigned)T;
+                }
+            }
+        }
+    }
+}
+
+template <int NW, int NH, int MB>
+int launch(const ResidentArgs& a, hipStream_t s) {
+    note_kernel("decode_resident_batch_kernel<%d, %d, %d>", NW, NH, MB);
+    constexpr int kOneEach = Hall<NW, NH, MB>::bytes > 84 * 1024 ? Hall<NW, NH, MB>::bytes : 84 * 1024;  // more than half of a compute unit's LDS: one workgroup each
+    static OncePerDevice once;
+    int dev = 0;
+    ZG_HIP(hipGetDevice(&dev));
+    ZG_TRY(once.run(dev, [&]() -> int {
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&decode_resident_batch_kernel<NW, NH, MB>), hipFuncAttributeMaxDynamicSharedMemorySize, kOneEach));
+        return ZG_OK;
+    }));
+    hipLaunchKernelGGL((decode_resident_batch_kernel<NW, NH, MB>), dim3(kXcds * kRanks), dim3(64 * (NW + 4)), kOneEach, s, a);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+}  // namespace
+
+size_t resident_batch_words(size_t n_embed) {
+    switch (n_embed / 64) {
+        case 6: return Spots<6, 1, 8>::words;
+        case 8: return Spots<8, 1, 8>::words;
+        case 12: return Spots<12, 2, 8>::words;
+        default: return 0;
+    }
+}
+
+int launch_decode_resident_batch(const ResidentArgs& a, int n_embed, hipStream_t s) {
+    ZG_REQUIRE(a.batch >= 2 && a.batch <= 8, ZG_ERR_ARG, "resident decode: %d sequences", a.batch);
+#define ZG_CASE(nw, nh) \
+    case nw:            \
+        return a.batch <= 4 ? launch<nw, nh, 4>(a, s) : launch<nw, nh, 8>(a, s);
+    switch (n_embed / 64) {
+        ZG_CASE(6, 1)
+        ZG_CASE(8, 1)
+        ZG_CASE(12, 2)
+    }
+#undef ZG_CASE
+    set_error("resident decode: n_embed %d", n_embed);
+    return ZG_ERR_UNSUPPORTED;
+}
+
+}  // namespace zg

@@ -331,24 +331,28 @@ struct ResidentArgs {
     size_t w_stride, kv_stride;
     char *k_cache, *v_cache;  // fp32, [head][ctx][64]
     const void *wte, *wpe;
-    const float *ln_f_g, *ln_f_b;
+    const float *ln_f_g, *ln_f_b, *lm_c2, *lm_c3;
     int n_layer, n_heads, ctx, vocab;
-    int n_prompt, s0, s1;  // steps s0 .. s1 - 1 of the generation
-    const int* prompt;
+    int batch;
+    int n_prompt, s0, s1;  // (shortest) prompt; steps s0 .. s1 - 1 of the generation
+    const int *prompt, *prompt_len;  // prompts and tokens: out_stride apart
+    int out_stride;
     int *out_tokens, *cur_token;
     StepCtrl* ctrl;
     float *x, *logits, *part_val;
     int* part_idx;
     int n_part;
-    unsigned long long* words;  // resident_words(n_embed), zeroed once; tags tag0 .. tag0 + (s1 - s0) (n_layer + 1) - 1 are this launch's alone
+    unsigned long long* words;  // resident_words(n_embed, batch), zeroed once; tags tag0 .. tag0 + (s1 - s0) (n_layer + 2) - 1 are this launch's alone
     ResidentCtl* ctl;
     unsigned tag0;
     unsigned spin_limit, start_limit;
     unsigned *fault, *withdrawn;  // pinned host words
 };
-bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx);
-size_t resident_words(size_t n_embed);
-int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s);
+bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer);
+size_t resident_words(size_t n_embed, size_t batch);
+int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s);  // one sequence: bf16 or fp32 weights; two to eight: bf16
+size_t resident_batch_words(size_t n_embed);
+int launch_decode_resident_batch(const ResidentArgs& a, int n_embed, hipStream_t s);
 
 // ------------------------------------------------------------------------------------ multi-GPU (dist.hip)
 int dist_broadcast(void* buf, size_t bytes, int root, hipStream_t s);  // in place, over the communicator of zg_dist_init
