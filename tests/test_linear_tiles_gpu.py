@@ -49,6 +49,22 @@ def test_both_sides_of_the_rule(zg, m, k, n, kernel):
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 
+@pytest.mark.parametrize("m", [5, 8, 9, 15])
+@pytest.mark.parametrize("k,n", [(64, 1), (120, 40), (136, 1), (136, 6145), (256, 16), (264, 17), (512, 15), (520, 33), (768, 2049), (1024, 2048), (1032, 31),
+                                 (1536, 1025), (1792, 4096), (1784, 4097), (1800, 40)])
+def test_few_rows_on_the_matrix_cores(zg, m, k, n):
+    """Five to fifteen rows: the last columns of a piece, weight rows around the tile's sixteen, one piece of a wave to seven, both sides of the
+    rule.  A row that is not finite stays by itself."""
+    w, b, x, y = run(m, k, n, bias=n % 2 == 1)
+    assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
+    xs = x.copy()
+    xs[m - 1, k - 1], xs[m - 2, k - 8] = np.inf, np.nan
+    ys = run(m, k, n, bias=n % 2 == 1, x=xs)[3]
+    with np.errstate(all="ignore"):
+        assert_same_class(oracle.linear_forward(k, n, w, b, xs)[m - 2:], ys[m - 2:], "not finite")
+    assert np.array_equal(ys[:m - 2], y[:m - 2])
+
+
 @pytest.mark.parametrize("m", [0, 1, 2, 8, 9, 16, 70])
 @pytest.mark.parametrize("k", [100, 128, 768, 8200, 16384])
 def test_no_outputs(zg, m, k):

@@ -1,5 +1,5 @@
 // linear_tiles.hip — fp32 Linears of nine rows to some thousand (y = x W^T + bias, src/ops.zig:21-46) in one pass over both operands, and of
-// two to eight rows (linear_few_kernel, below).
+// two to fifteen rows (linear_few_kernel and linear_few_mfma_kernel, below).
 //
 // Both operands are split exactly into three bf16 terms on their way into the LDS (x = hi + mid + lo) and the six products above 2^-24 of
 // the leading one are summed, as the persistent kernel for many rows does (gemm_s4.hip); here no planes are written to memory first, and
@@ -250,6 +250,69 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const float* __restrict
     if (lane < MR * R && m < M && n < N) Y[(size_t)m * N + n] = mine + (bias ? bias[n] : 0.0f);
 }
 
+// Five to fifteen rows: a workgroup multiplies sixteen weight rows with all of them, its waves pieces of 32 columns in turn, by the matrix
+// cores' fp32 products: a weight and an activation are loaded once a workgroup and nothing is summed over lanes.  RING pieces of a wave in
+// flight, at clamped addresses without a condition.  Eight sums a lane keep the chains of additions short and meet in 64 bits: against 64 bits
+// the outputs are as near as those of the kernels it took over from, or nearer (rms of 768 columns 5.8e-8 of the outputs' own, 8.2e-8 and 7.2e-8
+// there; with 32-bit sums 8.0e-8).
+// What bounds it: latency, the launch and one round of loads, and where a workgroup has many pieces the intake of its compute unit.  A call, us,
+// those kernels -> this one: 8 rows 768 -> 3072 15.2 -> 13.8, 768 -> 50257 55 -> 46, 1600 -> 6400 28.2 -> 23.8, 12 rows 768 -> 768 18.8 -> 14.3,
+// 520 -> 600 25.8 -> 13.1, 768 -> 50257 57 -> 49.
+template <int RING>
+__global__ __launch_bounds__(512) void linear_few_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
+                                                                    float* __restrict__ Y, int M, int N, int K) {
+    constexpr int kWaves = 8;
+    __shared__ double s_part[kWaves][4][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, row = lane & 15, n0 = blockIdx.x * 16;
+    const int on = n0 + (tid & 15), om = tid >> 4;  // the output a thread ends with
+    const float b = bias != nullptr ? bias[min(on, N - 1)] : 0.0f;
+    const float* const w = W + (size_t)min(n0 + row, N - 1) * K;
+    const float* const x = X + (size_t)min(row, M - 1) * K;
+    const int k_lane = wave * 32 + (lane >> 4) * 8;
+    f32x4 wr[RING][2], xr[RING][2];
+    auto fetch = [&](int slot, int p) {
+        const int k = min(k_lane + p * kWaves * 32, K - 8);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            wr[slot][i] = *reinterpret_cast<const f32x4*>(w + k + 4 * i);
+            xr[slot][i] = *reinterpret_cast<const f32x4*>(x + k + 4 * i);
+        }
+    };
+    f32x4 acc[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto multiply = [&](int slot, int p) {
+        const bool in = k_lane + p * kWaves * 32 < K;  // (K is whole eights)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(in ? wr[slot][i >> 2][i & 3] : 0.0f, in ? xr[slot][i >> 2][i & 3] : 0.0f, acc[i], 0, 0, 0);
+    };
+    const int mine = ((K + 31) / 32 - wave + kWaves - 1) / kWaves;  // pieces of this wave
+#pragma unroll
+    for (int i = 0; i < RING; ++i) fetch(i, i);
+    int p = 0;
+    for (; p + RING < mine; p += RING) {
+#pragma unroll
+        for (int i = 0; i < RING; ++i) {
+            multiply(i, p + i);
+            fetch(i, p + i + RING);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RING; ++i) multiply(i, p + i);  // (pieces beyond K: zeros)
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        s_part[wave][e][lane] = (((double)acc[0][e] + acc[1][e]) + ((double)acc[2][e] + acc[3][e])) + (((double)acc[4][e] + acc[5][e]) + ((double)acc[6][e] + acc[7][e]));
+    __syncthreads();
+    if (tid >= 256 || on >= N || om >= M) return;
+    // element e of a lane's four: weight row 4 (lane / 16) + e, row of X lane % 16
+    const int at = ((tid & 15) >> 2) * 16 + om, e = tid & 3;
+    double v[kWaves];
+#pragma unroll
+    for (int i = 0; i < kWaves; ++i) v[i] = s_part[i][e][at];
+    Y[(size_t)om * N + on] = (float)((((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]))) + b);
+}
+
 }  // namespace
 
 bool linear_tiles_pay(size_t M, size_t N) {
@@ -287,16 +350,45 @@ int launch_linear_tiles(const float* X, const float* W, const float* bias, float
     return ZG_OK;
 }
 
+// linear_few_mfma_kernel, or linear_few_kernel and the tiles; a call's us this : those.  Nine rows to fifteen (12 rows 768 -> 768 14.3 : 18.8,
+// 768 -> 3072 14.3 : 20.6, 1600 -> 1600 18.4 : 20.7; K in no whole 64s, as 520 -> 600, 13.1 : 25.8): the tiles, which have sixteen rows and more,
+// catch up where long rows make a compute unit's share long (16 rows 1600 -> 4800 25.0 : 24.0, 3072 -> 768 21.4 : 22.4, 6400 -> 1600 35.5 : 30.7);
+// rows shorter than their 128 columns stay on the general kernels.  Five to eight: linear_few_kernel has more workgroups and is ahead until they
+// are more than the compute units (8 rows 768 -> 768 13.0 : 12.8, 1024 -> 1024 13.7 : 12.9, 768 -> 2304 13.7 : 15.4; its long rows 1536 -> 384
+// 16.6 : 14.3, 1600 -> 1600 17.5 : 19.3, 3072 -> 1031 19.4 : 18.9; between them 1528 -> 2000 16.9 : 14.7); short rows are ahead at once here
+// (384 -> 384 12.7 : 13.2).
+static bool few_on_mfma(size_t M, size_t N, size_t K) {
+    if (M > 15) return false;
+    if (M > 8) return K >= 128 && (K <= 1024 || (K <= 1792 && N <= 4096));
+    if (M < 5 || (K < 256 && N > 6144)) return false;  // (so short and so many: still the general kernel, by linear_few_ok)
+    return K <= 512 || (K <= 1024 && N > 2048) || (K >= kLongRow && K <= 1792 && N > 1024);
+}
+
 bool linear_few_ok(size_t M, size_t N, size_t K) {
+    if (K < 64 || K > 8192 || K % 8 != 0 || N >= (1u << 30)) return false;
+    if (few_on_mfma(M, N, K)) return true;
     // Beyond four rows every workgroup's share of the activations outweighs its weights: with more than some three workgroups a compute unit
-    // the general kernel, which reads them less often, is faster (8 rows 1600 -> 4800, 1200 of them, 32.9 : 27.9; 6400 -> 1600, 400, 26 : 32).
+    // the general kernel, which reads them less often, is faster (6400 -> 1600, 400 of them, 26 : 32; 1200 of 1600 columns 32.9 : 27.9).
     const size_t groups = K >= kLongRow ? (N + 3) / 4 : (N + 7) / 8;
     // One row stays on the general kernels: a generation through op-tier calls with host buffers measured 782 tokens/s with it here, 819 there.
-    return M >= 2 && M <= 8 && K >= 64 && K <= 8192 && K % 8 == 0 && groups < (1u << 30) && (M <= 4 || groups <= 768);
+    return M >= 2 && M <= 8 && (M <= 4 || groups <= 768);
 }
 
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s) {
-    ZG_REQUIRE(M >= 1 && M <= 8 && N > 0 && K >= 8 && K % 8 == 0, ZG_ERR_UNSUPPORTED, "linear: M=%d N=%d K=%d", M, N, K);
+    ZG_REQUIRE(M >= 1 && M <= 15 && N > 0 && K >= 8 && K % 8 == 0, ZG_ERR_UNSUPPORTED, "linear: M=%d N=%d K=%d", M, N, K);
+    if (few_on_mfma(M, N, K)) {
+        const int each = (K + 255) / 256;  // pieces of a wave
+#define ZG_FEW(RING) linear_few_mfma_kernel<RING><<<(N + 15) / 16, 512, 0, s>>>(X, W, bias, Y, M, N, K)
+        if (each == 1) ZG_FEW(1);
+        else if (each == 2) ZG_FEW(2);
+        else if (each == 3) ZG_FEW(3);
+        else ZG_FEW(4);
+#undef ZG_FEW
+        note_kernel("linear_few_kernel");
+        ZG_HIP(hipGetLastError());
+        return ZG_OK;
+    }
+    ZG_REQUIRE(M <= 8, ZG_ERR_UNSUPPORTED, "linear: M=%d N=%d K=%d", M, N, K);
     const bool split = K >= kLongRow;
 #define ZG_FEW(MR)                                                                                             \
     do {                                                                                                       \

@@ -207,7 +207,7 @@ int gemm_s4_fault(unsigned* out);  // 1: a stream-K consumer of gemm_s4 gave up 
 int gemm_debug_stamps(unsigned long long* out, size_t n_words);  // of the kernel generation launched last
 unsigned long long gemm_mfma_launch_count();  // launches of the persistent MFMA GEMMs so far (tests assert the path taken)
 void gemm_note_launch();
-// fp32 Linears X [M][K], W [N][K] of few rows and of a medium number of rows (linear_tiles.hip).  Two to eight rows: K a multiple of 8.
+// fp32 Linears X [M][K], W [N][K] of few rows and of a medium number of rows (linear_tiles.hip).  Two to fifteen rows: K a multiple of 8.
 bool linear_few_ok(size_t M, size_t N, size_t K);
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 // Nine rows and more: K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N floats where that is more than one slice.
