@@ -53,6 +53,22 @@ def test_a_page_every_step(design, page_tokens):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("page_tokens", [4, 5, 64])
+@pytest.mark.parametrize("design", ["latent", "chunks"])
+def test_steps_enqueued_four_at_a_time(design, page_tokens):
+    """Lengths around whole fours, prompts that end anywhere in a page: fours, single steps, and both in turn."""
+    lib, cfg = DESIGNS[design]
+    w = lib.weights(cfg, seed=13)
+    runs = []
+    for use_graph in (True, False):
+        m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="float32", max_tokens=512, max_seqs=4, page_tokens=page_tokens, use_graph=use_graph)
+        m.load_weights(w)
+        runs.append([m.generate([lib.tokens(b, n + b, cfg["vocab"]) for b in range(3)], new) for n, new in ((1, 5), (2, 6), (3, 7), (4, 8), (6, 9), (9, 21), (11, 38))])
+        m.close()
+    for a, b in zip(*runs):
+        assert np.array_equal(a, b)
+
+
 def test_key_buckets():
     lib, cfg = DESIGNS["whole"]
     w = lib.weights(cfg, seed=2)
