@@ -1,6 +1,6 @@
 // Greedy decode of ONE sequence as a resident kernel: the whole chip stays inside one launch for up to 64 tokens (GPT.forward + the
 // argmax of generate, src/main.zig:178-195, :322-342), and the phases of a Block meet through tagged words instead of launch
-// boundaries.  Measured: GPT-2 124M 207 -> 117 us a token (256 tokens; 1024: 207 -> 131), fp32 weights 277 -> 155, the char model 94 -> 38.
+// boundaries.  Measured: GPT-2 124M 207 -> 110 us a token (256 tokens; 1024: 207 -> 122), fp32 weights 277 -> 147, the char model 94 -> 37.
 //
 // What bounded it: a step was 62 dependent launches (124M) of 2.7-4 us each, most of that the boundary, the first loads behind it
 // and the fetch of weights nobody could request ahead.  What a hand-over inside a kernel costs depends on how far it goes:
@@ -15,7 +15,7 @@
 //                                                   bias and residual, which stays in registers -> x (XCD)
 //   D  ln_2 + c_fc + GELU, an eighth             -> h            (XCD)
 //   E  mlp c_proj over that eighth               -> partial sums (all XCDs) -> x (XCD)
-// A Block takes 8 to 9 us at 124M; the hand-overs alone 7, the vocabulary's 77 MB 14 of a step's 117 (5.7 TB/s).
+// A Block takes 8 to 9 us at 124M; the hand-overs alone 7, the vocabulary's 77 MB 13 of a step's 110 (5.9 TB/s), its pick 2.
 //
 // What else it needed (us a token at 124M, 256 tokens, as each came in):
 //   149  weights of the next Block requested into registers by the waves that poll: a poll returns behind them, loads of a wave being in order
@@ -24,6 +24,8 @@
 //        store to a line that eight XCDs poll invalidates it in all of them
 //   119  the fetches where nobody's word waits behind them in the compute unit's one queue of vector memory (27 B a cycle with fetches in it)
 //   117  fewer registers in the vocabulary's loop: a spill there waits for the rows in flight
+//   112  no rows requested behind a wave's last (8.25 a half wave: 12 were)
+//   110  the pick's value first and then its index; the attention's weights without readlane, and a longer pause behind it
 //
 // Safety: every workgroup must be resident before any may wait for another.  Workgroups register; the last one commits, and
 // one that has waited too long withdraws the launch for all (a compare-and-swap decides, so all agree): then nothing has been
@@ -38,8 +40,8 @@ namespace {
 using namespace resident;
 constexpr int kFar = 32;         // words of a workgroup's partial sums: two cache lines of its own
 // Pauses, x 64 cycles, measured at 124M and the char model: before the first look at words of other XCDs (0: +4 %; 16: +1 %); before the
-// fetches of a Block, behind c_attn's words (0: +6 %) and behind the attention (4: +3 %)
-constexpr int kFarSleep = 8, kAfterA = 20, kAfterB = 12;
+// fetches of a Block, behind c_attn's words (0: +10 %; 12: +3 %; 24: +1 %) and behind the attention (4: +5 %; 12: +0.5 %; 32: +2 %)
+constexpr int kFarSleep = 8, kAfterA = 20, kAfterB = 18;
 
 // ------------------------------------------------------------------------------------------------ pieces of rows in registers
 // N consecutive elements of a row, at a byte offset of 32 bits from a scalar base (the address costs a lane one register)
@@ -147,7 +149,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
     __shared__ float2 s_stat[2][16];
     __shared__ __attribute__((aligned(16))) float s_new[192];  // q, k, v
     __shared__ __attribute__((aligned(16))) float s_o[4 * AW][64];
-    __shared__ float s_m[AW], s_l[AW];
+    __shared__ __attribute__((aligned(16))) float s_m[AW], s_l[AW];
     __shared__ __attribute__((aligned(16))) float s_part[MS][HC];
     __shared__ __attribute__((aligned(8))) float s_ml[NH][MS][2];
     __shared__ __attribute__((aligned(16))) float s_h[F];
@@ -255,6 +257,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                 }
             }
         };
+        // Eight lanes have a position's key, 16 lanes (a row) its values, four each: of eight positions a row has the values of the
+        // two that it scores, so that a weight is in its row already (or eight lanes away).  readlane for all of them: 0.15 us more
         f32x4 kr[PW / 8][2], vr[PW / 4];
         auto load_KV = [&](int l, int T) {  // the cache rows in front of position T - 1
             // rows this XCD's workgroups wrote: past the L1 (sc1), whose lines may be older.  Positions that are not there yet re-read
@@ -273,7 +277,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
             }
 #pragma unroll
             for (int i = 0; i < PW / 4; ++i)
-                vr[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i * 4 + (l8 >> 4), last) * 256 + (l8 & 15) * 16, 0, 16));
+                vr[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i / 2 * 8 + i % 2 + (l8 >> 4) * 2, last) * 256 + (l8 & 15) * 16, 0, 16));
         };
         constexpr int nKV = 2 * (PW / 8) + PW / 4;
         int vp = 0;
@@ -319,28 +323,25 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                             }
                             const float dot = sum8(acc0 + acc1) * 0.125f;  // 1 / sqrt(64): ops.zig:275
                             sc[i] = t < T ? dot : kNone;
-                            m = fmaxf(m, wave_allmax(sc[i]));
+                            m = fmaxf(m, sc[i]);
                         }
+                        auto over_rows = [&](float v, auto op) { return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48))); };
+                        m = over_rows(fmaxf(m, dpp_row_ror<8>(m)), [](float x, float y) { return fmaxf(x, y); });
                         f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};  // four columns, every fourth position
                         float lsum = 0.0f;
 #pragma unroll
                         for (int i = 0; i < PW / 8; ++i) {
-                            const int t = p0 + i * 8 + (lane >> 3);
-                            const float p = t < T ? __expf(sc[i] - m) : 0.0f;
-                            float pj[8];
-#pragma unroll
-                            for (int j = 0; j < 8; ++j) {
-                                pj[j] = lane_value(p, 8 * j);
-                                lsum += pj[j];
-                            }
+                            const float p = p0 + i * 8 + (lane >> 3) < T ? __expf(sc[i] - m) : 0.0f, other = dpp_row_ror<8>(p);
+                            lsum += p + other;
 #pragma unroll
                             for (int q = 0; q < 2; ++q) {
-                                const int g = lane >> 4, tj = p0 + i * 8 + q * 4 + g;
-                                const float pq = g & 2 ? (g & 1 ? pj[q * 4 + 3] : pj[q * 4 + 2]) : (g & 1 ? pj[q * 4 + 1] : pj[q * 4]);
+                                const int tj = p0 + i * 8 + q + (lane >> 4) * 2;
+                                const float pq = (lane >> 3 & 1) == q ? p : other;
 #pragma unroll
                                 for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? vr[i * 2 + q][d] : 0.0f, o[d]);
                             }
                         }
+                        lsum = over_rows(lsum, [](float x, float y) { return x + y; });
                         *reinterpret_cast<f32x4*>(&s_o[fw * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
                         if (lane == 0) {
                             s_m[fw] = m;
@@ -484,14 +485,15 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                     barrier();  // B2
                     barrier();  // B3
                     if (wave == 0) {
-                        float m = kNone, o = 0.0f, lsum = 0.0f;
-#pragma unroll
-                        for (int i = 0; i < AW; ++i) m = fmaxf(m, s_m[i]);
+                        static_assert(AW == 4, "waves that attend");
+                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(s_m), l4 = *reinterpret_cast<const f32x4*>(s_l);
+                        const float m = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w));
+                        float o = 0.0f, lsum = 0.0f;
 #pragma unroll
                         for (int i = 0; i < AW; ++i) {
-                            const float e = __expf(s_m[i] - m);
+                            const float e = __expf(m4[i] - m);
                             o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
-                            lsum = fmaf(e, s_l[i], lsum);
+                            lsum = fmaf(e, l4[i], lsum);
                         }
                         const unsigned to = P::att + (hi * G + sp) * kPartStride + lane;
                         if (lane < 2) put_near(near, to + 64, tagged(tag, lane ? lsum : m));
@@ -598,7 +600,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
         if (s >= a.n_prompt) {  // ---- ln_f + lm_head + argmax (main.zig:189-194, :337)
             const int wg = k * kRanks + r, V = a.vocab;
             const int pairs = (V + 1) >> 1, per = (pairs + kXcds * kRanks - 1) / (kXcds * kRanks);  // two rows at a time, half a wave each
-            const int p_end = min((wg + 1) * per, pairs), nj = (per + NW - 1) / NW;
+            const int p_end = min((wg + 1) * per, pairs), nj = (p_end - wg * per - wave + NW - 1) / NW;  // (negative: this wave has none)
             Piece<WT, LC> ring[LR][LN];
             auto row_of = [&](int j) { return 2 * (wg * per + wave + NW * j) + half; };
             auto fetch = [&](Piece<WT, LC> (&to)[LN], int j) {
@@ -617,31 +619,35 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                 barrier();  // B8
             }
             const unsigned at_z = lds_at(&s_z[1][l32 * LC]);  // (read again for every row: in registers z would push others out to memory)
-            for (int j0 = 0; j0 < nj; j0 += LR) {
+            auto row_dot = [&](const Piece<WT, LC> (&of)[LN], int j, auto behind) {
+                float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-                for (int u = 0; u < LR; ++u) {
-                    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                for (int q = 0; q < LN; ++q) {
+                    float z[LC];
 #pragma unroll
-                    for (int q = 0; q < LN; ++q) {
-                        float z[LC];
-#pragma unroll
-                        for (int d = 0; d < LC; d += 4) {
-                            const f32x4 v4 = lds_read<f32x4>(fresh(at_z) + (unsigned)(q * 32 * LC + d) * 4u);
-                            z[d] = v4.x; z[d + 1] = v4.y; z[d + 2] = v4.z; z[d + 3] = v4.w;
-                        }
-                        fma_piece<WT, LC>(ring[u][q], z, acc);
+                    for (int d = 0; d < LC; d += 4) {
+                        const f32x4 v4 = lds_read<f32x4>(fresh(at_z) + (unsigned)(q * 32 * LC + d) * 4u);
+                        z[d] = v4.x; z[d + 1] = v4.y; z[d + 2] = v4.z; z[d + 3] = v4.w;
                     }
-                    fetch(ring[u], j0 + u + LR);
-                    const float y = group_allsum<32>((acc[0] + acc[1]) + (acc[2] + acc[3]));
-                    const int row = row_of(j0 + u);
-                    const bool has = (row >> 1) < p_end && row < V;
-                    if (has && y > v) {  // rows of a lane ascend: the first of equal values stays
-                        v = y;
-                        i = row;
-                    }
-                    if (last && has && l32 == 0) *(gptr<float>)(base_at(a.logits) + fresh((unsigned)row * 4u)) = y;
+                    fma_piece<WT, LC>(of[q], z, acc);
                 }
+                behind();
+                const float y = group_allsum<32>((acc[0] + acc[1]) + (acc[2] + acc[3]));
+                const int row = row_of(j);
+                const bool has = (row >> 1) < p_end && row < V;
+                if (has && y > v) {  // rows of a lane ascend: the first of equal values stays
+                    v = y;
+                    i = row;
+                }
+                if (last && has && l32 == 0) *(gptr<float>)(base_at(a.logits) + fresh((unsigned)row * 4u)) = y;
+            };
+            int j0 = 0;
+            for (; j0 + LR < nj; j0 += LR) {
+#pragma unroll
+                for (int u = 0; u < LR; ++u) row_dot(ring[u], j0 + u, [&]() { fetch(ring[u], j0 + u + LR); });
             }
+#pragma unroll
+            for (int u = 0; u < LR; ++u) row_dot(ring[u], j0 + u, []() {});
             {
                 const float v1 = lane_value(v, 32);
                 const int i1 = __builtin_amdgcn_readlane(i, 32);
@@ -663,7 +669,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                 };
                 v = s_bv[min(lane, NW - 1)];
                 i = s_bi[min(lane, NW - 1)];
-                argmax_wave(v, i);
+                argmax_row(v, i);  // (the first row has them all)
                 if (lane < 2) put_near(near, P::best + 2 * r + lane, tagged(tag, lane ? __int_as_float(i) : v));
                 if (r == 0) {
                     pair_up(w.get(near, P::best + lane, tag));
@@ -672,7 +678,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                 }
                 __builtin_amdgcn_s_sleep(kFarSleep);
                 pair_up(w.get(picks, (unsigned)((lane >> 1 & 7) * 16 + (lane & 1)), tag));
-                argmax_wave(v, i);
+                argmax_row(v, i);
                 if (lane == 0) {
                     s_bv[12] = v;
                     s_bi[12] = i;

@@ -1,7 +1,6 @@
 // Greedy decode of two to eight sequences in lock step as a resident kernel: decode_resident.hip's cut of a Block over the XCDs and its
-// hand-overs, the products on the matrix cores.  GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 41.0 ms (318 -> 222 us a step; 33 + 991
-// tokens 322 -> 245 ms), 2 sequences 244 -> 150 us a step; char model, 8 sequences 36.8 -> 17.0 ms.
-//  bf16 weights: an activation travels as the exact three-term bf16 split of its
+// hand-overs, the products on the matrix cores.  GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 40.4 ms (318 -> 219 us a step; 33 + 991
+// tokens 322 -> 241 ms), 2 sequences 244 -> 148 us a step; char model, 8 sequences 36.8 -> 16.8 ms.  bf16 weights: an activation travels as the exact three-term bf16 split of its
 // fp32 value (zg_common.h split3_pk), split once by the thread that makes it, all three terms and a tag of 16 bits in ONE word; a wave
 // multiplies 16 weight rows with the terms of all sequences (v_mfma_f32_16x16x32_bf16: columns of a product are terms x sequences),
 // the waves split K and meet in the LDS.
@@ -57,18 +56,22 @@ __device__ __forceinline__ float sum_over_8(float v) {
     rows_apart_32(__float_as_uint(v), a, b);
     return __uint_as_float(a) + __uint_as_float(b);
 }
-__device__ __forceinline__ void best_over_rows(float& v, int& i) {  // over the lanes 16 apart, on all of them
-    unsigned a, b, ia, ib;
+// over the lanes 16 apart, or those with the same lane & 7, on all of them: the largest value, of equal ones the lowest index
+template <bool EIGHT>
+__device__ __forceinline__ void best_over(float& v, int& i) {
+    const float own = v;
+    unsigned a, b;
+    if (EIGHT) v = fmaxf(v, dpp_row_ror<8>(v));
     rows_apart_16(__float_as_uint(v), a, b);
-    rows_apart_16((unsigned)i, ia, ib);
-    v = __uint_as_float(a);
-    i = (int)ia;
-    better(v, i, __uint_as_float(b), (int)ib);
+    v = fmaxf(__uint_as_float(a), __uint_as_float(b));
     rows_apart_32(__float_as_uint(v), a, b);
-    rows_apart_32((unsigned)i, ia, ib);
-    v = __uint_as_float(a);
-    i = (int)ia;
-    better(v, i, __uint_as_float(b), (int)ib);
+    v = fmaxf(__uint_as_float(a), __uint_as_float(b));
+    int c = own == v ? i : 0x7fffffff;
+    if (EIGHT) c = min(c, __builtin_amdgcn_update_dpp(0, c, 0x128, 0xF, 0xF, true));
+    rows_apart_16((unsigned)c, a, b);
+    c = min((int)a, (int)b);
+    rows_apart_32((unsigned)c, a, b);
+    i = min((int)a, (int)b);
 }
 
 template <int NW, int NH, int MB>
@@ -222,7 +225,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                 }
             }
         }
-        best_over_rows(bv, bi);
+        best_over<false>(bv, bi);
         if (lane < 8) {
             s_bv[wave][lane] = bv;
             s_bi[wave][lane] = bi;
@@ -284,8 +287,9 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
         // =========================================================================================== fetch and attend
         const int fw = wave - NW;
         struct Rows {
-            f32x4 k[2][2], v[4];  // 16 positions: 8 x 8 dims of keys, 4 x 4 dims of values a lane
+            f32x4 k[2][2], v[4];  // 16 positions: 8 x 8 dims of keys, 4 x 4 dims of values a lane (laid out as in decode_resident.hip)
         };
+        auto over_rows = [](float v, auto op) { return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48))); };
         // (in front of loads that are not always made: the registers would be kept for the rows they held before)
         auto forget = [&](Rows& x) {
             asm volatile("" : "=v"(x.k[0][0]), "=v"(x.k[0][1]), "=v"(x.k[1][0]), "=v"(x.k[1][1]));
@@ -309,7 +313,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                to.v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i * 4 + (l8 >> 4), last) * 256 + (l8 & 15) * 16, 0, 16));
+                to.v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i / 2 * 8 + i % 2 + (l8 >> 4) * 2, last) * 256 + (l8 & 15) * 16, 0, 16));
         };
         int vp = 0;
         fetch_V(0, 0, fw);
@@ -367,7 +371,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                                 float top = sc[0];
 #pragma unroll
                                 for (int i = 1; i < 2 * N; ++i) top = fmaxf(top, sc[i]);
-                                mn = fmaxf(mn, wave_allmax(top));
+                                mn = fmaxf(mn, over_rows(fmaxf(top, dpp_row_ror<8>(top)), [](float x, float y) { return fmaxf(x, y); }));
                             }
                             const f32x4 vn = lds_read<f32x4>(fresh(lds_at(&s_new[128 + (lane & 15) * 4])));
                             const float e0 = __expf(m - mn);
@@ -375,18 +379,14 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                             o *= e0;
 #pragma unroll
                             for (int i = 0; i < 2 * N; ++i) {
-                                const int tb = p0 + i / 2 * 64 + i % 2 * 8, t = tb + (lane >> 3);
-                                const float p = t < T ? __expf(sc[i] - mn) : 0.0f;
-                                float pj[8];
-#pragma unroll
-                                for (int j = 0; j < 8; ++j) {
-                                    pj[j] = lane_value(p, 8 * j);
-                                    lsum += pj[j];
-                                }
+                                const int tb = p0 + i / 2 * 64 + i % 2 * 8;
+                                const float p = tb + (lane >> 3) < T ? __expf(sc[i] - mn) : 0.0f, other = dpp_row_ror<8>(p);
+                                lsum += p + other;
+                                if (N == 2) __builtin_amdgcn_sched_barrier(0);  // (the values, last to arrive, are not waited for earlier: 2 % of long contexts)
 #pragma unroll
                                 for (int q = 0; q < 2; ++q) {
-                                    const int g = lane >> 4, tj = tb + q * 4 + g;
-                                    const float pq = g & 2 ? (g & 1 ? pj[q * 4 + 3] : pj[q * 4 + 2]) : (g & 1 ? pj[q * 4 + 1] : pj[q * 4]);
+                                    const int tj = tb + q + (lane >> 4) * 2;
+                                    const float pq = (lane >> 3 & 1) == q ? p : other;
 #pragma unroll
                                     for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? kv[i / 2].v[i % 2 * 2 + q][d] : 0.0f, o[d]);
                                 }
@@ -402,6 +402,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                             forget(kv[1]);
                             if (c + 1 < c1) load_KV(kv[1], l, T, c + 1);
                         }
+                        lsum = over_rows(lsum, [](float x, float y) { return x + y; });
                         *reinterpret_cast<f32x4*>(&s_o[fw * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
                         if (lane == 0) {
                             s_m[fw] = m;
@@ -805,17 +806,21 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
             head_tiles(last);
             barrier();  // B8
             const unsigned tag = tag0 + (unsigned)a.n_layer + 1u;
-            if (wave == 0 && lane < 8) {  // the workgroup's
-                float v = -3.0e38f;
-                int i = 0x7fffffff;
-                for (int q = 0; q < NW + 4; ++q) better(v, i, s_bv[q][lane], s_bi[q][lane]);
-                put_near(near, P::best + (unsigned)(r * 16 + 2 * lane), tagged(tag, v));
-                put_near(near, P::best + (unsigned)(r * 16 + 2 * lane + 1), tagged(tag, __int_as_float(i)));
-            }
-            auto reduce8 = [&](float& v, int& i) {  // over lanes with the same lane & 7
-                better(v, i, dpp_row_ror<8>(v), __builtin_amdgcn_update_dpp(0, i, 0x128, 0xF, 0xF, true));
-                best_over_rows(v, i);
+            static_assert(NW + 4 <= 16, "two waves' bests a lane");
+            // (value, index): two words, in one store
+            auto put_pair = [&](u64* base, unsigned at, float v, int i, auto scope) {
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{__float_as_uint(v), tag, (unsigned)i, tag}, words_at(base), (int)fresh(at * 8u), 0, scope);
             };
+            constexpr std::integral_constant<int, 0> in_xcd{};
+            constexpr std::integral_constant<int, 16> everywhere{};
+            if (wave == 0) {  // the workgroup's: lane -> (waves lane >> 3 and that + 8, sequence lane & 7)
+                const int q = lane >> 3, q8 = min(q + 8, NW + 3);
+                float v = s_bv[min(q, NW + 3)][lane & 7];
+                int i = s_bi[min(q, NW + 3)][lane & 7];
+                better(v, i, s_bv[q8][lane & 7], s_bi[q8][lane & 7]);
+                best_over<true>(v, i);
+                if (lane < 8) put_pair(near, P::best + (unsigned)(r * 16 + 2 * lane), v, i, in_xcd);
+            }
             auto pair_at = [&](u64* base, unsigned at, float& v, int& i) {
                 const auto b = words_at(base);
                 u32x4 p;
@@ -842,18 +847,15 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                 }
 #pragma unroll
                 for (int q = 0; q < 4; ++q) better(v, i, __uint_as_float(p[q].x), (int)p[q].z);
-                reduce8(v, i);
-                if (lane < 8) {
-                    put_far(picks, (unsigned)(k * 16 + 2 * lane), tagged(tag, v));
-                    put_far(picks, (unsigned)(k * 16 + 2 * lane + 1), tagged(tag, __int_as_float(i)));
-                }
+                best_over<true>(v, i);
+                if (lane < 8) put_pair(picks, (unsigned)(k * 16 + 2 * lane), v, i, everywhere);
             }
             if (wave == 0) {
                 float v;
                 int i;
                 __builtin_amdgcn_s_sleep(kPause);
                 pair_at(picks, (unsigned)((lane >> 3) * 16 + 2 * (lane & 7)), v, i);
-                reduce8(v, i);
+                best_over<true>(v, i);
                 // logits that are all NaN: index 0, never one behind the table (embed_step_kernel)
                 if (lane < 8) {
                     s_tok[lane] = (unsigned)i < (unsigned)a.vocab ? i : 0;

@@ -78,14 +78,27 @@ __device__ __forceinline__ void better(float& v, int& i, float ov, int oi) {  //
     }
 }
 
-__device__ __forceinline__ void argmax_wave(float& v, int& i) {  // on all lanes
-#define ZG_AM_STEP(N) better(v, i, dpp_row_ror<N>(v), __builtin_amdgcn_update_dpp(0, i, 0x120 | N, 0xF, 0xF, true));
-    ZG_AM_STEP(8) ZG_AM_STEP(4) ZG_AM_STEP(2) ZG_AM_STEP(1)
-#undef ZG_AM_STEP
-    const float rv = v;
-    const int ri = i;
-#pragma unroll
-    for (int q = 0; q < 64; q += 16) better(v, i, lane_value(rv, q), __builtin_amdgcn_readlane(ri, q));
+// the largest value and of equal ones the lowest index: over the 16 lanes of a row; over the wave, on all lanes.  (First the value, then the
+// index among those that have it: a step is one instruction each, where pairs take five that depend on each other.)
+__device__ __forceinline__ int row_min(int i) {
+#define ZG_MIN_STEP(N) i = min(i, __builtin_amdgcn_update_dpp(0, i, 0x120 | N, 0xF, 0xF, true));
+    ZG_MIN_STEP(8) ZG_MIN_STEP(4) ZG_MIN_STEP(2) ZG_MIN_STEP(1)
+#undef ZG_MIN_STEP
+    return i;
+}
+__device__ __forceinline__ void argmax_row(float& v, int& i) {
+    const float own = v;
+    v = fmaxf(v, dpp_row_ror<8>(v));
+    v = fmaxf(v, dpp_row_ror<4>(v));
+    v = fmaxf(v, dpp_row_ror<2>(v));
+    v = fmaxf(v, dpp_row_ror<1>(v));
+    i = row_min(own == v ? i : 0x7fffffff);
+}
+__device__ __forceinline__ void argmax_wave(float& v, int& i) {
+    const float own = v;
+    v = wave_allmax(v);
+    const int c = row_min(own == v ? i : 0x7fffffff);
+    i = min(min(__builtin_amdgcn_readlane(c, 0), __builtin_amdgcn_readlane(c, 16)), min(__builtin_amdgcn_readlane(c, 32), __builtin_amdgcn_readlane(c, 48)));
 }
 
 template <int N>
