@@ -1,18 +1,20 @@
 // Greedy decode of two to eight sequences in lock step as a resident kernel: decode_resident.hip's cut of a Block over the XCDs and its
-// hand-overs, the products on the matrix cores.  GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 40.4 ms (318 -> 219 us a step; 33 + 991
-// tokens 322 -> 241 ms), 2 sequences 244 -> 148 us a step; char model, 8 sequences 36.8 -> 16.8 ms.  bf16 weights: an activation travels as the exact three-term bf16 split of its
-// fp32 value (zg_common.h split3_pk), split once by the thread that makes it, all three terms and a tag of 16 bits in ONE word; a wave
-// multiplies 16 weight rows with the terms of all sequences (v_mfma_f32_16x16x32_bf16: columns of a product are terms x sequences),
-// the waves split K and meet in the LDS.
+// hand-overs, the products on the matrix cores.  GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 35.7 ms (318 -> 194 us a step; 33 + 991
+// tokens 322 -> 217 ms), 2 sequences 244 -> 133 us a step; char model, 8 sequences 36.8 -> 15.3 ms.  bf16 weights: an activation travels as
+// the exact three-term bf16 split of its fp32 value (zg_common.h split3_pk), split once by the thread that makes it, all three terms and a
+// tag of 16 bits in ONE word; a wave multiplies 16 weight rows with the terms of all sequences (v_mfma_f32_16x16x32_bf16: columns of a
+// product are terms x sequences), the waves split K and meet in the LDS.  A wave polls for the words its own lanes multiply, laid out as they
+// ask for them, and the lanes that share a sequence hand its terms round (DPP): through the LDS and a barrier 40.4 ms.
 //
 // Per Block: x -> A c_attn -> q, k, v -> B attention -> C merge + c_proj -> (all XCDs) -> x -> D c_fc + GELU -> h -> E mlp c_proj -> (all XCDs) -> x.
 // The thread that adds up a column of x (bias, residual, eight partial sums) also multiplies it with the gain of the LayerNorm that
 // follows; mean and variance arrive as sums of 8 columns beside it and are applied to the product's outputs (LayerNorm linearised, as
 // in gemv_ksplit.hip).
 //
-// What bounds it (8 sequences, 256 tokens, 14 us a Block): x is 48 KB of words for every workgroup, twice a Block, weights 60, keys and values 64:
+// What bounds it (8 sequences, 256 tokens, 13 us a Block): x is 48 KB of words for every workgroup, twice a Block, weights 60, keys and values 64:
 // the compute unit's one queue of vector memory (27 to 64 B a cycle).  Measured and left out: a look at the sums alone before
-// the columns are asked for (+2 %, a round trip more), pauses between looks (+0.5 %), rows of keys kept in registers across Blocks (spills).
+// the columns are asked for (+2 %, a round trip more), pauses between looks (+0.5 %), keys of the next Block asked for beside the MLP
+// (+2 %), c_proj's weights behind the merge instead of in front of c_attn (+1 %), partial sums polled by their column's thread alone (+0.6 %).
 #include "decode_resident_parts.h"
 #include "zg_once.h"
 
@@ -26,6 +28,7 @@ using namespace resident;
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef unsigned short u16;
 constexpr int kPause = 8;                     // x 64 cycles before the first look at words of other XCDs
+constexpr int kAfterX = 22;                   // before the first loads of a Block, behind the far words of the one in front (0: +1 %; 36: +1 %; 60: +3 %)
 constexpr int kAfterA = 20;                   // before the fetches of a Block, behind c_attn's words
 constexpr int kMostSplits = 4;                // workgroups that share the positions of a (head, sequence)
 
@@ -94,7 +97,7 @@ struct Hall {
     static constexpr int step = 3 * MB * 64 + 64;              // the terms of 32 columns of all sequences (64 more: consecutive steps start in other banks)
     static constexpr int TI = (CPR + 15) / 16;                 // tiles of 16 rows of C and E
     static constexpr int A = 0, C = A + 2 * nA * 4096, D = C + nC * 4096, Eo = D + nD * 4096, X = Eo + nE * 4096, acc = X + (E / 32) * step,
-                         far_ = acc + NW * TI * 128 * 4, bytes = far_ + kXcds * CPR * 8 * 4;
+                         far_ = acc + (128 * NW + 16) * TI * 4, bytes = far_ + kXcds * CPR * 8 * 4;
 };
 
 template <int NW, int NH, int MB>
@@ -111,10 +114,10 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
 
     extern __shared__ __attribute__((aligned(16))) char s_hall[];
     __shared__ float s_vec[2][192];                                // c2, c3 of the rows of A (12 each) and D (20 each); biases of the columns (32 each); ln_1 g, ln_2 g (32 each)
-    __shared__ __attribute__((aligned(8))) float s_sum[NW][8][2];
+    __shared__ __attribute__((aligned(16))) float s_sum[2][8][NW];
     __shared__ __attribute__((aligned(16))) float s_new[192];      // q, k, v
     __shared__ __attribute__((aligned(16))) float s_o[16][64];
-    __shared__ float s_m[4], s_l[4];
+    __shared__ __attribute__((aligned(16))) float s_m[4], s_l[4];
     __shared__ float s_bv[16][8];
     __shared__ int s_bi[16][8];
     __shared__ int s_tok[8];
@@ -166,6 +169,33 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
     };
     const unsigned hall = lds_at(s_hall);
 
+    // the waves' shares of something, neighbours in the LDS
+    auto sum_shares = [&](unsigned at) {
+        if constexpr (NW % 4 == 0) {
+            f32x4 v[NW / 4];
+#pragma unroll
+            for (int q = 0; q < NW / 4; ++q) v[q] = lds_read<f32x4>(at + q * 16);
+            f32x4 s = v[0];
+#pragma unroll
+            for (int q = 1; q < NW / 4; ++q) s += v[q];
+            return (s.x + s.y) + (s.z + s.w);
+        } else {
+            f32x2 v[NW / 2];
+#pragma unroll
+            for (int q = 0; q < NW / 2; ++q) v[q] = lds_read<f32x2>(at + q * 8);
+            f32x2 s = v[0];
+#pragma unroll
+            for (int q = 1; q < NW / 2; ++q) s += v[q];
+            return s.x + s.y;
+        }
+    };
+    auto stats = [&](int m, float& mean, float& rstd) {
+        const unsigned at = fresh(lds_at(&s_sum[0][m][0]));
+        const float sx = sum_shares(at), sxx = sum_shares(at + 8 * NW * 4);
+        mean = sx * (1.0f / (float)E);
+        rstd = __builtin_amdgcn_rsqf(sxx * (1.0f / (float)E) - mean * mean + 1e-5f);
+    };
+
     // ---- the vocabulary's rows: 16 of them with all sequences, by any wave
     auto head_tiles = [&](bool last) {
         const int V = a.vocab, tiles = (V + 15) >> 4, row16 = lane & 15, g4 = lane >> 4, m = lane & 15;
@@ -200,17 +230,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                 }
             }
             float mean, rstd;
-            {
-                float sx = 0.0f, sxx = 0.0f;
-#pragma unroll
-                for (int q = 0; q < NW; ++q) {
-                    const f32x2 s2 = *reinterpret_cast<const f32x2*>(s_sum[q][m & 7]);
-                    sx += s2.x;
-                    sxx += s2.y;
-                }
-                mean = sx * (1.0f / (float)E);
-                rstd = __builtin_amdgcn_rsqf(sxx * (1.0f / (float)E) - mean * mean + 1e-5f);
-            }
+            stats(m & 7, mean, rstd);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const float s = MB == 8 ? (acc1[i] + dpp_row_ror<8>(acc[i])) + acc[i] : (dpp_row_ror<8>(acc[i]) + dpp_row_ror<12>(acc[i])) + acc[i];
@@ -326,8 +346,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
             for (int l = 0; l < a.n_layer; ++l) {
                 const int ln = l + 1 < a.n_layer ? l + 1 : 0;
                 anew();
-                barrier();  // B1
                 if (nh > 0) {
+                    __builtin_amdgcn_s_sleep(kAfterX);
                     if (!here) {
                         fetch_C(l, fw, 4);
                         barrier();  // B1a
@@ -410,6 +430,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                         }
                         barrier();  // B3
                     }
+                } else {
+                    barrier();  // B1
                 }
                 if (!(here && cps > 1)) {
                     fetch_D(l, fw, 4);
@@ -461,7 +483,28 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
         return true;
     };
     auto load16 = [&](__amdgpu_buffer_rsrc_t b, unsigned i) { return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(b, (int)fresh(i * 8u), 0, 16)); };
-    // terms of columns (c, c + 1) of sequence m: their place among the K steps' operands
+    // Words of x and h lie as the lanes of a product ask for them, 1 KB at a time: columns [64 w, 64 w + 64) of x are wave w's two K steps, and
+    // the MB lanes that share a sequence's columns in a product (its three terms) have a half or a quarter of them each.
+    auto x_at = [](int col, int m) {
+        const int w = col >> 6, i = col >> 5 & 1, g = col >> 3 & 3, u = col & 7;
+        return MB == 8 ? ((w * 4 + (u >> 1)) * 64 + g * 16 + i * 8 + m) * 2 + (u & 1) : ((w * 2 + (u >> 1 & 1)) * 64 + g * 16 + (i * 2 + (u >> 2)) * 4 + m) * 2 + (u & 1);
+    };
+    auto h_at = [](int col, int m) {
+        const int w = col >> 5, g = col >> 3 & 3, u = col & 7;
+        return MB == 8 ? ((w * 2 + (u >> 1 & 1)) * 64 + g * 16 + (u >> 2) * 8 + m) * 2 + (u & 1) : (w * 64 + g * 16 + (u >> 1) * 4 + m) * 2 + (u & 1);
+    };
+    auto lane_of = [&]() { return (lane & ~(MB - 1)) | min(lane & (MB - 1), M - 1); };  // (sequences that are not there: the last one's words)
+    // term 0, 1, 2 of a pair of columns
+    auto term = [](const u32x4& v, int i) { return i == 2 ? __builtin_amdgcn_perm(v.w, v.y, 0x05040100u) : __builtin_amdgcn_perm(v.z, v.x, i ? 0x07060302u : 0x05040100u); };
+    // the lanes of quarter `bank` take `v` of the lanes `by` quarters on, the others keep theirs
+    auto from_quarter = [](uint32_t old, uint32_t v, auto by, auto bank) {
+        constexpr int d = decltype(by)::value & 3, ctrl = d == 0 ? 0xE4 : 0x120 | (16 - 4 * d);
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, ctrl, 0xF, 1 << decltype(bank)::value, false);
+    };
+    auto from_half = [](uint32_t old, uint32_t v, auto bank) {  // the lanes of half `bank` take the other half's
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, 0x128, 0xF, decltype(bank)::value ? 0xC : 0x3, false);
+    };
+    // terms of columns (c, c + 1) of sequence m: their place among the K steps' operands in the LDS
     auto put_terms = [&](int c, int m, const u32x4& v) {
         const unsigned at = fresh(hall + R::X + (unsigned)(c >> 5) * R::step + (unsigned)m * 64u + (unsigned)(c & 31) * 2u);
         typedef __attribute__((address_space(3))) uint32_t lds_u32;
@@ -469,15 +512,14 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
         *(lds_u32*)(uintptr_t)(at + MB * 64u) = (v.x >> 16) | (v.z & 0xffff0000u);
         *(lds_u32*)(uintptr_t)(at + 2 * MB * 64u) = (v.y & 0xffffu) | (v.w << 16);
     };
-    // x and its sums of `tag` -> the operands of a product, the waves' shares of the sums
-    auto get_x = [&](unsigned at_x, unsigned at_st, unsigned tag) {
+    // x of `tag`: this wave's 64 columns of all sequences as its lanes multiply them (x_at), and the waves' shares of its sums
+    auto get_x = [&](unsigned at_x, unsigned at_st, unsigned tag, u32x4 (&v)[MX]) {
         const auto b = words_at(near);
-        const int xc = 2 * (tid % (E / 2)), xm = tid / (E / 2) * MX;  // this thread's columns and first sequence
-        u32x4 v[MX], st[NS];
+        u32x4 st[NS];
         for (unsigned n = 0;;) {
             bool ok = true;
 #pragma unroll
-            for (int j = 0; j < MX; ++j) v[j] = load16(b, at_x + (unsigned)(min(xm + j, M - 1) * E + xc));
+            for (int j = 0; j < MX; ++j) v[j] = load16(b, at_x + (unsigned)((wave * MX + j) * 64 + lane_of()) * 2u);
 #pragma unroll
             for (int i = 0; i < NS; ++i) st[i] = load16(b, at_st + 2u * (unsigned)min(tid + i * NT, P::sums / 2 - 1));
 #pragma unroll
@@ -486,8 +528,6 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
             for (int i = 0; i < NS; ++i) ok = ok && st[i].y == tag && st[i].w == tag;
             if (ok || !again(n)) break;
         }
-#pragma unroll
-        for (int j = 0; j < MX; ++j) put_terms(xc, xm + j, v[j]);
         float sx = __uint_as_float(st[0].x), sxx = __uint_as_float(st[0].z);
         if (NS > 1 && tid + NT < P::sums / 2) {
             sx += __uint_as_float(st[NS - 1].x);
@@ -496,20 +536,9 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
         sx = sum_over_8(sx);  // pair tid: sequence tid & 7
         sxx = sum_over_8(sxx);
         if (lane < 8) {
-            s_sum[wave][lane][0] = sx;
-            s_sum[wave][lane][1] = sxx;
+            s_sum[0][lane][wave] = sx;
+            s_sum[1][lane][wave] = sxx;
         }
-    };
-    auto stats = [&](int m, float& mean, float& rstd) {
-        float sx = 0.0f, sxx = 0.0f;
-#pragma unroll
-        for (int q = 0; q < NW; ++q) {
-            const f32x2 s2 = *reinterpret_cast<const f32x2*>(s_sum[q][m]);
-            sx += s2.x;
-            sxx += s2.y;
-        }
-        mean = sx * (1.0f / (float)E);
-        rstd = __builtin_amdgcn_rsqf(sxx * (1.0f / (float)E) - mean * mean + 1e-5f);
     };
     // N K steps from `ws` on (weights: rows of u_row units at `at_w`) times operands' steps of the same numbers, 16 rows from row0 on
     auto product = [&](auto n_steps, unsigned at_w, int u_row, int row0, int ws, f32x4& acc) {
@@ -534,25 +563,86 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
         for (int i = 0; i < 4; ++i)
             acc[i] = MB == 8 ? (s_low[i] + dpp_row_ror<8>(s_top[i])) + s_top[i] : (dpp_row_ror<8>(s_top[i]) + dpp_row_ror<12>(s_top[i])) + s_top[i];
     };
+    // The same with the operands made from the words this wave has: N = 2, x; 1, h.  The weights are in wt already (row lane & 15)
+    auto weights = [&](auto n_steps, unsigned at_w, int u_row, int row0, int ws, u32x4* wt) {
+        const int row = row0 + (lane & 15), g = lane >> 4;
+        const unsigned at_r = fresh(at_w + (unsigned)(row * u_row) * 16u), sw = (unsigned)(row & 7);
+#pragma unroll
+        for (int i = 0; i < decltype(n_steps)::value; ++i) wt[i] = lds_read<u32x4>(at_r + (((unsigned)((ws + i) * 4 + g)) ^ sw) * 16u);
+    };
+    constexpr std::integral_constant<int, 0> k0{};
     constexpr std::integral_constant<int, 1> k1{};
     constexpr std::integral_constant<int, 2> k2{};
-    // (row, sequence) of 16 x 8 outputs: thread row * 8 + sequence finds the waves' shares at the same place
-    float* const s_acc = reinterpret_cast<float*>(s_hall + R::acc);
-    auto share = [&](int slot, const f32x4& acc) {
-        if ((lane & 15) < 8) {
+    constexpr std::integral_constant<int, 3> k3{};
+    auto operands = [&](auto n_steps, const u32x4* v, u32x4* top, u32x4* low) {
+        constexpr int N = decltype(n_steps)::value;
+        if constexpr (MB == 8) {
+            const bool first = (lane & 8) == 0;
+            if constexpr (N == 2) {  // (a lane has all columns of K step lane / 8 & 1)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) s_acc[fresh((unsigned)(slot * 128 + (lane >> 4) * 32 + (lane & 7))) + i * 8] = acc[i];
+                for (int j = 0; j < 4; ++j) {
+                    const uint32_t hi = term(v[j], 0), mid = term(v[j], 1), lo = term(v[j], 2);
+                    top[0][j] = from_half(hi, mid, k1);
+                    top[1][j] = from_half(mid, hi, k0);
+                    low[0][j] = first ? lo : 0u;
+                    low[1][j] = first ? 0u : lo;  // (columns 8 to 15 of that product: added in the end)
+                }
+            } else {  // (the first or the last four columns)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t hi = term(v[j], 0), mid = term(v[j], 1), lo = term(v[j], 2);
+                    top[0][j] = from_half(hi, mid, k1);
+                    top[0][2 + j] = from_half(mid, hi, k0);
+                    low[0][j] = first ? lo : 0u;
+                    low[0][2 + j] = from_half(0u, lo, k0);
+                }
+            }
+        } else {
+            auto all_terms = [&](auto from_q, const u32x4& w) {  // of the pair of columns that quarter from_q has: leading, middle, last term to quarters 0, 1, 2
+                constexpr int q = decltype(from_q)::value;
+                uint32_t x = from_quarter(0u, term(w, 0), std::integral_constant<int, q>{}, k0);
+                x = from_quarter(x, term(w, 1), std::integral_constant<int, q - 1>{}, k1);
+                return from_quarter(x, term(w, 2), std::integral_constant<int, q - 2>{}, k2);
+            };
+            if constexpr (N == 2) {  // (quarter 2 i + h has half h of K step i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    top[0][j] = all_terms(k0, v[j]);
+                    top[0][2 + j] = all_terms(k1, v[j]);
+                    top[1][j] = all_terms(k2, v[j]);
+                    top[1][2 + j] = all_terms(k3, v[j]);
+                }
+            } else {
+                top[0][0] = all_terms(k0, v[0]);
+                top[0][1] = all_terms(k1, v[0]);
+                top[0][2] = all_terms(k2, v[0]);
+                top[0][3] = all_terms(k3, v[0]);
+            }
         }
     };
-    auto total = [&](int tile, int stride, int t) {
-        const unsigned at = fresh((unsigned)(tile * 128 + t));
-        float v[NW], y = 0.0f;
+    auto multiply = [&](auto n_steps, const u32x4* wt, const u32x4* top, const u32x4* low, f32x4& acc) {
+        f32x4 s_low = {0.0f, 0.0f, 0.0f, 0.0f}, s_top = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-        for (int q = 0; q < NW; ++q) v[q] = s_acc[at + q * stride * 128];
+        for (int i = 0; i < decltype(n_steps)::value; ++i) {
+            if (MB == 8) s_low = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wt[i]), __builtin_bit_cast(bf16x8, low[i]), s_low, 0, 0, 0);
+            s_top = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, wt[i]), __builtin_bit_cast(bf16x8, top[i]), s_top, 0, 0, 0);
+        }
 #pragma unroll
-        for (int q = 0; q < NW; ++q) y += v[q];
-        return y;
+        for (int i = 0; i < 4; ++i)
+            acc[i] = MB == 8 ? ((s_low[i] + dpp_row_ror<8>(s_low[i])) + dpp_row_ror<8>(s_top[i])) + s_top[i]
+                             : (dpp_row_ror<8>(s_top[i]) + dpp_row_ror<12>(s_top[i])) + s_top[i];
     };
+    // (row, sequence) of 16 x 8 outputs: thread row * 8 + sequence finds the waves' shares at the same place
+    auto acc_at = [&](int tile, int t) { return hall + R::acc + (unsigned)(tile * (128 * NW + 16) + t * NW + (t >> 5) * 4) * 4u; };  // (four words between the lanes' quarters: banks)
+    auto share = [&](int tile, int of, const f32x4& acc) {
+        if ((lane & 15) < 8) {
+            const unsigned at = fresh(acc_at(tile, (lane >> 4) * 32 + (lane & 7)) + (unsigned)of * 4u);
+            typedef __attribute__((address_space(3))) float lds_f32;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *(lds_f32*)(uintptr_t)(at + i * 8 * NW * 4) = acc[i];
+        }
+    };
+    auto total = [&](int tile, int t) { return sum_shares(fresh(acc_at(tile, t))); };
     float* const s_far = reinterpret_cast<float*>(s_hall + R::far_);
     // thread -> column oc of this workgroup, sequence om, which it owns
     auto om = [&]() { return tid & 7; };
@@ -561,8 +651,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
     auto ocol = [&]() { return r * CPR + min(oc(), CPR - 1); };
     float res = 0.0f;
     // x (in res) -> its terms times `gain`, sums of 8 columns
-    auto put_x = [&](unsigned at_x, unsigned at_st, unsigned tag, float gain) {
-        if (owns()) put_near(near, at_x + (unsigned)(om() * E + ocol()), terms(tag, res * gain));
+    auto put_x = [&](unsigned to_x, unsigned at_st, unsigned tag, float gain) {
+        if (owns()) put_near(near, to_x, terms(tag, res * gain));
         if (wave < OW) {
             const float v = owns() ? res : 0.0f;
             const float sx = sum_over_8(v), sxx = sum_over_8(v * v);
@@ -623,28 +713,33 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
             };
             res = value(a.wte, (size_t)tok) + value(a.wpe, (size_t)s);
         }
-        put_x(P::x2, P::st2, tag0, s_vec[vp][128 + min(oc(), 31)]);
+        put_x(P::x2 + (unsigned)x_at(ocol(), om()), P::st2, tag0, s_vec[vp][128 + min(oc(), 31)]);
         for (int l = 0; l < a.n_layer; ++l) {
             const unsigned tag = tag0 + 1u + (unsigned)l;
             anew();
             if (nh > 0) {
-                get_x(P::x2, P::st2, tag - 1u);
-                barrier();  // B1
                 // ---- A
-                float mean = 0.0f, rstd = 0.0f;
-                if (wave * 8 < 6 * nh) stats(om(), mean, rstd);
                 {
+                    u32x4 wt[2], v[MX], top[2], low[2];
                     f32x4 acc;
-                    product(k2, hall + R::A + vp * R::nA * 4096, E / 8, 0, 2 * wave, acc);
-                    share(wave, acc);
+                    weights(k2, hall + R::A + vp * R::nA * 4096, E / 8, 0, 2 * wave, wt);
+                    get_x(P::x2, P::st2, tag - 1u, v);
+                    operands(k2, v, top, low);
+                    multiply(k2, wt, top, low, acc);
+                    share(0, wave, acc);
                 }
-                barrier();  // B1a
-                float yA = 0.0f;
                 const int jA = tid >> 3, nA = r * 6 * nh + jA;
                 const bool hasA = jA < 6 * nh && om() < M;
+                // (what the outputs are made with and where they go: known before the last share is)
+                const unsigned toA = fresh(P::qkv + (unsigned)(om() * NH * 192 + nA));
+                const float c2A = s_vec[vp][min(jA, 11)], c3A = s_vec[vp][12 + min(jA, 11)];
+                barrier();  // B1a
+                float yA = 0.0f;
                 if (jA < 6 * nh) {
-                    yA = fmaf(rstd, fmaf(-mean, s_vec[vp][jA], total(0, 1, tid)), s_vec[vp][12 + jA]);
-                    if (hasA) put_near(near, P::qkv + (unsigned)(om() * NH * 192 + nA), tagged(tag, yA));
+                    float mean, rstd;
+                    stats(om(), mean, rstd);
+                    yA = fmaf(rstd, fmaf(-mean, c2A, total(0, tid)), c3A);
+                    if (hasA) put_near(near, toA, tagged(tag, yA));
                 }
                 if (here) {
                     if (tid < 192 && (tid < 64 || newest)) s_new[tid] = w.get(near, P::qkv + (unsigned)(im * NH * 192 + ih * 192 + tid), tag);
@@ -662,14 +757,14 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                     }
                     barrier();  // B3
                     if (wave == 0) {
-                        float m = kNone, o = 0.0f, lsum = 0.0f;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) m = fmaxf(m, s_m[i]);
+                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(s_m), l4 = *reinterpret_cast<const f32x4*>(s_l);
+                        const float m = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w));
+                        float o = 0.0f, lsum = 0.0f;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const float e = __expf(s_m[i] - m);
+                            const float e = __expf(m4[i] - m);
                             o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
-                            lsum = fmaf(e, s_l[i], lsum);
+                            lsum = fmaf(e, l4[i], lsum);
                         }
                         const unsigned to = (unsigned)((im * NH + ih) * kMostSplits + sp);
                         if (lane < 2) put_near(near, P::ml + to * 2u + lane, tagged(tag, lane ? lsum : m));
@@ -728,80 +823,93 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
                     const int ws = wave % (2 * NH), ti = wave / (2 * NH);
                     if (ws < 2 * nh) product(k1, hall + R::C, HC / 8, ti * 16, ws, acc);
-                    share(wave, acc);
+                    share(ti, ws, acc);
                 }
                 barrier();  // B4a
                 if (tid < CPR * 8) {
-                    const int ti = tid >> 7;
                     float y = 0.0f;
-                    const unsigned at = fresh((unsigned)(ti * 2 * NH * 128 + (tid & 127)));
-                    float v[2 * NH];
+                    const unsigned at = fresh(acc_at(tid >> 7, tid & 127));
+                    f32x2 v[NH];
 #pragma unroll
-                    for (int q = 0; q < 2 * NH; ++q) v[q] = s_acc[at + q * 128];
+                    for (int q = 0; q < NH; ++q) v[q] = lds_read<f32x2>(at + q * 8);
 #pragma unroll
-                    for (int q = 0; q < 2 * NH; ++q) y += q < 2 * nh ? v[q] : 0.0f;
+                    for (int q = 0; q < NH; ++q) y += q < nh ? v[q].x + v[q].y : 0.0f;
                     if (om() < M) put_far(far1, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, y));
                     else put_far(far1, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, 0.0f));
                 }
             } else {
-                barrier();  // B1
+                barrier();  // B1 (the helpers' fetches of vectors take the place of the Block's in front)
             }
+            unsigned to_x = fresh(P::x1 + (unsigned)x_at(ocol(), om()));
+            float bias = s_vec[vp][64 + min(oc(), 31)], gain = s_vec[vp][160 + min(oc(), 31)];
             gather(far1, nx, tag);
             barrier();  // B4b
-            add_up(nx, s_vec[vp][64 + min(oc(), 31)]);
-            put_x(P::x1, P::st1, tag, s_vec[vp][160 + min(oc(), 31)]);
-            get_x(P::x1, P::st1, tag);
+            add_up(nx, bias);
+            put_x(to_x, P::st1, tag, gain);
             barrier();  // B5
             // ---- D
-            float mean = 0.0f, rstd = 0.0f;
-            if (wave * 8 < NW) stats(om(), mean, rstd);
             {
+                u32x4 wt[2], v[MX], top[2], low[2];
                 f32x4 acc;
-                product(k2, hall + R::D, E / 8, 0, 2 * wave, acc);
-                share(wave, acc);
+                weights(k2, hall + R::D, E / 8, 0, 2 * wave, wt);
+                get_x(P::x1, P::st1, tag, v);
+                operands(k2, v, top, low);
+                multiply(k2, wt, top, low, acc);
+                share(0, wave, acc);
             }
+            const unsigned toD = fresh(P::h + (unsigned)h_at(r * NW + min(oc(), NW - 1), om()));
+            const float c2D = s_vec[vp][24 + min(oc(), NW - 1)], c3D = s_vec[vp][44 + min(oc(), NW - 1)];
             barrier();  // B5a
             if (oc() < NW) {
-                const float y = gelu_ref(fmaf(rstd, fmaf(-mean, s_vec[vp][24 + oc()], total(0, 1, tid)), s_vec[vp][44 + oc()]));
-                if (om() < M) put_near(near, P::h + (unsigned)(om() * F + r * NW + oc()), terms(tag, y));
+                float mean, rstd;
+                stats(om(), mean, rstd);
+                const float y = gelu_ref(fmaf(rstd, fmaf(-mean, c2D, total(0, tid)), c3D));
+                if (om() < M) put_near(near, toD, terms(tag, y));
             }
+            barrier();  // B6
             // ---- E
             {
-                const int c = 2 * (tid % (F / 2)), m0 = tid / (F / 2) * MF;
+                u32x4 wt[TI], v[MF], top[1], low[1];
+#pragma unroll
+                for (int ti = 0; ti < TI; ++ti) weights(k1, hall + R::Eo, F / 8, ti * 16, wave, wt + ti);
                 const auto b = words_at(near);
-                u32x4 v[MF];
                 for (unsigned n = 0;;) {
                     bool ok = true;
 #pragma unroll
                     for (int j = 0; j < MF; ++j) {
-                        v[j] = load16(b, P::h + (unsigned)(min(m0 + j, M - 1) * F + c));
+                        v[j] = load16(b, P::h + (unsigned)((wave * MF + j) * 64 + lane_of()) * 2u);
                         ok = ok && (v[j].y >> 16) == (tag & 0xffffu) && (v[j].w >> 16) == (tag & 0xffffu);
                     }
                     if (ok || !again(n)) break;
                 }
-#pragma unroll
-                for (int j = 0; j < MF; ++j) put_terms(c, m0 + j, v[j]);
-            }
-            barrier();  // B6
-            {
+                operands(k1, v, top, low);
 #pragma unroll
                 for (int ti = 0; ti < TI; ++ti) {
                     f32x4 acc;
-                    product(k1, hall + R::Eo, F / 8, ti * 16, wave, acc);
-                    share(wave * TI + ti, acc);
+                    multiply(k1, wt + ti, top, low, acc);
+                    share(ti, wave, acc);
                 }
             }
             barrier();  // B6a
-            if (tid < CPR * 8) put_far(far2, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, total(tid >> 7, TI, tid & 127)));
+            if (tid < CPR * 8) put_far(far2, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, total(tid >> 7, tid & 127)));
+            to_x = fresh(P::x2 + (unsigned)x_at(ocol(), om()));
+            bias = s_vec[vp][96 + min(oc(), 31)];
+            vp ^= 1;
+            gain = l + 1 < a.n_layer ? s_vec[vp][128 + min(oc(), 31)] : fin_g;
             gather(far2, kXcds, tag);
             barrier();  // B6b
-            add_up(kXcds, s_vec[vp][96 + min(oc(), 31)]);
-            vp ^= 1;
-            put_x(P::x2, P::st2, tag, l + 1 < a.n_layer ? s_vec[vp][128 + min(oc(), 31)] : fin_g);
+            add_up(kXcds, bias);
+            put_x(to_x, P::st2, tag, gain);
         }
         const bool last = s + 1 == a.s1;
         if (s >= a.n_prompt) {  // ---- ln_f + lm_head + argmax (main.zig:189-194, :337)
-            get_x(P::x2, P::st2, tag0 + (unsigned)a.n_layer);
+            {
+                u32x4 v[MX];
+                get_x(P::x2, P::st2, tag0 + (unsigned)a.n_layer, v);
+                const int q = lane >> 3 & 1, c = 64 * wave + (lane >> 4) * 8 + (MB == 8 ? q * 32 : q * 32 + (lane >> 2 & 1) * 4);
+#pragma unroll
+                for (int j = 0; j < MX; ++j) put_terms(c + 2 * j, lane & (MB - 1), v[j]);
+            }
             barrier();  // B7
             head_tiles(last);
             barrier();  // B8
