@@ -1102,7 +1102,7 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
 // Bound by the matrix cores and the LDS together: a fragment of keys (1 KB) serves one product (32 cycles), so the four SIMDs of a
 // compute unit ask the LDS for its whole 128 B per clock; two workgroups per compute unit hide the softmax of one under the
 // products of the other (hence 256 registers a lane: 72 of queries, 128 of sums).  The blocks with the most keys are dealt first.
-// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 121 us and 9 for the tiles (73 GFLOP: 560 TFLOP/s); 827 us when every workgroup
+// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 110 us and 9 for the tiles (73 GFLOP: 615 TFLOP/s); 827 us when every workgroup
 // converted and transposed its own tiles behind three barriers.
 template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
 __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, const bf16_t* qa16, float* ctx, bf16_t* ctx16, int H, int KR, int R, float scale,
@@ -1264,6 +1264,34 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     }
     if (!head_ok) return;
     const float L = lsum + __shfl_xor(lsum, 32, 64);
+    if (ctx16) {  // (KR is a multiple of 8)
+        // A lane has a query's values: turned in the tiles' place, half of the dimensions at a time, they leave as 16-byte pieces of whole rows.
+        // (8 bytes a lane to 32 rows, divided one by one: 6.1 us behind the last tile, 2.0 so)
+        constexpr int P = NT * 16, PITCH = P * 2 + 16;
+        static_assert(32 * PITCH <= T::BYTES / 2, "a wave's rows fit its half of a tile's place");
+        char* const img = &Ks[0][0] + wave * (T::BYTES / 2);
+        const size_t row = (size_t)(m_first + min(r, nq - 1));
+        const float gf = head_gate_f(gate, ldg, row, h);
+        const float by = sink ? gf * sink_norm_f(mx * 0.69314718055994531f, L, sink, h) : gf / L;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+#pragma unroll
+            for (int t = 0; t < NT / 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; i += 4) {
+                    const f32x16& v = o[half * (NT / 2) + t];
+                    *reinterpret_cast<u32x2*>(img + r * PITCH + (t * 32 + 8 * (i >> 2) + 4 * hf) * 2) = u32x2{cvt_pk_bf16(v[i] * by, v[i + 1] * by), cvt_pk_bf16(v[i + 2] * by, v[i + 3] * by)};
+                }
+            // (a wave's accesses to the LDS are in order)
+#pragma unroll
+            for (int q = 0; q < P / 16; ++q) {
+                const int u = q * 64 + lane, qr = u / (P / 8), c = u % (P / 8) * 8;
+                const u32x4 v = *reinterpret_cast<const u32x4*>(img + qr * PITCH + c * 2);
+                if (qr < nq && half * P + c < KR) *reinterpret_cast<u32x4*>(ctx16 + ((size_t)(m_first + qr) * H + h) * KR + half * P + c) = v;
+            }
+        }
+        return;
+    }
     if (r >= nq) return;
     const size_t out_at = ((size_t)(m_first + r) * H + h) * KR;
     float* out = ctx + out_at;
@@ -1277,9 +1305,7 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
             f32x4 v;
 #pragma unroll
             for (int u = 0; u < 4; ++u) v[u] = sink ? o[t][i + u] * gf : o[t][i + u] / L * gf;
-            if (ctx16) {  // (KR is a multiple of 8)
-                if (d < KR) *reinterpret_cast<u32x2*>(ctx16 + out_at + d) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
-            } else if (vec) {
+            if (vec) {
                 if (d < KR) *reinterpret_cast<f32x4*>(out + d) = v;
             } else {
 #pragma unroll
