@@ -1105,7 +1105,9 @@ def main():
             "achieved_layers_walked": round(dom["algorithmic_bytes_per_launch"] / dom["avg_launch_us_layers_walked"] / 1e3, 1),
             "frac_layers_walked": round(dom["algorithmic_bytes_per_launch"] / dom["avg_launch_us_layers_walked"] / 1e3 / HBM_PEAK_GBS, 4),
             "share_of_token_time": dom["share_of_token_time"],
-            "how": "the kernel class with the largest share of the decode-step time; duration = HIP events on the launch "
+            "how": "the kernel class with the largest share of the decode step as launches (what sampling, prompts token by token and the "
+                   "shapes without a resident kernel run; the generation timed here is inside decode_resident*_kernel where that applies: "
+                   "step_roofline is its figure); duration = HIP events on the launch "
                    "stream around a hipGraph chain of that kernel (launch boundary included), measured in this run; "
                    "kernel_classes also lists avg_launch_us_layers_walked: the same chain walking the layers, i.e. with "
                    "weights / KV coming from the memory side as in the real step (lm_head has one matrix: identical)",
@@ -1119,8 +1121,8 @@ def main():
             "achieved": round(step_bytes_total * a.steps / dev_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(step_bytes_total * a.steps / dev_s / 1e9 / HBM_PEAK_GBS, 4),
             "us_per_token_device": round(1e6 * dev_s / (a.steps * ctx), 2),
-            # two clocks that do not share code: torch events around the whole generations (above) against the sum of the per-class
-            # chain timings of kernel_classes (the library's HIP events around hipGraph chains), priced per token with the embed launch
+            # the step as launches, for comparison: the sum of the per-class chain timings of kernel_classes (the library's HIP events
+            # around hipGraph chains), priced per token with the embed launch.  With ZGPT2_RESIDENT=0 it is what us_per_token_device is held to
             "sum_of_kernel_class_chains_us": round(sum(r["avg_launch_us_layers_walked"] * r["launches_per_token"] for r in table) + prof_lo.get("embed", 0.0), 2),
             "per_kernel_class_us_eager_T_low": {k: round(v, 2) for k, v in prof_lo.items()},
             "per_kernel_class_us_eager_T_high": {k: round(v, 2) for k, v in prof_hi.items()},
