@@ -74,3 +74,15 @@ def test_router_with_the_norms_in_front(width, experts, top):
     refs = [oracle.forward(t)[0] for t in toks]
     for n in (1, 2):
         check(cfg, w, refs, toks, n, "float32")
+
+
+@pytest.mark.parametrize("width,ff", [(136, 2047), (136, 2049), (520, 2051), (1032, 2054), (511, 1536), (513, 1536), (515, 1544), (518, 2056)])
+def test_four_rows_a_wave(width, ff):
+    """The products of the norms (ff rows) and of the polynomial (width rows) on either side of where four weight rows share what a row
+    needs in front of them, with one to three left over."""
+    cfg = dl.config([dl.mamba_layer(mlp=dl.dense(ff=ff)), dl.attn_layer(mlp=dl.dense(ff=ff))], width=width)
+    w = dl.weights(cfg, seed=width + ff)
+    toks = [dl.tokens(7 + b, 5, cfg["vocab"]) for b in range(2)]
+    refs = [do.forward(w, cfg, t) for t in toks]
+    for n in (1, 2):
+        check(cfg, w, refs, toks, n, "float32")

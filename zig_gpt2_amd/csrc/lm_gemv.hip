@@ -7,6 +7,10 @@
 //
 // One row, us a launch inside a replayed step, this against the general kernel: 768 columns 4.3 : 5.6, 3072 columns through the polynomial
 // 4.7 : 7.4.  With the sum and the two norms in front of a product inside it 4.45, where their own launch took 5.25 more.
+// What a row needs before its products (norms, the polynomial) is worked out while the weights are on their way and shared by four weight rows
+// (the rule is at the launch): the polynomial had met its weights power by power, eleven sums and fifteen operations an element, where its
+// statistics now meet over the workgroup first and an element is one product a weight row.  Both, 64 tokens of one sequence (768 wide,
+// twelve layers, twelve feed-forwards through it) 19.4 -> 18.8 ms.
 //
 // Short rows: a wave has two whole weight rows.  Long rows (K of 1536 and more): a workgroup has two, its four waves a quarter of K each.
 #include "lm_linear_args.h"
@@ -37,19 +41,22 @@ struct GemvAt {
     int K, N, ldb, lda, a_zoff, b_zoff, a_glu;
     const float* a_norm = nullptr;  // GEMV_RMS: the rows' norm weights
     float eps = 0.0f;
+    const float* a_poly = nullptr;  // GEMV_POLY: its four factors
 };
 
-// INDIRECT: rows through an array, or a matrix chosen by a list
-template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT>
+// NR: weight rows of a wave (SPLIT: of a workgroup).  INDIRECT: rows through an array, or a matrix chosen by a list
+template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT, int NR = 2>
 __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, const int z, const NormIn& pre) {
-    constexpr int NS = KIND == GEMV_POLY ? 11 : KIND == GEMV_RMS ? 3 : 2;  // sums of a row: the two products, with the norm of squares; or q1 q2 q3 and four products for each weight row
-    __shared__ float s_part[SPLIT ? 4 : 1][MR][NS];
+    constexpr int NS = KIND == GEMV_RMS ? NR + 1 : NR;  // sums of a row: the products, then that of squares
+    __shared__ float s_part[SPLIT ? 4 : 1][MR][NS], s_pow[4][MR][3];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int n0 = SPLIT ? blockIdx.x * 2 : blockIdx.x * 8 + wave * 2;
+    const int n0 = SPLIT ? blockIdx.x * NR : (blockIdx.x * 4 + wave) * NR;
     if (n0 >= t.N) return;
     if (INDIRECT && p.z_group && p.z_group[z] >= p.z_limit) return;
     const bf16_t* B = t.B + (long long)(INDIRECT && p.z_group ? p.z_group[z] : z) * t.b_zoff;
-    const bf16_t* w[2] = {B + (long long)n0 * t.ldb, B + (long long)min(n0 + 1, t.N - 1) * t.ldb};
+    const bf16_t* w[NR];
+#pragma unroll
+    for (int c = 0; c < NR; ++c) w[c] = B + (long long)min(n0 + c, t.N - 1) * t.ldb;
     const int kq = SPLIT ? (((t.K + 3) / 4) + 7) & ~7 : t.K;  // a wave's share of K, whole pieces of 8
     const int k_lo = SPLIT ? wave * kq : 0, k_hi = SPLIT ? min(t.K, k_lo + kq) : t.K;
     int at[U];
@@ -60,13 +67,13 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
         in[u] = k < k_hi;
         at[u] = min(k, t.K - 8);
     }
-    u32x4 wr[2][U];
+    u32x4 wr[NR][U];
     f32x4 a[MR][U][2], g[KIND == GEMV_GLU ? MR : 1][U][2], nw[U][2];
     float asc[MR], agate[MR];
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int c = 0; c < 2; ++c) wr[c][u] = *reinterpret_cast<const u32x4*>(w[c] + at[u]);
+        for (int c = 0; c < NR; ++c) wr[c][u] = *reinterpret_cast<const u32x4*>(w[c] + at[u]);
     if constexpr (KIND == GEMV_NORM) {
         // the row is norm(x + norm(y) (1 + wb)) (1 + wn): every wave works it out for itself, the first one keeps the sum
         f32x4 y[U][2], vb[U][2], vn[U][2];
@@ -107,6 +114,11 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
 #pragma unroll
                 for (int e = 0; e < 4; ++e) a[0][u][i][e] = a[0][u][i][e] * r2 * (1.0f + vn[u][i][e]);
     } else {
+        float d[4];
+        if constexpr (KIND == GEMV_POLY) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = t.a_poly[i];
+        }
         const float* A = t.A + (long long)z * t.a_zoff;
         if constexpr (KIND == GEMV_RMS) {
 #pragma unroll
@@ -128,6 +140,52 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
             asc[m] = KIND == GEMV_GLU && p.glu_scale ? p.glu_scale[rid] : 1.0f;
             agate[m] = KIND == GEMV_GLU && p.glu_gate_col >= 0 ? 1.0f / (1.0f + expf(-row[p.glu_gate_col])) : 1.0f;
         }
+        if constexpr (KIND == GEMV_POLY) {
+            // the row is d0 n(v) + d1 n(v^2) + d2 n(v^3) + d3, every power divided by its root mean square: the workgroup's four shares meet, and the
+            // row is worked out, while the weights are on their way
+            static_assert(SPLIT, "the polynomial's rows are long");
+            float q[MR][3];
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+#pragma unroll
+                for (int i = 0; i < 3; ++i) q[m][i] = 0.0f;
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = in[u] ? a[m][u][i][e] : 0.0f, v2 = v * v, v3 = v2 * v;
+                            q[m][0] += v2;
+                            q[m][1] = fmaf(v2, v2, q[m][1]);
+                            q[m][2] = fmaf(v3, v3, q[m][2]);
+                        }
+                wave_sums(q[m]);
+            }
+            if (lane == 0) {
+#pragma unroll
+                for (int m = 0; m < MR; ++m)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i) s_pow[wave][m][i] = q[m][i];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                float f[3];
+#pragma unroll
+                for (int i = 0; i < 3; ++i)
+                    f[i] = d[i] / sqrtf(((s_pow[0][m][i] + s_pow[1][m][i]) + (s_pow[2][m][i] + s_pow[3][m][i])) / (float)t.K + t.eps);
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float v = a[m][u][i][e], v2 = v * v;
+                            a[m][u][i][e] = fmaf(f[2], v2 * v, fmaf(f[1], v2, fmaf(f[0], v, d[3])));
+                        }
+            }
+        }
     }
     ZG_PIN(p.C);
     ZG_PIN(p.bias);
@@ -141,9 +199,9 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
         for (int i = 0; i < NS; ++i) sum[m][i] = 0.0f;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-        float wf[2][8];
+        float wf[NR][8];
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
+        for (int c = 0; c < NR; ++c) {
             const u32x4 v = in[u] ? wr[c][u] : none;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -164,27 +222,14 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
                 if constexpr (KIND == GEMV_RMS) {
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        sum[m][2] = fmaf(x[e], x[e], sum[m][2]);
+                        sum[m][NR] = fmaf(x[e], x[e], sum[m][NR]);
                         x[e] *= nw[u][i][e];
                     }
                 }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const float w0 = wf[0][4 * i + e], w1 = wf[1][4 * i + e];
-                    if constexpr (KIND == GEMV_POLY) {
-                        float* s = sum[m];
-                        const float v = x[e], q = v * v, c = q * v;
-                        s[0] += q;
-                        s[1] = fmaf(q, q, s[1]);
-                        s[2] = fmaf(c, c, s[2]);
-                        s[3] = fmaf(v, w0, s[3]); s[7] = fmaf(v, w1, s[7]);
-                        s[4] = fmaf(q, w0, s[4]); s[8] = fmaf(q, w1, s[8]);
-                        s[5] = fmaf(c, w0, s[5]); s[9] = fmaf(c, w1, s[9]);
-                        s[6] += w0; s[10] += w1;
-                    } else {
-                        sum[m][0] = fmaf(x[e], w0, sum[m][0]);
-                        sum[m][1] = fmaf(x[e], w1, sum[m][1]);
-                    }
+#pragma unroll
+                    for (int r = 0; r < NR; ++r) sum[m][r] = fmaf(x[e], wf[r][4 * i + e], sum[m][r]);
                 }
             }
     }
@@ -192,12 +237,13 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
     for (int m = 0; m < MR; ++m) wave_sums(sum[m]);
     float* C = p.C + (long long)z * p.c_zoff;
     if constexpr (!SPLIT) {
-        static_assert(KIND != GEMV_POLY, "the polynomial's rows are long");
-        if (lane < 2 && n0 + lane < t.N) {
+        if (lane < NR && n0 + lane < t.N) {
 #pragma unroll
             for (int m = 0; m < MR; ++m) {
-                float v = lane ? sum[m][1] : sum[m][0];
-                if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum[m][2] / (float)t.K + t.eps);
+                float v = sum[m][0];
+#pragma unroll
+                for (int r = 1; r < NR; ++r) v = lane == r ? sum[m][r] : v;
+                if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum[m][NR] / (float)t.K + t.eps);
                 C[(long long)m * p.ldc + n0 + lane] = finish(v, n0 + lane, p);
             }
         }
@@ -209,36 +255,31 @@ __device__ __forceinline__ void gemv_body(const GemvAt& t, const LinArgs& p, con
                 for (int i = 0; i < NS; ++i) s_part[wave][m][i] = sum[m][i];
         }
         __syncthreads();
-        const int m = threadIdx.x >> 1, c = threadIdx.x & 1;
+        const int m = threadIdx.x / NR, c = threadIdx.x % NR;
         if (m < MR && n0 + c < t.N) {
             auto sum4 = [&](int i) { return (s_part[0][m][i] + s_part[1][m][i]) + (s_part[2][m][i] + s_part[3][m][i]); };
-            float v;
-            if constexpr (KIND == GEMV_POLY) {
-                const float K = (float)t.K, eps = p.poly_eps, *d = p.a_poly;
-                v = (d[0] / sqrtf(sum4(0) / K + eps) * sum4(3 + 4 * c) + d[1] / sqrtf(sum4(1) / K + eps) * sum4(4 + 4 * c)) +
-                    (d[2] / sqrtf(sum4(2) / K + eps) * sum4(5 + 4 * c) + d[3] * sum4(6 + 4 * c));
-            } else v = sum4(c);
-            if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum4(2) / (float)t.K + t.eps);
+            float v = sum4(c);
+            if constexpr (KIND == GEMV_RMS) v *= 1.0f / sqrtf(sum4(NR) / (float)t.K + t.eps);
             C[(long long)m * p.ldc + n0 + c] = finish(v, n0 + c, p);
         }
     }
 }
 
-template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT>
-__global__ __launch_bounds__(256) void lm_gemv_at_once_kernel(const float* A, const bf16_t* B, int K, int N, int ldb, int lda, int a_zoff, int b_zoff, int a_glu,
-                                                              const LinArgs p) {
-    gemv_body<MR, U, KIND, SPLIT, INDIRECT>(GemvAt{A, B, K, N, ldb, lda, a_zoff, b_zoff, a_glu}, p, blockIdx.z, NormIn());
+template <int MR, int U, int KIND, bool SPLIT, bool INDIRECT, int NR>
+__global__ __launch_bounds__(256) void lm_gemv_at_once_kernel(const float* A, const bf16_t* B, const float* a_poly, int K, int N, int ldb, int lda, int a_zoff,
+                                                              int b_zoff, int a_glu, float poly_eps, const LinArgs p) {
+    gemv_body<MR, U, KIND, SPLIT, INDIRECT, NR>(GemvAt{A, B, K, N, ldb, lda, a_zoff, b_zoff, a_glu, nullptr, poly_eps, a_poly}, p, blockIdx.z, NormIn());
 }
-template <int U>
+template <int U, int NR>
 __global__ __launch_bounds__(256) void lm_gemv_normed_kernel(const float* x, const float* y, const float* wb, const float* wn, const bf16_t* B, int K, int N, int ldb,
                                                              float eps, float* x_out, const LinArgs p) {
-    gemv_body<1, U, GEMV_NORM, false, false>(GemvAt{nullptr, B, K, N, ldb, 0, 0, 0, 0}, p, 0, NormIn{x, y, wb, wn, x_out, eps});
+    gemv_body<1, U, GEMV_NORM, false, false, NR>(GemvAt{nullptr, B, K, N, ldb, 0, 0, 0, 0}, p, 0, NormIn{x, y, wb, wn, x_out, eps});
 }
-template <int MR, int U, bool SPLIT>
+template <int MR, int U, bool SPLIT, int NR>
 __global__ __launch_bounds__(256) void lm_gemv_row_norm_kernel(const float* A, const bf16_t* B, const float* a_norm, int K, int N, int ldb, int lda, float eps, const LinArgs p,
                                                                const TailArgs tail) {
     if (blockIdx.y > 0) return move_tails(tail);
-    gemv_body<MR, U, GEMV_RMS, SPLIT, false>(GemvAt{A, B, K, N, ldb, lda, 0, 0, 0, a_norm, eps}, p, 0, NormIn());
+    gemv_body<MR, U, GEMV_RMS, SPLIT, false, NR>(GemvAt{A, B, K, N, ldb, lda, 0, 0, 0, a_norm, eps}, p, 0, NormIn());
 }
 // batches [0, za) are product a's, the rest product b's
 template <int U, int KIND>
@@ -274,16 +315,22 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     if (B && (split || A.M != 1)) return ZG_OK;
     const int share = split ? (((k_max + 3) / 4) + 7) & ~7 : k_max, pieces = (share + 511) / 512;
     if (pieces > (norm ? 2 : 3)) return ZG_OK;
-    const int rows = split ? 2 : 8;
-    const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, A.a_norm && A.tail ? 2 : 1, A.nz + (B ? B->nz : 0));
     const bool indirect = A.z_group || A.a_rows || A.a_div != 1;
+    // Where every wave prepares the row for itself, four weight rows share a preparation once two would be more workgroups than compute units (some
+    // then have two, each with the row's reads and arithmetic; up to there more waves are ahead).  One row, us a launch, four rows : two, 768 ->
+    // 3072 behind the two norms 3.68 : 4.24, 768 -> 1680 2.88 : 3.92, 1536 -> 768 behind its own 2.80 : 2.96.  Without a preparation two: 768 ->
+    // 3072 2.96 : 2.76, 768 -> 2304 2.84 : 2.76, 3072 -> 768 3.04 : 2.92, 768 -> 50264 12.3 : 12.0.
+    const bool four = !B && !indirect && A.nz == 1 && (kind == GEMV_NORM || kind == GEMV_RMS || kind == GEMV_POLY) && A.N > 256 * (split ? 2 : 8);
+    const int rows = (split ? 1 : 4) * (four ? 4 : 2);
+    const dim3 grid((std::max(A.N, B ? B->N : 0) + rows - 1) / rows, A.a_norm && A.tail ? 2 : 1, A.nz + (B ? B->nz : 0));
 #define ZG_GV(MR, U, KIND, SPLIT)                                                                                                                   \
     do {                                                                                                                                            \
-        if (indirect) ZG_GV_I(MR, U, KIND, SPLIT, true);                                                                                            \
-        else ZG_GV_I(MR, U, KIND, SPLIT, false);                                                                                                    \
+        if (indirect) ZG_GV_I(MR, U, KIND, SPLIT, true, 2);                                                                                         \
+        else if (four) ZG_GV_I(MR, U, KIND, SPLIT, false, (KIND == GEMV_POLY ? 4 : 2));                                                             \
+        else ZG_GV_I(MR, U, KIND, SPLIT, false, 2);                                                                                                 \
     } while (0)
-#define ZG_GV_I(MR, U, KIND, SPLIT, IND)                                                                                                            \
-    lm_gemv_at_once_kernel<MR, U, KIND, SPLIT, IND><<<grid, 256, 0, s>>>(a.A, a.B, a.K, a.N, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_glu, a)
+#define ZG_GV_I(MR, U, KIND, SPLIT, IND, NR)                                                                                                        \
+    lm_gemv_at_once_kernel<MR, U, KIND, SPLIT, IND, NR><<<grid, 256, 0, s>>>(a.A, a.B, a.a_poly, a.K, a.N, a.ldb, a.lda, (int)a.a_zoff, (int)a.b_zoff, a.a_glu, a.poly_eps, a)
 #define ZG_GV_P(KIND)                                                                              \
     do {                                                                                           \
         if (pieces == 1) lm_gemv_at_once_pair_kernel<1, KIND><<<grid, 256, 0, s>>>(a, b, A.nz);      \
@@ -304,14 +351,22 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
     if (B && kind == GEMV_GLU) ZG_GV_P(GEMV_GLU);
     else if (B) ZG_GV_P(GEMV_PLAIN);
     else if (norm) {
-        if (pieces == 1) lm_gemv_normed_kernel<1><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
-        else lm_gemv_normed_kernel<2><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a);
+#define ZG_GV_N(U, NR) lm_gemv_normed_kernel<U, NR><<<grid, 256, 0, s>>>(norm->x, norm->y, norm->wb, norm->wn, a.B, a.K, a.N, a.ldb, norm->eps, norm->x_out, a)
+        if (pieces == 1 && four) ZG_GV_N(1, 4);
+        else if (pieces == 1) ZG_GV_N(1, 2);
+        else if (four) ZG_GV_N(2, 4);
+        else ZG_GV_N(2, 2);
+#undef ZG_GV_N
     } else if (kind == GEMV_RMS) {
-#define ZG_GV_R(MR, U)                                                                                                                                      \
-    do {                                                                                                                                                    \
-        if (split) lm_gemv_row_norm_kernel<MR, U, true><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a, tail_args(A));                    \
-        else lm_gemv_row_norm_kernel<MR, U, false><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a, tail_args(A));                         \
+#define ZG_GV_R(MR, U)                               \
+    do {                                             \
+        if (split && four) ZG_GV_RN(MR, U, true, 4); \
+        else if (split) ZG_GV_RN(MR, U, true, 2);    \
+        else if (four) ZG_GV_RN(MR, U, false, 4);    \
+        else ZG_GV_RN(MR, U, false, 2);              \
     } while (0)
+#define ZG_GV_RN(MR, U, SPLIT, NR) \
+    lm_gemv_row_norm_kernel<MR, U, SPLIT, NR><<<grid, 256, 0, s>>>(a.A, a.B, a.a_norm, a.K, a.N, a.ldb, a.lda, a.norm_eps, a, tail_args(A))
 #define ZG_GV_RU(MR)                     \
     do {                                 \
         if (pieces == 1) ZG_GV_R(MR, 1); \
@@ -321,6 +376,7 @@ int launch_gemv_at_once(const Linear& A, const Linear* B, const NormIn* norm, hi
         if (A.M == 1) ZG_GV_RU(1);
         else ZG_GV_RU(2);
 #undef ZG_GV_R
+#undef ZG_GV_RN
 #undef ZG_GV_RU
     } else if (kind == GEMV_POLY) ZG_GV_M(GEMV_POLY, true);
     else if (kind == GEMV_GLU && split) ZG_GV_M(GEMV_GLU, true);
