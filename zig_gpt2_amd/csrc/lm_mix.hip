@@ -7,6 +7,7 @@
 #include <algorithm>
 
 #include "lm_latent_parts.h"
+#include "lm_quotient.h"
 
 namespace zg {
 namespace lm {
@@ -1266,13 +1267,13 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     const float L = lsum + __shfl_xor(lsum, 32, 64);
     if (ctx16) {  // (KR is a multiple of 8)
         // A lane has a query's values: turned in the tiles' place, half of the dimensions at a time, they leave as 16-byte pieces of whole rows.
-        // (8 bytes a lane to 32 rows, divided one by one: 6.1 us behind the last tile, 2.0 so)
+        // (8 bytes a lane to 32 rows, divided one by one: 6.1 us behind the last tile, 2.0 so.)  The quotients are those of a division.
         constexpr int P = NT * 16, PITCH = P * 2 + 16;
         static_assert(32 * PITCH <= T::BYTES / 2, "a wave's rows fit its half of a tile's place");
         char* const img = &Ks[0][0] + wave * (T::BYTES / 2);
         const size_t row = (size_t)(m_first + min(r, nq - 1));
-        const float gf = head_gate_f(gate, ldg, row, h);
-        const float by = sink ? gf * sink_norm_f(mx * 0.69314718055994531f, L, sink, h) : gf / L;
+        const float gf = head_gate_f(gate, ldg, row, h) * (sink ? sink_norm_f(mx * 0.69314718055994531f, L, sink, h) : 1.0f), inv = 1.0f / L;
+        auto value = [&](float v) { return (sink ? v : quotient(v, L, inv)) * gf; };
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -1280,7 +1281,7 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
 #pragma unroll
                 for (int i = 0; i < 16; i += 4) {
                     const f32x16& v = o[half * (NT / 2) + t];
-                    *reinterpret_cast<u32x2*>(img + r * PITCH + (t * 32 + 8 * (i >> 2) + 4 * hf) * 2) = u32x2{cvt_pk_bf16(v[i] * by, v[i + 1] * by), cvt_pk_bf16(v[i + 2] * by, v[i + 3] * by)};
+                    *reinterpret_cast<u32x2*>(img + r * PITCH + (t * 32 + 8 * (i >> 2) + 4 * hf) * 2) = u32x2{cvt_pk_bf16(value(v[i]), value(v[i + 1])), cvt_pk_bf16(value(v[i + 2]), value(v[i + 3]))};
                 }
             // (a wave's accesses to the LDS are in order)
 #pragma unroll
