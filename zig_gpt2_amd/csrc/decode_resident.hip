@@ -174,7 +174,6 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
     const int k = __builtin_amdgcn_readfirstlane((int)xcc), r = __builtin_amdgcn_readfirstlane((int)s_rank);
     const int H = a.n_heads;
     const int nh = k < H ? (H - k + kXcds - 1) / kXcds : 0;       // heads of this XCD: k, k + 8, ...
-    const int nx = H < kXcds ? H : kXcds;                         // XCDs with heads
     const int G = nh > 0 ? kRanks / nh : kRanks;                  // workgroups of a head
     const int hi = min(r / G, NH - 1), sp = r % G;                // this workgroup's head and 64 positions
     const int head = (k < H ? k : 0) + kXcds * (hi < nh ? hi : 0);
@@ -391,7 +390,6 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
     }
 
     // ================================================================================================ rows and words
-    const int rowC = r * CPR + 2 * wave + half;                   // also the row of E
     const int colC = l32 * CC;                                    // column among the XCD's
     const int owner = tid < 8 * CPR ? tid >> 3 : -1;              // column of this workgroup a thread helps to add up
     const int ocol = r * CPR + (owner < 0 ? 0 : owner);
@@ -557,8 +555,10 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                     barrier();  // B4a
                     if (tid < CPR) put_far(far1, (k * kRanks + r) * kFar + tid, tagged(tag, s_out[tid]));
                 }
+            } else if constexpr (NW < kFar1From) {  // far2 has been read here (decode_resident_order.h)
+                if (tid < CPR) put_far(far1, (k * kRanks + r) * kFar + tid, tagged(tag, 0.0f));
             }
-            add_up(far1, nx, v_small + 64, P::x1, tag);
+            add_up(far1, kFar1From, v_small + 64, P::x1, tag);
             x = w.get(near, P::x1 + tid, tag);
             // ---- D
             spread(1, x, x * vec(R::uG * 256 + tid));  // B5

@@ -143,7 +143,6 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
     const int k = __builtin_amdgcn_readfirstlane((int)xcc), r = __builtin_amdgcn_readfirstlane((int)s_rank);
     const int H = a.n_heads, M = a.batch;
     const int nh = k < H ? (H - k + kXcds - 1) / kXcds : 0;       // heads of this XCD: k, k + 8, ...
-    const int nx = H < kXcds ? H : kXcds;                         // XCDs with heads
     const int pairs = nh * M;                                     // (head, sequence)
     const int G = pairs > 0 ? min(kRanks / pairs, kMostSplits) : 1;  // workgroups of a pair
     const int my = r / G, sp = r % G;                             // this workgroup's
@@ -839,12 +838,14 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                 }
             } else {
                 barrier();  // B1 (the helpers' fetches of vectors take the place of the Block's in front)
+                if constexpr (NW < kFar1From)  // far2 has been read here (decode_resident_order.h)
+                    if (tid < CPR * 8) put_far(far1, (unsigned)((k * kRanks + r) * P::block + tid), tagged(tag, 0.0f));
             }
             unsigned to_x = fresh(P::x1 + (unsigned)x_at(ocol(), om()));
             float bias = s_vec[vp][64 + min(oc(), 31)], gain = s_vec[vp][160 + min(oc(), 31)];
-            gather(far1, nx, tag);
+            gather(far1, kFar1From, tag);
             barrier();  // B4b
-            add_up(nx, bias);
+            add_up(kFar1From, bias);
             put_x(to_x, P::st1, tag, gain);
             barrier();  // B5
             // ---- D

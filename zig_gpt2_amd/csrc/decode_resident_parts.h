@@ -1,12 +1,12 @@
 // decode_resident_parts.h — what the resident decode kernels share (decode_resident.hip: one sequence, decode_resident_batch.hip: two to eight in lock step)
 #pragma once
+#include "decode_resident_order.h"
 #include "zg_common.h"
 #include "zg_kernels.h"
 
 namespace zg {
 namespace resident {
 
-constexpr int kXcds = 8, kRanks = 32;
 constexpr float kNone = -1e30f;  // score of a position that is not there
 
 typedef unsigned long long u64;
