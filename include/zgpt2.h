@@ -313,7 +313,11 @@ int zg_gpt_generate_greedy(zg_gpt* g, const size_t* prompts, size_t prompt_strid
                            const size_t* prompt_lens, size_t n_steps, size_t* out_tokens,
                            size_t out_len);
 /* Asynchronous form used by the benchmark: enqueue the same n_steps on the stream and return;
- * results stay on the device until zg_gpt_generate_fetch. */
+ * results stay on the device until zg_gpt_generate_fetch.  The stream's end is the generation's end: an event behind the call says that all
+ * steps have run, also where a resident launch (one launch of up to 64 steps that needs all compute units at once: one
+ * sequence, or two to eight with bf16 weights, of widths 384, 512 and 768 on the library's stream) did not get them in time and the steps ran
+ * another way.  While a resident launch runs, up to 12 ms, other streams have what it leaves of every compute unit: work whose workgroups
+ * need more LDS than some 10 KB waits for its end (ZGPT2_RESIDENT=0 at creation: launches of a few microseconds each instead). */
 int zg_gpt_generate_enqueue(zg_gpt* g, const size_t* prompts, size_t prompt_stride,
                             const size_t* prompt_lens, size_t n_steps);
 int zg_gpt_generate_fetch(zg_gpt* g, size_t n_steps, size_t* out_tokens, size_t out_len);
@@ -591,6 +595,12 @@ int zg_gpt_time_kernel(zg_gpt* g, int which_and_options, int iters, float* avg_u
  *       boundary + event overhead contained in every interval above.
  * Intervals are event-to-event, so each includes the boundary to the next kernel. */
 int zg_gpt_profile_step(zg_gpt* g, size_t seq_len, int iters, float* us_out, size_t n_out);
+
+/* Diagnostic: the resident decode kernels of this handle (waits for the stream).  out[0] = 1 when greedy generations may go to them,
+ * out[1] = 1 when the last generation did, out[2] the steps since the handle was made that other kernels kept from them (they held compute
+ * units for too long) and that ran on the workgroups that were to be had instead, out[3] how many these were the last time.  n_out >= 4.  No
+ * reference counterpart. */
+int zg_debug_resident_stats(zg_gpt* g, unsigned* out, size_t n_out);
 
 /* Diagnostic: how the side-stream prefetcher of the last zg_gpt_generate_* call ended (waits for both streams).
  * out[0] = 1 when the handle has a prefetcher (2: it found no concurrency with the decode stream once and is no longer

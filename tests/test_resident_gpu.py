@@ -121,22 +121,53 @@ def test_nan_logits_pick_index_zero(zg, monkeypatch, batch):
 
 @pytest.mark.parametrize("batch", [1, 2])
 def test_withdrawn_launch_runs_on_the_chain(zg, monkeypatch, batch):
-    """No patience at the start: every workgroup leaves before it has touched anything, and the launch chain makes up for it, also
-    where another call than the fetch asks first.  The handle then stays on the chain for some generations."""
+    """No patience at the start: every workgroup leaves before it has touched anything, and the steps run on what workgroups there are, in
+    front of the end of the stream.  The handle then stays on the chain for some generations."""
     cfg = SHAPES["768"]
     w = synth.make_weights(cfg, seed=34, bf16=True)
     p = [synth.rand_tokens(341 + b, 5, cfg.vocab_size) for b in range(batch)]
     chain = make(monkeypatch, cfg, w, False, batch=batch)
     want = chain.generate(p, 150)
     hid = chain.hidden()
-    monkeypatch.setenv("ZGPT2_RESIDENT_START", "0")
+    monkeypatch.setenv("ZGPT2_RESIDENT_WITHDRAW", "0")
     m = make(monkeypatch, cfg, w, True, batch=batch)
     assert np.array_equal(m.generate(p, 150), want)
+    assert m.resident_stats()["ran"]
     for _ in range(8):
         assert np.array_equal(m.generate(p, 150), want)
+        assert not m.resident_stats()["ran"]
     m.generate_enqueue(p, 150)  # tried again, withdrawn again
     assert rel(m.hidden(), hid) < 2e-6
     assert np.array_equal(m.generate_fetch(150), want)
+    m.close()
+    chain.close()
+
+
+@pytest.mark.parametrize("name,batch,f32", [("384", 1, False), ("512", 1, True), ("768-odd", 1, False), ("768", 1, True), ("384", 8, False), ("768", 3, False)])
+@pytest.mark.parametrize("launch", [0, 1, 2])
+def test_launch_withdrawn_behind_others(zg, monkeypatch, name, batch, f32, launch):
+    """The first, second or third launch of a generation withdraws, its followers leave, and the steps that are missing have run when
+    the stream has: no call makes up for them.  Tokens, residual stream, pick, logits and cache are the chain's."""
+    import torch
+
+    c = SHAPES[name]
+    cfg = synth.GPTConfig(c.vocab_size, 215, c.n_layer, c.n_heads, c.n_embed)
+    w = synth.make_weights(cfg, seed=39, bf16=not f32)
+    p = [synth.rand_tokens(390 + b, 2 + (3 * b) % 7, cfg.vocab_size) for b in range(batch)]  # ragged; no prompt pass
+    steps = 210  # four launches
+    chain = make(monkeypatch, cfg, w, False, batch=batch, weights_f32=f32)
+    want = chain.generate(p, steps)
+    monkeypatch.setenv("ZGPT2_RESIDENT_WITHDRAW", str(launch))
+    m = make(monkeypatch, cfg, w, True, batch=batch, weights_f32=f32)
+    m.generate_enqueue(p, steps)
+    torch.cuda.synchronize()
+    st = m.resident_stats()
+    assert st["ran"] and st["rest_steps"] == steps - 64 * launch and st["rest_workgroups"] >= 1, st
+    assert np.array_equal(m.generate_fetch(steps), want)
+    assert rel(m.hidden(), chain.hidden()) < 2e-6
+    assert np.array_equal(m.argmax(), chain.argmax())
+    tok = want[:, -1]
+    assert rel(m.forward(steps + 1, tok), chain.forward(steps + 1, tok)) < 2e-6
     m.close()
     chain.close()
 

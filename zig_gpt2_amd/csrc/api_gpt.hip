@@ -124,23 +124,21 @@ struct zg_gpt {
     // greedy decode of one sequence as a resident kernel (decode_resident.hip)
     bool res_on;                     // the handle's shape takes it
     bool res_gen;                    // the generation in flight does
-    bool res_pending;                // resident launches are enqueued that no call has looked at yet (settle)
-    int res_strikes, res_sit_out;    // launches withdrawn so far (the third is final); generations left on the launch chain
+    int res_strikes, res_sit_out;    // generations with a withdrawn launch so far (the third is final); generations left on the launch chain
+    size_t res_launch;               // launches of the generation in flight
     unsigned res_tag;                // first unused tag
     unsigned res_start_limit;        // polls before a launch that is not resident as a whole is withdrawn
+    int res_none_at;                 // test: this launch of a generation has none (-1: all have res_start_limit)
     unsigned long long* res_words;
     size_t res_words_bytes;
     ResidentCtl* res_ctl;
+    float* rest_best;                // decode_rest_kernel's picks by workgroup
     unsigned* res_withdrawn;         // pinned
-    hipStream_t res_stream;          // where the pending launches are
     // a generation in flight between gen_begin and gen_end (zg_gpt_generate_enqueue / _many)
     size_t gen_pos, gen_n, gen_min_prompt, gen_since_sync;
     bool gen_open;
 };
 
-extern "C" {
-static int settle(zg_gpt* g);
-}
 static inline hipStream_t gs(const zg_gpt* g) { return g->stream ? g->stream : ctx().stream; }
 static inline zg_gpt* root(zg_gpt* g) { return g->parent ? g->parent : g; }
 
@@ -241,6 +239,7 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
     g->res_words_bytes = resident_words(E, B) * 8;
     g->res_words = (unsigned long long*)P(g->res_words_bytes);
     g->res_ctl = (ResidentCtl*)P(sizeof(ResidentCtl));
+    g->rest_best = (float*)P(g->res_words_bytes != 0 ? decode_rest_floats() * 4 : 0);
     g->pf_njobs = (int)(2 + 5 * L);
     g->pf_ctl = (PfCtl*)P(sizeof(PfCtl));
     g->pf_jobs = (PfJob*)P((size_t)g->pf_njobs * sizeof(PfJob));
@@ -644,6 +643,7 @@ int check_fault(zg_gpt* g) {
         volatile unsigned* f = g->fault;
         tag = *f;
         if (tag) *f = 0;
+        if (tag) g->res_tag = 0xffffffffu;  // (words that were not written keep old tags: all are cleared in front of the next launch)
     }
     if (sk) {
         set_error("a half-tile hand-over of the whole-prompt c_attn GEMM timed out%s: results discarded", tag ? " (and a tagged hand-over of the decode step)" : "");
@@ -766,30 +766,62 @@ int pf_stop(zg_gpt* g, hipStream_t s) {
 }
 
 // The resident kernels take greedy generations of one sequence, or of two to eight with bf16 weights, on the library's stream: shapes
-// they are built for, fp32 cache, all 256 compute units.  A handle with a private stream is one of several chains on the chip, and borrowed weights may be reloaded by
-// their owner before a withdrawn launch is made up for: both keep the launch chain.
+// they are built for, fp32 cache, all 256 compute units.  Handles with a private stream or borrowed weights are one of several chains on the
+// chip: they keep the launch chain.
 void setup_resident(zg_gpt* g) {
-    g->res_on = g->res_gen = g->res_pending = false;
+    g->res_on = g->res_gen = false;
     g->res_strikes = g->res_sit_out = 0;
     g->res_tag = 1;
-    g->res_stream = nullptr;
     g->res_withdrawn = reinterpret_cast<unsigned*>(reinterpret_cast<char*>(g->h_ctrl) + 264);
     *g->res_withdrawn = 0;
-    g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms (0: the test of a withdrawn launch)
+    g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms
+    g->res_none_at = env_int("ZGPT2_RESIDENT_WITHDRAW", -1);
     if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
     if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer) || !env_int("ZGPT2_RESIDENT", 1)) return;
     int cus = 0;
     g->res_on = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx().device) == hipSuccess && cus == 256;
 }
 
-// Whether the generation about to start goes to the resident kernel
+// Whether the generation about to start goes to the resident kernel.  Where a launch of an earlier one was withdrawn (other kernels held compute
+// units for longer than it waits) the handle stays on the launch chain for some generations.
 bool resident_takes(zg_gpt* g, bool sampled, hipStream_t s) {
+    volatile unsigned* w = g->res_withdrawn;
+    if (*w != 0) {
+        *w = 0;
+        ++g->res_strikes;
+        g->res_sit_out = 8;
+        g->res_tag = 0xffffffffu;  // (what was not written keeps an old tag: all words are cleared in front of the next launch)
+    }
     if (!g->res_on || sampled || s == nullptr || g->n_children != 0 || g->res_strikes >= 3) return false;
     if (g->res_sit_out > 0) {
         --g->res_sit_out;
         return false;
     }
     return true;
+}
+
+ResidentArgs resident_args(zg_gpt* g, size_t s0, size_t s1) {
+    const size_t L = g->cfg.n_layer;
+    const zg_layer &y = g->layers[0], &y1 = g->layers[L > 1 ? 1 : 0];
+    ResidentArgs a{};
+    a.c_attn_w = y.c_attn_w; a.c_proj_w = y.c_proj_w; a.c_fc_w = y.c_fc_w; a.mlp_proj_w = y.mlp_proj_w;
+    a.ln_1_g = y.ln_1_g; a.c_attn_c2 = y.c_attn_c2; a.c_attn_c3 = y.c_attn_c3; a.c_proj_b = y.c_proj_b;
+    a.ln_2_g = y.ln_2_g; a.c_fc_c2 = y.c_fc_c2; a.c_fc_c3 = y.c_fc_c3; a.mlp_proj_b = y.mlp_proj_b;
+    a.w_stride = (size_t)(reinterpret_cast<char*>(y1.c_attn_w) - reinterpret_cast<char*>(y.c_attn_w));
+    a.kv_stride = (size_t)(reinterpret_cast<char*>(y1.k_cache) - reinterpret_cast<char*>(y.k_cache));
+    a.k_cache = reinterpret_cast<char*>(y.k_cache);
+    a.v_cache = reinterpret_cast<char*>(y.v_cache);
+    a.wte = g->wte; a.wpe = g->wpe; a.ln_f_g = g->ln_f_g; a.ln_f_b = g->ln_f_b;
+    a.n_layer = (int)L; a.n_heads = (int)g->cfg.n_heads; a.ctx = (int)g->cfg.context_size; a.vocab = (int)g->cfg.vocab_size;
+    a.batch = (int)g->batch; a.prompt_len = g->prompt_len; a.out_stride = (int)g->cfg.context_size; a.lm_c2 = g->lm_c2; a.lm_c3 = g->lm_c3;
+    a.n_prompt = (int)g->gen_min_prompt; a.s0 = (int)s0; a.s1 = (int)s1;
+    a.prompt = g->prompt; a.out_tokens = g->out_tokens; a.cur_token = g->cur_token;
+    a.ctrl = g->ctrl; a.x = g->x; a.logits = g->logits; a.part_val = g->part_val; a.part_idx = g->part_idx; a.n_part = g->lm_grid;
+    a.words = g->res_words; a.ctl = g->res_ctl; a.tag0 = g->res_tag;
+    a.spin_limit = g->spin_limit;
+    a.start_limit = g->res_none_at == (int)g->res_launch ? 0u : g->res_start_limit;
+    a.fault = g->fault; a.withdrawn = g->res_withdrawn;
+    return a;
 }
 
 // One launch: up to kResidentSteps steps from gen_pos on.  Other streams' kernels get the chip between launches.
@@ -803,30 +835,17 @@ int enqueue_resident(zg_gpt* g, hipStream_t s) {
         g->res_tag = 1;
     }
     ZG_HIP(hipMemsetAsync(g->res_ctl->reg, 0, sizeof(ResidentCtl) - offsetof(ResidentCtl, reg), s));
-    const zg_layer &y = g->layers[0], &y1 = g->layers[L > 1 ? 1 : 0];
-    ResidentArgs a{};
-    a.c_attn_w = y.c_attn_w; a.c_proj_w = y.c_proj_w; a.c_fc_w = y.c_fc_w; a.mlp_proj_w = y.mlp_proj_w;
-    a.ln_1_g = y.ln_1_g; a.c_attn_c2 = y.c_attn_c2; a.c_attn_c3 = y.c_attn_c3; a.c_proj_b = y.c_proj_b;
-    a.ln_2_g = y.ln_2_g; a.c_fc_c2 = y.c_fc_c2; a.c_fc_c3 = y.c_fc_c3; a.mlp_proj_b = y.mlp_proj_b;
-    a.w_stride = (size_t)(reinterpret_cast<char*>(y1.c_attn_w) - reinterpret_cast<char*>(y.c_attn_w));
-    a.kv_stride = (size_t)(reinterpret_cast<char*>(y1.k_cache) - reinterpret_cast<char*>(y.k_cache));
-    a.k_cache = reinterpret_cast<char*>(y.k_cache);
-    a.v_cache = reinterpret_cast<char*>(y.v_cache);
-    a.wte = g->wte; a.wpe = g->wpe; a.ln_f_g = g->ln_f_g; a.ln_f_b = g->ln_f_b;
-    a.n_layer = (int)L; a.n_heads = (int)g->cfg.n_heads; a.ctx = (int)g->cfg.context_size; a.vocab = (int)g->cfg.vocab_size;
-    a.batch = (int)g->batch; a.prompt_len = g->prompt_len; a.out_stride = (int)g->cfg.context_size; a.lm_c2 = g->lm_c2; a.lm_c3 = g->lm_c3;
-    a.n_prompt = (int)g->gen_min_prompt; a.s0 = (int)st; a.s1 = (int)(st + n);
-    a.prompt = g->prompt; a.out_tokens = g->out_tokens; a.cur_token = g->cur_token;
-    a.ctrl = g->ctrl; a.x = g->x; a.logits = g->logits; a.part_val = g->part_val; a.part_idx = g->part_idx; a.n_part = g->lm_grid;
-    a.words = g->res_words; a.ctl = g->res_ctl; a.tag0 = g->res_tag;
-    a.spin_limit = g->spin_limit; a.start_limit = g->res_start_limit;
-    a.fault = g->fault; a.withdrawn = g->res_withdrawn;
-    ZG_TRY(launch_decode_resident(a, (int)g->cfg.n_embed, g->wt, s));
+    ZG_TRY(launch_decode_resident(resident_args(g, st, st + n), (int)g->cfg.n_embed, g->wt, s));
     g->res_tag += tags;
-    g->res_pending = true;
-    g->res_stream = s;
+    ++g->res_launch;
     g->gen_pos = st + n;
     return ZG_OK;
+}
+
+// Behind the last resident launch: the steps that withdrawn launches left
+int enqueue_rest(zg_gpt* g, hipStream_t s) {
+    const RestArgs a{resident_args(g, 0, g->gen_n), (int)g->cfg.n_embed, g->q, g->part, g->h4, g->rest_best, reinterpret_cast<int*>(g->rest_best + decode_rest_floats() / 2)};
+    return launch_decode_rest(a, g->wt, s);
 }
 
 size_t prefill_min() { return 4; }  // shorter prompts go through the decode chain (measured: the whole-prompt pass pays from 4 tokens up)
@@ -1136,7 +1155,6 @@ int zg_gpt_destroy(zg_gpt* g) {
     if (!g) return ZG_OK;
     ZG_REQUIRE(g->n_children == 0, ZG_ERR_ARG, "zg_gpt_destroy: %d handle(s) still borrow this one's weights (destroy them first)", g->n_children);
     (void)hipStreamSynchronize(gs(g));
-    if (g->res_pending) (void)hipStreamSynchronize(g->res_stream);
     drop_prefetcher(g);
     drop_graphs(g);
     if (g->stream) (void)hipStreamDestroy(g->stream);
@@ -1159,7 +1177,6 @@ int zg_gpt_load_block_tensor(zg_gpt* g, size_t layer, int slot, const float* src
     ZG_TRY(require_init());
     ZG_REQUIRE(g && src && layer < g->cfg.n_layer, ZG_ERR_ARG, "load_block_tensor: bad argument");
     ZG_REQUIRE(g->parent == nullptr, ZG_ERR_ARG, "load_block_tensor: this handle borrows its weights (load them into their owner)");
-    ZG_TRY(settle(g));
     const size_t E = g->cfg.n_embed;
     zg_layer& y = g->layers[layer];
     void* dst = nullptr;
@@ -1197,7 +1214,6 @@ int zg_gpt_load_tensor(zg_gpt* g, int slot, const float* src, size_t len) {
     ZG_TRY(require_init());
     ZG_REQUIRE(g && src, ZG_ERR_ARG, "load_tensor: bad argument");
     ZG_REQUIRE(g->parent == nullptr, ZG_ERR_ARG, "load_tensor: this handle borrows its weights (load them into their owner)");
-    ZG_TRY(settle(g));
     const size_t E = g->cfg.n_embed;
     void* dst = nullptr;
     size_t n = 0;
@@ -1216,7 +1232,6 @@ int zg_gpt_load_tensor(zg_gpt* g, int slot, const float* src, size_t len) {
 
 int zg_gpt_weight_arena(zg_gpt* g, void** device_ptr, size_t* bytes) {
     ZG_REQUIRE(g && device_ptr && bytes, ZG_ERR_ARG, "weight_arena: null argument");
-    ZG_TRY(settle(g));
     // The folded-LayerNorm vectors (c2 / c3) live inside the region handed out here.  A sender has to hold valid
     // ones before its bytes are copied, and a receiver must re-derive them from whatever lands in the region — also a
     // receiver that has run before (its flag would still say "folded").  So: fold now if needed (sender side: a few
@@ -1303,7 +1318,6 @@ static int forward_enqueue(zg_gpt* g, size_t seq_len, const size_t* tokens, size
     const size_t V = g->cfg.vocab_size;
     ZG_REQUIRE(!logits_out || (compute_logits && logits_len >= g->batch * V), ZG_ERR_SHAPE,
                "gpt_forward: logits_out needs compute_logits and %zu elements", g->batch * V);
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     for (size_t b = 0; b < g->batch; ++b) {
         ZG_REQUIRE(tokens[b] < V, ZG_ERR_SHAPE, "gpt_forward: token %zu >= vocab %zu", tokens[b], V);
@@ -1344,7 +1358,6 @@ int zg_gpt_prefill(zg_gpt* g, const size_t* tokens, size_t token_stride, size_t 
                "gpt_prefill: n_tokens %zu outside 1..%zu (stride %zu)", n_tokens, C, token_stride);
     ZG_REQUIRE(!logits_out || (compute_logits && logits_len >= B * V), ZG_ERR_SHAPE,
                "gpt_prefill: logits_out needs compute_logits and %zu elements", B * V);
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     ZG_HIP(hipStreamSynchronize(s));
     for (size_t b = 0; b < B; ++b)
@@ -1377,7 +1390,6 @@ int zg_gpt_prefill(zg_gpt* g, const size_t* tokens, size_t token_stride, size_t 
 int zg_gpt_argmax(zg_gpt* g, size_t* tokens_out, size_t n_tokens) {
     ZG_TRY(require_init());
     ZG_REQUIRE(g && tokens_out && n_tokens == g->batch, ZG_ERR_ARG, "gpt_argmax: bad argument");
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     ZG_TRY(launch_embed_step(embed_args(g, 2), s));
     ZG_HIP(hipMemcpyAsync(g->h_ints, g->cur_token, g->batch * sizeof(int), hipMemcpyDeviceToHost, s));
@@ -1426,7 +1438,6 @@ int zg_gpt_sample(zg_gpt* g, size_t seq_len, const size_t* tokens, size_t n_toke
 int zg_gpt_hidden(zg_gpt* g, float* x_out, size_t len) {
     ZG_TRY(require_init());
     ZG_REQUIRE(g && x_out && len >= g->batch * g->cfg.n_embed, ZG_ERR_ARG, "gpt_hidden: bad argument");
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     ZG_HIP(hipMemcpyAsync(x_out, g->x, g->batch * g->cfg.n_embed * sizeof(float),
                           is_device_ptr(x_out) ? hipMemcpyDeviceToDevice : hipMemcpyDeviceToHost, s));
@@ -1436,13 +1447,12 @@ int zg_gpt_hidden(zg_gpt* g, float* x_out, size_t len) {
 
 // A generation in three parts, so that several handles' generations can be fed to their streams turn by turn
 // (zg_gpt_generate_enqueue_many): gen_begin — prompts, cache clearing, the whole-prompt pass, the prefetcher's start;
-// gen_pump — ONE graph launch (graph_steps decode steps) or one single step, false when nothing is left; gen_end — the
-// prefetcher's stop word and the record of the last pick.  After a successful gen_begin, gen_end must run (also on failure:
+// gen_pump — ONE graph launch (graph_steps decode steps), one resident launch or one single step, false when nothing is left; gen_end — the
+// prefetcher's stop word and the record of the last pick, or the steps that resident launches left.  After a successful gen_begin, gen_end must run (also on failure:
 // the prefetcher must not wait for steps that never come).
 static int gen_begin(zg_gpt* g, const size_t* prompts, size_t prompt_stride, const size_t* prompt_lens, size_t n_steps, bool sampled = false,
                      float temp = 1.0f, uint64_t seed = 0) {
     ZG_REQUIRE(g && prompts && prompt_lens, ZG_ERR_ARG, "generate: null argument");
-    ZG_TRY(settle(g));
     const size_t C = g->cfg.context_size, V = g->cfg.vocab_size, B = g->batch;
     ZG_REQUIRE(n_steps >= 1 && n_steps <= C, ZG_ERR_SHAPE, "generate: n_steps %zu outside 1..%zu", n_steps, C);
     hipStream_t s = gs(g);
@@ -1492,6 +1502,7 @@ static int gen_begin(zg_gpt* g, const size_t* prompts, size_t prompt_stride, con
     else ZG_TRY(pf_start(g, n_steps, s));
     g->gen_pos = first;
     g->gen_n = n_steps;
+    g->res_launch = 0;
     g->gen_min_prompt = min_prompt;
     g->gen_since_sync = 0;
     g->gen_open = true;
@@ -1540,37 +1551,9 @@ static int gen_end(zg_gpt* g, int rs) {
     g->gen_open = false;
     if (!g->res_gen) ZG_TRY(pf_stop(g, s));  // also after a failed launch: the prefetcher must not wait for steps that never come
     ZG_TRY(rs);
-    ZG_TRY(launch_embed_step(embed_args(g, 1), s));  // record the pick of the last step
+    if (g->res_gen) ZG_TRY(enqueue_rest(g, s));
+    else ZG_TRY(launch_embed_step(embed_args(g, 1), s));  // record the pick of the last step (the resident kernels do)
     g->steps_enqueued = g->gen_n;
-    return ZG_OK;
-}
-
-// Every call that reads or changes what a generation leaves looks here first: were its resident launches withdrawn (other kernels
-// held compute units for longer than they wait)?  The steps that are missing then run on the launch chain, from where the last
-// finished launch left the sequence; the handle stays on the chain for some generations.
-static int settle(zg_gpt* g) {
-    if (!g->res_pending) return ZG_OK;
-    ZG_HIP(hipStreamSynchronize(g->res_stream));
-    g->res_pending = false;
-    volatile unsigned* w = g->res_withdrawn;
-    if (*w == 0) return ZG_OK;
-    *w = 0;
-    ZG_TRY(check_fault(g));  // (launches behind a failed one withdraw as well)
-    ++g->res_strikes;
-    g->res_sit_out = 8;
-    g->res_tag = 0xffffffffu;  // (what was not written keeps an old tag: all words are cleared in front of the next launch)
-    unsigned done = 0;
-    ZG_HIP(hipMemcpy(&done, &g->res_ctl->done, sizeof done, hipMemcpyDeviceToHost));
-    hipStream_t s = gs(g);
-    if (!(g->flags & ZG_GPT_NO_GRAPH) && s != nullptr && g->graph_stream != s) ZG_TRY(capture_all(g, s));
-    g->res_gen = false;
-    g->gen_pos = done;
-    g->gen_open = true;
-    ZG_TRY(pf_start(g, g->gen_n, s));
-    int rs = ZG_OK;
-    for (bool more = true; more && rs == ZG_OK;) rs = gen_pump(g, &more);
-    ZG_TRY(gen_end(g, rs));
-    ZG_HIP(hipStreamSynchronize(s));
     return ZG_OK;
 }
 
@@ -1706,14 +1689,8 @@ int zg_gpt_generate_fetch(zg_gpt* g, size_t n_steps, size_t* out_tokens, size_t 
     const size_t C = g->cfg.context_size, B = g->batch;
     ZG_REQUIRE(n_steps <= C && out_len >= B * n_steps, ZG_ERR_SHAPE, "generate_fetch: out_tokens too short");
     hipStream_t s = gs(g);
-    if (g->res_pending && g->res_stream != s) ZG_TRY(settle(g));
-    for (;;) {
-        ZG_HIP(hipMemcpyAsync(g->h_ints, g->out_tokens, B * C * sizeof(int), hipMemcpyDeviceToHost, s));
-        ZG_HIP(hipStreamSynchronize(s));
-        const bool made_up = g->res_pending && *static_cast<volatile unsigned*>(g->res_withdrawn) != 0;
-        ZG_TRY(settle(g));
-        if (!made_up) break;
-    }
+    ZG_HIP(hipMemcpyAsync(g->h_ints, g->out_tokens, B * C * sizeof(int), hipMemcpyDeviceToHost, s));
+    ZG_HIP(hipStreamSynchronize(s));
     ZG_TRY(check_fault(g));
     for (size_t b = 0; b < B; ++b)
         for (size_t i = 0; i < n_steps; ++i) out_tokens[b * n_steps + i] = (size_t)g->h_ints[b * C + i];
@@ -1732,7 +1709,6 @@ int zg_gpt_profile_step(zg_gpt* g, size_t seq_len, int iters, float* us_out, siz
     ZG_REQUIRE(g && us_out && n_out >= 8 && iters > 0, ZG_ERR_ARG, "profile_step: bad argument");
     ZG_REQUIRE(seq_len >= 1 && seq_len + (size_t)iters - 1 <= g->cfg.context_size, ZG_ERR_SHAPE,
                "profile_step: positions %zu..%zu outside the context", seq_len, seq_len + iters - 1);
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     ZG_HIP(hipStreamSynchronize(s));
     ZG_TRY(ensure_ln_folded(g, s));
@@ -1780,7 +1756,6 @@ int zg_gpt_time_kernel(zg_gpt* g, int which_and_options, int iters, float* avg_u
     const size_t t_opt = (size_t)((unsigned)which_and_options >> 16);    // another position for the attention kernel (0: mid-context)
     // (ZG_TIME_AT(t) occupies bits 16..30: t up to 32767 — every GPT-2 context; a larger t would set the sign bit)
     ZG_REQUIRE(g && avg_us && iters > 0 && which_and_options >= 0 && which <= 6, ZG_ERR_ARG, "time_kernel: bad argument (ZG_TIME_AT takes t < 32768)");
-    ZG_TRY(settle(g));
     hipStream_t s = gs(g);
     ZG_REQUIRE(s != nullptr, ZG_ERR_UNSUPPORTED, "time_kernel needs a capturable stream");
     const size_t E = g->cfg.n_embed, wb = g->wbytes;
@@ -1829,6 +1804,20 @@ int zg_gpt_time_kernel(zg_gpt* g, int which_and_options, int iters, float* avg_u
     *avg_us = ms * 1000.0f / (float)(reps * chain);
     if (algorithmic_bytes) *algorithmic_bytes = bytes_tab[which];
     return check_fault(g);
+}
+
+int zg_debug_resident_stats(zg_gpt* g, unsigned* out, size_t n_out) {
+    ZG_TRY(require_init());
+    ZG_REQUIRE(g && out && n_out >= 4, ZG_ERR_ARG, "resident_stats: need 4 words");
+    memset(out, 0, n_out * sizeof(unsigned));
+    ZG_HIP(hipStreamSynchronize(gs(g)));
+    ResidentCtl h;
+    ZG_HIP(hipMemcpy(&h, g->res_ctl, sizeof(ResidentCtl), hipMemcpyDeviceToHost));
+    out[0] = g->res_on;
+    out[1] = g->res_gen;
+    out[2] = h.rest_steps;
+    out[3] = h.rest_members;
+    return ZG_OK;
 }
 
 int zg_debug_prefetch_stats(zg_gpt* g, unsigned* out, size_t n_out) {

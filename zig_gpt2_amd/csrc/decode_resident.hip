@@ -29,7 +29,8 @@
 //
 // Safety: every workgroup must be resident before any may wait for another.  Workgroups register; the last one commits, and
 // one that has waited too long withdraws the launch for all (a compare-and-swap decides, so all agree): then nothing has been
-// touched and the host runs the launch chain instead.  Behind the commitment every wait is bounded as well (fault word).
+// touched, launches behind it leave at once, and the last one of the generation (decode_rest.hip), which needs no particular number of
+// workgroups, runs the steps that are missing.  Behind the commitment every wait is bounded as well (fault word).
 #include "decode_resident_parts.h"
 #include "zg_once.h"
 

@@ -316,13 +316,16 @@ int launch_sample_step(float* logits, int batch, int vocab, const SampleParams* 
 
 // ------------------------------------------------------------------------------------ resident decode (decode_resident.hip)
 struct ResidentCtl {
-    unsigned done;  // steps of the generation that resident launches have finished
-    unsigned pad[31];
+    unsigned done;  // steps of the generation that are finished
+    unsigned rest_steps, rest_members;  // steps that decode_rest_kernel has run since the handle was made, workgroups it last had
+    unsigned pad[29];
     // zeroed in front of every launch
     unsigned reg[8];  // workgroups registered by XCD
     unsigned total;   // in all
     unsigned state;   // 0 open, 1 committed: all workgroups are resident, 2 withdrawn
-    unsigned pad2[22];
+    unsigned joined, members, arrived;  // decode_rest_kernel: workgroups that came, those that share the work, arrivals at its barriers
+    unsigned pad2[19];
+    unsigned passed[8][32];  // its barriers that are complete, a line for every XCD
 };
 struct ResidentArgs {
     // layer 0; the others lie w_stride / kv_stride bytes apart
@@ -353,6 +356,16 @@ size_t resident_words(size_t n_embed, size_t batch);
 int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s);  // one sequence: bf16 or fp32 weights; two to eight: bf16
 size_t resident_batch_words(size_t n_embed);
 int launch_decode_resident_batch(const ResidentArgs& a, int n_embed, hipStream_t s);
+// the steps from ctl->done to s1 - 1 where launches were withdrawn (decode_rest.hip); any shape with 64 channels a head
+struct RestArgs {
+    ResidentArgs r;
+    int n_embed;
+    float *q, *z, *h;  // [batch][n_embed], [batch][n_embed], [batch][4 n_embed]
+    float* best_v;     // decode_rest_floats() in all
+    int* best_i;
+};
+size_t decode_rest_floats();
+int launch_decode_rest(const RestArgs& a, int weight_type, hipStream_t s);
 
 // ------------------------------------------------------------------------------------ multi-GPU (dist.hip)
 int dist_broadcast(void* buf, size_t bytes, int root, hipStream_t s);  // in place, over the communicator of zg_dist_init

@@ -180,6 +180,13 @@ class GPT:
         check(self._L.zg_gpt_profile_step(self.h, seq_len, iters, out.ctypes.data_as(_lib.f32p), out.size))
         return dict(zip(self.PROFILE_CLASSES + ["null_kernel_interval"], (float(v) for v in out)))
 
+    def resident_stats(self):
+        """zg_debug_resident_stats: whether greedy generations go to the resident kernels, whether the last one did, steps that were kept
+        from them."""
+        out = np.zeros(4, np.uint32)
+        check(self._L.zg_debug_resident_stats(self.h, out.ctypes.data_as(C.c_void_p), out.size))
+        return dict(zip(("on", "ran", "rest_steps", "rest_workgroups"), (int(v) for v in out)))
+
     def prefetch_stats(self):
         """zg_debug_prefetch_stats: {"on", "workgroups", "exit", "jobs"} (lists per XCD) of the last generate call."""
         out = np.zeros(25 + 256, np.uint32)
