@@ -128,7 +128,7 @@ __device__ __forceinline__ void in_flight() {  // at most N of this wave's vecto
 
 // ------------------------------------------------------------------------------------------------ the start
 // By one thread of every workgroup: register; the last one commits if the steps in front have run and every XCD has 32, one that has
-// waited too long withdraws the launch for all.  1: all workgroups are resident; 2: nothing may be touched.
+// waited too long (behind a withdrawn launch: at once) withdraws the launch for all.  1: all workgroups are resident; 2: nothing may be touched.
 __device__ inline unsigned join(ResidentCtl* ctl, unsigned xcc, unsigned s0, unsigned start_limit, unsigned* rank) {
     *rank = __hip_atomic_fetch_add(&ctl->reg[xcc], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const unsigned before = __hip_atomic_fetch_add(&ctl->total, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
@@ -141,7 +141,7 @@ __device__ inline unsigned join(ResidentCtl* ctl, unsigned xcc, unsigned s0, uns
     for (unsigned n = 0;; ++n) {
         const unsigned st = __hip_atomic_load(&ctl->state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (st != 0u) return st;
-        if (n >= start_limit) {
+        if (n >= start_limit || ctl->done != s0) {  // (final: no other launch is running)
             unsigned open = 0u;
             __hip_atomic_compare_exchange_strong(&ctl->state, &open, 2u, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             return open == 0u ? 2u : open;
