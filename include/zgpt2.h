@@ -314,10 +314,10 @@ int zg_gpt_generate_greedy(zg_gpt* g, const size_t* prompts, size_t prompt_strid
                            size_t out_len);
 /* Asynchronous form used by the benchmark: enqueue the same n_steps on the stream and return;
  * results stay on the device until zg_gpt_generate_fetch.  The stream's end is the generation's end: an event behind the call says that all
- * steps have run, also where a resident launch (one launch of up to 64 steps that needs all compute units at once: one
+ * steps have run, also where a resident launch (one launch of many steps that needs all compute units at once: one
  * sequence, or two to eight with bf16 weights, of widths 384, 512 and 768 on the library's stream) did not get them in time and the steps ran
- * another way.  While a resident launch runs, up to 12 ms, other streams have what it leaves of every compute unit: work whose workgroups
- * need more LDS than some 10 KB waits for its end (ZGPT2_RESIDENT=0 at creation: launches of a few microseconds each instead). */
+ * another way.  While a resident launch runs, some 3.5 ms, other streams have what it leaves of every compute unit: work whose workgroups
+ * need more LDS than that (about 10 KB at width 768) waits for its end (ZGPT2_RESIDENT=0 at creation: launches of a few microseconds each). */
 int zg_gpt_generate_enqueue(zg_gpt* g, const size_t* prompts, size_t prompt_stride,
                             const size_t* prompt_lens, size_t n_steps);
 int zg_gpt_generate_fetch(zg_gpt* g, size_t n_steps, size_t* out_tokens, size_t out_len);

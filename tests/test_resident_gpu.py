@@ -176,6 +176,52 @@ def test_launch_withdrawn_behind_others(zg, monkeypatch, name, batch, f32, launc
     chain.close()
 
 
+@pytest.mark.parametrize("batch", [1, 5])
+def test_beside_other_streams(zg, monkeypatch, batch):
+    """Generations beside matrix products on another stream, whose workgroups want most of a compute unit's LDS, and beside a handle with a
+    stream and a thread of its own: the tokens of each on its own, whichever way the steps ran; a product waits for one launch at most."""
+    import threading
+
+    import torch
+
+    cfg = synth.GPTConfig(1031, 256, 12, 12, 768)
+    w = synth.make_weights(cfg, seed=40, bf16=True)
+    p = [synth.rand_tokens(400 + b, 4 + b, cfg.vocab_size) for b in range(batch)]
+    m, own = make(monkeypatch, cfg, w, True, batch=batch), make(monkeypatch, cfg, w, True, batch=batch, own_stream=True)
+    want = m.generate(p, 256)
+    assert m.resident_stats()["ran"] and np.array_equal(own.generate(p, 256), want) and not own.resident_stats()["ran"]
+    side = torch.cuda.Stream()
+    a = torch.randn(2048, 2048, device="cuda").to(torch.bfloat16)
+    ref = a @ a
+    torch.cuda.synchronize()
+    got = []
+
+    def run():
+        for _ in range(3):
+            got.append(own.generate(p, 256))
+
+    t = threading.Thread(target=run)
+    t.start()
+    waits = []
+    for _ in range(6):
+        m.generate_enqueue(p, 256)
+        for _ in range(40):
+            t0 = time.perf_counter()
+            with torch.cuda.stream(side):
+                c = a @ a
+                done = torch.cuda.Event()
+                done.record(side)
+            done.synchronize()
+            waits.append(time.perf_counter() - t0)
+        assert np.array_equal(m.generate_fetch(256), want)
+    t.join()
+    assert len(got) == 3 and all(np.array_equal(g, want) for g in got)
+    assert torch.equal(c, ref)
+    print(f"products waited {1e3 * np.median(waits):.2f} ms, {1e3 * max(waits):.2f} at most; {m.resident_stats()}")
+    m.close()
+    own.close()
+
+
 @pytest.mark.parametrize("batch", [1, 4])
 def test_wait_that_runs_out_fails_the_call(zg, monkeypatch, batch):
     cfg = SHAPES["512"]

@@ -125,6 +125,7 @@ struct zg_gpt {
     bool res_on;                     // the handle's shape takes it
     bool res_gen;                    // the generation in flight does
     int res_strikes, res_sit_out;    // generations with a withdrawn launch so far (the third is final); generations left on the launch chain
+    size_t res_steps;                // steps of a launch at most
     size_t res_launch;               // launches of the generation in flight
     unsigned res_tag;                // first unused tag
     unsigned res_start_limit;        // polls before a launch that is not resident as a whole is withdrawn
@@ -778,6 +779,11 @@ void setup_resident(zg_gpt* g) {
     g->res_none_at = env_int("ZGPT2_RESIDENT_WITHDRAW", -1);
     if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
     if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer) || !env_int("ZGPT2_RESIDENT", 1)) return;
+    // Steps a launch takes: other streams' kernels that need more LDS than it leaves wait for its end, so it ends after some 3.5 ms (a Block takes
+    // about 9 us, 14 in a batch, half as much again with fp32 weights; the vocabulary 5.5 TB/s).  64 steps at most.  124M, one sequence, a
+    // matrix product beside it: waits of 7.1 ms with 64 steps a launch, 3.2 so; 256 tokens 28.20 and 28.27 ms (16 steps: 28.4)
+    const double us = (double)g->cfg.n_layer * (g->batch > 1 ? 14 : g->wt == WT_BF16 ? 9 : 13) + (double)g->cfg.vocab_size * g->cfg.n_embed * g->wbytes / 5.5e6;
+    g->res_steps = (size_t)std::min(64.0, std::max(1.0, 3500 / us));
     int cus = 0;
     g->res_on = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, ctx().device) == hipSuccess && cus == 256;
 }
@@ -824,11 +830,10 @@ ResidentArgs resident_args(zg_gpt* g, size_t s0, size_t s1) {
     return a;
 }
 
-// One launch: up to kResidentSteps steps from gen_pos on.  Other streams' kernels get the chip between launches.
-constexpr size_t kResidentSteps = 64;
+// One launch: up to res_steps steps from gen_pos on.  Other streams' kernels get the chip between launches.
 int enqueue_resident(zg_gpt* g, hipStream_t s) {
     const size_t L = g->cfg.n_layer;
-    const size_t st = g->gen_pos, n = std::min(kResidentSteps, g->gen_n - st);
+    const size_t st = g->gen_pos, n = std::min(g->res_steps, g->gen_n - st);
     const unsigned tags = (unsigned)(n * (L + 2));
     if (g->res_tag > 0xffffffffu - tags) {  // tags start over: none of the old ones may be found
         ZG_HIP(hipMemsetAsync(g->res_words, 0, g->res_words_bytes, s));
