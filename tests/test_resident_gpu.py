@@ -235,6 +235,25 @@ def test_wait_that_runs_out_fails_the_call(zg, monkeypatch, batch):
     m.close()
 
 
+def test_vocabulary_beyond_the_offsets_stays_on_the_chain(zg):
+    """1.4 million tokens of 768 columns: more than 32-bit offsets reach.  The launch chain takes them, as before."""
+    import torch
+
+    cfg = synth.GPTConfig(1_400_000, 8, 2, 12, 768)
+    m = zgpt.GPT(cfg, prefill=False)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(41)
+    w = {name: torch.randn(shape, generator=g, device="cuda") * 0.02 + mean for name, shape, mean, _ in synth.tensor_specs(cfg)}
+    m.load_weights(w)
+    ids = m.generate([[5]], 6)[0]
+    assert not m.resident_stats()["ran"]
+    x = torch.from_numpy(m.hidden()).cuda()  # of the last step: its pick is the largest product with the normed row
+    x = (x - x.mean()) / torch.sqrt(x.var(correction=0) + 1e-5) * w["ln_f_g"] + w["ln_f_b"]
+    logits = x @ w["wte"].to(torch.bfloat16).to(torch.float32).T
+    assert float(logits[0, int(ids[-1])]) >= float(logits.max()) - 1e-4
+    m.close()
+
+
 def test_what_the_chain_keeps(zg, monkeypatch):
     """Narrow caches, several sequences with fp32 weights, sampling, no graph, one layer: the launch chain, as before."""
     cfg = SHAPES["512"]

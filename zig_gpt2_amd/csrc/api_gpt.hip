@@ -778,7 +778,7 @@ void setup_resident(zg_gpt* g) {
     g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms
     g->res_none_at = env_int("ZGPT2_RESIDENT_WITHDRAW", -1);
     if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
-    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer) || !env_int("ZGPT2_RESIDENT", 1)) return;
+    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer, g->cfg.vocab_size) || !env_int("ZGPT2_RESIDENT", 1)) return;
     // Steps a launch takes: other streams' kernels that need more LDS than it leaves wait for its end, so it ends after some 3.5 ms (a Block takes
     // about 9 us, 14 in a batch, half as much again with fp32 weights; the vocabulary 5.5 TB/s).  64 steps at most.  124M, one sequence, a
     // matrix product beside it: waits of 7.1 ms with 64 steps a launch, 3.2 so; 256 tokens 28.20 and 28.27 ms (16 steps: 28.4)

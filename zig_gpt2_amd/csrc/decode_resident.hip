@@ -737,9 +737,9 @@ int launch(const ResidentArgs& a, hipStream_t s) {
 }  // namespace
 
 // (Two layers at least: the cache rows of the next step's first layer are requested during the last layer of this one, which has to be
-// another for the newest row to be known to have arrived.)
-bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer) {
-    if (n_heads * 64 != n_embed || n_heads > 16 || n_layer < 2) return false;
+// another for the newest row to be known to have arrived.  Rows of the vocabulary are found by 32-bit offsets of bytes.)
+bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer, size_t vocab) {
+    if (n_heads * 64 != n_embed || n_heads > 16 || n_layer < 2 || vocab < 1 || vocab > 0xffffffffu / (n_embed * 4)) return false;
     const size_t nw = n_embed / 64;
     if (nw != 6 && nw != 8 && nw != 12) return false;
     return ctx <= 64 * (n_heads > 8 ? kRanks / 2 : kRanks);  // a workgroup attends to 64 positions of one head
@@ -756,9 +756,7 @@ size_t resident_words(size_t n_embed, size_t batch) {
 }
 
 int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s) {
-    ZG_REQUIRE(resident_shape((size_t)n_embed, (size_t)a.n_heads, (size_t)a.ctx, (size_t)a.n_layer) && a.s0 >= 0 && a.s0 < a.s1 && a.s1 <= a.ctx && a.n_prompt >= 1 &&
-                   a.vocab >= 1 && (size_t)a.vocab * n_embed * 4 < ((size_t)1 << 32),
-               ZG_ERR_ARG, "resident decode: bad arguments");
+    ZG_REQUIRE(resident_shape((size_t)n_embed, (size_t)a.n_heads, (size_t)a.ctx, (size_t)a.n_layer, (size_t)a.vocab) && a.s0 >= 0 && a.s0 < a.s1 && a.s1 <= a.ctx && a.n_prompt >= 1, ZG_ERR_ARG, "resident decode: bad arguments");
     if (a.batch > 1) {
         ZG_REQUIRE(weight_type == WT_BF16, ZG_ERR_UNSUPPORTED, "resident decode: several sequences with fp32 weights");
         return launch_decode_resident_batch(a, n_embed, s);

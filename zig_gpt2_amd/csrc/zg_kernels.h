@@ -351,7 +351,7 @@ struct ResidentArgs {
     unsigned spin_limit, start_limit;
     unsigned *fault, *withdrawn;  // pinned host words
 };
-bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer);
+bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer, size_t vocab);
 size_t resident_words(size_t n_embed, size_t batch);
 int launch_decode_resident(const ResidentArgs& a, int n_embed, int weight_type, hipStream_t s);  // one sequence: bf16 or fp32 weights; two to eight: bf16
 size_t resident_batch_words(size_t n_embed);
