@@ -376,7 +376,7 @@ def other_config(lib, stream, model_name, ppg, gens, seed, kv_b24=False):
             "value": round(ppg * (ctx - 1) * gens / wall, 1), "unit": "tokens/s", "generations": gens, "ms_per_generation": round(1e3 * wall / gens, 3),
             "us_per_forward_device": round(1e6 * dev_s / (gens * ctx), 2),
             "kv_cache": "b24 (ZG_GPT_KV_B24: 24-bit elements, 4.7e-5 of the logit scale at full context)" if kv_b24 else "f32",
-            "l2_prefetcher": ("stalled" if pf["stalled"] else "on") if pf["on"] else "off",
+            "l2_prefetcher": "stalled" if pf["stalled"] else "on" if pf["ran"] else "off",
             "step_roofline": {"bound": "hbm", "algorithmic_bytes_per_generation": int(step_bytes_total),
                               "achieved": round(step_bytes_total * gens / dev_s / 1e9, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                               "frac": round(step_bytes_total * gens / dev_s / 1e9 / HBM_PEAK_GBS, 4)},
@@ -932,6 +932,7 @@ def main():
         elapsed = float(t.item())
     ids = model.generate_fetch(ctx)
     pf = model.prefetch_stats()  # how the side-stream prefetcher of the last generation ended (after the timed region)
+    res = model.resident_stats()  # whether it ran inside the resident kernel, and steps that were kept from it
 
     # tokens produced per generation: every position after the prompt is one generated token
     gen_tokens = ppg * (ctx - 1)
@@ -1088,7 +1089,8 @@ def main():
             "vocab": cfg.vocab_size, "context": cfg.context_size, "n_layer": cfg.n_layer, "n_heads": cfg.n_heads,
             "n_embed": cfg.n_embed, "prompts_per_gpu": ppg, "global_prompts": ppg * world,
             "kv_cache": "f16" if a.kv_f16 else "b24" if a.kv_b24 else "f32", "hip_graph": not a.no_graph,
-            "l2_prefetcher": ("stalled" if pf["stalled"] else "on") if pf["on"] else "off",
+            "l2_prefetcher": "stalled" if pf["stalled"] else "on" if pf["ran"] else "off",
+            "decode": "resident kernel" if res["ran"] else "launches", "steps_kept_from_the_resident_kernel": res["rest_steps"],
             "parallelism": f"replicated weights, prompts sharded x{world}, RCCL broadcast at start-up only",
             "tokens_counted": "generated tokens (context - prompt) per prompt",
             "scaling_note": ("N = 1 runs BASELINE configs[1] (one prompt: the headline metric); N > 1 runs configs[2] (8 prompts per GPU, "
@@ -1105,6 +1107,7 @@ def main():
             "achieved_layers_walked": round(dom["algorithmic_bytes_per_launch"] / dom["avg_launch_us_layers_walked"] / 1e3, 1),
             "frac_layers_walked": round(dom["algorithmic_bytes_per_launch"] / dom["avg_launch_us_layers_walked"] / 1e3 / HBM_PEAK_GBS, 4),
             "share_of_token_time": dom["share_of_token_time"],
+            "in_timed_region": not res["ran"],
             "how": "the kernel class with the largest share of the decode step as launches (what sampling, prompts token by token and the "
                    "shapes without a resident kernel run; the generation timed here is inside decode_resident*_kernel where that applies: "
                    "step_roofline is its figure); duration = HIP events on the launch "

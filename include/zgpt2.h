@@ -606,7 +606,8 @@ int zg_debug_resident_stats(zg_gpt* g, unsigned* out, size_t n_out);
  * out[0] = 1 when the handle has a prefetcher (2: it found no concurrency with the decode stream once and is no longer
  * launched); then per XCD x = 0..7: out[1 + x] prefetcher workgroups that ran
  * there, out[9 + x] why they left (1 = stop behind the last step, 2 = progress stalled), out[17 + x] launches they
- * fetched for.  n_out >= 25.  No reference counterpart. */
+ * fetched for; out[25] (when n_out >= 26) = 1 when the last zg_gpt_generate_* call launched it (greedy generations on the resident kernels do
+ * not: the words above are then an earlier call's).  n_out >= 25.  No reference counterpart. */
 int zg_debug_prefetch_stats(zg_gpt* g, unsigned* out, size_t n_out);
 
 /* ------------------------------------------------------------------------------------------------

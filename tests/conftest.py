@@ -33,12 +33,16 @@ def zg():
     yield lib
 
 
-# files whose subject is the launch chain: it stays the path of narrow caches, private streams, sampling and every shape the resident
-# kernels have not been built for
-LAUNCH_CHAIN = {"test_prefetch_gpu.py", "test_planes_gpu.py"}
+@pytest.fixture
+def launch_chain(monkeypatch):
+    """Greedy generation of handles made in the test as launches: the subject of a test that asks for this.  It stays the path of narrow caches,
+    private streams, sampling and every shape the resident kernels have not been built for."""
+    monkeypatch.setenv("ZGPT2_RESIDENT", "0")
 
 
-@pytest.fixture(autouse=True)
-def _launch_chain(request, monkeypatch):
-    if request.node.path.name in LAUNCH_CHAIN:
+@pytest.fixture(params=["default", "launches"])
+def decode_path(request, monkeypatch):
+    """Once as the library chooses, once as launches"""
+    if request.param == "launches":
         monkeypatch.setenv("ZGPT2_RESIDENT", "0")
+    return request.param

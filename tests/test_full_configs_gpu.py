@@ -33,7 +33,7 @@ def first_mismatch(a, b):
     return int(d[0]) if len(d) else None
 
 
-def test_124m_eight_prompts_full_context(zg):
+def test_124m_eight_prompts_full_context(zg, decode_path):
     """configs[2]'s per-GPU load: 8 sequences in lock step (matrix-core batched Linears, 8 private 1024-position KV
     caches) for the whole context."""
     cfg = synth.CONFIGS["124M"]
@@ -44,6 +44,7 @@ def test_124m_eight_prompts_full_context(zg):
     m8 = zgpt.GPT(cfg, batch=8)
     m8.load_weights(w)
     ids8 = m8.generate(prompts, ctx)
+    assert m8.resident_stats()["ran"] == (decode_path == "default")
     m8.close()
     assert ids8.shape == (8, ctx) and int(ids8.max()) < cfg.vocab_size
     for b in range(1, 6):  # identical prompts -> identical rows, all 1024 positions
@@ -59,7 +60,7 @@ def test_124m_eight_prompts_full_context(zg):
         ref, lg = oracle.GPT(cfg, w).generate_greedy(prompts[b], 64, want_logits=True)
         top = np.sort(lg, axis=1)
         assert_greedy_ids_match(ref[n:], ids8[b, n:64], top[:, -1], top[:, -2], f"124M x8 row {b}")
-    # the batch-1 path (VALU GEMVs, hipGraph) produces the same tokens, position for position
+    # the batch-1 path (resident, or VALU GEMVs in a hipGraph) produces the same tokens, position for position
     m1 = zgpt.GPT(cfg, batch=1)
     m1.load_weights(w)
     ids1 = m1.generate([p0], ctx)[0]

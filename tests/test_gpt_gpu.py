@@ -93,9 +93,9 @@ def test_full_context_nano_char_vs_oracle(zg):
     m.close()
 
 
-def test_124m_long_context_properties(zg):
+def test_124m_long_context_properties(zg, decode_path):
     """Full BASELINE size (124M, 1024 ctx): size-independent properties + an oracle spot check.
-    (a) graph replay == eager launches, token for token; (b) a batch of identical prompts yields
+    (a) graph replay, or the resident kernel, == eager launches, token for token; (b) a batch of identical prompts yields
     identical rows; (c) the first 96 steps equal the CPU oracle; (d) hidden state stays finite."""
     cfg = synth.CONFIGS["124M"]
     w = synth.make_weights(cfg, seed=0, bf16=True)
@@ -103,6 +103,7 @@ def test_124m_long_context_properties(zg):
     a = zgpt.GPT(cfg, use_graph=True)
     a.load_weights(w)
     ids_graph = a.generate([prompt], cfg.context_size)[0]
+    assert a.resident_stats()["ran"] == (decode_path == "default")
     assert np.isfinite(a.hidden()).all()
     a.close()
     b = zgpt.GPT(cfg, use_graph=False, batch=2)
@@ -289,7 +290,7 @@ def test_prompt_as_long_as_the_context(zg):
 
 
 @pytest.mark.parametrize("steps", [1, 4, 16])
-def test_steps_per_graph_do_not_change_tokens(zg, monkeypatch, steps):
+def test_steps_per_graph_do_not_change_tokens(zg, monkeypatch, launch_chain, steps):
     """The generate loop replays graphs of several consecutive steps (default 8, ZGPT2_GRAPH_STEPS): same ids as one
     step per graph, for prompts and lengths that are not multiples of the group."""
     cfg = synth.CONFIGS["nano-char"]
@@ -304,11 +305,12 @@ def test_steps_per_graph_do_not_change_tokens(zg, monkeypatch, steps):
     m.load_weights(w)
     for n, want in ref.items():
         assert np.array_equal(m.generate(prompts, n)[0], want), (steps, n)
+        assert not m.resident_stats()["ran"]
     m.close()
 
 
 @pytest.mark.parametrize("name", ["tiny3", "nano-char"])
-def test_batched_weight_load_shapes_agree(zg, monkeypatch, name):
+def test_batched_weight_load_shapes_agree(zg, monkeypatch, launch_chain, name):
     """The batched Linears fetch weights as full lines through a transposing LDS slot and lm_head runs one wave per
     tile; the fragment-shaped loads / the K-split lm_head remain as fall-backs (ZGPT2_DECODE_PATHS_OFF
     bits 16 / 32): same tokens either way, and both equal the oracle's."""
@@ -323,6 +325,7 @@ def test_batched_weight_load_shapes_agree(zg, monkeypatch, name):
         m = zgpt.GPT(cfg, batch=5, prefill=False)
         m.load_weights(w)
         outs.append(m.generate(prompts, n))
+        assert not m.resident_stats()["ran"]
         m.close()
     assert np.array_equal(outs[0], outs[1])
     for b, p in enumerate(prompts):

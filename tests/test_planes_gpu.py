@@ -14,7 +14,7 @@ from zig_gpt2_amd import gpt as zgpt
 from zig_gpt2_amd import synth
 from zig_gpt2_amd.synth import GPTConfig
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("launch_chain")]
 
 # ZGPT2_DECODE_PATHS_OFF bits (zg_common.h): 1 planes between kernels, 2 the four-wave Linear, 4 tagged hand-overs, 8 tile statistics
 VARIANTS = {"default": {}, "tickets": {"ZGPT2_DECODE_PATHS_OFF": "4"}, "16-wave": {"ZGPT2_DECODE_PATHS_OFF": "2"},
@@ -29,6 +29,7 @@ def run_variant(monkeypatch, env, cfg, w, batch, prompts, n_steps, **kw):
     m = zgpt.GPT(cfg, batch=batch, **kw)
     m.load_weights(w)
     ids = m.generate(prompts, n_steps)
+    assert not m.resident_stats()["ran"]
     lg = m.forward(3, [int(p[0]) for p in prompts])
     lg2 = m.forward(3, [int(p[0]) for p in prompts])  # the same step again: new tags, same numbers
     m.close()

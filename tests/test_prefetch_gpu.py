@@ -21,7 +21,7 @@ def make(cfg, w, **kw):
 
 @pytest.mark.parametrize("name,kw", [("nano-char", {}), ("nano-char", {"kv_f16": True}), ("nano-char", {"kv_b24": True}), ("nano-char", {"use_graph": False}),
                                      ("tiny3", {}), ("tiny3", {"prefill": False})])
-def test_same_tokens_with_and_without_prefetcher(zg, name, kw):
+def test_same_tokens_with_and_without_prefetcher(zg, launch_chain, name, kw):
     cfg = synth.CONFIGS[name]
     w = synth.make_weights(cfg, seed=21, bf16=True)
     prompt = synth.rand_tokens(211, 5, cfg.vocab_size)
@@ -32,7 +32,7 @@ def test_same_tokens_with_and_without_prefetcher(zg, name, kw):
             ids = m.generate([prompt], cfg.context_size)[0]
         st = m.prefetch_stats()
         m.close()
-        assert st["on"] == on
+        assert st["on"] == on and st["ran"] == on
         out[on] = ids
     assert np.array_equal(out[True], out[False])
     if not (kw.get("kv_f16") or kw.get("kv_b24")):  # (narrow caches: ids are compared between the two runs only)
@@ -41,7 +41,7 @@ def test_same_tokens_with_and_without_prefetcher(zg, name, kw):
         assert_greedy_ids_match(ref[len(prompt):], out[True][len(prompt):], top[:, -1], top[:, -2], f"{name} with prefetcher")
 
 
-def test_prefetcher_follows_the_chain_and_leaves(zg):
+def test_prefetcher_follows_the_chain_and_leaves(zg, launch_chain):
     cfg = synth.CONFIGS["nano-char"]
     w = synth.make_weights(cfg, seed=22, bf16=True)
     m = make(cfg, w)
@@ -96,6 +96,26 @@ def test_stalled_prefetcher_is_tried_again(zg, monkeypatch):
     assert np.array_equal(m.generate([prompt], cfg.context_size)[0], ref)  # tried again, with the default idle limit
     st = m.prefetch_stats()
     assert st["on"] and not st["stalled"] and st["exit"] == [1] * 8, st
+    m.close()
+
+
+def test_beside_the_resident_kernel(zg, monkeypatch):
+    """A handle whose greedy generations go to the resident kernel has the prefetcher for its sampled ones, and says which ran; a prefetcher
+    asked for by name is given the launches to fetch for."""
+    cfg = synth.CONFIGS["nano-char"]
+    w = synth.make_weights(cfg, seed=25, bf16=True)
+    p = [synth.rand_tokens(251, 2, cfg.vocab_size)]
+    m = make(cfg, w)
+    ids = m.generate(p, 40)
+    assert m.resident_stats()["ran"] and m.prefetch_stats()["on"] and not m.prefetch_stats()["ran"]
+    m.generate_sample(p, 40, 0.8, seed=1)
+    assert not m.resident_stats()["ran"] and m.prefetch_stats()["ran"]
+    m.close()
+    monkeypatch.setenv("ZGPT2_PREFETCH", "1")
+    m = make(cfg, w)
+    assert np.array_equal(m.generate(p, 40), ids)
+    st = m.prefetch_stats()
+    assert not m.resident_stats()["on"] and st["on"] and st["ran"] and st["exit"] == [1] * 8, st
     m.close()
 
 

@@ -109,7 +109,8 @@ struct zg_gpt {
     PfJob* pf_jobs;  // [pf_njobs]: embed, 5 per layer, lm_head
     int pf_njobs;
     bool pf_on;
-    bool pf_ran;      // a prefetcher was launched by the last generate call
+    bool pf_ran;      // a prefetcher was launched and nobody has looked at how it left
+    bool pf_last;     // the last generate call launched one
     bool pf_stalled;  // one left on its idle limit (no concurrency with the decode stream, or a host hiccup): sitting out
     int pf_strikes;   // idle-limit exits so far; the third one is final
     int pf_sit_out;   // generate calls left before a stalled prefetcher is tried again
@@ -679,12 +680,13 @@ int env_int(const char* name, int dflt) {
 // Side-stream prefetcher (prefetch.hip): job table, control block, low-priority stream.  Called from zg_gpt_create
 // BEFORE the graphs are captured (the decode kernels get the progress counter as an argument).
 int setup_prefetcher(zg_gpt* g) {
-    g->pf_on = g->pf_ran = g->pf_stalled = false;
+    g->pf_on = g->pf_ran = g->pf_last = g->pf_stalled = false;
     g->pf_strikes = g->pf_sit_out = 0;
     g->pf_stream = nullptr;
     g->pf_ev_main = g->pf_ev_side = nullptr;
     // Default: only where it was measured to pay — one sequence and Linears of a few MB (GPT-2 124M: 241 -> 224 us per
     // token; GPT-2 XL's 20 MB matrices cannot be fetched a launch ahead, 8 prompts gain < 1 %).  ZGPT2_PREFETCH=1 / 0 forces.
+    // (handles whose greedy generations go to the resident kernel have it for their sampled ones)
     // (not beside co-running handles: a handle with a private stream is one of several chains on the chip — §3.3 of DESIGN.md — and
     // the prefetcher's per-XCD placement follows ONE queue's block order; each would also park 96 polling workgroups)
     const bool small = g->stream == nullptr && g->batch == 1 && 4 * g->cfg.n_embed * g->cfg.n_embed * g->wbytes <= ((size_t)6 << 20);
@@ -756,7 +758,7 @@ int pf_start(zg_gpt* g, size_t last_T, hipStream_t s) {
     a.cls_mask = 0x3e;  // every class but lm_head (its head start measured a net loss)
     a.line_shift = 7;   // one touch per 128-byte line
     a.cap_bytes = 0;
-    g->pf_ran = true;
+    g->pf_ran = g->pf_last = true;
     return launch_prefetcher(a, g->pf_stream);
 }
 
@@ -778,7 +780,9 @@ void setup_resident(zg_gpt* g) {
     g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms
     g->res_none_at = env_int("ZGPT2_RESIDENT_WITHDRAW", -1);
     if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
-    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer, g->cfg.vocab_size) || !env_int("ZGPT2_RESIDENT", 1)) return;
+    if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer, g->cfg.vocab_size)) return;
+    // (a prefetcher that is asked for by name asks for the launches that it fetches for)
+    if (!env_int("ZGPT2_RESIDENT", env_int("ZGPT2_PREFETCH", 0) ? 0 : 1)) return;
     // Steps a launch takes: other streams' kernels that need more LDS than it leaves wait for its end, so it ends after some 3.5 ms (a Block takes
     // about 9 us, 14 in a batch, half as much again with fp32 weights; the vocabulary 5.5 TB/s).  64 steps at most.  124M, one sequence, a
     // matrix product beside it: waits of 7.1 ms with 64 steps a launch, 3.2 so; 256 tokens 28.20 and 28.27 ms (16 steps: 28.4)
@@ -1503,6 +1507,7 @@ static int gen_begin(zg_gpt* g, const size_t* prompts, size_t prompt_stride, con
     if (!(g->flags & ZG_GPT_NO_GRAPH) && s != nullptr && g->graph_stream != s) ZG_TRY(capture_all(g, s));  // before the prefetcher starts its idle clock
     ZG_TRY(note_steps(g, n_steps, s));
     g->res_gen = first < n_steps && resident_takes(g, sampled, s);
+    g->pf_last = false;
     if (g->res_gen) ZG_HIP(hipMemsetD32Async(reinterpret_cast<hipDeviceptr_t>(&g->res_ctl->done), (int)first, 1, s));
     else ZG_TRY(pf_start(g, n_steps, s));
     g->gen_pos = first;
@@ -1840,7 +1845,8 @@ int zg_debug_prefetch_stats(zg_gpt* g, unsigned* out, size_t n_out) {
         out[9 + x] = h.exit_reason[x];
         out[17 + x] = h.jobs_done[x];
     }
-    for (size_t i = 0; i < 256 && 25 + i < n_out; ++i) out[25 + i] = h.xcd_log[i];  // diagnostic (-DZG_STAMPS) builds only
+    if (n_out >= 26) out[25] = g->pf_last;
+    for (size_t i = 0; i < 256 && 26 + i < n_out; ++i) out[26 + i] = h.xcd_log[i];  // diagnostic (-DZG_STAMPS) builds only
     return ZG_OK;
 }
 

@@ -188,11 +188,12 @@ class GPT:
         return dict(zip(("on", "ran", "rest_steps", "rest_workgroups"), (int(v) for v in out)))
 
     def prefetch_stats(self):
-        """zg_debug_prefetch_stats: {"on", "workgroups", "exit", "jobs"} (lists per XCD) of the last generate call."""
-        out = np.zeros(25 + 256, np.uint32)
+        """zg_debug_prefetch_stats: {"on": the handle has one, "ran": the last generate call launched it, "workgroups", "exit", "jobs" (lists
+        per XCD) of the last call that did}."""
+        out = np.zeros(26 + 256, np.uint32)
         check(self._L.zg_debug_prefetch_stats(self.h, out.ctypes.data_as(C.c_void_p), out.size))
-        return {"on": bool(out[0]), "stalled": int(out[0]) == 2, "workgroups": out[1:9].tolist(), "exit": out[9:17].tolist(), "jobs": out[17:25].tolist(),
-                "xcd_of_block0": [int(v) & 15 for v in out[25:] if v & 0x100]}
+        return {"on": bool(out[0]), "ran": bool(out[25]), "stalled": int(out[0]) == 2, "workgroups": out[1:9].tolist(), "exit": out[9:17].tolist(), "jobs": out[17:25].tolist(),
+                "xcd_of_block0": [int(v) & 15 for v in out[26:] if v & 0x100]}
 
     def time_kernel(self, which, iters, walk_layers=False, at=0):
         """walk_layers: launch i of the chain takes layer i mod n_layer (weights / KV from the memory side, as in the real step);
