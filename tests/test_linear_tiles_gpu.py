@@ -49,12 +49,31 @@ def test_both_sides_of_the_rule(zg, m, k, n, kernel):
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 
+@pytest.mark.parametrize("m,k,n,kernel", [
+    (4, 512, 15, "linear_few_kernel"), (5, 512, 15, "linear_few_mfma_kernel"), (15, 512, 64, "linear_few_mfma_kernel"), (16, 512, 64, "linear_tiles_kernel"),
+    # five to eight rows: 512 columns, 1024 of more than 2048 outputs, 1536 to 1792 of more than 1024
+    (8, 248, 6144, "linear_few_mfma_kernel"), (8, 248, 6145, "gemv"), (8, 256, 6145, "linear_few_mfma_kernel"), (8, 520, 33, "linear_few_kernel"),
+    (8, 520, 2048, "linear_few_kernel"), (8, 520, 2049, "linear_few_mfma_kernel"), (8, 1024, 2049, "linear_few_mfma_kernel"), (8, 1032, 2049, "linear_few_kernel"),
+    (8, 1528, 1025, "linear_few_kernel"), (8, 1536, 1024, "linear_few_kernel"), (8, 1536, 1025, "linear_few_mfma_kernel"),
+    (5, 1792, 1025, "linear_few_mfma_kernel"), (5, 1800, 1025, "linear_few_kernel"),
+    # nine to fifteen: 128 to 1024 columns, to 1792 of up to 4096 outputs
+    (9, 120, 40, "gemv"), (9, 128, 40, "linear_few_mfma_kernel"), (9, 1024, 4097, "linear_few_mfma_kernel"), (9, 1088, 4096, "linear_few_mfma_kernel"),
+    (9, 1088, 4097, "linear_tiles_kernel"), (15, 1792, 4096, "linear_few_mfma_kernel"), (15, 1856, 40, "linear_tiles_kernel"), (15, 1800, 40, "gemv")])
+def test_which_kernel_takes_few_rows(zg, m, k, n, kernel):
+    run(1, 768, 768)  # (a general kernel; the ragged ones among them leave the note as it is)
+    w, b, x, y = run(m, k, n)
+    name = C.create_string_buffer(160)
+    _lib.check(zg.zg_debug_last_kernel(name, 160))
+    assert name.value.decode() == kernel or kernel == "gemv" and name.value.decode().startswith(kernel), name.value
+    assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
+
+
 @pytest.mark.parametrize("m", [5, 8, 9, 15])
 @pytest.mark.parametrize("k,n", [(64, 1), (120, 40), (136, 1), (136, 6145), (256, 16), (264, 17), (512, 15), (520, 33), (768, 2049), (1024, 2048), (1032, 31),
                                  (1536, 1025), (1792, 4096), (1784, 4097), (1800, 40)])
 def test_few_rows_on_the_matrix_cores(zg, m, k, n):
-    """Five to fifteen rows: the last columns of a piece, weight rows around the tile's sixteen, one piece of a wave to seven, both sides of the
-    rule.  A row that is not finite stays by itself."""
+    """Five to fifteen rows: the last columns of a piece, weight rows around the tile's sixteen, one piece of a wave to seven; those of them that the
+    rule gives to other kernels are held to the same.  A row that is not finite stays by itself."""
     w, b, x, y = run(m, k, n, bias=n % 2 == 1)
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
     xs = x.copy()

@@ -256,8 +256,8 @@ __global__ __launch_bounds__(256) void linear_few_kernel(const float* __restrict
 // the outputs are as near as those of the kernels it took over from, or nearer (rms of 768 columns 5.8e-8 of the outputs' own, 8.2e-8 and 7.2e-8
 // there; with 32-bit sums 8.0e-8).
 // What bounds it: latency, the launch and one round of loads, and where a workgroup has many pieces the intake of its compute unit.  A call, us,
-// those kernels -> this one: 8 rows 768 -> 3072 15.2 -> 13.8, 768 -> 50257 55 -> 46, 1600 -> 6400 28.2 -> 23.8, 12 rows 768 -> 768 18.8 -> 14.3,
-// 520 -> 600 25.8 -> 13.1, 768 -> 50257 57 -> 49.
+// repeated on the same buffers, those kernels -> this one: 8 rows 768 -> 3072 15.2 -> 13.8 (on new buffers every call 15.0 -> 14.4), 768 -> 50257 55 -> 46,
+// 1600 -> 6400 28.2 -> 23.8, 12 rows 768 -> 768 18.8 -> 14.3, 520 -> 600 25.8 -> 13.1, 768 -> 50257 57 -> 49.
 template <int RING>
 __global__ __launch_bounds__(512) void linear_few_mfma_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
                                                                     float* __restrict__ Y, int M, int N, int K) {
@@ -350,7 +350,7 @@ int launch_linear_tiles(const float* X, const float* W, const float* bias, float
     return ZG_OK;
 }
 
-// linear_few_mfma_kernel, or linear_few_kernel and the tiles; a call's us this : those.  Nine rows to fifteen (12 rows 768 -> 768 14.3 : 18.8,
+// linear_few_mfma_kernel, or linear_few_kernel and the tiles; a call's us on the same buffers, this : those.  Nine rows to fifteen (12 rows 768 -> 768 14.3 : 18.8,
 // 768 -> 3072 14.3 : 20.6, 1600 -> 1600 18.4 : 20.7; K in no whole 64s, as 520 -> 600, 13.1 : 25.8): the tiles, which have sixteen rows and more,
 // catch up where long rows make a compute unit's share long (16 rows 1600 -> 4800 25.0 : 24.0, 3072 -> 768 21.4 : 22.4, 6400 -> 1600 35.5 : 30.7);
 // rows shorter than their 128 columns stay on the general kernels.  Five to eight: linear_few_kernel has more workgroups and is ahead until they
@@ -384,7 +384,7 @@ int launch_linear_few(const float* X, const float* W, const float* bias, float* 
         else if (each == 3) ZG_FEW(3);
         else ZG_FEW(4);
 #undef ZG_FEW
-        note_kernel("linear_few_kernel");
+        note_kernel("linear_few_mfma_kernel");
         ZG_HIP(hipGetLastError());
         return ZG_OK;
     }
