@@ -88,6 +88,80 @@ def test_lock_step_batch_same_tokens_and_state_as_the_launch_chain(zg, monkeypat
     chain.close()
 
 
+@pytest.mark.parametrize("heads,batch,f32", [(6, 1, False), (8, 1, False), (8, 1, True), (6, 2, False), (6, 8, False), (8, 5, False), (8, 8, False)])
+def test_contexts_of_2048(zg, monkeypatch, heads, batch, f32):
+    """As many positions as the kernels take: 32 splits of a head, and in a batch eight chunks of a split and more."""
+    cfg = synth.GPTConfig(301, 2048, 2, heads, 64 * heads)
+    w = synth.make_weights(cfg, seed=42, bf16=not f32)
+    res, chain = (make(monkeypatch, cfg, w, r, batch=batch, weights_f32=f32) for r in (True, False))
+    for plen, steps in ((3, 2048), (1971, 2040), (1023, 1100)):
+        p = [synth.rand_tokens(420 + plen + b, plen - b % 3, cfg.vocab_size) for b in range(batch)]
+        a, b = res.generate(p, steps), chain.generate(p, steps)
+        assert res.resident_stats()["ran"] and not chain.resident_stats()["ran"]
+        assert np.array_equal(a, b), (plen, steps, np.argwhere(a != b)[:3])
+        assert rel(res.hidden(), chain.hidden()) < 2e-6, (plen, steps)
+        if steps < 2048:
+            assert rel(res.forward(steps + 1, a[:, -1]), chain.forward(steps + 1, a[:, -1])) < 2e-6, (plen, steps)
+    assert res.resident_stats()["rest_steps"] == 0
+    res.close()
+    chain.close()
+
+
+def classes(a):
+    return np.where(np.isnan(a), 3, np.where(np.isposinf(a), 1, np.where(np.isneginf(a), 2, 0)))
+
+
+@pytest.mark.parametrize("batch", [1, 3, 8])
+@pytest.mark.parametrize("where,what", [("k", np.inf), ("k", -np.inf), ("k", np.nan), ("v", np.inf), ("v", np.nan), ("k", 3e38), ("v", 3e38), ("wpe", np.inf),
+                                        ("wpe", np.nan)])
+def test_keys_and_values_that_are_not_finite(zg, monkeypatch, batch, where, what):
+    """A channel of every key or value, or one position's whole row (from there on in the cache), not finite or at the end of the range:
+    tokens and the class of every element of what is left are the chain's."""
+    cfg = SHAPES["768"]
+    w = dict(synth.make_weights(cfg, seed=43, bf16=True))
+    if where == "wpe":
+        w["wpe"] = w["wpe"].copy()
+        w["wpe"][67, 5] = what
+    else:
+        w["h1.c_attn_b"] = w["h1.c_attn_b"].copy()
+        w["h1.c_attn_b"][(768 if where == "k" else 1536) + 3 * 64 + 7] = what
+    p = [synth.rand_tokens(430 + b, 2, cfg.vocab_size) for b in range(batch)]
+    res, chain = (make(monkeypatch, cfg, w, r, batch=batch) for r in (True, False))
+    for steps in (3, 90):
+        a, b = res.generate(p, steps), chain.generate(p, steps)
+        assert res.resident_stats()["ran"]
+        assert np.array_equal(a, b), steps
+        assert np.array_equal(classes(res.hidden()), classes(chain.hidden())), steps
+        la, lb = res.forward(steps + 1, a[:, -1]), chain.forward(steps + 1, a[:, -1])
+        assert np.array_equal(classes(la), classes(lb)), steps
+    res.close()
+    chain.close()
+
+
+@pytest.mark.parametrize("batch", [2, 4, 5, 8])
+def test_one_sequence_that_is_not_finite_stays_by_itself(zg, monkeypatch, batch):
+    """A token whose embedding is NaN, in one sequence's prompt: the others' tokens, residual streams and logits are those of a batch without it, to the
+    bit."""
+    cfg = SHAPES["768"]
+    w = dict(synth.make_weights(cfg, seed=44, bf16=True))
+    w["wte"] = w["wte"].copy()
+    w["wte"][64] = np.nan
+    p = [synth.rand_tokens(440 + b, 2 + b % 2, 64) for b in range(batch)]
+    m = make(monkeypatch, cfg, w, True, batch=batch)
+    for bad in (0, batch - 1):
+        rest = [b for b in range(batch) if b != bad]
+        want, hid = m.generate(p, 100), m.hidden()
+        lg = m.forward(101, want[:, -1])
+        q = list(p)
+        q[bad] = np.array([64, 3], np.uint64)
+        got = m.generate(q, 100)
+        assert m.resident_stats()["ran"]
+        assert np.array_equal(got[rest], want[rest]) and np.array_equal(m.hidden()[rest], hid[rest])
+        assert not got[bad, 2:].any() and np.isnan(m.hidden()[bad]).all()
+        assert np.array_equal(m.forward(101, got[:, -1])[rest], lg[rest], equal_nan=True)
+    m.close()
+
+
 @pytest.mark.parametrize("batch", [1, 3])
 def test_tokens_of_the_oracle(zg, monkeypatch, batch):
     cfg = SHAPES["384"]
