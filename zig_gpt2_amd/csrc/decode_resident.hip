@@ -738,6 +738,8 @@ int launch(const ResidentArgs& a, hipStream_t s) {
 
 // (Two layers at least: the cache rows of the next step's first layer are requested during the last layer of this one, which has to be
 // another for the newest row to be known to have arrived.  Rows of the vocabulary are found by 32-bit offsets of bytes.)
+// Widths: the kernels are built for 384, 512 and 768, what was there to measure.  640 (10 waves with rows, heads on eight XCDs as 2, 2, 1, ...) would
+// be another instance and has not been; from 832 on a workgroup of n_embed / 64 + 4 waves is more than the 1024 threads there are.
 bool resident_shape(size_t n_embed, size_t n_heads, size_t ctx, size_t n_layer, size_t vocab) {
     if (n_heads * 64 != n_embed || n_heads > 16 || n_layer < 2 || vocab < 1 || vocab > 0xffffffffu / (n_embed * 4)) return false;
     const size_t nw = n_embed / 64;

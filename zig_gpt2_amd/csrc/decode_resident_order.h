@@ -18,6 +18,17 @@
 // orders an XCD without heads in front of the others: one that was a Block late found its word gone and waited until the call failed.)
 // Next x (MLP): behind x (c_proj) of the next Block, put by readers; an XCD without heads: behind far sums 1, 2 as above.  Picks and
 // bests: two hand-overs of the next step's first Block lie in between.
+//
+// What carries the words is gfx950's and not the language's memory model, which gives other workgroups no view of a store of workgroup scope
+// (tests/test_resident_words_cpu.py looks at the instructions these become):
+//   * a store without sc1 stops in the L2 of its XCD, all of whose compute units share it (their L1s are written through); one with sc1 goes on to
+//     the memory side.  A load with sc1 passes the L1.  So a near word is found by its own XCD, a far word by all.
+//   * eight aligned bytes are stored and loaded at once: a word's tag and its value belong together, also in 16-byte accesses of two words, each
+//     of which has a tag.  No other order between words is assumed: whoever needs two waits for both.
+//   * cache rows have no tags.  A wave's vector memory operations are counted in order (vmcnt), and every wave that stores rows polls x (c_proj)
+//     behind them, in front of its workgroup's h: when the polled word is there, so are the rows, in this XCD's L2.  They are asked for with
+//     sc1, by workgroups of the same XCD, that have waited for h of that Block since (the newest row travels as words).  Between launches the
+//     launch boundary does it.
 #pragma once
 
 namespace zg {

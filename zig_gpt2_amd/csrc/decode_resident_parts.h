@@ -4,6 +4,10 @@
 #include "zg_common.h"
 #include "zg_kernels.h"
 
+#if defined(__HIP_DEVICE_COMPILE__) && !defined(__gfx950__)
+#error "the words of the resident kernels rest on what gfx950's caches do (decode_resident_order.h)"
+#endif
+
 namespace zg {
 namespace resident {
 
@@ -30,7 +34,7 @@ __device__ __forceinline__ unsigned fresh(unsigned v) {
 // ------------------------------------------------------------------------------------------------ words with tags
 __device__ __forceinline__ u64 tagged(unsigned tag, float v) { return ((u64)tag << 32) | (u64)__float_as_uint(v); }
 __device__ __forceinline__ gword* word(const u64* base, unsigned i) { return (gword*)(base_at(base) + fresh(i * 8u)); }
-// word i of base.  Within the XCD: no bit of a wider scope, the word stays in this L2
+// word i of base.  Within the XCD: no bit of a wider scope, the word stays in this L2 (decode_resident_order.h: what this rests on)
 __device__ __forceinline__ void put_near(u64* base, unsigned i, u64 v) { __hip_atomic_store(word(base, i), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 // for every XCD: written through
 __device__ __forceinline__ void put_far(u64* base, unsigned i, u64 v) { __hip_atomic_store(word(base, i), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
