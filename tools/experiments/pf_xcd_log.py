@@ -4,6 +4,7 @@
 import json, os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch
+os.environ.setdefault("ZGPT2_RESIDENT", "0")  # (the launches are the subject)
 from zig_gpt2_amd import _lib, gpt, synth
 lib = _lib.load(); _lib.check(lib.zg_init(0))
 stream = torch.cuda.Stream(); _lib.check(lib.zg_set_stream(stream.cuda_stream))

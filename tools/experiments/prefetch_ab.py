@@ -6,6 +6,7 @@ import json, os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import numpy as np
 import torch
+os.environ.setdefault("ZGPT2_RESIDENT", "0")  # (the launches are the subject)
 from zig_gpt2_amd import _lib, gpt, synth
 
 lib = _lib.load(); _lib.check(lib.zg_init(0))

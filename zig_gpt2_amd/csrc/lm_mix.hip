@@ -1103,7 +1103,7 @@ __global__ __launch_bounds__(256) void latent_tiles_kernel(const float* cache, i
 // Bound by the matrix cores and the LDS together: a fragment of keys (1 KB) serves one product (32 cycles), so the four SIMDs of a
 // compute unit ask the LDS for its whole 128 B per clock; two workgroups per compute unit hide the softmax of one under the
 // products of the other (hence 256 registers a lane: 72 of queries, 128 of sums).  The blocks with the most keys are dealt first.
-// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 110 us and 9 for the tiles (73 GFLOP: 615 TFLOP/s); 827 us when every workgroup
+// 8 x 1023 tokens, 16 heads on latents of 256 + 32: 116 us and 9 for the tiles (73 GFLOP: 585 TFLOP/s); 827 us when every workgroup
 // converted and transposed its own tiles behind three barriers.
 template <int NKS, int NT>  // 16 NKS >= KR + R (score dimensions), 32 NT >= KR (latent dimensions)
 __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_kernel(const float* qa, const bf16_t* qa16, float* ctx, bf16_t* ctx16, int H, int KR, int R, float scale,
@@ -1267,7 +1267,8 @@ __global__ __launch_bounds__(256, NKS > 18 ? 1 : 2) void latent_attention_mfma_k
     const float L = lsum + __shfl_xor(lsum, 32, 64);
     if (ctx16) {  // (KR is a multiple of 8)
         // A lane has a query's values: turned in the tiles' place, half of the dimensions at a time, they leave as 16-byte pieces of whole rows.
-        // (8 bytes a lane to 32 rows, divided one by one: 6.1 us behind the last tile, 2.0 so.)  The quotients are those of a division.
+        // (8 bytes a lane to 32 rows, divided one by one: 6.1 us behind the last tile, 3.3 so; 2.0 with one reciprocal a
+        // row, whose quotients are a last bit off: these are the division's.)
         constexpr int P = NT * 16, PITCH = P * 2 + 16;
         static_assert(32 * PITCH <= T::BYTES / 2, "a wave's rows fit its half of a tile's place");
         char* const img = &Ks[0][0] + wave * (T::BYTES / 2);
