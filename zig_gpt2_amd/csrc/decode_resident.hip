@@ -139,7 +139,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
     constexpr int RA = (6 * NH + NW - 1) / NW;                     // rows of c_attn a wave has
     constexpr int HC = NH * 64, CC = 2 * NH;                       // columns of c_proj an XCD owns, a lane's share of them
     constexpr int NG = (NW - 1) * 64 / HC;                         // splits gathered at a time; the last wave has their maxima and sums
-    constexpr int PW = 16, AW = 4, MS = kRanks / NH;               // attention: positions of a wave, waves, most splits of a head
+    constexpr int AW = 4, MS = kRanks / NH;                        // attention: waves, most splits of a head
     constexpr int LC = NW % 4 == 0 ? 8 : 4, LN = 2 * NW / LC, LR = sizeof(WT) == 2 ? 2 : 1;  // lm_head: pieces of a row (half a wave), rows in flight
     static_assert(CH * NC == NW && LC * LN == 2 * NW && 8 * CPR <= E && NW <= 12 && 2 * NH * MS <= 64 && NG >= 1, "shapes");
     static_assert(R::nD + R::nE + R::nA + R::nC + R::nV + 8 < 64, "vmcnt counts to 63");
@@ -257,29 +257,12 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                 }
             }
         };
-        // Eight lanes have a position's key, 16 lanes (a row) its values, four each: of eight positions a row has the values of the
-        // two that it scores, so that a weight is in its row already (or eight lanes away).  readlane for all of them: 0.15 us more
-        f32x4 kr[PW / 8][2], vr[PW / 4];
+        KeyRows kv;
         auto load_KV = [&](int l, int T) {  // the cache rows in front of position T - 1
-            // rows this XCD's workgroups wrote: past the L1 (sc1), whose lines may be older.  Positions that are not there yet re-read
-            // the last one that is; they weigh nothing
             const size_t slab = (size_t)l * a.kv_stride + (size_t)head * a.ctx * 256;
-            const int bytes = a.ctx * 256;
-            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(a.k_cache + slab, 0, bytes, 0x00020000);
-            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(a.v_cache + slab, 0, bytes, 0x00020000);
-            const int p0 = sp * 64 + fw * PW, last = max(T - 2, 0);
-            const int l8 = (int)fresh((unsigned)lane);
-#pragma unroll
-            for (int i = 0; i < PW / 8; ++i) {
-                const int off = min(p0 + i * 8 + (l8 >> 3), last) * 256 + (l8 & 7) * 32;
-                kr[i][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 16));
-                kr[i][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16, 0, 16));
-            }
-#pragma unroll
-            for (int i = 0; i < PW / 4; ++i)
-                vr[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i / 2 * 8 + i % 2 + (l8 >> 4) * 2, last) * 256 + (l8 & 15) * 16, 0, 16));
+            load_rows(kv, a.k_cache + slab, a.v_cache + slab, a.ctx, sp * 64 + fw * 16, T, lane);
         };
-        constexpr int nKV = 2 * (PW / 8) + PW / 4;
+        constexpr int nKV = 8;
         int vp = 0;
         auto attends = [&](int T) { return hi < nh && sp < (T + 63) >> 6; };
         fetch_V(0, 0);
@@ -293,9 +276,9 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
             for (int l = 0; l < a.n_layer; ++l) {
                 const int ln = l + 1 < a.n_layer ? l + 1 : 0, Tn = l + 1 < a.n_layer ? T : T + 1;
                 barrier();  // B1
-                if (attends(T)) {
-#pragma unroll
-                    for (int i = 0; i < PW / 8; ++i) asm volatile("" ::"v"(kr[i][0]), "v"(kr[i][1]), "v"(vr[2 * i]), "v"(vr[2 * i + 1]));  // (here since B6; nobody waits for them behind the fetches)
+                if (attends(T)) {  // (here since B6; nobody waits for them behind the fetches)
+                    asm volatile("" ::"v"(kv.k[0][0]), "v"(kv.k[0][1]), "v"(kv.v[0]), "v"(kv.v[1]));
+                    asm volatile("" ::"v"(kv.k[1][0]), "v"(kv.k[1][1]), "v"(kv.v[2]), "v"(kv.v[3]));
                 }
                 if (R::copies == 1 && nh > 0) fetch_C(l, 0);
                 if (nh > 0) {
@@ -304,49 +287,10 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                     } else {
                         barrier();  // B2
                         // ---- B
-                        const int p0 = sp * 64 + fw * PW;
-                        float q8[8], k8[8];
-                        lds_floats<8>(&s_new[(lane & 7) * 8], q8);
-                        lds_floats<8>(&s_new[64 + (lane & 7) * 8], k8);
-                        const f32x4 vn = *reinterpret_cast<const f32x4*>(&s_new[128 + (lane & 15) * 4]);
-                        float sc[PW / 8];
-                        float m = kNone;
-#pragma unroll
-                        for (int i = 0; i < PW / 8; ++i) {
-                            const int t = p0 + i * 8 + (lane >> 3);
-                            const bool nw = t == T - 1;
-                            float acc0 = 0.0f, acc1 = 0.0f;
-#pragma unroll
-                            for (int d = 0; d < 4; ++d) {
-                                acc0 = fmaf(q8[d], nw ? k8[d] : kr[i][0][d], acc0);
-                                acc1 = fmaf(q8[4 + d], nw ? k8[4 + d] : kr[i][1][d], acc1);
-                            }
-                            const float dot = sum8(acc0 + acc1) * 0.125f;  // 1 / sqrt(64): ops.zig:275
-                            sc[i] = t < T ? dot : kNone;
-                            m = fmaxf(m, sc[i]);
-                        }
-                        auto over_rows = [&](float v, auto op) { return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48))); };
-                        m = over_rows(fmaxf(m, dpp_row_ror<8>(m)), [](float x, float y) { return fmaxf(x, y); });
-                        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};  // four columns, every fourth position
-                        float lsum = 0.0f;
-#pragma unroll
-                        for (int i = 0; i < PW / 8; ++i) {
-                            const float p = p0 + i * 8 + (lane >> 3) < T ? __expf(sc[i] - m) : 0.0f, other = dpp_row_ror<8>(p);
-                            lsum += p + other;
-#pragma unroll
-                            for (int q = 0; q < 2; ++q) {
-                                const int tj = p0 + i * 8 + q + (lane >> 4) * 2;
-                                const float pq = (lane >> 3 & 1) == q ? p : other;
-#pragma unroll
-                                for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? vr[i * 2 + q][d] : 0.0f, o[d]);
-                            }
-                        }
-                        lsum = over_rows(lsum, [](float x, float y) { return x + y; });
-                        *reinterpret_cast<f32x4*>(&s_o[fw * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
-                        if (lane == 0) {
-                            s_m[fw] = m;
-                            s_l[fw] = lsum;
-                        }
+                        float m = kNone, lsum = 0.0f;
+                        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+                        attend_rows<1, true>(&kv, sp * 64 + fw * 16, T, lane, s_new, m, lsum, o);
+                        put_share(fw, lane, m, lsum, o, s_o, s_m, s_l);
                         barrier();  // B3
                         __builtin_amdgcn_s_sleep(kAfterB);
                     }
@@ -484,16 +428,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_kernel(const Re
                     barrier();  // B2
                     barrier();  // B3
                     if (wave == 0) {
-                        static_assert(AW == 4, "waves that attend");
-                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(s_m), l4 = *reinterpret_cast<const f32x4*>(s_l);
-                        const float m = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w));
-                        float o = 0.0f, lsum = 0.0f;
-#pragma unroll
-                        for (int i = 0; i < AW; ++i) {
-                            const float e = __expf(m4[i] - m);
-                            o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
-                            lsum = fmaf(e, l4[i], lsum);
-                        }
+                        float m, lsum, o;
+                        merge_waves(lane, s_o, s_m, s_l, m, lsum, o);
                         const unsigned to = P::att + (hi * G + sp) * kPartStride + lane;
                         if (lane < 2) put_near(near, to + 64, tagged(tag, lane ? lsum : m));
                         put_near(near, to, tagged(tag, o));

@@ -305,34 +305,15 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
     if (wave >= NW) {
         // =========================================================================================== fetch and attend
         const int fw = wave - NW;
-        struct Rows {
-            f32x4 k[2][2], v[4];  // 16 positions: 8 x 8 dims of keys, 4 x 4 dims of values a lane (laid out as in decode_resident.hip)
-        };
-        auto over_rows = [](float v, auto op) { return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48))); };
         // (in front of loads that are not always made: the registers would be kept for the rows they held before)
-        auto forget = [&](Rows& x) {
+        auto forget = [&](KeyRows& x) {
             asm volatile("" : "=v"(x.k[0][0]), "=v"(x.k[0][1]), "=v"(x.k[1][0]), "=v"(x.k[1][1]));
             asm volatile("" : "=v"(x.v[0]), "=v"(x.v[1]), "=v"(x.v[2]), "=v"(x.v[3]));
         };
         // chunk c of 64 positions of this workgroup's (head, sequence): 16 a wave
-        auto load_KV = [&](Rows& to, int l, int T, int c) {
-            // rows this XCD's workgroups wrote: past the L1 (sc1), whose lines may be older.  Positions that are not there yet re-read
-            // the last one that is; they weigh nothing
+        auto load_KV = [&](KeyRows& to, int l, int T, int c) {
             const size_t slab = (size_t)l * a.kv_stride + ((size_t)im * H + head) * a.ctx * 256;
-            const int bytes = a.ctx * 256;
-            const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(a.k_cache + slab, 0, bytes, 0x00020000);
-            const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(a.v_cache + slab, 0, bytes, 0x00020000);
-            const int p0 = c * 64 + fw * 16, last = max(T - 2, 0);
-            const int l8 = (int)fresh((unsigned)lane);
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int off = min(p0 + i * 8 + (l8 >> 3), last) * 256 + (l8 & 7) * 32;
-                to.k[i][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 16));
-                to.k[i][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16, 0, 16));
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                to.v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i / 2 * 8 + i % 2 + (l8 >> 4) * 2, last) * 256 + (l8 & 15) * 16, 0, 16));
+            load_rows(to, a.k_cache + slab, a.v_cache + slab, a.ctx, c * 64 + fw * 16, T, lane);
         };
         int vp = 0;
         fetch_V(0, 0, fw);
@@ -353,7 +334,7 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                         __builtin_amdgcn_s_sleep(kAfterA);
                     } else {
                         // (asked for here: c_attn and its hand-over take longer than they do; across Blocks they would want 64 registers all along)
-                        Rows kv[2];
+                        KeyRows kv[2];
                         load_KV(kv[0], l, T, c0);
                         fetch_C(l, fw, 4);
                         barrier();  // B1a
@@ -362,71 +343,17 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                         barrier();  // B2
                         // ---- B
                         float m = kNone, lsum = 0.0f;
-                        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};  // four columns, every fourth position
-                        auto attend = [&](auto n_chunks, int c) {  // one chunk or two: their dependent steps side by side
-                            constexpr int N = decltype(n_chunks)::value;
-                            const int p0 = c * 64 + fw * 16;
-                            // (query and newest row are read where they are used: both chunks in flight take 64 registers)
-                            float sc[2 * N], mn = m;
-                            {
-                                const unsigned at = fresh(lds_at(&s_new[(lane & 7) * 8]));
-                                const f32x4 q0 = lds_read<f32x4>(at), q1 = lds_read<f32x4>(at + 16), n0 = lds_read<f32x4>(at + 256), n1 = lds_read<f32x4>(at + 272);
-#pragma unroll
-                                for (int i = 0; i < 2 * N; ++i) {
-                                    const Rows& x = kv[i / 2];
-                                    const int t = p0 + i / 2 * 64 + i % 2 * 8 + (lane >> 3);
-                                    const bool nw = t == T - 1;
-                                    float acc0 = 0.0f, acc1 = 0.0f;
-#pragma unroll
-                                    for (int d = 0; d < 4; ++d) {
-                                        acc0 = fmaf(q0[d], nw ? n0[d] : x.k[i % 2][0][d], acc0);
-                                        acc1 = fmaf(q1[d], nw ? n1[d] : x.k[i % 2][1][d], acc1);
-                                    }
-                                    const float dot = sum8(acc0 + acc1) * 0.125f;  // 1 / sqrt(64): ops.zig:275
-                                    sc[i] = t < T ? dot : kNone;
-                                }
-                            }
-                            {
-                                float top = sc[0];
-#pragma unroll
-                                for (int i = 1; i < 2 * N; ++i) top = fmaxf(top, sc[i]);
-                                mn = fmaxf(mn, over_rows(fmaxf(top, dpp_row_ror<8>(top)), [](float x, float y) { return fmaxf(x, y); }));
-                            }
-                            const f32x4 vn = lds_read<f32x4>(fresh(lds_at(&s_new[128 + (lane & 15) * 4])));
-                            const float e0 = __expf(m - mn);
-                            lsum *= e0;
-                            o *= e0;
-#pragma unroll
-                            for (int i = 0; i < 2 * N; ++i) {
-                                const int tb = p0 + i / 2 * 64 + i % 2 * 8;
-                                const float p = tb + (lane >> 3) < T ? __expf(sc[i] - mn) : 0.0f, other = dpp_row_ror<8>(p);
-                                lsum += p + other;
-                                if (N == 2) __builtin_amdgcn_sched_barrier(0);  // (the values, last to arrive, are not waited for earlier: 2 % of long contexts)
-#pragma unroll
-                                for (int q = 0; q < 2; ++q) {
-                                    const int tj = tb + q + (lane >> 4) * 2;
-                                    const float pq = (lane >> 3 & 1) == q ? p : other;
-#pragma unroll
-                                    for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? kv[i / 2].v[i % 2 * 2 + q][d] : 0.0f, o[d]);
-                                }
-                            }
-                            m = mn;
-                        };
+                        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
                         for (int c = c0;;) {
-                            if (c + 1 < c1) attend(std::integral_constant<int, 2>{}, c);
-                            else attend(std::integral_constant<int, 1>{}, c);
+                            if (c + 1 < c1) attend_rows<2, false>(kv, c * 64 + fw * 16, T, lane, s_new, m, lsum, o);  // one chunk or two
+                            else attend_rows<1, false>(kv, c * 64 + fw * 16, T, lane, s_new, m, lsum, o);
                             c += 2;
                             if (c >= c1) break;
                             load_KV(kv[0], l, T, c);
                             forget(kv[1]);
                             if (c + 1 < c1) load_KV(kv[1], l, T, c + 1);
                         }
-                        lsum = over_rows(lsum, [](float x, float y) { return x + y; });
-                        *reinterpret_cast<f32x4*>(&s_o[fw * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
-                        if (lane == 0) {
-                            s_m[fw] = m;
-                            s_l[fw] = lsum;
-                        }
+                        put_share(fw, lane, m, lsum, o, s_o, s_m, s_l);
                         barrier();  // B3
                     }
                 } else {
@@ -756,15 +683,8 @@ __global__ __launch_bounds__(64 * (NW + 4)) void decode_resident_batch_kernel(co
                     }
                     barrier();  // B3
                     if (wave == 0) {
-                        const f32x4 m4 = *reinterpret_cast<const f32x4*>(s_m), l4 = *reinterpret_cast<const f32x4*>(s_l);
-                        const float m = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w));
-                        float o = 0.0f, lsum = 0.0f;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) {
-                            const float e = __expf(m4[i] - m);
-                            o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
-                            lsum = fmaf(e, l4[i], lsum);
-                        }
+                        float m, lsum, o;
+                        merge_waves(lane, s_o, s_m, s_l, m, lsum, o);
                         const unsigned to = (unsigned)((im * NH + ih) * kMostSplits + sp);
                         if (lane < 2) put_near(near, P::ml + to * 2u + lane, tagged(tag, lane ? lsum : m));
                         put_near(near, P::att + to * 64u + lane, tagged(tag, o));

@@ -130,6 +130,105 @@ __device__ __forceinline__ void in_flight() {  // at most N of this wave's vecto
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
 }
 
+// ------------------------------------------------------------------------------------------------ attention
+// 16 positions of a head, by a wave.  Eight lanes have a position's key, 16 lanes (a row) its values, four each: of eight positions a row has the
+// values of the two that it scores, so that a weight is in its row already (or eight lanes away).  readlane for all of them: 0.15 us more
+struct KeyRows {
+    f32x4 k[2][2], v[4];
+};
+// The rows from p0 on.  This XCD's workgroups wrote them: past the L1 (sc1), whose lines may be older.  Positions that are not there yet re-read the
+// last one that is; they weigh nothing
+__device__ __forceinline__ void load_rows(KeyRows& to, char* k_rows, char* v_rows, int ctx, int p0, int T, int lane) {
+    const int bytes = ctx * 256, last = max(T - 2, 0);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(k_rows, 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(v_rows, 0, bytes, 0x00020000);
+    const int l8 = (int)fresh((unsigned)lane);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int off = min(p0 + i * 8 + (l8 >> 3), last) * 256 + (l8 & 7) * 32;
+        to.k[i][0] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 16));
+        to.k[i][1] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, off + 16, 0, 16));
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+        to.v[i] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, min(p0 + i / 2 * 8 + i % 2 + (l8 >> 4) * 2, last) * 256 + (l8 & 15) * 16, 0, 16));
+}
+template <typename Op>
+__device__ __forceinline__ float over_rows(float v, Op op) { return op(op(lane_value(v, 0), lane_value(v, 16)), op(lane_value(v, 32), lane_value(v, 48))); }
+
+// N pieces of 16 positions, the first from p0 on and 64 apart, their dependent steps side by side: running maximum and sum, o four columns of every
+// fourth position.  s_new: query, key and value of position T - 1 in the LDS, read where they are used (two pieces in flight take 64 registers)
+template <int N, bool FIRST>
+__device__ __forceinline__ void attend_rows(const KeyRows* kv, int p0, int T, int lane, const float* s_new, float& m, float& lsum, f32x4& o) {
+    float sc[2 * N], mn = m;
+    {
+        const unsigned at = fresh(lds_at(&s_new[(lane & 7) * 8]));
+        const f32x4 q0 = lds_read<f32x4>(at), q1 = lds_read<f32x4>(at + 16), n0 = lds_read<f32x4>(at + 256), n1 = lds_read<f32x4>(at + 272);
+#pragma unroll
+        for (int i = 0; i < 2 * N; ++i) {
+            const KeyRows& x = kv[i / 2];
+            const int t = p0 + i / 2 * 64 + i % 2 * 8 + (lane >> 3);
+            const bool nw = t == T - 1;
+            float acc0 = 0.0f, acc1 = 0.0f;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                acc0 = fmaf(q0[d], nw ? n0[d] : x.k[i % 2][0][d], acc0);
+                acc1 = fmaf(q1[d], nw ? n1[d] : x.k[i % 2][1][d], acc1);
+            }
+            const float dot = sum8(acc0 + acc1) * 0.125f;  // 1 / sqrt(64): ops.zig:275
+            sc[i] = t < T ? dot : kNone;
+        }
+    }
+    {
+        float top = sc[0];
+#pragma unroll
+        for (int i = 1; i < 2 * N; ++i) top = fmaxf(top, sc[i]);
+        mn = fmaxf(mn, over_rows(fmaxf(top, dpp_row_ror<8>(top)), [](float x, float y) { return fmaxf(x, y); }));
+    }
+    const f32x4 vn = lds_read<f32x4>(fresh(lds_at(&s_new[128 + (lane & 15) * 4])));
+    if (!FIRST) {
+        const float e0 = __expf(m - mn);
+        lsum *= e0;
+        o *= e0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2 * N; ++i) {
+        const int tb = p0 + i / 2 * 64 + i % 2 * 8;
+        const float p = tb + (lane >> 3) < T ? __expf(sc[i] - mn) : 0.0f, other = dpp_row_ror<8>(p);
+        lsum += p + other;
+        if (N == 2) __builtin_amdgcn_sched_barrier(0);  // (the values, last to arrive, are not waited for earlier: 2 % of long contexts)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const int tj = tb + q + (lane >> 4) * 2;
+            const float pq = (lane >> 3 & 1) == q ? p : other;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) o[d] = fmaf(pq, tj == T - 1 ? vn[d] : tj < T ? kv[i / 2].v[i % 2 * 2 + q][d] : 0.0f, o[d]);
+        }
+    }
+    m = mn;
+}
+// What wave w of four has, for merge_waves
+__device__ __forceinline__ void put_share(int w, int lane, float m, float lsum, const f32x4& o, float (*s_o)[64], float* s_m, float* s_l) {
+    lsum = over_rows(lsum, [](float x, float y) { return x + y; });
+    *reinterpret_cast<f32x4*>(&s_o[w * 4 + (lane >> 4)][(lane & 15) * 4]) = o;
+    if (lane == 0) {
+        s_m[w] = m;
+        s_l[w] = lsum;
+    }
+}
+// by one wave: the four waves' maxima, sums and (a lane a column) values
+__device__ __forceinline__ void merge_waves(int lane, const float (*s_o)[64], const float* s_m, const float* s_l, float& m, float& lsum, float& o) {
+    const f32x4 m4 = *reinterpret_cast<const f32x4*>(s_m), l4 = *reinterpret_cast<const f32x4*>(s_l);
+    m = fmaxf(fmaxf(m4.x, m4.y), fmaxf(m4.z, m4.w));
+    o = lsum = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float e = __expf(m4[i] - m);
+        o = fmaf(e, (s_o[4 * i][lane] + s_o[4 * i + 1][lane]) + (s_o[4 * i + 2][lane] + s_o[4 * i + 3][lane]), o);
+        lsum = fmaf(e, l4[i], lsum);
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ the start
 // By one thread of every workgroup: register; the last one commits if the steps in front have run and every XCD has 32, one that has
 // waited too long (behind a withdrawn launch: at once) withdraws the launch for all.  1: all workgroups are resident; 2: nothing may be touched.
