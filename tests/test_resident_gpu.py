@@ -318,6 +318,7 @@ def test_vocabulary_beyond_the_offsets_stays_on_the_chain(zg):
     g = torch.Generator(device="cuda")
     g.manual_seed(41)
     w = {name: torch.randn(shape, generator=g, device="cuda") * 0.02 + mean for name, shape, mean, _ in synth.tensor_specs(cfg)}
+    torch.cuda.synchronize()  # (made on torch's stream)
     m.load_weights(w)
     ids = m.generate([[5]], 6)[0]
     assert not m.resident_stats()["ran"]
