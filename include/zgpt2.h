@@ -150,6 +150,8 @@ int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_n
 /* Diagnostic: number of launches of the persistent matrix-core GEMMs (four and eight waves) by the op and GPT-2 tiers so far in this
  * process (tests assert which path a Linear took; no reference counterpart). */
 unsigned long long zg_debug_gemm_launches(void);
+/* Diagnostic: the same of the kernel that takes fp32 Linears of five to fifteen rows on the matrix cores. */
+unsigned long long zg_debug_linear_few_mfma_launches(void);
 /* Diagnostic: shader-clock stamps {count, start, end} of workgroup 0 / wave 0 of the last GEMM launched with
  * ZGPT2_GEMM_DBG bit 256 (tools/microbench/gemm_bench.cpp: cycles vs wall time = the clock the chip ran at). */
 int zg_debug_gemm_stamps(unsigned long long* out, size_t n_words);

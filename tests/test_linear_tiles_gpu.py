@@ -50,21 +50,23 @@ def test_both_sides_of_the_rule(zg, m, k, n, kernel):
 
 
 @pytest.mark.parametrize("m,k,n,kernel", [
-    (4, 512, 15, "linear_few_kernel"), (5, 512, 15, "linear_few_mfma_kernel"), (15, 512, 64, "linear_few_mfma_kernel"), (16, 512, 64, "linear_tiles_kernel"),
+    (4, 512, 15, "linear_few"), (5, 512, 15, "matrix cores"), (15, 512, 64, "matrix cores"), (16, 512, 64, "linear_tiles"),
     # five to eight rows: 512 columns, 1024 of more than 2048 outputs, 1536 to 1792 of more than 1024
-    (8, 248, 6144, "linear_few_mfma_kernel"), (8, 248, 6145, "gemv"), (8, 256, 6145, "linear_few_mfma_kernel"), (8, 520, 33, "linear_few_kernel"),
-    (8, 520, 2048, "linear_few_kernel"), (8, 520, 2049, "linear_few_mfma_kernel"), (8, 1024, 2049, "linear_few_mfma_kernel"), (8, 1032, 2049, "linear_few_kernel"),
-    (8, 1528, 1025, "linear_few_kernel"), (8, 1536, 1024, "linear_few_kernel"), (8, 1536, 1025, "linear_few_mfma_kernel"),
-    (5, 1792, 1025, "linear_few_mfma_kernel"), (5, 1800, 1025, "linear_few_kernel"),
+    (8, 248, 6144, "matrix cores"), (8, 248, 6145, "gemv"), (8, 256, 6145, "matrix cores"), (8, 520, 33, "linear_few"),
+    (8, 520, 2048, "linear_few"), (8, 520, 2049, "matrix cores"), (8, 1024, 2049, "matrix cores"), (8, 1032, 2049, "linear_few"),
+    (8, 1528, 1025, "linear_few"), (8, 1536, 1024, "linear_few"), (8, 1536, 1025, "matrix cores"),
+    (5, 1792, 1025, "matrix cores"), (5, 1800, 1025, "linear_few"),
     # nine to fifteen: 128 to 1024 columns, to 1792 of up to 4096 outputs
-    (9, 120, 40, "gemv"), (9, 128, 40, "linear_few_mfma_kernel"), (9, 1024, 4097, "linear_few_mfma_kernel"), (9, 1088, 4096, "linear_few_mfma_kernel"),
-    (9, 1088, 4097, "linear_tiles_kernel"), (15, 1792, 4096, "linear_few_mfma_kernel"), (15, 1856, 40, "linear_tiles_kernel"), (15, 1800, 40, "gemv")])
+    (9, 120, 40, "gemv"), (9, 128, 40, "matrix cores"), (9, 1024, 4097, "matrix cores"), (9, 1088, 4096, "matrix cores"),
+    (9, 1088, 4097, "linear_tiles"), (15, 1792, 4096, "matrix cores"), (15, 1856, 40, "linear_tiles"), (15, 1800, 40, "gemv")])
 def test_which_kernel_takes_few_rows(zg, m, k, n, kernel):
     run(1, 768, 768)  # (a general kernel; the ragged ones among them leave the note as it is)
+    before = zg.zg_debug_linear_few_mfma_launches()
     w, b, x, y = run(m, k, n)
     name = C.create_string_buffer(160)
     _lib.check(zg.zg_debug_last_kernel(name, 160))
-    assert name.value.decode() == kernel or kernel == "gemv" and name.value.decode().startswith(kernel), name.value
+    assert zg.zg_debug_linear_few_mfma_launches() - before == (kernel == "matrix cores")
+    assert name.value.decode().startswith("linear_few" if kernel == "matrix cores" else kernel), name.value
     assert_ref_close(oracle.linear_forward(k, n, w, b, x), y, f"Linear {m}x{k}x{n}", scale_floor=2e-6)
 
 

@@ -621,6 +621,7 @@ int zg_debug_prefill_route(int force_kernel, int slices) {
 }
 
 unsigned long long zg_debug_gemm_launches(void) { return gemm_mfma_launch_count(); }
+unsigned long long zg_debug_linear_few_mfma_launches(void) { return linear_few_mfma_launch_count(); }
 int zg_debug_gemm_stamps(unsigned long long* out, size_t n_words) { return gemm_debug_stamps(out, n_words); }
 
 int zg_f32_to_bf16(const float* src, uint16_t* dst_device, size_t len) {

@@ -8,6 +8,7 @@
 #include "zg_kernels.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace zg {
 
@@ -350,6 +351,9 @@ int launch_linear_tiles(const float* X, const float* W, const float* bias, float
     return ZG_OK;
 }
 
+static std::atomic<unsigned long long> g_few_mfma_launches{0};
+unsigned long long linear_few_mfma_launch_count() { return g_few_mfma_launches.load(std::memory_order_relaxed); }
+
 // linear_few_mfma_kernel, or linear_few_kernel and the tiles; a call's us on the same buffers, this : those.  Nine rows to fifteen (12 rows 768 -> 768 14.3 : 18.8,
 // 768 -> 3072 14.3 : 20.6, 1600 -> 1600 18.4 : 20.7; K in no whole 64s, as 520 -> 600, 13.1 : 25.8): the tiles, which have sixteen rows and more,
 // catch up where long rows make a compute unit's share long (16 rows 1600 -> 4800 25.0 : 24.0, 3072 -> 768 21.4 : 22.4, 6400 -> 1600 35.5 : 30.7);
@@ -384,7 +388,8 @@ int launch_linear_few(const float* X, const float* W, const float* bias, float* 
         else if (each == 3) ZG_FEW(3);
         else ZG_FEW(4);
 #undef ZG_FEW
-        note_kernel("linear_few_mfma_kernel");
+        note_kernel("linear_few_kernel");  // (the two have one name; the count says which)
+        g_few_mfma_launches.fetch_add(1, std::memory_order_relaxed);
         ZG_HIP(hipGetLastError());
         return ZG_OK;
     }

@@ -209,6 +209,7 @@ unsigned long long gemm_mfma_launch_count();  // launches of the persistent MFMA
 void gemm_note_launch();
 // fp32 Linears X [M][K], W [N][K] of few rows and of a medium number of rows (linear_tiles.hip).  Two to fifteen rows: K a multiple of 8.
 bool linear_few_ok(size_t M, size_t N, size_t K);
+unsigned long long linear_few_mfma_launch_count();  // launches of linear_few_mfma_kernel so far
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 // Nine rows and more: K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N floats where that is more than one slice.
 bool linear_tiles_pay(size_t M, size_t N);
