@@ -1,7 +1,8 @@
 """Greedy decode as resident kernels (zig_gpt2_amd/csrc/decode_resident.hip: one sequence, decode_resident_batch.hip: two to eight)
 against the launch chain they replace and the oracle: the edges of their shapes (64 positions of a workgroup, 64 steps of a launch,
 vocabularies that do not divide by the 256 workgroups, XCDs with no, one and two heads, sequences a tile of terms is not filled by),
-what a generation leaves behind, a withdrawn launch and a wait that runs out."""
+what a generation leaves behind, prompts token by token, values that are not finite, other streams, a withdrawn launch
+(decode_rest.hip runs its steps) and a wait that runs out."""
 import ctypes as C
 import time
 
@@ -247,6 +248,53 @@ def test_launch_withdrawn_behind_others(zg, monkeypatch, name, batch, f32, launc
     tok = want[:, -1]
     assert rel(m.forward(steps + 1, tok), chain.forward(steps + 1, tok)) < 2e-6
     m.close()
+    chain.close()
+
+
+@pytest.mark.parametrize("name,batch,f32", [("384", 1, False), ("768", 1, True), ("512", 8, False), ("768-odd", 2, False)])
+def test_rest_on_the_workgroups_that_came_first(zg, monkeypatch, name, batch, f32):
+    """The list of members closed at once: any number of workgroups, another one every time, run the steps."""
+    cfg = SHAPES[name]
+    w = synth.make_weights(cfg, seed=45, bf16=not f32)
+    p = [synth.rand_tokens(450 + b, 1 + b % 4, cfg.vocab_size) for b in range(batch)]
+    chain = make(monkeypatch, cfg, w, False, batch=batch, weights_f32=f32)
+    want = chain.generate(p, 40)
+    monkeypatch.setenv("ZGPT2_RESIDENT_WITHDRAW", "0")
+    monkeypatch.setenv("ZGPT2_REST_PATIENCE", "0")
+    members = []
+    for _ in range(6):
+        m = make(monkeypatch, cfg, w, True, batch=batch, weights_f32=f32)
+        assert np.array_equal(m.generate(p, 40), want), members
+        st = m.resident_stats()
+        assert st["rest_steps"] == 40
+        members.append(st["rest_workgroups"])
+        assert rel(m.hidden(), chain.hidden()) < 2e-6 and np.array_equal(m.argmax(), chain.argmax())
+        m.close()
+    print("members", members)
+    chain.close()
+
+
+@pytest.mark.parametrize("name,batch,f32", [("384", 1, False), ("768", 1, True), ("384", 6, False), ("768", 2, False)])
+@pytest.mark.parametrize("withdraw", [-1, 0, 1])
+def test_prompts_token_by_token(zg, monkeypatch, name, batch, f32, withdraw):
+    """Handles without the prompt pass: launches that end inside the prompts, whole launches of nothing else, the first pick behind them."""
+    cfg = SHAPES[name]
+    w = synth.make_weights(cfg, seed=46, bf16=not f32)
+    chain = make(monkeypatch, cfg, w, False, batch=batch, weights_f32=f32, prefill=False)
+    monkeypatch.setenv("ZGPT2_RESIDENT_WITHDRAW", str(withdraw))
+    for plen, steps in ((70, 64), (70, 65), (70, 70), (64, 71), (129, 130), (129, 128), (128, 130)):
+        res = make(monkeypatch, cfg, w, True, batch=batch, weights_f32=f32, prefill=False)
+        p = [synth.rand_tokens(460 + plen + b, plen - 5 * (b % 3), cfg.vocab_size) for b in range(batch)]
+        a, b = res.generate(p, steps), chain.generate(p, steps)
+        st = res.resident_stats()
+        assert st["ran"] and st["rest_steps"] == (0 if withdraw < 0 or 64 * withdraw >= steps else steps - 64 * withdraw), st
+        assert np.array_equal(a, b), (plen, steps)
+        assert rel(res.hidden(), chain.hidden()) < 2e-6, (plen, steps)
+        if steps > min(len(q) for q in p):
+            assert np.array_equal(res.argmax(), chain.argmax())
+        if steps < cfg.context_size:
+            assert rel(res.forward(steps + 1, a[:, -1]), chain.forward(steps + 1, a[:, -1])) < 2e-6, (plen, steps)
+        res.close()
     chain.close()
 
 

@@ -135,6 +135,7 @@ struct zg_gpt {
     size_t res_words_bytes;
     ResidentCtl* res_ctl;
     float* rest_best;                // decode_rest_kernel's picks by workgroup
+    unsigned rest_patience;          // its first workgroup's (0: the test of few members)
     unsigned* res_withdrawn;         // pinned
     // a generation in flight between gen_begin and gen_end (zg_gpt_generate_enqueue / _many)
     size_t gen_pos, gen_n, gen_min_prompt, gen_since_sync;
@@ -779,6 +780,7 @@ void setup_resident(zg_gpt* g) {
     *g->res_withdrawn = 0;
     g->res_start_limit = (unsigned)env_int("ZGPT2_RESIDENT_START", 1 << 14);  // about 10 ms
     g->res_none_at = env_int("ZGPT2_RESIDENT_WITHDRAW", -1);
+    g->rest_patience = (unsigned)env_int("ZGPT2_REST_PATIENCE", 1 << 11);
     if (g->batch > 8 || (g->batch > 1 && g->wt != WT_BF16) || g->kv_mode != 0 || g->stream != nullptr || g->parent != nullptr || (g->flags & ZG_GPT_NO_GRAPH)) return;
     if (!resident_shape(g->cfg.n_embed, g->cfg.n_heads, g->cfg.context_size, g->cfg.n_layer, g->cfg.vocab_size)) return;
     // (a prefetcher that is asked for by name asks for the launches that it fetches for)
@@ -853,7 +855,7 @@ int enqueue_resident(zg_gpt* g, hipStream_t s) {
 
 // Behind the last resident launch: the steps that withdrawn launches left
 int enqueue_rest(zg_gpt* g, hipStream_t s) {
-    const RestArgs a{resident_args(g, 0, g->gen_n), (int)g->cfg.n_embed, g->q, g->part, g->h4, g->rest_best, reinterpret_cast<int*>(g->rest_best + decode_rest_floats() / 2)};
+    const RestArgs a{resident_args(g, 0, g->gen_n), (int)g->cfg.n_embed, g->q, g->part, g->h4, g->rest_best, reinterpret_cast<int*>(g->rest_best + decode_rest_floats() / 2), g->rest_patience};
     return launch_decode_rest(a, g->wt, s);
 }
 

@@ -15,7 +15,6 @@ namespace {
 using namespace resident;
 constexpr int kWaves = 8, kGroups = 128;  // (256: barriers cost more than their loads gain, 1.00 : 0.79 ms a token; 64: 0.96)
 constexpr unsigned kClosed = 1u << 31;
-constexpr unsigned kPatience = 1u << 11;  // polls of the first workgroup, about a microsecond each, while not all have started
 
 template <typename WT>
 __device__ __forceinline__ void load8(const WT* p, float (&v)[8]) {
@@ -57,7 +56,7 @@ __global__ __launch_bounds__(64 * kWaves) void decode_rest_kernel(const RestArgs
         if (s_from < (unsigned)a.s1 && __hip_atomic_load(a.fault, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM) == 0u) {
             s_id = __hip_atomic_fetch_add(&ctl->joined, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if (s_id == 0u) {
-                for (unsigned n = 0; n < kPatience && __hip_atomic_load(&ctl->joined, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gridDim.x; ++n) __builtin_amdgcn_s_sleep(2);
+                for (unsigned n = 0; n < p.patience && __hip_atomic_load(&ctl->joined, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gridDim.x; ++n) __builtin_amdgcn_s_sleep(2);
                 s_n = __hip_atomic_fetch_or(&ctl->joined, kClosed, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 __hip_atomic_store(&ctl->members, s_n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             } else if (!(s_id & kClosed)) {  // (the first one is running and closes the list without waiting for anyone)

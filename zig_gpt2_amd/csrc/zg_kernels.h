@@ -364,6 +364,7 @@ struct RestArgs {
     float *q, *z, *h;  // [batch][n_embed], [batch][n_embed], [batch][4 n_embed]
     float* best_v;     // decode_rest_floats() in all
     int* best_i;
+    unsigned patience;  // polls of the first workgroup, about a microsecond each, while not all have started
 };
 size_t decode_rest_floats();
 int launch_decode_rest(const RestArgs& a, int weight_type, hipStream_t s);
