@@ -1,6 +1,6 @@
 // Greedy decode of ONE sequence as a resident kernel: the whole chip stays inside one launch for up to 64 tokens, some 3.5 ms (GPT.forward + the
 // argmax of generate, src/main.zig:178-195, :322-342), and the phases of a Block meet through tagged words instead of launch
-// boundaries.  Measured: GPT-2 124M 208 -> 110 us a token (256 tokens; 1024: 207 -> 122), fp32 weights 277 -> 149, the char model 92 -> 37.
+// boundaries.  Measured: GPT-2 124M 208 -> 110 us a token (256 tokens; 1024: 207 -> 121), fp32 weights 277 -> 147, the char model 92 -> 36.
 //
 // What bounded it: a step was 62 dependent launches (124M) of 2.7-4 us each, most of that the boundary, the first loads behind it
 // and the fetch of weights nobody could request ahead.  What a hand-over inside a kernel costs depends on how far it goes:

@@ -1,6 +1,6 @@
 // Greedy decode of two to eight sequences in lock step as a resident kernel: decode_resident.hip's cut of a Block over the XCDs and its
 // hand-overs, the products on the matrix cores.  A generation alone, launches -> here: GPT-2 124M, 8 sequences, 75 + 181 tokens 57.7 -> 35.8 ms
-// (33 + 991 322 -> 218), 4 sequences, 40 + 216 60.1 -> 34.3, 2 sequences 244 -> 133 us a step; char model, 8 sequences, 256 tokens 36.8 -> 15.3 ms.  bf16 weights: an activation travels as
+// (33 + 991 322 -> 218), 4 sequences, 40 + 216 60.1 -> 34.3, 2 sequences 244 -> 133 us a step; char model, 8 sequences, 256 tokens 36.8 -> 15.5 ms.  bf16 weights: an activation travels as
 // the exact three-term bf16 split of its fp32 value (zg_common.h split3_pk), split once by the thread that makes it, all three terms and a
 // tag of 16 bits in ONE word; a wave multiplies 16 weight rows with the terms of all sequences (v_mfma_f32_16x16x32_bf16: columns of a
 // product are terms x sequences), the waves split K and meet in the LDS.  A wave polls for the words its own lanes multiply, laid out as they
