@@ -1,0 +1,103 @@
+"""fp32 Linears of many rows and 512 columns or more: three products of two-term fp16 planes on the persistent GEMM (gemm_s4.hip), whose rows carry
+exponents of their own.  Tile edges, ragged widths, one and several tiles a workgroup, both sides of the column rule, rows of very different
+sizes, rows of zeros, of the smallest and of the largest values, values that are not finite.
+
+The bound, element by element, is what three products of such terms can be off: 2^-21 of the sum of |x w| for the terms (2^-23 each and 2^-22
+for the product that is left out), 2^-24 of it for each of the K / 8 additions of the matrix cores, and what values far below their row's
+largest lose, 2^-38 of the two largest values for each product."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from zig_gpt2_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def last_kernel(zg):
+    name = C.create_string_buffer(160)
+    _lib.check(zg.zg_debug_last_kernel(name, 160))
+    return name.value.decode()
+
+
+def draw(m, k, n, spread=0):
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m + 3 * n + 7 * k)
+    x, w, b = (torch.randn(*s, generator=g, device="cuda") for s in ((m, k), (n, k), (n,)))
+    if spread:
+        x *= torch.exp2(torch.randint(-spread, spread, (m, 1), generator=g, device="cuda").float())
+        w *= torch.exp2(torch.randint(-spread, spread, (n, 1), generator=g, device="cuda").float())
+    return x, w, b
+
+
+def forward(x, w, b):
+    y = torch.full((x.shape[0], w.shape[0]), 7.0, device="cuda")
+    torch.cuda.synchronize()  # (the library launches on a stream of its own)
+    ops.Linear(x.shape[1], w.shape[0], w, b).forward(x, y)
+    torch.cuda.synchronize()
+    return y
+
+
+def check(x, w, b, y):
+    k = x.shape[1]
+    ref = x.double() @ w.double().T
+    size = x.abs().double() @ w.abs().double().T
+    top = x.abs().amax(1).double()[:, None] * w.abs().amax(1).double()[None]
+    bound = (2.0 ** -21 + k / 8 * 2.0 ** -24) * size + k * 2.0 ** -38 * top + 2.0 ** -149
+    if b is not None:
+        ref, bound = ref + b.double(), bound + 2.0 ** -23 * b.abs().double()
+    over = ((y.double() - ref).abs() / bound).max().item()
+    assert over <= 1.0, over
+    return ((y.double() - ref).norm() / ref.norm()).item()
+
+
+@pytest.mark.parametrize("m,k,n", [(4096, 512, 3072), (4097, 576, 3071), (1537, 768, 3073), (8191, 640, 1601), (2047, 1600, 1601), (6001, 3072, 769), (12300, 512, 1029)])
+def test_tile_edges(zg, m, k, n):
+    x, w, b = draw(m, k, n)
+    b = None if n % 2 else b
+    before = zg.zg_debug_gemm_launches()
+    y = forward(x, w, b)
+    assert zg.zg_debug_gemm_launches() == before + 1 and last_kernel(zg) == "gemm_s4_kernel"
+    # (2-norm: what a chain of K products in two halves and the terms leave, each seen in the comments of the kernels, and a third more)
+    assert check(x, w, b, y) <= 1.33 * ((1.2e-7 * (k / 768) ** 0.5) ** 2 + 0.75e-7 ** 2) ** 0.5
+
+
+@pytest.mark.parametrize("wgs", ["3", "16"])
+def test_many_tiles_a_workgroup(zg, monkeypatch, wgs):
+    monkeypatch.setenv("ZGPT2_GEMM_WGS", wgs)  # the ring of exponents goes round several times
+    x, w, b = draw(2100, 768, 2400, spread=12)
+    check(x, w, b * 0, forward(x, w, b * 0))
+
+
+def test_rows_of_any_size(zg):
+    x, w, _ = draw(2048, 768, 3072, spread=40)
+    x[5] = 0.0
+    w[7] = 0.0
+    x[9] *= 2.0 ** -100  # subnormal products and results
+    x[11, 3] = 3.0e38
+    x[13] = 1e-40
+    w[15] = 1e-41
+    y = forward(x, w, None)
+    assert torch.equal(y[5], torch.zeros_like(y[5])) and torch.equal(y[:, 7], torch.zeros_like(y[:, 7]))
+    finite = (x.double() @ w.double().T).abs().amax(1) < 3e38
+    check(x[finite], w, None, y[finite])
+
+
+def test_values_that_are_not_finite_stay_in_their_row(zg):
+    x, w, b = draw(2048, 768, 3072)
+    clean = forward(x, w, b)
+    x[3, 100], x[700, 5], x[2047, 767] = float("nan"), float("inf"), -float("inf")
+    y = forward(x, w, b)
+    bad = torch.zeros(2048, dtype=torch.bool, device="cuda")
+    bad[[3, 700, 2047]] = True
+    assert torch.equal(y[~bad], clean[~bad]) and not torch.isfinite(y[bad]).any()
+
+
+def test_column_rule(zg):
+    for k, err in ((448, 1.33 * 1.58e-7 * (448 / 768) ** 0.5), (512, 1.33 * 1.25e-7)):  # three exact terms below 512 columns
+        x, w, b = draw(4096, k, 3072)
+        y = forward(x, w, None)
+        assert last_kernel(zg) == "gemm_s4_kernel"
+        assert check(x, w, None, y) <= err

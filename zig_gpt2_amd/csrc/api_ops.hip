@@ -238,7 +238,10 @@ struct CallGuard {
 
 // Linear.forward on the persistent matrix-core GEMMs, for the sizes that fill the chip with their tiles (16 rows at least; the rule in front
 // is linear_tiles_ok's; ops.zig:21-46 with M = inputs.len / in_features, :22).
-// The op tier is fp32 in, fp32 out, arbitrary fp32 weights: both operands are split EXACTLY into three bf16
+// The op tier is fp32 in, fp32 out, arbitrary fp32 weights.  From 512 columns on both operands become two fp16 planes of rows scaled by powers
+// of two (zg_common.h split2_f16), one pass over both, and the GEMM sums three products: 8192 x 768 x 3072 takes 150 us where six take 214
+// (the GEMM 132 and 190 under the tracer: both at the chip's power limit, where an fp16 product costs more than a bf16 one).
+// Below, and where the four-wave GEMM's arguments end, both operands are split EXACTLY into three bf16
 // planes (x = hi + mid + lo, 3 x 8 mantissa bits) and the GEMM sums the six plane products whose weight is
 // above 2^-24 of the leading one — every bf16 x bf16 product is exact in fp32 and accumulation is fp32, i.e. the
 // result is fp32-sgemm grade (measured against the oracle at the reference's tolerance in the tests).
@@ -254,6 +257,22 @@ static bool linear_mfma_ok(size_t in_f, size_t out_f, size_t m, size_t arena_lef
 
 static int linear_mfma(Call& call, size_t in_f, size_t out_f, const float* w, const float* bias, const float* x,
                        size_t m, float* y) {
+    GemmPlanes p2{};
+    p2.lda = p2.ldb = (int)(2 * in_f);
+    p2.kpp = (int)(in_f / 64);
+    p2.npairs = 3;  // (x plane, w plane): lo*hi, hi*lo, hi*hi
+    p2.pa_bits = 0x001u;
+    p2.pb_bits = 0x010u;
+    if (in_f >= kSplit2MinK && gemm_s4_args_ok(p2, (int)out_f)) {
+        uint16_t *xs, *ws;
+        int *xe, *we;
+        ZG_TRY(call.scratch(m * in_f * 2, &xs));
+        ZG_TRY(call.scratch(out_f * in_f * 2, &ws));
+        ZG_TRY(call.scratch(m, &xe));
+        ZG_TRY(call.scratch(out_f, &we));
+        ZG_TRY(launch_split2(Split2Job{x, xs, xe, (int)m}, Split2Job{w, ws, we, (int)out_f}, (int)in_f, call.stream()));
+        return launch_gemm_s4_f16(xs, ws, bias, y, (int)m, (int)out_f, p2, (int)out_f, PlaneExps{xe, we, true}, call.stream());
+    }
     bf16_t *xp, *wp;
     ZG_TRY(call.scratch(m * in_f * 3, &xp));
     ZG_TRY(call.scratch(out_f * in_f * 3, &wp));
@@ -280,7 +299,7 @@ static size_t gemv_rows(size_t in_f) {
 static bool linear_tiles_ok(size_t in_f, size_t out_f, size_t m, size_t arena_left) {
     if (in_f > 8192 ? !linear_mfma_ok(in_f, out_f, m, arena_left) : m <= gemv_rows(in_f)) return false;
     if (in_f < 128 || in_f % 64 != 0 || m >= (1u << 30) / in_f || out_f >= (1u << 30) / in_f) return false;
-    if (!linear_tiles_pay(m, out_f)) return false;
+    if (!linear_tiles_pay(m, out_f, in_f)) return false;
     const int slices = linear_tiles_slices(m, out_f, in_f);
     return slices == 1 || (size_t)slices * m * out_f * sizeof(float) + 1024 <= arena_left;
 }

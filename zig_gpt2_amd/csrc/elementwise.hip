@@ -228,6 +228,47 @@ __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ i
     }
 }
 
+// Rows of two matrices -> planes of fp16 (zg_common.h split2_f16), a wave a row, its values in registers between the search of the largest and the split
+// (NV quads a lane; rows beyond are read again).  One pass over memory: 8192 x 768 and 3072 x 768 together 69 MB.
+template <int NV>
+__global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const Split2Job jb, int K) {
+    const int lane = threadIdx.x & 63;
+    int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (row >= ja.rows + jb.rows) return;
+    const bool second = row >= ja.rows;
+    if (second) row -= ja.rows;
+    const float* x = (second ? jb.in : ja.in) + (size_t)row * K;
+    uint16_t* o = (second ? jb.out : ja.out) + (size_t)row * 2 * K;
+    int* e = (second ? jb.exps : ja.exps) + row;
+    const int n4 = K >> 2;
+    f32x4 v[NV];
+    uint32_t top = 0;
+    auto widen = [&](const f32x4& q) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) top = max(top, __float_as_uint(q[c]) & 0x7fffffffu);
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = *reinterpret_cast<const f32x4*>(x + 4 * min(lane + 64 * i, n4 - 1));
+#pragma unroll
+    for (int i = 0; i < NV; ++i) widen(v[i]);
+    for (int i = lane + 64 * NV; i < n4; i += 64) widen(*reinterpret_cast<const f32x4*>(x + 4 * i));
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
+    const int up = split2_exp(top);
+    if (lane == 0) *e = -up;
+    auto leave = [&](int i, const f32x4& q) {
+        uint32_t h0, h1, l0, l1;
+        split2_f16(ldexpf(q.x, up), ldexpf(q.y, up), h0, l0);
+        split2_f16(ldexpf(q.z, up), ldexpf(q.w, up), h1, l1);
+        *reinterpret_cast<u32x2*>(o + 4 * i) = u32x2{h0, h1};
+        *reinterpret_cast<u32x2*>(o + K + 4 * i) = u32x2{l0, l1};
+    };
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        if (lane + 64 * i < n4) leave(lane + 64 * i, v[i]);
+    for (int i = lane + 64 * NV; i < n4; i += 64) leave(i, *reinterpret_cast<const f32x4*>(x + 4 * i));
+}
+
 __device__ __forceinline__ float load_emb(const void* w, int wt, size_t off) {
     if (wt == WT_BF16) return __uint_as_float((uint32_t)reinterpret_cast<const bf16_t*>(w)[off] << 16);
     return reinterpret_cast<const float*>(w)[off];
@@ -635,6 +676,15 @@ int launch_kv_clear_tail(void* base, int n_caches, size_t cache_stride, size_t p
     ZG_REQUIRE(row_bytes % 64 == 0 && strips < 65536 * 32 && n_caches < 65536, ZG_ERR_UNSUPPORTED, "kv clear: %d-byte rows, %d strips", row_bytes, strips);
     hipLaunchKernelGGL(kv_clear_tail_kernel, dim3(strips, n_caches), dim3(256), 0, s, reinterpret_cast<char*>(base), cache_stride, plane_off, row_bytes,
                        strips, ctx, from_row);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s) {
+    ZG_REQUIRE(K > 0 && K % 4 == 0 && a.rows >= 0 && b.rows >= 0 && a.rows + b.rows > 0, ZG_ERR_UNSUPPORTED, "split2: %d + %d rows of %d", a.rows, b.rows, K);
+    const dim3 grid((unsigned)((a.rows + b.rows + 3) / 4));
+    if (K <= 768) split2_kernel<3><<<grid, 256, 0, s>>>(a, b, K);
+    else split2_kernel<8><<<grid, 256, 0, s>>>(a, b, K);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

@@ -40,6 +40,8 @@ typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16v;
 typedef __attribute__((ext_vector_type(4))) float f32x4v;
 typedef __attribute__((ext_vector_type(2))) float f32x2v;
+typedef __attribute__((ext_vector_type(4))) int i32x4v;
+typedef __attribute__((ext_vector_type(8))) uint32_t u32x8v;
 
 // gelu(x) = x / (1 + exp(-2u)), u = x * 0.7978845608 * (1 + 0.044715 x^2)  (src/ops.zig:225); the -2 log2(e)
 // factor is folded into the polynomial so that the exponential is a bare v_exp_f32
@@ -67,6 +69,9 @@ struct S4 {
     // bf16 epilogue staging, per wave: one 32-row m-tile x the wave's BN / 2 columns, rows padded by 16 B
     static constexpr int ST_ROW = NT * 64 + 16, ST_WAVE = 32 * ST_ROW, ST_OFF = BIAS_OFF + 2 * 1024;
     static constexpr int LDS = ST_OFF + 4 * ST_WAVE;      // 140 / 164 KiB
+    // F16: a ring of three tiles' [bias | column exponents | row exponents] (1 KiB each; read at a tile's end, when the tile after
+    // the next asks for its own) in place of the two bias rows in front of the staging
+    static constexpr int EXP_OFF = LDS, EXP_TILE = 3 * 1024, LDS_F16 = EXP_OFF + 3 * EXP_TILE;
     static constexpr int PB = BN / 32;          // B pieces (8 rows x 128 B) per wave per K-step: 6 or 8
     static constexpr int W3 = 8 + PB;           // pieces that may still be in flight when A half 1 of this K-step must have landed
 };
@@ -122,9 +127,10 @@ __device__ __forceinline__ void read_frag_b(bf16x8& f, const unsigned (&b_addr)[
 // the compiler keeps nothing of its own there across any of them.  Hazards are ours too: MFMA result ->
 // v_accvgpr_read needs the pipeline drained (s_nop in acc_settle), v_accvgpr_write -> MFMA source C two wait states.
 #define ZG_ACC_CLOBBERS "a0","a1","a2","a3","a4","a5","a6","a7","a8","a9","a10","a11","a12","a13","a14","a15","a16","a17","a18","a19","a20","a21","a22","a23","a24","a25","a26","a27","a28","a29","a30","a31","a32","a33","a34","a35","a36","a37","a38","a39","a40","a41","a42","a43","a44","a45","a46","a47","a48","a49","a50","a51","a52","a53","a54","a55","a56","a57","a58","a59","a60","a61","a62","a63","a64","a65","a66","a67","a68","a69","a70","a71","a72","a73","a74","a75","a76","a77","a78","a79","a80","a81","a82","a83","a84","a85","a86","a87","a88","a89","a90","a91","a92","a93","a94","a95","a96","a97","a98","a99","a100","a101","a102","a103","a104","a105","a106","a107","a108","a109","a110","a111","a112","a113","a114","a115","a116","a117","a118","a119","a120","a121","a122","a123","a124","a125","a126","a127","a128","a129","a130","a131","a132","a133","a134","a135","a136","a137","a138","a139","a140","a141","a142","a143","a144","a145","a146","a147","a148","a149","a150","a151","a152","a153","a154","a155","a156","a157","a158","a159","a160","a161","a162","a163","a164","a165","a166","a167","a168","a169","a170","a171","a172","a173","a174","a175","a176","a177","a178","a179","a180","a181","a182","a183","a184","a185","a186","a187","a188","a189","a190","a191"
-template <int BASE>
+template <int BASE, bool F16>
 __device__ __forceinline__ void mfma_acc(const bf16x8& a_op, const bf16x8& b_op) {
-    asm volatile("v_mfma_f32_32x32x16_bf16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
+    if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
+    else asm volatile("v_mfma_f32_32x32x16_bf16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
 }
 template <int BASE>
 __device__ __forceinline__ void acc_read8(float* v) {  // eight accumulator registers, one statement
@@ -207,10 +213,12 @@ __device__ __forceinline__ void read_b_all(bf16x8 (&fb)[4][NT], const unsigned (
 //   S4_SPLIT3   bias + GELU, then the exact three-term bf16 split as planes C[M][3N] = [hi | mid | lo]  (src/main.zig:79-80 feeding
 //               the next Linear's A operand)
 
-template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false>
+// F16: the planes are the two-term fp16 split of rows scaled by powers of two (zg_common.h split2_f16): the finished sums are scaled back by
+// the exponents of their row and column, and the bias is added behind that (the accumulators start at zero).
+template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
 __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                          const float* __restrict__ bias, void* __restrict__ C, int M, int N,
-                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa) {
+                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex) {
     // All 14 dwords of the arguments are preloaded into SGPRs at wave launch (zg_common.h ZG_PIN): the first version passed the
     // plane description and the tile counts behind them and began with a scalar round trip to the kernarg segment — cold for
     // every launch — before its first DMA.  p0 = lda | ldb << 16; p1 = ldc | K-steps per plane << 20 | plane pairs << 28;
@@ -304,9 +312,31 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     // allocator shuffle accumulators inside the K loop.
     const __amdgpu_buffer_rsrc_t rbias =
         __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias != nullptr ? (unsigned)N * 4u : 0u, 0x00020000);
-    int tile_par = 0;  // parity of the current tile: its bias row is in buffer tile_par, the next tile's in the other one
-    auto fetch_bias = [&](int n0_, int par) {
-        if (wave == 0) {
+    // (F16: the exponents of the tile's columns and rows travel with it)
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rcexp = __builtin_amdgcn_make_buffer_rsrc((void*)ex.w, 0, F16 ? (unsigned)N * 4u : 0u, 0x00020000);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rrexp =
+        __builtin_amdgcn_make_buffer_rsrc((void*)ex.a, 0, F16 ? (ex.a_each ? (unsigned)M * 4u : 4u) : 0u, 0x00020000);
+    int tile_par = 0;  // parity of the current tile: its bias row is in buffer tile_par, the next tile's in the other one (F16: of three)
+    auto par_after = [&](int par, int by) {
+        if constexpr (!F16) return par ^ (by & 1);
+        else return par + by >= 3 ? par + by - 3 : par + by;
+    };
+    auto fetch_bias = [&](int n0_, int par, [[maybe_unused]] int m0_) {
+        if constexpr (F16) {
+            const unsigned at = lds_base + P::EXP_OFF + par * P::EXP_TILE;
+            if (wave == 0)
+#pragma unroll
+                for (int p = 0; p < P::BN / 64; ++p) {
+                    const unsigned col = (unsigned)(n0_ + 64 * p) * 4u;
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rbias, to_lds(at + p * 256), 4, (unsigned)lane * 4u, col, 0, 0);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rcexp, to_lds(at + 1024 + p * 256), 4, (unsigned)lane * 4u, col, 0, 0);
+                }
+            if (wave == 1)
+#pragma unroll
+                for (int p = 0; p < 4; ++p)
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rrexp, to_lds(at + 2048 + p * 256), 4, ex.a_each ? (unsigned)lane * 4u : 0u,
+                                                             ex.a_each ? (unsigned)(m0_ + 64 * p) * 4u : 0u, 0, 0);
+        } else if (wave == 0) {
 #pragma unroll
             for (int p = 0; p < P::BN / 64; ++p)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rbias, to_lds(lds_base + P::BIAS_OFF + par * 1024 + p * 256), 4, (unsigned)lane * 4u,
@@ -395,6 +425,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         for (int e = 0; e < 8; ++e) zop[e] = (__bf16)0.0f;
         static_for<NT>([&](auto JT) {
             constexpr int j = decltype(JT)::value;
+            if constexpr (F16) {
+                const f32x4v z = {0.0f, 0.0f, 0.0f, 0.0f};
+                acc_init4<16 * (0 * NT + j), 16 * (1 * NT + j), 16 * (2 * NT + j), 16 * (3 * NT + j)>(zop, z, z, z, z);
+                return;
+            }
             const unsigned baddr_l = baddr;
             f32x4v b4[4];  // columns 32 j + 8 g + 4 hh + {0..3}: registers 4 g .. 4 g + 3 of the tile
 #pragma unroll
@@ -547,7 +582,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 if constexpr (m == NT) asm volatile("s_waitcnt lgkmcnt(%0)" ::"i"(mine) : "memory");
                 if constexpr (m == 0 || m == NT) ZG_SB();
             }
-            mfma_acc<16 * ((h * 2 + i) * NT + j)>(fb[X][ks][j], fa[cb][i]);
+            mfma_acc<16 * ((h * 2 + i) * NT + j), F16>(fb[X][ks][j], fa[cb][i]);
             gap(MT);
         };
         mma(Ic<0>{});
@@ -571,6 +606,34 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         step(XT, Ic<6>{});
         step(XT, Ic<7>{});
         s1 = s2;
+    };
+
+    // F16: half way through the leading products the sums leave their leading eight bits aside and go on with the rest (both exact), so that the second
+    // half is rounded at its own size: with 11-bit terms a chain of 768 products is 1.71e-7 off, in two halves 1.2e-7, which makes room for
+    // what the split leaves (0.75e-7); three exact bf16 terms in one chain are 1.58e-7 off.  8192 x 768 x 3072: 136 us of a call without, 150 with.
+    // (always_inline: left to itself the compiler keeps this in memory)
+    [[maybe_unused]] u32x8v aside[F16 ? 4 * NT : 1] = {};
+    auto set_aside = [&]() __attribute__((always_inline)) {
+        if constexpr (F16) {
+            acc_settle();
+            static_for<4 * NT>([&](auto QT) {
+                constexpr int q = decltype(QT)::value;
+                float av[16];
+                acc_read16<16 * q>(av);
+                u32x4 rest[4];
+                u32x8v lead;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    lead[e] = cvt_pk_bf16(av[2 * e], av[2 * e + 1]);
+                    rest[e >> 1][2 * (e & 1)] = __float_as_uint(av[2 * e] - bf16_lo(lead[e]));
+                    rest[e >> 1][2 * (e & 1) + 1] = __float_as_uint(av[2 * e + 1] - bf16_hi(lead[e]));
+                }
+                aside[q] = lead;
+                acc_write16<16 * q>(rest);
+            });
+            asm volatile("s_nop 7" ::: ZG_ACC_CLOBBERS);  // v_accvgpr_write -> MFMA source C
+            ZG_SB();
+        }
     };
 
     // ---- epilogue of one tile, straight from the registers: lane (l31, hh) holds output row l31 of each 32 x 32
@@ -623,10 +686,10 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             asm volatile("s_nop 7" ::: ZG_ACC_CLOBBERS);  // v_accvgpr_write -> MFMA source C
         }
     };
-    auto epilogue = [&]() {
+    auto epilogue = [&]() __attribute__((always_inline)) {
         if (SK && role_cur == 1) {  // a producer's half tile: no epilogue, the accumulators go to its consumer
             sk_spill();
-            if (has_nxt) init_acc_from_bias(tile_par ^ 1);
+            if (has_nxt) init_acc_from_bias(par_after(tile_par, 1));
             ZG_SB();
             return;
         }
@@ -640,6 +703,35 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         // Stores go through a buffer descriptor: a row past M lies past the descriptor's end and a column past N gets an
         // out-of-range offset, so the hardware drops them — no exec masking, one straight block of code per tile.
         flush_pending();  // (a tile of fewer K-steps than pending stores)
+        // F16: 2^(row + column exponent) times the sums, plus the bias
+        [[maybe_unused]] const unsigned exps = lds_base + P::EXP_OFF + tile_par * P::EXP_TILE;
+        [[maybe_unused]] int rexp[4];
+        if constexpr (F16) {
+            const unsigned raddr = exps + 2048u + (unsigned)(wr * 128 + l31e) * 4u;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(rexp[i]) : "v"(raddr), "i"(i * 128));
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(rexp[0]), "+v"(rexp[1]), "+v"(rexp[2]), "+v"(rexp[3]));
+        }
+        [[maybe_unused]] auto scale_back = [&](auto IT, auto JT, int row_exp, float (&av)[16]) __attribute__((always_inline)) {
+            constexpr int j = decltype(JT)::value, q = decltype(IT)::value * NT + j;
+            const u32x8v lead = aside[q];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                av[2 * e] += bf16_lo(lead[e]);
+                av[2 * e + 1] += bf16_hi(lead[e]);
+            }
+            const unsigned caddr = exps + (unsigned)(wc * (P::BN / 2) + 4 * hhe) * 4u;
+            f32x4v b4[4];
+            i32x4v c4[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b4[g]) : "v"(caddr), "i"((j * 32 + 8 * g) * 4));
+                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[g]) : "v"(caddr), "i"(1024 + (j * 32 + 8 * g) * 4));
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]), "+v"(c4[0]), "+v"(c4[1]), "+v"(c4[2]), "+v"(c4[3]));
+#pragma unroll
+            for (int e = 0; e < 16; ++e) av[e] = __builtin_amdgcn_ldexpf(av[e], row_exp + c4[e >> 2][e & 3]) + b4[e >> 2][e & 3];
+        };
         const unsigned row0 = (unsigned)(m0 + wr * 128 + l31e) * (unsigned)(ldc * ESZ);
         const int col0 = n0 + wc * (P::BN / 2) + 8 * hhe;
         // bf16: a lane's runs of 4 columns go through a wave-private LDS image of the m-tile and leave as 16-B pieces of
@@ -740,6 +832,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                     asm volatile("s_nop 3" ::: "memory");
                     float av[16];
                     acc_read16<16 * (i * NT + j)>(av);
+                    if constexpr (F16) scale_back(IT, JT, rexp[i], av);
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f32x4v v4 = {av[4 * g], av[4 * g + 1], av[4 * g + 2], av[4 * g + 3]};
@@ -791,6 +884,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 asm volatile("s_nop 3" ::: "memory");
                 float av[16];
                 acc_read16<16 * (i * NT + j)>(av);
+                if constexpr (F16) scale_back(IT, JT, rexp[i], av);
                 // eight pairs, every stage over all of them: independent chains side by side
                 f32x2v x[8];
 #pragma unroll
@@ -867,7 +961,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         });
         if (has_nxt) {  // the next tile starts at its bias row — or, a consumer's half tile, at its producer's partial
             if (SK && role_nxt == 2) sk_init_from_partial();
-            else init_acc_from_bias(tile_par ^ 1);
+            else init_acc_from_bias(par_after(tile_par, 1));
         }
         if constexpr (NPEND > 0) {
             pend_row = row0;
@@ -885,7 +979,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         half_cur = half_nxt;
         role_cur = role_nxt;
         if constexpr (SK) kps = role_cur != 0 ? kpp >> 1 : kps_full;
-        tile_par ^= 1;
+        tile_par = par_after(tile_par, 1);
         curA = nxtA;
         curB = nxtB;
         nxtA = kOob;
@@ -895,7 +989,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             locate(nidx, ntm, ntn, nsl);
             nxtA = (unsigned)ntm * strideA + (unsigned)nsl * strideK + (unsigned)half_nxt * halfK;
             nxtB = (unsigned)ntn * strideB + (unsigned)nsl * strideK + (unsigned)half_nxt * halfK;
-            fetch_bias(ntn * P::BN, tile_par ^ 1);  // a whole tile ahead of its use (its buffer was last read before this tile began)
+            fetch_bias(ntn * P::BN, par_after(tile_par, 1), ntm * 256);  // a whole tile ahead of its use (its buffer was last read before this tile began)
         }
     };
     auto advance = [&]() {  // K-step t -> t + 1; true at the end of the tile
@@ -912,8 +1006,8 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     // of "K-step -1" is skipped), then B, A half 1 of K-step 0 ... wait: per K-step the stream carries
     // [B of t + 2, A half 1 of t + 1, A half 0 of t + 2]; before K-step 0 that is [B 0, A0 0] and [B 1, A1 0, A0 1].
     {
-        fetch_bias(n0, 0);
-        if (has_nxt) fetch_bias(ntn * P::BN, 1);
+        fetch_bias(n0, 0, m0);
+        if (has_nxt) fetch_bias(ntn * P::BN, 1, ntm * 256);
         const Ahead s0 = ahead(0);
         s1 = ahead(1);
         s2 = s1;
@@ -938,6 +1032,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         phase_stamp();
     }
 
+    auto half_way = [&]() { return F16 && pi_cur == pl.npairs - 1 && kk_cur == kps >> 1; };
     // two K-steps per trip so that the slot is a compile-time constant; a tile may end after either
     for (;;) {
         kstep(Ic<0>{});
@@ -950,6 +1045,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             next_tile();
             read_kstep_head(Ic<1>{});
             bar();  // every wave has re-read the new tile's first B fragments: steps 0-2 may now overwrite that B region
+        } else if (half_way()) {
+            settle();
+            set_aside();
+            read_kstep_head(Ic<1>{});
+            bar();
         }
         kstep(Ic<1>{});
         if (advance()) {
@@ -959,6 +1059,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             phase_stamp();
             if (!has_nxt) break;
             next_tile();
+            read_kstep_head(Ic<0>{});
+            bar();
+        } else if (half_way()) {
+            settle();
+            set_aside();
             read_kstep_head(Ic<0>{});
             bar();
         }
@@ -974,16 +1079,17 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     }
 }
 
-template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false>
+template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
 int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, int n_sl,
-                  const PrefillQkv& qa, hipStream_t s) {
+                  const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}) {
     using P = S4<NT>;
+    constexpr int LDS = F16 ? P::LDS_F16 : P::LDS;
     static OncePerDevice raised;  // (handles of the layered tier may be on different devices)
     int device = 0;
     ZG_HIP(hipGetDevice(&device));
     ZG_TRY(raised.run(device, []() -> int {
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, P::LDS));
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK, F16>),
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         return ZG_OK;
     }));
     const int tiles_m = (M + 255) / 256, tiles_n = (N + P::BN - 1) / P::BN, n_tiles = tiles_m * tiles_n * n_sl;
@@ -1000,9 +1106,9 @@ int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
         pa2 |= ((pl.pa_bits >> (4 * i)) & 3u) << (2 * i);
         pb2 |= ((pl.pb_bits >> (4 * i)) & 3u) << (2 * i);
     }
-    hipLaunchKernelGGL((gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK>), dim3(grid), dim3(256), P::LDS, s, A, B, bias, C, M, N,
+    hipLaunchKernelGGL((gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK, F16>), dim3(grid), dim3(256), LDS, s, A, B, bias, C, M, N,
                        (unsigned)pl.lda | ((unsigned)pl.ldb << 16), (unsigned)ldc | ((unsigned)pl.kpp << 20) | ((unsigned)pl.npairs << 28),
-                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa);
+                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa, ex);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1055,6 +1161,15 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
                    bool gelu, bool out_bf16, int bn, hipStream_t s) {
     (void)bn;  // 192-wide tiles only: 256 x 256 needs all 256 accumulator registers plus 128 of B fragments
     return launch_s4_nt<3>(A, B, bias, C, M, N, pl, ldc, gelu, out_bf16, s);
+}
+
+int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s) {
+    const PrefillQkv none{};
+    ZG_REQUIRE((size_t)M * ldc * 4 < ((size_t)1 << 32) && (size_t)M * pl.lda < (1u << 30) && (size_t)N * pl.ldb < (1u << 30), ZG_ERR_SHAPE,
+               "gemm: operands of %d x %d x %d beyond the 32-bit buffer descriptors", M, N, pl.kpp * 64);
+    gemm_note_launch();
+    note_kernel("gemm_s4_kernel");
+    return launch_s4_kind<3, S4_PLAIN, false, false, false, true>(A, B, bias, C, M, N, pl, ldc, 1, none, s, ex);
 }
 
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s) {

@@ -316,13 +316,14 @@ __global__ __launch_bounds__(512) void linear_few_mfma_kernel(const float* __res
 
 }  // namespace
 
-bool linear_tiles_pay(size_t M, size_t N) {
-    // Against the persistent kernel behind two splitting passes, whose time goes by rounds of 256 tiles of 256 x 192 whether they are full or
-    // not (us of a call, this : that): 768 -> 3072 16 rows 21 : 83, 512 rows 42 : 90, 1500 rows (1152 tiles) 76 : 91, 2048 (1536) 90 : 95, 4096
-    // (3072) 165 : 122; 3072 -> 768 16 rows 24 : 255, 4096 (768) 161 : 271; 1600 -> 1600 2048 (800) 112 : 151, 4096 (1600) 184 : 168;
-    // 1600 -> 4800 1023 (1200) 135 : 159, 1500 (1800) 203 : 170; 6400 -> 1600 16 rows 33 : 504, 4096 (1600) 675 : 593.
+bool linear_tiles_pay(size_t M, size_t N, size_t K) {
+    // Against the persistent kernel behind its splitting pass, whose time goes by rounds of 256 tiles of 256 x 192 whether they are full or not.
+    // From 512 columns on that kernel takes three products of fp16 terms (us of a call, this : that): 768 -> 3072 1023 rows (768 tiles)
+    // 50 : 66, 1300 (1008) 62 : 67, 1500 (1152) 69 : 67, 2048 (1536) 83 : 68; 768 -> 1031 4096 rows (1088) 70 : 68; 1600 -> 1600 1500 rows (600) 80 : 101,
+    // 2048 (800) 107 : 101; 6400 -> 1600 1500 rows (600) 278 : 337, 2048 (800) 384 : 342; 3072 -> 768 4096 rows (768) 161 : 185, 6000 (1128) 240 : 192.
+    // Below, six of bf16: 128 -> 3072 1856 rows (1392 tiles) and more.
     const size_t tiles = ((M + 63) / 64) * ((N + 63) / 64), rounds = (((M + 255) / 256) * ((N + 191) / 192) + 255) / 256;
-    return tiles <= 1400 * rounds;
+    return tiles <= (K < kSplit2MinK ? 1400 : K < 1024 ? 1100 : 800) * rounds;
 }
 
 int linear_tiles_slices(size_t M, size_t N, size_t K) {

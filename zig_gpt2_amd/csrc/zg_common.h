@@ -95,6 +95,25 @@ __device__ __forceinline__ void split3_pk(float x0, float x1, uint32_t& hi, uint
     lo = cvt_pk_bf16(r0 - bf16_lo(mid), r1 - bf16_hi(mid));
 }
 
+// Two-term fp16 split of two fp32 values: x = hi + lo to within one unit in the last place of a 24-bit number (11 + 1 + 11 bits: three values of four
+// exactly), as long as |x| is in [2^-2, 2^16); below, to within 2^-25.  Rows are scaled by a power of two that brings their largest value
+// to [2^14, 2^15), so what a row loses is below 2^-39 of that value.  Three products of such terms (hi hi, hi lo, lo hi) stand for
+// an fp32 product where three bf16 terms take six, and two for a product with a bf16 value, which one fp16 term holds.  Measured against 64
+// bits, sums of such products are closer than the exact split's: they are rounded half as often.
+__device__ __forceinline__ void split2_f16(float x0, float x1, uint32_t& hi, uint32_t& lo) {
+    typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+    typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+    const f16x2_t h = __builtin_convertvector(f32x2_t{x0, x1}, f16x2_t);
+    const f32x2_t r = f32x2_t{x0, x1} - __builtin_convertvector(h, f32x2_t);
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2_t));
+}
+// what brings a row whose largest value (as bits without the sign) is `top` to [2^14, 2^15); rows of zeros and of values that are not finite: anything that is finite
+__device__ __forceinline__ int split2_exp(uint32_t top) {
+    const int e = (int)(top >> 23);
+    return 141 - (e < 1 ? 1 : e);
+}
+
 // Activation planes of the lock-step batch in global memory: the epilogue of the producing kernel writes the exact
 // three-term bf16 split of its output row, the consuming Linear loads them as MFMA A fragments — no LDS staging and no
 // split in front of its MFMAs.  Element (plane p, batch row m < 8, column k) of a [3][8][K] triple sits at

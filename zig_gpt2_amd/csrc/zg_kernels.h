@@ -170,6 +170,18 @@ int launch_copy_f32(const float* in, float* out, size_t n, hipStream_t s);
 int launch_f32_to_bf16(const float* in, bf16_t* out, size_t n, hipStream_t s);
 // fp32 [rows][K] -> bf16 [rows][3K] = [hi | mid | lo], hi + mid + lo == x exactly
 int launch_split3(const float* in, size_t rows, int K, bf16_t* out, hipStream_t s);
+// fp32 [rows][K] of one or two matrices (the second may have none) -> fp16 [rows][2K] = [hi | lo] of the rows times 2^-exps[row], which brings their
+// largest value to [2^14, 2^15): elementwise.hip
+// In front of a Linear's products from kSplit2MinK columns on: shorter sums of three exact bf16 terms are closer to 64 bits than two fp16 terms can be
+// (128 columns: 0.64e-7 against 0.98e-7 at best; 512: 1.29e-7 and 1.25e-7; 768: 1.58e-7 and 1.52e-7; 1600: 2.37e-7 and 1.99e-7).
+constexpr size_t kSplit2MinK = 512;
+struct Split2Job {
+    const float* in;
+    uint16_t* out;
+    int* exps;
+    int rows;
+};
+int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s);
 // rows [from_row, ctx) of every (cache, sequence x head) strip set to zero: n_caches caches cache_stride bytes apart, each holding a
 // plane of [strips][ctx] rows of row_bytes at plane_off (api_gpt.hip clear_kv: what a new sequence must not inherit)
 int launch_kv_clear_tail(void* base, int n_caches, size_t cache_stride, size_t plane_off, int row_bytes, int strips, int ctx, int from_row,
@@ -196,6 +208,13 @@ int launch_gemm_planes(const bf16_t* A, const bf16_t* B, const float* bias, void
 int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc,
                    bool gelu, bool out_bf16, int bn, hipStream_t s);  // gemm_s4.hip
 bool gemm_s4_args_ok(const GemmPlanes& pl, int ldc);            // the bounds of gemm_s4_kernel's packed arguments
+// ... with planes of fp16 (launch_split2): what the sums of output row m and column n are multiplied with, 2^(a[m] + w[n]) (a_each; else a[0] for every row)
+struct PlaneExps {
+    const int* a;
+    const int* w;
+    bool a_each;
+};
+int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s);
 // ... and its epilogue kinds for the whole-prompt Linears (gemm_s4.hip; PrefillQkv below)
 enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT3 = 3, S4_RELU2 = 4 };
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s);
@@ -212,7 +231,7 @@ bool linear_few_ok(size_t M, size_t N, size_t K);
 unsigned long long linear_few_mfma_launch_count();  // launches of linear_few_mfma_kernel so far
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 // Nine rows and more: K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N floats where that is more than one slice.
-bool linear_tiles_pay(size_t M, size_t N);
+bool linear_tiles_pay(size_t M, size_t N, size_t K);
 int linear_tiles_slices(size_t M, size_t N, size_t K);
 int launch_linear_tiles(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, float* slabs, hipStream_t s);
 
