@@ -1,0 +1,85 @@
+"""The whole-prompt pass on two-term fp16 planes: the exponents that a layer's activations get from its weights (launch_prefill_bounds) hold for weights of very
+different sizes, are made again when a tensor is loaded again, and travel to handles that share the weights."""
+import numpy as np
+import pytest
+
+import oracle
+from golden_io import assert_model_close
+from zig_gpt2_amd import gpt as zgpt
+from zig_gpt2_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+def uneven(cfg, seed, bf16):
+    """Weights whose layers' activations lie many binades apart: large and small gains and biases, rows of a matrix far smaller than the others."""
+    w = {k: np.array(v, np.float32) for k, v in synth.make_weights(cfg, seed=seed, bf16=bf16).items()}
+    rng = np.random.default_rng(seed)
+    for l in range(cfg.n_layer):
+        p = f"h{l}."
+        w[p + "ln_1_g"] *= np.float32(2.0 ** int(rng.integers(-6, 7)))
+        w[p + "ln_2_g"] *= np.float32(2.0 ** int(rng.integers(-6, 4)))
+        w[p + "ln_2_b"] += np.float32(0.5)
+        w[p + "c_fc_w"] = w[p + "c_fc_w"].reshape(4 * cfg.n_embed, cfg.n_embed)
+        w[p + "c_fc_w"][::3] *= np.float32(2.0 ** -14)
+        v = w[p + "c_attn_w"].reshape(3, cfg.n_embed, cfg.n_embed)
+        v[0] *= np.float32(0.25 / abs(w[p + "ln_1_g"]).max())  # (scores of an ordinary size)
+        v[2, ::5] *= np.float32(2.0 ** 6)
+        w[p + "c_attn_w"] = v.reshape(3 * cfg.n_embed, cfg.n_embed)
+        if bf16:
+            for k in ("c_fc_w", "c_attn_w"):
+                bits = synth.to_bf16_bits(w[p + k])
+                w[p + k] = (bits.astype(np.uint32) << 16).view(np.float32).reshape(w[p + k].shape)
+    return w
+
+
+@pytest.mark.parametrize("name,batch,n,bf16,route", [("tiny", 1, 33, True, 0), ("tiny3", 2, 47, False, 0), ("nano-char", 2, 129, True, 1), ("nano-char", 1, 70, False, 1),
+                                                     ("xl-slice", 1, 95, True, 2), ("medium-slice", 1, 64, False, 2), ("xl-slice", 1, 40, False, 3)])
+def test_weights_of_very_different_sizes(zg, name, batch, n, bf16, route):
+    cfg = synth.CONFIGS[name]
+    w = uneven(cfg, 61, bf16)
+    m = zgpt.GPT(cfg, batch=batch, weights_f32=not bf16)
+    m.load_weights(w)
+    toks = np.stack([synth.rand_tokens(610 + b, n + 1, cfg.vocab_size) for b in range(batch)])
+    zg.zg_debug_prefill_route(route, 0)
+    try:
+        lg = m.prefill(toks[:, :n]).copy()
+    finally:
+        zg.zg_debug_prefill_route(0, 0)
+    nxt = m.forward(n + 1, toks[:, n])
+    for b in range(batch):
+        ref = oracle.GPT(cfg, w).forced_logits(toks[b], n - 1)
+        assert_model_close(ref[0], lg[b], f"{name} uneven weights, row {b}")
+        assert_model_close(ref[1], nxt[b], f"{name} uneven weights, decode, row {b}")
+    m.close()
+
+
+def test_a_tensor_loaded_again(zg):
+    cfg = synth.CONFIGS["tiny3"]
+    toks = synth.rand_tokens(62, 40, cfg.vocab_size)
+    m = zgpt.GPT(cfg)
+    m.load_weights(synth.make_weights(cfg, seed=62, bf16=True))
+    m.prefill([toks])
+    w = uneven(cfg, 63, True)  # other planes, other exponents
+    m.load_weights(w)
+    other = zgpt.GPT(cfg, batch=2, share_weights_with=m)
+    ref = oracle.GPT(cfg, w).forced_logits(toks, len(toks) - 1)[0]
+    assert_model_close(ref, other.prefill(np.stack([toks, toks]))[1], "a handle that shares the weights")
+    assert_model_close(ref, m.prefill([toks])[0], "loaded again")
+    other.close()
+    m.close()
+
+
+def test_two_plane_handles_round_their_activations_to_16_bits(zg):
+    """What ZG_GPT_PREFILL_2PLANE asks for: 2^-17 of an activation, beside the 2^-23 of the default."""
+    cfg = synth.CONFIGS["nano-char"]
+    w = synth.make_weights(cfg, seed=64, bf16=True)
+    toks = synth.rand_tokens(640, 130, cfg.vocab_size)
+    ref = oracle.GPT(cfg, w).forced_logits(toks, len(toks) - 1)[0].astype(np.float64)
+    err = []
+    for planes in (3, 2):
+        m = zgpt.GPT(cfg, prefill_planes=planes)
+        m.load_weights(w)
+        err.append(np.linalg.norm(m.prefill([toks])[0] - ref) / np.linalg.norm(ref))
+        m.close()
+    assert err[0] < 2e-6 < err[1] < 1e-4, err

@@ -27,9 +27,11 @@ using namespace zg;
 
 struct zg_layer {
     void *c_attn_w, *c_proj_w, *c_fc_w, *mlp_proj_w;
-    // ZG_GPT_WEIGHTS_F32 handles only: the same matrices split exactly into bf16 planes [out][3 in] = [hi | mid | lo]
-    // (filled when the tensor is loaded) — the B operand of the whole-prompt GEMMs
-    bf16_t *c_attn_p, *c_proj_p, *c_fc_p, *mlp_proj_p;
+    // the same matrices for the whole-prompt GEMMs (none: ZG_GPT_NO_PREFILL), made when the tensor is loaded; the 2-norms of the rows of the two behind a
+    // LayerNorm, and the exponents of the layer's activations that follow from them (launch_prefill_bounds)
+    PrefillW c_attn_p, c_proj_p, c_fc_p, mlp_proj_p;
+    float *c_attn_n, *c_fc_n;
+    int* exps;
     // LayerNorm folded out of the two LayerNorm-fed Linears (gemv_ksplit.hip, gemv_lnk_kernel): c2 = W g, c3 = W b + bias
     float *c_attn_c2, *c_attn_c3, *c_fc_c2, *c_fc_c3;
     float *ln_1_g, *ln_1_b, *c_attn_b, *c_proj_b, *ln_2_g, *ln_2_b, *c_fc_b, *mlp_proj_b;
@@ -58,13 +60,13 @@ struct zg_gpt {
     float* sk_ws;
     int* sk_cnt;
     int sk_tiles;
-    // whole-prompt (prefill) scratch, rows = batch * ctx: x fp32 [E], qkv fp32 [3E], split bf16 [kSplit E] and [kSplit 4E]
+    // whole-prompt (prefill) scratch, rows = batch * ctx: x fp32 [E], qkv fp32 [3E], planes [kPair E] and [kPair 4E]
     float *pf_x, *pf_qkv, *pf_ws;
     size_t pf_ws_floats;
     unsigned* sk_flags;   // stream-K hand-over of the c_attn GEMM (PrefillQkv.sk_*): 512 flag words, zeroed at create
     unsigned sk_epoch;
     bool sk_used;         // a stream-K launch since the last check of gemm_s4_fault
-    bf16_t *pf_a, *pf_h;
+    uint16_t *pf_a, *pf_h;
     // lock-step batch with bf16 weights: activation planes between the kernels of a Block (GemvArgs.pl_in / pl_out):
     // xp = planes of g * x for the next LayerNorm-fed Linear [48 E bytes], hp = planes of gelu(c_fc) [48 * 4E bytes]
     // ap = planes of the merged attention output [48 E bytes], written by the last split of every (sequence, head)
@@ -103,7 +105,7 @@ struct zg_gpt {
     size_t graph_steps;
     hipStream_t graph_stream;
     size_t steps_enqueued;
-    bool ln_folded;  // c2 / c3 of every layer match the weights currently in the arena
+    bool ln_folded;  // c2 / c3 and the prompts' exponents of every layer match the weights currently in the arena
     // side-stream L2 prefetcher of the decode chain (prefetch.hip); runs during zg_gpt_generate_enqueue only
     PfCtl* pf_ctl;
     PfJob* pf_jobs;  // [pf_njobs]: embed, 5 per layer, lm_head
@@ -194,12 +196,22 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
         y.c_attn_c3 = (float*)P(3 * E * 4);
         y.c_fc_c2 = (float*)P(4 * E * 4);
         y.c_fc_c3 = (float*)P(4 * E * 4);
-        y.c_attn_p = y.c_proj_p = y.c_fc_p = y.mlp_proj_p = nullptr;
-        if (g->wt == WT_F32 && !(g->flags & ZG_GPT_NO_PREFILL)) {  // inside the weight region: broadcast with the weights
-            y.c_attn_p = (bf16_t*)P(3 * E * E * kSplit * 2);
-            y.c_proj_p = (bf16_t*)P(E * E * kSplit * 2);
-            y.c_fc_p = (bf16_t*)P(4 * E * E * kSplit * 2);
-            y.mlp_proj_p = (bf16_t*)P(4 * E * E * kSplit * 2);
+        y.c_attn_p = y.c_proj_p = y.c_fc_p = y.mlp_proj_p = PrefillW{};
+        y.c_attn_n = y.c_fc_n = nullptr;
+        y.exps = nullptr;
+        if (!(g->flags & ZG_GPT_NO_PREFILL)) {  // inside the weight region: broadcast with the weights
+            const int planes = g->wt == WT_F32 ? 2 : 1;
+            auto W = [&](size_t out, size_t in) {
+                uint16_t* p = (uint16_t*)P(out * in * planes * 2);
+                return PrefillW{p, (int*)P(out * 4), planes};
+            };
+            y.c_attn_p = W(3 * E, E);
+            y.c_proj_p = W(E, E);
+            y.c_fc_p = W(4 * E, E);
+            y.mlp_proj_p = W(E, 4 * E);
+            y.c_attn_n = (float*)P(3 * E * 4);
+            y.c_fc_n = (float*)P(4 * E * 4);
+            y.exps = (int*)P(kBounds * 4);
         }
     }
     g->weight_region_bytes = (cv.off + 255) & ~(size_t)255;
@@ -255,10 +267,10 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
     if (!(g->flags & ZG_GPT_NO_PREFILL)) {
         g->pf_x = (float*)P(B * C * E * 4);
         g->pf_qkv = (float*)P(B * C * 3 * E * 4);
-        g->pf_a = (bf16_t*)P(B * C * kSplit * E * 2);
-        g->pf_h = (bf16_t*)P(B * C * kSplit * 4 * E * 2);
-        // bf16 weights: 64 MiB of split-K partial sums; fp32 weights: a full fp32 [rows][4 E] GEMM output
-        // split-K partials of the prompt GEMMs; fp32 weights: three weight-plane passes of [B ctx, 4 E] at the least
+        g->pf_a = (uint16_t*)P(B * C * kPair * E * 2);
+        g->pf_h = (uint16_t*)P(B * C * kPair * 4 * E * 2);
+        // split-K partials of the prompt GEMMs: 64 MiB; fp32 weights: two weight-plane passes of [B ctx, 4 E] at the least
+        // (and as much as three of them, so that no K slicing is cut short)
         g->pf_ws_floats = g->wt == WT_BF16 ? (size_t)(16u << 20) : std::max((size_t)(16u << 20), 3 * B * C * 4 * E);
         g->pf_ws = (float*)P(g->pf_ws_floats * 4);
         g->sk_flags = (unsigned*)P(2048);
@@ -407,6 +419,7 @@ int ensure_ln_folded(zg_gpt* g, hipStream_t s) {
     for (const zg_layer& y : g->layers) {
         ZG_TRY(launch_ln_fold(y.c_attn_w, g->wt, y.ln_1_g, y.ln_1_b, y.c_attn_b, 3 * E, E, y.c_attn_c2, y.c_attn_c3, s));
         ZG_TRY(launch_ln_fold(y.c_fc_w, g->wt, y.ln_2_g, y.ln_2_b, y.c_fc_b, 4 * E, E, y.c_fc_c2, y.c_fc_c3, s));
+        if (y.exps) ZG_TRY(launch_prefill_bounds(PrefillBounds{y.ln_1_g, y.ln_1_b, y.c_attn_b, y.ln_2_g, y.ln_2_b, y.c_fc_b, y.c_attn_n, y.c_fc_n, y.exps}, E, s));
     }
     ZG_TRY(launch_ln_fold(g->wte, g->wt, g->ln_f_g, g->ln_f_b, nullptr, (int)g->cfg.vocab_size, E, g->lm_c2, g->lm_c3, s));
     // handles that share the region run on other streams: the vectors must be complete before any of them reads the flag
@@ -585,19 +598,17 @@ int enqueue_step(zg_gpt* g, bool with_logits, int t_hi, hipStream_t s, StepProf*
 // exactly as P calls of GPT.forward would (main.zig:331-334) and leaves the residual stream of all rows in
 // pf_x.  With `last_block_full` false the last Block stops after its cache append: nothing downstream of
 // it is needed when generation re-feeds the last prompt token (main.zig:337).
-// fp32 weights (ZG_GPT_WEIGHTS_F32): the same pass; the weight operand is then the exact three-term bf16 split of the fp32
-// matrix (plane-major, made when the tensor is loaded) and every GEMM runs as three partial passes of the same kernel — the
-// six plane products above 2^-24 of the leading one, fp32-sgemm grade (prefill.hip launch_prefill_gemm_wp).
+// fp32 weights (ZG_GPT_WEIGHTS_F32): the same pass with two planes of a weight instead of one (prefill.hip).
 // (Measured and dropped in round 4: replaying this pass from a hipGraph per prompt length.  0.844 against 0.749 ms at 64
 // tokens, 1.645 against 1.553 ms at 1023 — the ~10 us a launch costs here is the kernels' own latency at these sizes, not host
 // overhead, and a graph launch adds its own ~10 us; profiles/round4_prefill_graph.jsonl.)
 int enqueue_prefill(zg_gpt* g, size_t P, bool last_block_full, hipStream_t s) {
     const bool f32w = g->wt == WT_F32;
-    const int np = f32w ? kWeightPlanes : (g->flags & ZG_GPT_PREFILL_2PLANE) ? 2 : kSplit;
+    const int coarse = !f32w && (g->flags & ZG_GPT_PREFILL_2PLANE) ? 1 : 0;
     const size_t E = g->cfg.n_embed, L = g->cfg.n_layer, H = g->cfg.n_heads, C = g->cfg.context_size;
     const int B = (int)g->batch, M = (int)(g->batch * P), iE = (int)E;
     ZG_TRY(launch_embed_prefill(g->prompt, (int)C, B, (int)P, g->wte, g->wpe, g->wt, iE, g->pf_x, s));
-    ZG_TRY(launch_ln_split(g->pf_x, M, iE, g->layers[0].ln_1_g, g->layers[0].ln_1_b, 1e-5f, g->pf_a, s));
+    ZG_TRY(launch_ln_split(g->pf_x, M, iE, g->layers[0].ln_1_g, g->layers[0].ln_1_b, 1e-5f, g->pf_a, PlaneOut{g->layers[0].exps + PB_LN1, coarse}, s));
     for (size_t l = 0; l < L; ++l) {
         const zg_layer& y = g->layers[l];
         // pf_a holds split(ln_1(x)) here: from the line above or from the tail of the previous Block's last GEMM
@@ -611,21 +622,21 @@ int enqueue_prefill(zg_gpt* g, size_t P, bool last_block_full, hipStream_t s) {
             qa.sk_epoch = ++g->sk_epoch;
             g->sk_used = true;
         }
-        ZG_TRY(launch_prefill_gemm(g->pf_a, f32w ? y.c_attn_p : (const bf16_t*)y.c_attn_w, y.c_attn_b, g->pf_qkv, M, 3 * iE, iE, 3 * iE, PF_QKV,
-                                   g->pf_ws, g->pf_ws_floats, nullptr, s, &qa, np));
+        ZG_TRY(launch_prefill_gemm(PrefillA{g->pf_a, y.exps + PB_LN1, false}, y.c_attn_p, y.c_attn_b, g->pf_qkv, M, 3 * iE, iE, 3 * iE, PF_QKV,
+                                   g->pf_ws, g->pf_ws_floats, nullptr, s, &qa));
         if (l + 1 == L && !last_block_full) break;
         // (an fp32 cache is read directly: the c_attn epilogue then need not store the k / v columns of qkv)
         ZG_TRY(launch_attn_prefill(g->pf_qkv, g->pf_a, B, (int)P, iE, (int)H, g->pf_ws, g->pf_ws_floats, g->kv_mode == 0 ? (const float*)y.k_cache : nullptr,
-                                       g->kv_mode == 0 ? (const float*)y.v_cache : nullptr, (int)C, s));
-        const PrefillLn ln2{y.ln_2_g, y.ln_2_b, 1e-5f, g->pf_a};
-        ZG_TRY(launch_prefill_gemm(g->pf_a, f32w ? y.c_proj_p : (const bf16_t*)y.c_proj_w, y.c_proj_b, g->pf_x, M, iE, iE, iE, PF_RESID, g->pf_ws,
-                                   g->pf_ws_floats, &ln2, s, nullptr, np));
-        ZG_TRY(launch_prefill_gemm(g->pf_a, f32w ? y.c_fc_p : (const bf16_t*)y.c_fc_w, y.c_fc_b, g->pf_h, M, 4 * iE, iE, 0, PF_GELU_SPLIT, g->pf_ws,
-                                   g->pf_ws_floats, nullptr, s, nullptr, np));
+                                       g->kv_mode == 0 ? (const float*)y.v_cache : nullptr, (int)C, y.exps, coarse, s));
+        const PrefillLn ln2{y.ln_2_g, y.ln_2_b, 1e-5f, g->pf_a, PlaneOut{y.exps + PB_LN2, coarse}};
+        ZG_TRY(launch_prefill_gemm(PrefillA{g->pf_a, y.exps + PB_V, false}, y.c_proj_p, y.c_proj_b, g->pf_x, M, iE, iE, iE, PF_RESID, g->pf_ws,
+                                   g->pf_ws_floats, &ln2, s));
+        ZG_TRY(launch_prefill_gemm(PrefillA{g->pf_a, y.exps + PB_LN2, false}, y.c_fc_p, y.c_fc_b, g->pf_h, M, 4 * iE, iE, 0, PF_GELU_SPLIT, g->pf_ws,
+                                   g->pf_ws_floats, nullptr, s, nullptr, PlaneOut{y.exps + PB_GELU, coarse}));
         const bool more = l + 1 < L;
-        const PrefillLn ln1{more ? g->layers[l + 1].ln_1_g : nullptr, more ? g->layers[l + 1].ln_1_b : nullptr, 1e-5f, g->pf_a};
-        ZG_TRY(launch_prefill_gemm(g->pf_h, f32w ? y.mlp_proj_p : (const bf16_t*)y.mlp_proj_w, y.mlp_proj_b, g->pf_x, M, iE, 4 * iE, iE, PF_RESID, g->pf_ws,
-                                   g->pf_ws_floats, more ? &ln1 : nullptr, s, nullptr, np));
+        const PrefillLn ln1{more ? g->layers[l + 1].ln_1_g : nullptr, more ? g->layers[l + 1].ln_1_b : nullptr, 1e-5f, g->pf_a, PlaneOut{more ? g->layers[l + 1].exps + PB_LN1 : nullptr, coarse}};
+        ZG_TRY(launch_prefill_gemm(PrefillA{g->pf_h, y.exps + PB_GELU, false}, y.mlp_proj_p, y.mlp_proj_b, g->pf_x, M, iE, 4 * iE, iE, PF_RESID, g->pf_ws,
+                                   g->pf_ws_floats, more ? &ln1 : nullptr, s));
     }
     return ZG_OK;
 }
@@ -1211,11 +1222,14 @@ int zg_gpt_load_block_tensor(zg_gpt* g, size_t layer, int slot, const float* src
     ZG_REQUIRE(len == n, ZG_ERR_SHAPE, "block slot %d expects %zu elements, got %zu", slot, n, len);
     g->ln_folded = false;
     ZG_TRY(upload_f32(src, n, dst, mat && g->wt == WT_BF16, gs(g)));
-    if (mat && g->wt == WT_F32 && y.c_attn_p) {  // exact bf16 planes of the fp32 matrix for the whole-prompt GEMMs
-        bf16_t* pl = slot == ZG_C_ATTN_W ? y.c_attn_p : slot == ZG_C_PROJ_W ? y.c_proj_p : slot == ZG_C_FC_W ? y.c_fc_p : y.mlp_proj_p;
-        // plane-major [3][out][in]: the matrix as ONE row of out * in elements
-        ZG_REQUIRE(n <= (size_t)2147483647 / 3, ZG_ERR_SHAPE, "weight matrix of %zu elements", n);  // (split3_kernel indexes 3 n in int)
-        ZG_TRY(launch_split3(reinterpret_cast<const float*>(dst), 1, (int)n, pl, gs(g)));
+    if (mat && y.exps) {  // planes for the whole-prompt GEMMs
+        const PrefillW& p = slot == ZG_C_ATTN_W ? y.c_attn_p : slot == ZG_C_PROJ_W ? y.c_proj_p : slot == ZG_C_FC_W ? y.c_fc_p : y.mlp_proj_p;
+        float* norms = slot == ZG_C_ATTN_W ? y.c_attn_n : slot == ZG_C_FC_W ? y.c_fc_n : nullptr;
+        const int in = (int)(slot == ZG_MLP_PROJ_W ? 4 * E : E), out = (int)(n / in);
+        uint16_t* planes = const_cast<uint16_t*>(p.p);
+        int* exps = const_cast<int*>(p.exps);
+        if (g->wt == WT_F32) ZG_TRY(launch_split2(Split2Job{reinterpret_cast<const float*>(dst), planes, exps, out, n, norms}, Split2Job{}, in, gs(g)));
+        else ZG_TRY(launch_plane_bf16(reinterpret_cast<const bf16_t*>(dst), out, in, planes, exps, norms, gs(g)));
         ZG_HIP(hipStreamSynchronize(gs(g)));
     }
     return ZG_OK;

@@ -1,12 +1,11 @@
 // attn_prefill.hip — causal scaled_dot_product_attention for all n prompt positions at once (src/ops.zig:249-307: per head
-// two sgemm calls and a softmax per query row; the reference runs it once per token, src/main.zig:331-334), on the bf16
+// two sgemm calls and a softmax per query row; the reference runs it once per token, src/main.zig:331-334), on the
 // matrix cores at fp32 accuracy.
 //
-// Numerics.  q, k, v arrive as fp32 (the c_attn rows).  Every operand of a matrix product is the EXACT three-term bf16 split
-// x = hi + mid + lo (zg_common.h split3_pk), and a product a . b is the six plane products a_i b_j with i + j <= 2 — what is
-// dropped is below 2^-24 of the leading term, every bf16 x bf16 product is exact in fp32 and the MFMA accumulates in fp32: the
-// result is fp32-sgemm grade, as the fp32-weight Linears of prefill.hip.  The probabilities are split the same way after the
-// softmax.  16 x the matrix rate of v_mfma_f32_32x32x2_f32 for 6 x the products.
+// Numerics.  q, k, v arrive as fp32 (the c_attn rows).  Every operand of a matrix product is the two-term fp16 split of its value
+// times a power of two (zg_common.h split2_f16; the powers follow from the weights, launch_prefill_bounds, those of the probabilities
+// from their largest, 2^kDefer), and a product a . b is the three plane products hi hi, hi lo, lo hi: every fp16 x fp16 product is exact in fp32 and the
+// MFMA accumulates in fp32.  The probabilities are split the same way after the softmax.
 //
 // Structure.  A workgroup = four waves = four consecutive 32-query blocks of one head (128 queries) against a range of 32-key
 // tiles; the K / V tiles are shared: the four waves fetch a tile as fp32 (a quarter each, coalesced 256-byte rows), split it
@@ -20,12 +19,13 @@
 // partials a small kernel merges (one prompt of 1023 tokens would otherwise be 96 workgroups of up to 32 tiles).
 #include <type_traits>
 
+#include "prefill_epi.h"
 #include "zg_kernels.h"
 
 namespace zg {
 namespace {
 
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) short s16x4;
 typedef __attribute__((ext_vector_type(8))) short s16x8;
@@ -35,9 +35,10 @@ constexpr int kKPlane = 32 * 128;        // one K plane of a tile: [32 keys][64 
 constexpr int kVBlock = 32 * 32 + 128;   // one 16-d block of a V plane: [32 keys][16 d] bf16, + 128 B: the two blocks a half-wave reads
                                          // in one ds_read_b64_tr_b16 then lie 288 dwords apart — the two halves of the 64 banks
 constexpr int kVPlane = 4 * kVBlock;
-constexpr int kLds = 2 * 3 * kKPlane + 2 * 3 * kVPlane;  // K ring + V ring, two slots each: 52224 B
+constexpr int kLds = 2 * kPair * kKPlane + 2 * kPair * kVPlane;  // K ring + V ring, two slots each: 34816 B
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kDefer = 8.0f;  // log2 units
+constexpr float kProbUp = 7.0f;  // probabilities are made 2^7 times as large: at most 2^15
 
 // A query's 32 scores of a tile sit in two lanes (l and l ^ 32, 16 keys each): v_permlane32_swap hands every lane both halves'
 // values (vdst = {lower half's, lower half's}, src0 = {upper half's, upper half's}) — no LDS crossbar, no select
@@ -50,15 +51,7 @@ __device__ __forceinline__ float both_halves_sum(float v) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-__device__ __forceinline__ bf16x8 frag(uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return __builtin_bit_cast(bf16x8, u32x4{a, b, c, d}); }
-
-__device__ __forceinline__ void store_split4(bf16_t* dst, size_t plane, f32x4 v) {
-    uint32_t a[3], b[3];
-    split3_pk(v.x, v.y, a[0], a[1], a[2]);
-    split3_pk(v.z, v.w, b[0], b[1], b[2]);
-#pragma unroll
-    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{a[p], b[p]};
-}
+__device__ __forceinline__ f16x8 frag(uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return __builtin_bit_cast(f16x8, u32x4{a, b, c, d}); }
 
 // key tiles a group of four query blocks needs, and the key ranges (splits) it is cut into
 __host__ __device__ inline int group_tiles(int g, int nqb) { return 4 * g + 4 < nqb ? 4 * g + 4 : nqb; }
@@ -69,8 +62,8 @@ __host__ __device__ inline int group_splits(int g, int nqb, int nts) { return (g
 // One instruction stream per wave, software-pipelined over the key tiles so that the matrix pipe and the vector ALU of a SIMD
 // work side by side WITHIN a wave (the first version ran S -> softmax -> split -> PV -> staging in sequence: 48 MFMAs = 1.5 k
 // cycles of a 6.4 k-cycle tile, 45 % matrix-busy with two waves per SIMD):
-//   phase A   S^T(t + 1) = K(t + 1) Q^T  (24 MFMAs)   beside   exp / sum / three-plane split of tile t's scores
-//   phase B   O^T += V(t)^T P(t)^T       (24 MFMAs)   beside   split + LDS write of the tiles in flight: K(t + 2), V(t + 1)
+//   phase A   S^T(t + 1) = K(t + 1) Q^T  (12 MFMAs)   beside   exp / sum / split of tile t's scores
+//   phase B   O^T += V(t)^T P(t)^T       (12 MFMAs)   beside   split + LDS write of the tiles in flight: K(t + 2), V(t + 1)
 // so K runs one tile ahead of V through its own two-slot ring; one barrier per tile.  The loop body has no branch (tiles above a
 // wave's diagonal are computed fully masked: its siblings need the tile anyway, the barrier would make it wait for them), only
 // the rare rescale of the running maximum sits in front of phase A.
@@ -83,8 +76,10 @@ struct AttnKv {
     size_t stride_b, stride_h;
     unsigned stride_t;
 };
-__global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __restrict__ qkv, bf16_t* __restrict__ out, float* __restrict__ part,
-                                                                 int P, int E, unsigned geo, const AttnKv kv) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __restrict__ qkv, uint16_t* __restrict__ out, float* __restrict__ part,
+                                                                 int P, int E, unsigned geo, const AttnKv kv, const int* __restrict__ exps, int coarse) {
+    const int exp_q = exps[PB_Q], exp_k = exps[PB_K], exp_v = exps[PB_V];
+    const float s_back = ldexpf(1.0f, exp_q + exp_k);  // scores leave the products 2^-(exp_q + exp_k) times as large
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -108,20 +103,20 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
 
     // Q^T fragments (B operand of S^T = K Q^T): lane = query, 8 consecutive d per 16-d slice.  Scaled by log2(e) / sqrt(64) before the
     // split (one fp32 rounding, as the reference's own alpha of sgemm, ops.zig:275) so that the softmax runs on bare v_exp_f32.
-    bf16x8 qf[3][4];
+    f16x8 qf[kPair][4];
     {
-        const float sc = 0.125f * kLog2e;
+        const float sc = ldexpf(0.125f * kLog2e, -exp_q);
         const float* qp = qkv + (row0 + min(tq, P - 1)) * ld + h * 64 + hl * 8;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const f32x4 a = *reinterpret_cast<const f32x4*>(qp + 16 * ks), c = *reinterpret_cast<const f32x4*>(qp + 16 * ks + 4);
-            uint32_t w[4][3];
-            split3_pk(a.x * sc, a.y * sc, w[0][0], w[0][1], w[0][2]);
-            split3_pk(a.z * sc, a.w * sc, w[1][0], w[1][1], w[1][2]);
-            split3_pk(c.x * sc, c.y * sc, w[2][0], w[2][1], w[2][2]);
-            split3_pk(c.z * sc, c.w * sc, w[3][0], w[3][1], w[3][2]);
+            uint32_t w[4][kPair];
+            split2_f16(a.x * sc, a.y * sc, w[0][0], w[0][1]);
+            split2_f16(a.z * sc, a.w * sc, w[1][0], w[1][1]);
+            split2_f16(c.x * sc, c.y * sc, w[2][0], w[2][1]);
+            split2_f16(c.z * sc, c.w * sc, w[3][0], w[3][1]);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) qf[p][ks] = frag(w[0][p], w[1][p], w[2][p], w[3][p]);
+            for (int p = 0; p < kPair; ++p) qf[p][ks] = frag(w[0][p], w[1][p], w[2][p], w[3][p]);
         }
     }
 
@@ -151,56 +146,57 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         vr[0] = __builtin_amdgcn_raw_buffer_load_b128(rv, vvo, so, 0);
         vr[1] = __builtin_amdgcn_raw_buffer_load_b128(rv, vvo + row4, so, 0);
     };
-    char* const kring = lds;                    // [2 slots][3 planes][32 keys][64 d]
-    char* const vring = lds + 2 * 3 * kKPlane;  // [2 slots][3 planes][4 d blocks][32 keys][16 d]
+    char* const kring = lds;                        // [2 slots][2 planes][32 keys][64 d]
+    char* const vring = lds + 2 * kPair * kKPlane;  // [2 slots][2 planes][4 d blocks][32 keys][16 d]
+    const float k_up = ldexpf(1.0f, -exp_k), v_up = ldexpf(1.0f, -exp_v);
     const int kaddr = skey * 128 + (((sd0 >> 3) ^ ((skey >> 1) & 7)) << 4) + ((sd0 >> 2) & 1) * 8;  // (key + 4: same swizzle term + 2)
     const int kaddr1 = (skey + 4) * 128 + (((sd0 >> 3) ^ (((skey + 4) >> 1) & 7)) << 4) + ((sd0 >> 2) & 1) * 8;
     const int vaddr = (vd0 >> 4) * kVBlock + vkey * 32 + (vd0 & 15) * 2;
     auto store_k = [&](int slot, const u32x4(&kr)[2]) {
-        char* st = kring + slot * 3 * kKPlane;
+        char* st = kring + slot * kPair * kKPlane;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const f32x4 v = __builtin_bit_cast(f32x4, kr[j]);
-            uint32_t a[3], c[3];
-            split3_pk(v.x, v.y, a[0], a[1], a[2]);
-            split3_pk(v.z, v.w, c[0], c[1], c[2]);
+            const f32x4 v = __builtin_bit_cast(f32x4, kr[j]) * k_up;
+            uint32_t a[kPair], c[kPair];
+            split2_f16(v.x, v.y, a[0], a[1]);
+            split2_f16(v.z, v.w, c[0], c[1]);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(st + p * kKPlane + (j ? kaddr1 : kaddr)) = u32x2{a[p], c[p]};
+            for (int p = 0; p < kPair; ++p) *reinterpret_cast<u32x2*>(st + p * kKPlane + (j ? kaddr1 : kaddr)) = u32x2{a[p], c[p]};
         }
     };
     auto store_v = [&](int slot, const u32x4(&vr)[2]) {
-        char* st = vring + slot * 3 * kVPlane;
+        char* st = vring + slot * kPair * kVPlane;
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const f32x4 v = __builtin_bit_cast(f32x4, vr[j]);
-            uint32_t a[3], c[3];
-            split3_pk(v.x, v.y, a[0], a[1], a[2]);
-            split3_pk(v.z, v.w, c[0], c[1], c[2]);
+            const f32x4 v = __builtin_bit_cast(f32x4, vr[j]) * v_up;
+            uint32_t a[kPair], c[kPair];
+            split2_f16(v.x, v.y, a[0], a[1]);
+            split2_f16(v.z, v.w, c[0], c[1]);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) *reinterpret_cast<u32x2*>(st + p * kVPlane + vaddr + j * 4 * 32) = u32x2{a[p], c[p]};
+            for (int p = 0; p < kPair; ++p) *reinterpret_cast<u32x2*>(st + p * kVPlane + vaddr + j * 4 * 32) = u32x2{a[p], c[p]};
         }
     };
 
     // fragment addresses: K rows by key = l31; V blocks by the 16-lane group (d block) and the lane's place in the 4 x 16 read
     const int koff = l31 * 128, kswz = (l31 >> 1) & 7;
     const int voff = ((lane >> 4) & 1) * kVBlock + (4 * hl + ((lane & 15) >> 2)) * 32 + (lane & 3) * 8;
-    constexpr int PK[6] = {2, 0, 1, 1, 0, 0}, PQ[6] = {0, 2, 1, 0, 1, 0};  // the six plane pairs (k or v plane, q or p plane), smallest first
-    // S^T = K Q^T of the tile in K slot `slot`: ONE accumulator chain, the 24 MFMAs back to back (an MFMA that follows another one on
+    constexpr int PK[3] = {1, 0, 0}, PQ[3] = {0, 1, 0};  // the plane pairs (k or v plane, q or p plane), smallest first
+    // S^T = K Q^T of the tile in K slot `slot`: ONE accumulator chain, the 12 MFMAs back to back (an MFMA that follows another one on
     // the same accumulator must follow it directly: anything issued between them costs the accumulate forwarding, ~43 cycles —
     // MI355X_MICROARCH.md, per-instruction constants).  Two chains taking the plane pairs in turn — which let this wave's own vector
     // work issue between MFMAs — cost 16 additions per tile to join and ran 1 % slower (89.6 against 90.6 us at 8 x 1023, same box):
     // the SIMD's other wave fills the matrix pipe's shadow anyway (tools/microbench/pingpong_probe.hip).
     auto s_tile = [&](int slot, f32x16& sa) __attribute__((always_inline)) {
-        const char* kp = kring + slot * 3 * kKPlane;
+        const char* kp = kring + slot * kPair * kKPlane;
 #pragma unroll
         for (int r = 0; r < 16; ++r) sa[r] = 0.0f;
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            bf16x8 kf[3];
+            f16x8 kf[kPair];
 #pragma unroll
-            for (int p = 0; p < 3; ++p) kf[p] = *reinterpret_cast<const bf16x8*>(kp + p * kKPlane + koff + (((2 * ks + hl) ^ kswz) << 4));
+            for (int p = 0; p < kPair; ++p) kf[p] = *reinterpret_cast<const f16x8*>(kp + p * kKPlane + koff + (((2 * ks + hl) ^ kswz) << 4));
 #pragma unroll
-            for (int t = 0; t < 6; ++t) sa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PK[t]], qf[PQ[t]][ks], sa, 0, 0, 0);
+            for (int t = 0; t < 3; ++t) sa = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[PK[t]], qf[PQ[t]][ks], sa, 0, 0, 0);
         }
     };
 
@@ -232,7 +228,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         constexpr int SLOT = decltype(SLOT_T)::value;
         constexpr bool WITH_S = decltype(WITH_S_T)::value;
         const int kt = kt0 + i;
-        // sc[r] = log2(e) / 8 * q . k of key kt * 32 + (r & 3) + 8 (r >> 2) + 4 hl against query tq
+        // sc[r] = log2(e) / 8 * q . k / s_back of key kt * 32 + (r & 3) + 8 (r >> 2) + 4 hl against query tq
         if (kt >= qb) {  // diagonal tile (and the tiles past it, which a sibling wave needs): position tq sees keys 0 .. tq
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
@@ -248,8 +244,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         // set (fp32 accumulators: probabilities up to 2^kDefer lose nothing, and the planes split them exactly) — the rescale
         // of the 32 output registers then runs on a few tiles of a row instead of all.  Everything at the old reference (O, l) is
         // rescaled at the decision, before any probability of this tile exists.
-        if (__builtin_amdgcn_ballot_w64(mx > mrun + kDefer) != 0) {
-            const float mnew = fmaxf(mrun, mx);
+        if (__builtin_amdgcn_ballot_w64(mx * s_back > mrun + kDefer) != 0) {
+            const float mnew = fmaxf(mrun, mx * s_back);
             const float corr = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mrun - mnew);  // (a row that has seen no key yet)
             lrun *= corr;
             mrun = mnew;
@@ -262,42 +258,42 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         // ---- phase A: the next tile's scores beside this tile's probabilities
         f32x16 sn;
         if constexpr (WITH_S) s_tile(SLOT ^ 1, sn);
-        const float mref = fmaxf(mrun, -1e30f);  // (all keys masked so far: 2^(-inf - mref) = 0, not NaN)
+        const float mref = kProbUp - fmaxf(mrun, -1e30f);  // (all keys masked so far: 2^(-inf - mref) = 0, not NaN)
         float psum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            sc[r] = __builtin_amdgcn_exp2f(sc[r] - mref);
+            sc[r] = __builtin_amdgcn_exp2f(fmaf(sc[r], s_back, mref));
             psum += sc[r];
         }
         lrun += both_halves_sum(psum);
-        bf16x8 pf[3][2];  // P^T fragments: registers 8 s' .. 8 s' + 7 are the lane's 8 keys of key slice s'
+        f16x8 pf[kPair][2];  // P^T fragments: registers 8 s' .. 8 s' + 7 are the lane's 8 keys of key slice s'
 #pragma unroll
         for (int sp = 0; sp < 2; ++sp) {
-            uint32_t w[4][3];
+            uint32_t w[4][kPair];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) split3_pk(sc[8 * sp + 2 * e], sc[8 * sp + 2 * e + 1], w[e][0], w[e][1], w[e][2]);
+            for (int e = 0; e < 4; ++e) split2_f16(sc[8 * sp + 2 * e], sc[8 * sp + 2 * e + 1], w[e][0], w[e][1]);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) pf[p][sp] = frag(w[0][p], w[1][p], w[2][p], w[3][p]);
+            for (int p = 0; p < kPair; ++p) pf[p][sp] = frag(w[0][p], w[1][p], w[2][p], w[3][p]);
         }
         // ---- phase B: O^T += V^T P^T beside the staging of the tiles in flight.  The lane's V fragment = keys 16 s' + 4 hl + {0..3, 8..11}
         // of head dimension l31 (+ 32).
-        const char* vp = vring + SLOT * 3 * kVPlane + voff;
+        const char* vp = vring + SLOT * kPair * kVPlane + voff;
 #pragma unroll
         for (int sp = 0; sp < 2; ++sp) {
-            bf16x8 vf[2][3];
+            f16x8 vf[2][kPair];
 #pragma unroll
             for (int dh = 0; dh < 2; ++dh)
 #pragma unroll
-                for (int p = 0; p < 3; ++p) {
+                for (int p = 0; p < kPair; ++p) {
                     const char* a = vp + p * kVPlane + 2 * dh * kVBlock + 16 * sp * 32;
                     const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a));
                     const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_ptr)(a + 8 * 32));
-                    vf[dh][p] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+                    vf[dh][p] = __builtin_bit_cast(f16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
                 }
 #pragma unroll
-            for (int t = 0; t < 6; ++t) {  // the two halves of the head dimension in turn: two accumulator chains
-                o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0][PK[t]], pf[PQ[t]][sp], o0, 0, 0, 0);
-                o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][PK[t]], pf[PQ[t]][sp], o1, 0, 0, 0);
+            for (int t = 0; t < 3; ++t) {  // the two halves of the head dimension in turn: two accumulator chains
+                o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][PK[t]], pf[PQ[t]][sp], o0, 0, 0, 0);
+                o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[1][PK[t]], pf[PQ[t]][sp], o1, 0, 0, 0);
             }
         }
         store_k(SLOT, kr);       // K(i + 2): the slot K(i) left in the previous tile's phase A
@@ -339,13 +335,13 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
 
     // O^T: the lane holds d = (r & 3) + 8 (r >> 2) + 4 hl (+ 32 in o1) of its query
     if (group_splits(g, nqb, nts) == 1) {  // softmax divides by the sum (ops.zig:239); the c_proj GEMM takes the rows as planes
-        const float inv = 1.0f / lrun;
-        bf16_t* hi = out + (row0 + tq) * kSplit * E + h * 64;
+        const float inv = 1.0f / lrun;  // (o is a mean of v's planes: it leaves with v's exponent)
+        uint16_t* hi = out + (row0 + tq) * kPair * E + h * 64;
 #pragma unroll
         for (int gq = 0; gq < 4; ++gq) {
             const int d = 8 * gq + 4 * hl;
-            store_split4(hi + d, E, f32x4{o0[gq * 4] * inv, o0[gq * 4 + 1] * inv, o0[gq * 4 + 2] * inv, o0[gq * 4 + 3] * inv});
-            store_split4(hi + 32 + d, E, f32x4{o1[gq * 4] * inv, o1[gq * 4 + 1] * inv, o1[gq * 4 + 2] * inv, o1[gq * 4 + 3] * inv});
+            store_split4(hi + d, E, f32x4{o0[gq * 4] * inv, o0[gq * 4 + 1] * inv, o0[gq * 4 + 2] * inv, o0[gq * 4 + 3] * inv}, 0, coarse);
+            store_split4(hi + 32 + d, E, f32x4{o1[gq * 4] * inv, o1[gq * 4 + 1] * inv, o1[gq * 4 + 2] * inv, o1[gq * 4 + 3] * inv}, 0, coarse);
         }
     } else {
         float* pp = part + ((((size_t)b * H + h) * P + tq) * max_s + s) * 66;
@@ -363,8 +359,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
 
 // The key ranges of a query meet: weights 2^(m_s - max m), sums in split order, one division; rows of groups that ran as one
 // range were finished by the attention kernel itself.  One thread = four head dimensions of one (sequence, head, query).
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, bf16_t* __restrict__ out, int P, int E, int H, int B,
-                                                                 unsigned geo) {
+__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int P, int E, int H, int B,
+                                                                 unsigned geo, int coarse) {
     const int nts = (int)(geo & 0xffu), max_s = (int)((geo >> 8) & 0xffu);
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const int d = (int)(i & 15) * 4;
@@ -406,17 +402,17 @@ __global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __
         }
     }
     const float inv = 1.0f / l;
-    store_split4(out + ((size_t)b * P + q) * kSplit * E + h * 64 + d, E, f32x4{o.x * inv, o.y * inv, o.z * inv, o.w * inv});
+    store_split4(out + ((size_t)b * P + q) * kPair * E + h * 64 + d, E, f32x4{o.x * inv, o.y * inv, o.z * inv, o.w * inv}, 0, coarse);
 }
 
 }  // namespace
 
-// out[M][kSplit E] = split(causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t).  ws: fp32
+// out[M][kPair E] = planes of (causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t).  ws: fp32
 // workspace for the partials of split key ranges (B H P max_splits 66 floats; none needed when every group runs as one range).
 // k_cache / v_cache != null: K and V come from the head-major fp32 caches [b][h][ctx][64] (positions 0 .. P - 1 just appended
 // by the c_attn epilogue) instead of the k / v columns of qkv.
-int launch_attn_prefill(const float* qkv, bf16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache,
-                        const float* v_cache, int ctx, hipStream_t s, int force_tiles) {
+int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache,
+                        const float* v_cache, int ctx, const int* exps, int coarse, hipStream_t s, int force_tiles) {
     static bool raised = false;
     if (!raised) {
         ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_pl_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
@@ -456,11 +452,11 @@ int launch_attn_prefill(const float* qkv, bf16_t* out, int B, int P, int E, int 
         kv = AttnKv{reinterpret_cast<const char*>(qkv + E), reinterpret_cast<const char*>(qkv + 2 * E), (size_t)P * 3 * E * 4, (size_t)256, (unsigned)(3 * E * 4)};
     }
     ZG_REQUIRE((size_t)P * kv.stride_t < ((size_t)1 << 31), ZG_ERR_SHAPE, "attention prefill: rows beyond a 32-bit buffer descriptor");
-    hipLaunchKernelGGL(attn_prefill_pl_kernel, dim3(H, B, ng * max_s), dim3(256), kLds, s, qkv, out, ws, P, E, geo, kv);
+    hipLaunchKernelGGL(attn_prefill_pl_kernel, dim3(H, B, ng * max_s), dim3(256), kLds, s, qkv, out, ws, P, E, geo, kv, exps, coarse);
     ZG_HIP(hipGetLastError());
     if (max_s > 1) {
         const size_t n = (size_t)B * H * P * 16;
-        hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, out, P, E, H, B, geo);
+        hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, out, P, E, H, B, geo, coarse);
         ZG_HIP(hipGetLastError());
     }
     return ZG_OK;

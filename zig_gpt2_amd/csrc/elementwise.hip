@@ -237,12 +237,14 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     if (row >= ja.rows + jb.rows) return;
     const bool second = row >= ja.rows;
     if (second) row -= ja.rows;
-    const float* x = (second ? jb.in : ja.in) + (size_t)row * K;
-    uint16_t* o = (second ? jb.out : ja.out) + (size_t)row * 2 * K;
-    int* e = (second ? jb.exps : ja.exps) + row;
+    const Split2Job& j = second ? jb : ja;
+    const float* x = j.in + (size_t)row * K;
+    uint16_t* o = j.out + (size_t)row * (j.lo != 0 ? K : 2 * K);
+    const size_t lo = j.lo != 0 ? j.lo : (size_t)K;
     const int n4 = K >> 2;
     f32x4 v[NV];
     uint32_t top = 0;
+    float ss = 0.0f;
     auto widen = [&](const f32x4& q) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) top = max(top, __float_as_uint(q[c]) & 0x7fffffffu);
@@ -255,18 +257,111 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
     const int up = split2_exp(top);
-    if (lane == 0) *e = -up;
-    auto leave = [&](int i, const f32x4& q) {
+    if (lane == 0) j.exps[row] = -up;
+    auto leave = [&](int i, const f32x4& in) {
+        const f32x4 q = {ldexpf(in.x, up), ldexpf(in.y, up), ldexpf(in.z, up), ldexpf(in.w, up)};
         uint32_t h0, h1, l0, l1;
-        split2_f16(ldexpf(q.x, up), ldexpf(q.y, up), h0, l0);
-        split2_f16(ldexpf(q.z, up), ldexpf(q.w, up), h1, l1);
+        split2_f16(q.x, q.y, h0, l0);
+        split2_f16(q.z, q.w, h1, l1);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) ss = fmaf(q[c], q[c], ss);
         *reinterpret_cast<u32x2*>(o + 4 * i) = u32x2{h0, h1};
-        *reinterpret_cast<u32x2*>(o + K + 4 * i) = u32x2{l0, l1};
+        *reinterpret_cast<u32x2*>(o + lo + 4 * i) = u32x2{l0, l1};
     };
 #pragma unroll
     for (int i = 0; i < NV; ++i)
         if (lane + 64 * i < n4) leave(lane + 64 * i, v[i]);
     for (int i = lane + 64 * NV; i < n4; i += 64) leave(i, *reinterpret_cast<const f32x4*>(x + 4 * i));
+    if (j.norms != nullptr) {
+        ss = wave_allsum(ss);
+        if (lane == 0) j.norms[row] = ldexpf(sqrtf(ss), -up);
+    }
+}
+
+template <int PLANES>
+__global__ __launch_bounds__(256) void join_planes_kernel(const uint16_t* __restrict__ in, const int* __restrict__ exp, int K, void* __restrict__ out) {
+    const uint16_t* r = in + (size_t)blockIdx.x * PLANES * K;
+    for (int k = threadIdx.x; k < K; k += 256) {
+        if constexpr (PLANES == 3) {
+            const float hi = __uint_as_float((uint32_t)r[k] << 16), mid = __uint_as_float((uint32_t)r[K + k] << 16), lo = __uint_as_float((uint32_t)r[2 * K + k] << 16);
+            reinterpret_cast<float*>(out)[(size_t)blockIdx.x * K + k] = hi + (mid + lo);
+        } else {
+            const float v = ldexpf((float)__builtin_bit_cast(_Float16, r[k]) + (float)__builtin_bit_cast(_Float16, r[K + k]), *exp);
+            uint32_t h, m, l;
+            split3_pk(v, 0.0f, h, m, l);
+            bf16_t* o = reinterpret_cast<bf16_t*>(out) + (size_t)blockIdx.x * 3 * K;
+            o[k] = (bf16_t)h;
+            o[K + k] = (bf16_t)m;
+            o[2 * K + k] = (bf16_t)l;
+        }
+    }
+}
+
+// bf16 rows -> one plane, a wave a row (when a matrix is loaded)
+__global__ __launch_bounds__(256) void plane_bf16_kernel(const bf16_t* __restrict__ in, int rows, int K, uint16_t* __restrict__ out, int* __restrict__ exps,
+                                                         float* __restrict__ norms) {
+    const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), n2 = K >> 1;
+    if (row >= rows) return;
+    const uint32_t* x = reinterpret_cast<const uint32_t*>(in + (size_t)row * K);
+    uint32_t top = 0;
+    float ss = 0.0f;
+    for (int i = lane; i < n2; i += 64) {
+        const float a = bf16_lo(x[i]), b = bf16_hi(x[i]);
+        top = max(top, max(__float_as_uint(a) & 0x7fffffffu, __float_as_uint(b) & 0x7fffffffu));
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
+    const int up = split2_exp(top);
+    if (lane == 0) exps[row] = -up;
+    for (int i = lane; i < n2; i += 64) {
+        const float a = ldexpf(bf16_lo(x[i]), up), b = ldexpf(bf16_hi(x[i]), up);
+        uint32_t hi, lo;
+        split2_f16(a, b, hi, lo);
+        reinterpret_cast<uint32_t*>(out + (size_t)row * K)[i] = hi;
+        ss = fmaf(a, a, fmaf(b, b, ss));
+    }
+    ss = wave_allsum(ss);
+    if (lane == 0 && norms != nullptr) norms[row] = ldexpf(sqrtf(ss), -up);
+}
+
+// one workgroup: the exponents of a layer's activations (PrefillBounds); bounds go to [2^11, 2^12), so that values four binades beyond (a row whose
+// variance is cancelled away in 32 bits) still are fp16 numbers
+__global__ __launch_bounds__(256) void prefill_bounds_kernel(const PrefillBounds a, int E) {
+    __shared__ float s_red[4];
+    auto all = [&](float v, bool sum) {
+        v = sum ? wave_allsum(v) : wave_allmax(v);
+        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        const float r = sum ? (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]) : fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
+        __syncthreads();
+        return r;
+    };
+    auto most = [&](const float* p, int n) {  // the largest that is finite
+        float m = 0.0f;
+        for (int i = threadIdx.x; i < n; i += 256) m = fmaxf(m, fabsf(p[i]) < INFINITY ? fabsf(p[i]) : 0.0f);
+        return all(m, false);
+    };
+    auto length = [&](const float* p, int n) {
+        const float m = most(p, n);
+        float t = 0.0f;
+        for (int i = threadIdx.x; i < n; i += 256) {
+            const float v = m > 0.0f && fabsf(p[i]) < INFINITY ? p[i] / m : 0.0f;
+            t += v * v;
+        }
+        return m * sqrtf(all(t, true));
+    };
+    auto set = [&](int which, float bound) {
+        if (threadIdx.x != 0) return;
+        // (no bound, or one beyond fp32's range: the planes are what they are without a factor of more than 2^+-100)
+        const int e = bound > 0.0f ? (int)((__float_as_uint(fminf(bound, 3.0e38f)) >> 23) & 255u) - 127 : 0;
+        a.exps[which] = min(max(e - 11, -100), 100);
+    };
+    const float r = sqrtf((float)E);
+    const float a1 = r * most(a.ln_1_g, E) + length(a.ln_1_b, E), a2 = r * most(a.ln_2_g, E) + length(a.ln_2_b, E);
+    set(PB_LN1, a1);
+    set(PB_LN2, a2);
+    for (int p = 0; p < 3; ++p) set(PB_Q + p, a1 * most(a.c_attn_norms + p * E, E) + most(a.c_attn_b + p * E, E));
+    set(PB_GELU, a2 * most(a.c_fc_norms, 4 * E) + most(a.c_fc_b, 4 * E));
 }
 
 __device__ __forceinline__ float load_emb(const void* w, int wt, size_t off) {
@@ -685,6 +780,32 @@ int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s) 
     const dim3 grid((unsigned)((a.rows + b.rows + 3) / 4));
     if (K <= 768) split2_kernel<3><<<grid, 256, 0, s>>>(a, b, K);
     else split2_kernel<8><<<grid, 256, 0, s>>>(a, b, K);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_join_planes(const uint16_t* in, const int*, int rows, int K, int planes, float* out, hipStream_t s) {
+    ZG_REQUIRE(planes == 3, ZG_ERR_ARG, "join_planes: %d", planes);
+    join_planes_kernel<3><<<dim3((unsigned)rows), 256, 0, s>>>(in, nullptr, K, out);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, bf16_t* out, hipStream_t s) {
+    ZG_REQUIRE(planes == kPair, ZG_ERR_ARG, "join_planes: %d", planes);
+    join_planes_kernel<kPair><<<dim3((unsigned)rows), 256, 0, s>>>(in, exp, K, out);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s) {
+    ZG_REQUIRE(rows > 0 && K > 0 && K % 2 == 0, ZG_ERR_UNSUPPORTED, "plane_bf16: %d rows of %d", rows, K);
+    plane_bf16_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(in, rows, K, out, exps, norms);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_prefill_bounds(const PrefillBounds& b, int E, hipStream_t s) {
+    prefill_bounds_kernel<<<1, 256, 0, s>>>(b, E);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

@@ -147,7 +147,7 @@ __device__ __forceinline__ void acc_read16(float (&v)[16]) {  // the 16 register
     acc_read8<BASE + 8>(v + 8);
 }
 template <int BASE>
-__device__ __forceinline__ void acc_write16(const u32x4 (&v)[4]) {  // sixteen accumulator registers from four loaded quads (SK)
+__device__ __forceinline__ void acc_write16(const u32x4 (&v)[4]) {  // sixteen accumulator registers from four quads
     asm volatile(
         "v_accvgpr_write_b32 a[%c16], %0\n\tv_accvgpr_write_b32 a[%c17], %1\n\tv_accvgpr_write_b32 a[%c18], %2\n\tv_accvgpr_write_b32 a[%c19], %3\n\t"
         "v_accvgpr_write_b32 a[%c20], %4\n\tv_accvgpr_write_b32 a[%c21], %5\n\tv_accvgpr_write_b32 a[%c22], %6\n\tv_accvgpr_write_b32 a[%c23], %7\n\t"
@@ -210,15 +210,15 @@ __device__ __forceinline__ void read_b_all(bf16x8 (&fb)[4][NT], const unsigned (
 //               order and finish (bias, residual, LayerNorm + plane split)
 //   S4_QKV      bias, fp32 rows of qkv[M][3E] AND the cache append of src/ops.zig:152-157 for the K / V columns
 //   S4_RELU2    bias, then max(., 0)^2, rows as S4_PLAIN            (the layered tier's dense feed-forward)
-//   S4_SPLIT3   bias + GELU, then the exact three-term bf16 split as planes C[M][3N] = [hi | mid | lo]  (src/main.zig:79-80 feeding
-//               the next Linear's A operand)
+//   S4_SPLIT2   bias + GELU, then the two-term fp16 split as planes C[M][2N] = [hi | lo]  (src/main.zig:79-80 feeding
+//               the next Linear's A operand); F16 only
 
 // F16: the planes are the two-term fp16 split of rows scaled by powers of two (zg_common.h split2_f16): the finished sums are scaled back by
 // the exponents of their row and column, and the bias is added behind that (the accumulators start at zero).
 template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
 __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                          const float* __restrict__ bias, void* __restrict__ C, int M, int N,
-                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex) {
+                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
     // All 14 dwords of the arguments are preloaded into SGPRs at wave launch (zg_common.h ZG_PIN): the first version passed the
     // plane description and the tile counts behind them and began with a scalar round trip to the kernarg segment — cold for
     // every launch — before its first DMA.  p0 = lda | ldb << 16; p1 = ldc | K-steps per plane << 20 | plane pairs << 28;
@@ -237,7 +237,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     const int gw = (int)(p2 >> 24);
     const int dbg = (int)((p3 >> 10) & 0x3ffu);
     const int n_sl = KIND == S4_PARTIAL ? (int)((p3 >> 20) & 0xffu) : 1;  // K slices: slice s of a tile walks K-steps [s kps, (s + 1) kps) of every plane
-    const bool b_major = (p3 >> 31) != 0u;  // B = three plane matrices [3][N][ldb] (fp32 weights of the model) instead of planes side by side in a row
+    const bool b_major = (p3 >> 31) != 0u;  // B = two plane matrices [2][N][ldb] (fp32 weights of the model) instead of planes side by side in a row
     const int tiles_m = (M + 255) >> 8, tiles_n = (N + P::BN - 1) / P::BN;
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
@@ -257,7 +257,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     // empty): G workgroups, R G + G / 2 tiles.  Every workgroup walks R whole tiles and HALF of one of the last G / 2: the K-steps
     // [0, kpp / 2) of every plane (the producer: even place in its XCD, item 0 — it then spills its 192 accumulators per lane to
     // sk_ws and raises a per-wave flag) or [kpp / 2, kpp) (the consumer: odd place — dispatched behind its producer — last item:
-    // its accumulators START at the producer's partial, which left more than a whole tile earlier, and it runs the epilogue).
+    // it runs the epilogue and adds the producer's partial there, which left more than a whole tile earlier).
     int it = 0;
     const int sk_R = SK ? tmn / G : 0, sk_gx = G >> 3;  // (SK: G % 16 == 0, tmn = sk_R G + G / 2: the launcher's conditions)
     const bool sk_cons = SK && (loc & 1);
@@ -305,7 +305,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (unsigned)((size_t)M * pl.lda * 2), 0x00020000);
     const __amdgpu_buffer_rsrc_t rb =
-        __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (unsigned)((size_t)N * pl.ldb * 2) * (b_major ? 3u : 1u), 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)B, 0, (unsigned)((size_t)N * pl.ldb * 2) * (b_major ? 2u : 1u), 0x00020000);
     // The tile's bias row travels through LDS (wave 0 fetches it by LDS-DMA at the start of the tile; columns past N and a
     // null bias read as zero): the epilogue must not issue a global load — the compiler would wait for it with vmcnt(0),
     // i.e. drain the stores and the next tile's DMA — and 48 registers of bias held across the epilogue make the register
@@ -608,6 +608,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         s1 = s2;
     };
 
+    [[maybe_unused]] int out_exp = 0;  // S4_SPLIT2
     // F16: half way through the leading products the sums leave their leading eight bits aside and go on with the rest (both exact), so that the second
     // half is rounded at its own size: with 11-bit terms a chain of 768 products is 1.71e-7 off, in two halves 1.2e-7, which makes room for
     // what the split leaves (0.75e-7); three exact bf16 terms in one chain are 1.58e-7 off.  8192 x 768 x 3072: 136 us of a call without, 150 with.
@@ -643,7 +644,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     // through; then, its stores drained, one flag word per wave = this launch's epoch (the consumer's wave w polls wave w's flag
     // and loads exactly what that wave stored: no workgroup barrier on either side).  The poll is bounded: a consumer that
     // ran out raises g_s4_fault and carries on (the host checks the word where it drains the stream).
-    auto sk_spill = [&]() {
+    auto sk_spill = [&]() __attribute__((always_inline)) {
         if constexpr (SK) {
             acc_settle();
             const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(qa.sk_ws, 0, (unsigned)(G >> 1) * 196608u, 0x00020000);
@@ -652,6 +653,12 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 constexpr int q = decltype(QT)::value;
                 float av[16];
                 acc_read16<16 * q>(av);
+                const u32x8v lead = aside[q];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    av[2 * e] += bf16_lo(lead[e]);
+                    av[2 * e + 1] += bf16_hi(lead[e]);
+                }
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     const f32x4v v4 = {av[4 * e], av[4 * e + 1], av[4 * e + 2], av[4 * e + 3]};
@@ -662,7 +669,8 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             if (lane == 0) __hip_atomic_store(qa.sk_flags + sk_sh * 4 + wave, qa.sk_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
-    auto sk_init_from_partial = [&]() {
+    // the consumer's half starts at zero and meets its producer's in the epilogue (two halves, each rounded at its own size)
+    auto sk_wait = [&]() {
         if constexpr (SK) {
             unsigned spins = 0;
             while (__hip_atomic_load(qa.sk_flags + sk_sh * 4 + wave, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != qa.sk_epoch) {
@@ -674,16 +682,6 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             }
             // the partial's loads must not be hoisted above the flag: agent-scope acquire (the poll itself is relaxed)
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(qa.sk_ws, 0, (unsigned)(G >> 1) * 196608u, 0x00020000);
-            const unsigned base = (unsigned)(sk_sh * 4 + wave) * 49152u + (unsigned)lane * 16u;
-            static_for<12>([&](auto QT) {
-                constexpr int q = decltype(QT)::value;
-                u32x4 v[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rw, base + (unsigned)(q * 4 + e) * 1024u, 0, 16);
-                acc_write16<16 * q>(v);
-            });
-            asm volatile("s_nop 7" ::: ZG_ACC_CLOBBERS);  // v_accvgpr_write -> MFMA source C
         }
     };
     auto epilogue = [&]() __attribute__((always_inline)) {
@@ -712,6 +710,8 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             for (int i = 0; i < 4; ++i) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(rexp[i]) : "v"(raddr), "i"(i * 128));
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(rexp[0]), "+v"(rexp[1]), "+v"(rexp[2]), "+v"(rexp[3]));
         }
+        [[maybe_unused]] const __amdgpu_buffer_rsrc_t rpart = __builtin_amdgcn_make_buffer_rsrc(qa.sk_ws, 0, SK ? (unsigned)(G >> 1) * 196608u : 0u, 0x00020000);
+        if (SK && role_cur == 2) sk_wait();
         [[maybe_unused]] auto scale_back = [&](auto IT, auto JT, int row_exp, float (&av)[16]) __attribute__((always_inline)) {
             constexpr int j = decltype(JT)::value, q = decltype(IT)::value * NT + j;
             const u32x8v lead = aside[q];
@@ -719,6 +719,14 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             for (int e = 0; e < 8; ++e) {
                 av[2 * e] += bf16_lo(lead[e]);
                 av[2 * e + 1] += bf16_hi(lead[e]);
+            }
+            if (SK && role_cur == 2) {
+                const unsigned base = (unsigned)(sk_sh * 4 + wave) * 49152u + (unsigned)lane_e * 16u;
+                u32x4 v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rpart, base + (unsigned)(q * 4 + e) * 1024u, 0, 16);
+#pragma unroll
+                for (int e = 0; e < 16; ++e) av[e] += __uint_as_float(v[e >> 2][e & 3]);
             }
             const unsigned caddr = exps + (unsigned)(wc * (P::BN / 2) + 4 * hhe) * 4u;
             f32x4v b4[4];
@@ -749,30 +757,37 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 g_off[k] = (col < N ? (unsigned)(m0 + wr * 128 + row) * (unsigned)(ldc * 2) + (unsigned)col * 2u : 0xFFFFFFFFu) | no_store_mask;
             }
         }
-        if constexpr (KIND == S4_SPLIT3) {
-            // GELU, then the three planes of an m-tile one after the other through the wave's staging image (its LDS accesses
+        if constexpr (KIND == S4_SPLIT2) {
+            // GELU, then the two planes of an m-tile one after the other through the wave's staging image (its LDS accesses
             // complete in order: plane p + 1 is written behind the reads of plane p without a wait)
+            const int out_up = -out_exp;
             static_for<4>([&](auto IT) {
                 constexpr int i = decltype(IT)::value;
-                u32x2 w[3][NT][4];
+                u32x2 w[2][NT][4];
                 static_for<NT>([&](auto JT) {
                     constexpr int j = decltype(JT)::value;
                     asm volatile("s_nop 3" ::: "memory");
                     float av[16];
                     acc_read16<16 * (i * NT + j)>(av);
+                    scale_back(IT, JT, rexp[i], av);
                     f32x2v x[8];
 #pragma unroll
                     for (int k = 0; k < 8; ++k) x[k] = gelu2(f32x2v{av[2 * k], av[2 * k + 1]});
+                    if (po.coarse)
+#pragma unroll
+                        for (int k = 0; k < 8; ++k) x[k] = f32x2v{coarse16(x[k].x), coarse16(x[k].y)};
+#pragma unroll
+                    for (int k = 0; k < 8; ++k) x[k] = f32x2v{__builtin_amdgcn_ldexpf(x[k].x, out_up), __builtin_amdgcn_ldexpf(x[k].y, out_up)};
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
-                        uint32_t a[3], b[3];
-                        split3_pk(x[2 * g].x, x[2 * g].y, a[0], a[1], a[2]);
-                        split3_pk(x[2 * g + 1].x, x[2 * g + 1].y, b[0], b[1], b[2]);
+                        uint32_t a[2], b[2];
+                        split2_f16(x[2 * g].x, x[2 * g].y, a[0], a[1]);
+                        split2_f16(x[2 * g + 1].x, x[2 * g + 1].y, b[0], b[1]);
 #pragma unroll
-                        for (int p = 0; p < 3; ++p) w[p][j][g] = u32x2{a[p], b[p]};
+                        for (int p = 0; p < 2; ++p) w[p][j][g] = u32x2{a[p], b[p]};
                     }
                 });
-                static_for<3>([&](auto PT) {
+                static_for<2>([&](auto PT) {
                     constexpr int p = decltype(PT)::value;
                     static_for<NT>([&](auto JT) {
                         constexpr int j = decltype(JT)::value;
@@ -792,7 +807,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                     static_assert(NCH == 6, "staging read-back written for NT = 3");
                     asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(o[0]), "+v"(o[1]), "+v"(o[2]), "+v"(o[3]), "+v"(o[4]), "+v"(o[5]));
 #pragma unroll
-                    for (int k = 0; k < NCH; ++k) {  // plane p of row m: columns [p N, (p + 1) N) of the 3 N-wide row
+                    for (int k = 0; k < NCH; ++k) {  // plane p of row m: columns [p N, (p + 1) N) of the 2 N-wide row
                         const unsigned off = g_off[k] == 0xFFFFFFFFu ? g_off[k] : g_off[k] + (unsigned)(i * 32) * (unsigned)(ldc * 2) + (unsigned)(p * N) * 2u;
                         __builtin_amdgcn_raw_buffer_store_b128(o[k], rc, off, 0, ST_AUX);
                     }
@@ -959,10 +974,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 }
             }
         });
-        if (has_nxt) {  // the next tile starts at its bias row — or, a consumer's half tile, at its producer's partial
-            if (SK && role_nxt == 2) sk_init_from_partial();
-            else init_acc_from_bias(par_after(tile_par, 1));
-        }
+        if (has_nxt) init_acc_from_bias(par_after(tile_par, 1));  // the next tile starts at its bias row (F16: at zero)
         if constexpr (NPEND > 0) {
             pend_row = row0;
             pend_col = col0;
@@ -1021,6 +1033,10 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         for (int i = 0; i < 4; ++i) dma_a(0, 1, i, s0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dma_a(1, 0, i, s1);
+        if constexpr (KIND == S4_SPLIT2) {
+            out_exp = *po.exp;
+            ZG_PIN(out_exp);
+        }
         if constexpr (KIND == S4_QKV) {  // the epilogue's argument-block fields, fetched under the first DMA
             ZG_PIN(qa.P); ZG_PIN(qa.E); ZG_PIN(qa.H); ZG_PIN(qa.ctx); ZG_PIN(qa.kv_mode); ZG_PIN(qa.kv_lo); ZG_PIN(qa.k_cache); ZG_PIN(qa.v_cache);
         }
@@ -1081,7 +1097,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
 
 template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
 int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, int n_sl,
-                  const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}) {
+                  const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}, const PlaneOut& po = PlaneOut{}) {
     using P = S4<NT>;
     constexpr int LDS = F16 ? P::LDS_F16 : P::LDS;
     static OncePerDevice raised;  // (handles of the layered tier may be on different devices)
@@ -1108,7 +1124,7 @@ int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
     }
     hipLaunchKernelGGL((gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK, F16>), dim3(grid), dim3(256), LDS, s, A, B, bias, C, M, N,
                        (unsigned)pl.lda | ((unsigned)pl.ldb << 16), (unsigned)ldc | ((unsigned)pl.kpp << 20) | ((unsigned)pl.npairs << 28),
-                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa, ex);
+                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa, ex, po);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1178,42 +1194,32 @@ int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, vo
                     : launch_s4_kind<3, S4_RELU2, false, false>(A, B, bias, C, M, N, pl, ldc, 1, none, s);
 }
 
-// The whole-prompt Linears on the same kernel (prefill.hip decides when): A = the activation planes [M][nplanes K] (hi | mid | lo),
-// W = the bf16 weight [N][K]; the planes are plane pairs of ONE K loop, smallest first — a tile's accumulators see 3 K / 64
-// K-steps between two epilogues.  nplanes == kWeightPlanes: W = the three plane matrices [3][N][K] of an fp32 weight, and the six
-// plane products a_i w_j, i + j <= 2, are the pairs (6 K / 64 K-steps per tile; what is dropped is below 2^-24 of the leading
-// term).  kind: S4_PARTIAL (C = fp32 slabs [n_slices][M][N], bias must be null), S4_QKV (C = qkv [M][N] fp32 + cache append),
-// S4_SPLIT3 (C = bf16 planes [M][3 N] of gelu(...)).
-int launch_gemm_s4_prefill(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int nplanes, int kind, int n_slices,
-                           const PrefillQkv* qkv, hipStream_t s) {
-    ZG_REQUIRE(M > 0 && N % 64 == 0 && K % 64 == 0 && K >= 128 && (nplanes == 2 || nplanes == 3 || nplanes == kWeightPlanes), ZG_ERR_UNSUPPORTED,
-               "s4 prefill gemm: M=%d N=%d K=%d planes=%d", M, N, K, nplanes);
+// The whole-prompt Linears on the same kernel (prefill.hip decides when): A = the activation planes [M][2 K] (hi | lo), W = one plane [N][K] or two;
+// the plane products are pairs of ONE K loop, smallest first — (lo, w) (hi, w), or (lo, hi) (hi, lo) (hi, hi).  kind: S4_PARTIAL (C = fp32 slabs
+// [n_slices][M][N], bias must be null), S4_QKV (C = qkv [M][N] fp32 + cache append), S4_SPLIT2 (C = planes [M][2 N] of gelu(...)).
+int launch_gemm_s4_prefill(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int kind, int n_slices,
+                           const PrefillQkv* qkv, const PlaneOut& po, hipStream_t s) {
+    ZG_REQUIRE(M > 0 && N % 64 == 0 && K % 64 == 0 && K >= 128, ZG_ERR_UNSUPPORTED, "s4 prefill gemm: M=%d N=%d K=%d", M, N, K);
     GemmPlanes pl{};
-    pl.lda = kSplit * K;  // the plane buffer always holds three planes per row; nplanes = 2 multiplies hi + mid only
+    pl.lda = kPair * K;
     pl.ldb = K;
     pl.kpp = K / 64;
-    if (nplanes == kWeightPlanes) {  // (a, w) = (lo, hi) (mid, mid) (hi, lo) (mid, hi) (hi, mid) (hi, hi): smallest terms first
-        pl.npairs = 6;
-        pl.pa_bits = 0x001012u;
-        pl.pb_bits = 0x010210u;
-        pl.b_plane_major = true;
-        ZG_REQUIRE((size_t)N * K * 2 * 3 < ((size_t)1 << 31), ZG_ERR_SHAPE, "s4 prefill gemm: weight planes of %d x %d beyond a 32-bit buffer descriptor", N, K);
-    } else {
-        pl.npairs = nplanes;
-        pl.pa_bits = nplanes == 3 ? 0x012u : 0x01u;  // pair 0 = the smallest plane
-        pl.pb_bits = 0;
-    }
-    const int ldc = kind == S4_SPLIT3 ? kSplit * N : N;
-    const size_t out_bytes = (size_t)(kind == S4_PARTIAL ? n_slices : 1) * M * ldc * (kind == S4_SPLIT3 ? 2 : 4);
-    ZG_REQUIRE(out_bytes < ((size_t)1 << 32) && (size_t)M * pl.lda * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 < ((size_t)1 << 31), ZG_ERR_SHAPE,
+    pl.npairs = W.planes == 2 ? 3 : 2;
+    pl.pa_bits = W.planes == 2 ? 0x001u : 0x01u;  // pair 0 = the smallest
+    pl.pb_bits = W.planes == 2 ? 0x010u : 0x00u;
+    pl.b_plane_major = W.planes == 2;
+    const int ldc = kind == S4_SPLIT2 ? kPair * N : N;
+    const size_t out_bytes = (size_t)(kind == S4_PARTIAL ? n_slices : 1) * M * ldc * (kind == S4_SPLIT2 ? 2 : 4);
+    ZG_REQUIRE(out_bytes < ((size_t)1 << 32) && (size_t)M * pl.lda * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 * W.planes < ((size_t)1 << 31), ZG_ERR_SHAPE,
                "s4 prefill gemm: operands of %d x %d x %d beyond the 32-bit buffer descriptors", M, N, K);
     ZG_REQUIRE(n_slices >= 1 && pl.kpp % n_slices == 0 && pl.kpp / n_slices >= 2, ZG_ERR_ARG, "s4 prefill gemm: %d K slices of %d K-steps", n_slices, pl.kpp);
     const PrefillQkv none{};
+    const PlaneExps ex{A.exp, W.exps, A.each};
     gemm_note_launch();
     switch (kind) {
         case S4_PARTIAL:
             ZG_REQUIRE(bias == nullptr, ZG_ERR_ARG, "s4 prefill gemm: partial slabs carry no bias");
-            return launch_s4_kind<3, S4_PARTIAL, false, false>(A, W, nullptr, C, M, N, pl, ldc, n_slices, none, s);
+            return launch_s4_kind<3, S4_PARTIAL, false, false, false, true>(A.p, W.p, nullptr, C, M, N, pl, ldc, n_slices, none, s, ex);
         case S4_QKV: {
             ZG_REQUIRE(qkv && N == 3 * qkv->E && n_slices == 1, ZG_ERR_ARG, "s4 prefill gemm: S4_QKV needs the cache description");
             // 1.5 rounds of tiles (c_attn of eight 1023-token prompts: 384 tiles, 256 CUs): the last half round is split in K halves
@@ -1222,12 +1228,12 @@ int launch_gemm_s4_prefill(const bf16_t* A, const bf16_t* W, const float* bias, 
             const int G = cus_env > 0 ? cus_env : 256, tiles = ((M + 255) / 256) * ((N + 191) / 192);
             if (qkv->sk_ws != nullptr && qkv->sk_flags != nullptr && G % 16 == 0 && tiles > G && (tiles % G) * 2 == G && pl.kpp % 2 == 0 &&
                 pl.kpp >= 4 && (size_t)(G / 2) * 196608 <= qkv->sk_ws_bytes && (size_t)(G / 2) * 4 <= qkv->sk_flags_words)
-                return launch_s4_kind<3, S4_QKV, false, false, true>(A, W, bias, C, M, N, pl, ldc, 1, *qkv, s);
-            return launch_s4_kind<3, S4_QKV, false, false>(A, W, bias, C, M, N, pl, ldc, 1, *qkv, s);
+                return launch_s4_kind<3, S4_QKV, false, false, true, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
+            return launch_s4_kind<3, S4_QKV, false, false, false, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
         }
-        case S4_SPLIT3:
-            ZG_REQUIRE(n_slices == 1, ZG_ERR_ARG, "s4 prefill gemm: S4_SPLIT3 is not sliced");
-            return launch_s4_kind<3, S4_SPLIT3, true, true>(A, W, bias, C, M, N, pl, ldc, 1, none, s);
+        case S4_SPLIT2:
+            ZG_REQUIRE(n_slices == 1 && po.exp, ZG_ERR_ARG, "s4 prefill gemm: S4_SPLIT2 is not sliced");
+            return launch_s4_kind<3, S4_SPLIT2, true, true, false, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, none, s, ex, po);
     }
     ZG_REQUIRE(false, ZG_ERR_ARG, "s4 prefill gemm: kind %d", kind);
 }

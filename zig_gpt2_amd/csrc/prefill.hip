@@ -2,18 +2,16 @@
 // GPT.forward (src/main.zig:331-334); here the n prompt positions of every sequence go through each Block
 // together, so the Linears become GEMMs on the matrix cores and attention becomes one causal pass.
 //
-// Numerics.  The decode path keeps activations in fp32 and weights in bf16 (exact products, fp32
-// accumulation).  To stay inside the same tolerance the GEMM A operand here is the fp32 activation split
-// into three bf16 terms, x = hi + mid + lo EXACTLY (24 = 8 + 8 + 8 mantissa bits; a two-term split leaves
-// 2^-18 |x| behind, which showed up as 2e-5 of the logit scale — outside the parity bar for logits that
-// happen to lie near zero), laid out [M][3K] = [hi | mid | lo]; every staged weight tile is multiplied with
-// the three planes, so C = (hi + mid + lo) W^T accumulates in one fp32 MFMA chain.  Attention (attn_prefill.hip) splits q, k, v
-// and the probabilities the same way and multiplies the six plane products above 2^-24.
+// Numerics.  Activations stay fp32 values with two-term fp16 planes standing for them in the matrix products (zg_common.h split2_f16: 23 bits), laid
+// out [M][2K] = [hi | lo] and scaled by a power of two that is known from the weights (launch_prefill_bounds); a bf16 weight is one fp16 plane of
+// its row times a power of two, an fp32 weight two.  Products of two planes (bf16 weights) or three (fp32) stand where exact bf16 terms take three and six.
+// Sums of the leading products are cut into runs that start at zero, so that a result is closer to 64 bits than one chain of
+// exact products.  Attention (attn_prefill.hip) treats q, k, v and the probabilities the same way.
 //
 // Kernels
 //   embed_prefill      x[m] = wte[token[m]] + wpe[t]                         (src/main.zig:179-183)
 //   ln_split           a = split(LayerNorm(x))                               (src/ops.zig:82-104)
-//   prefill_gemm       128 x 128 (or 128 x 256) x 64 tile, weight tile shared by the three planes, LDS-DMA double
+//   prefill_gemm       128 x 128 (or 128 x 256) x 64 tile, weight tile shared by the planes, LDS-DMA double
 //                      buffer, epilogues:
 //                        F32 store | fp32 residual add | GELU + split        (ops.zig:21-46, main.zig:136-145, :79-80)
 //   (cache append)     K / V columns of the qkv rows -> head-major caches, in the c_attn GEMM epilogue (ops.zig:152-158)
@@ -22,16 +20,15 @@
 
 #include "prefill_epi.h"
 #include "zg_kernels.h"
+#include "zg_once.h"
 
 namespace zg {
-
-int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, bf16_t* out, hipStream_t s);
 
 namespace {
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 typedef const __attribute__((address_space(1))) void* gbl_ptr_t;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 // ------------------------------------------------------------------------------------------ embed
@@ -62,7 +59,8 @@ __global__ __launch_bounds__(256) void embed_prefill_kernel(const int* __restric
 // std = sqrt(E[x^2] - mean^2 + eps), (x - mean) / std * g + b   (src/ops.zig:88-101).
 __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__ x, int M, int E,
                                                        const float* __restrict__ g, const float* __restrict__ bta,
-                                                       float eps, bf16_t* __restrict__ out) {
+                                                       float eps, uint16_t* __restrict__ out, const PlaneOut po) {
+    const int exp = *po.exp;
     const int lane = threadIdx.x & 63, row = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (row >= M) return;
     const float* xr = x + (size_t)row * E;
@@ -76,7 +74,7 @@ __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__
     ss = wave_allsum(ss);
     const float mean = s / (float)E;
     const float sd = sqrtf(ss / (float)E - mean * mean + eps);
-    bf16_t* hi = out + (size_t)row * kSplit * E;
+    uint16_t* hi = out + (size_t)row * kPair * E;
     for (int e = lane * 4; e < E; e += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(xr + e);
         const f32x4 gg = *reinterpret_cast<const f32x4*>(g + e);
@@ -86,7 +84,7 @@ __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__
         o.y = (v.y - mean) / sd * gg.y + bb.y;
         o.z = (v.z - mean) / sd * gg.z + bb.z;
         o.w = (v.w - mean) / sd * gg.w + bb.w;
-        store_split4(hi + e, E, o);
+        store_split4(hi + e, E, o, exp, po.coarse);
     }
 }
 
@@ -94,17 +92,17 @@ __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__
 constexpr int BM = 128, BN = 128, BK = 64;
 constexpr int kTileBytes = BM * BK * 2;
 constexpr int kStages = 2;
-// stage = weight tile (128 NS rows) + the three activation planes: 64 KiB (NS = 1) or 80 KiB (NS = 2)
-constexpr int stage_bytes(int ns) { return (ns + kSplit) * kTileBytes; }
-constexpr int lds_bytes(int ns) { return kStages * stage_bytes(ns); }  // 128 / 160 KiB; reused as store staging
+// stage = weight tile (128 NS rows) + the two activation planes: 48 KiB (NS = 1) or 64 KiB (NS = 2)
+constexpr int stage_bytes(int ns) { return (ns + kPair) * kTileBytes; }
+constexpr int lds_bytes(int ns) { return kStages * stage_bytes(ns); }  // 96 / 128 KiB; reused as store staging
 
-__device__ __forceinline__ bf16x8 read_frag(const char* lds_tile, int row, int chunk) {
+__device__ __forceinline__ f16x8 read_frag(const char* lds_tile, int row, int chunk) {
     const int off = row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4);
-    return *reinterpret_cast<const bf16x8*>(lds_tile + off);
+    return *reinterpret_cast<const f16x8*>(lds_tile + off);
 }
 
-// A: [M][3K] bf16 (hi | mid | lo), B: [N][K] bf16, bias [N].  C: fp32 [M][ldc] (PF_F32, PF_RESID) or bf16
-// [M][3N] split planes (PF_GELU_SPLIT).  N % 64 == 0, K % 64 == 0, any M.
+// A: planes [M][2K] (hi | lo), B: one plane [N][K], bias [N].  C: fp32 [M][ldc] (PF_F32, PF_RESID) or planes [M][2N]
+// (PF_GELU_SPLIT).  N % 64 == 0, K % 64 == 0, any M.
 // (the body is shared by prefill_gemm_kernel and prefill_gemm_wp_kernel: sp = K slice of this workgroup, slab = the partial
 // slab it writes under PF_PARTIAL)
 #ifdef ZG_PF_STAMPS  // diagnostic build only (tools/pf_stamps.py): where one wave of a prompt GEMM spends its K loop
@@ -123,15 +121,13 @@ __device__ unsigned long long g_pf_stamps[32];
 #define ZG_PFS(i, expr) expr
 #endif
 template <int EPI, int NS, int NSPL>  // NS 64-column strips per wave: the tile is 128 x (128 NS); NSPL activation planes multiplied
-__device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B, const float* __restrict__ bias,
+__device__ __forceinline__ void prefill_gemm_body(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B, const float* __restrict__ bias,
                                                   void* __restrict__ C, int M, int N, int K, int ldc, unsigned tp, int n_tiles,
-                                                  const PrefillQkv& qa, const int sp, const int slab) {
+                                                  const PrefillQkv& qa, const PlaneExps& ex, const PlaneOut& po, const int sp, const int slab) {
     // tp = tiles_n | split-K slices << 12 | rows of the XCD grid << 24: the 14 preloaded argument dwords carry everything the
     // first DMA depends on (zg_common.h ZG_PIN; gridDim is a scalar load from the kernarg segment)
     const int tiles_n = (int)(tp & 0xfffu);
-    // nsplit = activation planes multiplied: 3 = exact fp32 activations (hi + mid + lo), 2 = hi + mid only
-    // (2^-17 relative per activation, ~2e-5 of the logit scale end to end: inside north_star's 1e-3, outside the
-    // strict near-zero floor of the tests; 2/3 of the matrix work)
+    // NSPL = activation planes multiplied: both, or the leading one (with the lesser plane of an fp32 weight)
     extern __shared__ __attribute__((aligned(1024))) char lds[];
 #ifdef ZG_PF_STAMPS
     const unsigned long long pfs_entry = __builtin_readcyclecounter();
@@ -163,18 +159,16 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
     constexpr int BNT = BN * NS, NJ = 2 * NS, kStageB = stage_bytes(NS), kBBytes = NS * kTileBytes;
     const int m0 = tm * BM, n0 = tn * BNT;
 
-    f32x16 acc[2][NJ];
+    f32x16 acc[2][NJ], total[2][NJ];  // total: the sums of finished runs of four K-steps
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = total[i][j][r] = 0.0f;
 
-    // A K-step stages ONE 128 x 64 weight tile and the matching tile of each of the three activation planes;
-    // the weight fragments are read from LDS once and multiplied with all three planes (the first version
-    // walked the weight rows once per plane: 2 tiles per 16 MFMAs, and was bound by LDS-DMA at ~7 TB/s; this
-    // is 4 tiles per 48 MFMAs).  Two 64-KiB slots: the DMA of step t + 1 runs under the MFMAs of step t.
+    // A K-step stages ONE 128 x 64 weight tile and the matching tile of the activation planes; the weight fragments are read
+    // from LDS once and multiplied with all of them.  Two slots: the DMA of step t + 1 runs under the MFMAs of step t.
     // Split-K slice sp takes the K-steps [t0, nt).
     const int nk = K / BK;
     const int t0 = (int)((long)nk * sp / n_sp), nt = (int)((long)nk * (sp + 1) / n_sp);
@@ -186,15 +180,15 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
     // arrive as zeros (they are never stored).
     constexpr int NPC = 4 * NS + 4 * NSPL;  // pieces per wave and K-step
     const int wv = __builtin_amdgcn_readfirstlane(wave);
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(A), 0, (unsigned)((size_t)M * kSplit * K * 2), 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(B), 0, (unsigned)((size_t)N * K * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(A), 0, (unsigned)((size_t)M * kPair * K * 2), 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(B), 0, (unsigned)((size_t)N * K * 2), 0x00020000);
     unsigned rel_a[2], rel_b[2];
     {
         const unsigned l3 = (unsigned)lane >> 3, pos = (unsigned)lane & 7u;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
             const unsigned chunk = pos ^ (((l3 >> 1) + 4u * e) & 7u);
-            rel_a[e] = l3 * (unsigned)(kSplit * K * 2) + chunk * 16u;
+            rel_a[e] = l3 * (unsigned)(kPair * K * 2) + chunk * 16u;
             rel_b[e] = l3 * (unsigned)(K * 2) + chunk * 16u;
         }
     }
@@ -208,7 +202,7 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
             __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(slot + piece * 1024), 16, rel_b[idx & 1], soff, 0, 0);
         } else {
             const int p = (idx - 4 * NS) >> 2, q = (idx - 4 * NS) & 3, piece = wv * 4 + q;
-            const unsigned soff = ((unsigned)(m0 + piece * 8) * (unsigned)(kSplit * K) + (unsigned)(p * K + t * BK)) * 2u + kill;
+            const unsigned soff = ((unsigned)(m0 + piece * 8) * (unsigned)(kPair * K) + (unsigned)(p * K + t * BK)) * 2u + kill;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(slot + kBBytes + p * kTileBytes + piece * 1024), 16, rel_a[q & 1], soff, 0, 0);
         }
     };
@@ -240,7 +234,7 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
 #endif
         const unsigned kill = more ? 0u : 0x80000000u;  // (operands < 2 GiB: offset + kill never wraps, and lies past every descriptor's end)
         const char* cur = lds + ((t - t0) & 1) * kStageB;
-        // 12 groups (16-k slice kk, plane p = 2, 1, 0: smallest plane first) of 2 NJ MFMAs.  The fragments of group g + 1 are
+        // Groups (16-k slice kk, plane p = 1, 0: smallest plane first) of 2 NJ MFMAs.  The fragments of group g + 1 are
         // read IN FRONT of group g's MFMAs (two register sets, sched barriers pin the order): with one wave per SIMD nothing
         // else covers the LDS latency — the first version read a group's fragments, waited, multiplied, and spent as long
         // waiting as multiplying.  Only the first group of a K-step is exposed (its data arrives with the barrier above).
@@ -248,9 +242,9 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
         // the prefetched ones included — in front of every group.)
         // The reads are hand-issued (asm) with COUNTED waits: left to itself the compiler waits for lgkmcnt(0) in front of
         // every second group, i.e. also for the reads it has just issued for the group after.
-        bf16x8 bq[2][NJ], aq[2][NSPL][2];
+        f16x8 bq[2][NJ], aq[2][NSPL][2];
         const unsigned cur_a = (unsigned)(unsigned long)(lds_ptr_t)cur;
-        auto rd = [&](bf16x8& dst, unsigned tile_off, int row, int chunk) {
+        auto rd = [&](f16x8& dst, unsigned tile_off, int row, int chunk) {
             const unsigned addr = cur_a + tile_off + (unsigned)(row * 128 + ((chunk ^ ((row >> 1) & 7)) << 4));
             asm volatile("ds_read_b128 %0, %1" : "=v"(dst) : "v"(addr));
         };
@@ -259,7 +253,7 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
         constexpr int RS = NJ + 2 * NSPL;   // fragment reads per slice
         constexpr int MS = 2 * NJ * NSPL;   // MFMAs per slice
         constexpr int RSLOT = (RS + 1) / 2; // MFMAs of a slice that carry two reads of the next slice each
-        auto rd_item = [&](int kk, int r, bf16x8(&bb)[NJ], bf16x8(&aa)[NSPL][2]) {
+        auto rd_item = [&](int kk, int r, f16x8(&bb)[NJ], f16x8(&aa)[NSPL][2]) {
             if (r < NJ) rd(bb[r], 0u, wn * 64 * NS + r * 32 + frow, kk * 2 + fk);
             else {
                 const int pi = (r - NJ) >> 1, i = (r - NJ) & 1, p = NSPL - 1 - pi;
@@ -288,9 +282,7 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
             // front of the wait (sched_barrier pins instruction order, not what register allocation inserts).
 #define ZG_TIE2(x) "+v"(x[0]), "+v"(x[1])
 #define ZG_TIE4(x) "+v"(x[0]), "+v"(x[1]), "+v"(x[NJ > 2 ? 2 : 0]), "+v"(x[NJ > 2 ? 3 : 1])
-            if constexpr (NSPL == 3 && NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(aq[cb][1]), ZG_TIE2(aq[cb][2]), ZG_TIE2(bq[cb])::"memory");
-            else if constexpr (NSPL == 3) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(aq[cb][1]), ZG_TIE2(aq[cb][2]), ZG_TIE4(bq[cb])::"memory");
-            else if constexpr (NSPL == 2 && NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(aq[cb][1]), ZG_TIE2(bq[cb])::"memory");
+            if constexpr (NSPL == 2 && NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(aq[cb][1]), ZG_TIE2(bq[cb])::"memory");
             else if constexpr (NSPL == 2) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(aq[cb][1]), ZG_TIE4(bq[cb])::"memory");
             else if constexpr (NJ == 2) asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE2(bq[cb])::"memory");
             else asm volatile("s_waitcnt lgkmcnt(0)" : ZG_TIE2(aq[cb][0]), ZG_TIE4(bq[cb])::"memory");
@@ -300,7 +292,7 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
 #pragma unroll
             for (int m = 0; m < MS; ++m) {
                 const int pi = m / (2 * NJ), i = (m / NJ) & 1, j = m % NJ, p = NSPL - 1 - pi;
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aq[cb][p][i], bq[cb][j], acc[i][j], 0, 0, 0);
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq[cb][p][i], bq[cb][j], acc[i][j], 0, 0, 0);
                 __builtin_amdgcn_sched_barrier(0);
                 if (m < RSLOT) {
 #if !(defined(ZG_PF_ABL) && (ZG_PF_ABL & 2))
@@ -320,7 +312,21 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
+        if (((t - t0) & 3) == 3)  // a run ends: the next one is rounded at its own size (768 columns: 1.7e-7 from 64 bits in one chain, 1.0e-7 in three)
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        total[i][j][r] += acc[i][j][r];
+                        acc[i][j][r] = 0.0f;
+                    }
     }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] += total[i][j];
 #ifdef ZG_PF_STAMPS
     const unsigned long long pfs_t1 = __builtin_readcyclecounter();
 #endif
@@ -336,26 +342,30 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             const int col = j * 32 + frow;
-            const float bv = (EPI != PF_PARTIAL && bias) ? bias[nw + col] : 0.0f;
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int row = i * 32 + (r & 3) + 8 * (r >> 2) + 4 * fk;
-                    float v = acc[i][st * 2 + j][r] + bv;
-                    if (EPI == PF_GELU_SPLIT) v = gelu_fast(v);
-                    wtile[row * 64 + col] = v;
+                    wtile[row * 64 + col] = acc[i][st * 2 + j][r];
                 }
         }
+        const int cc = lane & 15;
+        const i32x4 col_exp = *reinterpret_cast<const i32x4*>(ex.w + nw + cc * 4);
+        const f32x4 bv = EPI != PF_PARTIAL && bias ? *reinterpret_cast<const f32x4*>(bias + nw + cc * 4) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int it = 0; it < 16; ++it) {
-            const int c = it * 64 + lane;
-            const int row = c >> 4, cc = c & 15;
+            const int row = it * 4 + (lane >> 4);
             const int gm = m0 + wm * 64 + row;
             if (gm >= M) continue;
+            const int row_exp = ex.a[ex.a_each ? gm : 0];
             f32x4 v = *reinterpret_cast<const f32x4*>(wtile + row * 64 + cc * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], row_exp + col_exp[e]) + bv[e];
             if (EPI == PF_GELU_SPLIT) {
-                store_split4(reinterpret_cast<bf16_t*>(C) + (size_t)gm * kSplit * N + nw + cc * 4, N, v);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = gelu_fast(v[e]);
+                store_split4(reinterpret_cast<uint16_t*>(C) + (size_t)gm * kPair * N + nw + cc * 4, N, v, *po.exp, po.coarse);
             } else if (EPI == PF_PARTIAL) {  // C is the workspace [n_sp][M][N]
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)slab * M + gm) * N + nw + cc * 4) = v;
             } else {
@@ -379,30 +389,26 @@ __device__ __forceinline__ void prefill_gemm_body(const bf16_t* __restrict__ A, 
 #endif
 }
 
-template <int EPI, int NS, int NSPL = kSplit>
-__global__ __launch_bounds__(256, 1) void prefill_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+template <int EPI, int NS>
+__global__ __launch_bounds__(256, 1) void prefill_gemm_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                                               const float* __restrict__ bias, void* __restrict__ C, int M,
                                                               int N, int K, int ldc, unsigned tp, int n_tiles,
-                                                              const PrefillQkv qa) {
-    prefill_gemm_body<EPI, NS, NSPL>(A, B, bias, C, M, N, K, ldc, tp, n_tiles, qa, (int)blockIdx.y, (int)blockIdx.y);
+                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
+    prefill_gemm_body<EPI, NS, kPair>(A, B, bias, C, M, N, K, ldc, tp, n_tiles, qa, ex, po, (int)blockIdx.y, (int)blockIdx.y);
 }
 
-// fp32 WEIGHTS: B is the exact three-term bf16 split of the fp32 matrix, plane-major [3][N][K] (hi, mid, lo).  The six plane
-// products above 2^-24 of the leading one are three passes over the K slices — w_lo x a_hi, w_mid x (a_mid + a_hi),
-// w_hi x (a_lo + a_mid + a_hi): one weight plane each with 1 / 2 / 3 activation planes — dealt over blockIdx.y = pass * n_sp +
-// slice and written as partial slabs in that order (smallest terms first), which the reduce kernels sum and finish.  One
-// launch per Linear; 128-row tiles and K slices fill the chip at any prompt length.
+// fp32 WEIGHTS: B is the two planes [2][N][K] (hi, lo).  The three plane products are two passes over the K slices — w_lo x a_hi, w_hi x (a_lo + a_hi) —
+// dealt over blockIdx.y = pass * n_sp + slice and written as partial slabs in that order (smallest terms first), which the reduce kernels sum and
+// finish.  One launch per Linear; 128-row tiles and K slices fill the chip at any prompt length.
 template <int NS>
-__global__ __launch_bounds__(256, 1) void prefill_gemm_wp_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
+__global__ __launch_bounds__(256, 1) void prefill_gemm_wp_kernel(const uint16_t* __restrict__ A, const uint16_t* __restrict__ B,
                                                                  const float* __restrict__ bias, void* __restrict__ C, int M, int N,
-                                                                 int K, int ldc, unsigned tp, int n_tiles, const PrefillQkv qa) {
+                                                                 int K, int ldc, unsigned tp, int n_tiles, const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
     const int n_sp = (int)((tp >> 12) & 0xfffu), y = (int)blockIdx.y;
-    // dispatched heaviest first (w_hi with three activation planes), slabs ordered smallest terms first
-    const int sched = y / n_sp, sp = y - sched * n_sp, slab = (2 - sched) * n_sp + sp;
-    const size_t plane = (size_t)N * K;
-    if (sched == 0) prefill_gemm_body<PF_PARTIAL, NS, 3>(A, B, bias, C, M, N, K, ldc, tp, n_tiles, qa, sp, slab);
-    else if (sched == 1) prefill_gemm_body<PF_PARTIAL, NS, 2>(A, B + plane, bias, C, M, N, K, ldc, tp, n_tiles, qa, sp, slab);
-    else prefill_gemm_body<PF_PARTIAL, NS, 1>(A, B + 2 * plane, bias, C, M, N, K, ldc, tp, n_tiles, qa, sp, slab);
+    // dispatched heaviest first (w_hi with both activation planes), slabs ordered smallest terms first
+    const int sched = y / n_sp, sp = y - sched * n_sp, slab = (1 - sched) * n_sp + sp;
+    if (sched == 0) prefill_gemm_body<PF_PARTIAL, NS, 2>(A, B, bias, C, M, N, K, ldc, tp, n_tiles, qa, ex, po, sp, slab);
+    else prefill_gemm_body<PF_PARTIAL, NS, 1>(A, B + (size_t)N * K, bias, C, M, N, K, ldc, tp, n_tiles, qa, ex, po, sp, slab);
 }
 
 // Four columns of one row summed over the K-slice slabs, in slab order.  The loads go out four slabs at a time before the
@@ -427,7 +433,7 @@ __device__ __forceinline__ f32x4 sum_slabs(const float* __restrict__ ws, int n_s
 template <int EPI>
 __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __restrict__ ws, int n_sp,
                                                              const float* __restrict__ bias, void* __restrict__ C, int M,
-                                                             int N, int ldc, const PrefillQkv qa) {
+                                                             int N, int ldc, const PrefillQkv qa, const PlaneOut po) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const int n4 = N / 4;
     if (i >= (size_t)M * n4) return;
@@ -436,7 +442,7 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
     if (bias) v += *reinterpret_cast<const f32x4*>(bias + n);
     if (EPI == PF_GELU_SPLIT) {
         v.x = gelu_fast(v.x); v.y = gelu_fast(v.y); v.z = gelu_fast(v.z); v.w = gelu_fast(v.w);
-        store_split4(reinterpret_cast<bf16_t*>(C) + (size_t)m * kSplit * N + n, N, v);
+        store_split4(reinterpret_cast<uint16_t*>(C) + (size_t)m * kPair * N + n, N, v, *po.exp, po.coarse);
     } else {
         float* dst = reinterpret_cast<float*>(C) + (size_t)m * ldc + n;
         if (EPI == PF_RESID) v += *reinterpret_cast<const f32x4*>(dst);
@@ -448,13 +454,14 @@ __global__ __launch_bounds__(256) void prefill_reduce_kernel(const float* __rest
 // Split-K tail of a residual GEMM fused with the LayerNorm that follows it (main.zig:139-140 / the next
 // Block's ln_1): one workgroup per row, a float4 (two beyond E = 1024) per thread — the slices are summed in
 // fixed order, bias and the residual stream added, x stored, then the row it just produced is normalised and
-// written as the three bf16 planes of the next GEMM.  Two launches (reduce, ln_split) become one.
+// written as the planes of the next GEMM.  Two launches (reduce, ln_split) become one.
 __global__ __launch_bounds__(256) void prefill_reduce_resid_ln_kernel(const float* __restrict__ ws, int n_sp,
                                                                       const float* __restrict__ bias, float* __restrict__ x,
                                                                       int M, int N, const float* __restrict__ g,
                                                                       const float* __restrict__ bta, float eps,
-                                                                      bf16_t* __restrict__ out) {
+                                                                      uint16_t* __restrict__ out, const PlaneOut po) {
     __shared__ float s_red[8];
+    const int exp = *po.exp;
     const int row = blockIdx.x, tid = threadIdx.x, n4 = N >> 2;
     float* xr = x + (size_t)row * N;
     f32x4 v[2];
@@ -487,7 +494,7 @@ __global__ __launch_bounds__(256) void prefill_reduce_resid_ln_kernel(const floa
     ss = (s_red[1] + s_red[3]) + (s_red[5] + s_red[7]);
     const float mean = s / (float)N;
     const float sd = sqrtf(ss / (float)N - mean * mean + eps);
-    bf16_t* hi = out + (size_t)row * kSplit * N;
+    uint16_t* hi = out + (size_t)row * kPair * N;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int i = tid + 256 * j;
@@ -500,9 +507,25 @@ __global__ __launch_bounds__(256) void prefill_reduce_resid_ln_kernel(const floa
             o.y = (v[j].y - mean) / sd * gg.y + bb.y;
             o.z = (v[j].z - mean) / sd * gg.z + bb.z;
             o.w = (v[j].w - mean) / sd * gg.w + bb.w;
-            store_split4(hi + e, N, o);
+            store_split4(hi + e, N, o, exp, po.coarse);
         }
     }
+}
+
+// the second half of a Linear whose product lies in K-slice slabs of ws: their sum and the epilogue, a residual Linear's with the LayerNorm behind it
+template <int EPI>
+int finish_slabs(const float* ws, int n_sp, const float* bias, void* C, int M, int N, int ldc, const PrefillLn* ln, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
+    if (EPI == PF_RESID && ln && ldc == N && N <= 2048) {
+        hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, n_sp, bias, reinterpret_cast<float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out,
+                           ln->po);
+        ZG_HIP(hipGetLastError());
+        return ZG_OK;
+    }
+    const size_t n = (size_t)M * (N / 4);
+    hipLaunchKernelGGL((prefill_reduce_kernel<EPI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, n_sp, bias, C, M, N, ldc, qa, po);
+    ZG_HIP(hipGetLastError());
+    if (EPI == PF_RESID && ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, ln->po, s);
+    return ZG_OK;
 }
 
 // Rows of the XCD grid for a tiles_m x tiles_n launch (prefill_gemm_body): the divisor pair that makes an XCD's L2 fetch the
@@ -523,18 +546,18 @@ static unsigned xcd_grid_rows(int tiles_m, int tiles_n, size_t a_tile, size_t w_
     return best;
 }
 
-template <int EPI, int NS, int NSPL>
-int launch_prefill_gemm_np(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc,
-                           float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, hipStream_t s) {
-    constexpr int nsplit = NSPL;
-    static bool raised = false;
-    if (!raised) {
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<EPI, NS, NSPL>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NS)));
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<PF_PARTIAL, NS, NSPL>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NS)));
-        raised = true;
-    }
+template <int EPI, int NS>
+int launch_prefill_gemm_np(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc,
+                           float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
+    static OncePerDevice raised;
+    int device = 0;
+    ZG_HIP(hipGetDevice(&device));
+    ZG_TRY(raised.run(device, []() -> int {
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<EPI, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NS)));
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_kernel<PF_PARTIAL, NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NS)));
+        return ZG_OK;
+    }));
+    const PlaneExps ex{A.exp, W.exps, A.each};
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN * NS - 1) / (BN * NS), tiles = tiles_m * tiles_n;
     // Few output tiles (N = n_embed, or a short prompt): slice K so that about one workgroup per CU exists
     // (the LDS ring allows one), at least 3 K-steps per slice, partial sums through the workspace.
@@ -543,78 +566,57 @@ int launch_prefill_gemm_np(const bf16_t* A, const bf16_t* B, const float* bias, 
     if (n_sp > nt / 3) n_sp = nt / 3;
     if (n_sp < 1) n_sp = 1;
     while (n_sp > 1 && (size_t)n_sp * M * N > ws_floats) --n_sp;
-    const unsigned xg = xcd_grid_rows(tiles_m, tiles_n, (size_t)BM * (K / (n_sp > 1 && ws ? n_sp : 1)) * 2 * nsplit,
+    const unsigned xg = xcd_grid_rows(tiles_m, tiles_n, (size_t)BM * (K / (n_sp > 1 && ws ? n_sp : 1)) * 2 * kPair,
                                       (size_t)BN * NS * (K / (n_sp > 1 && ws ? n_sp : 1)) * 2);
     if (n_sp <= 1 || !ws) {
-        hipLaunchKernelGGL((prefill_gemm_kernel<EPI, NS, NSPL>), dim3(tiles), dim3(256), lds_bytes(NS), s, A, B, bias, C, M, N, K,
-                           ldc, (unsigned)tiles_n | (1u << 12) | (xg << 24), tiles, qa);
+        hipLaunchKernelGGL((prefill_gemm_kernel<EPI, NS>), dim3(tiles), dim3(256), lds_bytes(NS), s, A.p, W.p, bias, C, M, N, K,
+                           ldc, (unsigned)tiles_n | (1u << 12) | (xg << 24), tiles, qa, ex, po);
     } else {
-        hipLaunchKernelGGL((prefill_gemm_kernel<PF_PARTIAL, NS, NSPL>), dim3(tiles, n_sp), dim3(256), lds_bytes(NS), s, A, B, bias,
-                           (void*)ws, M, N, K, ldc, (unsigned)tiles_n | ((unsigned)n_sp << 12) | (xg << 24), tiles, qa);
-        if (EPI == PF_RESID && ln && ldc == N && N <= 2048) {
-            hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, n_sp, bias,
-                               reinterpret_cast<float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out);
-            ZG_HIP(hipGetLastError());
-            return ZG_OK;
-        }
-        const size_t n = (size_t)M * (N / 4);
-        hipLaunchKernelGGL((prefill_reduce_kernel<EPI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, n_sp, bias, C,
-                           M, N, ldc, qa);
+        hipLaunchKernelGGL((prefill_gemm_kernel<PF_PARTIAL, NS>), dim3(tiles, n_sp), dim3(256), lds_bytes(NS), s, A.p, W.p, bias,
+                           (void*)ws, M, N, K, ldc, (unsigned)tiles_n | ((unsigned)n_sp << 12) | (xg << 24), tiles, qa, ex, po);
+        return finish_slabs<EPI>(ws, n_sp, bias, C, M, N, ldc, ln, qa, po, s);
     }
     ZG_HIP(hipGetLastError());
-    if (EPI == PF_RESID && ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, s);
+    if (EPI == PF_RESID && ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, ln->po, s);
     return ZG_OK;
 }
 
-// fp32 weights (nsplit = kWeightPlanes): prefill_gemm_wp_kernel + the reduce kernels (which apply the epilogue)
+// fp32 weights: prefill_gemm_wp_kernel + the reduce kernels (which apply the epilogue)
 template <int EPI, int NS>
-int launch_prefill_gemm_wp(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc, float* ws,
-                           size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, hipStream_t s) {
-    static bool raised = false;
-    if (!raised) {
+int launch_prefill_gemm_wp(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, float* ws,
+                           size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
+    static OncePerDevice raised;
+    int device = 0;
+    ZG_HIP(hipGetDevice(&device));
+    ZG_TRY(raised.run(device, []() -> int {
         ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_gemm_wp_kernel<NS>), hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(NS)));
-        raised = true;
-    }
+        return ZG_OK;
+    }));
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN * NS - 1) / (BN * NS), tiles = tiles_m * tiles_n;
     const int nt = K / BK;
-    int n_sp = (256 + 3 * tiles - 1) / (3 * tiles);  // three passes per slice: about one workgroup per CU in all
+    int n_sp = (256 + 2 * tiles - 1) / (2 * tiles);  // two passes per slice: about one workgroup per CU in all
     if (n_sp > nt / 3) n_sp = nt / 3;
     if (n_sp < 1) n_sp = 1;
-    while (n_sp > 1 && (size_t)3 * n_sp * M * N > ws_floats) --n_sp;
-    ZG_REQUIRE(ws && (size_t)3 * n_sp * M * N <= ws_floats, ZG_ERR_ARG, "prefill GEMM (fp32 weights): workspace of %zu floats for %d x %d", ws_floats, M, N);
-    const unsigned xg = xcd_grid_rows(tiles_m, tiles_n, (size_t)BM * (K / n_sp) * 2 * 3, (size_t)BN * NS * (K / n_sp) * 2);
-    hipLaunchKernelGGL((prefill_gemm_wp_kernel<NS>), dim3(tiles, 3 * n_sp), dim3(256), lds_bytes(NS), s, A, B, bias, (void*)ws, M, N, K, ldc,
-                       (unsigned)tiles_n | ((unsigned)n_sp << 12) | (xg << 24), tiles, qa);
-    if (EPI == PF_RESID && ln && ldc == N && N <= 2048) {
-        hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, 3 * n_sp, bias, reinterpret_cast<float*>(C), M, N, ln->g,
-                           ln->b, ln->eps, ln->out);
-        ZG_HIP(hipGetLastError());
-        return ZG_OK;
-    }
-    const size_t n = (size_t)M * (N / 4);
-    hipLaunchKernelGGL((prefill_reduce_kernel<EPI>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, 3 * n_sp, bias, C, M, N, ldc, qa);
-    ZG_HIP(hipGetLastError());
-    if (EPI == PF_RESID && ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, s);
-    return ZG_OK;
+    while (n_sp > 1 && (size_t)2 * n_sp * M * N > ws_floats) --n_sp;
+    ZG_REQUIRE(ws && (size_t)2 * n_sp * M * N <= ws_floats, ZG_ERR_ARG, "prefill GEMM (fp32 weights): workspace of %zu floats for %d x %d", ws_floats, M, N);
+    const unsigned xg = xcd_grid_rows(tiles_m, tiles_n, (size_t)BM * (K / n_sp) * 2 * kPair, (size_t)BN * NS * (K / n_sp) * 2);
+    hipLaunchKernelGGL((prefill_gemm_wp_kernel<NS>), dim3(tiles, 2 * n_sp), dim3(256), lds_bytes(NS), s, A.p, W.p, bias, (void*)ws, M, N, K, ldc,
+                       (unsigned)tiles_n | ((unsigned)n_sp << 12) | (xg << 24), tiles, qa, PlaneExps{A.exp, W.exps, A.each}, po);
+    return finish_slabs<EPI>(ws, 2 * n_sp, bias, C, M, N, ldc, ln, qa, po, s);
 }
 
-template <int EPI, int NS>
-int launch_prefill_gemm_ns(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc,
-                           float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, int nsplit, hipStream_t s) {
-    if (nsplit == kWeightPlanes) return launch_prefill_gemm_wp<EPI, NS>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, s);
-    if (nsplit == 2) return launch_prefill_gemm_np<EPI, NS, 2>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, s);
-    return launch_prefill_gemm_np<EPI, NS, kSplit>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, s);
-}
-
-// 128 x 256 tiles (the staged weight tile is shared by the three planes, so widening N is the cheap direction:
-// 157 FLOP per staged byte against 96) once there are enough rows to fill the chip with them, else 128 x 128.
+// 128 x 256 tiles (the staged weight tile is shared by the planes, so widening N is the cheap direction)
+// once there are enough rows to fill the chip with them, else 128 x 128.
 template <int EPI>
-int launch_prefill_gemm_t(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc,
-                          float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, int nsplit, hipStream_t s) {
+int launch_prefill_gemm_t(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc,
+                          float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
     const int wide_tiles = ((M + BM - 1) / BM) * ((N + 2 * BN - 1) / (2 * BN));
     const bool wide = wide_tiles >= 256 && N >= 2 * BN;
-    if (wide) return launch_prefill_gemm_ns<EPI, 2>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, nsplit, s);
-    return launch_prefill_gemm_ns<EPI, 1>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, nsplit, s);
+    if (W.planes == 2)
+        return wide ? launch_prefill_gemm_wp<EPI, 2>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s)
+                    : launch_prefill_gemm_wp<EPI, 1>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s);
+    return wide ? launch_prefill_gemm_np<EPI, 2>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s)
+                : launch_prefill_gemm_np<EPI, 1>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s);
 }
 
 }  // namespace
@@ -627,8 +629,8 @@ int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, cons
     return ZG_OK;
 }
 
-int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, bf16_t* out, hipStream_t s) {
-    hipLaunchKernelGGL(ln_split_kernel, dim3((M + 3) / 4), dim3(256), 0, s, x, M, E, g, b, eps, out);
+int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, uint16_t* out, const PlaneOut& po, hipStream_t s) {
+    hipLaunchKernelGGL(ln_split_kernel, dim3((M + 3) / 4), dim3(256), 0, s, x, M, E, g, b, eps, out, po);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -649,7 +651,7 @@ static int s4_route(int M, int N, int K, int epi, size_t ws_floats, bool have_ws
     if (g_force_kernel >= 16) min_tiles = g_force_kernel;  // (measurement: another threshold)
     if (g_force_kernel == 2) return 0;
     const int kpp = K / 64;
-    if (K % 64 != 0 || kpp < 2 || kSplit * K >= 65536) return 0;
+    if (K % 64 != 0 || kpp < 2 || kPair * K >= 65536) return 0;
     const long tiles = (long)((M + 255) / 256) * ((N + 191) / 192);
     if (epi != PF_RESID) return tiles >= min_tiles ? 1 : 0;
     if (!have_ws) return 0;
@@ -672,56 +674,42 @@ static int s4_route(int M, int N, int K, int epi, size_t ws_floats, bool have_ws
     return best;
 }
 
-// the second half of a residual Linear whose product lies in K-slice slabs of ws: their sum, bias and residual (C [M][N]), and the LayerNorm behind it
-static int finish_resid(const float* ws, int n_sp, const float* bias, void* C, int M, int N, int ldc, const PrefillLn* ln, hipStream_t s) {
-    if (ln && N <= 2048) {
-        hipLaunchKernelGGL(prefill_reduce_resid_ln_kernel, dim3(M), dim3(256), 0, s, ws, n_sp, bias, reinterpret_cast<float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out);
-        ZG_HIP(hipGetLastError());
-        return ZG_OK;
-    }
-    const size_t n = (size_t)M * (N / 4);
-    hipLaunchKernelGGL((prefill_reduce_kernel<PF_RESID>), dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, n_sp, bias, C, M, N, ldc, PrefillQkv{});
-    ZG_HIP(hipGetLastError());
-    if (ln) return launch_ln_split(reinterpret_cast<const float*>(C), M, N, ln->g, ln->b, ln->eps, ln->out, s);
-    return ZG_OK;
-}
-
-int launch_prefill_gemm(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, int K, int ldc, int epi,
-                        float* ws, size_t ws_floats, const PrefillLn* ln, hipStream_t s, const PrefillQkv* qkv, int nsplit) {
+int launch_prefill_gemm(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi,
+                        float* ws, size_t ws_floats, const PrefillLn* ln, hipStream_t s, const PrefillQkv* qkv, const PlaneOut& po) {
     ZG_REQUIRE(M > 0 && N >= 64 && N % 64 == 0 && K >= 64 && K % 64 == 0, ZG_ERR_UNSUPPORTED, "prefill gemm: M=%d N=%d K=%d", M, N, K);
+    ZG_REQUIRE((W.planes == 1 || W.planes == 2) && A.exp && W.exps && (epi != PF_GELU_SPLIT || po.exp), ZG_ERR_ARG, "prefill gemm: %d weight planes", W.planes);
+    const PrefillQkv none{};
     {
         const int n_sl = s4_route(M, N, K, epi, ws_floats, ws != nullptr);
         if (n_sl > 0 && epi == PF_RESID && ldc == N) {
-            ZG_TRY(launch_gemm_s4_prefill(A, B, nullptr, ws, M, N, K, nsplit, S4_PARTIAL, n_sl, nullptr, s));
-            return finish_resid(ws, n_sl, bias, C, M, N, ldc, ln, s);
+            ZG_TRY(launch_gemm_s4_prefill(A, W, nullptr, ws, M, N, K, S4_PARTIAL, n_sl, nullptr, po, s));
+            return finish_slabs<PF_RESID>(ws, n_sl, bias, C, M, N, ldc, ln, none, po, s);
         }
-        if (n_sl == 1 && epi == PF_GELU_SPLIT) return launch_gemm_s4_prefill(A, B, bias, C, M, N, K, nsplit, S4_SPLIT3, 1, nullptr, s);
-        if (n_sl == 1 && epi == PF_QKV && qkv && ldc == N) return launch_gemm_s4_prefill(A, B, bias, C, M, N, K, nsplit, S4_QKV, 1, qkv, s);
+        if (n_sl == 1 && epi == PF_GELU_SPLIT) return launch_gemm_s4_prefill(A, W, bias, C, M, N, K, S4_SPLIT2, 1, nullptr, po, s);
+        if (n_sl == 1 && epi == PF_QKV && qkv && ldc == N) return launch_gemm_s4_prefill(A, W, bias, C, M, N, K, S4_QKV, 1, qkv, po, s);
     }
     if (g_force_kernel == 0 || g_force_kernel == 3) {  // prompts of some hundred rows (prefill_ring.hip)
         int tm = 1;
-        const bool planes = nsplit == kWeightPlanes, resid = epi == PF_RESID;
-        const int n_sp = (nsplit == kSplit || planes) && (!resid || (ldc == N && ws)) ? prefill_ring_route(M, N, K, resid, planes, ws_floats, g_force_kernel == 3, &tm) : 0;
-        if (n_sp > 0 && (size_t)N * K * 2 * 3 < ((size_t)1 << 31) && (size_t)M * kSplit * K * 2 < ((size_t)1 << 31)) {
-            ZG_TRY(launch_prefill_ring(A, B, bias, resid ? static_cast<void*>(ws) : C, M, N, K, ldc, resid ? PF_PARTIAL : epi, planes, tm, n_sp, qkv ? *qkv : PrefillQkv{}, s));
-            return resid ? finish_resid(ws, n_sp, bias, C, M, N, ldc, ln, s) : ZG_OK;
+        const bool resid = epi == PF_RESID;
+        const int n_sp = !resid || (ldc == N && ws) ? prefill_ring_route(M, N, K, resid, W.planes == 2, ws_floats, g_force_kernel == 3, &tm) : 0;
+        if (n_sp > 0 && (size_t)N * K * 2 * 2 < ((size_t)1 << 31) && (size_t)M * kPair * K * 2 < ((size_t)1 << 31)) {
+            ZG_TRY(launch_prefill_ring(A, W, bias, resid ? static_cast<void*>(ws) : C, M, N, K, ldc, resid ? PF_PARTIAL : epi, tm, n_sp, qkv ? *qkv : none, po, s));
+            return resid ? finish_slabs<PF_RESID>(ws, n_sp, bias, C, M, N, ldc, ln, none, po, s) : ZG_OK;
         }
     }
     // (the operands are addressed through 32-bit buffer descriptors; a piece is switched off by adding 2 GiB to its scalar offset,
     // which must then lie past the descriptor's end without wrapping: operands < 2 GiB.  That a raw buffer access is range-checked
     // on voffset + soffset — LLVM documents only voffset — is pinned on the hardware by tools/microbench/soffset_bounds_probe.hip,
     // tests/test_hw_rules_gpu.py)
-    ZG_REQUIRE((size_t)M * kSplit * K * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 < ((size_t)1 << 31), ZG_ERR_UNSUPPORTED,
+    ZG_REQUIRE((size_t)M * kPair * K * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 < ((size_t)1 << 31), ZG_ERR_UNSUPPORTED,
                "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
-    ZG_REQUIRE(nsplit == 2 || nsplit == kSplit || nsplit == kWeightPlanes, ZG_ERR_ARG, "prefill gemm: %d activation planes", nsplit);
-    const PrefillQkv none{};
     switch (epi) {
-        case PF_F32: return launch_prefill_gemm_t<PF_F32>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, none, nsplit, s);
-        case PF_RESID: return launch_prefill_gemm_t<PF_RESID>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, ln, none, nsplit, s);
-        case PF_GELU_SPLIT: return launch_prefill_gemm_t<PF_GELU_SPLIT>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, none, nsplit, s);
+        case PF_F32: return launch_prefill_gemm_t<PF_F32>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, none, po, s);
+        case PF_RESID: return launch_prefill_gemm_t<PF_RESID>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, none, po, s);
+        case PF_GELU_SPLIT: return launch_prefill_gemm_t<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, none, po, s);
         case PF_QKV:
             ZG_REQUIRE(qkv && N == 3 * qkv->E && ldc == N, ZG_ERR_ARG, "prefill gemm: PF_QKV needs the cache description");
-            return launch_prefill_gemm_t<PF_QKV>(A, B, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, *qkv, nsplit, s);
+            return launch_prefill_gemm_t<PF_QKV>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, nullptr, *qkv, po, s);
     }
     ZG_REQUIRE(false, ZG_ERR_ARG, "prefill gemm: epilogue %d", epi);
 }

@@ -4,14 +4,20 @@
 
 namespace zg {
 
-// four consecutive values -> 8 B into each of the kSplit planes (plane stride `plane` elements); the split
-// is exact: x = hi + mid + lo (zg_common.h split3_pk)
-__device__ __forceinline__ void store_split4(bf16_t* dst, size_t plane, f32x4 v) {
-    uint32_t a[3], b[3];
-    split3_pk(v.x, v.y, a[0], a[1], a[2]);
-    split3_pk(v.z, v.w, b[0], b[1], b[2]);
+// 16 significant bits (ZG_GPT_PREFILL_2PLANE)
+__device__ __forceinline__ float coarse16(float x) {
+    const uint32_t b = __float_as_uint(x);
+    return __uint_as_float((b + 0x7fu + ((b >> 8) & 1u)) & ~0xffu);
+}
+
+// four consecutive values -> 8 B into each of the two planes (plane stride `plane` elements), times 2^-exp
+__device__ __forceinline__ void store_split4(uint16_t* dst, size_t plane, f32x4 v, int exp, int coarse) {
+    if (coarse) v = f32x4{coarse16(v.x), coarse16(v.y), coarse16(v.z), coarse16(v.w)};
+    uint32_t a[2], b[2];
+    split2_f16(ldexpf(v.x, -exp), ldexpf(v.y, -exp), a[0], a[1]);
+    split2_f16(ldexpf(v.z, -exp), ldexpf(v.w, -exp), b[0], b[1]);
 #pragma unroll
-    for (int p = 0; p < kSplit; ++p) *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{a[p], b[p]};
+    for (int p = 0; p < kPair; ++p) *reinterpret_cast<u32x2*>(dst + p * plane) = u32x2{a[p], b[p]};
 }
 
 __device__ __forceinline__ float gelu_fast(float x) {

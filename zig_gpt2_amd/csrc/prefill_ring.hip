@@ -1,13 +1,14 @@
 // prefill_ring.hip — the Linears of the whole-prompt pass (src/ops.zig:21-46 for M = batch x prompt rows) where the large tiles leave the chip
 // idle: prompts of some hundred rows.
 //
-// A = the activation planes [M][3 K] (hi | mid | lo), W = the bf16 weight [N][K], or the three plane matrices [3][N][K] of an fp32 weight.  All the
-// products of a K step of 64 columns are made from ONE staging of the planes (three, or the six above 2^-24 of the leading one), where
-// the 128-row kernels of prefill.hip walk an fp32 weight in three passes that each stage the activations again and meet in slabs.
-// What bounds it: a compute unit takes in some 30 bytes a clock (48 KB a step of a 64 x 64 tile of six products: 1600 clocks, beside 768 of
+// A = the activation planes [M][2 K] (hi | lo), W = the one plane [N][K] of a bf16 weight, or the two [2][N][K] of an fp32 weight (zg_common.h split2_f16).
+// All the products of a K step of 64 columns (two, or three) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
+// walk an fp32 weight in two passes that each stage the activations again and meet in slabs.
+// What bounds it: a compute unit takes in some 30 bytes a clock (32 KB a step of a 64 x 64 tile of three products: 1100 clocks, beside 384 of
 // products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
-// K steps; a step costs one barrier; its fragments were read beside the products of the step before.  The leading products have sums of
-// their own, so that the small ones are not rounded at their size.
+// K steps; a step costs one barrier; its fragments were read beside the products of the step before.  The leading products of a step are a sum
+// of their own, added to the steps' before it beside the products of the next, so that neither they nor the small ones are rounded at the size of
+// the whole.
 #include <algorithm>
 #include <type_traits>
 
@@ -20,7 +21,7 @@ namespace zg {
 namespace {
 
 typedef __attribute__((address_space(3))) char* lds_at_t;
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
+typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int kBk = 64, kRow = 128, kCh = 8;  // columns of K of a step; bytes and 16-byte chunks of a row of them
@@ -41,10 +42,10 @@ __device__ __forceinline__ u32x4 rsrc_of(const void* base) {
 
 // 2 x 2 waves of TM x 1 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
 template <int EPI, int TM, int NW, int ST>
-__global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
-                                                              const PrefillQkv qa) {
-    constexpr int BM = 64 * TM, BN = 64, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = 3 * A_PLANE + NW * B_PLANE;
-    constexpr int REQ = 3 * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
+__global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
+                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
+    constexpr int BM = 64 * TM, BN = 64, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
+    constexpr int REQ = kPair * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
     extern __shared__ __attribute__((aligned(1024))) char s_ring[];
     const unsigned lds0 = (unsigned)(unsigned long)(lds_at_t)s_ring;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wy = wave >> 1, wx = wave & 1;
@@ -56,37 +57,37 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, c
     const u32x4 ra = rsrc_of(A), rb = rsrc_of(W);
     unsigned va[PA], vb[PB];
 #pragma unroll
-    for (int i = 0; i < PA; ++i) va[i] = (unsigned)min(m0 + (wave + 4 * i) * 8 + in_row, M - 1) * (unsigned)(kSplit * K) * 2u + chunk * 16u;  // (rows beyond the edge: never stored)
+    for (int i = 0; i < PA; ++i) va[i] = (unsigned)min(m0 + (wave + 4 * i) * 8 + in_row, M - 1) * (unsigned)(kPair * K) * 2u + chunk * 16u;  // (rows beyond the edge: never stored)
 #pragma unroll
     for (int i = 0; i < PB; ++i) vb[i] = (unsigned)(n0 + (wave + 4 * i) * 8 + in_row) * (unsigned)K * 2u + chunk * 16u;
     const int nk = K / kBk, t0 = nk * (int)blockIdx.y / n_sp, steps = nk * ((int)blockIdx.y + 1) / n_sp - t0;
     auto request = [&](int slot, int s) {
         const unsigned off = (unsigned)(t0 + min(s, steps - 1)) * kRow, to = lds0 + slot * SLOT + wave * 1024;
 #pragma unroll
-        for (int p = 0; p < 3; ++p)
+        for (int p = 0; p < kPair; ++p)
 #pragma unroll
             for (int i = 0; i < PA; ++i) dma_16(to + p * A_PLANE + i * 4096, ra, va[i], off + (unsigned)p * (unsigned)K * 2u);
 #pragma unroll
         for (int p = 0; p < NW; ++p)
 #pragma unroll
-            for (int i = 0; i < PB; ++i) dma_16(to + 3 * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
+            for (int i = 0; i < PB; ++i) dma_16(to + kPair * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
     };
-    f32x16 lead[TM], small[TM];
+    f32x16 lead[2][TM], small[TM], total[TM];  // leading products by the step's parity
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) lead[i][e] = small[i][e] = 0.0f;
+        for (int e = 0; e < 16; ++e) lead[0][i][e] = lead[1][i][e] = small[i][e] = total[i][e] = 0.0f;
     const int fr = lane & 31, kh = lane >> 5, fswz = fr & 7;
-    u32x4 af[2][kCh / 2][3][TM], bf[2][kCh / 2][NW];  // of the step that is multiplied, and of the one behind it on its way
+    u32x4 af[2][kCh / 2][kPair][TM], bf[2][kCh / 2][NW];  // of the step that is multiplied, and of the one behind it on its way
     auto read = [&](auto b, int slot) {
         const char* base = s_ring + slot * SLOT;
 #pragma unroll
         for (int kk = 0; kk < kCh / 2; ++kk) {
             const int c = ((2 * kk + kh) ^ fswz) * 16;
 #pragma unroll
-            for (int p = 0; p < NW; ++p) bf[b][kk][p] = *reinterpret_cast<const u32x4*>(base + 3 * A_PLANE + p * B_PLANE + (wx * 32 + fr) * kRow + c);
+            for (int p = 0; p < NW; ++p) bf[b][kk][p] = *reinterpret_cast<const u32x4*>(base + kPair * A_PLANE + p * B_PLANE + (wx * 32 + fr) * kRow + c);
 #pragma unroll
-            for (int p = 0; p < 3; ++p)
+            for (int p = 0; p < kPair; ++p)
 #pragma unroll
                 for (int i = 0; i < TM; ++i) af[b][kk][p][i] = *reinterpret_cast<const u32x4*>(base + p * A_PLANE + ((wy * TM + i) * 32 + fr) * kRow + c);
         }
@@ -94,25 +95,33 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, c
     // (the operands change places: an accumulator's registers are then runs of four columns of a row)
     auto multiply = [&](auto b) {
         auto one = [&](f32x16& acc, int kk, int pa, int pw, int i) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, bf[b][kk][pw]), __builtin_bit_cast(bf16x8, af[b][kk][pa][i]), acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bf[b][kk][pw]), __builtin_bit_cast(f16x8, af[b][kk][pa][i]), acc, 0, 0, 0);
         };
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            total[i] += lead[1 - b][i];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) lead[1 - b][i][e] = 0.0f;
+        }
 #pragma unroll
         for (int kk = 0; kk < kCh / 2; ++kk)
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {  // the smallest first
-                one(small[i], kk, 2, 0, i);
-                if constexpr (NW == 3) {
-                    one(lead[i], kk, 0, 0, i);
-                    one(small[i], kk, 1, 1, i);
-                    one(small[i], kk, 0, 2, i);
-                    one(small[i], kk, 1, 0, i);
-                    one(small[i], kk, 0, 1, i);
-                } else {
-                    one(lead[i], kk, 0, 0, i);
-                    one(small[i], kk, 1, 0, i);
-                }
+            for (int i = 0; i < TM; ++i) {
+                one(small[i], kk, 1, 0, i);
+                one(lead[b][i], kk, 0, 0, i);
+                if constexpr (NW == 2) one(small[i], kk, 0, 1, i);
             }
     };
+    // what the epilogue needs besides the sums, on its way before the requests
+    const int cc = (lane & 7) * 4, n = n0 + wx * 32 + cc;
+    const i32x4 col_exp = *reinterpret_cast<const i32x4*>(ex.w + n);
+    const f32x4 bv = EPI != PF_PARTIAL && bias ? *reinterpret_cast<const f32x4*>(bias + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    int row_exp[TM][4];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int r8i = 0; r8i < 4; ++r8i) row_exp[i][r8i] = ex.a[ex.a_each ? min(m0 + (wy * TM + i) * 32 + 8 * r8i + (lane >> 3), M - 1) : 0];
+    const int out_exp = EPI == PF_GELU_SPLIT ? *po.exp : 0;
 #pragma unroll
     for (int s = 0; s < ST; ++s) request(s, s);
     if (EPI == PF_QKV) {  // the epilogue's arguments, fetched under the first requests
@@ -131,7 +140,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, c
         __builtin_amdgcn_sched_barrier(0);
         read(std::integral_constant<int, other>(), slot);
         multiply(b);
-        constexpr int products = kCh / 2 * TM * (NW == 3 ? 6 : 3), reads = kCh / 2 * (3 * TM + NW);
+        constexpr int products = kCh / 2 * TM * (NW + 1), reads = kCh / 2 * (kPair * TM + NW);
 #pragma unroll
         for (int x = 0; x < products; ++x) {
             __builtin_amdgcn_sched_group_barrier(0x100, (reads + products - 1) / products, 0);
@@ -152,26 +161,26 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, c
     constexpr int PITCH = 32 * 4 + 16;
     static_assert(4 * 32 * PITCH <= SLOT, "the images fit the ring");
     char* img = s_ring + wave * 32 * PITCH;
-    const int cc = (lane & 7) * 4, n = n0 + wx * 32 + cc;
-    const f32x4 bv = EPI != PF_PARTIAL && bias ? *reinterpret_cast<const f32x4*>(bias + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
-            f32x4 v;
+            f32x4 v;  // (of the two leading sums one is in the total already, and zero)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = lead[i][4 * g + e] + small[i][4 * g + e];
+            for (int e = 0; e < 4; ++e) v[e] = (total[i][4 * g + e] + (lead[0][i][4 * g + e] + lead[1][i][4 * g + e])) + small[i][4 * g + e];
             *reinterpret_cast<f32x4*>(img + fr * PITCH + (8 * g + 4 * kh) * 4) = v;
         }
 #pragma unroll
         for (int r8i = 0; r8i < 4; ++r8i) {
             const int r = 8 * r8i + (lane >> 3), m = m0 + (wy * TM + i) * 32 + r;
-            f32x4 v = *reinterpret_cast<const f32x4*>(img + r * PITCH + cc * 4) + bv;
+            f32x4 v = *reinterpret_cast<const f32x4*>(img + r * PITCH + cc * 4);
             if (m >= M) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], row_exp[i][r8i] + col_exp[e]) + bv[e];
             if constexpr (EPI == PF_GELU_SPLIT) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = gelu_fast(v[e]);
-                store_split4(reinterpret_cast<bf16_t*>(C) + (size_t)m * kSplit * N + n, N, v);
+                store_split4(reinterpret_cast<uint16_t*>(C) + (size_t)m * kPair * N + n, N, v, out_exp, po.coarse);
             } else if constexpr (EPI == PF_PARTIAL) {  // C: slabs [n_sp][M][N]
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)blockIdx.y * M + m) * N + n) = v;
             } else {
@@ -183,8 +192,8 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const bf16_t* A, c
 }
 
 template <int EPI, int TM, int NW, int ST>
-int launch_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, hipStream_t s) {
-    constexpr int LDS = ST * (3 * 64 * TM + NW * 64) * kRow;
+int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
+    constexpr int LDS = ST * (kPair * 64 * TM + NW * 64) * kRow;
     static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
     static OncePerDevice raised;
     int device = 0;
@@ -194,17 +203,18 @@ int launch_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, in
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * (N / 64);
-    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A, W, bias, C, M, N, K, ldc, n_sp, qa);
+    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
 
 template <int EPI>
-int launch_ring_epi(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, bool planes, int tm, int n_sp, const PrefillQkv& qa,
+int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int tm, int n_sp, const PrefillQkv& qa, const PlaneOut& po,
                     hipStream_t s) {
-    if (planes) return tm == 1 ? launch_ring<EPI, 1, 3, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s) : launch_ring<EPI, 2, 3, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s);
-    return tm == 1 ? launch_ring<EPI, 1, 1, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s) : launch_ring<EPI, 2, 1, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, s);
+    if (W.planes == 2)
+        return tm == 1 ? launch_ring<EPI, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+    return tm == 1 ? launch_ring<EPI, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
 }
 
 }  // namespace
@@ -228,7 +238,7 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
         int n_sp = resid ? (int)std::max(1l, std::min(256 / tiles, (long)nk / 3)) : 1;
         while (resid && n_sp > 1 && (size_t)n_sp * M * N > ws_floats) --n_sp;
         if (resid && (size_t)n_sp * M * N > ws_floats) continue;
-        const double us = rounds(tiles * n_sp) * (3.0 + ((nk + n_sp - 1) / n_sp) * (planes ? (24.0 * t + 24.0) / 57.0 : t == 1 ? 32.0 / 65.0 : 56.0 / 42.0)) + (resid ? n_sp * slab : 0.0);
+        const double us = rounds(tiles * n_sp) * (3.0 + ((nk + n_sp - 1) / n_sp) * (planes ? (16.0 * t + 16.0) / 57.0 : (16.0 * t + 8.0) / 65.0)) + (resid ? n_sp * slab : 0.0);
         if (best == 0 || us < best_us) {
             best = n_sp;
             best_us = us;
@@ -239,23 +249,23 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
     const bool wide = (long)((M + 127) / 128) * ((N + 255) / 256) >= 256;
     const int bn = wide ? 256 : 128;
     const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
-    const int passes = planes ? 3 : 1;
-    const int n_sp = (int)std::max(1l, std::min(planes ? (256 + 3 * tiles - 1) / (3 * tiles) : 256 / tiles, (long)nk / 3));
-    const double us = rounds(tiles * n_sp * passes) * (3.0 + ((nk + n_sp - 1) / n_sp) * (48.0 + bn / 8.0) / 65.0) +
+    const int passes = planes ? 2 : 1;
+    const int n_sp = (int)std::max(1l, std::min(planes ? (256 + 2 * tiles - 1) / (2 * tiles) : 256 / tiles, (long)nk / 3));
+    const double us = rounds(tiles * n_sp * passes) * (3.0 + ((nk + n_sp - 1) / n_sp) * (32.0 + bn / 8.0) / 65.0) +
                       (resid || n_sp * passes > 1 ? n_sp * passes * slab : 0.0) + (!resid && n_sp * passes > 1 ? 3.0 : 0.0);
     return best_us + (planes || M <= 256 ? 0.0 : 1.0) <= us ? best : 0;
 }
 
-int launch_prefill_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, bool planes, int tm, int n_sp, const PrefillQkv& qa,
-                        hipStream_t s) {
-    ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kSplit * K * 2 < ((size_t)1 << 31) &&
-                   (size_t)N * K * 2 * (planes ? 3 : 1) < ((size_t)1 << 31),
+int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
+                        const PlaneOut& po, hipStream_t s) {
+    ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kPair * K * 2 < ((size_t)1 << 31) &&
+                   (size_t)N * K * 2 * W.planes < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
     switch (epi) {
-        case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
-        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, planes, tm, n_sp, qa, s);
-        case PF_GELU_SPLIT: return launch_ring_epi<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
-        case PF_QKV: return launch_ring_epi<PF_QKV>(A, W, bias, C, M, N, K, ldc, planes, tm, 1, qa, s);
+        case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
+        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, tm, n_sp, qa, po, s);
+        case PF_GELU_SPLIT: return launch_ring_epi<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
+        case PF_QKV: return launch_ring_epi<PF_QKV>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
     }
     ZG_REQUIRE(false, ZG_ERR_ARG, "prefill gemm: epilogue %d", epi);
 }

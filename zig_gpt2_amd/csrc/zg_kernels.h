@@ -180,7 +180,14 @@ struct Split2Job {
     uint16_t* out;
     int* exps;
     int rows;
+    size_t lo = 0;           // the second plane lies this many elements behind the first (0: beside it, rows of 2K)
+    float* norms = nullptr;  // 2-norms of the rows
 };
+// for the test hooks of one Linear and one attention: rows of three bf16 planes -> fp32, rows of two fp16 planes times 2^exp -> three bf16 planes
+int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, float* out, hipStream_t s);
+int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, bf16_t* out, hipStream_t s);
+// bf16 [rows][K] -> one plane of fp16 (a bf16 value has 8 significant bits: exact down to 2^-32 of its row's largest)
+int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s);
 int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s);
 // rows [from_row, ctx) of every (cache, sequence x head) strip set to zero: n_caches caches cache_stride bytes apart, each holding a
 // plane of [strips][ctx] rows of row_bytes at plane_off (api_gpt.hip clear_kv: what a new sequence must not inherit)
@@ -216,11 +223,14 @@ struct PlaneExps {
 };
 int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s);
 // ... and its epilogue kinds for the whole-prompt Linears (gemm_s4.hip; PrefillQkv below)
-enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT3 = 3, S4_RELU2 = 4 };
+enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT2 = 3, S4_RELU2 = 4 };
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s);
 struct PrefillQkv;
-int launch_gemm_s4_prefill(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int nplanes, int kind, int n_slices,
-                           const PrefillQkv* qkv, hipStream_t s);
+struct PrefillA;
+struct PrefillW;
+struct PlaneOut;
+int launch_gemm_s4_prefill(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int kind, int n_slices,
+                           const PrefillQkv* qkv, const PlaneOut& po, hipStream_t s);
 int gemm_s4_stamps(unsigned long long* out, size_t n_words);  // diagnostic (ZGPT2_GEMM_DBG bit 256)
 int gemm_s4_fault(unsigned* out);  // 1: a stream-K consumer of gemm_s4 gave up waiting for its producer since the last call (results wrong)
 int gemm_debug_stamps(unsigned long long* out, size_t n_words);  // of the kernel generation launched last
@@ -236,14 +246,25 @@ int linear_tiles_slices(size_t M, size_t N, size_t K);
 int launch_linear_tiles(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, float* slabs, hipStream_t s);
 
 // ------------------------------------------------------------------------------------ prefill (prefill.hip)
-// Whole-prompt forward.  Activations feeding a GEMM are fp32 split exactly into kSplit bf16 terms,
-// stored as planes [M][kSplit * K] = [hi | mid | lo].
-constexpr int kSplit = 3;
+// Whole-prompt forward.  Activations feeding a GEMM are two-term fp16 planes (zg_common.h split2_f16), [M][kPair * K] = [hi | lo] of the
+// fp32 values times 2^-exp, exp one number for all of them: a bound on the values that holds for any input follows from the weights alone
+// (launch_prefill_bounds), so that it is known before they are.
+constexpr int kPair = 2;
+struct PlaneOut {
+    const int* exp;
+    int coarse;  // ZG_GPT_PREFILL_2PLANE: values rounded to 16 significant bits first
+};
+// a Linear's weight: fp16 planes [planes][N][K] of its rows times 2^-exps[row]; one plane holds a bf16 value, two an fp32 value
+struct PrefillW {
+    const uint16_t* p;
+    const int* exps;
+    int planes;
+};
 enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4 };
 int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, const void* wte, const void* wpe,
                          int weight_type, int E, float* x, hipStream_t s);
-int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, bf16_t* out, hipStream_t s);
-// C = A[M][kSplit K] * W[N][K]^T + bias; PF_F32: fp32 C[M][ldc]; PF_RESID: C += ...; PF_GELU_SPLIT: bf16 C[M][kSplit N] = split(gelu(...))
+int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, uint16_t* out, const PlaneOut& po, hipStream_t s);
+// C = A[M][K] * W[N][K]^T + bias; PF_F32: fp32 C[M][ldc]; PF_RESID: C += ...; PF_GELU_SPLIT: planes C[M][kPair N] of gelu(...), as po says
 // ws: fp32 workspace for split-K partial sums (used when the output has too few tiles to fill the chip).
 // ln (PF_RESID only, may be null): LayerNorm of the updated rows, written as split planes to ln->out — fused
 // into the split-K tail when there is one, a separate launch_ln_split otherwise.
@@ -267,22 +288,36 @@ struct PrefillLn {
     const float* g;
     const float* b;
     float eps;
-    bf16_t* out;
+    uint16_t* out;
+    PlaneOut po;
 };
-int launch_prefill_gemm(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi,
-                        float* ws, size_t ws_floats, const PrefillLn* ln, hipStream_t s, const PrefillQkv* qkv = nullptr,
-                        int nsplit = kSplit);  // nsplit = 2: multiply the hi + mid planes only (2/3 of the matrix work);
-                                               // kWeightPlanes: W is the plane-major three-term split [3][N][K] of an fp32 matrix
-constexpr int kWeightPlanes = 33;
+// a: the exponents of A's rows (each: one for every row, else one for all)
+struct PrefillA {
+    const uint16_t* p;
+    const int* exp;
+    bool each;
+};
+int launch_prefill_gemm(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi,
+                        float* ws, size_t ws_floats, const PrefillLn* ln, hipStream_t s, const PrefillQkv* qkv = nullptr, const PlaneOut& po = PlaneOut{});
 // prefill_ring.hip: whole-prompt Linears of some hundred rows.  The route: K slices (slabs of a residual Linear, else 1), 0 = not taken; tm: rows / 64 of a tile.
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
-int launch_prefill_ring(const bf16_t* A, const bf16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, bool planes, int tm, int n_sp, const PrefillQkv& qa,
-                        hipStream_t s);
+int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
+                        const PlaneOut& po, hipStream_t s);
+// The exponents of a layer's activations, from its weights: the rows of a normed x are no longer than sqrt(E) max|g| + |b| (b's 2-norm), so no output of
+// a Linear behind it is larger than that times the longest row of its matrix plus its largest bias.  exps: kBounds of them (enum).
+enum { PB_LN1 = 0, PB_Q = 1, PB_K = 2, PB_V = 3, PB_LN2 = 4, PB_GELU = 5, kBounds = 8 };
+struct PrefillBounds {
+    const float *ln_1_g, *ln_1_b, *c_attn_b, *ln_2_g, *ln_2_b, *c_fc_b;
+    const float *c_attn_norms, *c_fc_norms;  // 2-norms of the rows (launch_split2, launch_plane_bf16)
+    int* exps;
+};
+int launch_prefill_bounds(const PrefillBounds& b, int E, hipStream_t s);
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
-// out[M][kSplit E] = split(causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t)
-// (attn_prefill.hip: bf16 matrix cores on exact plane splits; ws = fp32 workspace for the partials of split key ranges)
-int launch_attn_prefill(const float* qkv, bf16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache_or_null,
-                        const float* v_cache_or_null, int ctx, hipStream_t s, int force_tiles = 0);  // force_tiles: key tiles per workgroup (tests)
+// out[M][kPair E] = planes of the causal attention of the q / k / v columns of qkv[M][3E], M = B P rows ordered (b, t)
+// (attn_prefill.hip: matrix cores on two-term fp16 planes; ws = fp32 workspace for the partials of split key ranges).  exps: kBounds of them; the output
+// has v's (a weighted mean of rows of v is no larger than they are).
+int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache_or_null,
+                        const float* v_cache_or_null, int ctx, const int* exps, int coarse, hipStream_t s, int force_tiles = 0);  // force_tiles: key tiles per workgroup (tests)
 
 // GPT.sample tail: in-place softmax(logits / temp) per sequence + inverse-CDF draw with uniform u[b].
 // part_val / n_part / part_stride: the per-workgroup maxima lm_head's argmax epilogue left (the row maximum without a pass over the
