@@ -629,6 +629,17 @@ int zg_debug_prefill_linear(const uint16_t* A, const uint16_t* W, const float* b
         Split2Job jx{x, xp, xe, (int)M};
         jx.norms = xn;
         ZG_TRY(launch_split2(jx, Split2Job{}, (int)K, s));
+        const bool each = force_kernel == 2 || force_kernel == 3;  // (the persistent GEMM's prompt Linears have one exponent for all rows)
+        if (!each) {
+            std::vector<int> he(M);
+            ZG_HIP(hipMemcpyAsync(he.data(), xe, M * 4, hipMemcpyDeviceToHost, s));
+            ZG_HIP(hipStreamSynchronize(s));
+            const int top = *std::max_element(he.begin(), he.end());
+            ZG_HIP(hipMemcpyAsync(oe, &top, 4, hipMemcpyHostToDevice, s));
+            jx.one = oe;
+            ZG_TRY(launch_split2(jx, Split2Job{}, (int)K, s));
+            ZG_HIP(hipStreamSynchronize(s));
+        }
         ZG_TRY(launch_plane_bf16(W, (int)N, (int)K, wp, we, wn, s));
         PlaneOut po{nullptr, 0};
         if (epi == PF_GELU_SPLIT) {  // no gelu is larger than its row times the longest row of the weight, and the bias
@@ -648,7 +659,7 @@ int zg_debug_prefill_linear(const uint16_t* A, const uint16_t* W, const float* b
             po.exp = oe;
         }
         prefill_force_route(force_kernel, slices);
-        const int st = launch_prefill_gemm(PrefillA{xp, xe, true}, PrefillW{wp, we, 1}, bias, epi == PF_GELU_SPLIT ? static_cast<void*>(op) : C, (int)M, (int)N, (int)K,
+        const int st = launch_prefill_gemm(PrefillA{xp, xe, each}, PrefillW{wp, we, 1}, bias, epi == PF_GELU_SPLIT ? static_cast<void*>(op) : C, (int)M, (int)N, (int)K,
                                            epi == PF_GELU_SPLIT ? 0 : (int)N, epi, ws, ws_floats, nullptr, s, nullptr, po);
         prefill_force_route(0, 0);
         ZG_TRY(st);

@@ -256,7 +256,7 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     for (int i = lane + 64 * NV; i < n4; i += 64) widen(*reinterpret_cast<const f32x4*>(x + 4 * i));
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
-    const int up = split2_exp(top);
+    const int up = j.one != nullptr ? -*j.one : split2_exp(top);
     if (lane == 0) j.exps[row] = -up;
     auto leave = [&](int i, const f32x4& in) {
         const f32x4 q = {ldexpf(in.x, up), ldexpf(in.y, up), ldexpf(in.z, up), ldexpf(in.w, up)};

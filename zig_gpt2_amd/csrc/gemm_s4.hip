@@ -127,9 +127,9 @@ __device__ __forceinline__ void read_frag_b(bf16x8& f, const unsigned (&b_addr)[
 // the compiler keeps nothing of its own there across any of them.  Hazards are ours too: MFMA result ->
 // v_accvgpr_read needs the pipeline drained (s_nop in acc_settle), v_accvgpr_write -> MFMA source C two wait states.
 #define ZG_ACC_CLOBBERS "a0","a1","a2","a3","a4","a5","a6","a7","a8","a9","a10","a11","a12","a13","a14","a15","a16","a17","a18","a19","a20","a21","a22","a23","a24","a25","a26","a27","a28","a29","a30","a31","a32","a33","a34","a35","a36","a37","a38","a39","a40","a41","a42","a43","a44","a45","a46","a47","a48","a49","a50","a51","a52","a53","a54","a55","a56","a57","a58","a59","a60","a61","a62","a63","a64","a65","a66","a67","a68","a69","a70","a71","a72","a73","a74","a75","a76","a77","a78","a79","a80","a81","a82","a83","a84","a85","a86","a87","a88","a89","a90","a91","a92","a93","a94","a95","a96","a97","a98","a99","a100","a101","a102","a103","a104","a105","a106","a107","a108","a109","a110","a111","a112","a113","a114","a115","a116","a117","a118","a119","a120","a121","a122","a123","a124","a125","a126","a127","a128","a129","a130","a131","a132","a133","a134","a135","a136","a137","a138","a139","a140","a141","a142","a143","a144","a145","a146","a147","a148","a149","a150","a151","a152","a153","a154","a155","a156","a157","a158","a159","a160","a161","a162","a163","a164","a165","a166","a167","a168","a169","a170","a171","a172","a173","a174","a175","a176","a177","a178","a179","a180","a181","a182","a183","a184","a185","a186","a187","a188","a189","a190","a191"
-template <int BASE, bool F16>
+template <int BASE, int F16>
 __device__ __forceinline__ void mfma_acc(const bf16x8& a_op, const bf16x8& b_op) {
-    if constexpr (F16) asm volatile("v_mfma_f32_32x32x16_f16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
+    if constexpr (F16 != 0) asm volatile("v_mfma_f32_32x32x16_f16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
     else asm volatile("v_mfma_f32_32x32x16_bf16 a[%c2:%c3], %0, %1, a[%c2:%c3]" ::"v"(a_op), "v"(b_op), "i"(BASE), "i"(BASE + 15) : ZG_ACC_CLOBBERS);
 }
 template <int BASE>
@@ -213,9 +213,11 @@ __device__ __forceinline__ void read_b_all(bf16x8 (&fb)[4][NT], const unsigned (
 //   S4_SPLIT2   bias + GELU, then the two-term fp16 split as planes C[M][2N] = [hi | lo]  (src/main.zig:79-80 feeding
 //               the next Linear's A operand); F16 only
 
-// F16: the planes are the two-term fp16 split of rows scaled by powers of two (zg_common.h split2_f16): the finished sums are scaled back by
-// the exponents of their row and column, and the bias is added behind that (the accumulators start at zero).
-template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
+// F16: the planes are the two-term fp16 split of rows scaled by powers of two (zg_common.h split2_f16), and the finished sums are scaled back.  F16_ROWS:
+// every row of A has an exponent of its own (Linear.forward of any fp32 rows); the accumulators start at zero and the bias is added at the end.
+// F16_ONE: one for all (the whole-prompt Linears); the accumulators start at the bias as the sums are scaled.
+enum { F16_NO = 0, F16_ONE = 1, F16_ROWS = 2 };
+template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, int F16 = F16_NO>
 __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                          const float* __restrict__ bias, void* __restrict__ C, int M, int N,
                                                          unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
@@ -313,16 +315,17 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     const __amdgpu_buffer_rsrc_t rbias =
         __builtin_amdgcn_make_buffer_rsrc((void*)bias, 0, bias != nullptr ? (unsigned)N * 4u : 0u, 0x00020000);
     // (F16: the exponents of the tile's columns and rows travel with it)
-    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rcexp = __builtin_amdgcn_make_buffer_rsrc((void*)ex.w, 0, F16 ? (unsigned)N * 4u : 0u, 0x00020000);
+    [[maybe_unused]] const __amdgpu_buffer_rsrc_t rcexp = __builtin_amdgcn_make_buffer_rsrc((void*)ex.w, 0, F16 != 0 ? (unsigned)N * 4u : 0u, 0x00020000);
     [[maybe_unused]] const __amdgpu_buffer_rsrc_t rrexp =
-        __builtin_amdgcn_make_buffer_rsrc((void*)ex.a, 0, F16 ? (ex.a_each ? (unsigned)M * 4u : 4u) : 0u, 0x00020000);
+        __builtin_amdgcn_make_buffer_rsrc((void*)ex.a, 0, F16 == F16_ROWS ? (unsigned)M * 4u : 0u, 0x00020000);
+    [[maybe_unused]] int row_exp = 0, out_exp = 0;  // F16_ONE, S4_SPLIT2 (fetched under the first DMA)
     int tile_par = 0;  // parity of the current tile: its bias row is in buffer tile_par, the next tile's in the other one (F16: of three)
     auto par_after = [&](int par, int by) {
-        if constexpr (!F16) return par ^ (by & 1);
+        if constexpr (F16 == 0) return par ^ (by & 1);
         else return par + by >= 3 ? par + by - 3 : par + by;
     };
     auto fetch_bias = [&](int n0_, int par, [[maybe_unused]] int m0_) {
-        if constexpr (F16) {
+        if constexpr (F16 != 0) {
             const unsigned at = lds_base + P::EXP_OFF + par * P::EXP_TILE;
             if (wave == 0)
 #pragma unroll
@@ -331,11 +334,10 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rbias, to_lds(at + p * 256), 4, (unsigned)lane * 4u, col, 0, 0);
                     __builtin_amdgcn_raw_ptr_buffer_load_lds(rcexp, to_lds(at + 1024 + p * 256), 4, (unsigned)lane * 4u, col, 0, 0);
                 }
-            if (wave == 1)
+            if (F16 == F16_ROWS && wave == 1)
 #pragma unroll
                 for (int p = 0; p < 4; ++p)
-                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rrexp, to_lds(at + 2048 + p * 256), 4, ex.a_each ? (unsigned)lane * 4u : 0u,
-                                                             ex.a_each ? (unsigned)(m0_ + 64 * p) * 4u : 0u, 0, 0);
+                    __builtin_amdgcn_raw_ptr_buffer_load_lds(rrexp, to_lds(at + 2048 + p * 256), 4, (unsigned)lane * 4u, (unsigned)(m0_ + 64 * p) * 4u, 0, 0);
         } else if (wave == 0) {
 #pragma unroll
             for (int p = 0; p < P::BN / 64; ++p)
@@ -406,10 +408,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     // their dirty lines back — 4.2 us between the last workgroup's end and the next launch's first workgroup against 2.0 us
     // with write-through stores, at +0.6 us inside the launch (41.5 -> 40.2 us at M = 8192, profiles/round4_gemm_a.txt; nt: 40.7).
     constexpr int ST_AUX = 16;
+    // (F16: A's planes are read once a round and marked for early eviction, B's by every pair of planes: 4814 -> 4746 us)
     auto dma_a = [&](int X, int h, int i, const Ahead& s) {
         const unsigned rowd = (unsigned)((i >> 1) * 128 + h * 64 + (i & 1) * 32);
         const unsigned dst = lds_base + P::A_OFF + X * P::A_SLOT + h * 16384 + (wave + 4 * i) * 1024;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, to_lds(dst), 16, relA, s.baseA + rowd * lda2 + s.kbA, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, to_lds(dst), 16, relA, s.baseA + rowd * lda2 + s.kbA, 0, F16 != 0 ? 2 : 0);
     };
     auto dma_b = [&](int X, int i, const Ahead& s) {
         const unsigned dst = lds_base + P::B_OFF + X * P::B_SLOT + (wave + 4 * i) * 1024;
@@ -417,24 +420,34 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     };
     // accumulators: a[0 : 16 * 4 * NT - 1], owned by hand (see mfma_acc); start at zero
     static_assert(NT == 3, "the hand-owned accumulator file is laid out for NT = 3 (192 registers)");
-    // every tile starts at its bias row (buffer `par` of the LDS bias area): 12 MFMAs, see acc_init
-    auto init_acc_from_bias = [&](int par) {
-        const unsigned baddr = lds_base + P::BIAS_OFF + par * 1024 + (unsigned)(wc * (P::BN / 2) + 4 * (lane >> 5)) * 4u;
+    // every tile starts at its bias row (buffer `par` of the LDS bias area): 12 MFMAs, see acc_init.  F16_ONE: the bias times what the sums are
+    // scaled with; F16_ROWS, and a producer's half tile (zero): at zero.
+    auto init_acc_from_bias = [&](int par, [[maybe_unused]] bool zero) __attribute__((always_inline)) {
+        const unsigned baddr = lds_base + (F16 != 0 ? P::EXP_OFF + par * P::EXP_TILE : P::BIAS_OFF + par * 1024) + (unsigned)(wc * (P::BN / 2) + 4 * (lane >> 5)) * 4u;
         bf16x8 zop;
 #pragma unroll
         for (int e = 0; e < 8; ++e) zop[e] = (__bf16)0.0f;
-        static_for<NT>([&](auto JT) {
+        static_for<NT>([&](auto JT) __attribute__((always_inline)) {
             constexpr int j = decltype(JT)::value;
-            if constexpr (F16) {
-                const f32x4v z = {0.0f, 0.0f, 0.0f, 0.0f};
-                acc_init4<16 * (0 * NT + j), 16 * (1 * NT + j), 16 * (2 * NT + j), 16 * (3 * NT + j)>(zop, z, z, z, z);
-                return;
-            }
-            const unsigned baddr_l = baddr;
             f32x4v b4[4];  // columns 32 j + 8 g + 4 hh + {0..3}: registers 4 g .. 4 g + 3 of the tile
+            if constexpr (F16 == F16_ROWS) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b4[g]) : "v"(baddr_l), "i"((j * 32 + 8 * g) * 4));
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]));
+                for (int g = 0; g < 4; ++g) b4[g] = f32x4v{0.0f, 0.0f, 0.0f, 0.0f};
+            } else {
+                const unsigned baddr_l = baddr;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b4[g]) : "v"(baddr_l), "i"((j * 32 + 8 * g) * 4));
+                if constexpr (F16 == F16_ONE) {
+                    i32x4v c4[4];
+#pragma unroll
+                    for (int g = 0; g < 4; ++g) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[g]) : "v"(baddr_l), "i"(1024 + (j * 32 + 8 * g) * 4));
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]), "+v"(c4[0]), "+v"(c4[1]), "+v"(c4[2]), "+v"(c4[3]));
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) b4[e >> 2][e & 3] = zero ? 0.0f : __builtin_amdgcn_ldexpf(b4[e >> 2][e & 3], -(row_exp + c4[e >> 2][e & 3]));
+                } else {
+                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]));
+                }
+            }
             acc_init4<16 * (0 * NT + j), 16 * (1 * NT + j), 16 * (2 * NT + j), 16 * (3 * NT + j)>(zop, b4[0], b4[1], b4[2], b4[3]);
         });
     };
@@ -505,7 +518,44 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             for (; pend_n < NPEND; ++pend_n) emit_pending(pend_n);
     };
 
+    // F16: half way through the leading products the sums leave their leading eight bits aside and go on with the rest (both exact), so that the second
+    // half is rounded at its own size: with 11-bit terms a chain of 768 products is 1.71e-7 off, in two halves 1.2e-7, which makes room for
+    // what the split leaves (0.75e-7; a bf16 weight 0.44e-7); three exact bf16 terms in one chain are 1.58e-7 off.  8192 x 768 x 3072: 136 us of a call
+    // without, 150 with.  In the shadow of the products it would be free, but is not: K-steps of their own for it cost 48 moves of fragments in every
+    // K-step (what joins must meet in the same registers), branches behind every product 20 us.
+    // (always_inline: left to itself the compiler keeps this in memory)
+    [[maybe_unused]] u32x8v aside[F16 != 0 ? 4 * NT : 1] = {};
+    auto set_aside = [&]() __attribute__((always_inline)) {
+        if constexpr (F16 != 0) {
+            acc_settle();
+            static_for<4 * NT>([&](auto QT) __attribute__((always_inline)) {
+                constexpr int q = decltype(QT)::value;
+                float av[16];
+                acc_read16<16 * q>(av);
+                u32x4 rest[4];
+                u32x8v lead;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    lead[e] = cvt_pk_bf16(av[2 * e], av[2 * e + 1]);
+                    rest[e >> 1][2 * (e & 1)] = __float_as_uint(av[2 * e] - bf16_lo(lead[e]));
+                    rest[e >> 1][2 * (e & 1) + 1] = __float_as_uint(av[2 * e + 1] - bf16_hi(lead[e]));
+                }
+                aside[q] = lead;
+                acc_write16<16 * q>(rest);
+            });
+            asm volatile("s_nop 7" ::: ZG_ACC_CLOBBERS);  // v_accvgpr_write -> MFMA source C
+            ZG_SB();
+        }
+    };
+
     Ahead s1, s2;  // stream positions t + 1 / t + 2 of the current K-step t
+    // One step = one k-slice (16 of K) of one phase: 2 x NT MFMAs, and behind each MFMA at most ONE other item
+    // (a fragment read or a DMA piece: two ds_read_b128 in one MFMA shadow do not fit — tools/microbench/mfma_lds.hip).
+    // J = 4 h + ks.  Per K-step t (slot X):
+    //   steps 0-2   DMA: B of K-step t + 2 -> slot X, A half 1 of K-step t + 1 -> slot X ^ 1
+    //   step 3      barrier 1 (A half 0 of slot X read out; A half 1 of t, B and A half 0 of t + 1 landed)
+    //   steps 3-6   DMA: A half 0 of K-step t + 2 -> slot X (one piece per step); B fragments of K-step t + 1 -> registers
+    //   step 7      barrier 2 (A half 1 of slot X, B of slot X ^ 1 read out)
     // One step = one k-slice (16 of K) of one phase: 2 x NT MFMAs, and behind each MFMA at most ONE other item
     // (a fragment read or a DMA piece: two ds_read_b128 in one MFMA shadow do not fit — tools/microbench/mfma_lds.hip).
     // J = 4 h + ks.  Per K-step t (slot X):
@@ -608,38 +658,6 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         s1 = s2;
     };
 
-    [[maybe_unused]] int out_exp = 0;  // S4_SPLIT2
-    // F16: half way through the leading products the sums leave their leading eight bits aside and go on with the rest (both exact), so that the second
-    // half is rounded at its own size: with 11-bit terms a chain of 768 products is 1.71e-7 off, in two halves 1.2e-7, which makes room for
-    // what the split leaves (0.75e-7); three exact bf16 terms in one chain are 1.58e-7 off.  8192 x 768 x 3072: 136 us of a call without, 150 with.
-    // (always_inline: left to itself the compiler keeps this in memory)
-    [[maybe_unused]] u32x8v aside[F16 ? 4 * NT : 1] = {};
-    auto set_aside = [&]() __attribute__((always_inline)) {
-        if constexpr (F16) {
-            acc_settle();
-            static_for<4 * NT>([&](auto QT) {
-                constexpr int q = decltype(QT)::value;
-                float av[16];
-                acc_read16<16 * q>(av);
-                u32x4 rest[4];
-                u32x8v lead;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    lead[e] = cvt_pk_bf16(av[2 * e], av[2 * e + 1]);
-                    rest[e >> 1][2 * (e & 1)] = __float_as_uint(av[2 * e] - bf16_lo(lead[e]));
-                    rest[e >> 1][2 * (e & 1) + 1] = __float_as_uint(av[2 * e + 1] - bf16_hi(lead[e]));
-                }
-                aside[q] = lead;
-                acc_write16<16 * q>(rest);
-            });
-            asm volatile("s_nop 7" ::: ZG_ACC_CLOBBERS);  // v_accvgpr_write -> MFMA source C
-            ZG_SB();
-        }
-    };
-
-    // ---- epilogue of one tile, straight from the registers: lane (l31, hh) holds output row l31 of each 32 x 32
-    // tile and columns 8 g + 4 hh + {0..3} (register 4 g + e).  bf16: v_permlane32_swap makes 8 consecutive
-    // columns (16 B) per lane out of the two half-waves' runs of 4.
     // ---- SK: the producer's half tile leaves as raw accumulators, [shared tile][wave][48 register quads][lane] x 16 B, write-
     // through; then, its stores drained, one flag word per wave = this launch's epoch (the consumer's wave w polls wave w's flag
     // and loads exactly what that wave stored: no workgroup barrier on either side).  The poll is bounded: a consumer that
@@ -687,7 +705,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     auto epilogue = [&]() __attribute__((always_inline)) {
         if (SK && role_cur == 1) {  // a producer's half tile: no epilogue, the accumulators go to its consumer
             sk_spill();
-            if (has_nxt) init_acc_from_bias(par_after(tile_par, 1));
+            if (has_nxt) init_acc_from_bias(par_after(tile_par, 1), false);
             ZG_SB();
             return;
         }
@@ -701,19 +719,49 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         // Stores go through a buffer descriptor: a row past M lies past the descriptor's end and a column past N gets an
         // out-of-range offset, so the hardware drops them — no exec masking, one straight block of code per tile.
         flush_pending();  // (a tile of fewer K-steps than pending stores)
-        // F16: 2^(row + column exponent) times the sums, plus the bias
-        [[maybe_unused]] const unsigned exps = lds_base + P::EXP_OFF + tile_par * P::EXP_TILE;
+        const unsigned row0 = (unsigned)(m0 + wr * 128 + l31e) * (unsigned)(ldc * ESZ);
+        const int col0 = n0 + wc * (P::BN / 2) + 8 * hhe;
+        // F16: the sums get back what was set aside (and a consumer's half tile its producer's) and are scaled by 2^(row + column exponent), F16_ROWS with the
+        // bias behind it.  F16_ONE: the factors of the lane's columns stay in registers (the fragments' are free).
+        [[maybe_unused]] const unsigned exps = lds_base + P::EXP_OFF + tile_par * P::EXP_TILE + (unsigned)(wc * (P::BN / 2) + 4 * hhe) * 4u;
         [[maybe_unused]] int rexp[4];
-        if constexpr (F16) {
-            const unsigned raddr = exps + 2048u + (unsigned)(wr * 128 + l31e) * 4u;
+        constexpr bool HELD = F16 == F16_ONE && !SK;  // (with the hand-over's own there are not enough)
+        [[maybe_unused]] f32x4v scale[HELD ? NT : 1][4];
+        if constexpr (F16 == F16_ROWS) {
+            const unsigned raddr = lds_base + P::EXP_OFF + tile_par * P::EXP_TILE + 2048u + (unsigned)(wr * 128 + l31e) * 4u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(rexp[i]) : "v"(raddr), "i"(i * 128));
             asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(rexp[0]), "+v"(rexp[1]), "+v"(rexp[2]), "+v"(rexp[3]));
         }
+        if constexpr (HELD) {
+            i32x4v c4[NT][4];
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[j][g]) : "v"(exps), "i"(1024 + (j * 32 + 8 * g) * 4));
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(c4[j][0]), "+v"(c4[j][1]), "+v"(c4[j][2]), "+v"(c4[j][3]));
+#pragma unroll
+                for (int e = 0; e < 16; ++e) scale[j][e >> 2][e & 3] = __builtin_amdgcn_ldexpf(1.0f, row_exp + c4[j][e >> 2][e & 3]);
+            }
+        }
         [[maybe_unused]] const __amdgpu_buffer_rsrc_t rpart = __builtin_amdgcn_make_buffer_rsrc(qa.sk_ws, 0, SK ? (unsigned)(G >> 1) * 196608u : 0u, 0x00020000);
-        if (SK && role_cur == 2) sk_wait();
-        [[maybe_unused]] auto scale_back = [&](auto IT, auto JT, int row_exp, float (&av)[16]) __attribute__((always_inline)) {
-            constexpr int j = decltype(JT)::value, q = decltype(IT)::value * NT + j;
+        [[maybe_unused]] u32x4 part[4];  // what the consumer adds to its next tile of sums
+        auto fetch_part = [&](auto QT) __attribute__((always_inline)) {
+            constexpr int q = decltype(QT)::value;
+            if constexpr (SK && q < 4 * NT) {
+                const unsigned base = (unsigned)(sk_sh * 4 + wave) * 49152u + (unsigned)lane_e * 16u;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[e] = __builtin_amdgcn_raw_buffer_load_b128(rpart, base + (unsigned)(q * 4 + e) * 1024u, 0, 16);
+            }
+        };
+        if (SK && role_cur == 2) {
+            sk_wait();
+            fetch_part(Ic<0>{});
+        }
+        [[maybe_unused]] auto scale_back = [&](auto IT, auto JT, float (&av)[16]) __attribute__((always_inline)) {
+            constexpr int i = decltype(IT)::value, j = decltype(JT)::value, q = i * NT + j;
             const u32x8v lead = aside[q];
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
@@ -721,27 +769,35 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 av[2 * e + 1] += bf16_hi(lead[e]);
             }
             if (SK && role_cur == 2) {
-                const unsigned base = (unsigned)(sk_sh * 4 + wave) * 49152u + (unsigned)lane_e * 16u;
-                u32x4 v[4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[e] = __builtin_amdgcn_raw_buffer_load_b128(rpart, base + (unsigned)(q * 4 + e) * 1024u, 0, 16);
-#pragma unroll
-                for (int e = 0; e < 16; ++e) av[e] += __uint_as_float(v[e >> 2][e & 3]);
+                for (int e = 0; e < 16; ++e) av[e] += __uint_as_float(part[e >> 2][e & 3]);
+                fetch_part(Ic<q + 1>{});
             }
-            const unsigned caddr = exps + (unsigned)(wc * (P::BN / 2) + 4 * hhe) * 4u;
-            f32x4v b4[4];
-            i32x4v c4[4];
+            if constexpr (HELD) {
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b4[g]) : "v"(caddr), "i"((j * 32 + 8 * g) * 4));
-                asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[g]) : "v"(caddr), "i"(1024 + (j * 32 + 8 * g) * 4));
+                for (int e = 0; e < 16; ++e) av[e] *= scale[j][e >> 2][e & 3];
+            } else if constexpr (F16 == F16_ONE) {
+                const unsigned exps_l = exps;
+                i32x4v c4[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[g]) : "v"(exps_l), "i"(1024 + (j * 32 + 8 * g) * 4));
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(c4[0]), "+v"(c4[1]), "+v"(c4[2]), "+v"(c4[3]));
+#pragma unroll
+                for (int e = 0; e < 16; ++e) av[e] = __builtin_amdgcn_ldexpf(av[e], row_exp + c4[e >> 2][e & 3]);
+            } else {
+                const unsigned exps_l = exps;
+                f32x4v b4[4];
+                i32x4v c4[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(b4[g]) : "v"(exps_l), "i"((j * 32 + 8 * g) * 4));
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(c4[g]) : "v"(exps_l), "i"(1024 + (j * 32 + 8 * g) * 4));
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]), "+v"(c4[0]), "+v"(c4[1]), "+v"(c4[2]), "+v"(c4[3]));
+#pragma unroll
+                for (int e = 0; e < 16; ++e) av[e] = __builtin_amdgcn_ldexpf(av[e], rexp[i] + c4[e >> 2][e & 3]) + b4[e >> 2][e & 3];
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(b4[0]), "+v"(b4[1]), "+v"(b4[2]), "+v"(b4[3]), "+v"(c4[0]), "+v"(c4[1]), "+v"(c4[2]), "+v"(c4[3]));
-#pragma unroll
-            for (int e = 0; e < 16; ++e) av[e] = __builtin_amdgcn_ldexpf(av[e], row_exp + c4[e >> 2][e & 3]) + b4[e >> 2][e & 3];
         };
-        const unsigned row0 = (unsigned)(m0 + wr * 128 + l31e) * (unsigned)(ldc * ESZ);
-        const int col0 = n0 + wc * (P::BN / 2) + 8 * hhe;
         // bf16: a lane's runs of 4 columns go through a wave-private LDS image of the m-tile and leave as 16-B pieces of
         // whole rows (a store instruction that scatters 32-B pieces over 32 rows costs one L2 request per piece: the
         // epilogue was bounded by the request rate of the L2s, 6.8k cycles per tile)
@@ -760,7 +816,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         if constexpr (KIND == S4_SPLIT2) {
             // GELU, then the two planes of an m-tile one after the other through the wave's staging image (its LDS accesses
             // complete in order: plane p + 1 is written behind the reads of plane p without a wait)
-            const int out_up = -out_exp;
+            const float out_up = __builtin_amdgcn_ldexpf(1.0f, -out_exp);
             static_for<4>([&](auto IT) {
                 constexpr int i = decltype(IT)::value;
                 u32x2 w[2][NT][4];
@@ -769,7 +825,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                     asm volatile("s_nop 3" ::: "memory");
                     float av[16];
                     acc_read16<16 * (i * NT + j)>(av);
-                    scale_back(IT, JT, rexp[i], av);
+                    scale_back(IT, JT, av);
                     f32x2v x[8];
 #pragma unroll
                     for (int k = 0; k < 8; ++k) x[k] = gelu2(f32x2v{av[2 * k], av[2 * k + 1]});
@@ -777,7 +833,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
 #pragma unroll
                         for (int k = 0; k < 8; ++k) x[k] = f32x2v{coarse16(x[k].x), coarse16(x[k].y)};
 #pragma unroll
-                    for (int k = 0; k < 8; ++k) x[k] = f32x2v{__builtin_amdgcn_ldexpf(x[k].x, out_up), __builtin_amdgcn_ldexpf(x[k].y, out_up)};
+                    for (int k = 0; k < 8; ++k) x[k] = f32x2v{x[k].x * out_up, x[k].y * out_up};
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         uint32_t a[2], b[2];
@@ -847,7 +903,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                     asm volatile("s_nop 3" ::: "memory");
                     float av[16];
                     acc_read16<16 * (i * NT + j)>(av);
-                    if constexpr (F16) scale_back(IT, JT, rexp[i], av);
+                    if constexpr (F16 != 0) scale_back(IT, JT, av);
 #pragma unroll
                     for (int g = 0; g < 4; ++g) {
                         const f32x4v v4 = {av[4 * g], av[4 * g + 1], av[4 * g + 2], av[4 * g + 3]};
@@ -899,7 +955,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 asm volatile("s_nop 3" ::: "memory");
                 float av[16];
                 acc_read16<16 * (i * NT + j)>(av);
-                if constexpr (F16) scale_back(IT, JT, rexp[i], av);
+                if constexpr (F16 != 0) scale_back(IT, JT, av);
                 // eight pairs, every stage over all of them: independent chains side by side
                 f32x2v x[8];
 #pragma unroll
@@ -974,7 +1030,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
                 }
             }
         });
-        if (has_nxt) init_acc_from_bias(par_after(tile_par, 1));  // the next tile starts at its bias row (F16: at zero)
+        if (has_nxt) init_acc_from_bias(par_after(tile_par, 1), SK && role_nxt == 1);  // the next tile starts at its bias row (init_acc_from_bias)
         if constexpr (NPEND > 0) {
             pend_row = row0;
             pend_col = col0;
@@ -1033,6 +1089,10 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         for (int i = 0; i < 4; ++i) dma_a(0, 1, i, s0);
 #pragma unroll
         for (int i = 0; i < 4; ++i) dma_a(1, 0, i, s1);
+        if constexpr (F16 == F16_ONE) {
+            row_exp = *ex.a;
+            ZG_PIN(row_exp);
+        }
         if constexpr (KIND == S4_SPLIT2) {
             out_exp = *po.exp;
             ZG_PIN(out_exp);
@@ -1043,12 +1103,12 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
         if constexpr (P::PB == 6) asm volatile("s_waitcnt vmcnt(14)" ::: "memory");  // B and A half 0 of K-step 0 are in
         else asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
         bar();
-        init_acc_from_bias(0);  // (wave 0's bias pieces were the first of the stream: landed with the wait above)
+        init_acc_from_bias(0, SK && role_cur == 1);  // (wave 0's bias pieces were the first of the stream: landed with the wait above)
         read_kstep_head(Ic<0>{});
         phase_stamp();
     }
 
-    auto half_way = [&]() { return F16 && pi_cur == pl.npairs - 1 && kk_cur == kps >> 1; };
+    auto half_way = [&]() { return F16 != 0 && pi_cur == pl.npairs - 1 && kk_cur == kps >> 1; };
     // two K-steps per trip so that the slot is a compile-time constant; a tile may end after either
     for (;;) {
         kstep(Ic<0>{});
@@ -1095,11 +1155,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     }
 }
 
-template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, bool F16 = false>
+template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, int F16 = F16_NO>
 int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, int n_sl,
                   const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}, const PlaneOut& po = PlaneOut{}) {
     using P = S4<NT>;
-    constexpr int LDS = F16 ? P::LDS_F16 : P::LDS;
+    constexpr int LDS = F16 != 0 ? P::LDS_F16 : P::LDS;
     static OncePerDevice raised;  // (handles of the layered tier may be on different devices)
     int device = 0;
     ZG_HIP(hipGetDevice(&device));
@@ -1109,7 +1169,8 @@ int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
         return ZG_OK;
     }));
     const int tiles_m = (M + 255) / 256, tiles_n = (N + P::BN - 1) / P::BN, n_tiles = tiles_m * tiles_n * n_sl;
-    int gw = 8;  // tile-order band width (sweep 1 .. 16: profiles/NOTEBOOK.md)
+    // tile-order band width (sweep 1 .. 16: profiles/NOTEBOOK.md); F16: 8 x 1023 tokens of GPT-2 124M 4850 us at 4, 4820 at 8, 4814 at 16
+    int gw = F16 != 0 ? 16 : 8;
     if (gw > tiles_n) gw = tiles_n;
     const int cus_env = getenv("ZGPT2_GEMM_WGS") ? atoi(getenv("ZGPT2_GEMM_WGS")) : 0;  // tests: few workgroups, many tiles each
     const int cus = cus_env > 0 ? cus_env : 256;
@@ -1185,7 +1246,7 @@ int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, 
                "gemm: operands of %d x %d x %d beyond the 32-bit buffer descriptors", M, N, pl.kpp * 64);
     gemm_note_launch();
     note_kernel("gemm_s4_kernel");
-    return launch_s4_kind<3, S4_PLAIN, false, false, false, true>(A, B, bias, C, M, N, pl, ldc, 1, none, s, ex);
+    return launch_s4_kind<3, S4_PLAIN, false, false, false, F16_ROWS>(A, B, bias, C, M, N, pl, ldc, 1, none, s, ex);
 }
 
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s) {
@@ -1214,12 +1275,13 @@ int launch_gemm_s4_prefill(const PrefillA& A, const PrefillW& W, const float* bi
                "s4 prefill gemm: operands of %d x %d x %d beyond the 32-bit buffer descriptors", M, N, K);
     ZG_REQUIRE(n_slices >= 1 && pl.kpp % n_slices == 0 && pl.kpp / n_slices >= 2, ZG_ERR_ARG, "s4 prefill gemm: %d K slices of %d K-steps", n_slices, pl.kpp);
     const PrefillQkv none{};
-    const PlaneExps ex{A.exp, W.exps, A.each};
+    ZG_REQUIRE(!A.each, ZG_ERR_UNSUPPORTED, "s4 prefill gemm: one exponent for all rows");
+    const PlaneExps ex{A.exp, W.exps, false};
     gemm_note_launch();
     switch (kind) {
         case S4_PARTIAL:
             ZG_REQUIRE(bias == nullptr, ZG_ERR_ARG, "s4 prefill gemm: partial slabs carry no bias");
-            return launch_s4_kind<3, S4_PARTIAL, false, false, false, true>(A.p, W.p, nullptr, C, M, N, pl, ldc, n_slices, none, s, ex);
+            return launch_s4_kind<3, S4_PARTIAL, false, false, false, F16_ONE>(A.p, W.p, nullptr, C, M, N, pl, ldc, n_slices, none, s, ex);
         case S4_QKV: {
             ZG_REQUIRE(qkv && N == 3 * qkv->E && n_slices == 1, ZG_ERR_ARG, "s4 prefill gemm: S4_QKV needs the cache description");
             // 1.5 rounds of tiles (c_attn of eight 1023-token prompts: 384 tiles, 256 CUs): the last half round is split in K halves
@@ -1228,12 +1290,12 @@ int launch_gemm_s4_prefill(const PrefillA& A, const PrefillW& W, const float* bi
             const int G = cus_env > 0 ? cus_env : 256, tiles = ((M + 255) / 256) * ((N + 191) / 192);
             if (qkv->sk_ws != nullptr && qkv->sk_flags != nullptr && G % 16 == 0 && tiles > G && (tiles % G) * 2 == G && pl.kpp % 2 == 0 &&
                 pl.kpp >= 4 && (size_t)(G / 2) * 196608 <= qkv->sk_ws_bytes && (size_t)(G / 2) * 4 <= qkv->sk_flags_words)
-                return launch_s4_kind<3, S4_QKV, false, false, true, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
-            return launch_s4_kind<3, S4_QKV, false, false, false, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
+                return launch_s4_kind<3, S4_QKV, false, false, true, F16_ONE>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
+            return launch_s4_kind<3, S4_QKV, false, false, false, F16_ONE>(A.p, W.p, bias, C, M, N, pl, ldc, 1, *qkv, s, ex);
         }
         case S4_SPLIT2:
             ZG_REQUIRE(n_slices == 1 && po.exp, ZG_ERR_ARG, "s4 prefill gemm: S4_SPLIT2 is not sliced");
-            return launch_s4_kind<3, S4_SPLIT2, true, true, false, true>(A.p, W.p, bias, C, M, N, pl, ldc, 1, none, s, ex, po);
+            return launch_s4_kind<3, S4_SPLIT2, true, true, false, F16_ONE>(A.p, W.p, bias, C, M, N, pl, ldc, 1, none, s, ex, po);
     }
     ZG_REQUIRE(false, ZG_ERR_ARG, "s4 prefill gemm: kind %d", kind);
 }

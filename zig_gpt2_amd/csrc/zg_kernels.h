@@ -182,6 +182,7 @@ struct Split2Job {
     int rows;
     size_t lo = 0;           // the second plane lies this many elements behind the first (0: beside it, rows of 2K)
     float* norms = nullptr;  // 2-norms of the rows
+    const int* one = nullptr;  // the exponent of every row; else each gets its own
 };
 // for the test hooks of one Linear and one attention: rows of three bf16 planes -> fp32, rows of two fp16 planes times 2^exp -> three bf16 planes
 int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, float* out, hipStream_t s);
