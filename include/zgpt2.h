@@ -143,7 +143,8 @@ int zg_softmax(float* inputs, size_t inputs_len);
  * only, whose packed arguments end at K = 16320: beyond that ZG_ERR_UNSUPPORTED — zg_linear_forward, which has no such limit,
  * takes such a Linear through its GEMV kernels); K a multiple of 64 and at least 128.  Asynchronous on
  * the library stream.  zg_linear_forward itself takes this path for some thousand rows and more (fp32 operands split
- * exactly into bf16 planes, so the result stays fp32-sgemm grade); from nine rows on it splits inside smaller tiles.
+ * into planes — two-term fp16 of scaled rows, or three-term bf16 below 512 columns — so that the result stays fp32-sgemm grade); from nine rows on
+ * it splits inside smaller tiles.
  * zg_f32_to_bf16 converts a device or host fp32 array into a device bf16 array (round to nearest even). */
 int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_null, void* C, size_t M,
                     size_t N, size_t K, int gelu, int out_bf16);
@@ -152,6 +153,8 @@ int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_n
 unsigned long long zg_debug_gemm_launches(void);
 /* Diagnostic: the same of the kernel that takes fp32 Linears of five to fifteen rows on the matrix cores. */
 unsigned long long zg_debug_linear_few_mfma_launches(void);
+/* Diagnostic: the same of the kernel that takes fp32 Linears of some hundred rows and 1536 columns or more as fp16 planes. */
+unsigned long long zg_debug_linear_ring_launches(void);
 /* Diagnostic: shader-clock stamps {count, start, end} of workgroup 0 / wave 0 of the last GEMM launched with
  * ZGPT2_GEMM_DBG bit 256 (tools/microbench/gemm_bench.cpp: cycles vs wall time = the clock the chip ran at). */
 int zg_debug_gemm_stamps(unsigned long long* out, size_t n_words);

@@ -1,5 +1,5 @@
-"""fp32 Linears of many rows and 512 columns or more: three products of two-term fp16 planes on the persistent GEMM (gemm_s4.hip), whose rows carry
-exponents of their own.  Tile edges, ragged widths, one and several tiles a workgroup, both sides of the column rule, rows of very different
+"""fp32 Linears of many rows and 512 columns or more, and of some hundred rows and 1536 columns or more: three products of two-term fp16 planes on the
+persistent GEMM (gemm_s4.hip) and on prefill_ring_kernel, whose rows carry exponents of their own.  Tile edges, ragged widths, one and several tiles a workgroup, both sides of the column rule, rows of very different
 sizes, rows of zeros, of the smallest and of the largest values, values that are not finite.
 
 The bound, element by element, is what three products of such terms can be off: 2^-21 of the sum of |x w| for the terms (2^-23 each and 2^-22
@@ -53,7 +53,7 @@ def check(x, w, b, y):
     return ((y.double() - ref).norm() / ref.norm()).item()
 
 
-@pytest.mark.parametrize("m,k,n", [(4096, 512, 3072), (4097, 576, 3071), (1537, 768, 3073), (8191, 640, 1601), (2047, 1600, 1601), (6001, 3072, 769), (12300, 512, 1029)])
+@pytest.mark.parametrize("m,k,n", [(4096, 512, 3072), (4097, 576, 3071), (1537, 768, 3073), (8191, 640, 1601), (4501, 1600, 1601), (6401, 3072, 769), (12300, 512, 1029)])
 def test_tile_edges(zg, m, k, n):
     x, w, b = draw(m, k, n)
     b = None if n % 2 else b
@@ -62,6 +62,38 @@ def test_tile_edges(zg, m, k, n):
     assert zg.zg_debug_gemm_launches() == before + 1 and last_kernel(zg) == "gemm_s4_kernel"
     # (2-norm: what a chain of K products in two halves and the terms leave, each seen in the comments of the kernels, and a third more)
     assert check(x, w, b, y) <= 1.33 * ((1.2e-7 * (k / 768) ** 0.5) ** 2 + 0.75e-7 ** 2) ** 0.5
+
+
+@pytest.mark.parametrize("m,k,n,ring", [(700, 1600, 1600, 1), (700, 1600, 1603, 1), (321, 1600, 4800, 1), (1023, 3072, 769, 1), (700, 3072, 768, 1), (65, 6400, 9601, 1),
+                                        (450, 6400, 1600, 1), (2049, 1536, 1031, 1), (700, 1472, 1600, 0), (128, 1600, 1600, 0), (3000, 1600, 4800, 0)])
+def test_some_hundred_rows(zg, m, k, n, ring):
+    """Tiles of 64 and 128 rows, one slice of K and several, widths in no whole tiles and no whole fours, both sides of the rule."""
+    x, w, b = draw(m, k, n, spread=9)
+    b = None if n % 2 else b * 0.125
+    before = zg.zg_debug_linear_ring_launches()
+    y = forward(x, w, b)
+    assert zg.zg_debug_linear_ring_launches() == before + ring
+    check(x, w, b, y)
+
+
+@pytest.mark.parametrize("m,k,n", [(700, 1600, 1600), (700, 3072, 769)])  # one slice, several
+def test_values_that_are_not_finite_among_some_hundred_rows(zg, m, k, n):
+    """Outputs are what a plain sum makes of them: infinities stay infinities of their sign."""
+    x, w, b = draw(m, k, n)
+    clean = forward(x, w, b)
+    x[3, 100], x[300, 5], x[m - 1, k - 1] = float("nan"), float("inf"), -float("inf")
+    w[11, 5] = 0.0  # (times infinity)
+    before = zg.zg_debug_linear_ring_launches()
+    y = forward(x, w, b)
+    assert zg.zg_debug_linear_ring_launches() == before + 1
+    bad = torch.zeros(m, dtype=torch.bool, device="cuda")
+    bad[[3, 300, m - 1]] = True
+    keep = torch.ones(n, dtype=torch.bool, device="cuda")
+    keep[11] = False  # (its weight changed)
+    assert torch.equal(y[~bad][:, keep], clean[~bad][:, keep])
+    assert torch.isnan(y[3]).all() and torch.isnan(y[300, 11])
+    assert torch.equal(y[300][keep], torch.copysign(torch.full((n,), float("inf"), device="cuda"), w[:, 5])[keep])
+    assert torch.equal(y[m - 1], torch.copysign(torch.full((n,), float("inf"), device="cuda"), -w[:, k - 1]))
 
 
 @pytest.mark.parametrize("wgs", ["3", "16"])

@@ -116,6 +116,7 @@ SIGNATURES = {
     "zg_unregister_all": (C.c_int, []),
     "zg_debug_gemm_launches": (C.c_ulonglong, []),
     "zg_debug_linear_few_mfma_launches": (C.c_ulonglong, []),
+    "zg_debug_linear_ring_launches": (C.c_ulonglong, []),
     "zg_debug_gemm_stamps": (C.c_int, [vp, sz]),
     "zg_debug_last_kernel": (C.c_int, [C.c_char_p, sz]),
     "zg_debug_attn_prefill": (C.c_int, [vp, vp, sz, sz, sz, sz, vp, vp, sz, vp, sz, C.c_int]),

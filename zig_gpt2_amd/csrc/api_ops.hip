@@ -304,6 +304,13 @@ static bool linear_tiles_ok(size_t in_f, size_t out_f, size_t m, size_t arena_le
     return slices == 1 || (size_t)slices * m * out_f * sizeof(float) + 1024 <= arena_left;
 }
 
+// ... and those of some hundred rows, behind a pass that splits both operands (prefill_ring.hip): the slices of K, 0: another kernel's
+static int linear_ring_slices(size_t in_f, size_t out_f, size_t m, size_t arena_left, int* tm) {
+    if (in_f % 64 != 0 || in_f > 8192 || m < 16 || m >= (1u << 28) / in_f || out_f >= (1u << 28) / in_f) return 0;
+    const int slices = linear_ring_route(m, out_f, in_f, tm);
+    return slices > 0 && linear_ring_scratch(m, out_f, in_f, slices) + 1024 <= arena_left ? slices : 0;
+}
+
 static int linear_tiles(Call& call, size_t in_f, size_t out_f, const float* w, const float* bias, const float* x, size_t m, float* y) {
     const int slices = linear_tiles_slices(m, out_f, in_f);
     float* slabs = nullptr;
@@ -580,9 +587,14 @@ int zg_linear_forward(size_t in_features, size_t out_features, const float* weig
     ZG_TRY(call.in(inputs, inputs_len, &x));  // (read by every workgroup: device memory)
     if (in_features <= 8192) ZG_TRY(call.out_once(outputs, batch * out_features, &y));  // every element stored once
     else ZG_TRY(call.out(outputs, batch * out_features, &y));                          // K chunks accumulate into y
+    int ring_rows = 1;
     if (linear_few_ok(batch, out_features, in_features) && out_features < (1u << 30))
         ZG_TRY(launch_linear_few(x, w, b, y, (int)batch, (int)out_features, (int)in_features, call.stream()));
-    else if (linear_tiles_ok(in_features, out_features, batch, call.arena_left()))
+    else if (const int slices = linear_ring_slices(in_features, out_features, batch, call.arena_left(), &ring_rows)) {
+        char* scratch;
+        ZG_TRY(call.scratch(linear_ring_scratch(batch, out_features, in_features, slices), &scratch));
+        ZG_TRY(launch_linear_ring(x, w, b, y, (int)batch, (int)out_features, (int)in_features, ring_rows, slices, scratch, call.stream()));
+    } else if (linear_tiles_ok(in_features, out_features, batch, call.arena_left()))
         ZG_TRY(linear_tiles(call, in_features, out_features, w, b, x, batch, y));
     else if (linear_mfma_ok(in_features, out_features, batch, call.arena_left()))
         ZG_TRY(linear_mfma(call, in_features, out_features, w, b, x, batch, y));
@@ -725,6 +737,7 @@ int zg_debug_prefill_route(int force_kernel, int slices) {
 
 unsigned long long zg_debug_gemm_launches(void) { return gemm_mfma_launch_count(); }
 unsigned long long zg_debug_linear_few_mfma_launches(void) { return linear_few_mfma_launch_count(); }
+unsigned long long zg_debug_linear_ring_launches(void) { return linear_ring_launch_count(); }
 int zg_debug_gemm_stamps(unsigned long long* out, size_t n_words) { return gemm_debug_stamps(out, n_words); }
 
 int zg_f32_to_bf16(const float* src, uint16_t* dst_device, size_t len) {

@@ -40,21 +40,6 @@ __device__ __forceinline__ Terms split8(const f32x4& a, const f32x4& b) {
     return t;
 }
 
-// An output again as a plain fp32 sum.  The terms of a value that is not finite, or that rounds up to an infinity (above the largest bf16), meet
-// as infinity minus infinity and infinity times zero: outputs they leave not finite are worked out here, behind the stores (a sum that has become
-// NaN ends at once).  The others pay one comparison: 768 -> 3072, 16 rows 19.5 us (19.7 without), 512 rows 38.0 (39.0).
-__device__ __forceinline__ float plain_sum(const float* x, const float* w, int K) {
-    float s = 0.0f;
-#pragma unroll 1
-    for (int k = 0; k < K && s == s; k += 4) {
-        const f32x4 a = *reinterpret_cast<const f32x4*>(x + k), b = *reinterpret_cast<const f32x4*>(w + k);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
-    }
-    return s;
-}
-__device__ __forceinline__ float odd(float v) { return fabsf(v) <= 3.4028235e38f ? 0.0f : 1.0f; }  // not finite
-
 // What bounds it: the LDS, which takes 24 KB of terms and gives 48 KB of fragments a step, beside 384 cycles of products.
 __global__ __launch_bounds__(256, 2) void linear_tiles_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias,
                                                               float* __restrict__ Y, int M, int N, int K, int steps) {

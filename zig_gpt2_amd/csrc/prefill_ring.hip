@@ -10,6 +10,7 @@
 // of their own, added to the steps' before it beside the products of the next, so that neither they nor the small ones are rounded at the size of
 // the whole.
 #include <algorithm>
+#include <atomic>
 #include <type_traits>
 
 #include "prefill_epi.h"
@@ -40,10 +41,15 @@ __device__ __forceinline__ u32x4 rsrc_of(const void* base) {
     return u32x4{(uint32_t)a, (uint32_t)(a >> 32) & 0xffffu, 0x80000000u, 0x00020000u};
 }
 
+// PF_LINEAR: the fp32 operands themselves, for outputs that are not finite (plain_sum); ldc is then the number of columns, N the same in whole 64s
+struct RawRows {
+    const float *x, *w;
+};
+
 // 2 x 2 waves of TM x 1 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
 template <int EPI, int TM, int NW, int ST>
 __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
-                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
+                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw) {
     constexpr int BM = 64 * TM, BN = 64, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
     constexpr int REQ = kPair * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
     extern __shared__ __attribute__((aligned(1024))) char s_ring[];
@@ -115,7 +121,14 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     // what the epilogue needs besides the sums, on its way before the requests
     const int cc = (lane & 7) * 4, n = n0 + wx * 32 + cc;
     const i32x4 col_exp = *reinterpret_cast<const i32x4*>(ex.w + n);
-    const f32x4 bv = EPI != PF_PARTIAL && bias ? *reinterpret_cast<const f32x4*>(bias + n) : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 bv = {0.0f, 0.0f, 0.0f, 0.0f};
+    if (EPI == PF_LINEAR) {
+        if (bias)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bv[e] = bias[min(n + e, ldc - 1)];
+    } else if (EPI != PF_PARTIAL && bias) {
+        bv = *reinterpret_cast<const f32x4*>(bias + n);
+    }
     int row_exp[TM][4];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
@@ -181,6 +194,19 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = gelu_fast(v[e]);
                 store_split4(reinterpret_cast<uint16_t*>(C) + (size_t)m * kPair * N + n, N, v, out_exp, po.coarse);
+            } else if constexpr (EPI == PF_LINEAR) {
+                float* y = reinterpret_cast<float*>(C) + (size_t)m * ldc + n;
+                if ((ldc & 3) == 0 && n < ldc) {
+                    *reinterpret_cast<f32x4*>(y) = v;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < ldc) y[e] = v[e];
+                }
+                if (odd(v[0]) + odd(v[1]) + odd(v[2]) + odd(v[3]) > 0.0f)
+#pragma unroll 1
+                    for (int e = 0; e < 4; ++e)
+                        if (n + e < ldc && odd(v[e]) > 0.0f) y[e] = plain_sum(raw.x + (size_t)m * K, raw.w + (size_t)(n + e) * K, K) + bv[e];
             } else if constexpr (EPI == PF_PARTIAL) {  // C: slabs [n_sp][M][N]
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)blockIdx.y * M + m) * N + n) = v;
             } else {
@@ -192,7 +218,8 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 }
 
 template <int EPI, int TM, int NW, int ST>
-int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
+int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s,
+                const RawRows& raw = RawRows{}) {
     constexpr int LDS = ST * (kPair * 64 * TM + NW * 64) * kRow;
     static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
     static OncePerDevice raised;
@@ -203,7 +230,7 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * (N / 64);
-    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po);
+    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -217,7 +244,102 @@ int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, voi
     return tm == 1 ? launch_ring<EPI, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
 }
 
+// the slabs [n_sp][M][Np] of a Linear added, and its bias: a thread four columns of a row
+__global__ __launch_bounds__(256) void linear_ring_finish_kernel(const float* __restrict__ slabs, int n_sp, int M, int Np, const float* __restrict__ bias, float* __restrict__ Y, int N,
+                                                                 const float* __restrict__ X, const float* __restrict__ W, int K) {
+    const int n4 = (N + 3) / 4;
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (long long)M * n4) return;
+    const int m = (int)(i / n4), n = (int)(i % n4) * 4;
+    const float* p = slabs + (size_t)m * Np + n;
+    const size_t slab = (size_t)M * Np;
+    f32x4 v = *reinterpret_cast<const f32x4*>(p);
+    for (int s0 = 1; s0 < n_sp; s0 += 4) {
+        f32x4 t[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) t[u] = *reinterpret_cast<const f32x4*>(p + (size_t)min(s0 + u, n_sp - 1) * slab);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (s0 + u < n_sp) v += t[u];
+    }
+    float* y = Y + (size_t)m * N + n;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (n + e >= N) break;
+        const float b = bias ? bias[n + e] : 0.0f, sum = v[e] + b;
+        y[e] = odd(v[e]) > 0.0f ? plain_sum(X + (size_t)m * K, W + (size_t)(n + e) * K, K) + b : sum;
+    }
+}
+
 }  // namespace
+
+namespace {
+size_t whole(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
+size_t whole64(size_t n) { return (n + 63) / 64 * 64; }
+}  // namespace
+
+size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp) {
+    const size_t Np = whole64(N);
+    return whole(M * K * 4) + whole(Np * K * 4) + whole(M * 4) + whole(Np * 4) + (n_sp > 1 ? whole((size_t)n_sp * M * Np * 4) : 0);
+}
+
+static std::atomic<unsigned long long> g_linear_ring_launches{0};
+unsigned long long linear_ring_launch_count() { return g_linear_ring_launches.load(std::memory_order_relaxed); }
+
+int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s) {
+    const int Np = (int)whole64(N);
+    ZG_REQUIRE(M > 0 && N > 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (tm == 1 || tm == 2) && (size_t)M * K * 4 < ((size_t)1 << 31) && (size_t)Np * K * 4 < ((size_t)1 << 31),
+               ZG_ERR_UNSUPPORTED, "linear: %d x %d x %d", M, N, K);
+    uint16_t *xp = reinterpret_cast<uint16_t*>(scratch), *wp = reinterpret_cast<uint16_t*>(scratch += whole((size_t)M * K * 4));
+    int *xe = reinterpret_cast<int*>(scratch += whole((size_t)Np * K * 4)), *we = reinterpret_cast<int*>(scratch += whole((size_t)M * 4));
+    float* slabs = reinterpret_cast<float*>(scratch += whole((size_t)Np * 4));
+    // (the weight's rows beyond N hold whatever the scratch held: their columns are never stored)
+    ZG_TRY(launch_split2(Split2Job{X, xp, xe, M}, Split2Job{W, wp, we, N, (size_t)Np * K}, K, s));
+    const PrefillA A{xp, xe, true};
+    const PrefillW P{wp, we, 2};
+    g_linear_ring_launches.fetch_add(1, std::memory_order_relaxed);
+    if (n_sp == 1) {
+        const PrefillQkv none{};
+        const RawRows raw{X, W};
+        ZG_TRY(tm == 1 ? (launch_ring<PF_LINEAR, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
+                       : (launch_ring<PF_LINEAR, 2, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw)));
+        note_kernel("linear_tiles_kernel");  // (the Linears of a medium number of rows have one name; the count says which)
+        return ZG_OK;
+    }
+    ZG_TRY(launch_prefill_ring(A, P, nullptr, slabs, M, Np, K, Np, PF_PARTIAL, tm, n_sp, PrefillQkv{}, PlaneOut{}, s));
+    const size_t quads = (size_t)M * ((N + 3) / 4);
+    linear_ring_finish_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(slabs, n_sp, M, Np, bias, Y, N, X, W, K);
+    ZG_HIP(hipGetLastError());
+    note_kernel("linear_tiles_kernel");
+    return ZG_OK;
+}
+
+// Priced in us like the prompts' Linears below, with 3 for the launch that adds slabs.  It takes a Linear of 1536 columns and more where the kernel that splits in its own staging
+// has few slices of K to add up, whose chains are then so long that this kernel is closer to 64 bits as well (1600 columns in two slices 1.67e-7, here
+// 1.38e-7; 3072 in four 1.66e-7 and 1.63e-7; 768 in two 1.16e-7 and 1.22e-7), and where it is cheap beside the persistent one (rounds of 256 x 192 tiles).  us of a call
+// with it : without: 3072 -> 768 700 rows 42 : 50, 2048 73 : 93, 3000 120 : 143; 1600 -> 1600 700 rows 45 : 52, 2048 76 : 110; 1600 -> 4800 256 rows
+// 47 : 53, 700 77 : 110; 6400 -> 1600 400 rows 82 : 107, 2048 241 : 392; not taken: 1600 -> 4800 1500 rows 139 : 119, 768 -> 768 3000 rows 50 : 46.
+int linear_ring_route(size_t M, size_t N, size_t K, int* tm) {
+    if (K < 1536 || linear_tiles_slices(M, N, K) > (K < 3072 ? 2 : 4)) return 0;
+    const int nk = (int)(K / kBk);
+    const double slab = (double)M * (double)whole64(N) * 8.0 / 4e6;
+    auto rounds = [](long n) { return (double)((n + 255) / 256); };
+    int best = 0;
+    double best_us = rounds((long)((M + 255) / 256 * ((N + 191) / 192))) * (3.2 * nk + 10.0) * 0.75;
+    for (int t = 1; t <= 2; ++t) {
+        const long tiles = (long)((M + 64 * t - 1) / (64 * t)) * (long)((N + 63) / 64);
+        const long most = std::max(1l, std::min(256 / tiles, (long)nk / 3));
+        for (long n = 1; n <= most; ++n) {
+            const double us = rounds(tiles * n) * (3.0 + (double)((nk + n - 1) / n) * (16.0 * t + 16.0) / 57.0) + (n > 1 ? (double)n * slab + 3.0 : 0.0);
+            if (us < best_us) {
+                best = (int)n;
+                best_us = us;
+                *tm = t;
+            }
+        }
+    }
+    return best;
+}
 
 // K slices of the launch (1 unless it is a residual Linear, whose slices meet in slabs) and rows of a tile (64 tm); 0: the 128-row kernels take it.
 // Both sides are priced in us by what one compute unit takes in (65 bytes a ns; 57 with the weight's planes; 42 where two slots of 56 KB are

@@ -115,6 +115,21 @@ __device__ __forceinline__ int split2_exp(uint32_t top) {
     return 141 - (e < 1 ? 1 : e);
 }
 
+// An output again as a plain fp32 sum.  The terms of a value that is not finite, or of three bf16 terms one that rounds up to an infinity, meet
+// as infinity minus infinity and infinity times zero: outputs they leave not finite are worked out here, behind the stores (a sum that has become
+// NaN ends at once).  The others pay one comparison: 768 -> 3072, 16 rows 19.5 us (19.7 without), 512 rows 38.0 (39.0).
+__device__ __forceinline__ float plain_sum(const float* x, const float* w, int K) {
+    float s = 0.0f;
+#pragma unroll 1
+    for (int k = 0; k < K && s == s; k += 4) {
+        const f32x4 a = *reinterpret_cast<const f32x4*>(x + k), b = *reinterpret_cast<const f32x4*>(w + k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
+    }
+    return s;
+}
+__device__ __forceinline__ float odd(float v) { return fabsf(v) <= 3.4028235e38f ? 0.0f : 1.0f; }  // not finite
+
 // Activation planes of the lock-step batch in global memory: the epilogue of the producing kernel writes the exact
 // three-term bf16 split of its output row, the consuming Linear loads them as MFMA A fragments — no LDS staging and no
 // split in front of its MFMAs.  Element (plane p, batch row m < 8, column k) of a [3][8][K] triple sits at

@@ -261,7 +261,7 @@ struct PrefillW {
     const int* exps;
     int planes;
 };
-enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4 };
+enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4, PF_LINEAR = 5 /* internal: Linear.forward */ };
 int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, const void* wte, const void* wpe,
                          int weight_type, int E, float* x, hipStream_t s);
 int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, uint16_t* out, const PlaneOut& po, hipStream_t s);
@@ -313,6 +313,12 @@ struct PrefillBounds {
     int* exps;
 };
 int launch_prefill_bounds(const PrefillBounds& b, int E, hipStream_t s);
+// ... and the fp32 Linears of the op tier with some hundred rows on the same kernel, behind a pass that splits both operands.  The route: slices of K (0: not taken), tm
+// as above; scratch: linear_ring_scratch bytes.
+int linear_ring_route(size_t M, size_t N, size_t K, int* tm);
+unsigned long long linear_ring_launch_count();  // Linears it has taken so far
+size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp);
+int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s);
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
 // out[M][kPair E] = planes of the causal attention of the q / k / v columns of qkv[M][3E], M = B P rows ordered (b, t)
 // (attn_prefill.hip: matrix cores on two-term fp16 planes; ws = fp32 workspace for the partials of split key ranges).  exps: kBounds of them; the output
