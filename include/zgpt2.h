@@ -170,8 +170,8 @@ int zg_debug_prefill_linear(const uint16_t* A_planes, const uint16_t* W, const f
 /* Diagnostic / test entry: the causal prompt attention of zg_gpt_prefill alone (scaled_dot_product_attention of src/ops.zig:249-307
  * for all n_tokens positions of `batch` sequences at once).  qkv: fp32 [batch n_tokens][3 n_embed] rows (q | k | v columns);
  * out: bf16 planes [batch n_tokens][3 n_embed] = hi | mid | lo of the attention output; k_cache / v_cache: NULL (K and V are the
- * qkv columns) or head-major fp32 caches [batch][heads][ctx][64] holding the same rows; ws: fp32 workspace for the partials of
- * split key ranges (may be NULL: whole rows per workgroup); key_tiles: key tiles of 32 per workgroup, 0 = the library's choice.
+ * qkv columns) or head-major fp32 caches [batch][heads][ctx][64] holding the same rows; ws: of diagnostic builds (may be NULL);
+ * key_tiles: 0 = the library's choice, above: the kernel of many prompts (groups of 128 queries) at any size.
  * Device pointers. */
 int zg_debug_attn_prefill(const float* qkv, uint16_t* out, size_t batch, size_t n_tokens, size_t n_embed, size_t n_heads,
                           const float* k_cache, const float* v_cache, size_t ctx, float* ws, size_t ws_floats, int key_tiles);

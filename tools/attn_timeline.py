@@ -20,7 +20,7 @@ qkv_d, kc_d, vc_d = dev(qkv), dev(kc), dev(vc)
 out = torch.zeros((B * P, 3 * E), dtype=torch.int16, device="cuda")
 ws = torch.zeros(16 << 20, dtype=torch.float32, device="cuda")
 torch.cuda.synchronize()
-run = lambda: _lib.check(lib.zg_debug_attn_prefill(qkv_d.data_ptr(), out.data_ptr(), B, P, E, H, kc_d.data_ptr(), vc_d.data_ptr(), ctx, ws.data_ptr(), ws.numel(), 0))
+run = lambda: _lib.check(lib.zg_debug_attn_prefill(qkv_d.data_ptr(), out.data_ptr(), B, P, E, H, kc_d.data_ptr(), vc_d.data_ptr(), ctx, ws.data_ptr(), ws.numel(), 1))
 for _ in range(5): run()
 torch.cuda.synchronize()
 ng = ((P + 31) // 32 + 3) // 4

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Time the causal prompt attention kernel alone (zg_debug_attn_prefill): tools/bench_attn_prefill.py [batch] [tokens] [heads] [key_tiles]
-K / V from head-major fp32 caches, as zg_gpt_prefill runs it.  Prints us per call (merge kernel included when key ranges are split)
+K / V from head-major fp32 caches, as zg_gpt_prefill runs it.  Prints us per call (key_tiles 1: the kernel of many prompts at any size)
 and the matrix-core rate of the six plane products over the causal half."""
 import json, os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

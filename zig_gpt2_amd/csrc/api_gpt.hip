@@ -626,8 +626,8 @@ int enqueue_prefill(zg_gpt* g, size_t P, bool last_block_full, hipStream_t s) {
                                    g->pf_ws, g->pf_ws_floats, nullptr, s, &qa));
         if (l + 1 == L && !last_block_full) break;
         // (an fp32 cache is read directly: the c_attn epilogue then need not store the k / v columns of qkv)
-        ZG_TRY(launch_attn_prefill(g->pf_qkv, g->pf_a, B, (int)P, iE, (int)H, g->pf_ws, g->pf_ws_floats, g->kv_mode == 0 ? (const float*)y.k_cache : nullptr,
-                                       g->kv_mode == 0 ? (const float*)y.v_cache : nullptr, (int)C, y.exps, coarse, s));
+        ZG_TRY(launch_attn_prefill(g->pf_qkv, g->pf_a, B, (int)P, iE, (int)H, g->kv_mode == 0 ? (const float*)y.k_cache : nullptr,
+                                   g->kv_mode == 0 ? (const float*)y.v_cache : nullptr, (int)C, y.exps, coarse, s));
         const PrefillLn ln2{y.ln_2_g, y.ln_2_b, 1e-5f, g->pf_a, PlaneOut{y.exps + PB_LN2, coarse}};
         ZG_TRY(launch_prefill_gemm(PrefillA{g->pf_a, y.exps + PB_V, false}, y.c_proj_p, y.c_proj_b, g->pf_x, M, iE, iE, iE, PF_RESID, g->pf_ws,
                                    g->pf_ws_floats, &ln2, s));

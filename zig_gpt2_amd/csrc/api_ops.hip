@@ -720,7 +720,8 @@ int zg_debug_attn_prefill(const float* qkv, uint16_t* out, size_t batch, size_t 
         for (int which = 0; which < 3; ++which) e[PB_Q + which] = top[which] > 0.0f ? ilogbf(top[which]) - 11 : 0;
         ZG_HIP(hipMemcpyAsync(exps, e, sizeof e, hipMemcpyHostToDevice, s));
         ZG_HIP(hipStreamSynchronize(s));
-        ZG_TRY(launch_attn_prefill(qkv, planes, (int)batch, (int)n_tokens, (int)n_embed, (int)n_heads, ws, ws_floats, k_cache, v_cache, (int)ctx_len, exps, 0, s, key_tiles));
+        ZG_TRY(launch_attn_prefill(qkv, planes, (int)batch, (int)n_tokens, (int)n_embed, (int)n_heads, k_cache, v_cache, (int)ctx_len, exps, 0, s, key_tiles > 0,
+                                   reinterpret_cast<unsigned long long*>(ws)));
         return launch_join_planes(planes, exps + PB_V, (int)rows, (int)n_embed, kPair, out, s);
     };
     const int st = all();

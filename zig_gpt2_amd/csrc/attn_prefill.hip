@@ -15,8 +15,7 @@
 // global loads in flight under the current tile's products.  Everything is computed transposed (S^T = K Q^T, O^T = V^T P^T):
 // the query is the lane, so every per-query statistic is one register of one lane and P needs no transpose between the two
 // products (the k index of an MFMA step only has to agree between its operands: the keys a lane holds after S^T are the keys
-// its P fragment multiplies).  Long rows of few sequences are cut into key ranges over several workgroups whose (m, l, O)
-// partials a small kernel merges (one prompt of 1023 tokens would otherwise be 96 workgroups of up to 32 tiles).
+// its P fragment multiplies).  A few prompts have too few such workgroups: theirs are blocks of 32 queries (attn_prefill_block_kernel below).
 #include <type_traits>
 
 #include "prefill_epi.h"
@@ -53,12 +52,6 @@ __device__ __forceinline__ float both_halves_sum(float v) {
 
 __device__ __forceinline__ f16x8 frag(uint32_t a, uint32_t b, uint32_t c, uint32_t d) { return __builtin_bit_cast(f16x8, u32x4{a, b, c, d}); }
 
-// key tiles a group of four query blocks needs, and the key ranges (splits) it is cut into
-__host__ __device__ inline int group_tiles(int g, int nqb) { return 4 * g + 4 < nqb ? 4 * g + 4 : nqb; }
-__host__ __device__ inline int group_splits(int g, int nqb, int nts) { return (group_tiles(g, nqb) + nts - 1) / nts; }
-
-// geo = key tiles per split | most splits of a group << 8 | query groups << 16.  part: [B][H][P][max splits][66] (O^T[64], m, l).
-//
 // One instruction stream per wave, software-pipelined over the key tiles so that the matrix pipe and the vector ALU of a SIMD
 // work side by side WITHIN a wave (the first version ran S -> softmax -> split -> PV -> staging in sequence: 48 MFMAs = 1.5 k
 // cycles of a 6.4 k-cycle tile, 45 % matrix-busy with two waves per SIMD):
@@ -76,27 +69,24 @@ struct AttnKv {
     size_t stride_b, stride_h;
     unsigned stride_t;
 };
-__global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __restrict__ qkv, uint16_t* __restrict__ out, float* __restrict__ part,
-                                                                 int P, int E, unsigned geo, const AttnKv kv, const int* __restrict__ exps, int coarse) {
+__global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __restrict__ qkv, uint16_t* __restrict__ out, int P, int E, const AttnKv kv,
+                                                                 const int* __restrict__ exps, int coarse, unsigned long long* stamps) {
     const int exp_q = exps[PB_Q], exp_k = exps[PB_K], exp_v = exps[PB_V];
     const float s_back = ldexpf(1.0f, exp_q + exp_k);  // scores leave the products 2^-(exp_q + exp_k) times as large
     extern __shared__ __attribute__((aligned(1024))) char lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l31 = lane & 31, hl = lane >> 5;
-    const int nts = (int)(geo & 0xffu), max_s = (int)((geo >> 8) & 0xffu), ng = (int)(geo >> 16);
-    // grid (H, B, groups x splits): the dispatcher hands out workgroups in linear order, x fastest — the longest groups of EVERY
+    // grid (H, B, groups): the dispatcher hands out workgroups in linear order, x fastest — the longest groups of EVERY
     // (sequence, head) first, the short ones fill the tail (with the groups innermost the last sequence's 32-tile group started
     // when the rest of the chip was nearly done: 1.0 waves per SIMD on average instead of 2)
-    const int xg = (int)blockIdx.z / max_s, s = (int)blockIdx.z - xg * max_s, g = ng - 1 - xg;
-    const int h = blockIdx.x, b = blockIdx.y, H = gridDim.x;
+    const int g = (int)gridDim.z - 1 - (int)blockIdx.z;
+    const int h = blockIdx.x, b = blockIdx.y;
     const int nqb = (P + 31) >> 5;
-    const int kt0 = s * nts, kt1 = min((s + 1) * nts, group_tiles(g, nqb));
-    if (kt0 >= kt1) return;
-#ifdef ZG_STAMPS  // diagnostic build: every workgroup's start / end (s_memrealtime, 100 MHz) and where it ran -> part[] (unsplit launches only)
+    const int n_t = min(4 * g + 4, nqb);  // key tiles
+#ifdef ZG_STAMPS  // diagnostic build: every workgroup's start / end (s_memrealtime, 100 MHz) and where it ran
     const unsigned long long stamp0 = __builtin_amdgcn_s_memrealtime();
 #endif
-    const int n_t = kt1 - kt0;
     const int qb = 4 * g + wave, tq = qb * 32 + l31;
     const size_t row0 = (size_t)b * P;
     const int ld = 3 * E;
@@ -210,24 +200,23 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
     f32x16 sc;
     {
         u32x4 k1[2];
-        load_k(kt0, kr);
-        load_v(kt0, vr);
-        load_k(kt0 + 1, k1);
+        load_k(0, kr);
+        load_v(0, vr);
+        load_k(1, k1);
         store_k(0, kr);
         store_v(0, vr);
         store_k(1, k1);
-        load_k(kt0 + 2, kr);
-        load_v(kt0 + 1, vr);
+        load_k(2, kr);
+        load_v(1, vr);
         __syncthreads();
         s_tile(0, sc);
         __syncthreads();  // (K slot 0 is rewritten in the first tile's phase B: every wave must have read K(0) out)
     }
 
-    // one tile: i = its index in the range (slot parity SLOT = i & 1), WITH_S = a next tile exists
-    auto body = [&](auto SLOT_T, auto WITH_S_T, int i) {
+    // tile kt (slot parity SLOT = kt & 1), WITH_S = a next tile exists
+    auto body = [&](auto SLOT_T, auto WITH_S_T, int kt) {
         constexpr int SLOT = decltype(SLOT_T)::value;
         constexpr bool WITH_S = decltype(WITH_S_T)::value;
-        const int kt = kt0 + i;
         // sc[r] = log2(e) / 8 * q . k / s_back of key kt * 32 + (r & 3) + 8 (r >> 2) + 4 hl against query tq
         if (kt >= qb) {  // diagonal tile (and the tiles past it, which a sibling wave needs): position tq sees keys 0 .. tq
 #pragma unroll
@@ -296,8 +285,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
                 o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[1][PK[t]], pf[PQ[t]][sp], o1, 0, 0, 0);
             }
         }
-        store_k(SLOT, kr);       // K(i + 2): the slot K(i) left in the previous tile's phase A
-        store_v(SLOT ^ 1, vr);   // V(i + 1): the slot V(i - 1) left in the previous tile's phase B
+        store_k(SLOT, kr);       // K(kt + 2): the slot K(kt) left in the previous tile's phase A
+        store_v(SLOT ^ 1, vr);   // V(kt + 1): the slot V(kt - 1) left in the previous tile's phase B
         load_k(kt + 3, kr);
         load_v(kt + 2, vr);
         if constexpr (WITH_S) {
@@ -322,8 +311,8 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         }
     }
 #ifdef ZG_STAMPS
-    if (tid == 0 && max_s == 1) {
-        unsigned long long* st = reinterpret_cast<unsigned long long*>(part) + 4 * ((size_t)(blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
+    if (tid == 0 && stamps != nullptr) {
+        unsigned long long* st = stamps + 4 * ((size_t)(blockIdx.z * gridDim.y + blockIdx.y) * gridDim.x + blockIdx.x);
         st[0] = stamp0;
         st[1] = __builtin_amdgcn_s_memrealtime();
         st[2] = (unsigned long long)__builtin_amdgcn_s_getreg((4 << 0) | (0 << 6) | (31 << 11)) |         // HW_REG_HW_ID
@@ -334,117 +323,186 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
     if (qb >= nqb || tq >= P) return;
 
     // O^T: the lane holds d = (r & 3) + 8 (r >> 2) + 4 hl (+ 32 in o1) of its query
-    if (group_splits(g, nqb, nts) == 1) {  // softmax divides by the sum (ops.zig:239); the c_proj GEMM takes the rows as planes
-        const float inv = 1.0f / lrun;  // (o is a mean of v's planes: it leaves with v's exponent)
-        uint16_t* hi = out + (row0 + tq) * kPair * E + h * 64;
+    const float inv = 1.0f / lrun;  // softmax divides by the sum (ops.zig:239); the c_proj GEMM takes the rows as planes (a mean of v's: they leave with v's exponent)
+    uint16_t* hi = out + (row0 + tq) * kPair * E + h * 64;
 #pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-            const int d = 8 * gq + 4 * hl;
-            store_split4(hi + d, E, f32x4{o0[gq * 4] * inv, o0[gq * 4 + 1] * inv, o0[gq * 4 + 2] * inv, o0[gq * 4 + 3] * inv}, 0, coarse);
-            store_split4(hi + 32 + d, E, f32x4{o1[gq * 4] * inv, o1[gq * 4 + 1] * inv, o1[gq * 4 + 2] * inv, o1[gq * 4 + 3] * inv}, 0, coarse);
-        }
-    } else {
-        float* pp = part + ((((size_t)b * H + h) * P + tq) * max_s + s) * 66;
-#pragma unroll
-        for (int gq = 0; gq < 4; ++gq) {
-            const int d = 8 * gq + 4 * hl;  // (66-float records: 8-byte aligned)
-            *reinterpret_cast<float2*>(pp + d) = float2{o0[gq * 4], o0[gq * 4 + 1]};
-            *reinterpret_cast<float2*>(pp + d + 2) = float2{o0[gq * 4 + 2], o0[gq * 4 + 3]};
-            *reinterpret_cast<float2*>(pp + 32 + d) = float2{o1[gq * 4], o1[gq * 4 + 1]};
-            *reinterpret_cast<float2*>(pp + 32 + d + 2) = float2{o1[gq * 4 + 2], o1[gq * 4 + 3]};
-        }
-        if (hl == 0) *reinterpret_cast<float2*>(pp + 64) = float2{mrun, lrun};
+    for (int gq = 0; gq < 4; ++gq) {
+        const int d = 8 * gq + 4 * hl;
+        store_split4(hi + d, E, f32x4{o0[gq * 4] * inv, o0[gq * 4 + 1] * inv, o0[gq * 4 + 2] * inv, o0[gq * 4 + 3] * inv}, 0, coarse);
+        store_split4(hi + 32 + d, E, f32x4{o1[gq * 4] * inv, o1[gq * 4 + 1] * inv, o1[gq * 4 + 2] * inv, o1[gq * 4 + 3] * inv}, 0, coarse);
     }
 }
 
-// The key ranges of a query meet: weights 2^(m_s - max m), sums in split order, one division; rows of groups that ran as one
-// range were finished by the attention kernel itself.  One thread = four head dimensions of one (sequence, head, query).
-__global__ __launch_bounds__(256) void attn_prefill_merge_kernel(const float* __restrict__ part, uint16_t* __restrict__ out, int P, int E, int H, int B,
-                                                                 unsigned geo, int coarse) {
-    const int nts = (int)(geo & 0xffu), max_s = (int)((geo >> 8) & 0xffu);
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    const int d = (int)(i & 15) * 4;
-    const size_t rec = i >> 4;  // (b, h, q)
-    if (rec >= (size_t)B * H * P) return;
-    const int q = (int)(rec % P), h = (int)((rec / P) % H), b = (int)(rec / ((size_t)P * H));
-    const int n = group_splits(q >> 7, (P + 31) >> 5, nts);
-    if (n == 1) return;
-    const float* pp = part + rec * max_s * 66;
-    float m = -INFINITY;
-    f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
-    float l = 0.0f;
-    if (n <= 8) {
-        // every load of the (up to eight) ranges issued before the first use: a loop over n with the maximum threaded through it
-        // waits for each range's record in turn — 2 n dependent round trips, 7.4 us per launch at one 1023-token prompt
-        float2 ml[8], a[8], c[8];
+// A workgroup per query block of 32 rows of one (sequence, head): its waves take the block's key tiles in turn, each straight from memory into
+// fragments (a lane has a key of K, a head dimension of V), and their (m, l, O) meet in the LDS.  No barrier before that, no wave that
+// waits for another's staging, four times as many workgroups: what bounds prompts of a few sequences is how little of the chip the groups of
+// 128 queries fill and one tile's chain of latencies behind another's.  But every block splits the keys and values it sees again, four times as often.
+// us a launch, 12 heads, beside the kernel above (its key ranges cut over workgroups, with the launch that merged them): 1 x 64 tokens 4.9 : 7.0,
+// 1 x 300 8.5 : 16.0, 1 x 1023 21 : 27, 4 x 300 13 : 21, 8 x 150 9.2 : 18.8, 2 x 1023 31 : 36; 25 heads 1 x 400 12.4 : 20.6, 2 x 400 17 : 23.
+// Eight waves a block are slower from 1 x 300 on (9.0; 2 x 1023 36).
+constexpr int kBlockWaves = 4;
+__global__ __launch_bounds__(kBlockWaves * 64, 2) void attn_prefill_block_kernel(const float* __restrict__ qkv, uint16_t* __restrict__ out, int P, int E, const AttnKv kv,
+                                                                        const int* __restrict__ exps, int coarse) {
+    constexpr int PITCH = 68;  // floats of a query's row of a wave's partial sums
+    __shared__ __attribute__((aligned(16))) float s_part[kBlockWaves * 32 * PITCH];
+    __shared__ float s_m[kBlockWaves * 32], s_l[kBlockWaves * 32];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l31 = lane & 31, hl = lane >> 5;
+    const int h = blockIdx.x, b = blockIdx.y, qb = (int)gridDim.z - 1 - (int)blockIdx.z, tq = qb * 32 + l31;  // (the longest first)
+    const size_t row0 = (size_t)b * P;
+    const int exp_q = exps[PB_Q], exp_k = exps[PB_K], exp_v = exps[PB_V];
+    // (the descriptors end behind key P - 1: later keys read as zero)
+    const size_t kv_base = (size_t)b * kv.stride_b + (size_t)h * kv.stride_h;
+    const unsigned kv_bytes = (unsigned)(P - 1) * kv.stride_t + 256u;
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kv.ksrc + kv_base), 0, kv_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(kv.vsrc + kv_base), 0, kv_bytes, 0x00020000);
+    const unsigned kvo = (unsigned)l31 * kv.stride_t + (unsigned)hl * 32u, vvo = (unsigned)(4 * hl) * kv.stride_t + (unsigned)l31 * 4u;
+    u32x4 kr[8];
+    uint32_t vr[2][2][8];  // [16 keys][d, d + 32][key of the fragment]
+    auto load_k = [&](int kt) {
+        const unsigned so = (unsigned)kt * 32u * kv.stride_t;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const float* r = pp + (s < n ? s : 0) * 66;
-            ml[s] = *reinterpret_cast<const float2*>(r + 64);
-            a[s] = *reinterpret_cast<const float2*>(r + d);
-            c[s] = *reinterpret_cast<const float2*>(r + d + 2);
-        }
+        for (int i = 0; i < 8; ++i) kr[i] = __builtin_amdgcn_raw_buffer_load_b128(rk, kvo + 64u * (i >> 1) + 16u * (i & 1), so, 0);
+    };
+    auto load_v = [&](int kt) {
 #pragma unroll
-        for (int s = 0; s < 8; ++s) m = s < n ? fmaxf(m, ml[s].x) : m;
+        for (int sp = 0; sp < 2; ++sp)
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const float w = s < n ? __builtin_amdgcn_exp2f(ml[s].x - m) : 0.0f;
-            l += w * ml[s].y;
-            o.x += w * a[s].x; o.y += w * a[s].y; o.z += w * c[s].x; o.w += w * c[s].y;
-        }
-    } else {
-        for (int s = 0; s < n; ++s) m = fmaxf(m, pp[s * 66 + 64]);
-        for (int s = 0; s < n; ++s) {
-            const float w = __builtin_amdgcn_exp2f(pp[s * 66 + 64] - m);
-            l += w * pp[s * 66 + 65];
-            const float2 a = *reinterpret_cast<const float2*>(pp + s * 66 + d), c = *reinterpret_cast<const float2*>(pp + s * 66 + d + 2);
-            o.x += w * a.x; o.y += w * a.y; o.z += w * c.x; o.w += w * c.y;
-        }
+            for (int j = 0; j < 8; ++j) {
+                const unsigned so = (unsigned)(kt * 32 + 16 * sp + (j & 3) + 8 * (j >> 2)) * kv.stride_t;
+#pragma unroll
+                for (int dh = 0; dh < 2; ++dh) vr[sp][dh][j] = __builtin_amdgcn_raw_buffer_load_b32(rv, vvo + 128u * dh, so, 0);
+            }
+    };
+    f32x4 qr[8];
+    {
+        const float* qp = qkv + (row0 + min(tq, P - 1)) * 3 * E + h * 64 + hl * 8;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) qr[i] = *reinterpret_cast<const f32x4*>(qp + 16 * (i >> 1) + 4 * (i & 1));
     }
-    const float inv = 1.0f / l;
-    store_split4(out + ((size_t)b * P + q) * kPair * E + h * 64 + d, E, f32x4{o.x * inv, o.y * inv, o.z * inv, o.w * inv}, 0, coarse);
+    load_k(min(wave, qb));
+    load_v(min(wave, qb));
+    const float s_back = ldexpf(1.0f, exp_q + exp_k), k_up = ldexpf(1.0f, -exp_k), v_up = ldexpf(1.0f, -exp_v), q_up = ldexpf(0.125f * kLog2e, -exp_q);
+    // eight values times a power of two -> their two planes
+    auto planes = [](const float(&x)[8], float up, f16x8(&to)[kPair]) {
+        uint32_t w[4][kPair];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) split2_f16(x[2 * e] * up, x[2 * e + 1] * up, w[e][0], w[e][1]);
+#pragma unroll
+        for (int p = 0; p < kPair; ++p) to[p] = frag(w[0][p], w[1][p], w[2][p], w[3][p]);
+    };
+    f16x8 qf[4][kPair];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const f32x4 a = qr[2 * ks], c = qr[2 * ks + 1];
+        const float x[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+        planes(x, q_up, qf[ks]);
+    }
+    constexpr int PK[3] = {1, 0, 0}, PQ[3] = {0, 1, 0};  // the plane pairs, smallest first
+    f32x16 o0, o1;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
+    float mrun = -INFINITY, lrun = 0.0f;
+    for (int kt = wave; kt <= qb; kt += kBlockWaves) {
+        f32x16 sc;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sc[r] = 0.0f;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const f32x4 a = __builtin_bit_cast(f32x4, kr[2 * ks]), c = __builtin_bit_cast(f32x4, kr[2 * ks + 1]);
+            const float x[8] = {a.x, a.y, a.z, a.w, c.x, c.y, c.z, c.w};
+            f16x8 kf[kPair];
+            planes(x, k_up, kf);
+#pragma unroll
+            for (int t = 0; t < 3; ++t) sc = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[PK[t]], qf[ks][PQ[t]], sc, 0, 0, 0);
+        }
+        if (kt + kBlockWaves <= qb) load_k(kt + kBlockWaves);
+        if (kt == qb) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = kt * 32 + (r & 3) + 8 * (r >> 2) + 4 * hl <= tq ? sc[r] : -INFINITY;
+        }
+        float mx = sc[0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
+        mx = both_halves_max(mx);
+        if (__builtin_amdgcn_ballot_w64(mx * s_back > mrun + kDefer) != 0) {
+            const float mnew = fmaxf(mrun, mx * s_back);
+            const float corr = mnew == -INFINITY ? 1.0f : __builtin_amdgcn_exp2f(mrun - mnew);
+            lrun *= corr;
+            mrun = mnew;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o0[r] *= corr;
+                o1[r] *= corr;
+            }
+        }
+        const float mref = kProbUp - fmaxf(mrun, -1e30f);
+        float psum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            sc[r] = __builtin_amdgcn_exp2f(fmaf(sc[r], s_back, mref));
+            psum += sc[r];
+        }
+        lrun += both_halves_sum(psum);
+#pragma unroll
+        for (int sp = 0; sp < 2; ++sp) {
+            f16x8 pf[kPair], vf[2][kPair];
+            float x[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[j] = sc[8 * sp + j];
+            planes(x, 1.0f, pf);
+#pragma unroll
+            for (int dh = 0; dh < 2; ++dh) {
+#pragma unroll
+                for (int j = 0; j < 8; ++j) x[j] = __uint_as_float(vr[sp][dh][j]);
+                planes(x, v_up, vf[dh]);
+            }
+#pragma unroll
+            for (int t = 0; t < 3; ++t) {
+                o0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[0][PK[t]], pf[PQ[t]], o0, 0, 0, 0);
+                o1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[1][PK[t]], pf[PQ[t]], o1, 0, 0, 0);
+            }
+        }
+        if (kt + kBlockWaves <= qb) load_v(kt + kBlockWaves);
+    }
+    // O^T: the lane holds d = (r & 3) + 8 (r >> 2) + 4 hl (+ 32 in o1) of its query.  (a wave without a tile: m = -inf, nothing else)
+    float* mine = s_part + (wave * 32 + l31) * PITCH + 4 * hl;
+#pragma unroll
+    for (int gq = 0; gq < 4; ++gq) {
+        *reinterpret_cast<f32x4*>(mine + 8 * gq) = f32x4{o0[gq * 4], o0[gq * 4 + 1], o0[gq * 4 + 2], o0[gq * 4 + 3]};
+        *reinterpret_cast<f32x4*>(mine + 32 + 8 * gq) = f32x4{o1[gq * 4], o1[gq * 4 + 1], o1[gq * 4 + 2], o1[gq * 4 + 3]};
+    }
+    if (hl == 0) {
+        s_m[wave * 32 + l31] = mrun;
+        s_l[wave * 32 + l31] = lrun;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < 8 / kBlockWaves; ++it) {
+        const int q = it * 4 * kBlockWaves + (tid >> 4), d = (tid & 15) * 4, t = qb * 32 + q;
+        float m = s_m[q], l = 0.0f;
+#pragma unroll
+        for (int w = 1; w < kBlockWaves; ++w) m = fmaxf(m, s_m[w * 32 + q]);
+        f32x4 o = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < kBlockWaves; ++w) {
+            const float c = __builtin_amdgcn_exp2f(s_m[w * 32 + q] - m);
+            l = fmaf(c, s_l[w * 32 + q], l);
+            o += *reinterpret_cast<const f32x4*>(s_part + (w * 32 + q) * PITCH + d) * c;
+        }
+        if (t < P) store_split4(out + (row0 + t) * kPair * E + h * 64 + d, E, o * (1.0f / l), 0, coarse);
+    }
 }
 
 }  // namespace
 
-// out[M][kPair E] = planes of (causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t).  ws: fp32
-// workspace for the partials of split key ranges (B H P max_splits 66 floats; none needed when every group runs as one range).
+// out[M][kPair E] = planes of (causal attention of the q / k / v columns of qkv[M][3E]), M = B P rows ordered (b, t).
 // k_cache / v_cache != null: K and V come from the head-major fp32 caches [b][h][ctx][64] (positions 0 .. P - 1 just appended
-// by the c_attn epilogue) instead of the k / v columns of qkv.
-int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache,
-                        const float* v_cache, int ctx, const int* exps, int coarse, hipStream_t s, int force_tiles) {
-    static bool raised = false;
-    if (!raised) {
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_prefill_pl_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, kLds));
-        raised = true;
-    }
+// by the c_attn epilogue) instead of the k / v columns of qkv.  by_groups (test hook): groups of 128 queries at any size.  stamps: diagnostic builds.
+int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, const float* k_cache, const float* v_cache, int ctx, const int* exps, int coarse,
+                        hipStream_t s, bool by_groups, unsigned long long* stamps) {
     ZG_REQUIRE(E == H * 64, ZG_ERR_UNSUPPORTED, "attention prefill: head_dim must be 64 (n_embed %d, %d heads)", E, H);
     const int nqb = (P + 31) / 32, ng = (nqb + 3) / 4;
-    // key tiles per workgroup: whole rows once there is a group per CU (measured at 12 heads x 1023 tokens, tools/bench_attn_prefill.py:
-    // 4 / 5 sequences = 384 / 480 groups run 57 / 66 us whole against 62 / 75 us cut in two with the merge kernel behind; 3 sequences
-    // are even, 2 are faster cut), else ranges of >= 4 tiles chosen so that the launch fills the chip about twice (2 workgroups fit a
-    // CU) — as long as the partials fit the workspace
-    int nts = 32 * ((nqb + 31) / 32);
-    {
-        const long groups = (long)B * H * ng;
-        if (force_tiles > 0) nts = force_tiles;
-        else
-            for (int cand = nts; cand >= 4; cand /= 2) {
-                long wgs = 0;
-                for (int g = 0; g < ng; ++g) wgs += group_splits(g, nqb, cand);
-                nts = cand;
-                if (wgs * B * H >= 512 || groups >= 256) break;
-            }
-        if (nts > 255) nts = 255;
-    }
-    int max_s = group_splits(ng - 1, nqb, nts);
-    if (max_s > 1 && (ws == nullptr || (size_t)B * H * P * max_s * 66 > ws_floats)) {  // no room for partials: whole rows
-        nts = nqb < 255 ? nqb : 255;
-        max_s = group_splits(ng - 1, nqb, nts);
-        ZG_REQUIRE(max_s == 1, ZG_ERR_UNSUPPORTED, "attention prefill: %d positions without a workspace", P);
-    }
-    ZG_REQUIRE(ng < 65536 && max_s < 256, ZG_ERR_UNSUPPORTED, "attention prefill: %d positions", P);
-    const unsigned geo = (unsigned)nts | ((unsigned)max_s << 8) | ((unsigned)ng << 16);
+    ZG_REQUIRE(nqb < 65536, ZG_ERR_UNSUPPORTED, "attention prefill: %d positions", P);
     AttnKv kv;
     if (k_cache != nullptr) {  // head-major fp32 caches [b][h][ctx][64]
         kv = AttnKv{reinterpret_cast<const char*>(k_cache), reinterpret_cast<const char*>(v_cache), (size_t)H * ctx * 256, (size_t)ctx * 256, 256u};
@@ -452,13 +510,13 @@ int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, in
         kv = AttnKv{reinterpret_cast<const char*>(qkv + E), reinterpret_cast<const char*>(qkv + 2 * E), (size_t)P * 3 * E * 4, (size_t)256, (unsigned)(3 * E * 4)};
     }
     ZG_REQUIRE((size_t)P * kv.stride_t < ((size_t)1 << 31), ZG_ERR_SHAPE, "attention prefill: rows beyond a 32-bit buffer descriptor");
-    hipLaunchKernelGGL(attn_prefill_pl_kernel, dim3(H, B, ng * max_s), dim3(256), kLds, s, qkv, out, ws, P, E, geo, kv, exps, coarse);
+    // Groups of 128 queries once there is one for every compute unit; below, blocks of 32.  us, 12 heads, groups : blocks: 8 x 300 (288 groups)
+    // 18.1 : 18.6, 3 x 1023 (288) 39 : 40, 8 x 500 (384) 27 : 33; 25 heads 2 x 700 (300) 29 : 32.  240 groups of 4 x 600 31 : 26.
+    if (!by_groups && (long)B * H * ng < 256)
+        attn_prefill_block_kernel<<<dim3(H, B, nqb), kBlockWaves * 64, 0, s>>>(qkv, out, P, E, kv, exps, coarse);
+    else
+        attn_prefill_pl_kernel<<<dim3(H, B, ng), 256, kLds, s>>>(qkv, out, P, E, kv, exps, coarse, stamps);
     ZG_HIP(hipGetLastError());
-    if (max_s > 1) {
-        const size_t n = (size_t)B * H * P * 16;
-        hipLaunchKernelGGL(attn_prefill_merge_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, ws, out, P, E, H, B, geo, coarse);
-        ZG_HIP(hipGetLastError());
-    }
     return ZG_OK;
 }
 

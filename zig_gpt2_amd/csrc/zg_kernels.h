@@ -321,10 +321,9 @@ size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp);
 int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s);
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
 // out[M][kPair E] = planes of the causal attention of the q / k / v columns of qkv[M][3E], M = B P rows ordered (b, t)
-// (attn_prefill.hip: matrix cores on two-term fp16 planes; ws = fp32 workspace for the partials of split key ranges).  exps: kBounds of them; the output
-// has v's (a weighted mean of rows of v is no larger than they are).
-int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, float* ws, size_t ws_floats, const float* k_cache_or_null,
-                        const float* v_cache_or_null, int ctx, const int* exps, int coarse, hipStream_t s, int force_tiles = 0);  // force_tiles: key tiles per workgroup (tests)
+// (attn_prefill.hip: matrix cores on two-term fp16 planes).  exps: kBounds of them; the output has v's (a weighted mean of rows of v is no larger than they are).
+int launch_attn_prefill(const float* qkv, uint16_t* out, int B, int P, int E, int H, const float* k_cache_or_null, const float* v_cache_or_null, int ctx, const int* exps,
+                        int coarse, hipStream_t s, bool by_groups = false, unsigned long long* stamps = nullptr);
 
 // GPT.sample tail: in-place softmax(logits / temp) per sequence + inverse-CDF draw with uniform u[b].
 // part_val / n_part / part_stride: the per-workgroup maxima lm_head's argmax epilogue left (the row maximum without a pass over the
