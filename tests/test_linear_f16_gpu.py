@@ -65,9 +65,10 @@ def test_tile_edges(zg, m, k, n):
 
 
 @pytest.mark.parametrize("m,k,n,ring", [(700, 1600, 1600, 1), (700, 1600, 1603, 1), (321, 1600, 4800, 1), (1023, 3072, 769, 1), (700, 3072, 768, 1), (65, 6400, 9601, 1),
-                                        (450, 6400, 1600, 1), (2049, 1536, 1031, 1), (700, 1472, 1600, 0), (128, 1600, 1600, 0), (3000, 1600, 4800, 0)])
+                                        (450, 6400, 1600, 1), (2049, 1536, 1031, 1), (1501, 1600, 1600, 1), (1409, 1600, 1667, 1), (1500, 3072, 768, 1),
+                                        (2047, 6400, 1600, 1), (700, 1472, 1600, 0), (128, 1600, 1600, 0), (3000, 1600, 4800, 0)])
 def test_some_hundred_rows(zg, m, k, n, ring):
-    """Tiles of 64 and 128 rows, one slice of K and several, widths in no whole tiles and no whole fours, both sides of the rule."""
+    """Tiles of 64 and 128 rows, of 64 and 128 columns, one slice of K and several, widths in no whole tiles and no whole fours, both sides of the rule."""
     x, w, b = draw(m, k, n, spread=9)
     b = None if n % 2 else b * 0.125
     before = zg.zg_debug_linear_ring_launches()
@@ -76,7 +77,7 @@ def test_some_hundred_rows(zg, m, k, n, ring):
     check(x, w, b, y)
 
 
-@pytest.mark.parametrize("m,k,n", [(700, 1600, 1600), (700, 3072, 769)])  # one slice, several
+@pytest.mark.parametrize("m,k,n", [(700, 1600, 1600), (700, 3072, 769), (1501, 1600, 1600)])  # one slice, several; tiles of 128 columns
 def test_values_that_are_not_finite_among_some_hundred_rows(zg, m, k, n):
     """Outputs are what a plain sum makes of them: infinities stay infinities of their sign."""
     x, w, b = draw(m, k, n)

@@ -54,6 +54,26 @@ def test_weights_of_very_different_sizes(zg, name, batch, n, bf16, route):
     m.close()
 
 
+@pytest.mark.parametrize("batch,n", [(8, 250), (5, 255)])
+def test_tiles_of_128_columns(zg, batch, n):
+    """fp32 weights and one to two thousand rows: the ring kernel's 128 x 128 tiles (qkv with the cache append, GELU, slabs) against the persistent GEMM.
+    Both are within some 5e-7 of the exact logits, in the 2-norm."""
+    cfg = synth.CONFIGS["nano-char"]
+    m = zgpt.GPT(cfg, batch=batch, weights_f32=True)
+    m.load_weights(synth.make_weights(cfg, seed=64, bf16=False))
+    toks = np.stack([synth.rand_tokens(640 + b, n + 1, cfg.vocab_size) for b in range(batch)])
+    got = []
+    for route in (0, 1):
+        zg.zg_debug_prefill_route(route, 0)
+        try:
+            lg = m.prefill(toks[:, :n]).copy()
+        finally:
+            zg.zg_debug_prefill_route(0, 0)
+        got.append(np.concatenate([lg, m.forward(n + 1, toks[:, n])]).astype(np.float64))
+    m.close()
+    assert np.linalg.norm(got[0] - got[1]) <= 2e-6 * np.linalg.norm(got[1])
+
+
 def test_a_tensor_loaded_again(zg):
     cfg = synth.CONFIGS["tiny3"]
     toks = synth.rand_tokens(62, 40, cfg.vocab_size)

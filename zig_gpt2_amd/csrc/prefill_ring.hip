@@ -8,7 +8,10 @@
 // products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
 // K steps; a step costs one barrier; its fragments were read beside the products of the step before.  The leading products of a step are a sum
 // of their own, added to the steps' before it beside the products of the next, so that neither they nor the small ones are rounded at the size of
-// the whole.
+// the whole.  Tiles of 128 x 128 (fp32 weights, some thousand rows) stage 64 KB for what four tiles of 64 x 64 stage 128 KB for; their leading
+// products are a sum of four steps (a second set has no registers), and what the epilogue needs is fetched behind the products.  us, 768 columns,
+// 128 x 64 : 128 x 128: 1000 x 3072 33 : 28, 1500 x 2304 37 : 30; 3072 columns 1500 x 768 in slices, with the reduction 53 : 39; 2000 x 2304 (two rounds
+// for three) 50 : 53.  With one plane of a bf16 weight they are no faster than the 128-row kernel of prefill.hip (1000 x 3072 22 : 21): not built.
 #include <algorithm>
 #include <atomic>
 #include <type_traits>
@@ -46,17 +49,17 @@ struct RawRows {
     const float *x, *w;
 };
 
-// 2 x 2 waves of TM x 1 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
-template <int EPI, int TM, int NW, int ST>
+// 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
+template <int EPI, int TM, int TN, int NW, int ST>
 __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
                                                               const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw) {
-    constexpr int BM = 64 * TM, BN = 64, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
+    constexpr int BM = 64 * TM, BN = 64 * TN, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
     constexpr int REQ = kPair * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
     extern __shared__ __attribute__((aligned(1024))) char s_ring[];
     const unsigned lds0 = (unsigned)(unsigned long)(lds_at_t)s_ring;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), wy = wave >> 1, wx = wave & 1;
     // workgroups go round the eight XCDs: each gets a run of the tiles, row tiles of a column tile next to each other (the weights are read once)
-    const int tiles_m = (M + BM - 1) / BM, n_tiles = tiles_m * (N / BN), q8 = n_tiles >> 3, r8 = n_tiles & 7, xcd = blockIdx.x & 7;
+    const int tiles_m = (M + BM - 1) / BM, n_tiles = tiles_m * ((N + BN - 1) / BN), q8 = n_tiles >> 3, r8 = n_tiles & 7, xcd = blockIdx.x & 7;
     const int tile = xcd * q8 + min(xcd, r8) + (int)(blockIdx.x >> 3);
     const int m0 = (tile % tiles_m) * BM, n0 = (tile / tiles_m) * BN;
     const int in_row = lane >> 3, chunk = (lane & 7) ^ in_row;  // (every eighth row the swizzle repeats)
@@ -65,7 +68,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
     for (int i = 0; i < PA; ++i) va[i] = (unsigned)min(m0 + (wave + 4 * i) * 8 + in_row, M - 1) * (unsigned)(kPair * K) * 2u + chunk * 16u;  // (rows beyond the edge: never stored)
 #pragma unroll
-    for (int i = 0; i < PB; ++i) vb[i] = (unsigned)(n0 + (wave + 4 * i) * 8 + in_row) * (unsigned)K * 2u + chunk * 16u;
+    for (int i = 0; i < PB; ++i) vb[i] = (unsigned)(TN == 1 ? n0 + (wave + 4 * i) * 8 + in_row : min(n0 + (wave + 4 * i) * 8 + in_row, N - 1)) * (unsigned)K * 2u + chunk * 16u;
     const int nk = K / kBk, t0 = nk * (int)blockIdx.y / n_sp, steps = nk * ((int)blockIdx.y + 1) / n_sp - t0;
     auto request = [&](int slot, int s) {
         const unsigned off = (unsigned)(t0 + min(s, steps - 1)) * kRow, to = lds0 + slot * SLOT + wave * 1024;
@@ -78,20 +81,25 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < PB; ++i) dma_16(to + kPair * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
     };
-    f32x16 lead[2][TM], small[TM], total[TM];  // leading products by the step's parity
+    constexpr int NL = TN == 2 ? 1 : 2;  // leading products by the step's parity, or (registers) one sum of four steps
+    f32x16 lead[NL][TM][TN], small[TM][TN], total[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int e = 0; e < 16; ++e) lead[0][i][e] = lead[1][i][e] = small[i][e] = total[i][e] = 0.0f;
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) lead[0][i][j][e] = lead[NL - 1][i][j][e] = small[i][j][e] = total[i][j][e] = 0.0f;
     const int fr = lane & 31, kh = lane >> 5, fswz = fr & 7;
-    u32x4 af[2][kCh / 2][kPair][TM], bf[2][kCh / 2][NW];  // of the step that is multiplied, and of the one behind it on its way
+    u32x4 af[2][kCh / 2][kPair][TM], bf[2][kCh / 2][NW][TN];  // of the step that is multiplied, and of the one behind it on its way
     auto read = [&](auto b, int slot) {
         const char* base = s_ring + slot * SLOT;
 #pragma unroll
         for (int kk = 0; kk < kCh / 2; ++kk) {
             const int c = ((2 * kk + kh) ^ fswz) * 16;
 #pragma unroll
-            for (int p = 0; p < NW; ++p) bf[b][kk][p] = *reinterpret_cast<const u32x4*>(base + kPair * A_PLANE + p * B_PLANE + (wx * 32 + fr) * kRow + c);
+            for (int p = 0; p < NW; ++p)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) bf[b][kk][p][j] = *reinterpret_cast<const u32x4*>(base + kPair * A_PLANE + p * B_PLANE + ((wx * TN + j) * 32 + fr) * kRow + c);
 #pragma unroll
             for (int p = 0; p < kPair; ++p)
 #pragma unroll
@@ -100,40 +108,55 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     };
     // (the operands change places: an accumulator's registers are then runs of four columns of a row)
     auto multiply = [&](auto b) {
-        auto one = [&](f32x16& acc, int kk, int pa, int pw, int i) {
-            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bf[b][kk][pw]), __builtin_bit_cast(f16x8, af[b][kk][pa][i]), acc, 0, 0, 0);
+        auto one = [&](f32x16& acc, int kk, int pa, int pw, int i, int j) {
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, bf[b][kk][pw][j]), __builtin_bit_cast(f16x8, af[b][kk][pa][i]), acc, 0, 0, 0);
         };
+        constexpr int now = NL == 2 ? (int)decltype(b)::value : 0;
+        if constexpr (NL == 2)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) {
-            total[i] += lead[1 - b][i];
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) lead[1 - b][i][e] = 0.0f;
-        }
+                for (int j = 0; j < TN; ++j) {
+                    total[i][j] += lead[1 - now][i][j];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) lead[1 - now][i][j][e] = 0.0f;
+                }
 #pragma unroll
         for (int kk = 0; kk < kCh / 2; ++kk)
 #pragma unroll
-            for (int i = 0; i < TM; ++i) {
-                one(small[i], kk, 1, 0, i);
-                one(lead[b][i], kk, 0, 0, i);
-                if constexpr (NW == 2) one(small[i], kk, 0, 1, i);
-            }
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    one(small[i][j], kk, 1, 0, i, j);
+                    one(lead[now][i][j], kk, 0, 0, i, j);
+                    if constexpr (NW == 2) one(small[i][j], kk, 0, 1, i, j);
+                }
     };
     // what the epilogue needs besides the sums, on its way before the requests
-    const int cc = (lane & 7) * 4, n = n0 + wx * 32 + cc;
-    const i32x4 col_exp = *reinterpret_cast<const i32x4*>(ex.w + n);
-    f32x4 bv = {0.0f, 0.0f, 0.0f, 0.0f};
-    if (EPI == PF_LINEAR) {
-        if (bias)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) bv[e] = bias[min(n + e, ldc - 1)];
-    } else if (EPI != PF_PARTIAL && bias) {
-        bv = *reinterpret_cast<const f32x4*>(bias + n);
-    }
+    const int cc = (lane & 7) * 4, n_w = n0 + wx * TN * 32 + cc;
+    i32x4 col_exp[TN];
+    f32x4 bv[TN];
     int row_exp[TM][4];
+    auto fetch_scales = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+        for (int j = 0; j < TN; ++j) {
+            const int n = TN == 1 ? n_w : min(n_w + 32 * j, N - 4);  // (N: whole pieces of 32)
+            col_exp[j] = *reinterpret_cast<const i32x4*>(ex.w + n);
+            bv[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            if (EPI == PF_LINEAR) {
+                if (bias)
 #pragma unroll
-        for (int r8i = 0; r8i < 4; ++r8i) row_exp[i][r8i] = ex.a[ex.a_each ? min(m0 + (wy * TM + i) * 32 + 8 * r8i + (lane >> 3), M - 1) : 0];
+                    for (int e = 0; e < 4; ++e) bv[j][e] = bias[min(n + e, ldc - 1)];
+            } else if (EPI != PF_PARTIAL && bias) {
+                bv[j] = *reinterpret_cast<const f32x4*>(bias + n);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int r8i = 0; r8i < 4; ++r8i) row_exp[i][r8i] = ex.a[ex.a_each ? min(m0 + (wy * TM + i) * 32 + 8 * r8i + (lane >> 3), M - 1) : 0];
+    };
+    if (TN == 1) fetch_scales();  // (larger tiles have no registers for them beside the products)
     const int out_exp = EPI == PF_GELU_SPLIT ? *po.exp : 0;
 #pragma unroll
     for (int s = 0; s < ST; ++s) request(s, s);
@@ -153,13 +176,22 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
         __builtin_amdgcn_sched_barrier(0);
         read(std::integral_constant<int, other>(), slot);
         multiply(b);
-        constexpr int products = kCh / 2 * TM * (NW + 1), reads = kCh / 2 * (kPair * TM + NW);
+        constexpr int products = kCh / 2 * TM * TN * (NW + 1), reads = kCh / 2 * (kPair * TM + NW * TN);
 #pragma unroll
         for (int x = 0; x < products; ++x) {
             __builtin_amdgcn_sched_group_barrier(0x100, (reads + products - 1) / products, 0);
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
+        if (NL == 1 && other == 0 && (s & 2))
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    total[i][j] += lead[0][i][j];
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) lead[0][i][j][e] = 0.0f;
+                }
         ++s;
     };
     for (int pairs = steps >> 1; pairs > 0; --pairs) {
@@ -168,6 +200,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     }
     if (steps & 1) body(std::integral_constant<int, 0>());
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the requests behind the last step still write the ring)
+    if (TN > 1) fetch_scales();
 
     // element e of a 32 x 32 tile: column 8 (e / 4) + 4 (lane / 32) + e % 4, row lane % 32.  Every wave turns its rows in an image of its own
     // (its accesses to the LDS are in order), so that eight lanes store 128 bytes of a row.
@@ -175,12 +208,14 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     static_assert(4 * 32 * PITCH <= SLOT, "the images fit the ring");
     char* img = s_ring + wave * 32 * PITCH;
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int ij = 0; ij < TM * TN; ++ij) {
+        const int i = ij / TN, j = ij % TN, n = n_w + 32 * j;
+        if (TN > 1 && n >= N) continue;
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             f32x4 v;  // (of the two leading sums one is in the total already, and zero)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = (total[i][4 * g + e] + (lead[0][i][4 * g + e] + lead[1][i][4 * g + e])) + small[i][4 * g + e];
+            for (int e = 0; e < 4; ++e) v[e] = (total[i][j][4 * g + e] + (NL == 2 ? lead[0][i][j][4 * g + e] + lead[NL - 1][i][j][4 * g + e] : lead[0][i][j][4 * g + e])) + small[i][j][4 * g + e];
             *reinterpret_cast<f32x4*>(img + fr * PITCH + (8 * g + 4 * kh) * 4) = v;
         }
 #pragma unroll
@@ -189,7 +224,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
             f32x4 v = *reinterpret_cast<const f32x4*>(img + r * PITCH + cc * 4);
             if (m >= M) continue;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], row_exp[i][r8i] + col_exp[e]) + bv[e];
+            for (int e = 0; e < 4; ++e) v[e] = ldexpf(v[e], row_exp[i][r8i] + col_exp[j][e]) + bv[j][e];
             if constexpr (EPI == PF_GELU_SPLIT) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[e] = gelu_fast(v[e]);
@@ -206,7 +241,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
                 if (odd(v[0]) + odd(v[1]) + odd(v[2]) + odd(v[3]) > 0.0f)
 #pragma unroll 1
                     for (int e = 0; e < 4; ++e)
-                        if (n + e < ldc && odd(v[e]) > 0.0f) y[e] = plain_sum(raw.x + (size_t)m * K, raw.w + (size_t)(n + e) * K, K) + bv[e];
+                        if (n + e < ldc && odd(v[e]) > 0.0f) y[e] = plain_sum(raw.x + (size_t)m * K, raw.w + (size_t)(n + e) * K, K) + bv[j][e];
             } else if constexpr (EPI == PF_PARTIAL) {  // C: slabs [n_sp][M][N]
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)blockIdx.y * M + m) * N + n) = v;
             } else {
@@ -217,20 +252,20 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     }
 }
 
-template <int EPI, int TM, int NW, int ST>
+template <int EPI, int TM, int TN, int NW, int ST>
 int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s,
                 const RawRows& raw = RawRows{}) {
-    constexpr int LDS = ST * (kPair * 64 * TM + NW * 64) * kRow;
+    constexpr int LDS = ST * (kPair * 64 * TM + NW * 64 * TN) * kRow;
     static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
     static OncePerDevice raised;
     int device = 0;
     ZG_HIP(hipGetDevice(&device));
     ZG_TRY(raised.run(device, []() -> int {
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_ring_kernel<EPI, TM, NW, ST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_ring_kernel<EPI, TM, TN, NW, ST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         return ZG_OK;
     }));
-    const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * (N / 64);
-    prefill_ring_kernel<EPI, TM, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
+    const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * ((N + 64 * TN - 1) / (64 * TN));
+    prefill_ring_kernel<EPI, TM, TN, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -240,8 +275,10 @@ template <int EPI>
 int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int tm, int n_sp, const PrefillQkv& qa, const PlaneOut& po,
                     hipStream_t s) {
     if (W.planes == 2)
-        return tm == 1 ? launch_ring<EPI, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
-    return tm == 1 ? launch_ring<EPI, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
+               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
+                         : launch_ring<EPI, 2, 2, 2, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+    return tm == 1 ? launch_ring<EPI, 1, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
 }
 
 // the slabs [n_sp][M][Np] of a Linear added, and its bias: a thread four columns of a row
@@ -276,6 +313,10 @@ __global__ __launch_bounds__(256) void linear_ring_finish_kernel(const float* __
 namespace {
 size_t whole(size_t bytes) { return (bytes + 255) & ~(size_t)255; }
 size_t whole64(size_t n) { return (n + 63) / 64 * 64; }
+// tiles of form t: 64 x 64, 128 x 64, 128 x 128
+long ring_tiles(long M, long N, int t) { return (M + (t == 1 ? 63 : 127)) / (t == 1 ? 64 : 128) * ((N + (t == 3 ? 127 : 63)) / (t == 3 ? 128 : 64)); }
+// us of a K step of two weight planes, by form.  A round of workgroups costs 4.5 us besides: 768 columns in one round 11.7, 17 and 27.
+constexpr double kStepUs[4] = {0.0, 0.55, 1.02, 1.85};
 }  // namespace
 
 size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp) {
@@ -288,7 +329,7 @@ unsigned long long linear_ring_launch_count() { return g_linear_ring_launches.lo
 
 int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s) {
     const int Np = (int)whole64(N);
-    ZG_REQUIRE(M > 0 && N > 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (tm == 1 || tm == 2) && (size_t)M * K * 4 < ((size_t)1 << 31) && (size_t)Np * K * 4 < ((size_t)1 << 31),
+    ZG_REQUIRE(M > 0 && N > 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && tm >= 1 && tm <= 3 && (size_t)M * K * 4 < ((size_t)1 << 31) && (size_t)Np * K * 4 < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "linear: %d x %d x %d", M, N, K);
     uint16_t *xp = reinterpret_cast<uint16_t*>(scratch), *wp = reinterpret_cast<uint16_t*>(scratch += whole((size_t)M * K * 4));
     int *xe = reinterpret_cast<int*>(scratch += whole((size_t)Np * K * 4)), *we = reinterpret_cast<int*>(scratch += whole((size_t)M * 4));
@@ -301,8 +342,9 @@ int launch_linear_ring(const float* X, const float* W, const float* bias, float*
     if (n_sp == 1) {
         const PrefillQkv none{};
         const RawRows raw{X, W};
-        ZG_TRY(tm == 1 ? (launch_ring<PF_LINEAR, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
-                       : (launch_ring<PF_LINEAR, 2, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw)));
+        ZG_TRY(tm == 1   ? (launch_ring<PF_LINEAR, 1, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
+               : tm == 2 ? (launch_ring<PF_LINEAR, 2, 1, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
+                         : (launch_ring<PF_LINEAR, 2, 2, 2, 2>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw)));
         note_kernel("linear_tiles_kernel");  // (the Linears of a medium number of rows have one name; the count says which)
         return ZG_OK;
     }
@@ -316,21 +358,22 @@ int launch_linear_ring(const float* X, const float* W, const float* bias, float*
 
 // Priced in us like the prompts' Linears below, with 3 for the launch that adds slabs.  It takes a Linear of 1536 columns and more where the kernel that splits in its own staging
 // has few slices of K to add up, whose chains are then so long that this kernel is closer to 64 bits as well (1600 columns in two slices 1.67e-7, here
-// 1.38e-7; 3072 in four 1.66e-7 and 1.63e-7; 768 in two 1.16e-7 and 1.22e-7), and where it is cheap beside the persistent one (rounds of 256 x 192 tiles).  us of a call
-// with it : without: 3072 -> 768 700 rows 42 : 50, 2048 73 : 93, 3000 120 : 143; 1600 -> 1600 700 rows 45 : 52, 2048 76 : 110; 1600 -> 4800 256 rows
-// 47 : 53, 700 77 : 110; 6400 -> 1600 400 rows 82 : 107, 2048 241 : 392; not taken: 1600 -> 4800 1500 rows 139 : 119, 768 -> 768 3000 rows 50 : 46.
+// 0.9e-7; 3072 in four 1.66e-7 and 1.2e-7; 768 in two 1.16e-7 and 1.22e-7), and where it is cheap beside the persistent one (rounds of 256 x 192 tiles: one of
+// 1600 columns 90 predicted, 95 measured; beside several rounds here, which are a sixth longer than predicted, 0.85 of that).  us of a call
+// with it : without: 3072 -> 768 700 rows 44 : 50, 2048 74 : 93, 3000 114 : 143; 1600 -> 1600 700 rows 46 : 52, 2048 64 : 110; 1600 -> 4800 256 rows
+// 47 : 53, 700 65 : 110; 6400 -> 1600 400 rows 78 : 107, 2048 190 : 392; not taken: 1600 -> 4800 1500 rows 139 : 119, 768 -> 768 3000 rows 50 : 46.
 int linear_ring_route(size_t M, size_t N, size_t K, int* tm) {
     if (K < 1536 || linear_tiles_slices(M, N, K) > (K < 3072 ? 2 : 4)) return 0;
     const int nk = (int)(K / kBk);
     const double slab = (double)M * (double)whole64(N) * 8.0 / 4e6;
     auto rounds = [](long n) { return (double)((n + 255) / 256); };
     int best = 0;
-    double best_us = rounds((long)((M + 255) / 256 * ((N + 191) / 192))) * (3.2 * nk + 10.0) * 0.75;
-    for (int t = 1; t <= 2; ++t) {
-        const long tiles = (long)((M + 64 * t - 1) / (64 * t)) * (long)((N + 63) / 64);
+    double best_us = rounds((long)((M + 255) / 256 * ((N + 191) / 192))) * (3.2 * nk + 10.0) * 0.85;
+    for (int t = 1; t <= 3; ++t) {
+        const long tiles = ring_tiles((long)M, (long)N, t);
         const long most = std::max(1l, std::min(256 / tiles, (long)nk / 3));
         for (long n = 1; n <= most; ++n) {
-            const double us = rounds(tiles * n) * (3.0 + (double)((nk + n - 1) / n) * (16.0 * t + 16.0) / 57.0) + (n > 1 ? (double)n * slab + 3.0 : 0.0);
+            const double us = rounds(tiles * n) * (4.5 + (double)((nk + n - 1) / n) * kStepUs[t]) + (n > 1 ? (double)n * slab + 3.0 : 0.0);
             if (us < best_us) {
                 best = (int)n;
                 best_us = us;
@@ -342,10 +385,10 @@ int linear_ring_route(size_t M, size_t N, size_t K, int* tm) {
 }
 
 // K slices of the launch (1 unless it is a residual Linear, whose slices meet in slabs) and rows of a tile (64 tm); 0: the 128-row kernels take it.
-// Both sides are priced in us by what one compute unit takes in (65 bytes a ns; 57 with the weight's planes; 42 where two slots of 56 KB are
-// the whole ring), 3 us for each round of workgroups, and slabs at 4 TB/s.  At K = 768, bf16: 300 x 3072 predicts 9 here and 14 there
-// (measured 10.5 and 16.6), 800 x 3072 41 and 15 (31.7, 20.4); K = 3072: 300 x 768 10 and 13 (14.3, 16.1), 800 x 768 28 and 18 (27.6, 24.7);
-// fp32 weights: 300 x 3072 13 and 34 (14.5, 27.5), 1000 x 768 x 3072 36 and 62 (41, 51), 1600 x 768 x 3072 66 and 68 (68.5, 62.8).
+// Both sides are priced in us.  bf16 weights: by what one compute unit takes in (65 bytes a ns), 3 us for each round of workgroups, and slabs at
+// 4 TB/s.  At K = 768: 300 x 3072 predicts 9 here and 14 there (measured 10.5 and 16.6), 800 x 3072 41 and 15 (31.7, 20.4); K = 3072: 300 x 768
+// 10 and 13 (14.3, 16.1), 800 x 768 28 and 18 (27.6, 24.7).  fp32 weights: by the steps of the three tile forms and of the 128-row kernel (1 us for 128 columns):
+// 300 x 3072 11 and 33 (11.8, 27), 1000 x 768 x 3072 27 and 39 (28, 40), 1500 x 3072 x 768 41 and 54 (39, 56), 2000 x 768 x 3072 50 and 58 (52, 66).
 // bf16: beyond a few hundred rows what wins by less than a microsecond is lost again in the reduce kernel behind it, which finds one slab where
 // it found several (a whole prompt of 4 x 200 rows of 768 columns: 1377 us against 1359, 8 x 255 of 384: 600 against 588).
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm) {
@@ -355,12 +398,13 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
     auto rounds = [](long n) { return (double)((n + 255) / 256); };
     int best = 0;
     double best_us = 0.0;
-    for (int t = 1; t <= 2; ++t) {
-        const long tiles = (long)((M + 64 * t - 1) / (64 * t)) * (N / 64);
+    for (int t = 1; t <= (planes ? 3 : 2); ++t) {
+        const long tiles = ring_tiles(M, N, t);
         int n_sp = resid ? (int)std::max(1l, std::min(256 / tiles, (long)nk / 3)) : 1;
         while (resid && n_sp > 1 && (size_t)n_sp * M * N > ws_floats) --n_sp;
         if (resid && (size_t)n_sp * M * N > ws_floats) continue;
-        const double us = rounds(tiles * n_sp) * (3.0 + ((nk + n_sp - 1) / n_sp) * (planes ? (16.0 * t + 16.0) / 57.0 : (16.0 * t + 8.0) / 65.0)) + (resid ? n_sp * slab : 0.0);
+        const double us = (planes ? rounds(tiles * n_sp) * (4.5 + (nk + n_sp - 1) / n_sp * kStepUs[t]) : rounds(tiles * n_sp) * (3.0 + (nk + n_sp - 1) / n_sp * (16.0 * t + 8.0) / 65.0)) +
+                          (resid ? n_sp * slab : 0.0);
         if (best == 0 || us < best_us) {
             best = n_sp;
             best_us = us;
@@ -373,7 +417,7 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
     const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
     const int passes = planes ? 2 : 1;
     const int n_sp = (int)std::max(1l, std::min(planes ? (256 + 2 * tiles - 1) / (2 * tiles) : 256 / tiles, (long)nk / 3));
-    const double us = rounds(tiles * n_sp * passes) * (3.0 + ((nk + n_sp - 1) / n_sp) * (32.0 + bn / 8.0) / 65.0) +
+    const double us = rounds(tiles * n_sp * passes) * (planes ? 4.5 + (nk + n_sp - 1) / n_sp * bn / 128.0 : 3.0 + (nk + n_sp - 1) / n_sp * (32.0 + bn / 8.0) / 65.0) +
                       (resid || n_sp * passes > 1 ? n_sp * passes * slab : 0.0) + (!resid && n_sp * passes > 1 ? 3.0 : 0.0);
     return best_us + (planes || M <= 256 ? 0.0 : 1.0) <= us ? best : 0;
 }
