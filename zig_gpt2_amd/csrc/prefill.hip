@@ -605,13 +605,10 @@ int launch_prefill_gemm_wp(const PrefillA& A, const PrefillW& W, const float* bi
     return finish_slabs<EPI>(ws, 2 * n_sp, bias, C, M, N, ldc, ln, qa, po, s);
 }
 
-// 128 x 256 tiles (the staged weight tile is shared by the planes, so widening N is the cheap direction)
-// once there are enough rows to fill the chip with them, else 128 x 128.
 template <int EPI>
 int launch_prefill_gemm_t(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc,
                           float* ws, size_t ws_floats, const PrefillLn* ln, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s) {
-    const int wide_tiles = ((M + BM - 1) / BM) * ((N + 2 * BN - 1) / (2 * BN));
-    const bool wide = wide_tiles >= 256 && N >= 2 * BN;
+    const bool wide = prefill_rows_wide(M, N, W.planes);
     if (W.planes == 2)
         return wide ? launch_prefill_gemm_wp<EPI, 2>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s)
                     : launch_prefill_gemm_wp<EPI, 1>(A, W, bias, C, M, N, K, ldc, ws, ws_floats, ln, qa, po, s);
@@ -620,6 +617,16 @@ int launch_prefill_gemm_t(const PrefillA& A, const PrefillW& W, const float* bia
 }
 
 }  // namespace
+
+// 128 x 256 tiles (the staged weight tile is shared by the planes, so widening N is the cheap direction) or 128 x 128.  With one plane of a bf16 weight
+// a round of wide ones takes 1.6 to 1.7 times as long: they pay where they save every other round.  us, 128 x 128 : 128 x 256: 768 -> 2304 2000 rows (288 and 144
+// tiles) 42 : 38.7, 768 -> 3072 1500 rows (288) 39.8 : 36.3, 2000 (384) 41.2 : 36.7; 1600 -> 6400 700 rows (300) 62 : 56, 1600 -> 4800 1000 rows (304) 65 : 60; in one
+// round 768 -> 3072 1000 rows (192) 21.4 : 29.7.
+bool prefill_rows_wide(int M, int N, int planes) {
+    const long rows = (M + BM - 1) / BM, wide = rows * ((N + 2 * BN - 1) / (2 * BN)), narrow = rows * ((N + BN - 1) / BN);
+    if (N < 2 * BN) return false;
+    return planes == 2 ? wide >= 256 : 17 * ((wide + 255) / 256) <= 10 * ((narrow + 255) / 256);
+}
 
 int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, const void* wte, const void* wpe,
                          int weight_type, int E, float* x, hipStream_t s) {

@@ -412,7 +412,7 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
         }
     }
     if (best == 0 || force) return best;
-    const bool wide = (long)((M + 127) / 128) * ((N + 255) / 256) >= 256;
+    const bool wide = prefill_rows_wide(M, N, planes ? 2 : 1);
     const int bn = wide ? 256 : 128;
     const long tiles = (long)((M + 127) / 128) * ((N + bn - 1) / bn);
     const int passes = planes ? 2 : 1;

@@ -319,6 +319,7 @@ int linear_ring_route(size_t M, size_t N, size_t K, int* tm);
 unsigned long long linear_ring_launch_count();  // Linears it has taken so far
 size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp);
 int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s);
+bool prefill_rows_wide(int M, int N, int planes);  // the 128-row kernels' tiles: 256 columns for 128
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
 // out[M][kPair E] = planes of the causal attention of the q / k / v columns of qkv[M][3E], M = B P rows ordered (b, t)
 // (attn_prefill.hip: matrix cores on two-term fp16 planes).  exps: kBounds of them; the output has v's (a weighted mean of rows of v is no larger than they are).
