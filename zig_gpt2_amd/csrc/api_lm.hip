@@ -252,6 +252,10 @@ struct zg_lm {
     bf16_t *h16 = nullptr, *hc16 = nullptr, *o16 = nullptr, *u16 = nullptr;
     bf16_t* key_tiles = nullptr;  // cached latents of a portion's entries as bf16 tiles (latent attention of prompt portions)
     size_t key_tile_elems = 0, step_key_tiles = 0;  // its room; tiles the running portion needs
+    char* head_keys = nullptr;  // keys and values of the heads' own of a portion's entries
+    size_t head_key_bytes = 0;
+    bool no_head_keys = false;  // (a device without room for them)
+    PortionSize step_size;
     int step_longest = 0;  // rows of the longest entry of the running portion
     int step_blocks = 0;   // blocks of 32 rows of its entries
     int step_keys = 0;  // positions the longest sequence of the running portion has reached (what its rows can see at most)
@@ -346,7 +350,7 @@ void layout(zg_lm* g, Bump& b) {
     else vec("final.norm", g->final_norm, W, g->side ? INIT_PLAIN : INIT_OFFSET);
     if (g->cfg.flags & ZG_LM_SINUSOID_POSITIONS) g->pos_freq = b.take<float>((W + 1) / 2);
     size_t max_t = 1, max_win = 0, max_win_few = 0, max_vf = 0;
-    size_t max_proj = 1, max_qr = 1, max_q = 1, max_qa = 1, max_ctx = 1, max_o = 1, max_ff = 1, max_assign = 1, max_gu = 1, max_hb = 1, max_e = 1, max_att_part = 0, max_scan = 0, max_tile = 0;
+    size_t max_proj = 1, max_qr = 1, max_q = 1, max_qa = 1, max_ctx = 1, max_o = 1, max_ff = 1, max_assign = 1, max_gu = 1, max_hb = 1, max_e = 1, max_att_part = 0, max_scan = 0, max_tile = 0, max_record = 0;
     for (size_t i = 0; i < g->layers.size(); ++i) {
         LayerW& L = g->layers[i];
         const zg_lm_layer& d = L.d;
@@ -604,6 +608,7 @@ void layout(zg_lm* g, Bump& b) {
             max_ctx = std::max(max_ctx, H * KR);
             max_att_part = std::max(max_att_part, H * (KR + 2));
             if (!g->f32) max_tile = std::max(max_tile, latent_tile_elems((int)KR, (int)R));
+            if (!g->f32) max_record = std::max(max_record, latent_heads_record((int)H, (int)D, (int)R, (int)KR, (int)Vd, (int)d.rot_dims));
             max_o = std::max(max_o, HV);
         }
         if (d.ff != ZG_LM_FF_NONE && tn) {
@@ -759,6 +764,9 @@ void layout(zg_lm* g, Bump& b) {
     g->attn_ws = b.take<float>(std::max<size_t>(1, g->attn_ws_floats));
     g->key_tile_elems = g->lean ? 0 : ((size_t)g->n_pages * g->P / 32 + NS) * max_tile;  // every cached token, a partly filled tile per sequence
     g->key_tiles = g->key_tile_elems > 0 ? b.take<bf16_t>(g->key_tile_elems) : nullptr;
+    // ... and of keys and values per head up to 256 MB (eight full contexts of 1024 tokens and 16 heads: 35); portions that need more take the tiles
+    g->head_key_bytes = g->lean || g->no_head_keys ? 0 : std::min<size_t>(((size_t)g->n_pages * g->P / 32 + NS) * max_record, (size_t)256 << 20);
+    g->head_keys = g->head_key_bytes > 0 ? b.take<char>(g->head_key_bytes) : nullptr;
     // scores and partial sums of the split windowed attention: up to 2 GiB for a whole portion, else for steps of few rows only
     // (longer steps of such a model then take the general kernel)
     if (max_win > ((size_t)1 << 29)) max_win = 0;
@@ -1416,9 +1424,16 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             bf16_t* const cq16 = r16 && whole(QR) ? reinterpret_cast<bf16_t*>(g->cq) : nullptr;
             bf16_t* const qa16 = tiles && whole(KR) && whole(R) && whole(D) && (direct ? LD % 4 == 0 : true) && whole(D + R) ? reinterpret_cast<bf16_t*>(g->qa) : nullptr;
             bf16_t* const ctx16 = tiles && whole(KR) ? reinterpret_cast<bf16_t*>(g->ctx) : nullptr;
-            bf16_t* const o16 = ctx16 && whole(HV) ? g->o16 : nullptr;
             const float* q = direct ? g->proj : g->q;
             const int ldq = direct ? LD : H * (D + R);
+            // portions with enough rows: keys and values of the heads' own
+            LatentHeads lh;
+            lh.q = q; lh.ukT = L.ukT; lh.uv = L.uv; lh.cache = ps.cache; lh.gate = gate; lh.sink = L.sink; lh.ent_start = d_estart; lh.ent_len = d_elen; lh.ent_slot = d_eslot;
+            lh.row_pos = d_pos; lh.page_table = g->page_table; lh.n_entries = n_ent; lh.max_pages = g->max_pages; lh.page_tokens = g->P; lh.ldq = ldq; lh.ldg = LD; lh.ldo = HV;
+            lh.H = H; lh.D = D; lh.R = R; lh.KR = KR; lh.Vd = Vd; lh.scale = d.scale; lh.rot = rot; lh.size = g->step_size; lh.ws = g->head_keys; lh.ws_bytes = g->head_key_bytes;
+            lh.out = g->o16;
+            const bool by_heads = r16 && !single && !capturing && latent_heads_fit(lh);
+            bf16_t* const o16 = by_heads || (ctx16 && whole(HV)) ? g->o16 : nullptr;
             // decode steps: from the projected queries to the values in two launches, with the queries' own norm inside the product in front
             bool stepped = false;
             LatentStep st;
@@ -1441,9 +1456,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 if (queries) ZG_TRY(launch_latent_step(st, s, &stepped));
             }
             if (!stepped) {
-                bool absorbed = false;
+                bool absorbed = by_heads;  // (the queries are read as they are)
                 if (direct) {
-                    if (qa16) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
+                    if (qa16 && !by_heads) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
                     ZG_TRY(launch_latent_direct_prep(g->proj, LD, M, H, D, R, KR, H * (D + R), L.dkv_norm, eps, rot, d_pos, d_slot, g->page_table, g->max_pages,
                                                      g->P, absorbed ? nullptr : g->qa, d.kv_from > 0 ? nullptr : ps.cache, s, absorbed ? nullptr : qa16));
                 } else {
@@ -1453,7 +1468,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                     lin.A = cq16 ? nullptr : g->cq; lin.A16 = cq16; lin.lda = QR; lin.B = L.uq; lin.ldb = QR; lin.C = g->q; lin.ldc = H * (D + R); lin.M = M; lin.N = H * (D + R); lin.K = QR;
                     ZG_TRY(launch_linear(lin, f32, s));
                 }
-                if (qa16 && !direct) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
+                if (qa16 && !direct && !by_heads) ZG_TRY(launch_latent_queries(q, ldq, L.ukT, qa16, M, H, D, R, KR, rot, d_pos, s, &absorbed));
                 if (!absorbed) {
                     lin = Linear();  // the unrotated query part carried into the latent space, head by head
                     lin.A = q; lin.lda = ldq; lin.a_zoff = D + R; lin.B = L.ukT; lin.ldb = D; lin.b_zoff = (long long)KR * D;
@@ -1461,8 +1476,9 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                     ZG_TRY(launch_linear(lin, f32, s));
                     if (!direct) ZG_TRY(launch_q_rotary(g->q, H * (D + R), g->qa, H * (KR + R), M, H, D, R, KR, rot, d_pos, s, qa16));
                 }
-                bool tiled = false;
-                if (!f32 && !few)
+                bool tiled = by_heads;
+                if (by_heads) ZG_TRY(launch_latent_heads(lh, s));
+                if (!f32 && !few && !tiled)
                     ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
                                                          g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
                                                          L.sink, qa16, ctx16));
@@ -1473,10 +1489,10 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                 if (!tiled)
                     ZG_TRY(launch_latent_attention(g->qa, g->ctx, M, H, KR, R, d.scale, d_pos, d_slot, g->page_table, g->max_pages, g->P, ps.cache,
                                                    g->attn_ws, g->attn_ws_floats, s, gate, LD, L.sink));
-                lin = Linear();  // values of the weighted latent, head by head
+                lin = Linear();  // values of the weighted latent, head by head (by_heads: in the results)
                 lin.A = ctx16 ? nullptr : g->ctx; lin.A16 = ctx16; lin.lda = H * KR; lin.a_zoff = KR; lin.B = L.uv; lin.ldb = KR; lin.b_zoff = (long long)Vd * KR;
                 lin.C = o16 ? nullptr : g->o; lin.C16 = o16; lin.ldc = HV; lin.c_zoff = Vd; lin.M = M; lin.N = Vd; lin.K = KR; lin.nz = H;
-                ZG_TRY(launch_linear(lin, f32, s));
+                if (!by_heads) ZG_TRY(launch_linear(lin, f32, s));
             }
             lin = Linear();
             lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;
@@ -1746,12 +1762,19 @@ int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair
     g->step_keys = 0;
     g->step_key_tiles = 0;
     g->step_longest = g->step_blocks = 0;
+    g->step_size = PortionSize();
     for (int e = 0; e < n_ent; ++e) {
         const Piece& pc = pieces[e];
         g->step_keys = std::max(g->step_keys, pc.pos0 + pc.n);
         g->step_longest = std::max(g->step_longest, pc.n);
         g->step_key_tiles += (pc.pos0 + pc.n + 31) / 32;
         g->step_blocks += (pc.n + 31) / 32;
+        g->step_size.rows += pc.n;
+        g->step_size.tiles += (pc.pos0 + pc.n + 31) / 32;
+        g->step_size.all_keys += pc.pos0 + pc.n;
+        g->step_size.pairs += (size_t)pc.n * (pc.pos0 + (pc.n + 1) / 2);
+        g->step_size.blocks += (pc.n + 31) / 32;
+        g->step_size.wide_blocks += (pc.n + 127) / 128;
         ent_start[e] = r;
         ent_len[e] = pc.n;
         ent_slot[e] = pc.slot;
@@ -2307,6 +2330,10 @@ int zg_lm_create(zg_lm** out, const zg_lm_config* config, int device) {
         if (hipMalloc(reinterpret_cast<void**>(&g->arena), g->arena_bytes) == hipSuccess) break;
         (void)hipGetLastError();
         g->arena = nullptr;
+        if (g->head_key_bytes > 0) {
+            g->no_head_keys = true;
+            continue;
+        }
         if (!g->f32 && !g->lean) {
             g->lean = true;
             continue;

@@ -361,6 +361,29 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
                                   const float* gate = nullptr, int ldg = 0, const float* sink = nullptr, const bf16_t* qa16 = nullptr,
                                   bf16_t* ctx16 = nullptr);
 
+// The same over keys and values of the heads' own (lm_latent_heads.hip): out[m][h Vd + n] = the head's result times its gate, rounded; q rows of heads
+// [D | R], unrotated.  It has to fit: not a form it has, a portion whose keys in front of it weigh more than its rows, too little room.
+struct PortionSize {  // of a step: rows, key tiles of 32, positions reached, (row, key) pairs, blocks of 32 and of 128 rows of its entries
+    size_t rows = 0, tiles = 0, all_keys = 0, pairs = 0;
+    int blocks = 0, wide_blocks = 0;
+};
+struct LatentHeads {
+    const float* q = nullptr;
+    const bf16_t *ukT = nullptr, *uv = nullptr;  // [H][KR][D], [H][Vd][KR]
+    const float *cache = nullptr, *gate = nullptr, *sink = nullptr;
+    const int *ent_start = nullptr, *ent_len = nullptr, *ent_slot = nullptr, *row_pos = nullptr, *page_table = nullptr;
+    int n_entries = 0, max_pages = 0, page_tokens = 0, ldq = 0, ldg = 0, ldo = 0, H = 0, D = 0, R = 0, KR = 0, Vd = 0;
+    float scale = 1.0f;
+    Rotary rot{nullptr, 0, 1.0f, 0};
+    PortionSize size;
+    char* ws = nullptr;
+    size_t ws_bytes = 0;
+    bf16_t* out = nullptr;
+};
+size_t latent_heads_record(int H, int D, int R, int KR, int Vd, int rot_dims);  // bytes of a key tile in its workspace, 0: not a form it has
+bool latent_heads_fit(const LatentHeads& a);
+int launch_latent_heads(const LatentHeads& a, hipStream_t s);
+
 // ------------------------------------------------------------------------------------------------ input convolution of decode rows, residual sum
 // Steps of one row per entry: [x += x0] or [x += norm(y) * (1 + wb), y = yl or the mean of the two normed branches yl, yr with
 // plain weights wl, wr], then h = norm(x) * (1 + wn), out = h + conv(h) over the slot's tail, the tail moved on — one launch.
