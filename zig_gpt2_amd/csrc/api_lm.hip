@@ -1404,9 +1404,10 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             if (single) ZG_TRY(launch_gated_step(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_eslot, n_ent, H, D, Vd, L.fb,
                                                  L.lower, L.hnorm, eps, s, &stepped));
             if (!stepped) {
+                HeadNorm norm{L.hnorm, eps, o16};
                 ZG_TRY(launch_hgrn2_scan(g->proj, NP, g->o, HV, g->hgrn_state + ps.hgrn_off, g->hgrn_floats, d_estart, d_elen, d_eslot, n_ent, M, H, D, Vd,
-                                         L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s));
-                ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s, o16));
+                                         L.fb, L.lower, g->scan_ws, g->scan_ws_floats, g->step_longest, s, nullptr, nullptr, &norm));
+                if (!norm.done) ZG_TRY(launch_norm_plain(g->o, HV, H, Vd, M, L.hnorm, eps, s, o16));
             }
             lin = Linear();
             lin.A = o16 ? nullptr : g->o; lin.A16 = o16; lin.lda = HV; lin.B = L.o; lin.ldb = HV; lin.C = g->y; lin.ldc = W; lin.M = M; lin.N = W; lin.K = HV;

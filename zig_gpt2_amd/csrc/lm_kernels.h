@@ -205,15 +205,22 @@ struct GlaGate {
     const float* z_bias = nullptr;
     float inv_tau = 1.0f, q_scale = 1.0f;
 };
+// norm != null: a kernel that has whole heads leaves o / rms(o) * w instead, in out or rounded in out16 (rows of the same stride), and says so.
+struct HeadNorm {
+    const float* w;
+    float eps;
+    bf16_t* out16;
+    bool done = false;
+};
 int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start,
                       const int* ent_len, const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low,
-                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay = nullptr, const GlaGate* gla = nullptr);
+                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay = nullptr, const GlaGate* gla = nullptr, HeadNorm* norm = nullptr);
 
 // The same for prompt portions in chunks of 64 tokens as fp32 matrix products (lm_scan.hip): HGRN2, or gla != null.  ws as above.
 // *taken = false when the heads are larger than its tiles (D > 128) or ws is too small (nothing launched).
 int launch_gated_chunks(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start, const int* ent_len,
                         const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low, float* ws, size_t ws_floats,
-                        const GlaGate* gla, hipStream_t s, bool* taken);
+                        const GlaGate* gla, hipStream_t s, bool* taken, HeadNorm* norm = nullptr);
 
 // One token of every entry (HGRN2, decode steps) and the norm of each head's result, out = o / rms(o) * w, in one launch.  *taken = false:
 // heads wider than its tiles or values in no whole 16-byte pieces, nothing launched.

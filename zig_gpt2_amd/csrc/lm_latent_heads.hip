@@ -5,8 +5,8 @@
 // launches in front and behind, becomes one launch that brings every cached latent into the heads', and the queries are read where the projection left them.
 // A portion pays for the keys in front of it again, so it has to have enough rows (latent_heads_fit).
 // us a layer, latents of 256 + 32, in the latent space : here: 8 x 1023 tokens, 16 heads: queries 33, tiles 9, attention 107, values 25 : keys 28, attention 42;
-// 8 x 256 tokens, 12 heads: 8 + 8 + 29 + 8 : 13.6 + 15.2.  The attention is bound by the vector work of its softmax beside ten products a tile (27 us of
-// them at the matrix cores' rate would be 15), the keys' launch by a workgroup's chain from the weights over eight tiles.
+// 8 x 256 tokens, 12 heads: 8 + 8 + 29 + 8 : 13.6 + 15.2.  The attention is bound by the vector work of its softmax beside ten products a tile, the keys'
+// launch by a workgroup's chain from the weights over its tiles.
 #include <stdlib.h>
 
 #include <algorithm>

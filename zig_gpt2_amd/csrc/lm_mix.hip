@@ -1795,7 +1795,7 @@ int launch_state_carry(float* state, size_t slot_stride, const int* ent_len, con
 
 int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* state, size_t slot_stride, const int* ent_start,
                       const int* ent_len, const int* ent_slot, int n_entries, int M, int H, int D, int V, const float* bias, const float* low,
-                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay, const GlaGate* gla) {
+                      float* ws, size_t ws_floats, int longest, hipStream_t s, const float* decay, const GlaGate* gla, HeadNorm* norm) {
     if (n_entries <= 0) return ZG_OK;
     ZG_REQUIRE(!gla || (gla->z && gla->z_bias && !decay), ZG_ERR_ARG, "gated linear attention: its gate needs z and a bias, and no fixed decay");
     const GlaGate gg = gla ? *gla : GlaGate();
@@ -1827,7 +1827,7 @@ int launch_hgrn2_scan(const float* proj, int ld, float* out, int ldo, float* sta
     if (!decay && M > kGemvMaxRows && longest > 32 && getenv("ZGPT2_LM_SCAN_NO_CHUNKS") == nullptr) {
         bool taken = false;
         ZG_TRY(launch_gated_chunks(proj, ld, out, ldo, state, slot_stride, ent_start, ent_len, ent_slot, n_entries, M, H, D, V, bias, low, ws, ws_floats, gla, s,
-                                   &taken));
+                                   &taken, norm));
         if (taken) return ZG_OK;
     }
     int G = 1;
