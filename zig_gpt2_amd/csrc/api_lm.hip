@@ -1694,7 +1694,14 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             ZG_TRY(launch_norm_conv_single(x, nullptr, g->y, nullptr, nullptr, nullptr, L.norm1b, L.norm2, eps, M, W, g->canon, L.canon2,
                                            g->seq_state + ps.canon2_off, g->seq_floats, d_slot, g->hc, s, &mid_done));
         RoutePre pre;
-        if (mid_done) {
+        bool routed = false;  // the choice of experts has been made behind the norm
+        if (!mid_done && !few && !canon && d.ff == ZG_LM_FF_MOE && d.router == ZG_LM_ROUTE_SOFTMAX_ALL) {
+            NormRows r;
+            r.x = x; r.x_out = x; r.y = g->y; r.wb = L.norm1b; r.wn = L.norm2; r.eps = eps; r.out = h_r16 ? nullptr : g->h; r.out16 = h_r16 ? g->h16 : nullptr; r.M = M; r.W = W;
+            r.router = L.router; r.correction = L.correction; r.experts = d.experts; r.choices = d.top; r.pick = g->pick; r.pick_weight = g->wt;
+            ZG_TRY(launch_norm_rows(r, s, &routed));
+        }
+        if (mid_done || routed) {
         } else if (defer && d.ff == ZG_LM_FF_DENSE) defer_norm(g->y, L.norm1b, L.norm2);
         else if (few && !canon && d.ff == ZG_LM_FF_MOE && route_norm_fits(L.router, W)) {  // steps of few rows: the router's workgroups do it
             pre.rms = true;
@@ -1721,10 +1728,11 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             const int E = d.experts, top = d.top, NA = M * top;
             const bool glu = d.ff_act == ZG_LM_ACT_GLU_SILU;
             const int UF = glu ? 2 * F : F;
-            ZG_TRY(launch_route(hin, M, W, L.router, L.correction, E, top, g->pick, g->wt, d.router, s, d.route_groups, d.route_keep,
-                                d.route_scale != 0.0f ? d.route_scale : 1.0f, pre.x ? &pre : nullptr));
+            if (!routed)
+                ZG_TRY(launch_route(hin, M, W, L.router, L.correction, E, top, g->pick, g->wt, d.router, s, d.route_groups, d.route_keep,
+                                    d.route_scale != 0.0f ? d.route_scale : 1.0f, pre.x ? &pre : nullptr));
             Linear up, dn;
-            up.A = hin; up.A16 = hin16; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
+            up.A = routed && hin16 ? nullptr : hin; up.A16 = hin16; up.lda = W; up.a_div = top; up.B = L.gu; up.ldb = W; up.b_zoff = (long long)UF * W; up.C = g->gu_buf; up.ldc = UF;
             up.N = UF; up.K = W;
             if (!glu) up.act = ACT_GELU_ERF;
             dn.A = g->hb; dn.lda = F; dn.B = L.edown; dn.ldb = F; dn.b_zoff = (long long)W * F; dn.C = g->ye; dn.ldc = W; dn.N = W; dn.K = F;

@@ -135,7 +135,14 @@ struct NormRows {
     float* last_out = nullptr;
     float* shift_out = nullptr;  // steps of one row per entry: the row's own normed form straight into its slot's state (shift_state's layout)
     int run = 1;  // (set by the launch) consecutive rows of a wave
+    // router != null (rows from y, normed, not mixed; at most kNormExperts experts): the choice of experts behind the norm as well (launch_route, rule 0)
+    const bf16_t* router = nullptr;
+    const float* correction = nullptr;
+    int experts = 0, choices = 0;
+    int* pick = nullptr;
+    float* pick_weight = nullptr;
 };
+constexpr int kNormExperts = 8;
 int launch_norm_rows(const NormRows& p, hipStream_t s, bool* taken);
 // out[m] = x[m] + y[m] / rms(y[m]) * (1 + w)     (the norm behind a sublayer, then the residual sum; out may be x)
 int launch_norm_add(const float* x, float* out, const float* y, const float* w, float eps, int M, int W, hipStream_t s);
