@@ -24,7 +24,7 @@ def form(request, monkeypatch):
 
 
 def model(cfg, w, **kw):
-    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), dtype="bfloat16", **{"max_tokens": 1024, "max_seqs": 4, **kw})
+    m = lm.LayeredLM(lm.LMConfig.from_json(cfg), **{"dtype": "bfloat16", "max_tokens": 1024, "max_seqs": 4, **kw})
     m.load_weights(w)
     return m
 
@@ -126,4 +126,61 @@ def test_values_that_are_not_finite(form, bad):
     got = steps(m, [toks], [[140]])[0]
     m.close()
     tl.assert_close(got[:75], ref[:75], "bfloat16", bad)
+    assert np.isnan(got[75:]).any(axis=1).all()
+
+
+@pytest.mark.parametrize("rank,heads", [(256, 3), (128, 2), (256, 1)])
+def test_32_bit(monkeypatch, rank, heads):
+    """32-bit mode: rows around blocks and tiles, portions behind histories on pages that are no whole tiles."""
+    cfg = tl.config([tl.latent_layer(heads=heads, kv_rank=rank, q_rank=40, mlp=tl.dense_mlp(ff=96), **DIMS)], vocab=203, width=64)
+    w = tl.weights(cfg, seed=rank)
+    m = model(cfg, w, dtype="float32", page_tokens=24)
+    for rows in (9, 31, 32, 33, 128, 129, 300):
+        toks = [tl.tokens(rows, rows, cfg["vocab"])]
+        got = steps(m, toks, [[rows]])[0]
+        monkeypatch.setenv("ZGPT2_LM_LATENT_HEADS", "-1")
+        other = steps(m, toks, [[rows]])[0]
+        monkeypatch.delenv("ZGPT2_LM_LATENT_HEADS")
+        tl.assert_close(got, lm_oracle.Model(cfg, w).forward(toks[0])[0], "float32", (rank, heads, rows))
+        assert not np.array_equal(got, other)  # (another order of sums: it was this path that ran)
+    toks = [tl.tokens(80 + b, n, cfg["vocab"]) for b, n in enumerate((300, 97, 66))]
+    refs = [lm_oracle.Model(cfg, w).forward(t)[0] for t in toks]
+    cuts = [[33, 64, 31], [34, 95, 40], [163, 96, 65], [300, 97, 66]]
+    for got, want in zip(steps(m, toks, cuts), of(refs, cuts)):
+        tl.assert_close(got, want, "float32", cuts)
+    m.close()
+
+
+@pytest.mark.parametrize("design", ["gate", "sink"])
+def test_32_bit_other_designs(design):
+    if design == "gate":
+        lib, oracle = dl, duvulix_oracle
+        layers = [dl.latent_layer(heads=4, kv_rank=256, mlp=dl.dense(ff=64), **DIMS), dl.latent_layer(heads=3, kv_rank=256, kv_from=0, mlp=dl.dense(ff=64), **DIMS)]
+    else:
+        lib, oracle = pl, pemuvik_oracle
+        layers = [pl.latent_layer(heads=4, kv_rank=256, mlp=pl.dense(ff=64), **DIMS)]
+    cfg = lib.config(layers, vocab=203, width=64)
+    w = lib.weights(cfg, seed=4)
+    toks = [lib.tokens(90 + b, n, cfg["vocab"]) for b, n in enumerate((150, 97))]
+    cuts = [[130, 33], [150, 97]]
+    m = model(cfg, w, dtype="float32")
+    for got, want in zip(steps(m, toks, cuts), of([oracle.forward(w, cfg, t) for t in toks], cuts)):
+        tl.assert_close(got, want, "float32")
+    m.close()
+
+
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_32_bit_values_that_are_not_finite(bad):
+    cfg = tl.config([tl.latent_layer(heads=3, kv_rank=256, q_rank=40, mlp=tl.dense_mlp(ff=96), **DIMS)], vocab=203, width=64)
+    w = tl.weights(cfg, seed=3)
+    toks = tl.tokens(5, 140, cfg["vocab"])
+    toks[toks == 7] = 8
+    ref = lm_oracle.Model(cfg, w).forward(toks)[0]
+    toks[75] = 7
+    w["embed"] = w["embed"].copy()
+    w["embed"][7, 3] = bad
+    m = model(cfg, w, dtype="float32")
+    got = steps(m, [toks], [[140]])[0]
+    m.close()
+    tl.assert_close(got[:75], ref[:75], "float32", bad)
     assert np.isnan(got[75:]).any(axis=1).all()

@@ -608,7 +608,7 @@ void layout(zg_lm* g, Bump& b) {
             max_ctx = std::max(max_ctx, H * KR);
             max_att_part = std::max(max_att_part, H * (KR + 2));
             if (!g->f32) max_tile = std::max(max_tile, latent_tile_elems((int)KR, (int)R));
-            if (!g->f32) max_record = std::max(max_record, latent_heads_record((int)H, (int)D, (int)R, (int)KR, (int)Vd, (int)d.rot_dims));
+            max_record = std::max(max_record, latent_heads_record((int)H, (int)D, (int)R, (int)KR, (int)Vd, (int)d.rot_dims, g->f32));
             max_o = std::max(max_o, HV);
         }
         if (d.ff != ZG_LM_FF_NONE && tn) {
@@ -1432,9 +1432,10 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
             lh.q = q; lh.ukT = L.ukT; lh.uv = L.uv; lh.cache = ps.cache; lh.gate = gate; lh.sink = L.sink; lh.ent_start = d_estart; lh.ent_len = d_elen; lh.ent_slot = d_eslot;
             lh.row_pos = d_pos; lh.page_table = g->page_table; lh.n_entries = n_ent; lh.max_pages = g->max_pages; lh.page_tokens = g->P; lh.ldq = ldq; lh.ldg = LD; lh.ldo = HV;
             lh.H = H; lh.D = D; lh.R = R; lh.KR = KR; lh.Vd = Vd; lh.scale = d.scale; lh.rot = rot; lh.size = g->step_size; lh.ws = g->head_keys; lh.ws_bytes = g->head_key_bytes;
-            lh.out = g->o16;
-            const bool by_heads = r16 && !single && !capturing && latent_heads_fit(lh);
-            bf16_t* const o16 = by_heads || (ctx16 && whole(HV)) ? g->o16 : nullptr;
+            if (f32) lh.out32 = g->o;
+            else lh.out = g->o16;
+            const bool by_heads = (r16 || (f32 && !few)) && !single && !capturing && latent_heads_fit(lh);
+            bf16_t* const o16 = (by_heads && !f32) || (ctx16 && whole(HV)) ? g->o16 : nullptr;
             // decode steps: from the projected queries to the values in two launches, with the queries' own norm inside the product in front
             bool stepped = false;
             LatentStep st;
@@ -1483,7 +1484,7 @@ int enqueue_layers(zg_lm* g, int M, int n_ent, bool capturing, bool single, bool
                     ZG_TRY(launch_latent_attention_tiles(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
                                                          g->max_pages, g->P, ps.cache, g->key_tiles, g->key_tile_elems, g->step_key_tiles, g->step_keys, s, &tiled, gate, LD,
                                                          L.sink, qa16, ctx16));
-                if (f32 && !few)
+                if (f32 && !few && !tiled)
                     ZG_TRY(launch_latent_attention_f32(g->qa, g->ctx, M, H, KR, R, d.scale, d_estart, d_elen, d_eslot, n_ent, d_pos, g->page_table,
                                                        g->max_pages, g->P, ps.cache, s, &tiled, gate, LD, L.sink));
                 ZG_REQUIRE(tiled || !tiles, ZG_ERR_UNSUPPORTED, "latent attention: the tiles do not fit their workspace");
@@ -1781,6 +1782,7 @@ int stage_rows(zg_lm* g, const std::vector<Piece>& pieces, std::vector<std::pair
         g->step_size.rows += pc.n;
         g->step_size.tiles += (pc.pos0 + pc.n + 31) / 32;
         g->step_size.all_keys += pc.pos0 + pc.n;
+        g->step_size.longest = std::max<size_t>(g->step_size.longest, pc.pos0 + pc.n);
         g->step_size.pairs += (size_t)pc.n * (pc.pos0 + (pc.n + 1) / 2);
         g->step_size.blocks += (pc.n + 31) / 32;
         g->step_size.wide_blocks += (pc.n + 127) / 128;

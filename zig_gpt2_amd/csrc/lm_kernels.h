@@ -375,10 +375,10 @@ int launch_latent_attention_tiles(const float* qa, float* ctx, int M, int H, int
                                   const float* gate = nullptr, int ldg = 0, const float* sink = nullptr, const bf16_t* qa16 = nullptr,
                                   bf16_t* ctx16 = nullptr);
 
-// The same over keys and values of the heads' own (lm_latent_heads.hip): out[m][h Vd + n] = the head's result times its gate, rounded; q rows of heads
+// The same over keys and values of the heads' own (lm_latent_heads.hip): out[m][h Vd + n] = the head's result times its gate, rounded in bf16 mode; q rows of heads
 // [D | R], unrotated.  It has to fit: not a form it has, a portion whose keys in front of it weigh more than its rows, too little room.
-struct PortionSize {  // of a step: rows, key tiles of 32, positions reached, (row, key) pairs, blocks of 32 and of 128 rows of its entries
-    size_t rows = 0, tiles = 0, all_keys = 0, pairs = 0;
+struct PortionSize {  // of a step: rows, key tiles of 32, positions reached and the farthest of them, (row, key) pairs, blocks of 32 and of 128 rows of its entries
+    size_t rows = 0, tiles = 0, all_keys = 0, longest = 0, pairs = 0;
     int blocks = 0, wide_blocks = 0;
 };
 struct LatentHeads {
@@ -392,9 +392,10 @@ struct LatentHeads {
     PortionSize size;
     char* ws = nullptr;
     size_t ws_bytes = 0;
-    bf16_t* out = nullptr;
+    bf16_t* out = nullptr;   // bf16 mode
+    float* out32 = nullptr;  // 32-bit mode
 };
-size_t latent_heads_record(int H, int D, int R, int KR, int Vd, int rot_dims);  // bytes of a key tile in its workspace, 0: not a form it has
+size_t latent_heads_record(int H, int D, int R, int KR, int Vd, int rot_dims, bool f32);  // bytes of a key tile in its workspace, 0: not a form it has
 bool latent_heads_fit(const LatentHeads& a);
 int launch_latent_heads(const LatentHeads& a, hipStream_t s);
 

@@ -1,12 +1,12 @@
-// lm_latent_heads.hip — latent attention of prompt portions in bf16 mode, over keys and values of the heads' own.
+// lm_latent_heads.hip — latent attention of prompt portions, over keys and values of the heads' own.
 //
 // In the latent space a (query, key) pair of a head costs KR + R products for its score and KR for its value (544 with latents of 256 + 32); with the
 // key uk c and the value uv c of the head itself it costs D + R and V (160).  What brings queries into the latent space and results out of it, two
 // launches in front and behind, becomes one launch that brings every cached latent into the heads', and the queries are read where the projection left them.
 // A portion pays for the keys in front of it again, so it has to have enough rows (latent_heads_fit).
-// us a layer, latents of 256 + 32, in the latent space : here: 8 x 1023 tokens, 16 heads: queries 33, tiles 9, attention 107, values 25 : keys 28, attention 42;
+// us a layer, latents of 256 + 32, in the latent space : here, bf16 mode: 8 x 1023 tokens, 16 heads: queries 33, tiles 9, attention 107, values 25 : keys 28, attention 42;
 // 8 x 256 tokens, 12 heads: 8 + 8 + 29 + 8 : 13.6 + 15.2.  The attention is bound by the vector work of its softmax beside ten products a tile, the keys'
-// launch by a workgroup's chain from the weights over its tiles.
+// launch by a workgroup's chain from the weights over its tiles.  32-bit mode, 1 x 333 tokens, 12 heads: queries 9 + 3, attention 32, values 9 : 8.4 + 15.7.
 #include <stdlib.h>
 
 #include <algorithm>
@@ -29,8 +29,13 @@ typedef __attribute__((ext_vector_type(2))) float f32x2;
 // of its positions ([token][pair] cosine and sine, what the queries are rotated by), and for every head four pieces of its keys (16 channels each) and
 // four of its values ([16 tokens][32 channels]).  A piece is [lane] 16 bytes; which 16 of a fragment's 32 x 16 values are a lane's is the matrix
 // instruction's layout of results, so that a result is a fragment as it lies: of 16 channels (tokens) a lane has 4 half + 0..3 and 8 + 4 half + 0..3.
-constexpr int kD = 64, kR = 32, kV = 64, kAngles = 2048, kHeads = kAngles + 32 * (kR / 2) * 8, kHead = 32 * (kD + kV) * 2;
-__host__ __device__ constexpr size_t record_bytes(int H) { return kHeads + (size_t)H * kHead; }
+// In 32-bit mode the same values are fp32, pieces of 8 channels (tokens) of which a lane has 4 half + 0..3.
+constexpr int kD = 64, kR = 32, kV = 64;
+template <bool F32>
+struct Record {
+    static constexpr int EL = F32 ? 4 : 2, ANGLES = 32 * kR * EL, HEADS = ANGLES + 32 * (kR / 2) * 8, VALUES = 32 * kD * EL, HEAD = VALUES + 32 * kV * EL;
+    static __host__ __device__ constexpr size_t bytes(int H) { return HEADS + (size_t)H * HEAD; }
+};
 
 struct Entry {
     int first_tile, tiles;      // key tiles of the entries in front of it, its own
@@ -111,8 +116,11 @@ struct KeysShared {
 // Keys are multiplied as uk c^T and values as c uv^T, so that either result lies as the attention's fragment.
 // A latent with a value that is not finite is left out (a weight of zero times it would reach queries that do not see the key), and its rotated part
 // says so (NaN): the queries that see the key come out NaN.  Values are kept finite for the same reason.
-template <int KS, bool V>  // KR = 16 KS
+// F32 (32-bit mode): a latent as its exact three bf16 terms, three products each, the second and third terms' with sums of their own; one buffer.
+template <int KS, bool V, bool F32>  // KR = 16 KS
 __device__ __forceinline__ void head_keys(const KeysArgs& a, char* s_mem, KeysShared& sh) {
+    typedef Record<F32> REC;
+    constexpr int NP = F32 ? 3 : 1;
     constexpr int KR = 16 * KS, DT = KR + kR, NL = KR / 32, CH = KR / 4, STEP = 1024 + 16;  // 16-byte pieces of a tile a lane loads; of a row; bytes from k-step to k-step
     constexpr int PITCH = V ? KR * 2 + 8 : kD * 2, HEAD = V ? 64 * PITCH : KR * PITCH, NW = KR / 16;  // of the weights in the LDS (other banks); 16-byte pieces a lane loads
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 31, hf = lane >> 5, j = wave & 1;  // channels 32 j ..
@@ -186,8 +194,9 @@ __device__ __forceinline__ void head_keys(const KeysArgs& a, char* s_mem, KeysSh
     auto body = [&](auto buf, int l) {
         const int keys = __builtin_amdgcn_readfirstlane(sh.tokens[l]), pos = sh.pos[l];
         const f32x4 rope = rope_next[buf];
-        char* const tile = s_mem + buf * (KS * STEP);
-        constexpr unsigned kTop = 0x7F7F8000u;  // from here on a value rounds to an infinity
+        char* const tile = s_mem + (F32 ? 0 : buf * (KS * STEP));
+        if (F32) __syncthreads();  // (the tile in front has been read)
+        constexpr unsigned kTop = F32 ? 0x7F800000u : 0x7F7F8000u;  // from here on a value is not finite, rounds to an infinity
         unsigned most = 0;
 #pragma unroll
         for (int i = 0; i < NL; ++i)
@@ -209,51 +218,74 @@ __device__ __forceinline__ void head_keys(const KeysArgs& a, char* s_mem, KeysSh
 #pragma unroll
         for (int i = 0; i < NL; ++i) {
             const int key = (tid + 256 * i) / CH, c = (tid + 256 * i) % CH;
-            const f32x4 v = next[buf][i];
+            f32x4 v = next[buf][i];
             // (k-steps lie 16 bytes more than their size apart, so that a row's pieces go to different banks)
-            *reinterpret_cast<u32x2*>(tile + (c >> 2) * STEP + ((c & 1) * 32 + key) * 16 + ((c >> 1) & 1) * 8) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
+            char* const to = tile + (c >> 2) * STEP + ((c & 1) * 32 + key) * 16 + ((c >> 1) & 1) * 8;
+            if constexpr (!F32) *reinterpret_cast<u32x2*>(to) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
+            else
+#pragma unroll
+                for (int t = 0; t < 3; ++t) {  // 24 mantissa bits = 8 + 8 + 8, cut off
+                    uint32_t b[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        b[u] = __float_as_uint(v[u]);
+                        v[u] -= __uint_as_float(b[u] & 0xFFFF0000u);
+                    }
+                    *reinterpret_cast<u32x2*>(to + t * (KS * STEP)) = u32x2{__builtin_amdgcn_perm(b[1], b[0], 0x07060302u), __builtin_amdgcn_perm(b[3], b[2], 0x07060302u)};
+                }
         }
         __syncthreads();
         fetch(buf, l + 2);
-        char* rec = a.out + (size_t)(t0 + l) * record_bytes(a.H);
+        char* rec = a.out + (size_t)(t0 + l) * REC::bytes(a.H);
         if (shared_part) {
             const int key = tid >> 3, c = tid & 7;
             f32x4 v = key < keys ? rope : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (c == 0 && (sh.bad[slot] >> key & 1u)) v.x = __uint_as_float(0x7FC00000u);
-            *reinterpret_cast<u32x2*>(rec + (c >> 2) * 1024 + ((c & 1) * 32 + key) * 16 + ((c >> 1) & 1) * 8) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
+            if (F32) *reinterpret_cast<f32x4*>(rec + (c >> 1) * 1024 + ((c & 1) * 32 + key) * 16) = v;
+            else *reinterpret_cast<u32x2*>(rec + (c >> 2) * 1024 + ((c & 1) * 32 + key) * 16 + ((c >> 1) & 1) * 8) = u32x2{cvt_pk_bf16(v.x, v.y), cvt_pk_bf16(v.z, v.w)};
 }
         if (V)  // (the angles of a tile, 64 a wave, dealt over the heads: with all in the first head's workgroups 1.3 us more)
 #pragma unroll 1
             for (int x = wave * (int)gridDim.y + (int)blockIdx.y; x < 32 * (kR / 2) / 64; x += 4 * (int)gridDim.y) {
                 const float angle = (float)(pos + 4 * x + lane / (kR / 2)) * freq;
-                reinterpret_cast<f32x2*>(rec + kAngles)[64 * x + lane] = f32x2{cosf(angle) * a.rot.amp, sinf(angle) * a.rot.amp};
+                reinterpret_cast<f32x2*>(rec + REC::ANGLES)[64 * x + lane] = f32x2{cosf(angle) * a.rot.amp, sinf(angle) * a.rot.amp};
             }
-        f32x16 acc;
+        f32x16 acc, small;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) acc[e] = 0.0f;
-        auto part = [&](int s) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(tile + s * STEP + lane * 16)); };
+        for (int e = 0; e < 16; ++e) acc[e] = small[e] = 0.0f;
+        auto part = [&](int x) { return __builtin_bit_cast(bf16x8, *reinterpret_cast<const u32x4*>(tile + x * STEP + lane * 16)); };  // k-step x % KS of term x / KS
         constexpr int AHEAD = 4;  // (fragments on their way)
         bf16x8 c[AHEAD];
 #pragma unroll
-        for (int s = 0; s < AHEAD; ++s) c[s] = part(s);
+        for (int x = 0; x < AHEAD; ++x) c[x] = part(NP * KS - 1 - x);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            const bf16x8 ws = __builtin_bit_cast(bf16x8, w[s]);
-            acc = V ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[s % AHEAD], ws, acc, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ws, c[s % AHEAD], acc, 0, 0, 0);
-            if (s + AHEAD < KS) c[s % AHEAD] = part(s + AHEAD);
+        for (int x = 0; x < NP * KS; ++x) {  // the smallest term first
+            const int at = NP * KS - 1 - x;
+            const bf16x8 ws = __builtin_bit_cast(bf16x8, w[at % KS]);
+            f32x16& to = at >= KS ? small : acc;
+            to = V ? __builtin_amdgcn_mfma_f32_32x32x16_bf16(c[x % AHEAD], ws, to, 0, 0, 0) : __builtin_amdgcn_mfma_f32_32x32x16_bf16(ws, c[x % AHEAD], to, 0, 0, 0);
+            if (x + AHEAD < NP * KS) c[x % AHEAD] = part(at - AHEAD);
             __builtin_amdgcn_sched_barrier(0);
         }
-        if (V)
+        if (F32) acc += small;
+        if (V) {
+            constexpr float kMost = F32 ? 3.40282347e38f : 3.38953139e38f;
 #pragma unroll
             for (int e = 0; e < 16; ++e) {  // (NaN stays)
-                acc[e] = acc[e] > 3.38953139e38f ? 3.38953139e38f : acc[e];
-                acc[e] = acc[e] < -3.38953139e38f ? -3.38953139e38f : acc[e];
+                acc[e] = acc[e] > kMost ? kMost : acc[e];
+                acc[e] = acc[e] < -kMost ? -kMost : acc[e];
             }
+        }
         if (h < a.H) {
-            char* to = rec + kHeads + (size_t)h * kHead + (V ? 4096 : 0) + lane * 16;
+            char* to = rec + REC::HEADS + (size_t)h * REC::HEAD + (V ? REC::VALUES : 0) + lane * 16;
+            if constexpr (F32) {
 #pragma unroll
-            for (int x = 0; x < 2; ++x) *reinterpret_cast<u32x4*>(to + (V ? 2 * x + j : 2 * j + x) * 1024) = eight(acc, 8 * x);
+                for (int g = 0; g < 4; ++g) *reinterpret_cast<f32x4*>(to + (4 * j + g) * 1024) = f32x4{acc[4 * g], acc[4 * g + 1], acc[4 * g + 2], acc[4 * g + 3]};
+            } else {
+#pragma unroll
+                for (int x = 0; x < 2; ++x) *reinterpret_cast<u32x4*>(to + (V ? 2 * x + j : 2 * j + x) * 1024) = eight(acc, 8 * x);
+            }
         }
         if (tid == 0) sh.bad[slot == 0 ? 2 : slot - 1] = 0;  // (the slot of the tile in front: read before this tile's barrier, written next behind the next one's)
         slot = slot == 2 ? 0 : slot + 1;
@@ -264,24 +296,50 @@ __device__ __forceinline__ void head_keys(const KeysArgs& a, char* s_mem, KeysSh
     }
 }
 
-template <int KS>
+template <int KS, bool F32>
 __global__ __launch_bounds__(256, 2) void latent_head_keys_kernel(const KeysArgs a) {
-    constexpr int KR = 16 * KS, TILES = 2 * KS * 1040, WEIGHTS = 2 * 64 * (KR * 2 + 8);
+    constexpr int KR = 16 * KS, TILES = (F32 ? 3 : 2) * KS * 1040, WEIGHTS = 2 * 64 * (KR * 2 + 8);
     __shared__ __attribute__((aligned(1024))) char s_mem[TILES > WEIGHTS ? TILES : WEIGHTS];
     __shared__ KeysShared sh;
-    if (blockIdx.z == 0) head_keys<KS, false>(a, s_mem, sh);
-    else head_keys<KS, true>(a, s_mem, sh);
+    if (blockIdx.z == 0) head_keys<KS, false, F32>(a, s_mem, sh);
+    else head_keys<KS, true, F32>(a, s_mem, sh);
 }
 
 struct HeadsArgs {
     const float* q;
     const char* keys;
     bf16_t* out;
+    float* out32;
     const float *gate, *sink;
     const int *ent_start, *ent_len, *ent_slot, *row_pos;
     int ldq, ldo, ldg, H, n_entries, halves;
     float scale;
 };
+
+// A query's rotated part, channel 8 i + 4 half + u of it in v[8 + i][u], by its position's cosines and sines.
+__device__ __forceinline__ void rotate(f32x4 (&v)[12], const f32x2* cs, int halves, int hf) {
+    if (halves) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const f32x2 c = cs[8 * i + 4 * hf + u];
+                const float x = v[8 + i][u], y = v[10 + i][u];
+                v[8 + i][u] = x * c.x - y * c.y;
+                v[10 + i][u] = y * c.x + x * c.y;
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; u += 2) {
+                const f32x2 c = cs[4 * i + 2 * hf + u / 2];
+                const float x = v[8 + i][u], y = v[8 + i][u + 1];
+                v[8 + i][u] = x * c.x - y * c.y;
+                v[8 + i][u + 1] = y * c.x + x * c.y;
+            }
+    }
+}
 
 // A wave takes 32 queries of one head.  KW = 1: the four waves of a workgroup have queries behind each other and share the tiles of 32 keys; KW = 4: they
 // have the same queries and every fourth tile each, and meet in the LDS.  Tiles arrive by DMA as whole fragments, two (four) to a buffer, in two buffers.
@@ -289,7 +347,8 @@ struct HeadsArgs {
 // probabilities a lane computed are the ones it has to feed back.  Scores, softmax and both accumulations are fp32.
 template <int KW>
 __global__ __launch_bounds__(256, KW == 1 ? 4 : 2) void latent_heads_kernel(const HeadsArgs a) {
-    constexpr int S = KW == 1 ? 2 : 4, BQ = 32 * (4 / KW), TILE = 2048 + kHead, PIECES = S * TILE / 1024;  // tiles of a buffer, queries of a workgroup
+    typedef Record<false> REC;
+    constexpr int S = KW == 1 ? 2 : 4, BQ = 32 * (4 / KW), TILE = 2048 + REC::HEAD, PIECES = S * TILE / 1024;  // tiles of a buffer, queries of a workgroup
     __shared__ __attribute__((aligned(1024))) char s_k[2][S * TILE];
     Entry at;
     int h = 0, block = 0;
@@ -299,14 +358,14 @@ __global__ __launch_bounds__(256, KW == 1 ? 4 : 2) void latent_heads_kernel(cons
     const int nq = min(32, at.len - q0);                    // (none: the wave only brings tiles)
     const int m_first = at.start + q0, pos_first = at.pos + q0, qpos = pos_first + r;
     const int my_tiles = nq > 0 ? (pos_first + nq + 31) / 32 : 0, n_tiles = (at.pos + min(at.len, block * BQ + BQ) + 31) / 32, n_iter = (n_tiles + S - 1) / S;
-    const size_t record = record_bytes(a.H);
+    const size_t record = REC::bytes(a.H);
     const char* src = a.keys + (size_t)at.first_tile * record + lane * 16;
     const unsigned lds0 = (unsigned)(unsigned long)(__attribute__((address_space(3))) char*)&s_k[0][0];
     auto request = [&](int it, int buf) {
 #pragma unroll
         for (int i = 0; i < PIECES / 4; ++i) {
             const int p = wave + 4 * i, j = p / 10, x = p - 10 * j;  // (beyond the last tile: the last, not used)
-            const char* g = src + (size_t)min(it * S + j, n_tiles - 1) * record + (x < 2 ? x * 1024 : kHeads + h * kHead + (x - 2) * 1024);
+            const char* g = src + (size_t)min(it * S + j, n_tiles - 1) * record + (x < 2 ? x * 1024 : REC::HEADS + h * REC::HEAD + (x - 2) * 1024);
             asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds0 + buf * (S * TILE) + p * 1024), "v"(g) : "memory", "m0");
         }
     };
@@ -318,30 +377,8 @@ __global__ __launch_bounds__(256, KW == 1 ? 4 : 2) void latent_heads_kernel(cons
         f32x4 v[12];
 #pragma unroll
         for (int i = 0; i < 12; ++i) v[i] = *reinterpret_cast<const f32x4*>(qr + 8 * i);
-        // channel 8 i + 4 half + u of the rotated part in v[8 + i][u]
         const int kp = min(qpos, at.pos + at.len - 1);
-        const f32x2* cs = reinterpret_cast<const f32x2*>(a.keys + (size_t)(at.first_tile + kp / 32) * record + kAngles) + (kp % 32) * (kR / 2);
-        if (a.halves) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    const f32x2 c = cs[8 * i + 4 * hf + u];
-                    const float x = v[8 + i][u], y = v[10 + i][u];
-                    v[8 + i][u] = x * c.x - y * c.y;
-                    v[10 + i][u] = y * c.x + x * c.y;
-                }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int u = 0; u < 4; u += 2) {
-                    const f32x2 c = cs[4 * i + 2 * hf + u / 2];
-                    const float x = v[8 + i][u], y = v[8 + i][u + 1];
-                    v[8 + i][u] = x * c.x - y * c.y;
-                    v[8 + i][u + 1] = y * c.x + x * c.y;
-                }
-        }
+        rotate(v, reinterpret_cast<const f32x2*>(a.keys + (size_t)(at.first_tile + kp / 32) * record + REC::ANGLES) + (kp % 32) * (kR / 2), a.halves, hf);
 #pragma unroll
         for (int k = 0; k < 6; ++k)
             qf[k] = __builtin_bit_cast(bf16x8, u32x4{cvt_pk_bf16(v[2 * k].x, v[2 * k].y), cvt_pk_bf16(v[2 * k].z, v[2 * k].w), cvt_pk_bf16(v[2 * k + 1].x, v[2 * k + 1].y),
@@ -473,16 +510,141 @@ __global__ __launch_bounds__(256, KW == 1 ? 4 : 2) void latent_heads_kernel(cons
     }
 }
 
+// exp(x) for x <= 0 (x log2 e in two pieces; below what fp32 holds: 0)
+__device__ __forceinline__ float exp_of(float x) {
+    x = x < -150.0f ? -150.0f : x;  // (NaN stays)
+    const float t = x * 1.44269502f, rest = fmaf(x, 1.44269502f, -t) + x * 1.92596303e-8f;
+    const float p = __builtin_amdgcn_exp2f(t);
+    return fmaf(p, rest * 0.693147182f, p);
+}
+
+// 32-bit mode: the same in true fp32 (v_mfma_f32_32x32x2_f32), 32 queries of a head to a workgroup, whose four waves take every fourth tile.  Keys and
+// values go from memory to registers, whole fragments of 1 KB, 20 of them a tile beside 80 products of 64 cycles, which bound it.
+__global__ __launch_bounds__(256, 2) void latent_heads_f32_kernel(const HeadsArgs a) {
+    typedef Record<true> REC;
+    __shared__ __attribute__((aligned(16))) float s_part[4 * 34 * 64];
+    __shared__ __attribute__((aligned(16))) float s_img[32 * (kV + 4)];
+    Entry at;
+    int h = 0, block = 0;
+    if (!find<true>(blockIdx.x, a.ent_start, a.ent_len, a.ent_slot, a.n_entries, a.row_pos, 32, a.H, at, h, block)) return;
+    const int tid = threadIdx.x, lane = tid & 63, r = lane & 31, hf = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q0 = block * 32, nq = min(32, at.len - q0), m_first = at.start + q0, pos_first = at.pos + q0, qpos = pos_first + r, n_tiles = (pos_first + nq + 31) / 32;
+    const size_t record = REC::bytes(a.H), row = (size_t)(m_first + min(r, nq - 1));  // (beyond the block: some valid row, never stored)
+    const char* src = a.keys + (size_t)at.first_tile * record + lane * 16;
+    f32x4 q[12];
+    {
+        const float* qr = a.q + row * a.ldq + (size_t)h * (kD + kR) + 4 * hf;
+#pragma unroll
+        for (int i = 0; i < 12; ++i) q[i] = *reinterpret_cast<const f32x4*>(qr + 8 * i);
+        const int kp = min(qpos, at.pos + at.len - 1);
+        rotate(q, reinterpret_cast<const f32x2*>(a.keys + (size_t)(at.first_tile + kp / 32) * record + REC::ANGLES) + (kp % 32) * (kR / 2), a.halves, hf);
+    }
+    f32x16 o[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) o[t][i] = 0.0f;
+    float mx = -INFINITY, lsum = 0.0f;
+    f32x4 k[12];
+    auto fetch = [&](int kt) {  // (beyond the last tile: the last, not used)
+        const char* g = src + (size_t)min(kt, n_tiles - 1) * record;
+#pragma unroll
+        for (int i = 0; i < 12; ++i) k[i] = *reinterpret_cast<const f32x4*>(g + (i < 8 ? REC::HEADS + (size_t)h * REC::HEAD + i * 1024 : (i - 8) * 1024));
+    };
+    fetch(wave);
+    for (int kt = wave; kt < n_tiles; kt += 4) {
+        f32x4 v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const f32x4*>(src + (size_t)kt * record + REC::HEADS + (size_t)h * REC::HEAD + REC::VALUES + i * 1024);
+        f32x16 s;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 12; ++i)
+#pragma unroll
+            for (int u = 0; u < 4; ++u) s = __builtin_amdgcn_mfma_f32_32x32x2f32(k[i][u], q[i][u], s, 0, 0, 0);
+        fetch(kt + 4);
+        float top = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] *= a.scale;
+        if (kt * 32 + 31 > pos_first) {  // some query does not see the whole tile
+#pragma unroll
+            for (int i = 0; i < 16; ++i)
+                if (kt * 32 + 8 * (i >> 2) + 4 * hf + (i & 3) > qpos) s[i] = -INFINITY;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) top = fmaxf(top, s[i]);
+        top = fmaxf(mx, fmaxf(top, __shfl_xor(top, 32, 64)));
+        if (__any(top > mx)) {
+            const float f = mx == top ? 1.0f : exp_of(mx - top);  // (none so far: 0)
+            lsum *= f;
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) o[t][i] *= f;
+            mx = top;
+        }
+        const float ref = mx == -INFINITY ? 0.0f : mx;
+        float part[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = exp_of(s[i] - ref);
+            part[i & 1] += s[i];
+        }
+        lsum += part[0] + part[1];
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+#pragma unroll
+            for (int t = 0; t < 2; ++t) o[t] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[4 * t + (i >> 2)][i & 3], s[i], o[t], 0, 0, 0);
+    }
+    float* mine = s_part + wave * 34 * 64 + lane;
+    mine[0] = mx;
+    mine[64] = lsum + __shfl_xor(lsum, 32, 64);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mine[(2 + t * 16 + i) * 64] = o[t][i];
+    __syncthreads();
+    float top = -INFINITY, sum = 0.0f, v[8];  // a quarter of the channels to a wave
+#pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, s_part[w * 34 * 64 + lane]);
+    const float ref = top == -INFINITY ? 0.0f : top;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float* p = s_part + w * 34 * 64 + lane;
+        const float f = exp_of(p[0] - ref);
+        sum = fmaf(p[64], f, sum);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = fmaf(p[(2 + 8 * wave + e) * 64], f, v[e]);
+    }
+    const float gf = head_gate_f(a.gate, a.ldg, row, h) * (a.sink ? sink_norm_f(top, sum, a.sink, h) : 1.0f), inv = 1.0f / sum;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {  // channels 16 wave + 8 i + 4 half + ..
+        f32x4 y;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) y[u] = (a.sink ? v[4 * i + u] : quotient(v[4 * i + u], sum, inv)) * gf;
+        *reinterpret_cast<f32x4*>(s_img + r * (kV + 4) + 16 * wave + 8 * i + 4 * hf) = y;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int x = tid; x < 32 * kV / 4; x += 256) {
+        const int qr = x / (kV / 4), c = x % (kV / 4) * 4;
+        if (qr < nq) *reinterpret_cast<f32x4*>(a.out32 + (size_t)(m_first + qr) * a.ldo + h * kV + c) = *reinterpret_cast<const f32x4*>(s_img + qr * (kV + 4) + c);
+    }
+}
+
 }  // namespace
 
-size_t latent_heads_record(int H, int D, int R, int KR, int Vd, int rot_dims) {
-    return D == kD && R == kR && Vd == kV && rot_dims == kR && (KR == 128 || KR == 256) ? record_bytes(H) : 0;
+size_t latent_heads_record(int H, int D, int R, int KR, int Vd, int rot_dims, bool f32) {
+    return D == kD && R == kR && Vd == kV && rot_dims == kR && (KR == 128 || KR == 256) ? (f32 ? Record<true>::bytes(H) : Record<false>::bytes(H)) : 0;
 }
 
 bool latent_heads_fit(const LatentHeads& a) {
     const uintptr_t all = reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.cache) | reinterpret_cast<uintptr_t>(a.ukT) | reinterpret_cast<uintptr_t>(a.uv) |
-                          reinterpret_cast<uintptr_t>(a.ws) | reinterpret_cast<uintptr_t>(a.out);
-    const size_t record = latent_heads_record(a.H, a.D, a.R, a.KR, a.Vd, a.rot.dims);
+                          reinterpret_cast<uintptr_t>(a.ws) | reinterpret_cast<uintptr_t>(a.out) | reinterpret_cast<uintptr_t>(a.out32);
+    const size_t record = latent_heads_record(a.H, a.D, a.R, a.KR, a.Vd, a.rot.dims, a.out32 != nullptr);
     const PortionSize& p = a.size;
     const char* force = getenv("ZGPT2_LM_LATENT_HEADS");  // test hook: -1 never, 1 or 4 that form of the attention at any size
     const int f = force ? atoi(force) : 0;
@@ -491,7 +653,11 @@ bool latent_heads_fit(const LatentHeads& a) {
     // A key costs KR (D + V) products a head whoever sees it, a pair saves 2 KR - D - V.  Portions of few rows behind much are let in as long as that is a
     // short launch: up to 8192 keys of 12 heads (28 us) every shape was faster, whole steps of 9 rows and more on the 12-layer stacks, in the latent space : here,
     // us: 1 x 9 rows behind nothing 909 : 856, behind 1000 1110 : 906, behind 7000 2166 : 1238; 8 x 2 behind 900 1152 : 1069; 8 x 64 behind 256 1399 : 1313.
-    return f > 0 || p.all_keys * a.H <= 8192 * 12 || (double)(p.all_keys - p.rows) * a.KR * (a.D + a.Vd) <= 0.5 * (double)p.pairs * (2 * a.KR - a.D - a.Vd);
+    // In 32-bit mode the keys' launch is dearer (8 x 2 behind 900 1303 : 1326, 8 x 16 behind 900 1482 : 1490, 8 x 64 behind 900 2093 : 1868, 1 x 9 behind 7000
+    // 3023 : 2062, 1 x 9 990 : 967, 1 x 1000 2475 : 1812): there many sequences with few rows stay where they were.
+    const bool f32 = a.out32 != nullptr;
+    const bool brief = p.all_keys * a.H <= 8192 * 12 && (!f32 || p.all_keys * a.H <= 1024 * 12 || p.all_keys <= 2 * p.longest);
+    return f > 0 || brief || (double)(p.all_keys - p.rows) * a.KR * (a.D + a.Vd) <= (f32 ? 2.0 : 0.5) * (double)p.pairs * (2 * a.KR - a.D - a.Vd);
 }
 
 int launch_latent_heads(const LatentHeads& a, hipStream_t s) {
@@ -503,20 +669,23 @@ int launch_latent_heads(const LatentHeads& a, hipStream_t s) {
     const int pairs = (a.H + 1) / 2;
     k.per = (int)std::max(1ll, std::min<long long>(kMostTiles, (long long)p.tiles * pairs * 2 / 512));
     const dim3 kg((unsigned)((p.tiles + k.per - 1) / k.per), (unsigned)pairs, 2);
-    if (a.KR == 128) latent_head_keys_kernel<8><<<kg, 256, 0, s>>>(k);
-    else latent_head_keys_kernel<16><<<kg, 256, 0, s>>>(k);
+    const bool f32 = a.out32 != nullptr;
+    if (a.KR == 128) f32 ? latent_head_keys_kernel<8, true><<<kg, 256, 0, s>>>(k) : latent_head_keys_kernel<8, false><<<kg, 256, 0, s>>>(k);
+    else f32 ? latent_head_keys_kernel<16, true><<<kg, 256, 0, s>>>(k) : latent_head_keys_kernel<16, false><<<kg, 256, 0, s>>>(k);
     ZG_HIP(hipGetLastError());
     HeadsArgs h;
-    h.q = a.q; h.keys = a.ws; h.out = a.out; h.gate = a.gate; h.sink = a.sink; h.ent_start = a.ent_start; h.ent_len = a.ent_len; h.ent_slot = a.ent_slot; h.row_pos = a.row_pos;
+    h.q = a.q; h.keys = a.ws; h.out = a.out; h.out32 = a.out32; h.gate = a.gate; h.sink = a.sink; h.ent_start = a.ent_start; h.ent_len = a.ent_len; h.ent_slot = a.ent_slot; h.row_pos = a.row_pos;
     h.ldq = a.ldq; h.ldo = a.ldo; h.ldg = a.ldg; h.H = a.H; h.n_entries = a.n_entries; h.halves = a.rot.halves; h.scale = a.scale;
     // Blocks of 128 queries once there are some for most compute units.  us a step of the 12-layer stack, 32 : 128 queries (workgroups of the latter): 1 x 1000 rows
     // (96) 1399 : 1445, 8 x 128 behind 800 (96) 1651 : 1672, 8 x 250 (192) 1755 : 1721, 8 x 256 behind 256 (192) 1847 : 1813.
     const char* force = getenv("ZGPT2_LM_LATENT_HEADS");
     const bool wide = force && atoi(force) > 0 ? atoi(force) == 1 : (long long)p.wide_blocks * a.H >= 160;
-    if (wide) latent_heads_kernel<1><<<(unsigned)(p.wide_blocks * a.H), 256, 0, s>>>(h);
+    if (f32) latent_heads_f32_kernel<<<(unsigned)(p.blocks * a.H), 256, 0, s>>>(h);
+    else if (wide) latent_heads_kernel<1><<<(unsigned)(p.wide_blocks * a.H), 256, 0, s>>>(h);
     else latent_heads_kernel<4><<<(unsigned)(p.blocks * a.H), 256, 0, s>>>(h);
     ZG_HIP(hipGetLastError());
-    note_kernel("latent_heads_kernel<%d>", wide ? 1 : 4);
+    if (f32) note_kernel("latent_heads_f32_kernel");
+    else note_kernel("latent_heads_kernel<%d>", wide ? 1 : 4);
     return ZG_OK;
 }
 
