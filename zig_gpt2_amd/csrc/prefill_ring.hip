@@ -2,7 +2,7 @@
 // idle: prompts of some hundred rows.
 //
 // A = the activation planes [M][2 K] (hi | lo), W = the one plane [N][K] of a bf16 weight, or the two [2][N][K] of an fp32 weight (zg_common.h split2_f16).
-// All the products of a K step of 64 columns (two, or three) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
+// All the products of a K step of 64 columns (two, or four; three of an op-tier Linear) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
 // walk an fp32 weight in two passes that each stage the activations again and meet in slabs.
 // What bounds it: a compute unit takes in some 30 bytes a clock (32 KB a step of a 64 x 64 tile of three products: 1100 clocks, beside 384 of
 // products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
@@ -81,6 +81,10 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < PB; ++i) dma_16(to + kPair * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
     };
+    // A prompt's fp32 Linears make the product of the two second terms as well: with 384 columns, where the rest of a sum is near to exact, three products of
+    // a whole small model were further from 64 bits than six of three bf16 terms (2 x 20 tokens 3.1e-7 against 2.6e-7, of eight prompts of 200 2.8 and 2.7;
+    // with the fourth 2.9 and 2.6).  It hides beside the staging: 300 rows 10.3 -> 10.8 us, 14.2 -> 14.2, 13.9 -> 14.1 (1 x 300 tokens 850 -> 866).
+    constexpr bool ALL = NW == 2 && EPI != PF_LINEAR;
     constexpr int NL = TN == 2 ? 1 : 2;  // leading products by the step's parity, or (registers) one sum of four steps
     f32x16 lead[NL][TM][TN], small[TM][TN], total[TM][TN];
 #pragma unroll
@@ -127,6 +131,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
             for (int i = 0; i < TM; ++i)
 #pragma unroll
                 for (int j = 0; j < TN; ++j) {
+                    if constexpr (ALL) one(small[i][j], kk, 1, 1, i, j);
                     one(small[i][j], kk, 1, 0, i, j);
                     one(lead[now][i][j], kk, 0, 0, i, j);
                     if constexpr (NW == 2) one(small[i][j], kk, 0, 1, i, j);
@@ -176,7 +181,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
         __builtin_amdgcn_sched_barrier(0);
         read(std::integral_constant<int, other>(), slot);
         multiply(b);
-        constexpr int products = kCh / 2 * TM * TN * (NW + 1), reads = kCh / 2 * (kPair * TM + NW * TN);
+        constexpr int products = kCh / 2 * TM * TN * (NW + 1 + ALL), reads = kCh / 2 * (kPair * TM + NW * TN);
 #pragma unroll
         for (int x = 0; x < products; ++x) {
             __builtin_amdgcn_sched_group_barrier(0x100, (reads + products - 1) / products, 0);
