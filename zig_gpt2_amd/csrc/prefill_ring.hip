@@ -50,7 +50,10 @@ struct RawRows {
 };
 
 // 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
-template <int EPI, int TM, int TN, int NW, int ST>
+// ALL: a prompt's fp32 Linears make the product of the two second terms as well.  With three products short sums, the rest of which is near to exact, left a small
+// model's logits further from 64 bits than six of three bf16 terms; the fourth hides beside the staging (300 rows 10.3 -> 10.8 us, 14.2 -> 14.2, 13.9 ->
+// 14.1; 1 x 300 tokens 850 -> 866).  NEAR (models of fewer than 512 columns): totals that keep what an addition rounds away, too dear (12.3 us) where sums are longer.
+template <int EPI, int TM, int TN, int NW, int ST, bool NEAR>
 __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
                                                               const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw) {
     constexpr int BM = 64 * TM, BN = 64 * TN, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
@@ -81,9 +84,6 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < PB; ++i) dma_16(to + kPair * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
     };
-    // A prompt's fp32 Linears make the product of the two second terms as well: with 384 columns, where the rest of a sum is near to exact, three products of
-    // a whole small model were further from 64 bits than six of three bf16 terms (2 x 20 tokens 3.1e-7 against 2.6e-7, of eight prompts of 200 2.8 and 2.7;
-    // with the fourth 2.9 and 2.6).  It hides beside the staging: 300 rows 10.3 -> 10.8 us, 14.2 -> 14.2, 13.9 -> 14.1 (1 x 300 tokens 850 -> 866).
     constexpr bool ALL = NW == 2 && EPI != PF_LINEAR;
     constexpr int NL = TN == 2 ? 1 : 2;  // leading products by the step's parity, or (registers) one sum of four steps
     f32x16 lead[NL][TM][TN], small[TM][TN], total[TM][TN];
@@ -93,6 +93,18 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
         for (int j = 0; j < TN; ++j)
 #pragma unroll
             for (int e = 0; e < 16; ++e) lead[0][i][j][e] = lead[NL - 1][i][j][e] = small[i][j][e] = total[i][j][e] = 0.0f;
+    auto gather = [&](f32x16& to, f32x16& from, f32x16& rest) {  // NEAR: what the addition rounds away joins the small products
+        if constexpr (NEAR) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const float t = to[e], y = from[e], sum = t + y, z = sum - t;
+                rest[e] += (t - (sum - z)) + (y - z);
+                to[e] = sum;
+            }
+        } else to += from;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) from[e] = 0.0f;
+    };
     const int fr = lane & 31, kh = lane >> 5, fswz = fr & 7;
     u32x4 af[2][kCh / 2][kPair][TM], bf[2][kCh / 2][NW][TN];  // of the step that is multiplied, and of the one behind it on its way
     auto read = [&](auto b, int slot) {
@@ -120,11 +132,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    total[i][j] += lead[1 - now][i][j];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) lead[1 - now][i][j][e] = 0.0f;
-                }
+                for (int j = 0; j < TN; ++j) gather(total[i][j], lead[1 - now][i][j], small[i][j]);
 #pragma unroll
         for (int kk = 0; kk < kCh / 2; ++kk)
 #pragma unroll
@@ -192,11 +200,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    total[i][j] += lead[0][i][j];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) lead[0][i][j][e] = 0.0f;
-                }
+                for (int j = 0; j < TN; ++j) gather(total[i][j], lead[0][i][j], small[i][j]);
         ++s;
     };
     for (int pairs = steps >> 1; pairs > 0; --pairs) {
@@ -206,6 +210,11 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     if (steps & 1) body(std::integral_constant<int, 0>());
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");  // (the requests behind the last step still write the ring)
     if (TN > 1) fetch_scales();
+    if constexpr (NEAR)
+#pragma unroll
+        for (int ij = 0; ij < TM * TN; ++ij)
+#pragma unroll
+            for (int l = 0; l < NL; ++l) gather(total[ij / TN][ij % TN], lead[l][ij / TN][ij % TN], small[ij / TN][ij % TN]);
 
     // element e of a 32 x 32 tile: column 8 (e / 4) + 4 (lane / 32) + e % 4, row lane % 32.  Every wave turns its rows in an image of its own
     // (its accesses to the LDS are in order), so that eight lanes store 128 bytes of a row.
@@ -257,7 +266,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     }
 }
 
-template <int EPI, int TM, int TN, int NW, int ST>
+template <int EPI, int TM, int TN, int NW, int ST, bool NEAR = false>
 int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s,
                 const RawRows& raw = RawRows{}) {
     constexpr int LDS = ST * (kPair * 64 * TM + NW * 64 * TN) * kRow;
@@ -266,11 +275,11 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
     int device = 0;
     ZG_HIP(hipGetDevice(&device));
     ZG_TRY(raised.run(device, []() -> int {
-        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_ring_kernel<EPI, TM, TN, NW, ST>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
+        ZG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR>), hipFuncAttributeMaxDynamicSharedMemorySize, LDS));
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * ((N + 64 * TN - 1) / (64 * TN));
-    prefill_ring_kernel<EPI, TM, TN, NW, ST><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
+    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -279,6 +288,10 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
 template <int EPI>
 int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int tm, int n_sp, const PrefillQkv& qa, const PlaneOut& po,
                     hipStream_t s) {
+    if (W.planes == 2 && std::min(N, K) < 512)
+        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
+               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
+                         : launch_ring<EPI, 2, 2, 2, 2, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
     if (W.planes == 2)
         return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
                : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
