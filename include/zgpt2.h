@@ -204,9 +204,9 @@ enum {
     ZG_GPT_NO_GRAPH = 1 << 1,    /* launch kernels eagerly instead of replaying a hipGraph */
     ZG_GPT_KV_F16 = 1 << 2,      /* store the KV cache as fp16 instead of fp32 */
     ZG_GPT_NO_PREFILL = 1 << 3,  /* generate: feed prompts one position at a time, as main.zig:331-334 does */
-    ZG_GPT_PREFILL_2PLANE = 1 << 4, /* whole-prompt GEMMs multiply two bf16 planes of the fp32 activations instead of the exact
-                                      three: 2/3 of the matrix work, ~2e-5 of the logit scale (inside the 1e-3 parity bound,
-                                      outside the tests' near-zero floor); bf16-weight handles only */
+    ZG_GPT_PREFILL_2PLANE = 1 << 4, /* whole-prompt GEMMs multiply the fp32 activations rounded to 16 significant bits: ~2e-5 of the
+                                      logit scale (inside the 1e-3 parity bound, outside the tests' near-zero floor);
+                                      bf16-weight handles only */
     ZG_GPT_NO_PREFETCH = 1 << 5, /* zg_gpt_generate_*: no side-stream L2 prefetcher beside the decode chain (results are
                                     identical either way; a measurement switch) */
     ZG_GPT_SAMPLED_GENERATE = 1 << 7, /* capture the decode graphs of zg_gpt_generate_sample_* at create as well (otherwise they are

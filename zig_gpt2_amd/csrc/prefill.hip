@@ -4,7 +4,7 @@
 //
 // Numerics.  Activations stay fp32 values with two-term fp16 planes standing for them in the matrix products (zg_common.h split2_f16: 23 bits), laid
 // out [M][2K] = [hi | lo] and scaled by a power of two that is known from the weights (launch_prefill_bounds); a bf16 weight is one fp16 plane of
-// its row times a power of two, an fp32 weight two.  Products of two planes (bf16 weights) or three (fp32) stand where exact bf16 terms take three and six.
+// its row times a power of two, an fp32 weight two.  Products of two planes (bf16 weights) or three (fp32; four in prefill_ring.hip) stand where exact bf16 terms take three and six.
 // Sums of the leading products are cut into runs that start at zero, so that a result is closer to 64 bits than one chain of
 // exact products.  Attention (attn_prefill.hip) treats q, k, v and the probabilities the same way.
 //
@@ -643,7 +643,7 @@ int launch_ln_split(const float* x, int M, int E, const float* g, const float* b
 }
 
 // Large prompts (several sequences): the Linears run on the persistent four-wave kernel of gemm_s4.hip with the activation
-// planes as plane pairs of ONE K loop (K_eff = 3 K between two epilogues) once its 256 x 192 tiles fill most of the chip; the
+// planes as plane pairs of ONE K loop (K_eff = 2 K, with fp32 weights 3 K, between two epilogues) once its 256 x 192 tiles fill most of the chip; the
 // N = n_embed Linears (residual adds) get there by slicing K over the tile list, their partial slabs summed by the reduce
 // kernels above in fixed order (which also apply bias, residual and the LayerNorm + split that follows).  Returns the slice
 // count, 0 = the 128-row kernels of this file take the launch.

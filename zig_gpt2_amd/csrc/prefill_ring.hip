@@ -4,7 +4,7 @@
 // A = the activation planes [M][2 K] (hi | lo), W = the one plane [N][K] of a bf16 weight, or the two [2][N][K] of an fp32 weight (zg_common.h split2_f16).
 // All the products of a K step of 64 columns (two, or four; three of an op-tier Linear) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
 // walk an fp32 weight in two passes that each stage the activations again and meet in slabs.
-// What bounds it: a compute unit takes in some 30 bytes a clock (32 KB a step of a 64 x 64 tile of three products: 1100 clocks, beside 384 of
+// What bounds it: a compute unit takes in some 30 bytes a clock (32 KB a step of a 64 x 64 tile of an fp32 weight: 1100 clocks, beside 384 or 512 of
 // products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
 // K steps; a step costs one barrier; its fragments were read beside the products of the step before.  The leading products of a step are a sum
 // of their own, added to the steps' before it beside the products of the next, so that neither they nor the small ones are rounded at the size of
