@@ -35,9 +35,9 @@
 // Rotary attention whose passes mix the first such pass's values into their own passes those along in a scratch row per token (every
 // token runs through all passes in one portion): only the mixed values are cached.
 //
-// Latent attention runs in its absorbed form in prompts and in decoding alike: score_j = (W_uk^T q_nope) . c_j + q_rot . k_rot_j,
-// out = W_uv (sum_j p_j c_j) — only the latent c_j and the rotated key part are cached, and a portion of a prompt needs nothing
-// of the tokens before it but their cache rows.
+// Latent attention caches the latent c_j and the rotated key part only, and a portion of a prompt needs nothing of the tokens before it but their
+// cache rows.  Decode steps run in the absorbed form: score_j = (W_uk^T q_nope) . c_j + q_rot . k_rot_j, out = W_uv (sum_j p_j c_j); portions make
+// the heads' keys W_uk c_j and values W_uv c_j first where that pays (lm_latent_heads.hip).
 #include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
