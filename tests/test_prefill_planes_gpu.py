@@ -103,3 +103,41 @@ def test_two_plane_handles_round_their_activations_to_16_bits(zg):
         err.append(np.linalg.norm(m.prefill([toks])[0] - ref) / np.linalg.norm(ref))
         m.close()
     assert err[0] < 2e-6 < err[1] < 1e-4, err
+
+
+@pytest.mark.parametrize("name,batch,n,bf16,route,wgs", [("nano-char", 1, 70, True, 1, 0), ("nano-char", 1, 70, False, 1, 0), ("nano-char", 4, 250, True, 1, 16),
+                                                         ("nano-char", 4, 250, False, 1, 16), ("nano-char", 2, 70, True, 2, 0), ("nano-char", 2, 70, False, 2, 0),
+                                                         ("nano-char", 2, 70, True, 3, 0), ("nano-char", 2, 70, False, 3, 0)])
+def test_rows_of_zeros_and_of_next_to_nothing(zg, monkeypatch, name, batch, n, bf16, route, wgs):
+    """Outputs whose weights are all zero (pruned ones), or so small that nothing is left of them beside the bias, are the bias.  (16 workgroups: 24 tiles of the
+    c_attn Linear, the last eight in halves that meet.)"""
+    cfg = synth.CONFIGS[name]
+    E = cfg.n_embed
+    w = {k: np.array(v, np.float32) for k, v in synth.make_weights(cfg, seed=65, bf16=bf16).items()}
+    rng = np.random.default_rng(65)
+    for l in range(cfg.n_layer):
+        for k, rows in (("c_attn", 3 * E), ("c_fc", 4 * E)):
+            m = w[f"h{l}.{k}_w"].reshape(rows, E)
+            for i, size in enumerate((0.0, 2.0 ** -140, 2.0 ** -118, 2.0 ** -100, 2.0 ** -60, 0.0)):
+                m[i::23] *= np.float32(size)
+            m[7::23] = 0.0
+            w[f"h{l}.{k}_w"] = m
+            w[f"h{l}.{k}_b"] = rng.normal(0.0, 0.05, rows).astype(np.float32)
+        w[f"h{l}.c_proj_w"] = w[f"h{l}.c_proj_w"].reshape(E, E)
+        w[f"h{l}.c_proj_w"][3] = 0.0
+    if wgs:
+        monkeypatch.setenv("ZGPT2_GEMM_WGS", str(wgs))
+    m = zgpt.GPT(cfg, batch=batch, weights_f32=not bf16)
+    m.load_weights(w)
+    toks = np.stack([synth.rand_tokens(650 + b, n + 1, cfg.vocab_size) for b in range(batch)])
+    zg.zg_debug_prefill_route(route, 0)
+    try:
+        lg = m.prefill(toks[:, :n]).copy()
+    finally:
+        zg.zg_debug_prefill_route(0, 0)
+    nxt = m.forward(n + 1, toks[:, n])  # (the cache)
+    m.close()
+    for b in {0, batch - 1}:
+        ref = oracle.GPT(cfg, w).forced_logits(toks[b], n - 1)
+        assert_model_close(ref[0], lg[b], f"rows of zeros, row {b}")
+        assert_model_close(ref[1], nxt[b], f"rows of zeros, decode, row {b}")

@@ -410,7 +410,17 @@ inline int prof_mark(StepProf* p, int cls, hipStream_t s) {
     return ZG_OK;
 }
 
-// (Re)derive the folded-LayerNorm vectors from the weights in the arena: after loading, or on ranks that received
+// a matrix as the whole-prompt GEMMs' planes
+int make_planes(const zg_gpt* g, const void* w, const PrefillW& p, int out, int in, float* norms, const PlaneFloor& floor, hipStream_t s) {
+    uint16_t* planes = const_cast<uint16_t*>(p.p);
+    int* exps = const_cast<int*>(p.exps);
+    if (g->wt != WT_F32) return launch_plane_bf16(static_cast<const bf16_t*>(w), out, in, planes, exps, norms, s, floor);
+    Split2Job j{static_cast<const float*>(w), planes, exps, out, (size_t)out * in, norms};
+    j.floor = floor;
+    return launch_split2(j, Split2Job{}, in, s);
+}
+
+// (Re)derive the folded-LayerNorm vectors and the prompts' planes from the weights in the arena: after loading, or on ranks that received
 // the weight region by broadcast.  A handful of small launches outside any graph.
 int ensure_ln_folded(zg_gpt* g, hipStream_t s) {
     zg_gpt* r = root(g);  // the vectors live in the weight region: one flag per region, kept by its owner
@@ -419,7 +429,13 @@ int ensure_ln_folded(zg_gpt* g, hipStream_t s) {
     for (const zg_layer& y : g->layers) {
         ZG_TRY(launch_ln_fold(y.c_attn_w, g->wt, y.ln_1_g, y.ln_1_b, y.c_attn_b, 3 * E, E, y.c_attn_c2, y.c_attn_c3, s));
         ZG_TRY(launch_ln_fold(y.c_fc_w, g->wt, y.ln_2_g, y.ln_2_b, y.c_fc_b, 4 * E, E, y.c_fc_c2, y.c_fc_c3, s));
-        if (y.exps) ZG_TRY(launch_prefill_bounds(PrefillBounds{y.ln_1_g, y.ln_1_b, y.c_attn_b, y.ln_2_g, y.ln_2_b, y.c_fc_b, y.c_attn_n, y.c_fc_n, y.exps}, E, s));
+        if (!y.exps) continue;
+        ZG_TRY(launch_prefill_bounds(PrefillBounds{y.ln_1_g, y.ln_1_b, y.c_attn_b, y.ln_2_g, y.ln_2_b, y.c_fc_b, y.c_attn_n, y.c_fc_n, y.exps}, E, s));
+        // (again: a row's exponent depends on that of the activations and on its bias)
+        ZG_TRY(make_planes(g, y.c_attn_w, y.c_attn_p, 3 * E, E, nullptr, PlaneFloor{y.exps + PB_LN1, y.c_attn_b}, s));
+        ZG_TRY(make_planes(g, y.c_proj_w, y.c_proj_p, E, E, nullptr, PlaneFloor{y.exps + PB_V, nullptr}, s));
+        ZG_TRY(make_planes(g, y.c_fc_w, y.c_fc_p, 4 * E, E, nullptr, PlaneFloor{y.exps + PB_LN2, y.c_fc_b}, s));
+        ZG_TRY(make_planes(g, y.mlp_proj_w, y.mlp_proj_p, E, 4 * E, nullptr, PlaneFloor{y.exps + PB_GELU, nullptr}, s));
     }
     ZG_TRY(launch_ln_fold(g->wte, g->wt, g->ln_f_g, g->ln_f_b, nullptr, (int)g->cfg.vocab_size, E, g->lm_c2, g->lm_c3, s));
     // handles that share the region run on other streams: the vectors must be complete before any of them reads the flag
@@ -1226,10 +1242,7 @@ int zg_gpt_load_block_tensor(zg_gpt* g, size_t layer, int slot, const float* src
         const PrefillW& p = slot == ZG_C_ATTN_W ? y.c_attn_p : slot == ZG_C_PROJ_W ? y.c_proj_p : slot == ZG_C_FC_W ? y.c_fc_p : y.mlp_proj_p;
         float* norms = slot == ZG_C_ATTN_W ? y.c_attn_n : slot == ZG_C_FC_W ? y.c_fc_n : nullptr;
         const int in = (int)(slot == ZG_MLP_PROJ_W ? 4 * E : E), out = (int)(n / in);
-        uint16_t* planes = const_cast<uint16_t*>(p.p);
-        int* exps = const_cast<int*>(p.exps);
-        if (g->wt == WT_F32) ZG_TRY(launch_split2(Split2Job{reinterpret_cast<const float*>(dst), planes, exps, out, n, norms}, Split2Job{}, in, gs(g)));
-        else ZG_TRY(launch_plane_bf16(reinterpret_cast<const bf16_t*>(dst), out, in, planes, exps, norms, gs(g)));
+        ZG_TRY(make_planes(g, dst, p, out, in, norms, PlaneFloor{}, gs(g)));
         ZG_HIP(hipStreamSynchronize(gs(g)));
     }
     return ZG_OK;

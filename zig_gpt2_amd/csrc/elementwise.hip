@@ -228,6 +228,14 @@ __global__ __launch_bounds__(256) void split3_kernel(const float* __restrict__ i
     }
 }
 
+__device__ __forceinline__ int above_floor(int up, const PlaneFloor& f, int row) {
+    if (f.a == nullptr) return up;
+    const int a = *f.a;
+    int least = -120 - a;
+    if (f.bias != nullptr) least = max(least, (int)(__float_as_uint(f.bias[row]) >> 23 & 255u) - 127 - 90 - a);
+    return min(up, -least);
+}
+
 // Rows of two matrices -> planes of fp16 (zg_common.h split2_f16), a wave a row, its values in registers between the search of the largest and the split
 // (NV quads a lane; rows beyond are read again).  One pass over memory: 8192 x 768 and 3072 x 768 together 69 MB.
 template <int NV>
@@ -256,7 +264,7 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     for (int i = lane + 64 * NV; i < n4; i += 64) widen(*reinterpret_cast<const f32x4*>(x + 4 * i));
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
-    const int up = j.one != nullptr ? -*j.one : split2_exp(top);
+    const int up = j.one != nullptr ? -*j.one : above_floor(split2_exp(top), j.floor, row);
     if (lane == 0) j.exps[row] = -up;
     auto leave = [&](int i, const f32x4& in) {
         const f32x4 q = {ldexpf(in.x, up), ldexpf(in.y, up), ldexpf(in.z, up), ldexpf(in.w, up)};
@@ -299,7 +307,7 @@ __global__ __launch_bounds__(256) void join_planes_kernel(const uint16_t* __rest
 
 // bf16 rows -> one plane, a wave a row (when a matrix is loaded)
 __global__ __launch_bounds__(256) void plane_bf16_kernel(const bf16_t* __restrict__ in, int rows, int K, uint16_t* __restrict__ out, int* __restrict__ exps,
-                                                         float* __restrict__ norms) {
+                                                         float* __restrict__ norms, const PlaneFloor floor) {
     const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6), n2 = K >> 1;
     if (row >= rows) return;
     const uint32_t* x = reinterpret_cast<const uint32_t*>(in + (size_t)row * K);
@@ -311,7 +319,7 @@ __global__ __launch_bounds__(256) void plane_bf16_kernel(const bf16_t* __restric
     }
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
-    const int up = split2_exp(top);
+    const int up = above_floor(split2_exp(top), floor, row);
     if (lane == 0) exps[row] = -up;
     for (int i = lane; i < n2; i += 64) {
         const float a = ldexpf(bf16_lo(x[i]), up), b = ldexpf(bf16_hi(x[i]), up);
@@ -797,9 +805,9 @@ int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int 
     return ZG_OK;
 }
 
-int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s) {
+int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s, const PlaneFloor& floor) {
     ZG_REQUIRE(rows > 0 && K > 0 && K % 2 == 0, ZG_ERR_UNSUPPORTED, "plane_bf16: %d rows of %d", rows, K);
-    plane_bf16_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(in, rows, K, out, exps, norms);
+    plane_bf16_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(in, rows, K, out, exps, norms, floor);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

@@ -109,10 +109,10 @@ __device__ __forceinline__ void split2_f16(float x0, float x1, uint32_t& hi, uin
     hi = __builtin_bit_cast(uint32_t, h);
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(r, f16x2_t));
 }
-// what brings a row whose largest value (as bits without the sign) is `top` to [2^14, 2^15); rows of zeros and of values that are not finite: anything that is finite
+// what brings a row whose largest value (as bits without the sign) is `top` to [2^14, 2^15); rows of zeros: nothing; of values that are not finite: anything that is finite
 __device__ __forceinline__ int split2_exp(uint32_t top) {
     const int e = (int)(top >> 23);
-    return 141 - (e < 1 ? 1 : e);
+    return top == 0 ? 0 : 141 - (e < 1 ? 1 : e);
 }
 
 // An output again as a plain fp32 sum.  The terms of a value that is not finite, or of three bf16 terms one that rounds up to an infinity, meet

@@ -175,6 +175,13 @@ int launch_split3(const float* in, size_t rows, int K, bf16_t* out, hipStream_t 
 // In front of a Linear's products from kSplit2MinK columns on: shorter sums of three exact bf16 terms are closer to 64 bits than two fp16 terms can be
 // (128 columns: 0.64e-7 against 0.98e-7 at best; 512: 1.29e-7 and 1.25e-7; 768: 1.58e-7 and 1.52e-7; 1600: 2.37e-7 and 1.99e-7).
 constexpr size_t kSplit2MinK = 512;
+// A prompt Linear's sums are in units of 2^(a + e), a the exponent of the activations and e of the weight's row: a row's exponent is never so low that its bias leaves
+// fp32's range in those units (where the persistent GEMM starts its sums) or the unit itself does.  What such a row of tiny weights loses lies some 60 binades
+// below the bias, or beyond the smallest fp32 number.
+struct PlaneFloor {
+    const int* a = nullptr;
+    const float* bias = nullptr;
+};
 struct Split2Job {
     const float* in;
     uint16_t* out;
@@ -182,13 +189,14 @@ struct Split2Job {
     int rows;
     size_t lo = 0;           // the second plane lies this many elements behind the first (0: beside it, rows of 2K)
     float* norms = nullptr;  // 2-norms of the rows
-    const int* one = nullptr;  // the exponent of every row; else each gets its own
+    const int* one = nullptr;  // the exponent of every row; else each gets its own, ...
+    PlaneFloor floor;          // ... no lower than this
 };
 // for the test hooks of one Linear and one attention: rows of three bf16 planes -> fp32, rows of two fp16 planes times 2^exp -> three bf16 planes
 int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, float* out, hipStream_t s);
 int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, bf16_t* out, hipStream_t s);
 // bf16 [rows][K] -> one plane of fp16 (a bf16 value has 8 significant bits: exact down to 2^-32 of its row's largest)
-int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s);
+int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s, const PlaneFloor& floor = PlaneFloor{});
 int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s);
 // rows [from_row, ctx) of every (cache, sequence x head) strip set to zero: n_caches caches cache_stride bytes apart, each holding a
 // plane of [strips][ctx] rows of row_bytes at plane_off (api_gpt.hip clear_kv: what a new sequence must not inherit)
