@@ -238,8 +238,9 @@ __device__ __forceinline__ int above_floor(int up, const PlaneFloor& f, int row)
 
 // Rows of two matrices -> planes of fp16 (zg_common.h split2_f16), a wave a row, its values in registers between the search of the largest and the split
 // (NV quads a lane; rows beyond are read again).  One pass over memory: 8192 x 768 and 3072 x 768 together 69 MB.
-template <int NV>
-__global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const Split2Job jb, int K) {
+// SEEN: with the look at the rows (SplitSeen), else with their norms.
+template <int NV, bool SEEN>
+__global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const Split2Job jb, int K, const SplitSeen seen) {
     const int lane = threadIdx.x & 63;
     int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
     if (row >= ja.rows + jb.rows) return;
@@ -266,13 +267,22 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
     const int up = j.one != nullptr ? -*j.one : above_floor(split2_exp(top), j.floor, row);
     if (lane == 0) j.exps[row] = -up;
+    [[maybe_unused]] const uint32_t large_from = __float_as_uint(__uint_as_float(top) * 0.0009765625f);  // 2^-10 of the largest
+    [[maybe_unused]] const uint32_t small_below = up < 140 ? __float_as_uint(ldexpf(1.0f, -2 - up)) : 0u;  // (the smallest numbers there are have no bits below two terms)
+    [[maybe_unused]] int large = 0, small = 0;  // how many, in the first lane
     auto leave = [&](int i, const f32x4& in) {
         const f32x4 q = {ldexpf(in.x, up), ldexpf(in.y, up), ldexpf(in.z, up), ldexpf(in.w, up)};
         uint32_t h0, h1, l0, l1;
         split2_f16(q.x, q.y, h0, l0);
         split2_f16(q.z, q.w, h1, l1);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) ss = fmaf(q[c], q[c], ss);
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (SEEN) {
+                const uint32_t bits = __float_as_uint(in[c]) & 0x7fffffffu;
+                large += __builtin_popcountll(__ballot(bits >= large_from));
+                small += __builtin_popcountll(__ballot(bits < small_below && bits != 0));
+            } else ss = fmaf(q[c], q[c], ss);
+        }
         *reinterpret_cast<u32x2*>(o + 4 * i) = u32x2{h0, h1};
         *reinterpret_cast<u32x2*>(o + lo + 4 * i) = u32x2{l0, l1};
     };
@@ -280,7 +290,21 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     for (int i = 0; i < NV; ++i)
         if (lane + 64 * i < n4) leave(lane + 64 * i, v[i]);
     for (int i = lane + 64 * NV; i < n4; i += 64) leave(i, *reinterpret_cast<const f32x4*>(x + 4 * i));
-    if (j.norms != nullptr) {
+    if constexpr (SEEN) {
+        if (lane != 0) return;
+        auto say = [&](int word) { seen.words[word] = seen.call; };  // (plain stores, merged in the L2s: thousands at agent scope to one line took 7 ns each)
+        const bool few = 64 * small > K;
+        const int mark = top == 0 ? 0 : top >= 0x7f800000u ? MARK_ODD : few || 8 * large < 3 * K ? MARK_UNEVEN | MARK_SPARSE : 4 * large < 3 * K ? MARK_UNEVEN : 0;
+        seen.marks[second ? ja.rows + row : row] = mark;
+        if (mark == 0) return;
+        if (mark == MARK_ODD) {
+            say(SEEN_ODD);
+            return;
+        }
+        say(SEEN_ANY);
+        const int kind = (second ? SEEN_W_UNEVEN : SEEN_X_UNEVEN) + (mark & MARK_SPARSE ? 1 : 0);
+        say(SEEN_ROWS + 16 * kind + row % 16);
+    } else if (j.norms != nullptr) {
         ss = wave_allsum(ss);
         if (lane == 0) j.norms[row] = ldexpf(sqrtf(ss), -up);
     }
@@ -783,11 +807,14 @@ int launch_kv_clear_tail(void* base, int n_caches, size_t cache_stride, size_t p
     return ZG_OK;
 }
 
-int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s) {
+int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s, const SplitSeen& seen) {
     ZG_REQUIRE(K > 0 && K % 4 == 0 && a.rows >= 0 && b.rows >= 0 && a.rows + b.rows > 0, ZG_ERR_UNSUPPORTED, "split2: %d + %d rows of %d", a.rows, b.rows, K);
     const dim3 grid((unsigned)((a.rows + b.rows + 3) / 4));
-    if (K <= 768) split2_kernel<3><<<grid, 256, 0, s>>>(a, b, K);
-    else split2_kernel<8><<<grid, 256, 0, s>>>(a, b, K);
+    if (seen.words != nullptr) {
+        if (K <= 768) split2_kernel<3, true><<<grid, 256, 0, s>>>(a, b, K, seen);
+        else split2_kernel<8, true><<<grid, 256, 0, s>>>(a, b, K, seen);
+    } else if (K <= 768) split2_kernel<3, false><<<grid, 256, 0, s>>>(a, b, K, seen);
+    else split2_kernel<8, false><<<grid, 256, 0, s>>>(a, b, K, seen);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

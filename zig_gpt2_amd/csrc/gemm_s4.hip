@@ -1093,6 +1093,11 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             row_exp = *ex.a;
             ZG_PIN(row_exp);
         }
+        if constexpr (F16 == F16_ROWS)
+            if (seen_refused(ex.seen)) {  // (every wave alike; its requests still write the LDS)
+                asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+                return;
+            }
         if constexpr (KIND == S4_SPLIT2) {
             out_exp = *po.exp;
             ZG_PIN(out_exp);

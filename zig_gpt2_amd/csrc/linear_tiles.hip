@@ -5,6 +5,7 @@
 // the leading one are summed, as the persistent kernel for many rows does (gemm_s4.hip); here no planes are written to memory first, and
 // the tiles are small enough to use the whole chip: 64 x 64, and K in slices over grid.z while there are too few of them (each slice leaves
 // a slab, linear_slabs_kernel adds them).  The leading products have sums of their own, so that the small ones are not rounded at their size.
+#include "prefill_epi.h"
 #include "zg_kernels.h"
 
 #include <algorithm>
@@ -299,16 +300,62 @@ __global__ __launch_bounds__(512) void linear_few_mfma_kernel(const float* __res
     Y[(size_t)om * N + on] = (float)((((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]))) + b);
 }
 
+// The outputs of marked rows of X and of W again: every wave looks through the marks and takes its share of a marked row's outputs, a dot product at a time (one
+// row of 8192 x 768 x 3072: 20 us, half of it the look through the marks).
+constexpr int kMarkedGroups = 512;
+__global__ __launch_bounds__(256) void linear_marked_rows_kernel(const float* __restrict__ X, const float* __restrict__ W, const float* __restrict__ bias, float* __restrict__ Y,
+                                                                 int M, int N, int K, const SplitSeen seen) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)), all = M + N;
+    const SeenPlan p = seen_plan(seen);
+    auto redo = [&](int at) {
+        const bool of_w = at >= M;
+        const int row = of_w ? at - M : at;
+        const float* mine = (of_w ? W : X) + (size_t)row * K;
+        for (int o = wave; o < (of_w ? M : N); o += 4 * kMarkedGroups) {
+            const float* other = (of_w ? X : W) + (size_t)o * K;
+            float s = 0.0f;
+            for (int k = 4 * lane; k < K; k += 256) {
+                const f32x4 a = *reinterpret_cast<const f32x4*>(mine + k), b = *reinterpret_cast<const f32x4*>(other + k);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) s = fmaf(a[e], b[e], s);
+            }
+            s = wave_allsum(s);
+            const int m = of_w ? o : row, n = of_w ? row : o;
+            if (lane == 0) Y[(size_t)m * N + n] = s + (bias ? bias[n] : 0.0f);
+        }
+    };
+    for (int base = 0; base < all; base += 1024) {
+        i32x4 mark[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) mark[u] = reinterpret_cast<const i32x4*>(seen.marks)[min(base / 4 + 64 * u + lane, (all - 1) / 4)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int first = base + 256 * u + e, at = first + 4 * lane;
+                unsigned long long some = __ballot(at < all && (mark[u][e] & (MARK_ODD | (at >= M ? p.w : p.x))) != 0);
+                for (; some != 0; some &= some - 1) redo(first + 4 * __builtin_ctzll(some));
+            }
+    }
+}
+
 }  // namespace
 
-bool linear_tiles_pay(size_t M, size_t N, size_t K) {
+bool linear_tiles_pay(size_t M, size_t N, size_t K, bool planes) {
     // Against the persistent kernel behind its splitting pass, whose time goes by rounds of 256 tiles of 256 x 192 whether they are full or not.
     // From 512 columns on that kernel takes three products of fp16 terms (us of a call, this : that): 768 -> 3072 1023 rows (768 tiles)
     // 50 : 66, 1300 (1008) 62 : 67, 1500 (1152) 69 : 67, 2048 (1536) 83 : 68; 768 -> 1031 4096 rows (1088) 70 : 68; 1600 -> 1600 1500 rows (600) 80 : 101,
     // 2048 (800) 107 : 101; 6400 -> 1600 1500 rows (600) 278 : 337, 2048 (800) 384 : 342; 3072 -> 768 4096 rows (768) 161 : 185, 6000 (1128) 240 : 192.
-    // Below, six of bf16: 128 -> 3072 1856 rows (1392 tiles) and more.
+    // Below, and for rows that are not for two terms, six of bf16: 128 -> 3072 1856 rows (1392 tiles) and more.
     const size_t tiles = ((M + 63) / 64) * ((N + 63) / 64), rounds = (((M + 255) / 256) * ((N + 191) / 192) + 255) / 256;
-    return tiles <= (K < kSplit2MinK ? 1400 : K < 1024 ? 1100 : 800) * rounds;
+    return tiles <= (!planes || K < kSplit2MinK ? 1400 : K < 1024 ? 1100 : 800) * rounds;
+}
+
+int launch_linear_marked_rows(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, const SplitSeen& seen, hipStream_t s) {
+    ZG_REQUIRE(M > 0 && N > 0 && M < (1 << 30) && N < (1 << 30) && K > 0 && K % 4 == 0, ZG_ERR_ARG, "linear: %d x %d x %d", M, N, K);
+    linear_marked_rows_kernel<<<kMarkedGroups, 256, 0, s>>>(X, W, bias, Y, M, N, K, seen);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
 }
 
 int linear_tiles_slices(size_t M, size_t N, size_t K) {

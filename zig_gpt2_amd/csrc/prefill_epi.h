@@ -10,6 +10,43 @@ __device__ __forceinline__ float coarse16(float x) {
     return __uint_as_float((b + 0x7fu + ((b >> 8) & 1u)) & ~0xffu);
 }
 
+// What is to be done about a Linear's rows that are not for two terms (zg_kernels.h SplitSeen): the marks of x and of w whose rows are worked out again, whether
+// the call is refused for them.  (The words are written by the launch in front: scalar loads, which wait for none of the requests in flight.)
+struct SeenPlan {
+    int x, w;
+    bool odd, refused;
+};
+__device__ __forceinline__ SeenPlan seen_plan(const SplitSeen& seen) {
+    typedef const __attribute__((address_space(4))) unsigned* scalar_t;
+    const scalar_t words = (scalar_t)reinterpret_cast<unsigned long long>(seen.words);
+    SeenPlan p{0, 0, words[SEEN_ODD] == seen.call, false};
+    if (words[SEEN_ANY] == seen.call) {
+        int n[4] = {0, 0, 0, 0};
+#pragma unroll 1
+        for (int kind = 0; kind < 4; ++kind) {
+            n[kind] = 0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) n[kind] += words[SEEN_ROWS + 16 * kind + i] == seen.call;
+        }
+        // either way leaves no sparse rows, and uneven ones of one operand only
+        const int uneven_w = n[SEEN_X_SPARSE] + n[SEEN_W_SPARSE] + n[SEEN_W_UNEVEN], uneven_x = n[SEEN_X_SPARSE] + n[SEEN_W_SPARSE] + n[SEEN_X_UNEVEN], rows = min(uneven_w, uneven_x);
+        p.x = rows == 0 ? 0 : uneven_w <= uneven_x ? MARK_SPARSE : MARK_UNEVEN;
+        p.w = rows == 0 ? 0 : uneven_w <= uneven_x ? MARK_UNEVEN : MARK_SPARSE;
+        p.refused = rows > kSeenFew;
+    }
+    return p;
+}
+// ... seen by a kernel of the call; the first workgroup tells the host
+__device__ __forceinline__ bool seen_refused(const SplitSeen& seen) {
+    const SeenPlan p = seen_plan(seen);
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) {
+        if (p.refused) __hip_atomic_store(seen.host, seen.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if ((p.x | p.w) != 0) __hip_atomic_store(seen.host + 1, seen.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (p.odd) __hip_atomic_store(seen.host + 2, seen.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return p.refused;
+}
+
 // four consecutive values -> 8 B into each of the two planes (plane stride `plane` elements), times 2^-exp
 __device__ __forceinline__ void store_split4(uint16_t* dst, size_t plane, f32x4 v, int exp, int coarse) {
     if (coarse) v = f32x4{coarse16(v.x), coarse16(v.y), coarse16(v.z), coarse16(v.w)};

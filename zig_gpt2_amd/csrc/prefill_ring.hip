@@ -171,6 +171,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     };
     if (TN == 1) fetch_scales();  // (larger tiles have no registers for them beside the products)
     const int out_exp = EPI == PF_GELU_SPLIT ? *po.exp : 0;
+    if ((EPI == PF_LINEAR || EPI == PF_PARTIAL) && ex.seen.words != nullptr && seen_refused(ex.seen)) return;
 #pragma unroll
     for (int s = 0; s < ST; ++s) request(s, s);
     if (EPI == PF_QKV) {  // the epilogue's arguments, fetched under the first requests
@@ -268,7 +269,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 
 template <int EPI, int TM, int TN, int NW, int ST, bool NEAR = false>
 int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp, const PrefillQkv& qa, const PlaneOut& po, hipStream_t s,
-                const RawRows& raw = RawRows{}) {
+                const RawRows& raw = RawRows{}, const SplitSeen& seen = SplitSeen{}) {
     constexpr int LDS = ST * (kPair * 64 * TM + NW * 64 * TN) * kRow;
     static_assert(LDS <= 160 * 1024, "the ring fits the LDS");
     static OncePerDevice raised;
@@ -279,7 +280,7 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * ((N + 64 * TN - 1) / (64 * TN));
-    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw);
+    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each, seen}, po, raw);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -287,21 +288,22 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
 
 template <int EPI>
 int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int tm, int n_sp, const PrefillQkv& qa, const PlaneOut& po,
-                    hipStream_t s) {
+                    hipStream_t s, const SplitSeen& seen = SplitSeen{}) {
     if (W.planes == 2 && std::min(N, K) < 512)
-        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
-               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
-                         : launch_ring<EPI, 2, 2, 2, 2, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
+               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
+                         : launch_ring<EPI, 2, 2, 2, 2, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
     if (W.planes == 2)
-        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
-               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s)
-                         : launch_ring<EPI, 2, 2, 2, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
-    return tm == 1 ? launch_ring<EPI, 1, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+        return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
+               : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
+                         : launch_ring<EPI, 2, 2, 2, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
+    return tm == 1 ? launch_ring<EPI, 1, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen) : launch_ring<EPI, 2, 1, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
 }
 
 // the slabs [n_sp][M][Np] of a Linear added, and its bias: a thread four columns of a row
 __global__ __launch_bounds__(256) void linear_ring_finish_kernel(const float* __restrict__ slabs, int n_sp, int M, int Np, const float* __restrict__ bias, float* __restrict__ Y, int N,
-                                                                 const float* __restrict__ X, const float* __restrict__ W, int K) {
+                                                                 const float* __restrict__ X, const float* __restrict__ W, int K, const SplitSeen seen) {
+    if (seen_plan(seen).refused) return;
     const int n4 = (N + 3) / 4;
     const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
     if (i >= (long long)M * n4) return;
@@ -339,36 +341,38 @@ constexpr double kStepUs[4] = {0.0, 0.55, 1.02, 1.85};
 
 size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp) {
     const size_t Np = whole64(N);
-    return whole(M * K * 4) + whole(Np * K * 4) + whole(M * 4) + whole(Np * 4) + (n_sp > 1 ? whole((size_t)n_sp * M * Np * 4) : 0);
+    return whole(M * K * 4) + whole(Np * K * 4) + whole(M * 4) + whole(Np * 4) + whole((M + N) * 4) + (n_sp > 1 ? whole((size_t)n_sp * M * Np * 4) : 0);
 }
 
 static std::atomic<unsigned long long> g_linear_ring_launches{0};
 unsigned long long linear_ring_launch_count() { return g_linear_ring_launches.load(std::memory_order_relaxed); }
 
-int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s) {
+int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, SplitSeen* in, hipStream_t s) {
     const int Np = (int)whole64(N);
     ZG_REQUIRE(M > 0 && N > 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && tm >= 1 && tm <= 3 && (size_t)M * K * 4 < ((size_t)1 << 31) && (size_t)Np * K * 4 < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "linear: %d x %d x %d", M, N, K);
     uint16_t *xp = reinterpret_cast<uint16_t*>(scratch), *wp = reinterpret_cast<uint16_t*>(scratch += whole((size_t)M * K * 4));
     int *xe = reinterpret_cast<int*>(scratch += whole((size_t)Np * K * 4)), *we = reinterpret_cast<int*>(scratch += whole((size_t)M * 4));
-    float* slabs = reinterpret_cast<float*>(scratch += whole((size_t)Np * 4));
+    in->marks = reinterpret_cast<int*>(scratch += whole((size_t)Np * 4));
+    float* slabs = reinterpret_cast<float*>(scratch += whole(((size_t)M + N) * 4));
+    const SplitSeen seen = *in;
     // (the weight's rows beyond N hold whatever the scratch held: their columns are never stored)
-    ZG_TRY(launch_split2(Split2Job{X, xp, xe, M}, Split2Job{W, wp, we, N, (size_t)Np * K}, K, s));
+    ZG_TRY(launch_split2(Split2Job{X, xp, xe, M}, Split2Job{W, wp, we, N, (size_t)Np * K}, K, s, seen));
     const PrefillA A{xp, xe, true};
     const PrefillW P{wp, we, 2};
     g_linear_ring_launches.fetch_add(1, std::memory_order_relaxed);
     if (n_sp == 1) {
         const PrefillQkv none{};
         const RawRows raw{X, W};
-        ZG_TRY(tm == 1   ? (launch_ring<PF_LINEAR, 1, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
-               : tm == 2 ? (launch_ring<PF_LINEAR, 2, 1, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw))
-                         : (launch_ring<PF_LINEAR, 2, 2, 2, 2>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw)));
+        ZG_TRY(tm == 1   ? (launch_ring<PF_LINEAR, 1, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen))
+               : tm == 2 ? (launch_ring<PF_LINEAR, 2, 1, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen))
+                         : (launch_ring<PF_LINEAR, 2, 2, 2, 2>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen)));
         note_kernel("linear_tiles_kernel");  // (the Linears of a medium number of rows have one name; the count says which)
         return ZG_OK;
     }
-    ZG_TRY(launch_prefill_ring(A, P, nullptr, slabs, M, Np, K, Np, PF_PARTIAL, tm, n_sp, PrefillQkv{}, PlaneOut{}, s));
+    ZG_TRY(launch_prefill_ring(A, P, nullptr, slabs, M, Np, K, Np, PF_PARTIAL, tm, n_sp, PrefillQkv{}, PlaneOut{}, s, seen));
     const size_t quads = (size_t)M * ((N + 3) / 4);
-    linear_ring_finish_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(slabs, n_sp, M, Np, bias, Y, N, X, W, K);
+    linear_ring_finish_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(slabs, n_sp, M, Np, bias, Y, N, X, W, K, seen);
     ZG_HIP(hipGetLastError());
     note_kernel("linear_tiles_kernel");
     return ZG_OK;
@@ -441,13 +445,13 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
 }
 
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
-                        const PlaneOut& po, hipStream_t s) {
+                        const PlaneOut& po, hipStream_t s, const SplitSeen& seen) {
     ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kPair * K * 2 < ((size_t)1 << 31) &&
                    (size_t)N * K * 2 * W.planes < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
     switch (epi) {
         case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
-        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, tm, n_sp, qa, po, s);
+        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, tm, n_sp, qa, po, s, seen);
         case PF_GELU_SPLIT: return launch_ring_epi<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
         case PF_QKV: return launch_ring_epi<PF_QKV>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
     }

@@ -182,6 +182,22 @@ struct PlaneFloor {
     const int* a = nullptr;
     const float* bias = nullptr;
 };
+// What the pass over both operands of a Linear saw of their rows.  A value below 2^-17 of its row's largest loses bits in two fp16 terms: 2^-39 of the largest is what is
+// left out.  In a sum of products that is nothing as long as they are few and there are others beside them: three quarters of one operand's row and three
+// eighths of the other's within 2^-10 of their largest value leave an eighth of the products above 2^-20 of the two largest, and what a 64th of the values
+// in either row loses is below 2^-21 of the sum of |x w|.  Rows of normal values, of ReLU or GELU outputs, rows with a value some hundred times the others' are so; a
+// row with one of a million, or of softmax weights, need not be.  Outputs of rows that are not are worked out again: as plain sums where the rows are few, else the kernels
+// leave at once and the call takes exact planes.
+// Words are equal to the call's number where the thing is so; rows are counted by how many of their sixteen words are.
+enum { SEEN_ANY = 0 /* a row that is not even */, SEEN_ODD = 1 /* one with a value that is not finite */, SEEN_ROWS = 16, SEEN_X_UNEVEN = 0, SEEN_X_SPARSE = 1, SEEN_W_UNEVEN = 2,
+       SEEN_W_SPARSE = 3, kSeenWords = SEEN_ROWS + 4 * 16, kSeenFew = 12 };
+enum { MARK_ODD = 1, MARK_UNEVEN = 2 /* fewer than three quarters */, MARK_SPARSE = 4 /* than three eighths, or too many small ones */ };
+struct SplitSeen {
+    unsigned* words = nullptr;
+    unsigned* host = nullptr;  // pinned: [0] the call was refused, [1] it has rows to be worked out again, [2] rows with values that are not finite
+    int* marks = nullptr;      // of x's rows, then w's (in whole fours)
+    unsigned call = 0;
+};
 struct Split2Job {
     const float* in;
     uint16_t* out;
@@ -197,7 +213,7 @@ int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int 
 int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, bf16_t* out, hipStream_t s);
 // bf16 [rows][K] -> one plane of fp16 (a bf16 value has 8 significant bits: exact down to 2^-32 of its row's largest)
 int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s, const PlaneFloor& floor = PlaneFloor{});
-int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s);
+int launch_split2(const Split2Job& a, const Split2Job& b, int K, hipStream_t s, const SplitSeen& seen = SplitSeen{});
 // rows [from_row, ctx) of every (cache, sequence x head) strip set to zero: n_caches caches cache_stride bytes apart, each holding a
 // plane of [strips][ctx] rows of row_bytes at plane_off (api_gpt.hip clear_kv: what a new sequence must not inherit)
 int launch_kv_clear_tail(void* base, int n_caches, size_t cache_stride, size_t plane_off, int row_bytes, int strips, int ctx, int from_row,
@@ -225,10 +241,12 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
                    bool gelu, bool out_bf16, int bn, hipStream_t s);  // gemm_s4.hip
 bool gemm_s4_args_ok(const GemmPlanes& pl, int ldc);            // the bounds of gemm_s4_kernel's packed arguments
 // ... with planes of fp16 (launch_split2): what the sums of output row m and column n are multiplied with, 2^(a[m] + w[n]) (a_each; else a[0] for every row)
+// seen.words != nullptr: nothing is computed where the rows are not for two terms (the caller takes another kernel).
 struct PlaneExps {
     const int* a;
     const int* w;
     bool a_each;
+    SplitSeen seen;
 };
 int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s);
 // ... and its epilogue kinds for the whole-prompt Linears (gemm_s4.hip; PrefillQkv below)
@@ -250,7 +268,9 @@ bool linear_few_ok(size_t M, size_t N, size_t K);
 unsigned long long linear_few_mfma_launch_count();  // launches of linear_few_mfma_kernel so far
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 // Nine rows and more: K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N floats where that is more than one slice.
-bool linear_tiles_pay(size_t M, size_t N, size_t K);
+bool linear_tiles_pay(size_t M, size_t N, size_t K, bool planes);  // planes: beside the persistent GEMM on fp16 planes where it takes them; else on exact bf16 ones
+// Outputs of rows (of X and W) that are not for two terms or have values that are not finite, as plain fp32 sums
+int launch_linear_marked_rows(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, const SplitSeen& seen, hipStream_t s);
 int linear_tiles_slices(size_t M, size_t N, size_t K);
 int launch_linear_tiles(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, float* slabs, hipStream_t s);
 
@@ -311,7 +331,7 @@ int launch_prefill_gemm(const PrefillA& A, const PrefillW& W, const float* bias,
 // prefill_ring.hip: whole-prompt Linears of some hundred rows.  The route: K slices (slabs of a residual Linear, else 1), 0 = not taken; tm: rows / 64 of a tile.
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
-                        const PlaneOut& po, hipStream_t s);
+                        const PlaneOut& po, hipStream_t s, const SplitSeen& seen = SplitSeen{});
 // The exponents of a layer's activations, from its weights: the rows of a normed x are no longer than sqrt(E) max|g| + |b| (b's 2-norm), so no output of
 // a Linear behind it is larger than that times the longest row of its matrix plus its largest bias.  exps: kBounds of them (enum).
 enum { PB_LN1 = 0, PB_Q = 1, PB_K = 2, PB_V = 3, PB_LN2 = 4, PB_GELU = 5, kBounds = 8 };
@@ -326,7 +346,7 @@ int launch_prefill_bounds(const PrefillBounds& b, int E, hipStream_t s);
 int linear_ring_route(size_t M, size_t N, size_t K, int* tm);
 unsigned long long linear_ring_launch_count();  // Linears it has taken so far
 size_t linear_ring_scratch(size_t M, size_t N, size_t K, int n_sp);
-int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, hipStream_t s);
+int launch_linear_ring(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, int tm, int n_sp, char* scratch, SplitSeen* seen, hipStream_t s);  // (seen->marks: set)
 bool prefill_rows_wide(int M, int N, int planes);  // the 128-row kernels' tiles: 256 columns for 128
 void prefill_force_route(int kernel, int slices);  // zg_debug_prefill_route / _linear: pin the GEMM family (1 gemm_s4, 2 the 128-row kernels, 3 prefill_ring) and the K slices
 // out[M][kPair E] = planes of the causal attention of the q / k / v columns of qkv[M][3E], M = B P rows ordered (b, t)

@@ -49,6 +49,9 @@ struct Ctx {
     unsigned* done_flag = nullptr;  // pinned completion word of op-tier calls (d_flag + 8), its sequence number, calls since a real drain
     unsigned done_seq = 0;
     unsigned calls_since_sync = 0;
+    unsigned* split_words = nullptr;  // what the last split of a Linear's operands saw (SplitSeen), its three pinned words (d_flag + 12) and its number
+    unsigned* split_host = nullptr;
+    unsigned split_call = 0;
     int* d_flag = nullptr;         // pinned host int the kernels raise for index-range checks (read after the call's drain)
     float* d_zero = nullptr;       // 64 zero bytes (stand-in operand for absent bias / residual)
     float* attn_part = nullptr;    // op-tier attention partials (sized at init)
@@ -117,6 +120,8 @@ class Call {
     void announced(bool yes) { announced_ = yes; }
     // Copies outputs back (if any were staged), synchronises the stream, releases the arenas.
     int finish();
+    int drain();   // ... its first half: behind it the call may still launch (and is drained again) ...
+    void leave();  // ... and the rest
     hipStream_t stream() const { return s_; }
 
   private:
