@@ -143,7 +143,7 @@ int zg_softmax(float* inputs, size_t inputs_len);
  * only, whose packed arguments end at K = 16320: beyond that ZG_ERR_UNSUPPORTED — zg_linear_forward, which has no such limit,
  * takes such a Linear through its GEMV kernels); K a multiple of 64 and at least 128.  Asynchronous on
  * the library stream.  zg_linear_forward itself takes this path for some thousand rows and more (fp32 operands split
- * into planes — two-term fp16 of scaled rows, or three-term bf16 below 512 columns — so that the result stays fp32-sgemm grade: rows whose values lie too
+ * into planes — two-term fp16 of scaled rows, or three-term bf16 below 640 columns — so that the result stays fp32-sgemm grade: rows whose values lie too
  * far apart for two terms are found in passing and worked out exactly); from nine rows on it splits inside smaller tiles.
  * zg_f32_to_bf16 converts a device or host fp32 array into a device bf16 array (round to nearest even). */
 int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_null, void* C, size_t M,

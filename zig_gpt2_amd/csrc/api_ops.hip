@@ -248,7 +248,7 @@ struct CallGuard {
 
 // Linear.forward on the persistent matrix-core GEMMs, for the sizes that fill the chip with their tiles (16 rows at least; the rule in front
 // is linear_tiles_ok's; ops.zig:21-46 with M = inputs.len / in_features, :22).
-// The op tier is fp32 in, fp32 out, arbitrary fp32 weights.  From 512 columns on both operands become two fp16 planes of rows scaled by powers
+// The op tier is fp32 in, fp32 out, arbitrary fp32 weights.  From 640 columns on both operands become two fp16 planes of rows scaled by powers
 // of two (zg_common.h split2_f16), one pass over both, and the GEMM sums three products: 8192 x 768 x 3072 takes 150 us where six take 214
 // (the GEMM 132 and 190 under the tracer: both at the chip's power limit, where an fp16 product costs more than a bf16 one).
 // Below, and where the four-wave GEMM's arguments end, both operands are split EXACTLY into three bf16

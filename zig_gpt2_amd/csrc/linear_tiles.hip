@@ -343,7 +343,7 @@ __global__ __launch_bounds__(256) void linear_marked_rows_kernel(const float* __
 
 bool linear_tiles_pay(size_t M, size_t N, size_t K, bool planes) {
     // Against the persistent kernel behind its splitting pass, whose time goes by rounds of 256 tiles of 256 x 192 whether they are full or not.
-    // From 512 columns on that kernel takes three products of fp16 terms (us of a call, this : that): 768 -> 3072 1023 rows (768 tiles)
+    // From 640 columns on that kernel takes three products of fp16 terms (us of a call, this : that): 768 -> 3072 1023 rows (768 tiles)
     // 50 : 66, 1300 (1008) 62 : 67, 1500 (1152) 69 : 67, 2048 (1536) 83 : 68; 768 -> 1031 4096 rows (1088) 70 : 68; 1600 -> 1600 1500 rows (600) 80 : 101,
     // 2048 (800) 107 : 101; 6400 -> 1600 1500 rows (600) 278 : 337, 2048 (800) 384 : 342; 3072 -> 768 4096 rows (768) 161 : 185, 6000 (1128) 240 : 192.
     // Below, and for rows that are not for two terms, six of bf16: 128 -> 3072 1856 rows (1392 tiles) and more.

@@ -173,8 +173,9 @@ int launch_split3(const float* in, size_t rows, int K, bf16_t* out, hipStream_t 
 // fp32 [rows][K] of one or two matrices (the second may have none) -> fp16 [rows][2K] = [hi | lo] of the rows times 2^-exps[row], which brings their
 // largest value to [2^14, 2^15): elementwise.hip
 // In front of a Linear's products from kSplit2MinK columns on: shorter sums of three exact bf16 terms are closer to 64 bits than two fp16 terms can be
-// (128 columns: 0.64e-7 against 0.98e-7 at best; 512: 1.29e-7 and 1.25e-7; 768: 1.58e-7 and 1.52e-7; 1600: 2.37e-7 and 1.99e-7).
-constexpr size_t kSplit2MinK = 512;
+// (4096 rows, 3072 outputs: 512 columns 1.27e-7 against 1.34e-7, 576 1.35e-7 and 1.39e-7, 640 1.43e-7 both, 704 1.51e-7 and 1.48e-7, 768 1.58e-7 and 1.52e-7, 1536 2.32e-7 and
+// 1.96e-7; us a call 90 : 66, 95 : 69, 103 : 72, 109 : 76, 117 : 81, 207 : 136).
+constexpr size_t kSplit2MinK = 640;
 // A prompt Linear's sums are in units of 2^(a + e), a the exponent of the activations and e of the weight's row: a row's exponent is never so low that its bias leaves
 // fp32's range in those units (where the persistent GEMM starts its sums) or the unit itself does.  What such a row of tiny weights loses lies some 60 binades
 // below the bias, or beyond the smallest fp32 number.
