@@ -55,8 +55,8 @@ __global__ __launch_bounds__(256) void embed_prefill_kernel(const int* __restric
 }
 
 // ------------------------------------------------------------------------------------------ LayerNorm + split
-// One wave per row.  Same arithmetic as LayerNorm.forward: single pass sum / sum of squares,
-// std = sqrt(E[x^2] - mean^2 + eps), (x - mean) / std * g + b   (src/ops.zig:88-101).
+// One wave per row.  LayerNorm.forward (src/ops.zig:88-101): (x - mean) / std * g + b, with std = sqrt(E[(x - mean)^2] + eps) in place of sqrt(E[x^2] - mean^2 + eps), which
+// cancels where a row's mean is far above its spread: a normed row is then never longer than sqrt(E), which the planes' exponent rests on (launch_prefill_bounds).
 __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__ x, int M, int E,
                                                        const float* __restrict__ g, const float* __restrict__ bta,
                                                        float eps, uint16_t* __restrict__ out, const PlaneOut po) {
@@ -68,12 +68,13 @@ __global__ __launch_bounds__(256) void ln_split_kernel(const float* __restrict__
     for (int e = lane * 4; e < E; e += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(xr + e);
         s += (v.x + v.y) + (v.z + v.w);
-        ss += (v.x * v.x + v.y * v.y) + (v.z * v.z + v.w * v.w);
     }
-    s = wave_allsum(s);
-    ss = wave_allsum(ss);
-    const float mean = s / (float)E;
-    const float sd = sqrtf(ss / (float)E - mean * mean + eps);
+    const float mean = wave_allsum(s) / (float)E;
+    for (int e = lane * 4; e < E; e += 256) {
+        const f32x4 d = *reinterpret_cast<const f32x4*>(xr + e) - mean;
+        ss += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+    }
+    const float sd = sqrtf(wave_allsum(ss) / (float)E + eps);
     uint16_t* hi = out + (size_t)row * kPair * E;
     for (int e = lane * 4; e < E; e += 256) {
         const f32x4 v = *reinterpret_cast<const f32x4*>(xr + e);
@@ -480,20 +481,21 @@ __global__ __launch_bounds__(256) void prefill_reduce_resid_ln_kernel(const floa
             *reinterpret_cast<f32x4*>(xr + e) = a;
             v[j] = a;
             s += (a.x + a.y) + (a.z + a.w);
-            ss += (a.x * a.x + a.y * a.y) + (a.z * a.z + a.w * a.w);
         }
     }
     s = wave_allsum(s);
-    ss = wave_allsum(ss);
-    if ((tid & 63) == 0) {
-        s_red[(tid >> 6) * 2] = s;
-        s_red[(tid >> 6) * 2 + 1] = ss;
-    }
+    if ((tid & 63) == 0) s_red[tid >> 6] = s;
     __syncthreads();
-    s = (s_red[0] + s_red[2]) + (s_red[4] + s_red[6]);
-    ss = (s_red[1] + s_red[3]) + (s_red[5] + s_red[7]);
-    const float mean = s / (float)N;
-    const float sd = sqrtf(ss / (float)N - mean * mean + eps);
+    const float mean = ((s_red[0] + s_red[1]) + (s_red[2] + s_red[3])) / (float)N;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const f32x4 d = tid + 256 * j < n4 ? v[j] - mean : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        ss += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+    }
+    ss = wave_allsum(ss);
+    if ((tid & 63) == 0) s_red[4 + (tid >> 6)] = ss;
+    __syncthreads();
+    const float sd = sqrtf(((s_red[4] + s_red[5]) + (s_red[6] + s_red[7])) / (float)N + eps);  // (ln_split_kernel)
     uint16_t* hi = out + (size_t)row * kPair * N;
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
