@@ -192,3 +192,51 @@ def test_rows_whose_mean_is_far_above_their_spread(zg, name, n, route):
     m.close()
     ref = exact_logits(cfg, w, toks)
     assert np.linalg.norm(got - ref) <= 1e-2 * np.linalg.norm(ref)
+
+
+def trained(cfg, seed, bf16, far):
+    """Gains and rows that differ as a trained model's do: by factors of some e around the usual ones; a channel in a hundred has a gain `far` times the others' and
+    weights that make up for it."""
+    rng = np.random.default_rng(seed)
+    E = cfg.n_embed
+    w = {k: np.array(v, np.float32) for k, v in synth.make_weights(cfg, seed=seed, bf16=bf16).items()}
+    for l in range(cfg.n_layer):
+        p = f"h{l}."
+        for q, behind, rows in (("ln_1", "c_attn", 3 * E), ("ln_2", "c_fc", 4 * E)):
+            g = 0.4 * np.exp(rng.normal(0.0, 1.0, E))
+            at = rng.permutation(E)[:max(1, E // 100)]
+            g[at] *= far
+            w[p + q + "_g"], w[p + q + "_b"] = g.astype(np.float32), rng.normal(0.0, 0.1, E).astype(np.float32)
+            w[p + behind + "_w"] = w[p + behind + "_w"].reshape(rows, E)
+            w[p + behind + "_w"][:, at] /= np.float32(far)
+        for q, o, i in (("c_attn", 3 * E, E), ("c_fc", 4 * E, E), ("c_proj", E, E), ("mlp_proj", E, 4 * E)):
+            m = w[p + q + "_w"].reshape(o, i) * np.exp(rng.normal(0.0, 0.7, o)).astype(np.float32)[:, None]
+            if q == "c_attn":
+                m[:2 * E] *= np.float32(0.5)  # (scores of an ordinary size)
+            if bf16:
+                m = (synth.to_bf16_bits(m).astype(np.uint32) << 16).view(np.float32).reshape(m.shape)
+            w[p + q + "_w"], w[p + q + "_b"] = m, rng.normal(0.0, 0.2, o).astype(np.float32)
+    return w
+
+
+@pytest.mark.parametrize("far", [2.0 ** 5, 2.0 ** 8, 2.0 ** 10])
+@pytest.mark.parametrize("bf16", [True, False])
+@pytest.mark.parametrize("route", [1, 2, 3])
+def test_gains_and_rows_that_differ_as_a_trained_models(zg, far, bf16, route):
+    """The exponents' bounds stay so near to what such layers compute that two terms hold it.  The bound: exact planes of three terms are 1.7e-7 to 3.6e-7 off with these weights."""
+    cfg = synth.CONFIGS["nano-char"]
+    errs = []
+    for seed in (67, 68, 69):
+        w = trained(cfg, seed, bf16, far)
+        toks = synth.rand_tokens(10 * seed, 100, cfg.vocab_size)
+        m = zgpt.GPT(cfg, weights_f32=not bf16)
+        m.load_weights(w)
+        zg.zg_debug_prefill_route(route, 0)
+        try:
+            got = m.prefill([toks])[0].astype(np.float64)
+        finally:
+            zg.zg_debug_prefill_route(0, 0)
+        m.close()
+        ref = exact_logits(cfg, w, toks)
+        errs.append(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+    assert max(errs) <= 4e-7, errs

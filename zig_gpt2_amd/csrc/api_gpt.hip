@@ -27,10 +27,10 @@ using namespace zg;
 
 struct zg_layer {
     void *c_attn_w, *c_proj_w, *c_fc_w, *mlp_proj_w;
-    // the same matrices for the whole-prompt GEMMs (none: ZG_GPT_NO_PREFILL), made when the tensor is loaded; the 2-norms of the rows of the two behind a
-    // LayerNorm, and the exponents of the layer's activations that follow from them (launch_prefill_bounds)
+    // the same matrices for the whole-prompt GEMMs (none: ZG_GPT_NO_PREFILL), bounds on the outputs of the two behind a LayerNorm, and the exponents of the
+    // layer's activations that follow from them (launch_prefill_bounds): all made by ensure_ln_folded
     PrefillW c_attn_p, c_proj_p, c_fc_p, mlp_proj_p;
-    float *c_attn_n, *c_fc_n;
+    double *c_attn_n, *c_fc_n;
     int* exps;
     // LayerNorm folded out of the two LayerNorm-fed Linears (gemv_ksplit.hip, gemv_lnk_kernel): c2 = W g, c3 = W b + bias
     float *c_attn_c2, *c_attn_c3, *c_fc_c2, *c_fc_c3;
@@ -209,8 +209,8 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
             y.c_proj_p = W(E, E);
             y.c_fc_p = W(4 * E, E);
             y.mlp_proj_p = W(E, 4 * E);
-            y.c_attn_n = (float*)P(3 * E * 4);
-            y.c_fc_n = (float*)P(4 * E * 4);
+            y.c_attn_n = (double*)P(3 * E * 8);
+            y.c_fc_n = (double*)P(4 * E * 8);
             y.exps = (int*)P(kBounds * 4);
         }
     }
@@ -411,11 +411,11 @@ inline int prof_mark(StepProf* p, int cls, hipStream_t s) {
 }
 
 // a matrix as the whole-prompt GEMMs' planes
-int make_planes(const zg_gpt* g, const void* w, const PrefillW& p, int out, int in, float* norms, const PlaneFloor& floor, hipStream_t s) {
+int make_planes(const zg_gpt* g, const void* w, const PrefillW& p, int out, int in, const PlaneFloor& floor, hipStream_t s) {
     uint16_t* planes = const_cast<uint16_t*>(p.p);
     int* exps = const_cast<int*>(p.exps);
-    if (g->wt != WT_F32) return launch_plane_bf16(static_cast<const bf16_t*>(w), out, in, planes, exps, norms, s, floor);
-    Split2Job j{static_cast<const float*>(w), planes, exps, out, (size_t)out * in, norms};
+    if (g->wt != WT_F32) return launch_plane_bf16(static_cast<const bf16_t*>(w), out, in, planes, exps, nullptr, s, floor);
+    Split2Job j{static_cast<const float*>(w), planes, exps, out, (size_t)out * in};
     j.floor = floor;
     return launch_split2(j, Split2Job{}, in, s);
 }
@@ -430,12 +430,13 @@ int ensure_ln_folded(zg_gpt* g, hipStream_t s) {
         ZG_TRY(launch_ln_fold(y.c_attn_w, g->wt, y.ln_1_g, y.ln_1_b, y.c_attn_b, 3 * E, E, y.c_attn_c2, y.c_attn_c3, s));
         ZG_TRY(launch_ln_fold(y.c_fc_w, g->wt, y.ln_2_g, y.ln_2_b, y.c_fc_b, 4 * E, E, y.c_fc_c2, y.c_fc_c3, s));
         if (!y.exps) continue;
-        ZG_TRY(launch_prefill_bounds(PrefillBounds{y.ln_1_g, y.ln_1_b, y.c_attn_b, y.ln_2_g, y.ln_2_b, y.c_fc_b, y.c_attn_n, y.c_fc_n, y.exps}, E, s));
-        // (again: a row's exponent depends on that of the activations and on its bias)
-        ZG_TRY(make_planes(g, y.c_attn_w, y.c_attn_p, 3 * E, E, nullptr, PlaneFloor{y.exps + PB_LN1, y.c_attn_b}, s));
-        ZG_TRY(make_planes(g, y.c_proj_w, y.c_proj_p, E, E, nullptr, PlaneFloor{y.exps + PB_V, nullptr}, s));
-        ZG_TRY(make_planes(g, y.c_fc_w, y.c_fc_p, 4 * E, E, nullptr, PlaneFloor{y.exps + PB_LN2, y.c_fc_b}, s));
-        ZG_TRY(make_planes(g, y.mlp_proj_w, y.mlp_proj_p, E, 4 * E, nullptr, PlaneFloor{y.exps + PB_GELU, nullptr}, s));
+        ZG_TRY(launch_row_bounds(y.c_attn_w, g->wt, y.ln_1_g, y.ln_1_b, y.c_attn_b, 3 * E, E, y.c_attn_n, s));
+        ZG_TRY(launch_row_bounds(y.c_fc_w, g->wt, y.ln_2_g, y.ln_2_b, y.c_fc_b, 4 * E, E, y.c_fc_n, s));
+        ZG_TRY(launch_prefill_bounds(PrefillBounds{y.ln_1_g, y.ln_1_b, y.ln_2_g, y.ln_2_b, y.c_attn_n, y.c_fc_n, y.exps}, E, s));
+        ZG_TRY(make_planes(g, y.c_attn_w, y.c_attn_p, 3 * E, E, PlaneFloor{y.exps + PB_LN1, y.c_attn_b}, s));
+        ZG_TRY(make_planes(g, y.c_proj_w, y.c_proj_p, E, E, PlaneFloor{y.exps + PB_V, nullptr}, s));
+        ZG_TRY(make_planes(g, y.c_fc_w, y.c_fc_p, 4 * E, E, PlaneFloor{y.exps + PB_LN2, y.c_fc_b}, s));
+        ZG_TRY(make_planes(g, y.mlp_proj_w, y.mlp_proj_p, E, 4 * E, PlaneFloor{y.exps + PB_GELU, nullptr}, s));
     }
     ZG_TRY(launch_ln_fold(g->wte, g->wt, g->ln_f_g, g->ln_f_b, nullptr, (int)g->cfg.vocab_size, E, g->lm_c2, g->lm_c3, s));
     // handles that share the region run on other streams: the vectors must be complete before any of them reads the flag
@@ -1237,15 +1238,7 @@ int zg_gpt_load_block_tensor(zg_gpt* g, size_t layer, int slot, const float* src
     }
     ZG_REQUIRE(len == n, ZG_ERR_SHAPE, "block slot %d expects %zu elements, got %zu", slot, n, len);
     g->ln_folded = false;
-    ZG_TRY(upload_f32(src, n, dst, mat && g->wt == WT_BF16, gs(g)));
-    if (mat && y.exps) {  // planes for the whole-prompt GEMMs
-        const PrefillW& p = slot == ZG_C_ATTN_W ? y.c_attn_p : slot == ZG_C_PROJ_W ? y.c_proj_p : slot == ZG_C_FC_W ? y.c_fc_p : y.mlp_proj_p;
-        float* norms = slot == ZG_C_ATTN_W ? y.c_attn_n : slot == ZG_C_FC_W ? y.c_fc_n : nullptr;
-        const int in = (int)(slot == ZG_MLP_PROJ_W ? 4 * E : E), out = (int)(n / in);
-        ZG_TRY(make_planes(g, dst, p, out, in, norms, PlaneFloor{}, gs(g)));
-        ZG_HIP(hipStreamSynchronize(gs(g)));
-    }
-    return ZG_OK;
+    return upload_f32(src, n, dst, mat && g->wt == WT_BF16, gs(g));
 }
 
 int zg_gpt_load_tensor(zg_gpt* g, int slot, const float* src, size_t len) {

@@ -356,44 +356,54 @@ __global__ __launch_bounds__(256) void plane_bf16_kernel(const bf16_t* __restric
     if (lane == 0 && norms != nullptr) norms[row] = ldexpf(sqrtf(ss), -up);
 }
 
-// one workgroup: the exponents of a layer's activations (PrefillBounds); bounds go to [2^11, 2^12), so that values four binades beyond (a row whose
-// variance is cancelled away in 32 bits) still are fp16 numbers
+// a wave a row: sqrt(E) |g w| + |w b + bias|, the most an output behind a LayerNorm can be (PrefillBounds), in 64 bits (any row of fp32 numbers has a bound then)
+template <typename WT>
+__global__ __launch_bounds__(256) void row_bounds_kernel(const WT* __restrict__ W, const float* __restrict__ g, const float* __restrict__ b, const float* __restrict__ bias, int rows, int E,
+                                                         double* __restrict__ out) {
+    const int lane = threadIdx.x & 63, row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    if (row >= rows) return;
+    const WT* w = W + (size_t)row * E;
+    double ss = 0.0, at = 0.0;
+    for (int k = lane; k < E; k += 64) {
+        double v;
+        if constexpr (sizeof(WT) == 2) v = (double)__uint_as_float((uint32_t)w[k] << 16);
+        else v = (double)w[k];
+        ss += v * g[k] * (v * g[k]);
+        at += v * b[k];
+    }
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) {
+        ss += __shfl_xor(ss, d, 64);
+        at += __shfl_xor(at, d, 64);
+    }
+    if (lane == 0) out[row] = sqrt((double)E * ss) + fabs(at + (double)bias[row]);
+}
+
+// one workgroup: the exponents of a layer's activations (PrefillBounds); bounds go to [2^14, 2^15): another binade is left for what 32 bits round
 __global__ __launch_bounds__(256) void prefill_bounds_kernel(const PrefillBounds a, int E) {
-    __shared__ float s_red[4];
-    auto all = [&](float v, bool sum) {
-        v = sum ? wave_allsum(v) : wave_allmax(v);
-        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = v;
-        __syncthreads();
-        const float r = sum ? (s_red[0] + s_red[1]) + (s_red[2] + s_red[3]) : fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-        __syncthreads();
-        return r;
-    };
-    auto most = [&](const float* p, int n) {  // the largest that is finite
-        float m = 0.0f;
-        for (int i = threadIdx.x; i < n; i += 256) m = fmaxf(m, fabsf(p[i]) < INFINITY ? fabsf(p[i]) : 0.0f);
-        return all(m, false);
-    };
-    auto length = [&](const float* p, int n) {
-        const float m = most(p, n);
-        float t = 0.0f;
+    __shared__ double s_red[4];
+    auto most = [&](auto value, int n) {  // the largest that is finite
+        double m = 0.0;
         for (int i = threadIdx.x; i < n; i += 256) {
-            const float v = m > 0.0f && fabsf(p[i]) < INFINITY ? p[i] / m : 0.0f;
-            t += v * v;
+            const double v = value(i);
+            if (v < INFINITY && v > m) m = v;
         }
-        return m * sqrtf(all(t, true));
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) m = fmax(m, __shfl_xor(m, d, 64));
+        if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = m;
+        __syncthreads();
+        m = fmax(fmax(s_red[0], s_red[1]), fmax(s_red[2], s_red[3]));
+        __syncthreads();
+        return m;
     };
-    auto set = [&](int which, float bound) {
-        if (threadIdx.x != 0) return;
-        // (no bound, or one beyond fp32's range: the planes are what they are without a factor of more than 2^+-100)
-        const int e = bound > 0.0f ? (int)((__float_as_uint(fminf(bound, 3.0e38f)) >> 23) & 255u) - 127 : 0;
-        a.exps[which] = min(max(e - 11, -100), 100);
+    auto set = [&](int which, double bound) {
+        if (threadIdx.x == 0) a.exps[which] = bound > 0.0 ? min(max(ilogb(bound) - 14, -100), 100) : 0;  // (beyond fp32's range: a factor of 2^+-100 at most)
     };
-    const float r = sqrtf((float)E);
-    const float a1 = r * most(a.ln_1_g, E) + length(a.ln_1_b, E), a2 = r * most(a.ln_2_g, E) + length(a.ln_2_b, E);
-    set(PB_LN1, a1);
-    set(PB_LN2, a2);
-    for (int p = 0; p < 3; ++p) set(PB_Q + p, a1 * most(a.c_attn_norms + p * E, E) + most(a.c_attn_b + p * E, E));
-    set(PB_GELU, a2 * most(a.c_fc_norms, 4 * E) + most(a.c_fc_b, 4 * E));
+    const double r = sqrt((double)E);
+    set(PB_LN1, most([&](int i) { return r * fabs((double)a.ln_1_g[i]) + fabs((double)a.ln_1_b[i]); }, E));
+    set(PB_LN2, most([&](int i) { return r * fabs((double)a.ln_2_g[i]) + fabs((double)a.ln_2_b[i]); }, E));
+    for (int p = 0; p < 3; ++p) set(PB_Q + p, most([&](int i) { return a.c_attn_rows[p * E + i]; }, E));
+    set(PB_GELU, most([&](int i) { return a.c_fc_rows[i]; }, 4 * E));
 }
 
 __device__ __forceinline__ float load_emb(const void* w, int wt, size_t off) {
@@ -835,6 +845,14 @@ int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int 
 int launch_plane_bf16(const bf16_t* in, int rows, int K, uint16_t* out, int* exps, float* norms, hipStream_t s, const PlaneFloor& floor) {
     ZG_REQUIRE(rows > 0 && K > 0 && K % 2 == 0, ZG_ERR_UNSUPPORTED, "plane_bf16: %d rows of %d", rows, K);
     plane_bf16_kernel<<<dim3((unsigned)((rows + 3) / 4)), 256, 0, s>>>(in, rows, K, out, exps, norms, floor);
+    ZG_HIP(hipGetLastError());
+    return ZG_OK;
+}
+
+int launch_row_bounds(const void* W, int weight_type, const float* g, const float* b, const float* bias, int rows, int E, double* out, hipStream_t s) {
+    const dim3 grid((unsigned)((rows + 3) / 4));
+    if (weight_type == WT_BF16) row_bounds_kernel<<<grid, 256, 0, s>>>(static_cast<const bf16_t*>(W), g, b, bias, rows, E, out);
+    else row_bounds_kernel<<<grid, 256, 0, s>>>(static_cast<const float*>(W), g, b, bias, rows, E, out);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }

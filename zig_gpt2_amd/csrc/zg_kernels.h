@@ -333,14 +333,17 @@ int launch_prefill_gemm(const PrefillA& A, const PrefillW& W, const float* bias,
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
                         const PlaneOut& po, hipStream_t s, const SplitSeen& seen = SplitSeen{});
-// The exponents of a layer's activations, from its weights: the rows of a normed x are no longer than sqrt(E) max|g| + |b| (b's 2-norm), so no output of
-// a Linear behind it is larger than that times the longest row of its matrix plus its largest bias.  exps: kBounds of them (enum).
+// The exponents of a layer's activations, from its weights: of a normed x g + b, with x's rows no longer than sqrt(E), column e is no larger than sqrt(E) |g_e| + |b_e|, and
+// an output of a Linear behind it no larger than sqrt(E) |g w| + |w b + bias| (2-norm over the row's columns; launch_row_bounds).  Bounds that hold for
+// any input, and no looser than they have to be: a trained layer's gains and rows differ by factors of ten and more, and what lies far below its bound has
+// fewer bits (2^-17 of the bound and more: all of two terms; below, 2^-40 of the bound is left out).  exps: kBounds of them (enum).
 enum { PB_LN1 = 0, PB_Q = 1, PB_K = 2, PB_V = 3, PB_LN2 = 4, PB_GELU = 5, kBounds = 8 };
 struct PrefillBounds {
-    const float *ln_1_g, *ln_1_b, *c_attn_b, *ln_2_g, *ln_2_b, *c_fc_b;
-    const float *c_attn_norms, *c_fc_norms;  // 2-norms of the rows (launch_split2, launch_plane_bf16)
+    const float *ln_1_g, *ln_1_b, *ln_2_g, *ln_2_b;
+    const double *c_attn_rows, *c_fc_rows;  // bounds on the outputs (launch_row_bounds)
     int* exps;
 };
+int launch_row_bounds(const void* W, int weight_type, const float* g, const float* b, const float* bias, int rows, int E, double* out, hipStream_t s);
 int launch_prefill_bounds(const PrefillBounds& b, int E, hipStream_t s);
 // ... and the fp32 Linears of the op tier with some hundred rows on the same kernel, behind a pass that splits both operands.  The route: slices of K (0: not taken), tm
 // as above; scratch: linear_ring_scratch bytes.
