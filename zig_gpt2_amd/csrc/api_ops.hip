@@ -291,7 +291,7 @@ static int linear_mfma(Call& call, size_t in_f, size_t out_f, const float* w, co
         *seen = next_split();
         ZG_TRY(call.scratch(m + out_f + 4, &seen->marks));
         ZG_TRY(launch_split2(Split2Job{x, xs, xe, (int)m}, Split2Job{w, ws, we, (int)out_f}, (int)in_f, call.stream(), *seen));
-        return launch_gemm_s4_f16(xs, ws, bias, y, (int)m, (int)out_f, p2, (int)out_f, PlaneExps{xe, we, true, *seen}, call.stream());
+        return launch_gemm_s4_f16(xs, ws, bias, y, (int)m, (int)out_f, p2, (int)out_f, PlaneExps{xe, we, true}, *seen, call.stream());
     }
     bf16_t *xp, *wp;
     ZG_TRY(call.scratch(m * in_f * 3, &xp));

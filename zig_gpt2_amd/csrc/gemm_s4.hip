@@ -220,7 +220,7 @@ enum { F16_NO = 0, F16_ONE = 1, F16_ROWS = 2 };
 template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, int F16 = F16_NO>
 __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ B,
                                                          const float* __restrict__ bias, void* __restrict__ C, int M, int N,
-                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex, const PlaneOut po) {
+                                                         unsigned p0, unsigned p1, unsigned p2, unsigned p3, const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const SplitSeen seen) {
     // All 14 dwords of the arguments are preloaded into SGPRs at wave launch (zg_common.h ZG_PIN): the first version passed the
     // plane description and the tile counts behind them and began with a scalar round trip to the kernarg segment — cold for
     // every launch — before its first DMA.  p0 = lda | ldb << 16; p1 = ldc | K-steps per plane << 20 | plane pairs << 28;
@@ -1094,7 +1094,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             ZG_PIN(row_exp);
         }
         if constexpr (F16 == F16_ROWS)
-            if (seen_refused(ex.seen)) {  // (every wave alike; its requests still write the LDS)
+            if (seen_refused(seen)) {  // (every wave alike; its requests still write the LDS)
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 return;
             }
@@ -1162,7 +1162,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
 
 template <int NT, int KIND, bool GELU, bool OUT_BF16, bool SK = false, int F16 = F16_NO>
 int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, int n_sl,
-                  const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}, const PlaneOut& po = PlaneOut{}) {
+                  const PrefillQkv& qa, hipStream_t s, const PlaneExps& ex = PlaneExps{}, const PlaneOut& po = PlaneOut{}, const SplitSeen& seen = SplitSeen{}) {
     using P = S4<NT>;
     constexpr int LDS = F16 != 0 ? P::LDS_F16 : P::LDS;
     static OncePerDevice raised;  // (handles of the layered tier may be on different devices)
@@ -1190,7 +1190,7 @@ int launch_s4_kind(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
     }
     hipLaunchKernelGGL((gemm_s4_kernel<NT, KIND, GELU, OUT_BF16, SK, F16>), dim3(grid), dim3(256), LDS, s, A, B, bias, C, M, N,
                        (unsigned)pl.lda | ((unsigned)pl.ldb << 16), (unsigned)ldc | ((unsigned)pl.kpp << 20) | ((unsigned)pl.npairs << 28),
-                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa, ex, po);
+                       pa2 | (pb2 << 12) | ((unsigned)gw << 24), (unsigned)grid | (dbg << 10) | ((unsigned)n_sl << 20) | (pl.b_plane_major ? 0x80000000u : 0u), qa, ex, po, seen);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
 }
@@ -1245,13 +1245,14 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
     return launch_s4_nt<3>(A, B, bias, C, M, N, pl, ldc, gelu, out_bf16, s);
 }
 
-int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s) {
+int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, const SplitSeen& seen,
+                       hipStream_t s) {
     const PrefillQkv none{};
     ZG_REQUIRE((size_t)M * ldc * 4 < ((size_t)1 << 32) && (size_t)M * pl.lda < (1u << 30) && (size_t)N * pl.ldb < (1u << 30), ZG_ERR_SHAPE,
                "gemm: operands of %d x %d x %d beyond the 32-bit buffer descriptors", M, N, pl.kpp * 64);
     gemm_note_launch();
     note_kernel("gemm_s4_kernel");
-    return launch_s4_kind<3, S4_PLAIN, false, false, false, F16_ROWS>(A, B, bias, C, M, N, pl, ldc, 1, none, s, ex);
+    return launch_s4_kind<3, S4_PLAIN, false, false, false, F16_ROWS>(A, B, bias, C, M, N, pl, ldc, 1, none, s, ex, PlaneOut{}, seen);
 }
 
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s) {

@@ -49,13 +49,13 @@ struct RawRows {
     const float *x, *w;
 };
 
-// 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL).
+// 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL, PF_LINEAR_PART).
 // ALL: a prompt's fp32 Linears make the product of the two second terms as well.  With three products short sums, the rest of which is near to exact, left a small
 // model's logits further from 64 bits than six of three bf16 terms; the fourth hides beside the staging (300 rows 10.3 -> 10.8 us, 14.2 -> 14.2, 13.9 ->
 // 14.1; 1 x 300 tokens 850 -> 866).  NEAR (models of fewer than 512 columns): totals that keep what an addition rounds away, too dear (12.3 us) where sums are longer.
 template <int EPI, int TM, int TN, int NW, int ST, bool NEAR>
 __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
-                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw) {
+                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw, const SplitSeen seen) {
     constexpr int BM = 64 * TM, BN = 64 * TN, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
     constexpr int REQ = kPair * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
     extern __shared__ __attribute__((aligned(1024))) char s_ring[];
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
                 if (bias)
 #pragma unroll
                     for (int e = 0; e < 4; ++e) bv[j][e] = bias[min(n + e, ldc - 1)];
-            } else if (EPI != PF_PARTIAL && bias) {
+            } else if (EPI != PF_PARTIAL && EPI != PF_LINEAR_PART && bias) {
                 bv[j] = *reinterpret_cast<const f32x4*>(bias + n);
             }
         }
@@ -171,11 +171,14 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
     };
     if (TN == 1) fetch_scales();  // (larger tiles have no registers for them beside the products)
     const int out_exp = EPI == PF_GELU_SPLIT ? *po.exp : 0;
-    if ((EPI == PF_LINEAR || EPI == PF_PARTIAL) && ex.seen.words != nullptr && seen_refused(ex.seen)) return;
 #pragma unroll
     for (int s = 0; s < ST; ++s) request(s, s);
     if (EPI == PF_QKV) {  // the epilogue's arguments, fetched under the first requests
         ZG_PIN(qa.P); ZG_PIN(qa.E); ZG_PIN(qa.H); ZG_PIN(qa.ctx); ZG_PIN(qa.kv_mode); ZG_PIN(qa.kv_lo); ZG_PIN(qa.k_cache); ZG_PIN(qa.v_cache);
+    }
+    if ((EPI == PF_LINEAR || EPI == PF_LINEAR_PART) && seen_refused(seen)) {  // (every wave alike; its requests still write the ring)
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
     }
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0), said to the compiler: with scalar loads in flight it would wait for all fragments at once
     arrive<(ST - 1) * REQ>();
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll 1
                     for (int e = 0; e < 4; ++e)
                         if (n + e < ldc && odd(v[e]) > 0.0f) y[e] = plain_sum(raw.x + (size_t)m * K, raw.w + (size_t)(n + e) * K, K) + bv[j][e];
-            } else if constexpr (EPI == PF_PARTIAL) {  // C: slabs [n_sp][M][N]
+            } else if constexpr (EPI == PF_PARTIAL || EPI == PF_LINEAR_PART) {  // C: slabs [n_sp][M][N]
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + ((size_t)blockIdx.y * M + m) * N + n) = v;
             } else {
                 *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(C) + (size_t)m * ldc + n) = v;
@@ -280,7 +283,7 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * ((N + 64 * TN - 1) / (64 * TN));
-    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each, seen}, po, raw);
+    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw, seen);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
@@ -297,7 +300,8 @@ int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, voi
         return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
                : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
                          : launch_ring<EPI, 2, 2, 2, 2>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
-    return tm == 1 ? launch_ring<EPI, 1, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen) : launch_ring<EPI, 2, 1, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
+    if constexpr (EPI == PF_LINEAR_PART) ZG_REQUIRE(false, ZG_ERR_ARG, "linear: %d planes", W.planes);
+    else return tm == 1 ? launch_ring<EPI, 1, 1, 1, 5>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s) : launch_ring<EPI, 2, 1, 1, 3>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
 }
 
 // the slabs [n_sp][M][Np] of a Linear added, and its bias: a thread four columns of a row
@@ -370,7 +374,7 @@ int launch_linear_ring(const float* X, const float* W, const float* bias, float*
         note_kernel("linear_tiles_kernel");  // (the Linears of a medium number of rows have one name; the count says which)
         return ZG_OK;
     }
-    ZG_TRY(launch_prefill_ring(A, P, nullptr, slabs, M, Np, K, Np, PF_PARTIAL, tm, n_sp, PrefillQkv{}, PlaneOut{}, s, seen));
+    ZG_TRY(launch_ring_epi<PF_LINEAR_PART>(A, P, nullptr, slabs, M, Np, K, Np, tm, n_sp, PrefillQkv{}, PlaneOut{}, s, seen));
     const size_t quads = (size_t)M * ((N + 3) / 4);
     linear_ring_finish_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(slabs, n_sp, M, Np, bias, Y, N, X, W, K, seen);
     ZG_HIP(hipGetLastError());
@@ -445,13 +449,13 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
 }
 
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
-                        const PlaneOut& po, hipStream_t s, const SplitSeen& seen) {
+                        const PlaneOut& po, hipStream_t s) {
     ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kPair * K * 2 < ((size_t)1 << 31) &&
                    (size_t)N * K * 2 * W.planes < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
     switch (epi) {
         case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
-        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, tm, n_sp, qa, po, s, seen);
+        case PF_PARTIAL: return launch_ring_epi<PF_PARTIAL>(A, W, nullptr, C, M, N, K, ldc, tm, n_sp, qa, po, s);
         case PF_GELU_SPLIT: return launch_ring_epi<PF_GELU_SPLIT>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
         case PF_QKV: return launch_ring_epi<PF_QKV>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);
     }

@@ -242,14 +242,13 @@ int launch_gemm_s4(const bf16_t* A, const bf16_t* B, const float* bias, void* C,
                    bool gelu, bool out_bf16, int bn, hipStream_t s);  // gemm_s4.hip
 bool gemm_s4_args_ok(const GemmPlanes& pl, int ldc);            // the bounds of gemm_s4_kernel's packed arguments
 // ... with planes of fp16 (launch_split2): what the sums of output row m and column n are multiplied with, 2^(a[m] + w[n]) (a_each; else a[0] for every row)
-// seen.words != nullptr: nothing is computed where the rows are not for two terms (the caller takes another kernel).
 struct PlaneExps {
     const int* a;
     const int* w;
     bool a_each;
-    SplitSeen seen;
 };
-int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, hipStream_t s);
+int launch_gemm_s4_f16(const uint16_t* A, const uint16_t* B, const float* bias, float* C, int M, int N, const GemmPlanes& pl, int ldc, const PlaneExps& ex, const SplitSeen& seen,
+                       hipStream_t s);  // (nothing is computed of a call that is refused: SplitSeen)
 // ... and its epilogue kinds for the whole-prompt Linears (gemm_s4.hip; PrefillQkv below)
 enum { S4_PLAIN = 0, S4_PARTIAL = 1, S4_QKV = 2, S4_SPLIT2 = 3, S4_RELU2 = 4 };
 int launch_gemm_s4_relu2(const bf16_t* A, const bf16_t* B, const float* bias, void* C, int M, int N, const GemmPlanes& pl, int ldc, bool out_bf16, hipStream_t s);
@@ -290,7 +289,7 @@ struct PrefillW {
     const int* exps;
     int planes;
 };
-enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4, PF_LINEAR = 5 /* internal: Linear.forward */ };
+enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4, PF_LINEAR = 5, PF_LINEAR_PART = 6 /* internal: Linear.forward, and a slice of one */ };
 int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, const void* wte, const void* wpe,
                          int weight_type, int E, float* x, hipStream_t s);
 int launch_ln_split(const float* x, int M, int E, const float* g, const float* b, float eps, uint16_t* out, const PlaneOut& po, hipStream_t s);
@@ -332,7 +331,7 @@ int launch_prefill_gemm(const PrefillA& A, const PrefillW& W, const float* bias,
 // prefill_ring.hip: whole-prompt Linears of some hundred rows.  The route: K slices (slabs of a residual Linear, else 1), 0 = not taken; tm: rows / 64 of a tile.
 int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_floats, bool force, int* tm);
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
-                        const PlaneOut& po, hipStream_t s, const SplitSeen& seen = SplitSeen{});
+                        const PlaneOut& po, hipStream_t s);
 // The exponents of a layer's activations, from its weights: of a normed x g + b, with x's rows no longer than sqrt(E), column e is no larger than sqrt(E) |g_e| + |b_e|, and
 // an output of a Linear behind it no larger than sqrt(E) |g w| + |w b + bias| (2-norm over the row's columns; launch_row_bounds).  Bounds that hold for
 // any input, and no looser than they have to be: a trained layer's gains and rows differ by factors of ten and more, and what lies far below its bound has
