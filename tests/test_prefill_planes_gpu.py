@@ -240,3 +240,24 @@ def test_gains_and_rows_that_differ_as_a_trained_models(zg, far, bf16, route):
         ref = exact_logits(cfg, w, toks)
         errs.append(np.linalg.norm(got - ref) / np.linalg.norm(ref))
     assert max(errs) <= 4e-7, errs
+
+
+@pytest.mark.parametrize("batch,n", [(1, 9), (2, 20), (1, 64)])
+def test_short_prompts_of_small_models_have_the_last_bit_of_an_fp32_weight(zg, batch, n):
+    """Outputs w - w of weights that two terms round up: nothing, where two planes leave the eighth that the 24th bit is worth."""
+    cfg = synth.CONFIGS["nano-char"]
+    E = cfg.n_embed
+    w = {k: np.array(v, np.float32) for k, v in synth.make_weights(cfg, seed=70, bf16=False).items()}
+    for l in range(cfg.n_layer):
+        w[f"h{l}.ln_2_g"] = np.zeros(E, np.float32)
+        w[f"h{l}.ln_2_b"] = np.ones(E, np.float32)
+        m = np.zeros((4 * E, E), np.float32)
+        m[np.arange(4 * E), np.arange(4 * E) % E] = np.float32(2.0 ** 20 * (1.0 + 4095 * 2.0 ** -23))
+        w[f"h{l}.c_fc_w"], w[f"h{l}.c_fc_b"] = m, -m.max(1)
+    m = zgpt.GPT(cfg, batch=batch, weights_f32=True)
+    m.load_weights(w)
+    toks = np.stack([synth.rand_tokens(700 + b, n, cfg.vocab_size) for b in range(batch)])
+    for got, t in zip(m.prefill(toks).astype(np.float64), toks):
+        ref = exact_logits(cfg, w, t)
+        assert np.linalg.norm(got - ref) <= 2e-6 * np.linalg.norm(ref)
+    m.close()

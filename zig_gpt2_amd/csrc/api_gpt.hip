@@ -201,9 +201,10 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
         y.exps = nullptr;
         if (!(g->flags & ZG_GPT_NO_PREFILL)) {  // inside the weight region: broadcast with the weights
             const int planes = g->wt == WT_F32 ? 2 : 1;
+            const bool rest = planes == 2 && E < kNearColumns;
             auto W = [&](size_t out, size_t in) {
-                uint16_t* p = (uint16_t*)P(out * in * planes * 2);
-                return PrefillW{p, (int*)P(out * 4), planes};
+                uint16_t* p = (uint16_t*)P(out * in * (planes + rest) * 2);
+                return PrefillW{p, (int*)P(out * 4), planes, rest};
             };
             y.c_attn_p = W(3 * E, E);
             y.c_proj_p = W(E, E);
@@ -417,6 +418,7 @@ int make_planes(const zg_gpt* g, const void* w, const PrefillW& p, int out, int 
     if (g->wt != WT_F32) return launch_plane_bf16(static_cast<const bf16_t*>(w), out, in, planes, exps, nullptr, s, floor);
     Split2Job j{static_cast<const float*>(w), planes, exps, out, (size_t)out * in};
     j.floor = floor;
+    if (p.rest) j.rest = planes + 2 * (size_t)out * in;
     return launch_split2(j, Split2Job{}, in, s);
 }
 

@@ -285,6 +285,13 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
         }
         *reinterpret_cast<u32x2*>(o + 4 * i) = u32x2{h0, h1};
         *reinterpret_cast<u32x2*>(o + lo + 4 * i) = u32x2{l0, l1};
+        if (!SEEN && j.rest != nullptr) {
+            typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
+            const f16x2_t h[2] = {__builtin_bit_cast(f16x2_t, h0), __builtin_bit_cast(f16x2_t, h1)}, l[2] = {__builtin_bit_cast(f16x2_t, l0), __builtin_bit_cast(f16x2_t, l1)};
+#pragma unroll
+            for (int c = 0; c < 4; ++c)
+                j.rest[(size_t)row * K + 4 * i + c] = __builtin_bit_cast(uint16_t, (_Float16)((q[c] - (float)h[c >> 1][c & 1]) - (float)l[c >> 1][c & 1]));
+        }
     };
 #pragma unroll
     for (int i = 0; i < NV; ++i)

@@ -49,10 +49,13 @@ struct RawRows {
     const float *x, *w;
 };
 
-// 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight; ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL, PF_LINEAR_PART).
+// 2 x 2 waves of TM x TN 32 x 32 tiles; NW planes of the weight (3: the last bits of an fp32 one as well); ST steps in the ring.  blockIdx.y: the K slice (PF_PARTIAL, PF_LINEAR_PART).
 // ALL: a prompt's fp32 Linears make the product of the two second terms as well.  With three products short sums, the rest of which is near to exact, left a small
 // model's logits further from 64 bits than six of three bf16 terms; the fourth hides beside the staging (300 rows 10.3 -> 10.8 us, 14.2 -> 14.2, 13.9 ->
-// 14.1; 1 x 300 tokens 850 -> 866).  NEAR (models of fewer than 512 columns): totals that keep what an addition rounds away, too dear (12.3 us) where sums are longer.
+// 14.1; 1 x 300 tokens 850 -> 866).  Models of fewer than 512 columns: few rows have the weight's last bits as a third plane, more rows NEAR, totals that keep what an addition
+// rounds away (both are too dear: 337 us for 1 x 9 tokens of the char model, where a third plane alone takes 296, NEAR alone 306 and three exact terms took 295).
+// Errors against 64 bits of that model, twelve weights by eight prompts, e-7, three exact terms / NEAR / third plane: 1 x 9 tokens 2.92 / 2.97 / 2.91, 2 x 20 3.02 / 3.00 / 2.95,
+// 1 x 64 2.91 / 2.90 / 2.79, 3 x 40 2.99 / 2.96 / 2.87, 1 x 130 3.03 / 2.79 / 2.75.
 template <int EPI, int TM, int TN, int NW, int ST, bool NEAR>
 __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
                                                               const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw, const SplitSeen seen) {
@@ -84,7 +87,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
             for (int i = 0; i < PB; ++i) dma_16(to + kPair * A_PLANE + p * B_PLANE + i * 4096, rb, vb[i], off + (unsigned)p * (unsigned)N * (unsigned)K * 2u);
     };
-    constexpr bool ALL = NW == 2 && EPI != PF_LINEAR;
+    constexpr bool ALL = NW >= 2 && EPI != PF_LINEAR;
     constexpr int NL = TN == 2 ? 1 : 2;  // leading products by the step's parity, or (registers) one sum of four steps
     f32x16 lead[NL][TM][TN], small[TM][TN], total[TM][TN];
 #pragma unroll
@@ -142,7 +145,8 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
                     if constexpr (ALL) one(small[i][j], kk, 1, 1, i, j);
                     one(small[i][j], kk, 1, 0, i, j);
                     one(lead[now][i][j], kk, 0, 0, i, j);
-                    if constexpr (NW == 2) one(small[i][j], kk, 0, 1, i, j);
+                    if constexpr (NW >= 2) one(small[i][j], kk, 0, 1, i, j);
+                    if constexpr (NW == 3) one(small[i][j], kk, 0, 2, i, j);
                 }
     };
     // what the epilogue needs besides the sums, on its way before the requests
@@ -292,7 +296,9 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
 template <int EPI>
 int launch_ring_epi(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int tm, int n_sp, const PrefillQkv& qa, const PlaneOut& po,
                     hipStream_t s, const SplitSeen& seen = SplitSeen{}) {
-    if (W.planes == 2 && std::min(N, K) < 512)
+    if constexpr (EPI != PF_LINEAR_PART)
+        if (W.rest && tm == 1) return launch_ring<EPI, 1, 1, 3, 4>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s);
+    if (W.planes == 2 && std::min(N, K) < (int)kNearColumns)
         return tm == 1   ? launch_ring<EPI, 1, 1, 2, 4, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
                : tm == 2 ? launch_ring<EPI, 2, 1, 2, 3, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen)
                          : launch_ring<EPI, 2, 2, 2, 2, true>(A, W, bias, C, M, N, K, ldc, n_sp, qa, po, s, RawRows{}, seen);
@@ -451,7 +457,7 @@ int prefill_ring_route(int M, int N, int K, bool resid, bool planes, size_t ws_f
 int launch_prefill_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C, int M, int N, int K, int ldc, int epi, int tm, int n_sp, const PrefillQkv& qa,
                         const PlaneOut& po, hipStream_t s) {
     ZG_REQUIRE(M > 0 && N % 64 == 0 && K % kBk == 0 && n_sp >= 1 && n_sp <= K / kBk && (size_t)M * kPair * K * 2 < ((size_t)1 << 31) &&
-                   (size_t)N * K * 2 * W.planes < ((size_t)1 << 31),
+                   (size_t)N * K * 2 * (W.planes + W.rest) < ((size_t)1 << 31),
                ZG_ERR_UNSUPPORTED, "prefill gemm: operands of %d x %d x %d beyond 2 GiB", M, N, K);
     switch (epi) {
         case PF_F32: return launch_ring_epi<PF_F32>(A, W, bias, C, M, N, K, ldc, tm, 1, qa, po, s);

@@ -208,6 +208,7 @@ struct Split2Job {
     float* norms = nullptr;  // 2-norms of the rows
     const int* one = nullptr;  // the exponent of every row; else each gets its own, ...
     PlaneFloor floor;          // ... no lower than this
+    uint16_t* rest = nullptr;  // what two terms leave (the 24th bit of one value in four), a plane of its own
 };
 // for the test hooks of one Linear and one attention: rows of three bf16 planes -> fp32, rows of two fp16 planes times 2^exp -> three bf16 planes
 int launch_join_planes(const uint16_t* in, const int* exp, int rows, int K, int planes, float* out, hipStream_t s);
@@ -283,12 +284,15 @@ struct PlaneOut {
     const int* exp;
     int coarse;  // ZG_GPT_PREFILL_2PLANE: values rounded to 16 significant bits first
 };
-// a Linear's weight: fp16 planes [planes][N][K] of its rows times 2^-exps[row]; one plane holds a bf16 value, two an fp32 value
+// a Linear's weight: fp16 planes [planes][N][K] of its rows times 2^-exps[row]; one plane holds a bf16 value, two 23 bits of an fp32 value, and the third behind them, where
+// there is one (models of fewer than kNearColumns columns), the last
 struct PrefillW {
     const uint16_t* p;
     const int* exps;
     int planes;
+    bool rest = false;
 };
+constexpr size_t kNearColumns = 512;
 enum PrefillEpilogue { PF_F32 = 0, PF_RESID = 1, PF_GELU_SPLIT = 2, PF_PARTIAL = 3 /* internal: split-K slice */, PF_QKV = 4, PF_LINEAR = 5, PF_LINEAR_PART = 6 /* internal: Linear.forward, and a slice of one */ };
 int launch_embed_prefill(const int* tokens, int token_stride, int B, int P, const void* wte, const void* wpe,
                          int weight_type, int E, float* x, hipStream_t s);
