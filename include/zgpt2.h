@@ -158,23 +158,30 @@ unsigned long long zg_debug_linear_ring_launches(void);
 /* Diagnostic: shader-clock stamps {count, start, end} of workgroup 0 / wave 0 of the last GEMM launched with
  * ZGPT2_GEMM_DBG bit 256 (tools/microbench/gemm_bench.cpp: cycles vs wall time = the clock the chip ran at). */
 int zg_debug_gemm_stamps(unsigned long long* out, size_t n_words);
-/* Diagnostic / test entry: ONE whole-prompt Linear exactly as zg_gpt_prefill launches it (src/ops.zig:21-46 for M = batch x
- * prompt rows).  A = the activation planes [M][3 K] bf16 (hi | mid | lo: the exact split of the fp32 rows), W = bf16 weights
- * [N][K], all device pointers.  epilogue: 0 fp32 C[M][N] = A W^T + bias; 1 C[M][N] += ... (residual add; ws required);
+/* Diagnostic / test entry: ONE whole-prompt Linear on the kernels of zg_gpt_prefill (src/ops.zig:21-46 for M = batch x prompt rows).  A = fp32 rows as their
+ * exact three-term split [M][3 K] bf16 (hi | mid | lo), W = bf16 weights [N][K], all device pointers: they become what a prompt's pass works on, two fp16
+ * planes of the rows with one exponent and one of the weights.  The exponent (and that of the planes a GELU's output leaves as) is here that of the data's largest value (of a
+ * bound on the outputs from the longest rows of both); a model's follow from its weights and lie some binades higher: zg_debug_prefill_linear_at, slack binades.
+ * epilogue: 0 fp32 C[M][N] = A W^T + bias; 1 C[M][N] += ... (residual add; ws required);
  * 2 bf16 planes C[M][3 N] of gelu(...).  force_kernel: 0 = the library's choice, 1 = the persistent four-wave GEMM
  * (gemm_s4.hip; slices = its K slices for epilogue 1, 0 = chosen), 2 = the 128-row prompt GEMM (prefill.hip), 3 = the ring
  * kernel of short prompts (prefill_ring.hip; epilogue 1 needs a slab of M N floats in ws, else the 128-row kernel runs).  ws: fp32
- * workspace of ws_floats elements for partial slabs.  The cache-append epilogue is exercised through zg_gpt_prefill. */
+ * workspace of ws_floats elements for partial slabs.  The cache-append epilogue is exercised through zg_gpt_prefill.
+ * _at: launched `repeats` times; us (may be NULL): microseconds a launch, the Linear's own (and its slabs' sum), after one more that is not timed. */
 int zg_debug_prefill_linear(const uint16_t* A_planes, const uint16_t* W, const float* bias_or_null, void* C, size_t M, size_t N,
                             size_t K, int epilogue, int force_kernel, int slices, float* ws, size_t ws_floats);
+int zg_debug_prefill_linear_at(const uint16_t* A_planes, const uint16_t* W, const float* bias_or_null, void* C, size_t M, size_t N,
+                               size_t K, int epilogue, int force_kernel, int slices, float* ws, size_t ws_floats, int slack, int repeats, float* us);
 /* Diagnostic / test entry: the causal prompt attention of zg_gpt_prefill alone (scaled_dot_product_attention of src/ops.zig:249-307
  * for all n_tokens positions of `batch` sequences at once).  qkv: fp32 [batch n_tokens][3 n_embed] rows (q | k | v columns);
  * out: bf16 planes [batch n_tokens][3 n_embed] = hi | mid | lo of the attention output; k_cache / v_cache: NULL (K and V are the
  * qkv columns) or head-major fp32 caches [batch][heads][ctx][64] holding the same rows; ws: of diagnostic builds (may be NULL);
- * key_tiles: 0 = the library's choice, above: the kernel of many prompts (groups of 128 queries) at any size.
- * Device pointers. */
+ * key_tiles: 0 = the library's choice, above: the kernel of many prompts (groups of 128 queries) at any size.  The exponents of q, k and v are those of their largest
+ * values; _at: slack binades more, repeats and us as above.  Device pointers. */
 int zg_debug_attn_prefill(const float* qkv, uint16_t* out, size_t batch, size_t n_tokens, size_t n_embed, size_t n_heads,
                           const float* k_cache, const float* v_cache, size_t ctx, float* ws, size_t ws_floats, int key_tiles);
+int zg_debug_attn_prefill_at(const float* qkv, uint16_t* out, size_t batch, size_t n_tokens, size_t n_embed, size_t n_heads, const float* k_cache, const float* v_cache,
+                             size_t ctx, float* ws, size_t ws_floats, int key_tiles, int slack, int repeats, float* us);
 /* Test hook: pin the route of every whole-prompt Linear of this process until called again with (0, 0) — force_kernel / slices
  * as in zg_debug_prefill_linear; force_kernel >= 16: the library's rule with that many 256 x 192 tiles (x K slices) as the
  * threshold from which the persistent GEMM takes a Linear (default 192; tools/experiments/pf_route_ab.py).

@@ -1,7 +1,8 @@
 """The causal prompt attention kernel alone (zg_debug_attn_prefill: scaled_dot_product_attention of src/ops.zig:249-307 for all prompt
-positions at once, on the bf16 matrix cores with exact three-plane splits) against a float64 softmax(q k^T / 8) v per head:
+positions at once, on the matrix cores with two fp16 terms a value) against a float64 softmax(q k^T / 8) v per head:
 prompt lengths around every tile boundary, K / V from the qkv rows and from head-major caches (with NaN behind the prompt's
-last row: a cache holds anything there), whole rows and split key ranges, a dominant key (the deferred rescale must fire)."""
+last row: a cache holds anything there), the library's choice of kernel and (tiles > 0, whatever the number) the kernel of many prompts, a dominant key (the
+deferred rescale must fire).  Exponents are those of the data; test_prefill_scaling_gpu.py has others."""
 import numpy as np
 import pytest
 import torch

@@ -1,8 +1,8 @@
-"""One whole-prompt Linear at a time (zg_debug_prefill_linear: Linear.forward of src/ops.zig:21-46 for M = batch x prompt rows, as
-zg_gpt_prefill launches it) on both GEMM families — the persistent four-wave kernel of gemm_s4.hip with the three activation
-planes in one K loop (K slices + partial slabs for the residual adds, GELU + three-plane split), and the 128-row kernels of
-prefill.hip — against a float64 product of the same operands.  The operands are exact (fp32 rows as three bf16 planes, bf16
-weights), so the only error is fp32 accumulation order: the reference tolerance of src/tests.zig:4-20 applies."""
+"""One whole-prompt Linear at a time (zg_debug_prefill_linear: Linear.forward of src/ops.zig:21-46 for M = batch x prompt rows, on the kernels of
+zg_gpt_prefill) on both GEMM families — the persistent four-wave kernel of gemm_s4.hip with the two activation
+planes in one K loop (K slices + partial slabs for the residual adds, GELU + split into planes), and the 128-row kernels of
+prefill.hip — against a float64 product of the same operands.  The fp32 rows become two fp16 terms (23 bits), the bf16 weights one plane (exact), the sums are
+fp32: the reference tolerance of src/tests.zig:4-20 applies.  Exponents are those of the data here; test_prefill_scaling_gpu.py has them as far above it as a model's may be."""
 import numpy as np
 import pytest
 import torch

@@ -666,125 +666,6 @@ int zg_gemm_bf16_nt(const uint16_t* A, const uint16_t* B, const float* bias_or_n
                                ctx().stream);
 }
 
-int zg_debug_prefill_linear(const uint16_t* A, const uint16_t* W, const float* bias, void* C, size_t M, size_t N, size_t K, int epilogue,
-                            int force_kernel, int slices, float* ws, size_t ws_floats) {
-    ZG_TRY(require_init());
-    ZG_REQUIRE(A && W && C && is_device_ptr(A) && is_device_ptr(W) && is_device_ptr(C) && (!bias || is_device_ptr(bias)) && (!ws || is_device_ptr(ws)),
-               ZG_ERR_ARG, "debug_prefill_linear: device pointers");
-    ZG_REQUIRE(M >= 1 && M < (1u << 30) && N >= 64 && N < (1u << 30) && K >= 64 && K < (1u << 30) && epilogue >= 0 && epilogue <= 2 && force_kernel >= 0 &&
-                   force_kernel <= 3 && slices >= 0,
-               ZG_ERR_ARG, "debug_prefill_linear: arguments");
-    const int epi = epilogue == 0 ? PF_F32 : epilogue == 1 ? PF_RESID : PF_GELU_SPLIT;
-    // the caller's three-term bf16 planes stand for fp32 rows; the Linear is launched on what a prompt pass would have made of them
-    hipStream_t s = ctx().stream;
-    char* scratch = nullptr;
-    const size_t need[] = {M * K * 4, M * K * 4, M * 4, M * 4, N * K * 2, N * 4, N * 4, epi == PF_GELU_SPLIT ? M * N * 4 : 0, 4};
-    size_t at[10] = {0};
-    for (int i = 0; i < 9; ++i) at[i + 1] = (at[i] + need[i] + 255) & ~(size_t)255;
-    ZG_HIP(hipMalloc(reinterpret_cast<void**>(&scratch), at[9]));
-    float *x = reinterpret_cast<float*>(scratch), *xn = reinterpret_cast<float*>(scratch + at[3]), *wn = reinterpret_cast<float*>(scratch + at[6]);
-    uint16_t *xp = reinterpret_cast<uint16_t*>(scratch + at[1]), *wp = reinterpret_cast<uint16_t*>(scratch + at[4]), *op = reinterpret_cast<uint16_t*>(scratch + at[7]);
-    int *xe = reinterpret_cast<int*>(scratch + at[2]), *we = reinterpret_cast<int*>(scratch + at[5]), *oe = reinterpret_cast<int*>(scratch + at[8]);
-    auto all = [&]() -> int {
-        ZG_TRY(launch_join_planes(A, nullptr, (int)M, (int)K, 3, x, s));
-        Split2Job jx{x, xp, xe, (int)M};
-        jx.norms = xn;
-        ZG_TRY(launch_split2(jx, Split2Job{}, (int)K, s));
-        const bool each = force_kernel == 2 || force_kernel == 3;  // (the persistent GEMM's prompt Linears have one exponent for all rows)
-        if (!each) {
-            std::vector<int> he(M);
-            ZG_HIP(hipMemcpyAsync(he.data(), xe, M * 4, hipMemcpyDeviceToHost, s));
-            ZG_HIP(hipStreamSynchronize(s));
-            const int top = *std::max_element(he.begin(), he.end());
-            ZG_HIP(hipMemcpyAsync(oe, &top, 4, hipMemcpyHostToDevice, s));
-            jx.one = oe;
-            ZG_TRY(launch_split2(jx, Split2Job{}, (int)K, s));
-            ZG_HIP(hipStreamSynchronize(s));
-        }
-        ZG_TRY(launch_plane_bf16(W, (int)N, (int)K, wp, we, wn, s));
-        PlaneOut po{nullptr, 0};
-        if (epi == PF_GELU_SPLIT) {  // no gelu is larger than its row times the longest row of the weight, and the bias
-            std::vector<float> hx(M), hw(N), hb(N, 0.0f);
-            ZG_HIP(hipMemcpyAsync(hx.data(), xn, M * 4, hipMemcpyDeviceToHost, s));
-            ZG_HIP(hipMemcpyAsync(hw.data(), wn, N * 4, hipMemcpyDeviceToHost, s));
-            if (bias) ZG_HIP(hipMemcpyAsync(hb.data(), bias, N * 4, hipMemcpyDeviceToHost, s));
-            ZG_HIP(hipStreamSynchronize(s));
-            float mx = 0.0f, mw = 0.0f, mb = 0.0f;
-            for (float v : hx) mx = fmaxf(mx, v);
-            for (float v : hw) mw = fmaxf(mw, v);
-            for (float v : hb) mb = fmaxf(mb, fabsf(v));
-            const float bound = mx * mw + mb;
-            const int e = bound > 0.0f && std::isfinite(bound) ? ilogbf(bound) - 11 : 0;
-            ZG_HIP(hipMemcpyAsync(oe, &e, 4, hipMemcpyHostToDevice, s));
-            ZG_HIP(hipStreamSynchronize(s));
-            po.exp = oe;
-        }
-        prefill_force_route(force_kernel, slices);
-        const int st = launch_prefill_gemm(PrefillA{xp, xe, each}, PrefillW{wp, we, 1}, bias, epi == PF_GELU_SPLIT ? static_cast<void*>(op) : C, (int)M, (int)N, (int)K,
-                                           epi == PF_GELU_SPLIT ? 0 : (int)N, epi, ws, ws_floats, nullptr, s, nullptr, po);
-        prefill_force_route(0, 0);
-        ZG_TRY(st);
-        if (epi == PF_GELU_SPLIT) ZG_TRY(launch_join_planes(op, oe, (int)M, (int)N, kPair, static_cast<bf16_t*>(C), s));
-        return ZG_OK;
-    };
-    const int st = all();
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(scratch);
-    return st;
-}
-
-int zg_debug_attn_prefill(const float* qkv, uint16_t* out, size_t batch, size_t n_tokens, size_t n_embed, size_t n_heads, const float* k_cache,
-                          const float* v_cache, size_t ctx_len, float* ws, size_t ws_floats, int key_tiles) {
-    ZG_TRY(require_init());
-    ZG_REQUIRE(qkv && out && is_device_ptr(qkv) && is_device_ptr(out) && (!k_cache || (v_cache && is_device_ptr(k_cache) && is_device_ptr(v_cache))) &&
-                   (!ws || is_device_ptr(ws)),
-               ZG_ERR_ARG, "debug_attn_prefill: device pointers");
-    ZG_REQUIRE(batch >= 1 && n_tokens >= 1 && n_heads >= 1 && n_embed == 64 * n_heads && batch * n_tokens < (1u << 24) && n_embed < (1u << 16) && (!k_cache || ctx_len >= n_tokens) &&
-                   key_tiles >= 0 && key_tiles <= 255,
-               ZG_ERR_ARG, "debug_attn_prefill: arguments");
-    hipStream_t s = ctx().stream;
-    const size_t rows = batch * n_tokens;
-    char* scratch = nullptr;
-    ZG_HIP(hipMalloc(reinterpret_cast<void**>(&scratch), rows * n_embed * kPair * 2 + 256));
-    uint16_t* planes = reinterpret_cast<uint16_t*>(scratch + 256);
-    int* exps = reinterpret_cast<int*>(scratch);
-    auto all = [&]() -> int {
-        // the exponents a layer's weights would have given: of the largest q, k and v
-        std::vector<float> h(rows * 3 * n_embed), c(k_cache ? n_tokens * 64 : 0);
-        ZG_HIP(hipMemcpyAsync(h.data(), qkv, h.size() * 4, hipMemcpyDeviceToHost, s));
-        ZG_HIP(hipStreamSynchronize(s));
-        float top[3] = {0.0f, 0.0f, 0.0f};
-        for (size_t i = 0; i < h.size(); ++i) {
-            const int which = (int)(i % (3 * n_embed) / n_embed);
-            if (std::isfinite(h[i]) && (which == 0 || !k_cache)) top[which] = fmaxf(top[which], fabsf(h[i]));
-        }
-        for (int which = 1; which < 3 && k_cache; ++which)
-            for (size_t bh = 0; bh < batch * n_heads; ++bh) {
-                ZG_HIP(hipMemcpyAsync(c.data(), (which == 1 ? k_cache : v_cache) + bh * ctx_len * 64, c.size() * 4, hipMemcpyDeviceToHost, s));
-                ZG_HIP(hipStreamSynchronize(s));
-                for (float v : c)
-                    if (std::isfinite(v)) top[which] = fmaxf(top[which], fabsf(v));
-            }
-        int e[kBounds] = {0};
-        for (int which = 0; which < 3; ++which) e[PB_Q + which] = top[which] > 0.0f ? ilogbf(top[which]) - 11 : 0;
-        ZG_HIP(hipMemcpyAsync(exps, e, sizeof e, hipMemcpyHostToDevice, s));
-        ZG_HIP(hipStreamSynchronize(s));
-        ZG_TRY(launch_attn_prefill(qkv, planes, (int)batch, (int)n_tokens, (int)n_embed, (int)n_heads, k_cache, v_cache, (int)ctx_len, exps, 0, s, key_tiles > 0,
-                                   reinterpret_cast<unsigned long long*>(ws)));
-        return launch_join_planes(planes, exps + PB_V, (int)rows, (int)n_embed, kPair, out, s);
-    };
-    const int st = all();
-    (void)hipStreamSynchronize(s);
-    (void)hipFree(scratch);
-    return st;
-}
-
-int zg_debug_prefill_route(int force_kernel, int slices) {
-    ZG_REQUIRE(force_kernel >= 0 && (force_kernel <= 3 || force_kernel >= 16) && slices >= 0, ZG_ERR_ARG, "debug_prefill_route: arguments");
-    prefill_force_route(force_kernel, slices);
-    return ZG_OK;
-}
-
 unsigned long long zg_debug_gemm_launches(void) { return gemm_mfma_launch_count(); }
 unsigned long long zg_debug_linear_few_mfma_launches(void) { return linear_few_mfma_launch_count(); }
 unsigned long long zg_debug_linear_ring_launches(void) { return linear_ring_launch_count(); }
