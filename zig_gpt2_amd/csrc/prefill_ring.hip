@@ -2,7 +2,7 @@
 // idle: prompts of some hundred rows.
 //
 // A = the activation planes [M][2 K] (hi | lo), W = the one plane [N][K] of a bf16 weight, or the two [2][N][K] of an fp32 weight (zg_common.h split2_f16).
-// All the products of a K step of 64 columns (two, or four; three of an op-tier Linear) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
+// All the products of a K step of 64 columns (two; four, or five with a third plane; three of an op-tier Linear in one piece, four of one in slices) are made from ONE staging of the planes, where the 128-row kernels of prefill.hip
 // walk an fp32 weight in two passes that each stage the activations again and meet in slabs.
 // What bounds it: a compute unit takes in some 30 bytes a clock (32 KB a step of a 64 x 64 tile of an fp32 weight: 1100 clocks, beside 384 or 512 of
 // products).  So tiles are small while they are few, and no operand is staged twice for one tile.  The planes arrive by LDS-DMA in a ring of
@@ -377,14 +377,12 @@ int launch_linear_ring(const float* X, const float* W, const float* bias, float*
         ZG_TRY(tm == 1   ? (launch_ring<PF_LINEAR, 1, 1, 2, 4>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen))
                : tm == 2 ? (launch_ring<PF_LINEAR, 2, 1, 2, 3>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen))
                          : (launch_ring<PF_LINEAR, 2, 2, 2, 2>(A, P, bias, Y, M, Np, K, N, 1, none, PlaneOut{}, s, raw, seen)));
-        note_kernel("linear_tiles_kernel");  // (the Linears of a medium number of rows have one name; the count says which)
         return ZG_OK;
     }
     ZG_TRY(launch_ring_epi<PF_LINEAR_PART>(A, P, nullptr, slabs, M, Np, K, Np, tm, n_sp, PrefillQkv{}, PlaneOut{}, s, seen));
     const size_t quads = (size_t)M * ((N + 3) / 4);
     linear_ring_finish_kernel<<<(unsigned)((quads + 255) / 256), 256, 0, s>>>(slabs, n_sp, M, Np, bias, Y, N, X, W, K, seen);
     ZG_HIP(hipGetLastError());
-    note_kernel("linear_tiles_kernel");
     return ZG_OK;
 }
 
