@@ -709,17 +709,17 @@ def lm_bench(a):
     print(json.dumps(out))
 
 
-def prefill_flops(cfg, prompts, n, ms, planes=3):
+def prefill_flops(cfg, prompts, n, ms, planes=2):
     """Matrix-core work of one whole-prompt pass: the useful Linear FLOPs (2 M K N each), and what the MFMAs execute — `planes`
-    bf16 plane products per Linear (exact split of the fp32 activations), six per attention product (both operands split),
+    fp16 plane products per Linear (two terms of the fp32 activations against a bf16 weight), three per attention product (both operands in two terms),
     causal attention counted over the 32 x 32 tiles it visits."""
     E, L, H = cfg.n_embed, cfg.n_layer, cfg.n_heads
     lin = 2.0 * prompts * n * 12 * E * E * L
     nqb = (n + 31) // 32
     tiles = nqb * (nqb + 1) // 2
     attn = 2.0 * 2 * tiles * 32 * 32 * 64 * H * prompts * L  # S = q k^T and P v per visited tile
-    return {"linear_tflops_useful": round(lin / ms / 1e9, 1), "mfma_tflops": round((planes * lin + 6 * attn) / ms / 1e9, 1),
-            "mfma_frac_of_2.5PF": round((planes * lin + 6 * attn) / ms / 1e9 / 2500.0, 4)}
+    return {"linear_tflops_useful": round(lin / ms / 1e9, 1), "mfma_tflops": round((planes * lin + 3 * attn) / ms / 1e9, 1),
+            "mfma_frac_of_2.5PF": round((planes * lin + 3 * attn) / ms / 1e9 / 2500.0, 4)}
 
 
 def main():
@@ -1013,12 +1013,11 @@ def main():
             p_ms = time_prefill(model)
             prefill = {"prompt_tokens": n_p, "prompts": ppg, "ms": round(p_ms, 3),
                        "prompt_tokens_per_s": round(ppg * n_p / p_ms * 1e3, 1),
-                       **prefill_flops(cfg, ppg, n_p, p_ms),
+                       **prefill_flops(cfg, ppg, n_p, p_ms, 3 if a.weights_f32 else 2),
                        "vs_token_at_a_time": round((1e3 * elapsed / a.steps) * n_p / ctx / p_ms, 1),
                        "how": "synchronous zg_gpt_prefill calls (host wall clock, 5 repetitions after 3 warm-ups); "
-                              + ("fp32 weights: both GEMM operands as exact bf16 plane triples, the six plane products as three "
-                                 "passes of one launch of the 128-row prompt GEMM per Linear" if a.weights_f32 else
-                                 "activations split exactly 3-way into bf16 for the MFMA GEMMs") + ", causal attention on the bf16 matrix cores with exact three-plane splits of q, k, v and the probabilities (six plane products per matrix product)"}
+                              + ("fp32 weights: both GEMM operands as two fp16 terms of scaled values, three or four products" if a.weights_f32 else
+                                 "activations as two fp16 terms of scaled values, bf16 weights as one exact fp16 plane, two products") + ", causal attention with two terms of q, k, v and the probabilities (three plane products per matrix product)"}
             if not a.weights_f32:  # the two-plane mode (inside north_star's 1e-3, outside the tests' near-zero floor)
                 m2 = gpt.GPT(cfg, batch=ppg, use_graph=False, kv_f16=a.kv_f16, kv_b24=a.kv_b24, prefill_planes=2)
                 m2.load_weights(weights)

@@ -211,7 +211,8 @@ enum {
     ZG_GPT_NO_GRAPH = 1 << 1,    /* launch kernels eagerly instead of replaying a hipGraph */
     ZG_GPT_KV_F16 = 1 << 2,      /* store the KV cache as fp16 instead of fp32 */
     ZG_GPT_NO_PREFILL = 1 << 3,  /* generate: feed prompts one position at a time, as main.zig:331-334 does */
-    ZG_GPT_PREFILL_2PLANE = 1 << 4, /* whole-prompt GEMMs multiply the fp32 activations rounded to 16 significant bits: ~2e-5 of the
+    ZG_GPT_PREFILL_2PLANE = 1 << 4, /* whole-prompt GEMMs multiply the fp32 activations rounded to 16 significant bits, as ever with this flag; it saves no
+                                      time any more (the default makes no more products): ~2e-5 of the
                                       logit scale (inside the 1e-3 parity bound, outside the tests' near-zero floor);
                                       bf16-weight handles only */
     ZG_GPT_NO_PREFETCH = 1 << 5, /* zg_gpt_generate_*: no side-stream L2 prefetcher beside the decode chain (results are
@@ -295,9 +296,9 @@ int zg_gpt_forward(zg_gpt* g, size_t seq_len, const size_t* tokens, size_t n_tok
  * (Linears as matrix-core GEMMs, causal attention), filling the KV caches exactly as n_tokens calls of
  * zg_gpt_forward would.  tokens is [batch][token_stride].  With compute_logits != 0 the logits of position
  * n_tokens-1 are produced as zg_gpt_forward(n_tokens, ...) would (zg_gpt_argmax / logits_out as there).
- * Afterwards decoding continues with zg_gpt_forward(n_tokens + 1, ...).  Both weight modes: bf16-weight handles multiply the
- * exact three-plane split of the activations with the weights, ZG_GPT_WEIGHTS_F32 handles split both operands (six plane
- * products: fp32-sgemm grade).  Not available on handles created with ZG_GPT_NO_PREFILL. */
+ * Afterwards decoding continues with zg_gpt_forward(n_tokens + 1, ...).  Both weight modes: activations (and fp32 weights) are multiplied as two fp16 terms, 23
+ * bits, scaled by powers of two that follow from the weights, so that no input leaves their range; logits are no further from exact ones than with
+ * exact three-term planes.  LayerNorm takes its variance from the differences to the mean.  Not available on handles created with ZG_GPT_NO_PREFILL. */
 int zg_gpt_prefill(zg_gpt* g, const size_t* tokens, size_t token_stride, size_t n_tokens,
                    int compute_logits, float* logits_out, size_t logits_len);
 /* argmax of the logits of the last zg_gpt_forward(compute_logits=1) per sequence (lowest index

@@ -56,7 +56,7 @@ def test_prefill_logits_and_cache_match_oracle(zg, name, lengths):
 @pytest.mark.parametrize("name,batch,lengths,wgs", [("tiny", 1, [5, 33, 64], None), ("tiny", 3, [21, 64], 2), ("tiny3", 2, [48], 3),
                                                     ("nano-char", 4, [129, 256], None), ("xl-slice", 1, [95], 5), ("medium-slice", 2, [80], None)])
 def test_prefill_linears_on_the_persistent_four_wave_gemm(zg, monkeypatch, every_linear_on_s4, name, batch, lengths, wgs):
-    """Large prompts run their Linears on gemm_s4 (three planes in one K loop; slab epilogue + reduce for the residual adds,
+    """Large prompts run their Linears on gemm_s4 (two planes in one K loop; slab epilogue + reduce for the residual adds,
     GELU + split, qkv + cache append).  zg_debug_prefill_route(1, 0) sends every shape there: small models, ragged tile edges (M far
     below 256, N = 1600 = 8.33 tiles), several tiles per workgroup (ZGPT2_GEMM_WGS), K slices.  Same checks as the 128-row
     path: last-position logits and the decode step on top of the prefilled caches against the oracle."""
@@ -200,9 +200,9 @@ def test_prefill_124m_full_context_equals_decode_loop(zg):
 @pytest.mark.parametrize("weights_f32", [False, True])
 def test_prefill_124m_eight_full_prompts_equal_one_prompt_passes(zg, weights_f32):
     """BASELINE config 3's prompt side at full size: eight 1023-token prompts in one pass — every Linear on the persistent
-    four-wave GEMM (three / six plane pairs in one K loop, K slices + reduce, the stream-K hand-over of c_attn's 384 tiles at its
+    four-wave GEMM (two / three plane pairs in one K loop, K slices + reduce, the stream-K hand-over of c_attn's 384 tiles at its
     real geometry), whole-row attention — against the same prompts passed one at a time, which run the 128-row GEMM family and
-    split key ranges: last-position logits and the decode step on top of the caches, rows 0, 3 and 7."""
+    blocks of 32 queries: last-position logits and the decode step on top of the caches, rows 0, 3 and 7."""
     cfg = synth.CONFIGS["124M"]
     w = synth.make_weights(cfg, seed=5, bf16=not weights_f32)
     n = cfg.context_size - 1
@@ -275,8 +275,8 @@ def test_prefill_errors(zg):
 
 @pytest.mark.parametrize("name,lengths", [("tiny", [1, 5, 33, 64]), ("tiny3", [7, 48]), ("xl-slice", [40])])
 def test_prefill_with_fp32_weights(zg, name, lengths):
-    """ZG_GPT_WEIGHTS_F32 handles (checkpoints that are not bf16-representable): the whole-prompt pass multiplies exact
-    bf16 plane triples of BOTH operands (six plane products) and must meet the same tolerance against the fp32 oracle
+    """ZG_GPT_WEIGHTS_F32 handles (checkpoints that are not bf16-representable): the whole-prompt pass multiplies two
+    fp16 terms of BOTH operands (three or four plane products) and must meet the same tolerance against the fp32 oracle
     as the decode path; the decode step on top pins the cache contents."""
     cfg = synth.CONFIGS[name]
     w = synth.make_weights(cfg, seed=73, bf16=False)
@@ -301,8 +301,8 @@ def test_prefill_with_fp32_weights(zg, name, lengths):
 
 @pytest.mark.parametrize("name,batch,n,wgs", [("tiny3", 2, 48, None), ("nano-char", 4, 256, 16), ("xl-slice", 1, 95, 5), ("medium-slice", 2, 80, None)])
 def test_prefill_fp32_weights_on_the_persistent_four_wave_gemm(zg, monkeypatch, every_linear_on_s4, name, batch, n, wgs):
-    """fp32 weights on gemm_s4: the six plane products a_i w_j (i + j <= 2) of the activation planes and the weight's three plane
-    matrices are the plane pairs of ONE K loop (6 K / 64 K-steps per tile) instead of three passes over partial slabs.  Same
+    """fp32 weights on gemm_s4: the three plane products a_i w_j (i + j <= 1) of the activation planes and the weight's two plane
+    matrices are the plane pairs of ONE K loop (3 K / 64 K-steps per tile) instead of three passes over partial slabs.  Same
     checks as with bf16 weights, against the fp32 oracle; nano-char 4 x 256 on 16 workgroups also hands half tiles over."""
     if wgs:
         monkeypatch.setenv("ZGPT2_GEMM_WGS", str(wgs))
@@ -324,9 +324,9 @@ def test_prefill_fp32_weights_on_the_persistent_four_wave_gemm(zg, monkeypatch, 
 
 
 def test_prefill_two_plane_mode_is_inside_the_parity_bound(zg):
-    """ZG_GPT_PREFILL_2PLANE: hi + mid planes of the activations only.  north_star's bound is 1e-3 relative; the
+    """ZG_GPT_PREFILL_2PLANE: activations rounded to 16 significant bits.  north_star's bound is 1e-3 relative; the
     two-plane error is ~2e-5 of the logit scale, so it is stated against the logit scale (not against the
-    near-zero floor of assert_model_close, which the exact three-plane default meets)."""
+    near-zero floor of assert_model_close, which the default meets)."""
     cfg = synth.CONFIGS["124M"]
     w = synth.make_weights(cfg, seed=74, bf16=True)
     toks = synth.rand_tokens(741, 96, cfg.vocab_size)

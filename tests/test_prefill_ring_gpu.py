@@ -1,6 +1,6 @@
 """The ring kernel of prompts of some hundred rows (prefill_ring.hip): Linear.forward of src/ops.zig:21-46 for M = batch x prompt
-rows.  bf16 weights one Linear at a time against a float64 product of the same (exact) operands: single rows, ragged last tiles, one
-K step, an odd number of them, tiles of 64 and of 128 rows, K slices.  fp32 weights (three planes, six products) through whole
+rows.  bf16 weights one Linear at a time against a float64 product of the same operands: single rows, ragged last tiles, one
+K step, an odd number of them, tiles of 64 and of 128 rows, K slices.  fp32 weights (two planes, three or four products; three planes of a small model's) through whole
 small models against the oracle, every Linear forced onto the ring."""
 import ctypes as C
 

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(256, 2) void attn_prefill_pl_kernel(const float* __
         for (int r = 1; r < 16; ++r) mx = fmaxf(mx, sc[r]);
         mx = both_halves_max(mx);
         // The reference point of the exponentials moves only when some query's maximum grew by more than 2^kDefer since it was
-        // set (fp32 accumulators: probabilities up to 2^kDefer lose nothing, and the planes split them exactly) — the rescale
+        // set (fp32 accumulators: probabilities up to 2^kDefer lose nothing, and their planes have the same bits) — the rescale
         // of the 32 output registers then runs on a few tiles of a row instead of all.  Everything at the old reference (O, l) is
         // rescaled at the decision, before any probability of this tile exists.
         if (__builtin_amdgcn_ballot_w64(mx * s_back > mrun + kDefer) != 0) {

@@ -556,13 +556,6 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
     //   step 3      barrier 1 (A half 0 of slot X read out; A half 1 of t, B and A half 0 of t + 1 landed)
     //   steps 3-6   DMA: A half 0 of K-step t + 2 -> slot X (one piece per step); B fragments of K-step t + 1 -> registers
     //   step 7      barrier 2 (A half 1 of slot X, B of slot X ^ 1 read out)
-    // One step = one k-slice (16 of K) of one phase: 2 x NT MFMAs, and behind each MFMA at most ONE other item
-    // (a fragment read or a DMA piece: two ds_read_b128 in one MFMA shadow do not fit — tools/microbench/mfma_lds.hip).
-    // J = 4 h + ks.  Per K-step t (slot X):
-    //   steps 0-2   DMA: B of K-step t + 2 -> slot X, A half 1 of K-step t + 1 -> slot X ^ 1
-    //   step 3      barrier 1 (A half 0 of slot X read out; A half 1 of t, B and A half 0 of t + 1 landed)
-    //   steps 3-6   DMA: A half 0 of K-step t + 2 -> slot X (one piece per step); B fragments of K-step t + 1 -> registers
-    //   step 7      barrier 2 (A half 1 of slot X, B of slot X ^ 1 read out)
     auto step = [&](auto XT, auto JT) {
         constexpr int X = decltype(XT)::value, J = decltype(JT)::value;
         constexpr int h = J >> 2, ks = J & 3, cb = J & 1, nb = cb ^ 1;
@@ -687,7 +680,7 @@ __global__ __launch_bounds__(256, 1) void gemm_s4_kernel(const bf16_t* __restric
             if (lane == 0) __hip_atomic_store(qa.sk_flags + sk_sh * 4 + wave, qa.sk_epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     };
-    // the consumer's half starts at zero and meets its producer's in the epilogue (two halves, each rounded at its own size)
+    // (the producer's half starts at zero, the consumer's at the bias, and they meet in the consumer's epilogue: two halves, each rounded at its own size)
     auto sk_wait = [&]() {
         if constexpr (SK) {
             unsigned spins = 0;
