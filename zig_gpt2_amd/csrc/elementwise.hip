@@ -242,14 +242,21 @@ __device__ __forceinline__ int above_floor(int up, const PlaneFloor& f, int row)
 template <int NV, bool SEEN>
 __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const Split2Job jb, int K, const SplitSeen seen) {
     const int lane = threadIdx.x & 63;
-    int row = (int)blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+    int row = __builtin_amdgcn_readfirstlane((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6));
     if (row >= ja.rows + jb.rows) return;
     const bool second = row >= ja.rows;
     if (second) row -= ja.rows;
-    const Split2Job& j = second ? jb : ja;
-    const float* x = j.in + (size_t)row * K;
-    uint16_t* o = j.out + (size_t)row * (j.lo != 0 ? K : 2 * K);
-    const size_t lo = j.lo != 0 ? j.lo : (size_t)K;
+    // (member by member: a reference to one of the two put both on the stack, 16.7 us for 9.9 of 2048 + 3072 rows of 768)
+#define ZG_OF(member) (second ? jb.member : ja.member)
+    const float* const x = ZG_OF(in) + (size_t)row * K;
+    const size_t behind = ZG_OF(lo), lo = behind != 0 ? behind : (size_t)K;
+    uint16_t* const o = ZG_OF(out) + (size_t)row * (behind != 0 ? K : 2 * K);
+    const int* const one = ZG_OF(one);
+    const PlaneFloor floor{ZG_OF(floor.a), ZG_OF(floor.bias)};
+    int* const exps = ZG_OF(exps);
+    [[maybe_unused]] float* const norms = ZG_OF(norms);
+    [[maybe_unused]] uint16_t* const rest = ZG_OF(rest);
+#undef ZG_OF
     const int n4 = K >> 2;
     f32x4 v[NV];
     uint32_t top = 0;
@@ -265,8 +272,8 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
     for (int i = lane + 64 * NV; i < n4; i += 64) widen(*reinterpret_cast<const f32x4*>(x + 4 * i));
 #pragma unroll
     for (int d = 32; d >= 1; d >>= 1) top = max(top, (uint32_t)__shfl_xor((int)top, d, 64));
-    const int up = j.one != nullptr ? -*j.one : above_floor(split2_exp(top), j.floor, row);
-    if (lane == 0) j.exps[row] = -up;
+    const int up = one != nullptr ? -*one : above_floor(split2_exp(top), floor, row);
+    if (lane == 0) exps[row] = -up;
     [[maybe_unused]] const uint32_t large_from = __float_as_uint(__uint_as_float(top) * 0.0009765625f);  // 2^-10 of the largest
     [[maybe_unused]] const uint32_t small_below = up < 140 ? __float_as_uint(ldexpf(1.0f, -2 - up)) : 0u;  // (the smallest numbers there are have no bits below two terms)
     [[maybe_unused]] int large = 0, small = 0;  // how many, in the first lane
@@ -285,12 +292,12 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
         }
         *reinterpret_cast<u32x2*>(o + 4 * i) = u32x2{h0, h1};
         *reinterpret_cast<u32x2*>(o + lo + 4 * i) = u32x2{l0, l1};
-        if (!SEEN && j.rest != nullptr) {
+        if (!SEEN && rest != nullptr) {
             typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
             const f16x2_t h[2] = {__builtin_bit_cast(f16x2_t, h0), __builtin_bit_cast(f16x2_t, h1)}, l[2] = {__builtin_bit_cast(f16x2_t, l0), __builtin_bit_cast(f16x2_t, l1)};
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                j.rest[(size_t)row * K + 4 * i + c] = __builtin_bit_cast(uint16_t, (_Float16)((q[c] - (float)h[c >> 1][c & 1]) - (float)l[c >> 1][c & 1]));
+                rest[(size_t)row * K + 4 * i + c] = __builtin_bit_cast(uint16_t, (_Float16)((q[c] - (float)h[c >> 1][c & 1]) - (float)l[c >> 1][c & 1]));
         }
     };
 #pragma unroll
@@ -311,9 +318,9 @@ __global__ __launch_bounds__(256) void split2_kernel(const Split2Job ja, const S
         say(SEEN_ANY);
         const int kind = (second ? SEEN_W_UNEVEN : SEEN_X_UNEVEN) + (mark & MARK_SPARSE ? 1 : 0);
         say(SEEN_ROWS + 16 * kind + row % 16);
-    } else if (j.norms != nullptr) {
+    } else if (norms != nullptr) {
         ss = wave_allsum(ss);
-        if (lane == 0) j.norms[row] = ldexpf(sqrtf(ss), -up);
+        if (lane == 0) norms[row] = ldexpf(sqrtf(ss), -up);
     }
 }
 
