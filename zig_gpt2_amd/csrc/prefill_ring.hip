@@ -57,8 +57,11 @@ struct RawRows {
 // Errors against 64 bits of that model, twelve weights by eight prompts, e-7, three exact terms / NEAR / third plane: 1 x 9 tokens 2.92 / 2.97 / 2.91, 2 x 20 3.02 / 3.00 / 2.95,
 // 1 x 64 2.91 / 2.90 / 2.79, 3 x 40 2.99 / 2.96 / 2.87, 1 x 130 3.03 / 2.79 / 2.75.
 template <int EPI, int TM, int TN, int NW, int ST, bool NEAR>
-__global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const float* bias, void* C, int M, int N, int K, int ldc, int n_sp,
-                                                              const PrefillQkv qa, const PlaneExps ex, const PlaneOut po, const RawRows raw, const SplitSeen seen) {
+__global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A, const uint16_t* W, const int* ex_a, const int* ex_w, const float* bias, int M, int N, int K, int n_sp_each,
+                                                              void* C, int ldc, const PrefillQkv qa, const PlaneOut po, const RawRows raw, const SplitSeen seen) {
+    // (in front of C what the first loads need: the leading arguments are in registers when a wave starts.  n_sp_each: K slices, and whether A's rows have exponents of their own)
+    const int n_sp = n_sp_each >> 1;
+    const bool a_each = n_sp_each & 1;
     constexpr int BM = 64 * TM, BN = 64 * TN, PA = BM / 32, PB = BN / 32, A_PLANE = BM * kRow, B_PLANE = BN * kRow, SLOT = kPair * A_PLANE + NW * B_PLANE;
     constexpr int REQ = kPair * PA + NW * PB;  // 1 KB pieces (8 rows) a wave asks for in a step
     extern __shared__ __attribute__((aligned(1024))) char s_ring[];
@@ -158,7 +161,7 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const int n = TN == 1 ? n_w : min(n_w + 32 * j, N - 4);  // (N: whole pieces of 32)
-            col_exp[j] = *reinterpret_cast<const i32x4*>(ex.w + n);
+            col_exp[j] = *reinterpret_cast<const i32x4*>(ex_w + n);
             bv[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
             if (EPI == PF_LINEAR) {
                 if (bias)
@@ -171,13 +174,18 @@ __global__ __launch_bounds__(256, 1) void prefill_ring_kernel(const uint16_t* A,
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int r8i = 0; r8i < 4; ++r8i) row_exp[i][r8i] = ex.a[ex.a_each ? min(m0 + (wy * TM + i) * 32 + 8 * r8i + (lane >> 3), M - 1) : 0];
+            for (int r8i = 0; r8i < 4; ++r8i) row_exp[i][r8i] = ex_a[a_each ? min(m0 + (wy * TM + i) * 32 + 8 * r8i + (lane >> 3), M - 1) : 0];
     };
     if (TN == 1) fetch_scales();  // (larger tiles have no registers for them beside the products)
-    const int out_exp = EPI == PF_GELU_SPLIT ? *po.exp : 0;
 #pragma unroll
     for (int s = 0; s < ST; ++s) request(s, s);
-    if (EPI == PF_QKV) {  // the epilogue's arguments, fetched under the first requests
+    int out_exp = 0;  // the epilogue's arguments, fetched under the first requests
+    if (EPI == PF_GELU_SPLIT) {
+        out_exp = *po.exp;
+        ZG_PIN(out_exp);
+    }
+    ZG_PIN(C); ZG_PIN(ldc);
+    if (EPI == PF_QKV) {
         ZG_PIN(qa.P); ZG_PIN(qa.E); ZG_PIN(qa.H); ZG_PIN(qa.ctx); ZG_PIN(qa.kv_mode); ZG_PIN(qa.kv_lo); ZG_PIN(qa.k_cache); ZG_PIN(qa.v_cache);
     }
     if ((EPI == PF_LINEAR || EPI == PF_LINEAR_PART) && seen_refused(seen)) {  // (every wave alike; its requests still write the ring)
@@ -287,7 +295,7 @@ int launch_ring(const PrefillA& A, const PrefillW& W, const float* bias, void* C
         return ZG_OK;
     }));
     const int tiles = ((M + 64 * TM - 1) / (64 * TM)) * ((N + 64 * TN - 1) / (64 * TN));
-    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, bias, C, M, N, K, ldc, n_sp, qa, PlaneExps{A.exp, W.exps, A.each}, po, raw, seen);
+    prefill_ring_kernel<EPI, TM, TN, NW, ST, NEAR><<<dim3(tiles, n_sp), 256, LDS, s>>>(A.p, W.p, A.exp, W.exps, bias, M, N, K, 2 * n_sp + A.each, C, ldc, qa, po, raw, seen);
     note_kernel("prefill_ring_kernel<%d, %d>", TM, NW);
     ZG_HIP(hipGetLastError());
     return ZG_OK;
