@@ -65,9 +65,10 @@ def test_tile_edges(zg, m, k, n):
     assert check(x, w, b, y) <= 1.33 * ((1.2e-7 * (k / 768) ** 0.5) ** 2 + 0.75e-7 ** 2) ** 0.5
 
 
-@pytest.mark.parametrize("m,k,n,ring", [(700, 1600, 1600, 1), (700, 1600, 1603, 1), (321, 1600, 4800, 1), (1023, 3072, 769, 1), (700, 3072, 768, 1), (65, 6400, 9601, 1),
+@pytest.mark.parametrize("m,k,n,ring", [(700, 1600, 1600, 1), (700, 1600, 1603, 1), (321, 1600, 4800, 1), (1023, 3072, 769, 1), (700, 3072, 768, 1), (300, 2048, 8193, 1),
                                         (450, 6400, 1600, 1), (2049, 1536, 1031, 1), (1501, 1600, 1600, 1), (1409, 1600, 1667, 1), (1500, 3072, 768, 1),
-                                        (2047, 6400, 1600, 1), (700, 1472, 1600, 0), (128, 1600, 1600, 0), (3000, 1600, 4800, 0)])
+                                        (2047, 6400, 1600, 1), (700, 1472, 1600, 0), (128, 1600, 1600, 0), (3000, 1600, 4800, 0),
+                                        (65, 6400, 9601, 0), (128, 4800, 5120, 0), (192, 6400, 6400, 0), (478, 4096, 1024, 0), (420, 6400, 9601, 0)])  # (the weight's split pass would be most of the call)
 def test_some_hundred_rows(zg, m, k, n, ring):
     """Tiles of 64 and 128 rows, of 64 and 128 columns, one slice of K and several, widths in no whole tiles and no whole fours, both sides of the rule."""
     x, w, b = draw(m, k, n, spread=9)

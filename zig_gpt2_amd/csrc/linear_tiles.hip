@@ -348,7 +348,22 @@ bool linear_tiles_pay(size_t M, size_t N, size_t K, bool planes) {
     // 2048 (800) 107 : 101; 6400 -> 1600 1500 rows (600) 278 : 337, 2048 (800) 384 : 342; 3072 -> 768 4096 rows (768) 161 : 185, 6000 (1128) 240 : 192.
     // Below, and for rows that are not for two terms, six of bf16: 128 -> 3072 1856 rows (1392 tiles) and more.
     const size_t tiles = ((M + 63) / 64) * ((N + 63) / 64), rounds = (((M + 255) / 256) * ((N + 191) / 192) + 255) / 256;
-    return tiles <= (!planes || K < kSplit2MinK ? 1400 : K < 1024 ? 1100 : 800) * rounds;
+    // Where the splitting pass leaves the last level's cache it is priced as well: 6400 -> 9601 420 rows 440 : 469, 512 458 : 486 (predicted 453 : 499 and 453 : 504).
+    if (tiles <= (!planes || K < kSplit2MinK ? 1400 : K < 1024 ? 1100 : 800) * rounds) return true;
+    return planes && K >= kSplit2MinK && linear_split_mb(M, N, K) > 240.0 && linear_tiles_us(M, N, K) < (double)rounds * (3.2 * (double)(K / 64) + 10.0) + linear_split_us(M, N, K);
+}
+
+// 13 us, 0.44 a step of 32 columns of the compute unit with the most tiles, and the slabs (within 5 % over 40 to 1200 rows of 14 shapes of 1536 to 8192 columns)
+double linear_tiles_us(size_t M, size_t N, size_t K) {
+    const size_t slices = linear_tiles_slices(M, N, K), steps = (K / kBk + slices - 1) / slices, tiles = ((M + 63) / 64) * ((N + 63) / 64) * slices;
+    return 13.0 + 0.44 * (double)((tiles + 255) / 256 * steps) + (slices > 1 ? 2e-6 * (double)slices * (double)M * (double)N : 0.0);
+}
+
+// The pass that splits both operands in two terms, and the launches: 4 bytes read and 4 written a value, dearer where they leave the last level's cache
+double linear_split_mb(size_t M, size_t N, size_t K) { return (double)(M + N) * (double)K * 8e-6; }
+double linear_split_us(size_t M, size_t N, size_t K) {
+    const double mb = linear_split_mb(M, N, K);
+    return 9.0 + 0.144 * mb + 0.257 * std::max(0.0, mb - 240.0) + 0.0027 * (double)K;
 }
 
 int launch_linear_marked_rows(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, const SplitSeen& seen, hipStream_t s) {

@@ -395,11 +395,13 @@ int launch_linear_ring(const float* X, const float* W, const float* bias, float*
 }
 
 // Priced in us like the prompts' Linears below, with 3 for the launch that adds slabs.  It takes a Linear of 1536 columns and more where the kernel that splits in its own staging
-// has few slices of K to add up, whose chains are then so long that this kernel is closer to 64 bits as well (1600 columns in two slices 1.67e-7, here
-// 0.9e-7; 3072 in four 1.66e-7 and 1.2e-7; 768 in two 1.16e-7 and 1.22e-7), and where it is cheap beside the persistent one (rounds of 256 x 192 tiles: one of
-// 1600 columns 90 predicted, 95 measured; beside several rounds here, which are a sixth longer than predicted, 0.85 of that).  us of a call
-// with it : without: 3072 -> 768 700 rows 44 : 50, 2048 74 : 93, 3000 114 : 143; 1600 -> 1600 700 rows 46 : 52, 2048 64 : 110; 1600 -> 4800 256 rows
-// 47 : 53, 700 65 : 110; 6400 -> 1600 400 rows 78 : 107, 2048 190 : 392; not taken: 1600 -> 4800 1500 rows 139 : 119, 768 -> 768 3000 rows 50 : 46.
+// has few slices of K to add up, whose chains are then so long that this kernel is closer to 64 bits as well (e-7 of the result, that kernel : this: 700 x 1600 x 1600 1.67 : 1.38,
+// 2048 x 3072 x 768 2.35 : 1.64, 400 x 6400 x 1600 2.81 : 1.43), and where it is cheap beside the persistent one (rounds of 256 x 192 tiles: one of
+// 1600 columns 90 predicted, 95 measured; beside several rounds here, which are a sixth longer than predicted, 0.85 of that) and beside the kernel that splits in its
+// own staging.  There the pass over both operands counts, which for few rows is the weight's and most of the call (this kernel behind it: within 9 % over the shapes of
+// linear_tiles_us).  us of a call, without : with: 3072 -> 768 700 rows 48 : 44; 1600 -> 1600 700 rows 49 : 45, 1200 66 : 46; 1600 -> 4800 256 rows 50 : 46,
+// 700 103 : 63; 6400 -> 1600 420 rows 100 : 84, 1200 204 : 131; 4800 -> 5120 300 rows 154 : 117; not taken: 4800 -> 5120 128 rows 66 : 84,
+// 6400 -> 6400 128 rows 103 : 147, 300 205 : 208; 6400 -> 9601 64 rows 83 : 210, 256 270 : 330; 4096 -> 1024 478 rows 47 : 48; 1600 -> 4800 1500 rows 119 : 139.
 int linear_ring_route(size_t M, size_t N, size_t K, int* tm) {
     if (K < 1536 || linear_tiles_slices(M, N, K) > (K < 3072 ? 2 : 4)) return 0;
     const int nk = (int)(K / kBk);
@@ -419,6 +421,7 @@ int linear_ring_route(size_t M, size_t N, size_t K, int* tm) {
             }
         }
     }
+    if (best > 0 && linear_tiles_pay(M, N, K, true) && linear_split_us(M, N, K) + 0.78 * best_us > 0.97 * linear_tiles_us(M, N, K)) return 0;
     return best;
 }
 

@@ -270,6 +270,8 @@ unsigned long long linear_few_mfma_launch_count();  // launches of linear_few_mf
 int launch_linear_few(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, hipStream_t s);
 // Nine rows and more: K a multiple of 64; slabs: linear_tiles_slices(M, N, K) * M * N floats where that is more than one slice.
 bool linear_tiles_pay(size_t M, size_t N, size_t K, bool planes);  // planes: beside the persistent GEMM on fp16 planes where it takes them; else on exact bf16 ones
+double linear_tiles_us(size_t M, size_t N, size_t K);  // what a call by it takes, in us
+double linear_split_mb(size_t M, size_t N, size_t K), linear_split_us(size_t M, size_t N, size_t K);  // the pass in front of the kernels on planes of two terms
 // Outputs of rows (of X and W) that are not for two terms or have values that are not finite, as plain fp32 sums
 int launch_linear_marked_rows(const float* X, const float* W, const float* bias, float* Y, int M, int N, int K, const SplitSeen& seen, hipStream_t s);
 int linear_tiles_slices(size_t M, size_t N, size_t K);
