@@ -215,7 +215,9 @@ void carve(zg_gpt* g, char* wbase, char* sbase) {
             y.exps = (int*)P(kBounds * 4);
         }
     }
-    g->weight_region_bytes = (cv.off + 255) & ~(size_t)255;
+    // The state behind it starts on a border of 64 KB wherever the weights end.  124M, 256 tokens of eight sequences, ms: 36.4 at the 256 bytes or 4 KB that the weights
+    // with the bounds' vectors ended on, 36.2 at 64 KB as at 2 MB.
+    g->weight_region_bytes = (cv.off + 65535) & ~(size_t)65535;
     cv = Carver{};
     base = sbase;
     for (size_t l = 0; l < L; ++l) {
